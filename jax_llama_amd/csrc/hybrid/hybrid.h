@@ -60,6 +60,9 @@ inline bool hy_act_gated(int act) {
 // R <= HY_GEMV_MAX_R and (offs == nullptr or row_expert != nullptr): one wave per output column (weights streamed once
 // per row group); else the 64 x 64 MFMA tiles (offs: expert-grouped).
 constexpr int HY_GEMV_MAX_R = 8;
+// the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, and the launch
+bool hy_rows_gemm_takes(const RowLinear& p);
+int hy_rows_gemm(const RowLinear& p, hipStream_t s);
 int hy_linear_rows(const RowLinear& p, hipStream_t s);
 // two independent linears; one launch where both run the GEMV with the same kind of epilogue (gated or not) at the row counts
 // of a mixture's experts (p) beside its shared expert (q), else one after the other

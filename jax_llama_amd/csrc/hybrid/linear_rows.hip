@@ -5,7 +5,8 @@
 //
 //  * tiles: 64 x 64 or (with rows to fill them) 128 x 64 outputs per 256-thread workgroup, four waves of 32 x 32 /
 //    64 x 32, K staged 32 deep through LDS (several workgroups per CU hide each other's staging; a 128 x 128 tile with
-//    register prefetch and a 64-deep K stage measured slower). The activations may be a bf16 copy and the output bf16
+//    register prefetch and a 64-deep K stage measured slower). A prompt's bf16 rows with K >= 1024 run the 256-row tiles
+//    of rows_gemm.hip instead; these are for few rows per expert, short or odd K, fp32 and scaled activations. The activations may be a bf16 copy and the output bf16
 //    (the expert pair of a prompt: x -> bf16 once, hidden kept bf16), which halves the activation traffic. With an
 //    expert offset table the m-tiles of the launch are dealt to the experts in order (a workgroup finds its expert by
 //    walking the table; surplus workgroups exit), so one launch covers every expert of a token-sorted batch.
@@ -19,6 +20,7 @@
 // The table router's counting sort is here too.
 #include "hy_util.h"
 #include "hybrid.h"
+#include "row_act.h"
 
 namespace jla {
 
@@ -91,33 +93,6 @@ JLA_DEV void lr_zero8(T* dst) {
   const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   lr_store8(dst, z);
 }
-JLA_DEV void lr_out(float* p, float v) { *p = v; }
-JLA_DEV void lr_out(bf16_t* p, float v) { *p = f2bf(v); }
-
-// the epilogue of one output element: g the (gate) accumulator, u the up accumulator of the gated forms
-JLA_DEV float lr_act(const RowLinear& p, float g, float u) {
-  switch (p.act) {
-    case HY_ACT_RELU2: {
-      const float r = fmaxf(g, 0.f);
-      return r * r;
-    }
-    case HY_ACT_SWIGLU:
-      return hy_silu(g) * u;
-    case HY_ACT_CLAMP_GLU: {
-      const float gc = fminf(g, p.act_limit), uc = fminf(fmaxf(u, -p.act_limit), p.act_limit);
-      return gc * hy_sigmoid(p.act_alpha * gc) * (uc + 1.f);
-    }
-    case HY_ACT_SOFTCAP:
-      return p.act_limit * tanhf(g / p.act_limit);
-    case HY_ACT_GELU_GLU:
-      return hy_gelu_tanh(g) * u;
-    default:
-      return g;
-  }
-}
-JLA_DEV float lr_in(const float* p) { return *p; }
-JLA_DEV float lr_in(const bf16_t* p) { return bf2f(*p); }
-
 // WT: weight / tile type; AT: activation type in memory (fp32, or a bf16 copy); OT: output type; TMM: 32-row tiles per
 // wave along M (workgroup tile 64 TMM x 64: the 128-row form halves the weight traffic per output row).
 template <typename WT, int SWIGLU, typename AT, typename OT, int TMM>
@@ -468,6 +443,7 @@ int hy_linear_rows(const RowLinear& p, hipStream_t s) {
   }
   if (!p.offs && p.E != 1) return -3;
   if ((p.a_bf16 || p.out_bf16) && !p.wbf16) return -5;
+  if (hy_rows_gemm_takes(p)) return hy_rows_gemm(p, s);
   // 128-row tiles once every expert (or the whole batch) has rows to fill them; the SwiGLU form (two accumulator sets)
   // only with many such tiles per expert (measured: 512 rows per expert run faster on 64-row tiles, 4096 on 128-row)
   const long long per_e = p.R / (p.offs ? p.E : 1);

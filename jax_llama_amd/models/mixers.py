@@ -437,7 +437,7 @@ class GatedDenseFF:
         self.w_gu, self.w_o, self.limit, self.alpha, self.act = w_gu, w_down, limit, alpha, act
 
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
-        return hy.linear(h, self.w_gu, act=self.act, limit=self.limit, alpha=self.alpha)
+        return hy.linear(h, self.w_gu, act=self.act, limit=self.limit, alpha=self.alpha, out_dtype=self.w_gu.dtype)
 
     def __call__(self, h, ctx: StepContext) -> torch.Tensor:
         return hy.linear(self.features(h, ctx), self.w_o)

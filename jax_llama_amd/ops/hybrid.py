@@ -225,13 +225,14 @@ def _act_cpu(y: torch.Tensor, act: int, limit: float, alpha: float) -> torch.Ten
 
 
 def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit: float = 0.0,
-           alpha: float = 1.0) -> torch.Tensor:
+           alpha: float = 1.0, out_dtype=F32) -> torch.Tensor:
     """``act(x [M, K] (fp32, or an ``RmsInput``) @ w^T)`` -> fp32 ``[M, N]``. ``act``: none, ``ACT_RELU2`` (``max(y, 0)^2``),
     ``ACT_SOFTCAP`` (``limit * tanh(y / limit)``; ``limit = 1`` is a plain tanh), or a gated
     form for which ``w`` is ``[2N, K]`` (gate rows, then up rows): ``ACT_SWIGLU`` (``silu(g) * u``; also
     ``swiglu=True``), ``ACT_GELU_GLU`` (``gelu_tanh(g) * u``) or ``ACT_CLAMP_GLU`` (``g' sigmoid(alpha g') (u' + 1)``,
     ``g' = min(g, limit)``, ``u' = clamp(u, -limit, limit)``). ``x`` may be a column-contiguous view with strided rows; with
-    bf16 weights and no activation it may be bf16 already (the operand it would be rounded to anyway)."""
+    bf16 weights and no activation it may be bf16 already (the operand it would be rounded to anyway). ``out_dtype`` bf16:
+    the result as the next product's operand, where that saves a pass (a prompt on the large tiles); else fp32 all the same."""
     if swiglu:
         act = ACT_SWIGLU
     n = w.shape[0] // 2 if act_gated(act) else w.shape[0]
@@ -241,6 +242,12 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     if act == ACT_NONE and norm_w is None and _use_packed_gemm(x, w):
         from . import linear as packed_linear
         return packed_linear(_bf16_rows(x), _packed_weight(w), out_dtype=F32)
+    if act_gated(act) and norm_w is None and x.shape[0] >= PACKED_GEMM_MIN_M and ext().rows_gemm_takes(x.shape[0], w, int(act)):
+        # a prompt's gated product: bf16 rows (the operands they would be rounded to anyway) on the large tiles
+        xb = _bf16_rows(x) if x.is_contiguous() and x.numel() % 8 == 0 else x.to(BF16).contiguous()
+        out = torch.empty(x.shape[0], n, dtype=out_dtype, device=x.device)
+        ext().linear_rows(xb, None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, None, 0.0)
+        return out
     out = torch.empty(x.shape[0], n, dtype=F32, device=x.device)
     ext().linear_rows(x, None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, norm_w,
                       norm_eps)
@@ -327,9 +334,7 @@ def linear_add_(res: torch.Tensor, x, w: torch.Tensor) -> torch.Tensor:
         return res.add_(_round_like(x, w) @ w.float().t())
     if norm_w is None and res.is_contiguous() and _use_packed_gemm(x, w):
         from . import linear_residual as packed_linear_residual
-        xb = torch.empty(x.shape, dtype=BF16, device=x.device)
-        ext().cast_bf16(x, xb)
-        return packed_linear_residual(xb, _packed_weight(w), res)
+        return packed_linear_residual(_bf16_rows(x), _packed_weight(w), res)
     ext().linear_rows(x, None, w, res, None, None, None, x.shape[0], ACT_NONE, 0.0, 1.0, None, norm_w, norm_eps, 0, True)
     return res
 

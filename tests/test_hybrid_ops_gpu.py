@@ -420,3 +420,31 @@ def test_moe_grouped_and_the_stream_update(dt, m, experts, identity, top):
     _close(ug, u, 5e-5, "next input")
     s_up, s_down = _rand(ff, d, dt=dt, std=d ** -0.5), _rand(d, ff, dt=dt, std=ff ** -0.5)
     _close(hy.ff_dense(x.to(DEV), s_up.to(DEV), s_down.to(DEV)), hy.ff_dense(x, s_up, s_down), 2e-5, "one-accumulator FF")
+
+
+@pytest.mark.parametrize("counts", [[300], [255, 0, 257, 1, 512], [128] * 7 + [0, 33]])
+@pytest.mark.parametrize("k,n", [(1024, 260), (1088, 516), (1024, 8192 + 4)])
+@pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_RELU2, hy.ACT_SWIGLU, hy.ACT_CLAMP_GLU, hy.ACT_GELU_GLU])
+def test_rows_on_the_large_tiles(counts, k, n, act):
+    """Prompt-sized bf16 rows on the 256-row tiles (both tile widths): ragged and empty experts, gathered rows, scattered
+    results, every activation, both result types, the add into the output. fp32 sums of k products of about 1 / sqrt(k)
+    each differ from the reference's by their order alone (1e-6 of the result's size; squared-ReLU doubles it); a bf16
+    result by its own rounding, 2^-9."""
+    e, r = len(counts), sum(counts)
+    gated = hy.act_gated(act)
+    g = torch.Generator().manual_seed(k + n + act)
+    w = (torch.randn(e, 2 * n if gated else n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    x = torch.randn(r + 5, k, generator=g).to(torch.bfloat16).to(DEV)
+    src = torch.randperm(r + 5, generator=g)[:r].to(torch.int32).to(DEV)
+    dst = torch.randperm(r, generator=g).to(torch.int32).to(DEV)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(DEV)
+    xs = x[src.long()].float()
+    ref = torch.empty(r, n, device=DEV)
+    for i in range(e):
+        a, b = int(offs[i]), int(offs[i + 1])
+        ref[dst[a:b].long()] = hy._act_cpu(xs[a:b] @ w[i].float().t(), act, 2.0, 1.7)
+    for out_dtype, add in ((torch.float32, False), (torch.float32, True), (torch.bfloat16, False)):
+        out = torch.full((r, n + 4), 0.5, dtype=out_dtype, device=DEV)[:, :n]
+        ww = w if e > 1 else w[0]
+        hy.ext().linear_rows(x, src, ww, out, dst, offs if e > 1 else None, None, r, act, 2.0, 1.7, None, None, 0.0, 0, add)
+        _close(out.float() - (0.5 if add else 0.0), ref, 2e-5 if out_dtype == torch.float32 else 4e-3, "large tiles")
