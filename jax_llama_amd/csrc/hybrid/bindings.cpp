@@ -615,6 +615,13 @@ void delta_scan(Tensor qn, Tensor kn, Tensor v, Tensor beta, Tensor decay, Tenso
   p.state = f32w(state, "state");
   p.o = f32w(o, "o");
   p.B = B; p.S = S; p.H = H; p.G = G; p.dim = dim; p.vdim = vdim;
+  // a prompt whose rows the chunked form can read (16-byte rows) runs on the matrix cores, the rest token by token
+  const long long floats = ((uintptr_t)p.qn | (uintptr_t)p.kn) & 15 ? 0 : jla::hy_delta_chunk_floats(p);
+  if (floats > 0) {
+    Tensor ws = torch::empty({floats}, qn.options());
+    rc(jla::hy_delta_chunk(p, reinterpret_cast<float*>(ws.data_ptr()), stream()), "delta_scan");
+    return;
+  }
   rc(jla::hy_delta_scan(p, stream()), "delta_scan");
 }
 

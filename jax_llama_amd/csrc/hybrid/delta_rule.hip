@@ -10,7 +10,8 @@
 //                          g = exp(-exp(A_log) softplus(a + dt_bias)).
 //   hy_conv_state_update : the carried tail <- the last taps - 1 inputs of every channel (after hy_delta_prep; a
 //                          one-token step does it inside hy_delta_prep and launches nothing here).
-//   hy_delta_scan        : the recurrence, token by token. A thread owns 16 key rows of one value column in registers;
+//   hy_delta_scan        : the recurrence, token by token (a decode step, short prompts and head sizes that the chunked
+//                          form of delta_chunk.hip does not take). A thread owns 16 key rows of one value column in registers;
 //                          the lanes sharing a column (dim / 16 of them, adjacent) combine their partial S^T k and
 //                          S^T q by lane exchange. k, q, v, g, beta of the next tokens are staged through LDS.
 //   hy_gated_rmsnorm     : o / rms(o) * w * act(gate) per head (silu or sigmoid; the gain per column or per head and

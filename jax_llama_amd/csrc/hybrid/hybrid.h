@@ -306,6 +306,9 @@ struct DeltaScan {
   int B, S, H, G, dim, vdim;
 };
 int hy_delta_scan(const DeltaScan& p, hipStream_t s);
+// the same recurrence in chunks on the matrix cores (delta_chunk.hip): floats of scratch it needs, 0 where it does not apply
+long long hy_delta_chunk_floats(const DeltaScan& p);
+int hy_delta_chunk(const DeltaScan& p, float* ws, hipStream_t s);
 
 // out[m * ldo + h * vdim + j] = x[m, h, j] / sqrt(mean_j(x^2) + eps) * w[w_heads ? h * vdim + j : j] *
 // act(gate[m * ldg + h * vdim + j]) * gain, act = silu (gate_act 0), sigmoid (1) or no gate (2). x = o, or with

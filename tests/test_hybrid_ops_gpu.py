@@ -124,6 +124,12 @@ def test_attention(dt, shape, own_kv):
 @pytest.mark.parametrize("shape", [dict(b=1, s=1, h=4, g=2, dim=32, vdim=32, taps=4),
                                    dict(b=2, s=2, h=2, g=1, dim=40, vdim=24, taps=4),
                                    dict(b=1, s=37, h=6, g=3, dim=128, vdim=72, taps=3),
+                                   # the chunked form: its shortest prompt, whole and ragged chunks, idle waves
+                                   dict(b=1, s=19, h=2, g=1, dim=64, vdim=64, taps=4),
+                                   dict(b=2, s=20, h=2, g=1, dim=64, vdim=16, taps=4),
+                                   dict(b=1, s=64, h=4, g=2, dim=128, vdim=128, taps=4),
+                                   dict(b=3, s=97, h=2, g=2, dim=128, vdim=80, taps=4),
+                                   dict(b=1, s=321, h=2, g=1, dim=64, vdim=48, taps=2),
                                    dict(b=2, s=9, h=2, g=2, dim=16, vdim=130, taps=1)])
 def test_delta_rule(shape):
     b, s, h, g, dim, vdim, taps = (shape[k] for k in ("b", "s", "h", "g", "dim", "vdim", "taps"))
@@ -132,6 +138,7 @@ def test_delta_rule(shape):
     conv_w, tail = _rand(c, taps, std=0.6), _rand(b, c, max(taps - 1, 0))
     a_log, dt_bias = torch.rand(h) - 1.0, torch.randn(h)
     state = _rand(b, h, dim, vdim, std=0.3)
+    state64 = state.double()
     tail_g, state_g = tail.clone().to(DEV), state.clone().to(DEV)
     ref = hy.delta_prep(proj, b, s, h, g, dim, vdim, conv_w, tail, a_log, dt_bias)
     got = hy.delta_prep(proj.to(DEV), b, s, h, g, dim, vdim, conv_w.to(DEV), tail_g, a_log.to(DEV), dt_bias.to(DEV))
@@ -142,6 +149,17 @@ def test_delta_rule(shape):
     o_got = hy.delta_scan(*(x.to(DEV) for x in ref), state_g, b, s)
     _close(o_got, o_ref, 5e-5, "delta o")
     _close(state_g, state, 5e-5, "delta state")
+    # against 64 bits from the same operands: the chunked form rounds a sum where the token loop rounds each step
+    st = state64
+    q64, k64, v64, be, de = (x.double() for x in ref)
+    for t in range(s):
+        at = torch.arange(b) * s + t
+        kk, qq = (x[at].repeat_interleave(h // g, 1) for x in (k64, q64))
+        st = st * de[at][..., None, None]
+        u = be[at][..., None] * (v64[at] - torch.einsum("bhdv,bhd->bhv", st, kk))
+        st = st + kk[..., None] * u[:, :, None]
+    err = float((state_g.cpu().double() - st).norm() / st.norm())
+    assert err < 5e-7, f"state against 64 bits: {err:.2e}"
     gate, w = _rand(b * s, h * vdim), torch.rand(vdim) + 0.5
     _close(hy.gated_rmsnorm(o_ref.to(DEV), gate.to(DEV), w.to(DEV), 1e-6), hy.gated_rmsnorm(o_ref, gate, w, 1e-6), 2e-5,
            "gated norm")
