@@ -62,6 +62,9 @@ inline bool hy_act_gated(int act) {
 constexpr int HY_GEMV_MAX_R = 8;
 // the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, and the launch
 bool hy_rows_gemm_takes(const RowLinear& p);
+// the matrix-core form of a few bf16 rows (rows_gemv.hip)
+bool hy_rows_gemv_takes(const RowLinear& p);
+int hy_rows_gemv(const RowLinear& p, hipStream_t s);
 int hy_rows_gemm(const RowLinear& p, hipStream_t s);
 int hy_linear_rows(const RowLinear& p, hipStream_t s);
 // two independent linears; one launch where both run the GEMV with the same kind of epilogue (gated or not) at the row counts

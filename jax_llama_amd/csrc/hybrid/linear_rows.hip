@@ -404,6 +404,7 @@ int hy_linear_rows(const RowLinear& p, hipStream_t s) {
   if (p.offs && p.E > 65535) return -2;
   const bool grouped = lr_grouped(p);
   const bool small = hy_linear_rows_is_gemv(p);
+  if (!lr_skinny(p) && hy_rows_gemv_takes(p)) return hy_rows_gemv(p, s);
   if (p.a_norm_w && (!small || p.a_bf16)) return -10;  // (the tiles take a normed activation, they do not norm it)
   if (small) {
     if (p.a_bf16 || p.out_bf16) return -7;  // (the GEMV reads and writes fp32)

@@ -466,3 +466,48 @@ def test_rows_on_the_large_tiles(counts, k, n, act):
         ww = w if e > 1 else w[0]
         hy.ext().linear_rows(x, src, ww, out, dst, offs if e > 1 else None, None, r, act, 2.0, 1.7, None, None, 0.0, 0, add)
         _close(out.float() - (0.5 if add else 0.0), ref, 2e-5 if out_dtype == torch.float32 else 4e-3, "large tiles")
+
+
+@pytest.mark.parametrize("r", [1, 2, 4, 5, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("k,n", [(264, 20), (2048, 130), (1096, 4100), (448, 2)])
+@pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_SWIGLU, hy.ACT_SOFTCAP])
+def test_few_rows_on_the_matrix_cores(r, k, n, act):
+    """A few rows on bf16 weights: every rows-per-pass form and tile count, K that ends inside a step, ragged columns; dense
+    (strided rows, per-row scale, add into the output, scattered results), a norm on the way in, one expert per row and
+    expert-sorted rows. Sums of k products differ from the reference's by their order."""
+    gated = hy.act_gated(act)
+    g = torch.Generator().manual_seed(r * 1000 + k + n + act)
+    e = 3
+    w = (torch.randn(e, 2 * n if gated else n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    x = torch.randn(r, k + 4, generator=g).to(DEV)[:, :k]
+    sc = (torch.rand(r, generator=g) + 0.5).to(DEV)
+    dst = torch.randperm(r, generator=g).to(torch.int32).to(DEV)
+    gain = (torch.rand(k, generator=g) + 0.5).to(DEV)
+    ex = torch.randint(0, e + 1, (r,), generator=g).to(torch.int32)  # (e: an expert without weights)
+    order = torch.argsort(ex, stable=True)
+    offs = torch.tensor([int((ex < i).sum()) for i in range(e + 1)], dtype=torch.int32).to(DEV)
+
+    def product(rows, wi):
+        return hy._act_cpu(rows.to(torch.bfloat16).float() @ wi.float().t(), act, 1.5, 1.0)
+
+    def run(wt, out, dst_=None, offs_=None, row_expert=None, a_idx=None, a_scale=None, norm=None, add=False):
+        hy.ext().linear_rows(x, a_idx, wt, out, dst_, offs_, row_expert, r, act, 1.5, 1.0, a_scale, norm, 1e-5, 0, add)
+        return out
+
+    new = lambda: torch.full((r, n + 3), 0.25, device=DEV)[:, :n]  # noqa: E731
+    ref = product(x, w[1])
+    _close(run(w[1], new()), ref, 2e-5, "dense")
+    _close(run(w[1], new(), add=True) - 0.25, ref, 3e-5, "added")
+    _close(run(w[1], new(), dst_=dst, a_scale=sc)[dst.long()], product(x * sc[:, None], w[1]), 2e-5, "scaled, scattered")
+    if r <= 2:
+        normed = (x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5)) * gain
+        # (the norm's own sum differs by its order, which can round an operand to the neighbouring bf16)
+        _close(run(w[1], new(), norm=gain), product(normed, w[1]), 3e-3, "normed")
+    per = torch.full((r, n), 0.25, device=DEV)
+    for i in range(e):
+        sel = (ex == i).nonzero().squeeze(1).to(DEV)
+        per[sel] = product(x[sel], w[i])
+    if r <= hy.ext().GEMV_MAX_R:
+        _close(run(w, new(), row_expert=ex.to(DEV)), per, 2e-5, "an expert per row")
+    idx = order.to(torch.int32).to(DEV)
+    _close(run(w, new(), dst_=idx, offs_=offs, a_idx=idx), per, 2e-5, "expert-sorted")
