@@ -127,7 +127,11 @@ void gemm_f32(Tensor x, Tensor w, Tensor y) {
   check(x.dim() == 2 && w.dim() == 2 && y.dim() == 2 && x.size(1) == w.size(1) && y.size(0) == x.size(0) &&
             y.size(1) == w.size(0),
         "gemm_f32 shapes");
-  rc(jla::gemm_f32(ptr<float>(x), ptr<float>(w), ptr<float>(y), x.size(0), w.size(0), x.size(1), stream()), "gemm_f32");
+  const int64_t floats = jla::gemm_f32_workspace(ptr<float>(x), ptr<float>(w), ptr<float>(y), x.size(0), w.size(0), x.size(1));
+  Tensor ws;  // (split K: partial sums, freed on the stream that used them)
+  if (floats > 0) ws = torch::empty({floats}, x.options());
+  rc(jla::gemm_f32(ptr<float>(x), ptr<float>(w), ptr<float>(y), x.size(0), w.size(0), x.size(1),
+                   floats > 0 ? ptr<float>(ws) : nullptr, stream()), "gemm_f32");
 }
 
 void check_packed(const Tensor& w, int64_t n, int64_t k) {

@@ -118,18 +118,27 @@ jla::RowLinear row_linear(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_i
   return p;
 }
 
+// scratch of a call, from the allocator of the stream that uses it
+Tensor row_scratch(long long floats, const Tensor& like) {
+  return floats > 0 ? torch::empty({floats}, like.options().dtype(torch::kFloat32)) : Tensor();
+}
+float* scratch_ptr(const Tensor& t) { return t.defined() ? reinterpret_cast<float*>(t.data_ptr()) : nullptr; }
+
 void linear_rows(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT offs, OptT row_expert, int64_t R,
                  int64_t act, double act_limit, double act_alpha, OptT a_scale, OptT a_norm_w, double a_norm_eps,
                  int64_t even_rows, bool add_out) {
-  rc(jla::hy_linear_rows(row_linear(a, a_idx, w, out, dst_idx, offs, row_expert, R, act, act_limit, act_alpha, a_scale, a_norm_w,
-                                    a_norm_eps, even_rows, add_out),
-                         stream()),
-     "linear_rows");
+  const jla::RowLinear p = row_linear(a, a_idx, w, out, dst_idx, offs, row_expert, R, act, act_limit, act_alpha, a_scale,
+                                      a_norm_w, a_norm_eps, even_rows, add_out);
+  const Tensor ws = row_scratch(jla::hy_linear_rows_floats(p), out);
+  rc(jla::hy_linear_rows(p, scratch_ptr(ws), stream()), "linear_rows");
 }
 
 // p and q from row_linear: the tensors they were made from must be alive
 void linear_rows_pair(const jla::RowLinear& p, const jla::RowLinear& q) {
-  rc(jla::hy_linear_rows_pair(p, q, stream()), "linear_rows_pair");
+  const long long a = jla::hy_linear_rows_floats(p), b = jla::hy_linear_rows_floats(q);
+  Tensor ws;
+  if (a > 0 || b > 0) ws = torch::empty({a > b ? a : b}, torch::TensorOptions().dtype(torch::kFloat32).device(torch::kCUDA));
+  rc(jla::hy_linear_rows_pair(p, q, scratch_ptr(ws), stream()), "linear_rows_pair");
 }
 
 // whether a dense linear of `rows` rows with `n` output columns runs the GEMV (where an input norm can be fused)

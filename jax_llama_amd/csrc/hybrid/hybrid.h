@@ -62,14 +62,20 @@ inline bool hy_act_gated(int act) {
 constexpr int HY_GEMV_MAX_R = 8;
 // the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, and the launch
 bool hy_rows_gemm_takes(const RowLinear& p);
+// the fp32 tiles as split products on the bf16 matrix cores (rows_f32.hip)
+bool hy_rows_f32_takes(const RowLinear& p);
+long long hy_rows_f32_floats(const RowLinear& p);  // scratch of its split-K form (0: none)
+int hy_rows_f32(const RowLinear& p, float* ws, hipStream_t s);
 // the matrix-core form of a few bf16 rows (rows_gemv.hip)
 bool hy_rows_gemv_takes(const RowLinear& p);
 int hy_rows_gemv(const RowLinear& p, hipStream_t s);
 int hy_rows_gemm(const RowLinear& p, hipStream_t s);
-int hy_linear_rows(const RowLinear& p, hipStream_t s);
+// ws: hy_linear_rows_floats() floats of scratch, 16-byte aligned (0: none needed)
+long long hy_linear_rows_floats(const RowLinear& p);
+int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s);
 // two independent linears; one launch where both run the GEMV with the same kind of epilogue (gated or not) at the row counts
 // of a mixture's experts (p) beside its shared expert (q), else one after the other
-int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, hipStream_t s);
+int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, float* ws, hipStream_t s);
 
 // Table routing: expert of (token m, choice c) = table[ids[m], c]. Writes row_expert[R] and row_tok[R] in (m, c) order
 // (R = M * top), and the expert-sorted order: sort_tok[p] (token of sorted row p), sort_dst[p] (its (m, c) row),

@@ -351,7 +351,7 @@ static int lr_pass_rows(const RowLinear& p) {
   return want > 4 ? HY_GEMV_MAX_R : (want > 2 ? 4 : (want > 1 ? 2 : 1));
 }
 
-int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, hipStream_t s) {
+int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, float* ws, hipStream_t s) {
   auto plain = [](const RowLinear& x) {  // what the one-launch form takes
     return x.R > 0 && x.N > 0 && x.K > 0 && x.lda >= x.K && x.ldo >= x.N && x.E >= 1 && x.E <= 65535 && x.N < 8192 &&
            !x.a_norm_w && lr_fp32_io(x) && hy_linear_rows_is_gemv(x) && x.act >= HY_ACT_NONE && x.act <= HY_ACT_GELU_GLU &&
@@ -361,8 +361,8 @@ int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, hipStream_t s) {
   const int ra = lr_pass_rows(p), rb = lr_pass_rows(q);  // instances: per-row experts beside 1, 2 or 4 rows; 8 beside 8
   if (!plain(p) || !plain(q) || p.wbf16 != q.wbf16 || gated != hy_act_gated(q.act) ||
       !((ra == 1 && rb <= 4) || (ra == 8 && rb == 8))) {
-    const int r = hy_linear_rows(p, s);
-    return r ? r : hy_linear_rows(q, s);
+    const int r = hy_linear_rows(p, ws, s);
+    return r ? r : hy_linear_rows(q, ws, s);
   }
   RowLinear a = p, b = q;
   if (!lr_grouped(p)) a.offs = nullptr;
@@ -393,7 +393,14 @@ int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, hipStream_t s) {
   return 0;
 }
 
-int hy_linear_rows(const RowLinear& p, hipStream_t s) {
+long long hy_linear_rows_floats(const RowLinear& p) {
+  if (p.R <= 0 || p.N <= 0 || p.K <= 0 || hy_linear_rows_is_gemv(p) || hy_rows_gemv_takes(p) || hy_rows_gemm_takes(p) ||
+      !hy_rows_f32_takes(p))
+    return 0;
+  return hy_rows_f32_floats(p);
+}
+
+int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s) {
   if (p.R < 0 || p.N <= 0 || p.K <= 0 || p.lda < p.K || p.ldo < p.N || p.E < 1) return -1;
   if (p.act < HY_ACT_NONE || p.act > HY_ACT_GELU_GLU) return -8;
   if (p.act == HY_ACT_SOFTCAP && !(p.act_limit > 0.f)) return -8;
@@ -445,6 +452,7 @@ int hy_linear_rows(const RowLinear& p, hipStream_t s) {
   if (!p.offs && p.E != 1) return -3;
   if ((p.a_bf16 || p.out_bf16) && !p.wbf16) return -5;
   if (hy_rows_gemm_takes(p)) return hy_rows_gemm(p, s);
+  if (hy_rows_f32_takes(p)) return hy_rows_f32(p, ws, s);
   // 128-row tiles once every expert (or the whole batch) has rows to fill them; the SwiGLU form (two accumulator sets)
   // only with many such tiles per expert (measured: 512 rows per expert run faster on 64-row tiles, 4096 on 128-row)
   const long long per_e = p.R / (p.offs ? p.E : 1);

@@ -15,6 +15,7 @@
 // The epilogue passes 64 rows at a time through the wave's own 32 KiB of LDS: the activation is then one small loop and
 // rows leave as full lines (fp32: 512 B per row and wave).
 #include "../kernels/gemm4w.h"
+#include "../kernels/row_tiles.h"
 #include "hy_util.h"
 #include "hybrid.h"
 #include "row_act.h"
@@ -23,51 +24,6 @@ namespace jla {
 
 constexpr int RG_BM = 256, RG_BK = 64;
 constexpr int RG_SLOT_U4 = 2 * RG_BM * RG_BK * 2 / 16;  // u32x4 of one slot: A 32 KiB + W 32 KiB (NJ = 4: half of it used)
-
-// Tile pid of the launch order -> expert e, its rows [r0, rend) and the column tile; false: no such tile. Workgroups are
-// dealt round robin to the 8 XCDs, so XCD x takes the x-th eighth of the order (expert by expert, groups of 4 m-tiles
-// across every column tile): the tiles that run side by side behind one L2 share weight columns and activation rows.
-// Every wave computes the same answer: lane l looks at experts l, l + 64, ...
-JLA_DEV bool rg_tile(const RowLinear& p, int tiles_n, int lane, int& e, int& r0, int& rend, int& tn) {
-  const int E = p.offs ? p.E : 1;
-  auto rows = [&](int x) { return x < E ? (p.offs ? p.offs[x + 1] - p.offs[x] : p.R) : 0; };
-  int total = 0;
-  for (int b = 0; b < E; b += 64) {
-    int n = (rows(b + lane) + RG_BM - 1) / RG_BM;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-    total += n;
-  }
-  total *= tiles_n;
-  const int per = (total + 7) / 8, at = blockIdx.x >> 3;
-  const int pid = (int)(blockIdx.x & 7) * per + at;
-  if (at >= per || pid >= total) return false;
-  int before = 0;  // m-tiles of the experts passed
-  for (int b = 0; b < E; b += 64) {
-    const int n = (rows(b + lane) + RG_BM - 1) / RG_BM;
-    int inc = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += v;
-    }
-    const unsigned long long hit = __ballot(pid < (before + inc) * tiles_n);
-    if (hit) {
-      const int src = (int)__builtin_ctzll(hit);
-      e = __builtin_amdgcn_readfirstlane(b + src);
-      const int mine = __builtin_amdgcn_readlane(n, src);
-      const int start = (before + __builtin_amdgcn_readlane(inc, src) - mine) * tiles_n;
-      int tm;
-      g4_tile_coords(pid - start, mine, tiles_n, tm, tn, 4);
-      const int first = p.offs ? p.offs[e] : 0;
-      r0 = first + tm * RG_BM;
-      rend = p.offs ? p.offs[e + 1] : p.R;
-      return true;
-    }
-    before += __builtin_amdgcn_readlane(inc, 63);
-  }
-  return false;
-}
 
 template <int NJ>
 __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gated, int tiles_n) {
@@ -78,7 +34,7 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
   const int wu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wu >> 1, wc = wu & 1;
   int e = 0, r0 = 0, rend = 0, tn = 0;
-  if (!rg_tile(p, tiles_n, lane, e, r0, rend, tn)) return;
+  if (!row_tile<RG_BM>(p.offs, p.E, p.R, tiles_n, lane, e, r0, rend, tn)) return;
   const int K = p.K, N = p.N, KT = K / RG_BK;
   const int cols = gated ? 16 * NJ : 32 * NJ;  // output columns of the workgroup
   const int n0 = tn * cols;

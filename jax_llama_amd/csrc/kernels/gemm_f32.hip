@@ -1,12 +1,14 @@
 // fp32 GEMM for the precision='highest' lm_head (reference model.py:698-736: only the lm_head honours
 // `precision`, jax_test.py:433 runs the parity harness with precision='highest').
 //
-// y[M, N] = x[M, K] @ W[N, K]^T with fp32 inputs, fp32 accumulation and fp32 output on the exact-f32 MFMA
-// (v_mfma_f32_32x32x2_f32: a k-ordered fmaf chain, no xf32 shortcut on gfx950). Opt-in path (the default
-// lm_head is the bf16 GEMV/GEMM), so the design is simple and robust rather than tuned: 128 x 128 output tile per
-// 256-thread workgroup, four waves of 64 x 64 (2 x 2 MFMA tiles), K staged 32 deep through LDS in k-major images
-// ([k][row]) so a lane's fragment element (row l & 31, k l >> 5) is one conflict-free ds_read_b32.
+// y[M, N] = x[M, K] @ W[N, K]^T with fp32 inputs, fp32 accumulation and fp32 output. Rows of whole 16-byte pieces run as
+// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 146, 100 567 -> 222,
+// 600 1780 -> 1028, 6000 15484 -> 8514); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
+// k-ordered fmaf chain, no xf32 shortcut on gfx950): 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64
+// (2 x 2 MFMA tiles), K staged 32 deep through LDS in k-major images ([k][row]) so a lane's fragment element (row l & 31, k
+// l >> 5) is one conflict-free ds_read_b32.
 #include "common.h"
+#include "gemm_f32x3.h"
 #include "launchers.h"
 
 namespace jla {
@@ -93,8 +95,56 @@ __global__ void __launch_bounds__(GF_THREADS)
     }
 }
 
-int gemm_f32(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
+template <int BM>
+__global__ void __launch_bounds__(256, 2) gemm_f32x3_kernel(F3Rows p, int tiles_n, int steps) {
+  __shared__ u32x4 lds[f3_lds<BM>()];
+  const int t0 = blockIdx.y * steps;
+  p.out += (size_t)blockIdx.y * p.R * p.ldo;
+  f3_tile<BM, 0>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
+                 [](const f32x4 g, const f32x4) { return g; });
+}
+
+__global__ void __launch_bounds__(256) gemm_f32_sum_kernel(const f32x4* slabs, f32x4* y, size_t n, int splits) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  f32x4 v = slabs[i];
+  for (int s = 1; s < splits; ++s) v += slabs[s * n + i];
+  y[i] = v;
+}
+
+static bool f32x3_takes(const float* x, const float* w, const float* y, int M, int N, int K) {
+  return M > 0 && N > 0 && K > 0 && K % 8 == 0 && N % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
+}
+static F3Plan f32x3_plan(int M, int N, int K) {
+  return f3_plan((M + 127) / 128, (M + 63) / 64, (N + F3_BN - 1) / F3_BN, K);
+}
+
+long long gemm_f32_workspace(const float* x, const float* w, const float* y, int M, int N, int K) {
+  if (!f32x3_takes(x, w, y, M, N, K)) return 0;
+  const F3Plan pl = f32x3_plan(M, N, K);
+  return pl.splits > 1 ? (long long)pl.splits * M * N : 0;
+}
+
+int gemm_f32(const float* x, const float* w, float* y, int M, int N, int K, float* ws, hipStream_t s) {
   if (M <= 0 || N <= 0 || K <= 0) return M < 0 || N < 0 || K < 0 ? -1 : 0;
+  if (f32x3_takes(x, w, y, M, N, K)) {
+    const F3Plan pl = f32x3_plan(M, N, K);
+    if (pl.splits > 1 && (!ws || ((uintptr_t)ws & 15))) return -3;
+    const F3Rows p{x, K, nullptr, nullptr, w, (long long)N * K, N, K, pl.splits > 1 ? ws : y, N, nullptr, 0, nullptr, 1, M};
+    const long long tn = (N + F3_BN - 1) / F3_BN, tiles = ((M + pl.bm - 1) / pl.bm * tn + 7) / 8 * 8;
+    if (tiles > 0x7fffffffLL) return -2;
+    const dim3 grid((unsigned)tiles, pl.splits);
+    if (pl.bm == 64) gemm_f32x3_kernel<64><<<grid, 256, 0, s>>>(p, (int)tn, pl.steps);
+    else gemm_f32x3_kernel<128><<<grid, 256, 0, s>>>(p, (int)tn, pl.steps);
+    JLA_CHECK_LAUNCH();
+    if (pl.splits > 1) {
+      const size_t n = (size_t)M * N / 4;
+      gemm_f32_sum_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(reinterpret_cast<const f32x4*>(ws),
+                                                                      reinterpret_cast<f32x4*>(y), n, pl.splits);
+      JLA_CHECK_LAUNCH();
+    }
+    return 0;
+  }
   dim3 grid((N + GF_BN - 1) / GF_BN, (M + GF_BM - 1) / GF_BM);
   if (grid.y > 65535) return -2;
   gemm_f32_kernel<<<grid, GF_THREADS, 0, s>>>(x, w, y, M, N, K);

@@ -17,7 +17,9 @@ int rms_rowinv(const bf16_t* x, float* inv, int M, int D, float eps, hipStream_t
 int residual_add(float* h, const void* p, int p_bf16, bf16_t* hb, long long n, hipStream_t s);
 int prefetch(const void* p, long long nbytes, int grid, unsigned* sink, hipStream_t s);
 int stream_probe(const void* p, long long nbytes, int grid, unsigned* sink, hipStream_t s);  // bytes read: per-wave contiguous ranges
-int gemm_f32(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s);
+// (ws: gemm_f32_workspace() floats, 16-byte aligned; 0: none needed)
+long long gemm_f32_workspace(const float* x, const float* w, const float* y, int M, int N, int K);
+int gemm_f32(const float* x, const float* w, float* y, int M, int N, int K, float* ws, hipStream_t s);
 int rmsnorm(const float* x, const float* w, float* out, int M, int D, float eps, hipStream_t s);
 
 // Epilogue arguments of the fused qkv projection (MODE_QKV): RoPE + KV-cache write.

@@ -511,3 +511,52 @@ def test_few_rows_on_the_matrix_cores(r, k, n, act):
         _close(run(w, new(), row_expert=ex.to(DEV)), per, 2e-5, "an expert per row")
     idx = order.to(torch.int32).to(DEV)
     _close(run(w, new(), dst_=idx, offs_=offs, a_idx=idx), per, 2e-5, "expert-sorted")
+
+
+@pytest.mark.parametrize("counts", [[9], [65], [300], [255, 0, 257, 1, 64], [33] * 9])
+@pytest.mark.parametrize("k,n", [(256, 260), (1096, 132), (2048, 20)])
+@pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_CLAMP_GLU])
+def test_fp32_rows_as_split_products(counts, k, n, act):
+    """fp32 tiles on the bf16 matrix cores: both row tiles, one and several K splits, K that ends inside a step, ragged and
+    empty experts, gathered, scaled and scattered rows, the add into the output. Against 64 bits: every product is exact to
+    2^-23 and the fp32 sum of k of them rounds like any other (5e-6 of the summed magnitudes, as for the exact-f32 path)."""
+    e, r = len(counts), sum(counts)
+    gated = hy.act_gated(act)
+    g = torch.Generator().manual_seed(k + n + act + r)
+    w = (torch.randn(e, 2 * n if gated else n, k, generator=g) * k ** -0.5).to(DEV)
+    x = torch.randn(r + 5, k + 4, generator=g).to(DEV)[:, :k]
+    src = torch.randperm(r + 5, generator=g)[:r].to(torch.int32).to(DEV)
+    dst = torch.randperm(r, generator=g).to(torch.int32).to(DEV)
+    sc = (torch.rand(r, generator=g) + 0.5).to(DEV)
+    offs = torch.tensor([0] + counts).cumsum(0).to(torch.int32).to(DEV)
+    xs = x[src.long()].double() * sc.double()[:, None]
+    ref = torch.empty(r, n, dtype=torch.float64, device=DEV)
+    for i in range(e):
+        a, b = int(offs[i]), int(offs[i + 1])
+        y = xs[a:b] @ w[i].double().t()
+        if gated:
+            gt, up = y[:, :n].clamp(max=2.0), y[:, n:].clamp(-2.0, 2.0)
+            y = gt * torch.sigmoid(1.7 * gt) * (up + 1.0)
+        ref[dst[a:b].long()] = y
+    for add in (False, True):
+        out = torch.full((r, n + 4), 0.5, device=DEV)[:, :n]
+        hy.ext().linear_rows(x, src, w if e > 1 else w[0], out, dst, offs if e > 1 else None, None, r, act, 2.0, 1.7, sc, None,
+                             0.0, 0, add)
+        got = out.double() - (0.5 if add else 0.0)
+        assert float((got - ref).abs().max() / ref.abs().max()) < 5e-6
+
+
+def test_fp32_split_products_keep_infinities():
+    """An infinity or NaN among the operands: what plain fp32 products give."""
+    from jax_llama_amd import ops
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(70, 256, generator=g), torch.randn(132, 256, generator=g)
+    x[3, 5], x[40, 7], x[50, 1], x[51, 1], w[100, 9] = float("inf"), float("nan"), 3.3e38, 1e-41, float("-inf")
+    want = x @ w.t()
+    for got in (ops.linear_f32(x.to(DEV), w.to(DEV)).cpu(), hy.linear(x.to(DEV), w.to(DEV)).cpu()):
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want))
+        ok = torch.isfinite(want)
+        assert float(((got - want)[ok].abs() / want[ok].abs().clamp_min(1e-3)).max()) < 1e-2  # (3.3e38 rows cancel)
+        fine = ok & (want.abs() < 1e3)
+        assert float((got - want)[fine].abs().max()) < 1e-3
