@@ -15,6 +15,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..ops import hybrid as hy
+from ..ops.slots import step_slot
 from ..parallel.comm import NO_COMM
 from .kv_cache import HybridCache
 from .mixers import StepContext
@@ -127,6 +128,7 @@ class LayerListLM:
         b, s = ids.shape
         d = self.config.hidden_size
         idf = ids.reshape(-1).to(self.device, torch.int32).contiguous()
+        slot0 = step_slot(slot0, self.device)
         ctx = StepContext(idf, positions.reshape(-1).to(self.device, torch.int32).contiguous(), b, s, cache, slot0)
         hidden = []
         if self.streams:
@@ -213,7 +215,7 @@ class LayerListLM:
         if slot0 + s > cache.max_length:
             raise ValueError(f"cache overflow: {slot0}+{s} > {cache.max_length}")
         if position_ids is None:
-            position_ids = torch.arange(slot0, slot0 + s, dtype=torch.int32).expand(b, s)
+            position_ids = torch.arange(slot0, slot0 + s, dtype=torch.int32, device=self.device).expand(b, s)
         pos = torch.as_tensor(position_ids).to(self.device, torch.int32).reshape(b, s).contiguous()
         logits, _, hidden, _ = self.forward_tokens(ids, pos, cache, slot0, logits_mode="all",
                                                    collect_hidden=output_hidden_states)

@@ -30,6 +30,7 @@ import torch
 from .. import ops
 from ..config import LLaMAConfig
 from ..ops import reference as ref
+from ..ops.slots import step_slot
 from ..parallel.comm import NO_COMM, TPComm
 from ..parallel.partition import shard_tree
 from .kv_cache import KVCache
@@ -363,6 +364,7 @@ class LLaMAForCausalLM:
                         collect_attn):
         b, s = ids.shape
         d = self.config.hidden_size
+        slot0 = step_slot(slot0, self.device)
         # residual stream: fp32 h plus its bf16 mirror hb (the A operand of every projection
         # that follows a norm; RMSNorm statistics are taken from these bf16 values)
         hb = torch.empty(b * s, d, dtype=BF16, device=self.device)
@@ -400,7 +402,7 @@ class LLaMAForCausalLM:
         if position_ids is None:
             if past_key_values is not None:
                 raise ValueError("Make sure to provide `position_ids` when passing `past_key_values`.")
-            position_ids = torch.arange(s, dtype=torch.int32).expand(b, s)
+            position_ids = torch.arange(s, dtype=torch.int32, device=self.device).expand(b, s)
         pos = _t(position_ids).to(self.device, torch.int32).reshape(b, s).contiguous()
         if past_key_values is None:
             cache = KVCache(self.config.num_hidden_layers, b, self.n_kv_heads, s, self.head_dim, self.device)
@@ -411,8 +413,8 @@ class LLaMAForCausalLM:
             if slot0 + s > cache.max_length:
                 raise ValueError(f"cache overflow: {slot0}+{s} > {cache.max_length}")
         t_valid = slot0 + s
-        if attention_mask is None:
-            mask = torch.ones(b, t_valid, dtype=torch.int32)
+        if attention_mask is None:  # (every key of every row: nothing to look through on the host)
+            return ids, pos, cache, slot0, torch.zeros(b, dtype=torch.int32, device=self.device), None
         else:
             mask = _t(attention_mask).to("cpu").to(torch.int32)
             if mask.shape[1] >= t_valid:

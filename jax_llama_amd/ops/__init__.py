@@ -19,6 +19,7 @@ from . import autotune
 from . import reference as ref
 from ._ext import available as ext_available  # noqa: F401
 from ._ext import ext
+from .slots import slot_tensor as _slot_tensor
 
 BF16 = torch.bfloat16
 
@@ -647,17 +648,6 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, slo
     else:
         e.attn_prefill(q, k_cache, v_cache, slot_t, kv_start, key_mask, out)
     return out
-
-
-_SLOT_CACHE = {}
-
-
-def _slot_tensor(slot0, device):
-    if torch.is_tensor(slot0):
-        return slot0
-    # Host int -> small device tensor (not graph-capturable; the engine passes tensors).
-    t = torch.tensor([int(slot0)], dtype=torch.int32, device=device)
-    return t
 
 
 # ----------------------------------------------------------------------------------

@@ -53,6 +53,8 @@ from typing import Optional, Tuple
 
 import torch
 
+from .slots import slot_tensor as _slot_tensor
+
 BF16 = torch.bfloat16
 F32 = torch.float32
 
@@ -97,12 +99,6 @@ def so_path() -> Optional[str]:
 
 def _gpu(t: torch.Tensor) -> bool:
     return t.device.type == "cuda"
-
-
-def _slot_tensor(slot, device) -> torch.Tensor:
-    if torch.is_tensor(slot):
-        return slot
-    return torch.tensor([int(slot)], dtype=torch.int32, device=device)
 
 
 def _slot_int(slot) -> int:

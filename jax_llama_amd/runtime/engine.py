@@ -193,22 +193,23 @@ class DecodeEngine:
         ids = input_ids.to(dev, torch.int32)
         b, s = ids.shape
         assert b == self.b and s < self.max_length
-        if attention_mask is None:
-            mask = torch.ones(b, s, dtype=torch.int32)
+        if attention_mask is None:  # every key of every row: positions on the device, nothing to look through on the host
+            pos_dev = torch.arange(s, dtype=torch.int32, device=dev).expand(b, s).contiguous()
+            self.kv_start.zero_()
+            self.key_mask = None
         else:
             mask = attention_mask.to("cpu", torch.int32)
-        positions = (mask.cumsum(-1) - 1).to(torch.int32)
-        ext_mask = torch.ones(b, self.max_length, dtype=torch.int32)
-        ext_mask[:, :s] = mask
-        from ..models.llama import mask_to_kv_start
-        kv_start, key_mask = mask_to_kv_start(ext_mask, dev)
-        self.kv_start.copy_(kv_start)
-        self.key_mask = key_mask
+            pos_dev = (mask.cumsum(-1) - 1).to(torch.int32).to(dev)
+            ext_mask = torch.ones(b, self.max_length, dtype=torch.int32)
+            ext_mask[:, :s] = mask
+            from ..models.llama import mask_to_kv_start
+            kv_start, key_mask = mask_to_kv_start(ext_mask, dev)
+            self.kv_start.copy_(kv_start)
+            self.key_mask = key_mask
         self.cache.reset()
         self.sequences.fill_(self.gc.pad_token_id)
         self.sequences[:, :s] = ids
         self.finished.zero_()
-        pos_dev = positions.to(dev)
         logits = self._prefill_rows(ids, pos_dev)
         self.cache.advance(s)
         # state for the loop body: cur_len = S (also the sampler's Philox step), token/pos of the

@@ -207,3 +207,14 @@ def test_llama2_7b_config_two_layer_greedy_plumbing():
             top2 = step.topk(2).values
             if float(top2[0] - top2[1]) > 1e-3 * float(step.abs().max()):  # skip near-ties (bf16 weights)
                 assert int(step.argmax()) == int(seq[0, n0 + j]), (row, j)
+
+
+def test_host_slot_is_an_int_with_one_device_copy():
+    """A step's host-known slot: an int to whoever computes with it, one device copy for every op of the step."""
+    from jax_llama_amd.ops.slots import HostSlot, slot_tensor, step_slot
+    t = torch.tensor([5], dtype=torch.int32)
+    assert step_slot(t, "cpu") is t and step_slot(7, "cpu") == 7
+    s = HostSlot(9, "cpu")
+    assert s == 9 and s + 1 == 10 and not torch.is_tensor(s)
+    assert slot_tensor(s, "cpu") is slot_tensor(s, "cpu") and int(slot_tensor(s, "cpu")) == 9
+    assert int(slot_tensor(s - 4, "cpu")) == 5 and slot_tensor(t, "cpu") is t
