@@ -872,6 +872,63 @@ void lin_scan(int64_t mode, Tensor q, Tensor k, Tensor v, Tensor decay, OptT wri
   rc(jla::hy_lin_scan(p, stream()), "lin_scan");
 }
 
+bool rec_step_takes(int64_t dim, int64_t vdim) {
+  return dim <= 0x7fffffff && vdim <= 0x7fffffff && jla::hy_rec_step_takes((int)dim, (int)vdim);
+}
+
+// gates: mode 0: (projection [B, .], column of the input gates, column of the forget gates, biases, running maximum [B, H])
+void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT u, OptT beta, OptT decay, OptT proj, int64_t col_i,
+              int64_t col_f, OptT gate_bias, double cap, OptT mstate, double q_scale, Tensor state, OptT gate, Tensor w,
+              double eps, int64_t gate_act, double gain, Tensor out) {
+  jla::RecStep p{};
+  check(mode >= 0 && mode <= 3, "rec_step: mode");
+  check(q.dim() == 3 && v.dim() == 3, "rec_step: q is [B, H (mode 3: G), dim], v is [B, H, vdim]");
+  const int64_t B = v.size(0), H = v.size(1), dim = q.size(2), vdim = v.size(2), G = q.size(1);
+  check(rec_step_takes(dim, vdim), "rec_step: head sizes");
+  check(mode == 3 ? (G >= 1 && H % G == 0) : G == H, "rec_step: heads");
+  p.mode = mode; p.B = B; p.H = H; p.G = G; p.dim = dim; p.vdim = vdim;
+  p.q = heads3d(q, "q", B, G, dim, &p.ldq);
+  check(k.has_value() == (mode != 2), "rec_step: k");
+  if (k.has_value()) p.k = heads3d(*k, "k", B, G, dim, &p.ldk);
+  p.v = heads3d(v, "v", B, H, vdim, &p.ldv);
+  if (mode == 0) {
+    check(proj.has_value() && gate_bias.has_value() && mstate.has_value() && cap > 0, "rec_step: gates");
+    check(proj->dim() == 2 && proj->size(0) == B && col_i >= 0 && col_f >= 0 && col_i + H <= proj->size(1) &&
+              col_f + H <= proj->size(1), "rec_step: gate columns");
+    const float* base = rows2d(*proj, "proj", proj->size(1), &p.ldgate);
+    p.gate_i = base + col_i;
+    p.gate_f = base + col_f;
+    check(gate_bias->numel() == 2 * H && mstate->numel() == B * H, "rec_step: gate biases, running maximum");
+    p.gate_bias = f32(*gate_bias, "gate_bias");
+    p.mstate = f32w(*mstate, "mstate");
+    p.cap = cap;
+  } else if (mode == 3) {
+    check(beta.has_value() && decay.has_value() && beta->numel() == B * H && decay->numel() == B * H, "rec_step: beta, decay");
+    p.beta = f32(*beta, "beta");
+    p.decay = f32(*decay, "decay");
+  } else {
+    check(pre.has_value() && w0.has_value() && u.has_value() && w0->numel() == H * dim && u->numel() == H * dim,
+          "rec_step: pre, w0, u");
+    p.pre = heads3d(*pre, "pre", B, H, dim, &p.ldpre);
+    p.w0 = f32(*w0, "w0");
+    p.u = f32(*u, "u");
+  }
+  p.q_scale = q_scale;
+  check(state.numel() == B * H * dim * (mode == 0 ? vdim + 1 : vdim), "rec_step: state");
+  p.state = f32w(state, "state");
+  check(gate_act >= 0 && gate_act <= 2 && gate.has_value() == (gate_act != 2), "rec_step: gate");
+  if (gate.has_value()) {
+    check(gate->dim() == 2 && gate->size(0) == B, "rec_step: gate rows");
+    p.gate = rows2d(*gate, "gate", H * vdim, &p.ldg);
+  }
+  check(w.numel() == vdim || w.numel() == H * vdim, "rec_step: norm gain");
+  p.w = f32(w, "w");
+  p.w_heads = w.numel() != vdim || H == 1;
+  p.eps = eps; p.gate_act = gate_act; p.gain = gain;
+  p.out = slice2d(out, "out", B, H * vdim, &p.ldo);
+  rc(jla::hy_rec_step(p, stream()), "rec_step");
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -925,6 +982,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
   m.def("delta_scan", &delta_scan);
+  m.def("rec_step_takes", &rec_step_takes);
+  m.def("rec_step", &rec_step, py::arg("mode"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("pre") = py::none(),
+        py::arg("w0") = py::none(), py::arg("u") = py::none(), py::arg("beta") = py::none(), py::arg("decay") = py::none(),
+        py::arg("proj") = py::none(), py::arg("col_i") = 0, py::arg("col_f") = 0, py::arg("gate_bias") = py::none(),
+        py::arg("cap") = 1.0, py::arg("mstate") = py::none(), py::arg("q_scale") = 1.0, py::arg("state"), py::arg("gate"),
+        py::arg("w"), py::arg("eps"), py::arg("gate_act"), py::arg("gain"), py::arg("out"));
   m.def("gated_rmsnorm", &gated_rmsnorm, py::arg("o"), py::arg("gate"), py::arg("w"), py::arg("eps"), py::arg("out"),
         py::arg("H"), py::arg("vdim"), py::arg("gate_act") = 0, py::arg("denom_floor") = py::none(),
         py::arg("gain") = 1.0);

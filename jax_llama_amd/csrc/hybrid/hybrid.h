@@ -450,4 +450,40 @@ struct LinScan {
 };
 int hy_lin_scan(const LinScan& p, hipStream_t s);
 
+// One token of a matrix-state recurrence with its gates and its gated head norm (rec_step.hip). mode 0: exponential gates
+// (state [B, H, dim, vdim + 1], mstate advanced), 1: time mix, 2: running memory, 3: delta rule. Row b, head h at x + b * ldx +
+// h * dim (or vdim; mode 3: q and k by key head, h / (H / G)). out[b * ldo + h * vdim + j] as hy_gated_rmsnorm gives it.
+struct RecStep {
+  int mode, B, H, G, dim, vdim;
+  const float* q;
+  int ldq;
+  const float* k;
+  int ldk;
+  const float* v;
+  int ldv;
+  const float* pre;  // modes 1, 2: gate pre-activations
+  int ldpre;
+  const float* w0;   // modes 1, 2: [H, dim]
+  const float* u;
+  const float* beta; // mode 3: [B, H]
+  const float* decay;
+  const float* gate_i;  // mode 0: pre-activations of row b, head h at gate_i[b * ldgate + h]
+  const float* gate_f;
+  int ldgate;
+  const float* gate_bias;  // [2 H]
+  float cap;
+  float* mstate;  // [B, H]
+  float q_scale;
+  float* state;
+  const float* gate;  // gate_act 0, 1
+  int ldg;
+  const float* w;
+  int w_heads, gate_act;
+  float eps, gain;
+  float* out;
+  int ldo;
+};
+bool hy_rec_step_takes(int dim, int vdim);
+int hy_rec_step(const RecStep& p, hipStream_t s);
+
 }  // namespace jla

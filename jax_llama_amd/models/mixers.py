@@ -123,10 +123,9 @@ class GatedDeltaMixer:
         state, tail = ctx.cache.recurrent(self.i)
         q, k, v, beta, decay = hy.delta_prep(proj, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w,
                                              tail, self.a_log, self.dt_bias)
-        o = hy.delta_scan(q, k, v, beta, decay, state, ctx.b, ctx.s)
         c = 2 * sp.kv_heads * sp.dim + sp.heads * sp.vdim
         gate = proj[:, c:c + sp.heads * sp.vdim]
-        return hy.linear(hy.gated_rmsnorm(o, gate, self.norm_w, self.eps), self.w_o)
+        return hy.linear(hy.delta_memory(q, k, v, beta, decay, state, ctx.b, ctx.s, gate, self.norm_w, self.eps), self.w_o)
 
 
 class TableMoE:
@@ -351,17 +350,10 @@ class MatrixLSTM:
         self.width = heads * vdim
 
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
-        nh, dim, vdim, m = self.heads, self.dim, self.vdim, ctx.b * ctx.s
         proj = hy.linear(h, self.w_in)
         state, mrun = ctx.cache.recurrent(self.i)
-        qk, vv = nh * dim, nh * vdim
-        keep, write, floor = hy.mlstm_prep(proj, 2 * qk + 2 * vv, 2 * qk + 2 * vv + nh, self.gate_bias, self.cap, mrun,
-                                           ctx.b, ctx.s, nh)
-        o = hy.mlstm_scan(proj[:, :qk].unflatten(1, (nh, dim)), proj[:, qk:2 * qk].unflatten(1, (nh, dim)),
-                          proj[:, 2 * qk:2 * qk + vv].unflatten(1, (nh, vdim)), keep, write, state, ctx.b, ctx.s,
-                          q_scale=dim ** -0.5)
-        return hy.gated_rmsnorm(o, proj[:, 2 * qk + vv:2 * qk + 2 * vv], self.norm_w, self.eps, hy.GATE_SIGMOID,
-                                denom_floor=floor, gain=gain, out=out)
+        return hy.mlstm_memory(proj, self.heads, self.dim, self.vdim, self.gate_bias, self.cap, mrun, state, ctx.b, ctx.s,
+                               self.norm_w, self.eps, gain, out)
 
     def __call__(self, h, ctx: StepContext) -> torch.Tensor:
         return hy.linear(self.features(h, ctx), self.w_o)
@@ -397,9 +389,8 @@ class TimeMix:
             r, k, v, g = (hy.linear(mixes[j], self.w_each[j]) for j in range(4))
         wpre = hy.linear(hy.linear_softcap(mixes[4], self.w_d1, 1.0), self.w_d2)
         hd = (nh, dim)
-        o = hy.timemix_scan(r.unflatten(1, hd), k.unflatten(1, hd), v.unflatten(1, hd), wpre.unflatten(1, hd), self.w0,
-                            self.u, state, ctx.b, ctx.s)
-        return hy.gated_rmsnorm(o, g, self.norm_w, self.eps, hy.GATE_SILU, gain=gain, out=out)
+        return hy.timemix_memory(r.unflatten(1, hd), k.unflatten(1, hd), v.unflatten(1, hd), wpre.unflatten(1, hd), self.w0,
+                                 self.u, state, ctx.b, ctx.s, g, self.norm_w, self.eps, gain, out)
 
     def __call__(self, h, ctx: StepContext) -> torch.Tensor:
         return hy.linear(self.features(h, ctx), self.w_o)
@@ -702,9 +693,9 @@ class GatedRunningMixer:
         sp = self.spec
         qk, hd = sp.heads * sp.dim, (sp.heads, sp.dim)
         state, _ = ctx.cache.recurrent(self.i)
-        o = hy.gated_running_scan(proj[:, :qk].unflatten(1, hd), proj[:, 2 * qk:2 * qk + self.width].unflatten(
-            1, (sp.heads, sp.vdim)), proj[:, qk:2 * qk].unflatten(1, hd), self.f_bias, self.room, state, ctx.b, ctx.s)
-        return hy.gated_rmsnorm(o, None, self.norm_w, self.eps, hy.GATE_NONE, out=out)
+        return hy.running_memory(proj[:, :qk].unflatten(1, hd), proj[:, 2 * qk:2 * qk + self.width].unflatten(
+            1, (sp.heads, sp.vdim)), proj[:, qk:2 * qk].unflatten(1, hd), self.f_bias, self.room, state, ctx.b, ctx.s,
+            self.norm_w, self.eps, out)
 
 
 class GatedMoE:

@@ -1147,6 +1147,28 @@ def gated_rmsnorm(o: torch.Tensor, gate: Optional[torch.Tensor], w: torch.Tensor
     return out
 
 
+def _step_out(x: torch.Tensor, width: int, dim: int, vdim: int, s: int, out: Optional[torch.Tensor]):
+    """Where a recurrence's one-token kernel (csrc/hybrid/rec_step.hip: gates, state and gated head norm in one launch) writes,
+    or None where the separate ops run: more tokens, the CPU, head sizes it does not take, a bf16 buffer, more rows than a
+    grid's second axis."""
+    if s != 1 or not _gpu(x) or x.shape[0] > 65535 or (out is not None and out.dtype != F32) or \
+            not ext().rec_step_takes(dim, vdim):
+        return None
+    return out if out is not None else torch.empty(x.shape[0], width, dtype=F32, device=x.device)
+
+
+def delta_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor,
+                 state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """``gated_rmsnorm(delta_scan(...), gate, w, eps)``."""
+    h, vdim = v.shape[1], v.shape[2]
+    out = _step_out(q, h * vdim, q.shape[2], vdim, s, None)
+    if out is None:
+        return gated_rmsnorm(delta_scan(q, k, v, beta, decay, state, b, s), gate, w, eps)
+    ext().rec_step(3, q, k, v, beta=beta, decay=decay, state=state, gate=gate, w=w, eps=float(eps), gate_act=GATE_SILU, gain=1.0,
+                   out=out)
+    return out
+
+
 # ------------------------------------------------------------------------------------------------ rotary positions
 def rotary_freqs(base: float, dims: int, device) -> torch.Tensor:
     """float64 ``[dims / 2]``: ``base^(-2 i / dims)``, the turn per position of pair ``i``. Angles are formed in 64-bit
@@ -1445,3 +1467,49 @@ def gated_running_scan(q: torch.Tensor, v: torch.Tensor, fpre: torch.Tensor, f_b
     ext().lin_scan(2, q, fpre, v, fpre, None, f_bias.reshape(h, dim), room.reshape(h, dim), state, o, b, s, 1.0, nseg,
                    seg_len, ws)
     return o
+
+
+def mlstm_memory(proj: torch.Tensor, heads: int, dim: int, vdim: int, gate_bias: torch.Tensor, cap: float, mstate: torch.Tensor,
+                 state: torch.Tensor, b: int, s: int, w: torch.Tensor, eps: float, gain: float = 1.0,
+                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The exponential-gate memory of a fused projection ``proj [B*S, q | k | v | gate | input gates | forget gates]``:
+    ``mlstm_prep``, ``mlstm_scan`` (queries times ``dim^-1/2``) and ``gated_rmsnorm`` with the sigmoid of the gate columns."""
+    qk, vv = heads * dim, heads * vdim
+    q, k = (proj[:, i * qk:(i + 1) * qk].unflatten(1, (heads, dim)) for i in (0, 1))
+    v, gate = proj[:, 2 * qk:2 * qk + vv].unflatten(1, (heads, vdim)), proj[:, 2 * qk + vv:2 * qk + 2 * vv]
+    col = 2 * qk + 2 * vv
+    to = _step_out(proj, vv, dim, vdim, s, out)
+    if to is not None:
+        ext().rec_step(0, q, k, v, proj=proj, col_i=col, col_f=col + heads, gate_bias=gate_bias, cap=float(cap), mstate=mstate,
+                       q_scale=dim ** -0.5, state=state, gate=gate, w=w, eps=float(eps), gate_act=GATE_SIGMOID, gain=float(gain),
+                       out=to)
+        return to
+    keep, write, floor = mlstm_prep(proj, col, col + heads, gate_bias, cap, mstate, b, s, heads)
+    o = mlstm_scan(q, k, v, keep, write, state, b, s, q_scale=dim ** -0.5)
+    return gated_rmsnorm(o, gate, w, eps, GATE_SIGMOID, denom_floor=floor, gain=gain, out=out)
+
+
+def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre: torch.Tensor, w0: torch.Tensor, u: torch.Tensor,
+                   state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float, gain: float = 1.0,
+                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``gated_rmsnorm(timemix_scan(...), gate, w, eps, GATE_SILU, gain=gain, out=out)``."""
+    h, dim, vdim = r.shape[1], r.shape[2], v.shape[2]
+    to = _step_out(r, h * vdim, dim, vdim, s, out)
+    if to is None:
+        return gated_rmsnorm(timemix_scan(r, k, v, wpre, w0, u, state, b, s), gate, w, eps, GATE_SILU, gain=gain, out=out)
+    ext().rec_step(1, r, k, v, pre=wpre, w0=w0.reshape(h, dim), u=u.reshape(h, dim), state=state, gate=gate, w=w, eps=float(eps),
+                   gate_act=GATE_SILU, gain=float(gain), out=to)
+    return to
+
+
+def running_memory(q: torch.Tensor, v: torch.Tensor, fpre: torch.Tensor, f_bias: torch.Tensor, room: torch.Tensor,
+                   state: torch.Tensor, b: int, s: int, w: torch.Tensor, eps: float,
+                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``gated_rmsnorm(gated_running_scan(...), None, w, eps, GATE_NONE, out=out)``."""
+    h, dim, vdim = q.shape[1], q.shape[2], v.shape[2]
+    to = _step_out(q, h * vdim, dim, vdim, s, out)
+    if to is None:
+        return gated_rmsnorm(gated_running_scan(q, v, fpre, f_bias, room, state, b, s), None, w, eps, GATE_NONE, out=out)
+    ext().rec_step(2, q, None, v, pre=fpre, w0=f_bias.reshape(h, dim), u=room.reshape(h, dim), state=state, gate=None, w=w,
+                   eps=float(eps), gate_act=GATE_NONE, gain=1.0, out=to)
+    return to

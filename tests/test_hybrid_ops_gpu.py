@@ -560,3 +560,42 @@ def test_fp32_split_products_keep_infinities():
         assert float(((got - want)[ok].abs() / want[ok].abs().clamp_min(1e-3)).max()) < 1e-2  # (3.3e38 rows cancel)
         fine = ok & (want.abs() < 1e3)
         assert float((got - want)[fine].abs().max()) < 1e-3
+
+
+@pytest.mark.parametrize("kind", ["mlstm", "timemix", "running", "delta"])
+@pytest.mark.parametrize("b,h,dim,vdim", [(1, 4, 128, 128), (3, 2, 64, 64), (2, 6, 40, 24), (1, 2, 256, 64), (5, 2, 33, 130),
+                                          (2, 1, 64, 256), (1, 2, 1, 1), (2, 2, 128, 256), (1, 1, 130, 192)])
+def test_one_token_recurrence(kind, b, h, dim, vdim):
+    """Gates, state and gated norm in one launch (the last two sizes: the separate kernels) against the CPU ops; the norm
+    divides by the head's own size, so the error is a few fp32 roundings of sums of ``dim`` terms."""
+    ncols = vdim + 1 if kind == "mlstm" else vdim
+    state = _rand(b, h, dim, ncols, std=0.3)
+    w = torch.rand(vdim if kind == "delta" else h * vdim) + 0.5
+    gate = _rand(b, h * vdim + 3)[:, :h * vdim]  # strided rows
+    mstate, bias = _rand(b, h), _rand(2 * h)
+    proj = _rand(b, 2 * h * dim + 2 * h * vdim + 2 * h)
+    g = h // 2 if kind == "delta" and h > 1 else h
+    q, k = _rand(b, 2, g, dim, std=dim ** -0.5).unbind(1)
+    v, pre = _rand(b, h, vdim), _rand(b, h, dim)
+    w0, u = _rand(h * dim), torch.rand(h * dim)
+    beta, decay = torch.rand(b, h), torch.rand(b, h)
+    res = []
+    for dev in ("cpu", DEV):
+        st, ms = state.clone().to(dev), mstate.clone().to(dev)
+        a = lambda *ts: [t.to(dev) for t in ts]
+        big = torch.zeros(b, h * vdim + 5, device=dev)
+        out = big[:, 5:]
+        gd = torch.empty(b, h * vdim + 3, device=dev)[:, :h * vdim].copy_(gate)
+        if kind == "mlstm":
+            y = hy.mlstm_memory(proj.to(dev), h, dim, vdim, bias.to(dev), 15.0, ms, st, b, 1, w.to(dev), 1e-6, 0.5, out)
+        elif kind == "timemix":
+            y = hy.timemix_memory(*a(q, k, v, pre, w0, u), st, b, 1, gd, w.to(dev), 1e-6, 0.5, out)
+        elif kind == "running":
+            y = hy.running_memory(*a(q, v, pre, w0, u), st, b, 1, w.to(dev), 1e-6, out)
+        else:
+            y = hy.delta_memory(*a(q, k, v, beta, decay), st, b, 1, gd, w.to(dev), 1e-6)
+        if kind != "delta":
+            assert float(big[:, :5].abs().max()) == 0.0
+        res.append((y, st, ms))
+    for r, x, name in zip(*res, ("out", "state", "running maximum")):
+        _close(x, r, 2e-5, name)
