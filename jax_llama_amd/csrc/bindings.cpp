@@ -548,7 +548,11 @@ void argmax(Tensor logits, Tensor idx, Tensor val) {
   check(idx.scalar_type() == torch::kInt32 && val.scalar_type() == torch::kFloat32 &&
             idx.numel() == logits.size(0) && val.numel() == logits.size(0),
         "argmax outputs");
-  rc(jla::argmax(ptr<float>(logits), logits.size(0), logits.size(1), ptr<int32_t>(idx), ptr<float>(val), stream()),
+  const int64_t n = jla::argmax_workspace(logits.size(0), logits.size(1));
+  Tensor ws;  // (from the allocator of the stream that uses it)
+  if (n > 0) ws = torch::empty({n}, logits.options());
+  rc(jla::argmax(ptr<float>(logits), logits.size(0), logits.size(1), ptr<int32_t>(idx), ptr<float>(val),
+                 n > 0 ? ptr<float>(ws) : nullptr, stream()),
      "argmax");
 }
 

@@ -139,7 +139,9 @@ int attn_prefill(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, const int3
                  const uint8_t* key_mask, int mask_len, bf16_t* out, int B, int S, int H, int Hkv, int Dh, int T,
                  hipStream_t s);
 
-int argmax(const float* logits, int B, int V, int32_t* idx, float* val, hipStream_t s);
+// ws: argmax_workspace() floats, 8-byte aligned (0: none needed)
+long long argmax_workspace(int B, int V);
+int argmax(const float* logits, int B, int V, int32_t* idx, float* val, float* ws, hipStream_t s);
 // top-k / top-p sampler (topk_sample.hip): cv/ci [B, topk_chunks(V) * K] candidates
 int topk_chunks(int V);
 int topk_chunk(const float* logits, int B, int V, int K, int idx_offset, float* cv, int32_t* ci, hipStream_t s);

@@ -363,3 +363,23 @@ def test_gemm4_256x128_tiles(m, n, k, ks, tile):
     if ks == 1:
         _close(t10[3], ref.linear(x, w, 1e-5, torch.float32), 1e-2, 2e-3)
         _close(t10[5], ref.linear_swiglu(x, gu, 1e-5), 3e-2, 3e-2)
+
+
+@pytest.mark.parametrize("b,v", [(1, 1), (1, 2047), (3, 4096), (1, 32000), (2, 32001), (7, 128256), (200, 8190), (1024, 512)])
+def test_argmax_rows(b, v):
+    """Rows cut over several workgroups: index and value bit for bit, the first of equal maxima (set on both sides of the cuts),
+    a NaN never chosen, a row of -inf and an unaligned base."""
+    from jax_llama_amd import ops
+    g = torch.Generator().manual_seed(b * v)
+    flat = torch.randn(b * v + 1, generator=g)
+    for off in (0, 1):
+        x = flat[off:off + b * v].reshape(b, v).clone()
+        x[0, [v // 3, v // 2, v - 1]] = 9.0
+        if b > 2:
+            x[1] = float("-inf")
+            x[2, ::3] = float("nan")
+        want = torch.nan_to_num(x, nan=float("-inf"), neginf=float("-inf"), posinf=float("inf"))
+        wv, wi = want.max(1).values, (want == want.max(1, keepdim=True).values).int().argmax(1)
+        dev = torch.empty(b * v + 1, device="cuda")[off:off + b * v].view(b, v).copy_(x)
+        idx, val = ops.argmax(dev)
+        assert torch.equal(idx.cpu().long(), wi) and torch.equal(val.cpu(), wv), (off, b, v)
