@@ -75,9 +75,9 @@ void embed_rows(Tensor ids, Tensor table, int64_t col0, Tensor out, double scale
      "embed_rows");
 }
 
-jla::RowLinear row_linear(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT offs, OptT row_expert, int64_t R,
+jla::RowLinear row_linear_any(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT offs, OptT row_expert, int64_t R,
                           int64_t act, double act_limit, double act_alpha, OptT a_scale, OptT a_norm_w, double a_norm_eps,
-                          int64_t even_rows, bool add_out) {
+                          int64_t even_rows, bool add_out, bool tabled) {
   jla::RowLinear p{};
   p.even_rows = even_rows;
   p.add_out = add_out;
@@ -114,8 +114,15 @@ jla::RowLinear row_linear(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_i
     p.a_norm_w = f32(*a_norm_w, "a_norm_w");
     p.a_norm_eps = a_norm_eps;
   }
-  check(p.E == 1 || p.offs || p.row_expert, "linear_rows: stacked experts need offs or row_expert");
+  check(p.E == 1 || p.offs || p.row_expert || tabled, "linear_rows: stacked experts need offs or row_expert");
   return p;
+}
+
+jla::RowLinear row_linear(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT offs, OptT row_expert, int64_t R,
+                          int64_t act, double act_limit, double act_alpha, OptT a_scale, OptT a_norm_w, double a_norm_eps,
+                          int64_t even_rows, bool add_out) {
+  return row_linear_any(a, a_idx, w, out, dst_idx, offs, row_expert, R, act, act_limit, act_alpha, a_scale, a_norm_w, a_norm_eps,
+                        even_rows, add_out, false);
 }
 
 // scratch of a call, from the allocator of the stream that uses it
@@ -131,6 +138,70 @@ void linear_rows(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT 
                                       a_norm_w, a_norm_eps, even_rows, add_out);
   const Tensor ws = row_scratch(jla::hy_linear_rows_floats(p), out);
   rc(jla::hy_linear_rows(p, scratch_ptr(ws), stream()), "linear_rows");
+}
+
+// A pending residual add (res_y .. res_out) onto the activations of p: [rows, K], rows of y res_nsum per activation row
+void set_residual(jla::RowLinear& p, const Tensor& a, const OptT& y, int64_t nsum, double ysc, const OptT& w, double eps,
+                  const OptT& x_out) {
+  if (!y.has_value()) return;
+  check(w.has_value() && x_out.has_value() && w->numel() == 1 && nsum >= 1, "residual: one gain, nsum >= 1");
+  check(a.is_contiguous() && y->numel() == a.numel() * nsum && x_out->sizes() == a.sizes() &&
+            x_out->data_ptr() != a.data_ptr(), "residual: y is [rows * nsum, K], x_out another [rows, K]");
+  p.res_y = f32(*y, "y");
+  p.res_nsum = nsum;
+  p.res_ysc = ysc;
+  p.res_w = f32(*w, "w");
+  p.res_eps = eps;
+  p.res_out = f32w(*x_out, "x_out");
+}
+
+// out = f(a' @ w^T) for a few rows in one launch: a' = a + rms_norm(ysc * sum of nsum rows of y) * res_w with y (written to x_out
+// too), f = gelu_tanh * table[ids, col0 ..] with ids. False: not a call of that kernel, nothing was launched.
+bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc, OptT res_w, double eps, OptT x_out, OptT ids,
+                OptT table, int64_t col0) {
+  jla::RowLinear p = row_linear(a, c10::nullopt, w, out, c10::nullopt, c10::nullopt, c10::nullopt, a.size(0), 0, 0.0, 1.0,
+                                c10::nullopt, c10::nullopt, 0.0, 0, false);
+  set_residual(p, a, y, nsum, ysc, res_w, eps, x_out);
+  if (ids.has_value()) {
+    check(table.has_value() && table->dim() == 2 && col0 >= 0 && col0 + p.N <= table->size(1), "rows_fused: table columns");
+    p.mul_ids = i32(*ids, "ids", p.R);
+    p.mul_bf16 = wtype(*table, "table");
+    p.mul_table = table->data_ptr();
+    p.mul_V = table->size(0); p.mul_ld = table->size(1); p.mul_col0 = col0;
+    check(p.mul_V >= 1, "rows_fused: empty table");
+  }
+  if (p.R == 0 || p.N < 1 || !(p.res_y ? jla::hy_rows_gemv_takes_residual(p) : jla::hy_rows_gemv_takes(p))) return false;
+  rc(jla::hy_rows_gemv(p, stream()), "rows_fused");
+  return true;
+}
+
+// Both products of a few tokens' table-chosen SwiGLU experts, the table read by the products: h [M * top, F], out [M * top, D] in
+// (token, choice) order. False: not a call of that kernel, nothing was launched.
+bool table_rows(Tensor a, Tensor ids, Tensor table, Tensor w_gu, Tensor w_down, Tensor h, Tensor out, OptT y, int64_t nsum,
+                double ysc, OptT res_w, double eps, OptT x_out) {
+  check(table.dim() == 2 && w_gu.dim() == 3 && w_down.dim() == 3 && w_gu.size(0) == w_down.size(0), "table_rows: shapes");
+  const int64_t M = a.size(0), top = table.size(1), R = M * top;
+  check(top >= 1 && R <= 0x7fffffff && h.size(0) == R && out.size(0) == R, "table_rows: rows");
+  if (R == 0 || R > jla::HY_GEMV_MAX_R) return false;
+  // (checked as M rows: linear row r of the first product reads activation row r / top)
+  jla::RowLinear p = row_linear_any(a, c10::nullopt, w_gu, h, c10::nullopt, c10::nullopt, c10::nullopt, M, jla::HY_ACT_SWIGLU, 0.0,
+                                1.0, c10::nullopt, c10::nullopt, 0.0, 0, false, true);
+  jla::RowLinear q = row_linear_any(h, c10::nullopt, w_down, out, c10::nullopt, c10::nullopt, c10::nullopt, R, 0, 0.0, 1.0,
+                                c10::nullopt, c10::nullopt, 0.0, 0, false, true);
+  p.R = R;
+  p.a_div = top;
+  for (jla::RowLinear* l : {&p, &q}) {
+    l->tab = i32(table, "table", table.numel());
+    l->tab_ids = i32(ids, "ids", M);
+    l->tab_V = table.size(0);
+    l->tab_top = top;
+  }
+  check(p.tab_V >= 1 && q.K == p.N, "table_rows: shapes");
+  set_residual(p, a, y, nsum, ysc, res_w, eps, x_out);
+  if (!(p.res_y ? jla::hy_rows_gemv_takes_residual(p) : jla::hy_rows_gemv_takes(p)) || !jla::hy_rows_gemv_takes(q)) return false;
+  rc(jla::hy_rows_gemv(p, stream()), "table_rows");
+  rc(jla::hy_rows_gemv(q, stream()), "table_rows");
+  return true;
 }
 
 // p and q from row_linear: the tensors they were made from must be alive
@@ -982,6 +1053,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
   m.def("delta_scan", &delta_scan);
+  m.def("rows_fused", &rows_fused, py::arg("a"), py::arg("w"), py::arg("out"), py::arg("y"), py::arg("nsum"), py::arg("ysc"),
+        py::arg("res_w"), py::arg("eps"), py::arg("x_out"), py::arg("ids") = py::none(), py::arg("table") = py::none(),
+        py::arg("col0") = 0);
+  m.def("table_rows", &table_rows);
   m.def("rec_step_takes", &rec_step_takes);
   m.def("rec_step", &rec_step, py::arg("mode"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("pre") = py::none(),
         py::arg("w0") = py::none(), py::arg("u") = py::none(), py::arg("beta") = py::none(), py::arg("decay") = py::none(),

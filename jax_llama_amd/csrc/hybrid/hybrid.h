@@ -53,6 +53,21 @@ struct RowLinear {
   float act_limit;       // HY_ACT_CLAMP_GLU
   float act_alpha;
   int add_out;           // out += act(...) instead of out = (fp32 outputs): a residual add in the epilogue
+  // the rest: hy_rows_gemv only
+  int a_div;             // > 1: activation row of linear row r is r / a_div
+  const int32_t* tab;    // optional: expert of linear row r = tab[tab_ids[r / tab_top] * tab_top + r % tab_top] ([tab_V, tab_top])
+  const int32_t* tab_ids;
+  int tab_V, tab_top;
+  const int32_t* mul_ids;  // optional: out = gelu_tanh(act(...)) * mul_table[mul_ids[r], mul_col0 + column]
+  const void* mul_table;
+  int mul_bf16, mul_V, mul_ld, mul_col0;
+  // optional: the activation row m is a[m] + rms_norm(res_ysc * sum of rows m res_nsum ... of res_y [., K]) * res_w (one
+  // number), also written to res_out [., K] (not a)
+  const float* res_y;
+  int res_nsum;
+  float res_ysc, res_eps;
+  const float* res_w;
+  float* res_out;
 };
 inline bool hy_act_gated(int act) {
   return act == HY_ACT_SWIGLU || act == HY_ACT_CLAMP_GLU || act == HY_ACT_GELU_GLU;
@@ -68,6 +83,7 @@ long long hy_rows_f32_floats(const RowLinear& p);  // scratch of its split-K for
 int hy_rows_f32(const RowLinear& p, float* ws, hipStream_t s);
 // the matrix-core form of a few bf16 rows (rows_gemv.hip)
 bool hy_rows_gemv_takes(const RowLinear& p);
+bool hy_rows_gemv_takes_residual(const RowLinear& p);
 int hy_rows_gemv(const RowLinear& p, hipStream_t s);
 int hy_rows_gemm(const RowLinear& p, hipStream_t s);
 // ws: hy_linear_rows_floats() floats of scratch, 16-byte aligned (0: none needed)

@@ -11,7 +11,9 @@
 // The waves of a workgroup deal the K steps among themselves, U in flight each, and sum their blocks through LDS.
 // Us before -> after, weights in no cache, 1 | 8 | 33 rows: K 2048 x N 5152 11.1 -> 7.7 | 27.4 -> 10.7 | 54 -> 21; 4096 x 10304 42.6 ->
 // 19.1 | 62.6 -> 26.6 | 108 -> 59; 2048 x 32000 49.6 -> 24.3 (5.4 TB/s) | 99 -> 29.4 | 67 -> 63; gated 2048 x 5632 17.2 -> 12.4 |
-// 44.8 -> 16.0 | 82 -> 34; both products of 2 of 8 experts (4096 x 7168) for 1 | 8 tokens 105 -> 68 | 403 -> 230.
+// 44.8 -> 16.0 | 82 -> 34; both products of 2 of 8 experts (4096 x 7168) for 1 | 8 tokens 105 -> 68 | 403 -> 230. With one output element
+// per thread (a third of the epilogue's code to fetch) and the arguments read at once, one row: 2048 x 2048 5.2 -> 4.7, 2048 x 5152
+// 7.9 -> 7.2, gated 5632 12.3 -> 11.5, 2048 x 32000 24.3 -> 22.7.
 #include "hy_util.h"
 #include "hybrid.h"
 #include "row_act.h"
@@ -23,8 +25,46 @@ JLA_DEV u32x4 rv_round8(const f32x4 a, const f32x4 b) {
   return pack8(f);
 }
 
+// The launch's arguments into registers at once: read where they are used, behind each other's branches, they are a chain of
+// scalar loads at the start of a kernel that lasts a few microseconds.
+JLA_DEV void rv_arguments(const RowLinear& p) {
+  asm volatile("" ::"s"(p.a), "s"(p.lda), "s"(p.a_idx), "s"(p.a_scale), "s"(p.w), "s"(p.w_stride), "s"(p.N), "s"(p.K),
+               "s"(p.out), "s"(p.ldo), "s"(p.dst_idx), "s"(p.offs), "s"(p.row_expert), "s"(p.R), "s"(p.a_div), "s"(p.tab));
+}
+
+// the expert of linear row r where every row has its own (0: one matrix); -1: none (an identity expert: nothing to compute)
+JLA_DEV int rv_expert(const RowLinear& p, int r) {
+  if (p.row_expert) {
+    const int e = p.row_expert[r];
+    return e < 0 || e >= p.E ? -1 : e;
+  }
+  if (p.tab) {  // choice r % top of token r / top, as the routing kernel reads the table
+    int id = p.tab_ids[r / p.tab_top];
+    id = id < 0 || id >= p.tab_V ? 0 : id;
+    const int e = p.tab[(size_t)id * p.tab_top + r % p.tab_top];
+    return e < 0 || e >= p.E ? 0 : e;
+  }
+  return 0;
+}
+
+// the table entry that the gated output column `col` of row r is multiplied by (gelu_gate_rows)
+JLA_DEV float rv_table(const RowLinear& p, int r, int col) {
+  int id = p.mul_ids[r];
+  id = id < 0 || id >= p.mul_V ? 0 : id;
+  const size_t at = (size_t)id * p.mul_ld + p.mul_col0 + col;
+  return p.mul_bf16 ? bf2f(reinterpret_cast<const bf16_t*>(p.mul_table)[at]) : reinterpret_cast<const float*>(p.mul_table)[at];
+}
+
+// output column col of linear row r from its accumulators
+JLA_DEV void rv_store(const RowLinear& p, int r, int col, float g, float v) {
+  float* dst = reinterpret_cast<float*>(p.out) + (size_t)(p.dst_idx ? p.dst_idx[r] : r) * p.ldo + col;
+  float val = lr_act(p, g, v);
+  if (p.mul_ids) val = hy_gelu_tanh(val) * rv_table(p, r, col);
+  *dst = p.add_out ? *dst + val : val;
+}
+
 // G: output columns of a tile, and rows of a pass per 16 MT / (16 / G); NT: tiles of a workgroup (gated: gate and up tiles
-// alternate); MT: 16-row tiles (G = 16); U: K steps in flight per wave. NORM (MT = 1): rows are RMS-normed with a gain
+// alternate); MT: 16-row tiles (G = 16); U: K steps in flight per wave. NORM 1 (MT = 1): rows are RMS-normed with a gain
 // first, in the order (a * scale) * gain of the norm kernel.
 template <int G, int NT, int MT, int WAVES, int U, int NORM>
 __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int rows_per_group, int gated) {
@@ -36,15 +76,16 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   __shared__ f32x4 red[WAVES][NT * MT][64];
   __shared__ float stat[NORM ? WAVES : 1][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
+  rv_arguments(p);
   // rows of this group: a fixed count, one row with its own expert, or (offs) every row of expert blockIdx.y
   int g0 = blockIdx.y * rows_per_group, g1 = min(g0 + rows_per_group, p.R), e = 0;
   if (p.offs) {
     e = blockIdx.y;
     g0 = p.offs[e];
     g1 = p.offs[e + 1];
-  } else if (p.row_expert) {
-    e = p.row_expert[g0];
-    if (e < 0 || e >= p.E) return;  // (a row of an expert without weights, an identity expert: nothing to compute)
+  } else {
+    e = rv_expert(p, g0);
+    if (e < 0) return;
   }
   const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP;
   const int k0 = 32 * (c / G) + 8 * q;  // this lane's place in a step
@@ -63,7 +104,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int rr = r0 + min(16 * m + c % G, nr - 1);  // (surplus lanes repeat the last row; their results are dropped)
-      xp[m] = reinterpret_cast<const float*>(p.a) + (size_t)(p.a_idx ? p.a_idx[rr] : rr) * p.lda;
+      xp[m] = reinterpret_cast<const float*>(p.a) + (size_t)(p.a_idx ? p.a_idx[rr] : (p.a_div > 1 ? rr / p.a_div : rr)) * p.lda;
       xs[m] = p.a_scale ? p.a_scale[rr] : 1.f;
     }
     // (a lane past the end of a ragged last step reads the row's start; its operands are zeroed before they are used)
@@ -158,33 +199,204 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
 #pragma unroll
       for (int m = 0; m < MT; ++m) red[wave][t * MT + m][lane] = acc[t][m];
     __syncthreads();
-    constexpr int QUADS = G / 4, PER = QUADS * G;  // column quads of a tile; (quad, row) pairs per tile
+    // one output element per thread: the epilogue's code, which a short launch has to fetch, stays small
+    constexpr int PER = G * G;  // (column, row) pairs of a tile
     const int outs = (gated ? NT / 2 : NT) * MT * PER;
     for (int i = tid; i < outs; i += 64 * WAVES) {
-      const int x = i % PER, tm = i / PER, to = tm / MT, m = tm - to * MT;  // output tile, row tile
-      const int row = 16 * m + x % G, cq = x / G, col = G * (blockIdx.x * (gated ? NT / 2 : NT) + to) + 4 * cq;
+      const int y = i % G, x = i / G % G, tm = i / PER, to = tm / MT, m = tm - to * MT;  // column, row; output tile, row tile
+      const int row = 16 * m + x, col = G * (blockIdx.x * (gated ? NT / 2 : NT) + to) + y;
       if (row >= nr || col >= N) continue;
       const int slot = (gated ? 2 * to : to) * MT + m;
-      f32x4 g = f32x4{0.f, 0.f, 0.f, 0.f}, v = g;
+      float g = 0.f, v = 0.f;
 #pragma unroll
       for (int sg = 0; sg < SEG; ++sg) {  // the diagonal block of range sg
-        const int l = 16 * (QUADS * sg + cq) + G * sg + x % G;
+        const int l = 16 * (G / 4 * sg + y / 4) + G * sg + x;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-          g += red[w][slot][l];
-          if (gated) v += red[w][slot + MT][l];
+          g += red[w][slot][l][y % 4];
         }
       }
-      const int r = r0 + row, drow = p.dst_idx ? p.dst_idx[r] : r;
-      float* dst = reinterpret_cast<float*>(p.out) + (size_t)drow * p.ldo + col;
+      if (gated) {
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
-        if (col + y < N) {
-          const float val = lr_act(p, g[y], v[y]);
-          dst[y] = p.add_out ? dst[y] + val : val;
-        }
+        for (int sg = 0; sg < SEG; ++sg)
+#pragma unroll
+          for (int w = 0; w < WAVES; ++w) v += red[w][slot + MT][16 * (G / 4 * sg + y / 4) + G * sg + x][y % 4];
+      }
+      rv_store(p, r0 + row, col, g, v);
     }
     __syncthreads();
+  }
+}
+
+// Linear row r as the product reads it, to row i of the staged activations; K <= 1024 V. Every thread of the workgroup (256)
+// holds columns 4 tid + 1024 u. load() only issues loads: the weights of the first steps are issued behind
+// them, and a wave's loads return in order. With res_y: x + rms(ysc * sum of the row's nsum rows of y) * w, in the
+// norm_residual kernel's order, also written to res_out by the launch's first workgroup.
+JLA_DEV float rv_block_sum(float v, float (*stat)[16]) {
+  v = wave_sum(v);
+  __syncthreads();  // (the sum before is read)
+  if ((threadIdx.x & 63) == 0) stat[threadIdx.x >> 6][0] = v;
+  __syncthreads();
+  return stat[0][0] + stat[1][0] + stat[2][0] + stat[3][0];
+}
+template <int V>
+struct RvRow {
+  f32x4 x[V], y[V], g[V];
+  float scale, w;
+  JLA_DEV void load(const RowLinear& p, int r, int K, int tid) {
+    const int src = p.a_idx ? p.a_idx[r] : (p.a_div > 1 ? r / p.a_div : r);
+    const float* xp = reinterpret_cast<const float*>(p.a) + (size_t)src * p.lda;
+    scale = p.a_scale ? p.a_scale[r] : 1.f;
+    w = p.res_y ? p.res_w[0] : 0.f;
+    int k[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      k[u] = 4 * tid + 1024 * u < K ? 4 * tid + 1024 * u : 0;
+      x[u] = *reinterpret_cast<const f32x4*>(xp + k[u]);
+      y[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (p.a_norm_w) {
+#pragma unroll
+      for (int u = 0; u < V; ++u) g[u] = *reinterpret_cast<const f32x4*>(p.a_norm_w + k[u]);
+    }
+    if (p.res_y) {
+      const float* yp = p.res_y + (size_t)src * p.res_nsum * K;
+#pragma unroll
+      for (int u = 0; u < V; ++u) y[u] = *reinterpret_cast<const f32x4*>(yp + k[u]);
+      for (int n = 1; n < p.res_nsum; ++n) {
+#pragma unroll
+        for (int u = 0; u < V; ++u) y[u] += *reinterpret_cast<const f32x4*>(yp + (size_t)n * K + k[u]);
+      }
+    }
+  }
+  JLA_DEV void stage(const RowLinear& p, int r, int i, int K, int tid, float (*stat)[16], f32x4* staged) {
+    if (p.res_y) {
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < V; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          y[u][j] *= p.res_ysc;
+          ss = 4 * tid + 1024 * u < K ? fmaf(y[u][j], y[u][j], ss) : ss;
+        }
+      const float sc = 1.f / sqrtf(rv_block_sum(ss, stat) / (float)K + p.res_eps);
+      // (with several linear rows of a source row, its first writes)
+      const int src = p.a_idx ? p.a_idx[r] : (p.a_div > 1 ? r / p.a_div : r);
+      const bool put = blockIdx.x == 0 && (p.a_div <= 1 || r % p.a_div == 0);
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const int k = 4 * tid + 1024 * u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[u][j] += y[u][j] * sc * w;
+        if (put && k < K) *reinterpret_cast<f32x4*>(p.res_out + (size_t)src * K + k) = x[u];
+      }
+    }
+    if (p.a_norm_w) {
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < V; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss = 4 * tid + 1024 * u < K ? fmaf(x[u][j], x[u][j], ss) : ss;
+      scale = 1.f / sqrtf(rv_block_sum(ss, stat) / (float)K + p.a_norm_eps);
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const int k = 4 * tid + 1024 * u;
+      f32x4 v = x[u] * scale;
+      if (p.a_norm_w) v *= g[u];
+      if (k < K) staged[((size_t)i * K + k) / 4] = v;
+    }
+  }
+};
+
+// One or two rows, K <= 128 WAVES U: a wave's share of K is U steps, so the rows' operands stay in its registers, and a
+// workgroup walks over groups of NT tiles with the next group's weights issued as this one's are consumed. The rows pass
+// through LDS once per workgroup, where a pending residual add (res_y) and the norm are applied behind the first weights.
+// grid (workgroups, linear rows with their own expert, else 1).
+template <int NT, int U, int V>
+__global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups) {
+  constexpr int G = 4, WAVES = 4, STEP = 128;
+  extern __shared__ f32x4 staged[];  // [rows][K]
+  __shared__ f32x4 red[2][WAVES][NT][64];
+  __shared__ float stat[WAVES][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
+  rv_arguments(p);
+  const int r0 = blockIdx.y * rows_per_group, nr = min(rows_per_group, p.R - r0);
+  const int e = rv_expert(p, r0);
+  if (e < 0) return;  // (the whole workgroup)
+  const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP, k0 = 32 * (c / G) + 8 * q;
+  const bf16_t* wbase = reinterpret_cast<const bf16_t*>(p.w) + (size_t)e * p.w_stride;
+  // this lane's place in step u (a lane past the end of K reads the row's start; its operand is zero)
+  auto at = [&](int u) {
+    const int k = STEP * (wave + WAVES * u) + k0;
+    return k < K ? k : 0;
+  };
+  u32x4 wf[U][NT];
+  auto weight_row = [&](int tg, int t) {
+    const int T = tg * NT + t, col = min(G * (gated ? T >> 1 : T) + c % G, N - 1);
+    return wbase + (size_t)(gated && (T & 1) ? N + col : col) * K;
+  };
+  RvRow<V> row;
+  row.load(p, r0, K, tid);
+  int tg = blockIdx.x;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const bf16_t* w = weight_row(tg, t);
+#pragma unroll
+    for (int u = 0; u < U; ++u) wf[u][t] = load_nt(reinterpret_cast<const u32x4*>(w + at(u)));
+  }
+  row.stage(p, r0, 0, K, tid, stat, staged);
+  if (nr > 1) {
+    row.load(p, r0 + 1, K, tid);
+    row.stage(p, r0 + 1, 1, K, tid, stat, staged);
+  }
+  __syncthreads();
+  u32x4 xr[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {  // (surplus B columns repeat the last row; their results are dropped)
+    const f32x4* x = staged + ((size_t)min(c % G, nr - 1) * K + at(u)) / 4;
+    xr[u] = STEP * (wave + WAVES * u) + k0 < K ? rv_round8(x[0], x[1]) : u32x4{0, 0, 0, 0};
+  }
+  for (int buf = 0; tg < tgroups; tg += gridDim.x, buf ^= 1) {
+    const int next = tg + (int)gridDim.x;
+    const bool more = next < tgroups;  // (workgroup-uniform)
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const bf16_t* w = more ? weight_row(next, t) : wbase;  // (after the last group: one line, unused)
+      acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // (past the end of K both operands are zero: an infinite weight must not meet a zero)
+        const bool in = STEP * (wave + WAVES * u) + k0 < K;
+        acc[t] = mfma16x16x32(in ? wf[u][t] : u32x4{0, 0, 0, 0}, xr[u], acc[t]);
+        wf[u][t] = load_nt(reinterpret_cast<const u32x4*>(w + (more ? at(u) : 0)));
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) red[buf][wave][t][lane] = acc[t];
+    __syncthreads();  // (one per group: the other buffer's readers are past the barrier before)
+    const int outs = (gated ? NT / 2 : NT) * nr * G;
+    if (tid < outs) {
+      const int y = tid % G, to = tid / G / nr, x = tid / G - to * nr, slot = gated ? 2 * to : to;
+      const int col = G * (tg * (gated ? NT / 2 : NT) + to) + y;
+      float g = 0.f, v = 0.f;
+#pragma unroll
+      for (int sg = 0; sg < 4; ++sg) {  // the diagonal block of K range sg
+        const int l = 20 * sg + x;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+          g += red[buf][w][slot][l][y];
+        }
+      }
+      if (gated) {
+#pragma unroll
+        for (int sg = 0; sg < 4; ++sg)
+#pragma unroll
+          for (int w = 0; w < WAVES; ++w) v += red[buf][w][slot + 1][20 * sg + x][y];
+      }
+      if (col < N) rv_store(p, r0 + x, col, g, v);
+    }
   }
 }
 
@@ -195,15 +407,31 @@ constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_N
 bool hy_rows_gemv_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return p.wbf16 && !p.a_bf16 && !p.out_bf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
-         (p.offs || p.row_expert || p.E == 1) && p.K % 8 == 0 &&
+         (p.offs || p.row_expert || p.tab || p.E == 1) && p.K % 8 == 0 &&
          p.K >= (p.R > 2 ? 64 : 256) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
-         (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.offs && !p.row_expert && aligned(p.a_norm_w)));
+         (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && aligned(p.a_norm_w)));
+}
+
+// One or two normed rows, or with a pending residual add, walk: the plain form would read them twice, the norm ahead of the
+// first weight (RMS norm and product, K 2048 x N 2048 | 5152 | 8224 | 32000 | gated 5632: 6.1 | 9.5 | 12.3 | 34.6 | 13.5 us in the
+// plain form, 5.3 | 7.5 | 9.7 | 23.0 | 10.8 walking; K 4096 x 10304: 26.1 -> 17.8). Rows as they are gain nothing from it (4.7 | 7.2 |
+// 9.3 | 22.7 | 11.5 plain, 5.2 | 7.5 | 9.8 | 22.7 | 11.0 walking). Further rows would not fit the registers.
+constexpr int RV_WALK_K = 4096, RV_WALK_ROWS = 2;
+static bool rv_walks(const RowLinear& p, int rows) {
+  return (p.a_norm_w || p.res_y) && !p.offs && rows <= RV_WALK_ROWS && p.K <= RV_WALK_K;
+}
+
+// A pending residual add (res_y) exists in the walking form only: the caller asks first.
+bool hy_rows_gemv_takes_residual(const RowLinear& p) {
+  auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  return hy_rows_gemv_takes(p) && rv_walks(p, p.row_expert || p.tab ? 1 : p.R) && p.R <= RV_WALK_ROWS * (p.a_div > 1 ? p.a_div : 1) &&
+         aligned(p.res_y) && aligned(p.res_out);
 }
 
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   const int gated = hy_act_gated(p.act);
   RowLinear q = p;
-  const bool each = !p.offs && p.row_expert;  // one row, one expert per group
+  const bool each = !p.offs && (p.row_expert || p.tab);  // one row, one expert per group
   if (p.offs) q.row_expert = nullptr;
   const int groups = p.offs ? p.E : (each ? p.R : 1);
   const int rpg = each ? 1 : p.R;
@@ -211,6 +439,29 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // rows of a pass: a dense batch's count rounded up; an expert's share of the sorted rows, twice the mean (at least 4)
   const int even = p.offs && p.even_rows > 0 ? p.even_rows : 0;
   const int rows = each ? 1 : (p.offs ? (even ? even : (p.R < 2 * ((p.R + p.E - 1) / p.E) ? p.R : 2 * ((p.R + p.E - 1) / p.E))) : p.R);
+  if (rv_walks(p, rows)) {
+    // two tiles per step from a few workgroups for every compute unit on; as many workgroups as are resident (four of 88
+    // registers per unit, or two of 156, K > 2048), with equally many steps each
+    const int occ = p.K <= 2048 ? 4 : 2;
+    const long long tiles = (gated ? 2LL : 1LL) * ((p.N + 3) / 4);
+    const int wnt = gated || tiles * groups >= 1024 ? 2 : 1;
+    const long long tg = (tiles + wnt - 1) / wnt;
+    if (tg > 0x7fffffffLL) return -4;
+    const long long room = 256LL * occ / groups > 0 ? 256LL * occ / groups : 1, rounds = (tg + room - 1) / room;
+    const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
+    const unsigned lds = (unsigned)(rows * p.K * sizeof(float));
+#define RV_WALK(NT, U, V) rows_gemv_walk_kernel<NT, U, V><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg)
+    if (p.K <= 2048) {
+      if (wnt == 1) RV_WALK(1, 4, 2);
+      else RV_WALK(2, 4, 2);
+    } else {
+      if (wnt == 1) RV_WALK(1, 8, 4);
+      else RV_WALK(2, 8, 4);
+    }
+#undef RV_WALK
+    JLA_CHECK_LAUNCH();
+    return 0;
+  }
   const int G = rows <= 4 ? 4 : (rows <= 8 ? 8 : 16), mt = rows <= 16 ? 1 : (rows <= 32 ? 2 : 4);
   const long long tiles = (gated ? 2LL : 1LL) * ((p.N + G - 1) / G);
   // one tile per workgroup until there are a few workgroups for every compute unit; then tiles share the workgroup's

@@ -169,10 +169,12 @@ class LayerListLM:
             x = hy.embed_rows(idf, self.embed, scale=self.embed_scale)
             if self.embed_norm is not None:
                 x = hy.rms_rows(x, self.embed_norm, self.eps)
+            r = hy.Residual(x)
             for blk in self.blocks:
-                blk(x, ctx)
+                blk(r if getattr(blk, "takes_residual", False) else r.value(), ctx)
                 if collect_hidden:
-                    hidden.append(x.reshape(b, s, d).clone())
+                    hidden.append(r.value().reshape(b, s, d).clone())
+            x = r.value()
         if logits_mode == "none":
             return None, x, hidden, []
         if logits_mode in ("last", "argmax"):

@@ -146,26 +146,32 @@ class TokenSide:
         self.table, self.col0 = table, col0
         self.w_gate, self.w_proj, self.norm_w, self.eps = w_gate, w_proj, norm_w, eps
 
-    def __call__(self, x: torch.Tensor, ctx: StepContext) -> None:
-        g = hy.gelu_gate_rows(hy.linear(x, self.w_gate), ctx.ids, self.table, self.col0)
-        hy.norm_residual_(x, hy.linear(g, self.w_proj), self.norm_w, self.eps)
+    def __call__(self, x, ctx: StepContext) -> None:
+        g = hy.linear_rows_gated(x, self.w_gate, ctx.ids, self.table, self.col0)
+        x.add(hy.linear(g, self.w_proj), self.norm_w, self.eps)
 
 
 class OutputNormBlock:
     """``x += norm1(mixer(x)); x += norm2(ff(x)); x += side(x)``: the norm sits on each sublayer's OUTPUT (a scalar
-    gain), the sublayers read the residual itself."""
+    gain), the sublayers read the residual itself. ``x``: a ``Residual``, whose last addition is left to its next reader, or
+    a tensor updated in place."""
+
+    takes_residual = True
 
     def __init__(self, mixer, norm1: torch.Tensor, mlp: Optional[TableMoE], norm2: Optional[torch.Tensor],
                  side: Optional[TokenSide], eps: float):
         self.mixer, self.norm1, self.mlp, self.norm2, self.side, self.eps = mixer, norm1, mlp, norm2, side, eps
 
-    def __call__(self, x: torch.Tensor, ctx: StepContext) -> None:
-        hy.norm_residual_(x, self.mixer(x, ctx), self.norm1, self.eps)
+    def __call__(self, x, ctx: StepContext) -> None:
+        r = x if isinstance(x, hy.Residual) else hy.Residual(x)
+        r.add(self.mixer(r, ctx), self.norm1, self.eps)
         if self.mlp is not None:
             top = self.mlp.spec.top
-            hy.norm_residual_(x, self.mlp(x, ctx), self.norm2, self.eps, nsum=top, ysc=1.0 / top)
+            r.add(self.mlp(r, ctx), self.norm2, self.eps, nsum=top, ysc=1.0 / top)
         if self.side is not None:
-            self.side(x, ctx)
+            self.side(r, ctx)
+        if r is not x and r.value() is not x:
+            x.copy_(r.x)
 
 
 class LatentAttention:

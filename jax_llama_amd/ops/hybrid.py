@@ -134,6 +134,7 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, col0: int = 0, ncols: Opt
 # (N % 16 == 0, K % 32 == 0); the row-major kernel here serves every other case. JLA_HY_PACKED_GEMM=0: never.
 PACKED_GEMM = os.environ.get("JLA_HY_PACKED_GEMM", "1") != "0"
 PACKED_GEMM_MIN_M = 256
+SKINNY_MAX_N = 16  # output columns up to which a dense linear of any row count runs the GEMV (csrc: HY_SKINNY_MAX_N)
 GROUPED_GEMV_MAX_R = 64  # rows up to which an expert-sorted batch runs the expert-grouped GEMV (csrc: HY_GROUPED_GEMV_MAX_R)
 _PACKED = {}
 
@@ -220,6 +221,56 @@ def _act_cpu(y: torch.Tensor, act: int, limit: float, alpha: float) -> torch.Ten
     return g * torch.sigmoid(alpha * g) * (u.clamp(-limit, limit) + 1.0)
 
 
+class Residual:
+    """A step's residual stream ``x [M, D]`` with its last sublayer's result not added yet (``norm_residual_``'s arguments): the
+    product that reads the stream next adds it where it has few rows (``rows_gemv.hip``), ``value()`` everywhere else."""
+
+    __slots__ = ("x", "pending")
+
+    def __init__(self, x: torch.Tensor):
+        self.x, self.pending = x, None
+
+    def add(self, y: torch.Tensor, w: torch.Tensor, eps: float, nsum: int = 1, ysc: float = 1.0) -> None:
+        self.value()
+        self.pending = (y, int(nsum), float(ysc), w.reshape(-1), float(eps))
+
+    def value(self) -> torch.Tensor:
+        if self.pending is not None:
+            (y, nsum, ysc, w, eps), self.pending = self.pending, None
+            norm_residual_(self.x, y, w, eps, nsum, ysc)
+        return self.x
+
+    def fusable(self) -> bool:
+        return (self.pending is not None and _gpu(self.x) and self.x.shape[0] <= RESIDUAL_MAX_ROWS and self.x.is_contiguous()
+                and self.pending[3].numel() == 1)
+
+
+RESIDUAL_MAX_ROWS = 2  # csrc: RV_WALK_ROWS
+FEW_ROWS = 64          # csrc: RV_MAX_ROWS
+
+
+def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, table: Optional[torch.Tensor] = None,
+                      col0: int = 0) -> torch.Tensor:
+    """``x @ w^T`` of a ``Residual`` (or a tensor), with ``ids``: ``gelu_gate_rows(x @ w^T, ids, table, col0)``. A few bf16 rows
+    take the pending residual add and the gate in the product's launch; else the separate ops."""
+    r = x if isinstance(x, Residual) else None
+    ids = ids.reshape(-1).to(torch.int32).contiguous() if ids is not None else None
+    if r is not None and r.fusable():
+        out = torch.empty(r.x.shape[0], w.shape[0], dtype=F32, device=r.x.device)
+        new = torch.empty_like(r.x)
+        if ext().rows_fused(r.x, w, out, *r.pending, new, ids, table, int(col0)):
+            r.x, r.pending = new, None
+            return out
+    xv = r.value() if r is not None else x
+    if ids is None:
+        return linear(xv, w)
+    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and xv.dtype == F32:
+        out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
+        if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, ids, table, int(col0)):
+            return out
+    return gelu_gate_rows(linear(xv, w), ids, table, col0)
+
+
 def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit: float = 0.0,
            alpha: float = 1.0, out_dtype=F32) -> torch.Tensor:
     """``act(x [M, K] (fp32, or an ``RmsInput``) @ w^T)`` -> fp32 ``[M, N]``. ``act``: none, ``ACT_RELU2`` (``max(y, 0)^2``),
@@ -229,6 +280,10 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     ``g' = min(g, limit)``, ``u' = clamp(u, -limit, limit)``). ``x`` may be a column-contiguous view with strided rows; with
     bf16 weights and no activation it may be bf16 already (the operand it would be rounded to anyway). ``out_dtype`` bf16:
     the result as the next product's operand, where that saves a pass (a prompt on the large tiles); else fp32 all the same."""
+    if isinstance(x, Residual):
+        if act == ACT_NONE and not swiglu and x.fusable() and w.shape[0] > SKINNY_MAX_N:
+            return linear_rows_gated(x, w)
+        x = x.value()
     if swiglu:
         act = ACT_SWIGLU
     n = w.shape[0] // 2 if act_gated(act) else w.shape[0]
@@ -424,9 +479,26 @@ def moe_table(x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, w_gu: tor
 
     ``w_gu [E, 2F, K]`` (gate rows then up rows), ``w_down [E, D, F]``. Returns the chosen experts' outputs, fp32
     ``[M * top, D]`` in (token, choice) order; the caller averages them (``norm_residual_(nsum=top, ysc=1/top)``)."""
+    res = x if isinstance(x, Residual) else None
+    x = x.x if res is not None else x
     m, top, e_n = x.shape[0], table.shape[1], w_gu.shape[0]
     r = m * top
     ids = ids.reshape(-1)
+    if _gpu(x) and 0 < r <= ext().GEMV_MAX_R and x.dtype == F32 and w_gu.dtype == w_down.dtype == BF16:
+        # decode: the products read the table themselves, and the first one adds a pending residual
+        h = torch.empty(r, w_gu.shape[1] // 2, dtype=F32, device=x.device)
+        y = torch.empty(r, w_down.shape[1], dtype=F32, device=x.device)
+        args = (ids.to(torch.int32).contiguous(), table, w_gu, w_down, h, y)
+        if res is not None and res.fusable():
+            new = torch.empty_like(x)
+            if ext().table_rows(x, *args, *res.pending, new):
+                res.x, res.pending = new, None
+                return y
+        x = res.value() if res is not None else x
+        if ext().table_rows(x, *args, None, 1, 1.0, None, 0.0, None):
+            return y
+    if res is not None:
+        x = res.value()
     if not _gpu(x):
         ex = table[ids.long()].reshape(-1).long()  # [R]
         xr = _round_like(x, w_gu).repeat_interleave(top, 0)

@@ -599,3 +599,52 @@ def test_one_token_recurrence(kind, b, h, dim, vdim):
         res.append((y, st, ms))
     for r, x, name in zip(*res, ("out", "state", "running maximum")):
         _close(x, r, 2e-5, name)
+
+
+def _residual(m, d, nsum, dev, seed=5):
+    g = torch.Generator().manual_seed(seed)
+    x, y = torch.randn(m, d, generator=g), torch.randn(m * nsum, d, generator=g) * 3.0
+    r = hy.Residual(x.clone().to(dev))
+    r.add(y.to(dev), torch.tensor([0.7]).to(dev), 1e-6, nsum, 1.0 / nsum)
+    return r
+
+
+@pytest.mark.parametrize("m,k,n,nsum", [(1, 2048, 2048, 1), (2, 2048, 5153, 2), (1, 64, 17, 1), (1, 4096, 516, 3), (2, 2056, 40, 1),
+                                        (1, 1024, 20000, 2), (3, 256, 64, 1), (1, 4104, 96, 1), (1, 250, 96, 1), (1, 256, 9, 2)])
+def test_pending_residual_in_the_product(m, k, n, nsum):
+    """The product that adds the sublayer's result itself (up to two rows, K <= 4096) against the separate ops on the CPU. The
+    residual is fp32 sums in another order; a bf16 operand may then round to its other neighbour (2^-9 of one of k terms)."""
+    w, gate = _rand(n, k, dt=torch.bfloat16, std=k ** -0.5), _rand(9, 3 * n)
+    ids = torch.randint(-1, 10, (m,), dtype=torch.int32).clamp(0, 8)
+    for gated in (False, True):
+        out = []
+        for dev in ("cpu", DEV):
+            r = _residual(m, k, nsum, dev)
+            y = hy.linear_rows_gated(r, w.to(dev), ids.to(dev), gate.to(dev), n) if gated else hy.linear(r, w.to(dev))
+            out.append((y, r.value()))
+        _close(out[1][1], out[0][1], 2e-6, "residual")
+        _close(out[1][0], out[0][0], 2e-3, "product")
+    x, gw = _rand(m, k), torch.rand(k) + 0.5  # a normed row walks too
+    got = hy.linear(hy.RmsInput(x.to(DEV), gw.to(DEV), 1e-6), w.to(DEV))
+    _close(got, hy.linear(hy.RmsInput(x, gw, 1e-6), w), 2e-3, "normed product")
+
+
+@pytest.mark.parametrize("m,top,e,d,f", [(1, 2, 8, 256, 96), (2, 2, 8, 2048, 704), (4, 2, 3, 64, 72), (1, 1, 4, 256, 264), (3, 3, 5, 128, 64),
+                                         (1, 2, 4, 130, 64)])
+def test_table_experts_without_a_routing_launch(m, top, e, d, f):
+    """The products that read the expert table themselves, with and without the pending residual."""
+    w_gu, w_dn = _rand(e, 2 * f, d, dt=torch.bfloat16, std=d ** -0.5), _rand(e, d, f, dt=torch.bfloat16, std=f ** -0.5)
+    table = torch.randint(0, e, (50, top), dtype=torch.int32)
+    ids = torch.randint(0, 50, (m,), dtype=torch.int32)
+    for pending in (False, True):
+        out = []
+        for dev in ("cpu", DEV):
+            r = _residual(m, d, 2, dev) if pending else _rand_fixed(m, d).to(dev)
+            y = hy.moe_table(r, ids.to(dev), table.to(dev), w_gu.to(dev), w_dn.to(dev))
+            out.append((y, r.value() if pending else y))
+        _close(out[1][0], out[0][0], 4e-3, "experts")  # (bf16: see test_moe_table)
+        _close(out[1][1], out[0][1], 2e-6 if pending else 4e-3, "residual")
+
+
+def _rand_fixed(m, d):
+    return torch.randn(m, d, generator=torch.Generator().manual_seed(m * d))
