@@ -65,13 +65,14 @@ const float* rows2d(const Tensor& t, const char* name, int64_t cols, int* ld) {
   return reinterpret_cast<const float*>(t.data_ptr());
 }
 
-void embed_rows(Tensor ids, Tensor table, int64_t col0, Tensor out, double scale, int64_t copies) {
+void embed_rows(Tensor ids, Tensor table, int64_t col0, Tensor out, double scale, int64_t copies, OptT norm, double eps) {
   const int wb = wtype(table, "table");
   check(table.dim() == 2 && out.dim() == 2 && copies >= 1 && out.size(0) % copies == 0,
         "embed_rows: 2-d table, out is [copies * M, D]");
   const int M = out.size(0) / copies, D = out.size(1);
+  check(!norm.has_value() || norm->numel() == D, "embed_rows: norm is [D]");
   rc(jla::hy_embed_rows(i32(ids, "ids", M), table.data_ptr(), wb, table.size(0), table.size(1), col0,
-                        (float)scale, f32w(out, "out"), M, D, copies, stream()),
+                        (float)scale, f32w(out, "out"), M, D, copies, norm.has_value() ? f32(*norm, "norm") : nullptr, eps, stream()),
      "embed_rows");
 }
 
@@ -144,23 +145,26 @@ void linear_rows(Tensor a, OptT a_idx, Tensor w, Tensor out, OptT dst_idx, OptT 
 void set_residual(jla::RowLinear& p, const Tensor& a, const OptT& y, int64_t nsum, double ysc, const OptT& w, double eps,
                   const OptT& x_out) {
   if (!y.has_value()) return;
-  check(w.has_value() && x_out.has_value() && w->numel() == 1 && nsum >= 1, "residual: one gain, nsum >= 1");
+  check(w.has_value() && x_out.has_value() && (w->numel() == 1 || w->numel() == p.K) && nsum >= 1,
+        "residual: one gain or one per column, nsum >= 1");
   check(a.is_contiguous() && y->numel() == a.numel() * nsum && x_out->sizes() == a.sizes() &&
             x_out->data_ptr() != a.data_ptr(), "residual: y is [rows * nsum, K], x_out another [rows, K]");
   p.res_y = f32(*y, "y");
   p.res_nsum = nsum;
   p.res_ysc = ysc;
   p.res_w = f32(*w, "w");
+  p.res_w_vec = w->numel() != 1;
   p.res_eps = eps;
   p.res_out = f32w(*x_out, "x_out");
 }
 
 // out = f(a' @ w^T) for a few rows in one launch: a' = a + rms_norm(ysc * sum of nsum rows of y) * res_w with y (written to x_out
-// too), f = gelu_tanh * table[ids, col0 ..] with ids. False: not a call of that kernel, nothing was launched.
+// too), then normed with gain a_norm_w where that is given; f = act, then with ids gelu_tanh * table[ids, col0 ..]. False: not a call of that kernel, nothing was launched.
 bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc, OptT res_w, double eps, OptT x_out, OptT ids,
-                OptT table, int64_t col0) {
-  jla::RowLinear p = row_linear(a, c10::nullopt, w, out, c10::nullopt, c10::nullopt, c10::nullopt, a.size(0), 0, 0.0, 1.0,
-                                c10::nullopt, c10::nullopt, 0.0, 0, false);
+                OptT table, int64_t col0, OptT a_norm_w, double a_norm_eps, int64_t act, double act_limit) {
+  jla::RowLinear p = row_linear(a, c10::nullopt, w, out, c10::nullopt, c10::nullopt, c10::nullopt, a.size(0), act, act_limit, 1.0,
+                                c10::nullopt, a_norm_w, a_norm_eps, 0, false);
+  check(act != jla::HY_ACT_SOFTCAP || act_limit > 0, "rows_fused: softcap");
   set_residual(p, a, y, nsum, ysc, res_w, eps, x_out);
   if (ids.has_value()) {
     check(table.has_value() && table->dim() == 2 && col0 >= 0 && col0 + p.N <= table->size(1), "rows_fused: table columns");
@@ -880,11 +884,13 @@ void rotate_heads(Tensor a, Tensor positions, OptT freq, int64_t H, double sign,
      "rotate_heads");
 }
 
-void token_shift(Tensor h, Tensor prev, Tensor mu, Tensor out, int64_t B, int64_t S) {
+void token_shift(Tensor h, Tensor prev, Tensor mu, Tensor out, int64_t B, int64_t S, OptT w, double eps) {
   check(mu.dim() == 2, "token_shift: mu is [n, D]");
   const int64_t n = mu.size(0), D = mu.size(1);
+  check(!w.has_value() || w->numel() == D, "token_shift: w is [D]");
   check(h.numel() == B * S * D && prev.numel() == B * D && out.numel() == n * B * S * D, "token_shift shapes");
-  rc(jla::hy_token_shift(f32(h, "h"), f32w(prev, "prev"), f32(mu, "mu"), n, f32w(out, "out"), B, S, D, stream()),
+  rc(jla::hy_token_shift(f32(h, "h"), f32w(prev, "prev"), f32(mu, "mu"), n, f32w(out, "out"), B, S, D,
+                         w.has_value() ? f32(*w, "w") : nullptr, eps, stream()),
      "token_shift");
 }
 
@@ -1005,7 +1011,7 @@ void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("GEMV_MAX_R") = jla::HY_GEMV_MAX_R;
   m.def("embed_rows", &embed_rows, py::arg("ids"), py::arg("table"), py::arg("col0"), py::arg("out"), py::arg("scale"),
-        py::arg("copies") = 1);
+        py::arg("copies") = 1, py::arg("norm") = py::none(), py::arg("eps") = 0.0);
   m.def("route_grouped", &route_grouped, py::arg("z"), py::arg("correction"), py::arg("E"), py::arg("top"),
         py::arg("groups"), py::arg("keep"), py::arg("row_expert"), py::arg("row_tok"), py::arg("row_w"),
         py::arg("sort_tok"), py::arg("sort_dst"), py::arg("sort_w"), py::arg("offs"), py::arg("sigmoid") = false,
@@ -1055,7 +1061,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_scan", &delta_scan);
   m.def("rows_fused", &rows_fused, py::arg("a"), py::arg("w"), py::arg("out"), py::arg("y"), py::arg("nsum"), py::arg("ysc"),
         py::arg("res_w"), py::arg("eps"), py::arg("x_out"), py::arg("ids") = py::none(), py::arg("table") = py::none(),
-        py::arg("col0") = 0);
+        py::arg("col0") = 0, py::arg("a_norm_w") = py::none(), py::arg("a_norm_eps") = 0.0, py::arg("act") = 0,
+        py::arg("act_limit") = 0.0);
   m.def("table_rows", &table_rows);
   m.def("rec_step_takes", &rec_step_takes);
   m.def("rec_step", &rec_step, py::arg("mode"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("pre") = py::none(),
@@ -1079,7 +1086,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("depth_update", &depth_update);
   m.def("rotate_heads", &rotate_heads, py::arg("a"), py::arg("positions"), py::arg("freq"), py::arg("H"), py::arg("sign"),
         py::arg("gain"), py::arg("out"), py::arg("offset") = 0, py::arg("interleaved") = false);
-  m.def("token_shift", &token_shift);
+  m.def("token_shift", &token_shift, py::arg("h"), py::arg("prev"), py::arg("mu"), py::arg("out"), py::arg("B"), py::arg("S"),
+        py::arg("w") = py::none(), py::arg("eps") = 0.0);
   m.def("mlstm_prep", &mlstm_prep);
   m.def("lin_scan", &lin_scan, py::arg("mode"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("decay"),
         py::arg("write"), py::arg("w0"), py::arg("u"), py::arg("state"), py::arg("o"), py::arg("B"), py::arg("S"),

@@ -15,7 +15,7 @@ namespace jla {
 // out[c][M, D] (fp32) = table[ids[m], col0 : col0 + D] * scale for c < copies (the same rows `copies` times: the residual
 // streams of a hyper-connected stack); table rows are `ld` elements apart. Ids outside [0, V) read row 0.
 int hy_embed_rows(const int32_t* ids, const void* table, int wbf16, int V, int ld, int col0, float scale, float* out,
-                  int M, int D, int copies, hipStream_t s);
+                  int M, int D, int copies, const float* w, float eps, hipStream_t s);  // w: optional [D] gain, the rows normed
 
 // Epilogue of a row linear. Plain forms take one accumulator, gated forms two (gate rows [0, N), up rows [N, 2N)).
 enum RowAct {
@@ -62,11 +62,12 @@ struct RowLinear {
   const void* mul_table;
   int mul_bf16, mul_V, mul_ld, mul_col0;
   // optional: the activation row m is a[m] + rms_norm(res_ysc * sum of rows m res_nsum ... of res_y [., K]) * res_w (one
-  // number), also written to res_out [., K] (not a)
+  // number, or with res_w_vec [K]), also written to res_out [., K] (not a); a_norm_w then norms that row
   const float* res_y;
   int res_nsum;
   float res_ysc, res_eps;
   const float* res_w;
+  int res_w_vec;
   float* res_out;
 };
 inline bool hy_act_gated(int act) {
@@ -416,7 +417,9 @@ int hy_rotate_heads(const float* a, int lda, const int32_t* positions, const dou
 
 // out[i][m][:] = h[m] + (h[m - 1] - h[m]) * mu[i] for i < n; the row before a sequence's first is prev[b] (then set to
 // the sequence's last row)
-int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, hipStream_t s);
+// w: optional [D] gain, h is RMS-normed first (S = 1, D <= 4096)
+int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, const float* w, float eps,
+                   hipStream_t s);
 
 struct MlstmPrep {
   const float* proj;  // [M, ld]: input-gate pre-activations at columns [col_i, col_i + H), forget-gate at [col_f, col_f + H)

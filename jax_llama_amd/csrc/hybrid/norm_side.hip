@@ -14,29 +14,57 @@ namespace jla {
 JLA_DEV float ns_ld(const float* p) { return *p; }
 JLA_DEV float ns_ld(const bf16_t* p) { return bf2f(*p); }
 
+// one workgroup per row; with a gain w the row is RMS-normed (the row is read a second time, from the cache)
 template <typename WT>
 __global__ void __launch_bounds__(256) embed_rows_kernel(const int32_t* ids, const WT* table, int V, int ld, int col0,
-                                                         float scale, float* out, int D, int copies) {
+                                                         float scale, float* out, int D, int copies, const float* w, float eps) {
+  __shared__ float red[16];
   const int m = blockIdx.x, M = gridDim.x;
   int id = ids[m];
   id = id < 0 || id >= V ? 0 : id;
   const WT* row = table + (size_t)id * ld + col0;
-  for (int d = threadIdx.x; d < D; d += 256) {
-    const float v = ns_ld(row + d) * scale;
-    for (int c = 0; c < copies; ++c) out[((size_t)c * M + m) * D + d] = v;
+  float sc = 1.f;
+  if (w) {
+    float ss = 0.f;
+#pragma unroll 4
+    for (int d = 8 * threadIdx.x; d < D; d += 8 * 256) {
+      float f[8];
+      hy_load8(row + d, D - d, f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = fmaf(f[i] * scale, f[i] * scale, ss);
+    }
+    sc = 1.f / sqrtf(block_sum(ss, red) / (float)D + eps);
+  }
+  for (int d = 8 * threadIdx.x; d < D; d += 8 * 256) {
+    float f[8], g[8];
+    hy_load8(row + d, D - d, f);
+    if (w) hy_load8(w + d, D - d, g);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = w ? f[i] * scale * sc * g[i] : f[i] * scale;
+    for (int c = 0; c < copies; ++c) {
+      float* to = out + ((size_t)c * M + m) * D + d;
+      if (D - d >= 8 && ((uintptr_t)to & 15) == 0) {
+        *reinterpret_cast<float4*>(to) = make_float4(f[0], f[1], f[2], f[3]);
+        *reinterpret_cast<float4*>(to + 4) = make_float4(f[4], f[5], f[6], f[7]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (d + i < D) to[i] = f[i];
+      }
+    }
   }
 }
 
 int hy_embed_rows(const int32_t* ids, const void* table, int wbf16, int V, int ld, int col0, float scale, float* out,
-                  int M, int D, int copies, hipStream_t s) {
+                  int M, int D, int copies, const float* w, float eps, hipStream_t s) {
   if (M < 0 || D < 1 || V < 1 || col0 < 0 || col0 + D > ld || copies < 1) return -1;
   if (M == 0) return 0;
   if (wbf16)
     embed_rows_kernel<bf16_t><<<M, 256, 0, s>>>(ids, reinterpret_cast<const bf16_t*>(table), V, ld, col0, scale, out, D,
-                                                copies);
+                                                copies, w, eps);
   else
     embed_rows_kernel<float><<<M, 256, 0, s>>>(ids, reinterpret_cast<const float*>(table), V, ld, col0, scale, out, D,
-                                               copies);
+                                               copies, w, eps);
   JLA_CHECK_LAUNCH();
   return 0;
 }

@@ -37,12 +37,42 @@ __global__ void __launch_bounds__(256) token_shift_kernel(const float* __restric
   if (s == 0) prev[(size_t)b * D + d] = last;  // (this thread was the only reader of prev[b, d])
 }
 
-int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, hipStream_t s) {
+// one token per row, the token RMS-normed first (every workgroup of a row repeats its sum, which a launch of the norm would
+// cost more than); prev holds normed tokens
+__global__ void __launch_bounds__(256) token_shift_norm_kernel(const float* __restrict__ x, const float* __restrict__ w, float eps,
+                                                               float* prev, const float* __restrict__ mu, int n,
+                                                               float* __restrict__ out, int D, size_t MD) {
+  __shared__ float red[16];
+  const int m = blockIdx.x, d = blockIdx.y * 256 + threadIdx.x;
+  const float* row = x + (size_t)m * D;
+  float v[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) v[u] = row[min((int)threadIdx.x + 256 * u, D - 1)];
+  const int dc = min(d, D - 1);
+  const float own = row[dc], before = prev[(size_t)m * D + dc], g = w[dc];
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) ss = (int)threadIdx.x + 256 * u < D ? fmaf(v[u], v[u], ss) : ss;
+  ss = block_sum(ss, red);
+  if (d >= D) return;
+  const float c = own * (1.f / sqrtf(ss / (float)D + eps)) * g, diff = before - c;
+  for (int i = 0; i < n; ++i) out[(size_t)i * MD + (size_t)m * D + d] = fmaf(diff, mu[(size_t)i * D + d], c);
+  prev[(size_t)m * D + d] = c;  // (this thread is its only reader)
+}
+
+int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, const float* w, float eps,
+                   hipStream_t s) {
   if (B < 0 || S < 1 || D < 1 || n < 1) return -1;
   if (B == 0) return 0;
   const long long M = (long long)B * S;
   if (M > 0x7fffffffLL || (D + 255) / 256 > 65535) return -2;
-  token_shift_kernel<<<dim3((unsigned)M, (D + 255) / 256), 256, 0, s>>>(h, prev, mu, n, out, S, D, (size_t)M * D);
+  const dim3 grid((unsigned)M, (D + 255) / 256);
+  if (w) {
+    if (S != 1 || D > 4096) return -3;
+    token_shift_norm_kernel<<<grid, 256, 0, s>>>(h, w, eps, prev, mu, n, out, D, (size_t)M * D);
+  } else {
+    token_shift_kernel<<<grid, 256, 0, s>>>(h, prev, mu, n, out, S, D, (size_t)M * D);
+  }
   JLA_CHECK_LAUNCH();
   return 0;
 }

@@ -241,13 +241,12 @@ JLA_DEV float rv_block_sum(float v, float (*stat)[16]) {
 }
 template <int V>
 struct RvRow {
-  f32x4 x[V], y[V], g[V];
-  float scale, w;
+  f32x4 x[V], y[V], g[V], w[V];
+  float scale;
   JLA_DEV void load(const RowLinear& p, int r, int K, int tid) {
     const int src = p.a_idx ? p.a_idx[r] : (p.a_div > 1 ? r / p.a_div : r);
     const float* xp = reinterpret_cast<const float*>(p.a) + (size_t)src * p.lda;
     scale = p.a_scale ? p.a_scale[r] : 1.f;
-    w = p.res_y ? p.res_w[0] : 0.f;
     int k[V];
 #pragma unroll
     for (int u = 0; u < V; ++u) {
@@ -263,6 +262,14 @@ struct RvRow {
       const float* yp = p.res_y + (size_t)src * p.res_nsum * K;
 #pragma unroll
       for (int u = 0; u < V; ++u) y[u] = *reinterpret_cast<const f32x4*>(yp + k[u]);
+      if (p.res_w_vec) {
+#pragma unroll
+        for (int u = 0; u < V; ++u) w[u] = *reinterpret_cast<const f32x4*>(p.res_w + k[u]);
+      } else {
+        const float w0 = p.res_w[0];
+#pragma unroll
+        for (int u = 0; u < V; ++u) w[u] = f32x4{w0, w0, w0, w0};
+      }
       for (int n = 1; n < p.res_nsum; ++n) {
 #pragma unroll
         for (int u = 0; u < V; ++u) y[u] += *reinterpret_cast<const f32x4*>(yp + (size_t)n * K + k[u]);
@@ -287,7 +294,7 @@ struct RvRow {
       for (int u = 0; u < V; ++u) {
         const int k = 4 * tid + 1024 * u;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[u][j] += y[u][j] * sc * w;
+        for (int j = 0; j < 4; ++j) x[u][j] += y[u][j] * sc * w[u][j];
         if (put && k < K) *reinterpret_cast<f32x4*>(p.res_out + (size_t)src * K + k) = x[u];
       }
     }
@@ -425,7 +432,7 @@ static bool rv_walks(const RowLinear& p, int rows) {
 bool hy_rows_gemv_takes_residual(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return hy_rows_gemv_takes(p) && rv_walks(p, p.row_expert || p.tab ? 1 : p.R) && p.R <= RV_WALK_ROWS * (p.a_div > 1 ? p.a_div : 1) &&
-         aligned(p.res_y) && aligned(p.res_out);
+         aligned(p.res_y) && aligned(p.res_out) && (!p.res_w_vec || aligned(p.res_w));
 }
 
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {

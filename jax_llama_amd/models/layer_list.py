@@ -166,14 +166,14 @@ class LayerListLM:
                 if collect_hidden:
                     hidden.append(x.reshape(b, s, d).clone())
         else:
-            x = hy.embed_rows(idf, self.embed, scale=self.embed_scale)
-            if self.embed_norm is not None:
-                x = hy.rms_rows(x, self.embed_norm, self.eps)
-            r = hy.Residual(x)
+            r = hy.Residual(hy.embed_rows(idf, self.embed, scale=self.embed_scale, norm=self.embed_norm, eps=self.eps))
             for blk in self.blocks:
                 blk(r if getattr(blk, "takes_residual", False) else r.value(), ctx)
                 if collect_hidden:
                     hidden.append(r.value().reshape(b, s, d).clone())
+            if s == 1 and logits_mode in ("last", "argmax", "all") and not isinstance(self.final_norm, hy.SquashNorm):
+                logits = hy.head_linear(r, self.final_norm, self.eps, self.head, float(self.logit_softcap or 0.0))
+                return logits, r.value(), hidden, []
             x = r.value()
         if logits_mode == "none":
             return None, x, hidden, []

@@ -388,7 +388,7 @@ class TimeMix:
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
         nh, dim, m = self.heads, self.dim, ctx.b * ctx.s
         state, prev = ctx.cache.recurrent(self.i)
-        mixes = hy.token_shift(_value(h), prev, self.mu, ctx.b, ctx.s)
+        mixes = hy.token_shift(h, prev, self.mu, ctx.b, ctx.s)
         if 4 * m <= hy.STACKED_MAX_ROWS:  # a few tokens: the four same-shaped projections as one grouped launch
             r, k, v, g = hy.stacked_linear(mixes[:4], self.w_rkvg).unbind(0)
         else:
@@ -413,9 +413,11 @@ class SideBySide:
         self.width = sum(mm.width for mm in self.members)
 
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
-        hv = _value(h)
+        m = ctx.b * ctx.s
+        # (each member norms its own copy of the input where that costs nothing, else they share one)
+        hv = h if ctx.s == 1 and isinstance(h, hy.RmsInput) and hy.norms_free(m, self.w_o, h.x.shape[1]) else _value(h)
         if out is None:
-            out = torch.empty(ctx.b * ctx.s, self.width, dtype=torch.float32, device=hv.device)
+            out = torch.empty(m, self.width, dtype=torch.float32, device=hv.device if torch.is_tensor(hv) else hv.x.device)
         c = 0
         for mm, sc in zip(self.members, self.scales):
             mm.features(hv, ctx, out=out[:, c:c + mm.width], gain=gain * sc)

@@ -112,20 +112,26 @@ def _round_like(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # ------------------------------------------------------------------------------------------------ rows
 def embed_rows(ids: torch.Tensor, table: torch.Tensor, col0: int = 0, ncols: Optional[int] = None,
-               scale: float = 1.0, copies: int = 1, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+               scale: float = 1.0, copies: int = 1, out: Optional[torch.Tensor] = None,
+               norm: Optional[torch.Tensor] = None, eps: float = 0.0) -> torch.Tensor:
     """fp32 ``[M, ncols]`` = ``table[ids, col0 : col0 + ncols] * scale``; ``copies > 1``: ``[copies, M, ncols]``, the
     same rows ``copies`` times (the residual streams of a hyper-connected stack all start from the embedding). ``out``
-    (one copy): a contiguous ``[M, ncols]`` tensor to write into."""
+    (one copy): a contiguous ``[M, ncols]`` tensor to write into. ``norm [ncols]``: the rows ``rms_rows(., norm, eps)``."""
     ncols = table.shape[1] - col0 if ncols is None else ncols
     ids = ids.reshape(-1)
     if not _gpu(table):
         x = table[ids.long(), col0:col0 + ncols].float() * torch.tensor(scale, dtype=F32)
+        if norm is not None:
+            x = rms_rows(x, norm, eps)
         if out is not None:
             return out.copy_(x)
         return x if copies == 1 else x[None].repeat(copies, 1, 1)
     if out is None:
         out = torch.empty(copies * ids.numel(), ncols, dtype=F32, device=table.device)
-    ext().embed_rows(ids.to(torch.int32).contiguous(), table, int(col0), out, float(scale), int(copies))
+    fused = norm if norm is not None and norm.numel() == ncols else None
+    ext().embed_rows(ids.to(torch.int32).contiguous(), table, int(col0), out, float(scale), int(copies), fused, float(eps))
+    if norm is not None and fused is None:
+        out = rms_rows(out, norm, eps)
     return out if copies == 1 else out.reshape(copies, ids.numel(), ncols)
 
 
@@ -242,7 +248,7 @@ class Residual:
 
     def fusable(self) -> bool:
         return (self.pending is not None and _gpu(self.x) and self.x.shape[0] <= RESIDUAL_MAX_ROWS and self.x.is_contiguous()
-                and self.pending[3].numel() == 1)
+                and self.pending[3].numel() in (1, self.x.shape[1]))
 
 
 RESIDUAL_MAX_ROWS = 2  # csrc: RV_WALK_ROWS
@@ -269,6 +275,33 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, ids, table, int(col0)):
             return out
     return gelu_gate_rows(linear(xv, w), ids, table, col0)
+
+
+def norms_free(rows: int, w: torch.Tensor, k: Optional[int] = None) -> bool:
+    """Whether a product of ``rows`` rows of ``k`` numbers (``w``'s columns) on matrices like ``w`` norms them at no cost (csrc: the
+    walking form of rows_gemv.hip)."""
+    k = w.shape[1] if k is None else k
+    return (_gpu(w) and w.dtype == BF16 and w.dim() == 2 and rows <= RESIDUAL_MAX_ROWS and w.shape[0] > SKINNY_MAX_N
+            and k % 8 == 0 and 256 <= k <= 4096)
+
+
+def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float = 0.0) -> torch.Tensor:
+    """``linear(rms_rows(x, gain, eps), w)``, softcapped if ``cap > 0``, of a ``Residual`` or a tensor: one or two rows take the
+    pending add and the norm in the product's launch."""
+    act, r = ACT_SOFTCAP if cap > 0 else ACT_NONE, x if isinstance(x, Residual) else None
+    xv = r.x if r is not None else x
+    if norms_free(xv.shape[0], w) and gain.numel() == xv.shape[1] and xv.is_contiguous():
+        out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
+        norm = dict(a_norm_w=gain, a_norm_eps=float(eps), act=act, act_limit=float(cap))
+        if r is not None and r.fusable():
+            new = torch.empty_like(xv)
+            if ext().rows_fused(xv, w, out, *r.pending, new, **norm):
+                r.x, r.pending = new, None
+                return out
+        xv = r.value() if r is not None else x
+        if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, **norm):
+            return out
+    return linear(rms_rows(r.value() if r is not None else x, gain, eps), w, act=act, limit=cap)
 
 
 def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit: float = 0.0,
@@ -1399,11 +1432,17 @@ def rotate_heads(a: torch.Tensor, positions: torch.Tensor, freq: Optional[torch.
 
 
 # ------------------------------------------------------------------------------------------------ linear recurrences
-def token_shift(h: torch.Tensor, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int) -> torch.Tensor:
+def token_shift(h, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int) -> torch.Tensor:
     """``out[n, m] = h[m] + (h[m - 1] - h[m]) * mu[n]`` for the ``n`` rows of ``mu [n, D]``; the token before a call's
     first comes from ``prev [B, D]`` (zeros at a sequence start), which is then set to the call's last token. fp32
-    ``[n, B*S, D]``."""
+    ``[n, B*S, D]``. ``h`` may be an ``RmsInput``: one token per row is normed by the same launch."""
     n, d = mu.shape
+    if isinstance(h, RmsInput):
+        if s == 1 and _gpu(h.x) and h._value is None and d <= 4096 and h.gain.numel() == d and h.x.is_contiguous():
+            out = torch.empty(n, b, d, dtype=F32, device=h.x.device)
+            ext().token_shift(h.x, prev, mu, out, b, s, h.gain, h.eps)
+            return out
+        h = h.value()
     if not _gpu(h):
         hh = h.float().reshape(b, s, d)
         before = torch.cat([prev.float()[:, None], hh[:, :-1]], 1)

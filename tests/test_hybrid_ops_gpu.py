@@ -601,11 +601,12 @@ def test_one_token_recurrence(kind, b, h, dim, vdim):
         _close(x, r, 2e-5, name)
 
 
-def _residual(m, d, nsum, dev, seed=5):
+def _residual(m, d, nsum, dev, seed=5, vector=False):
     g = torch.Generator().manual_seed(seed)
     x, y = torch.randn(m, d, generator=g), torch.randn(m * nsum, d, generator=g) * 3.0
     r = hy.Residual(x.clone().to(dev))
-    r.add(y.to(dev), torch.tensor([0.7]).to(dev), 1e-6, nsum, 1.0 / nsum)
+    w = torch.rand(d, generator=g) + 0.5 if vector else torch.tensor([0.7])
+    r.add(y.to(dev), w.to(dev), 1e-6, nsum, 1.0 / nsum)
     return r
 
 
@@ -619,7 +620,7 @@ def test_pending_residual_in_the_product(m, k, n, nsum):
     for gated in (False, True):
         out = []
         for dev in ("cpu", DEV):
-            r = _residual(m, k, nsum, dev)
+            r = _residual(m, k, nsum, dev, vector=gated)
             y = hy.linear_rows_gated(r, w.to(dev), ids.to(dev), gate.to(dev), n) if gated else hy.linear(r, w.to(dev))
             out.append((y, r.value()))
         _close(out[1][1], out[0][1], 2e-6, "residual")
@@ -648,3 +649,37 @@ def test_table_experts_without_a_routing_launch(m, top, e, d, f):
 
 def _rand_fixed(m, d):
     return torch.randn(m, d, generator=torch.Generator().manual_seed(m * d))
+
+
+@pytest.mark.parametrize("m,k,n,cap", [(1, 2048, 1003, 0.0), (2, 256, 40, 30.0), (1, 4096, 64, 5.0), (3, 512, 64, 0.0), (1, 250, 64, 2.0)])
+def test_head_with_its_norm(m, k, n, cap):
+    """The final norm (behind a pending residual add or not) in the head's launch; more rows and odd sizes: the separate ops."""
+    w, gw = _rand(n, k, dt=torch.bfloat16, std=k ** -0.5), torch.rand(k) + 0.5
+    for pending in (False, True):
+        out = []
+        for dev in ("cpu", DEV):
+            r = _residual(m, k, 1, dev, vector=True)
+            x = r if pending else r.value()
+            out.append((hy.head_linear(x, gw.to(dev), 1e-6, w.to(dev), cap), r.value()))
+        _close(out[1][0], out[0][0], 2e-3, "logits")
+        _close(out[1][1], out[0][1], 2e-6, "residual")
+
+
+@pytest.mark.parametrize("d,ld,col0", [(2048, 2048, 0), (20, 65, 3), (4096, 4100, 4), (1, 9, 8), (72, 80, 8)])
+def test_embedding_with_its_norm(d, ld, col0):
+    for dt in DTYPES:
+        table, ids, gw = _rand(30, ld, dt=dt), torch.tensor([0, 29, 7, 31, -1], dtype=torch.int32).clamp(0, 29), torch.rand(d) + 0.5
+        for norm in (None, gw):
+            ref = hy.embed_rows(ids, table, col0, d, scale=1.5, norm=norm, eps=1e-6)
+            got = hy.embed_rows(ids.to(DEV), table.to(DEV), col0, d, scale=1.5, norm=norm.to(DEV) if norm is not None else None, eps=1e-6)
+            _close(got, ref, 0.0 if norm is None else 2e-6, "embedding")
+
+
+@pytest.mark.parametrize("b,d,n", [(1, 2048, 5), (2, 4096, 5), (3, 40, 2), (1, 4100, 1), (2, 257, 3)])
+def test_token_shift_with_its_norm(b, d, n):
+    x, gw, prev, mu = _rand(b, d), torch.rand(d) + 0.5, _rand(b, d), torch.rand(n, d)
+    pg = prev.clone().to(DEV)
+    ref = hy.token_shift(hy.RmsInput(x, gw, 1e-6), prev, mu, b, 1)
+    got = hy.token_shift(hy.RmsInput(x.to(DEV), gw.to(DEV), 1e-6), pg, mu.to(DEV), b, 1)
+    _close(got, ref, 2e-6, "mixes")
+    _close(pg, prev, 2e-6, "previous token")
