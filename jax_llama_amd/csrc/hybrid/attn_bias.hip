@@ -488,31 +488,65 @@ __global__ void __launch_bounds__(64) attn_latent_decode_kernel(AttnBias p) {
   }
 }
 
-// grid (H, B, ceil(vdim / 64)), 64 threads: merge the splits (at most 64: lane sp holds split sp's maximum and sum) for
-// one 64-column slice of the head's output
-__global__ void __launch_bounds__(64) attn_bias_merge_kernel(AttnBias p) {
-  const int lane = threadIdx.x, h = blockIdx.x, b = blockIdx.y, c0 = blockIdx.z * 64;
+// The splits of head h of row b merged for column c (at most 64: lane sp holds split sp's maximum and sum), gated. Whole waves.
+JLA_DEV float ab_merge(const AttnBias& p, int b, int h, int c) {
+  const int lane = threadIdx.x & 63;
   const float* w = p.ws + ((size_t)b * p.H + h) * p.splits * (p.vdim + 2);
   float ms = -INFINITY, ls = 0.f;
   if (lane < p.splits) {
     ms = w[(size_t)lane * (p.vdim + 2)];
     ls = w[(size_t)lane * (p.vdim + 2) + 1];
   }
-  const int c = min(c0 + lane, p.vdim - 1);
   float part[64];
 #pragma unroll
-  for (int sp = 0; sp < 64; ++sp) part[sp] = w[(size_t)min(sp, p.splits - 1) * (p.vdim + 2) + 2 + c];  // one round trip
+  for (int s0 = 0; s0 < 64; s0 += 16) {  // one round trip
+    if (s0 < p.splits) {
+#pragma unroll
+      for (int sp = s0; sp < s0 + 16; ++sp) part[sp] = w[(size_t)min(sp, p.splits - 1) * (p.vdim + 2) + 2 + c];
+    }
+  }
+  const float gt = ab_gate(p, b, h, c);
   const float m = wave_max(ls > 0.f ? ms : -INFINITY);
   const float wt = ls > 0.f ? expf(ms - m) : 0.f;  // weight of this lane's split
   const float l = wave_sum(ls * wt);
-  const float gt = ab_gate(p, b, h, c);
   float a = 0.f;
 #pragma unroll
-  for (int sp = 0; sp < 64; ++sp) {  // (a split without keys holds zeros and has weight 0)
-    const float ws = __shfl(wt, sp, 64);
-    a = fmaf(part[sp], sp < p.splits ? ws : 0.f, a);
+  for (int s0 = 0; s0 < 64; s0 += 16) {
+    if (s0 < p.splits) {
+#pragma unroll
+      for (int sp = s0; sp < s0 + 16; ++sp) {  // (a split without keys holds zeros and has weight 0)
+        const float ws = __shfl(wt, sp, 64);
+        a = fmaf(part[sp], sp < p.splits ? ws : 0.f, a);
+      }
+    }
   }
-  if (c0 + lane < p.vdim) ab_out(p, b, h, c, a / l * gt);
+  return a / l * gt;
+}
+
+// grid (H, B, ceil(vdim / 64)), 64 threads: one 64-column slice of the head's output
+__global__ void __launch_bounds__(64) attn_bias_merge_kernel(AttnBias p) {
+  const int lane = threadIdx.x, h = blockIdx.x, b = blockIdx.y, c0 = blockIdx.z * 64;
+  const float v = ab_merge(p, b, h, min(c0 + lane, p.vdim - 1));
+  if (c0 + lane < p.vdim) ab_out(p, b, h, c0 + lane, v);
+}
+
+// grid (H, B), a wave per 64 value columns: the merged head turned by its query's position (rotate_heads: pairs i, i +
+// turn_half), which as a launch of its own costs as much as the merge
+__global__ void __launch_bounds__(64 * AB_MAX_VREG) attn_bias_merge_turn_kernel(AttnBias p) {
+  __shared__ float row[64 * AB_MAX_VREG];
+  const int c = threadIdx.x, h = blockIdx.x, b = blockIdx.y, half = p.turn_half;
+  float sn = 0.f, cs = 1.f;
+  if (c < 2 * half) {  // sine and cosine of position * frequency, the angle formed and reduced in 64-bit
+    const double a = (double)p.turn_pos[b] * p.turn_freq[c < half ? c : c - half];
+    sincosf((float)(a - 6.283185307179586476925 * rint(a * 0.159154943091895335769)), &sn, &cs);
+    sn *= p.turn_sign;
+  }
+  const float v = ab_merge(p, b, h, min(c, p.vdim - 1));
+  row[c] = v;
+  __syncthreads();
+  if (c >= p.vdim) return;
+  const float o = c < 2 * half ? (c < half ? v * cs - row[c + half] * sn : v * cs + row[c - half] * sn) : v;
+  ab_out(p, b, h, c, o * p.turn_gain);
 }
 
 // differential heads: grid (H, B), a wave per 64 value columns; both maps' splits merged, then the head's norm over all of
@@ -851,6 +885,7 @@ int hy_attn_bias(const AttnBias& p, hipStream_t s) {
   if (p.maps != 1 && p.maps != 2) return -10;
   if (p.ldk < p.maps * p.dim) return -8;
   if (p.ldv < p.vdim || (p.gate && p.ldg < (p.gate_cols ? p.H * p.vdim : p.H)) || p.ldo < p.H * p.vdim) return -8;
+  if (p.turn_pos && (p.S != 1 || p.maps != 1 || p.turn_half < 0 || 2 * p.turn_half > p.vdim || (p.turn_half && !p.turn_freq))) return -11;
   if (p.B == 0) return 0;
   if ((long long)p.H * p.maps > 65535 || p.B > 65535) return -4;
   if (p.S == 1) {
@@ -872,6 +907,7 @@ int hy_attn_bias(const AttnBias& p, hipStream_t s) {
     }
     JLA_CHECK_LAUNCH();
     if (p.maps == 2) attn_diff_merge_kernel<<<dim3(p.H, p.B), (p.vdim + 63) / 64 * 64, 0, s>>>(p);
+    else if (p.turn_pos) attn_bias_merge_turn_kernel<<<dim3(p.H, p.B), (p.vdim + 63) / 64 * 64, 0, s>>>(p);
     else attn_bias_merge_kernel<<<dim3(p.H, p.B, (p.vdim + 63) / 64), 64, 0, s>>>(p);
     JLA_CHECK_LAUNCH();
     return 0;

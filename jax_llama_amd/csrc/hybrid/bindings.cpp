@@ -577,7 +577,7 @@ int64_t attn_prefill_ws_bytes(int64_t B, int64_t S, int64_t G, int64_t dim, int6
 void attn_bias(Tensor q, Tensor kc, Tensor vc, Tensor slot, double scale, double softcap, OptT bias, Tensor out,
                int64_t t_cap, OptT ws, int64_t splits, OptT vt_ws, OptT sink, int64_t chunk, OptT head_scale, int64_t window,
                int64_t keep_first, OptT gate, c10::optional<int64_t> vdim, bool gate_cols, int64_t maps, double diff_lambda,
-               double diff_eps, double diff_gain) {
+               double diff_eps, double diff_gain, OptT turn_pos, OptT turn_freq, double turn_sign, double turn_gain) {
   jla::AttnBias p{};
   check(maps == 1 || maps == 2, "attn_bias: one or two maps per head");
   check(q.dim() == 4 && q.size(2) % maps == 0, "attn_bias: q is [B, S, H * maps, dim]");
@@ -640,6 +640,16 @@ void attn_bias(Tensor q, Tensor kc, Tensor vc, Tensor slot, double scale, double
               jla::hy_attn_prefill_ws_bytes(p.B, p.S, p.G, p.dim, p.vdim, p.T, p.cbf16),
           "attn_bias: transposed-value workspace too small");
     p.vt_ws = vt_ws->data_ptr();
+  }
+  if (turn_pos.has_value()) {
+    check(p.S == 1 && maps == 1, "attn_bias: one query per row is turned");
+    p.turn_pos = i32(*turn_pos, "turn_pos", p.B);
+    if (turn_freq.has_value()) {
+      check(2 * turn_freq->numel() <= p.vdim, "attn_bias: more rotated numbers than a head holds");
+      p.turn_freq = f64(*turn_freq, "turn_freq");
+      p.turn_half = turn_freq->numel();
+    }
+    p.turn_sign = turn_sign; p.turn_gain = turn_gain;
   }
   rc(jla::hy_attn_bias(p, stream()), "attn_bias");
 }
@@ -1054,7 +1064,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("vt_ws"), py::arg("sink"), py::arg("chunk") = 0, py::arg("head_scale") = py::none(),
         py::arg("window") = 0, py::arg("keep_first") = 0, py::arg("gate") = py::none(), py::arg("vdim") = py::none(),
         py::arg("gate_cols") = false, py::arg("maps") = 1, py::arg("diff_lambda") = 0.0, py::arg("diff_eps") = 0.0,
-        py::arg("diff_gain") = 1.0);
+        py::arg("diff_gain") = 1.0, py::arg("turn_pos") = py::none(), py::arg("turn_freq") = py::none(),
+        py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);

@@ -299,6 +299,10 @@ struct AttnBias {
                    // d / sqrt(mean(d^2) + diff_eps) * diff_gain with d = a_0 - diff_lambda * a_1 over the head's vdim
                    // numbers; sink, head_scale and bias columns are per query head, gates per output head; the decode
   float diff_lambda, diff_eps, diff_gain;  // partials take B * H * maps * splits * (vdim + 2) floats
+  const int32_t* turn_pos;  // optional, S = 1, one map: [B] positions; every head's output is turned by turn_sign times its
+  const double* turn_freq;  // row's position (numbers i and i + turn_half, [turn_half] frequencies), then times turn_gain
+  int turn_half;
+  float turn_sign, turn_gain;
 };
 int hy_attn_bias(const AttnBias& p, hipStream_t s);
 long long hy_attn_prefill_ws_bytes(int B, int S, int G, int dim, int vdim, int T, int cbf16);

@@ -330,10 +330,9 @@ class RotaryChunkAttention:
         kc, vc = ctx.cache.layer(self.i)
         q = hy.rope_prep(proj, self.bias, ctx.positions, ctx.slot0, ctx.b, ctx.s, self.heads, self.kv_heads, self.dim,
                          self.vdim, kc, vc, self.qk_freq, self.v_freq)
-        a = hy.attn_bias(q, kc, vc, ctx.slot0, self.scale, sink=self.sink, chunk=self.chunk, head_scale=self.temp)
-        if self.v_freq is None and out is None and gain == 1.0:
-            return a
-        return hy.rotate_heads(a, ctx.positions, self.v_freq, self.heads, sign=-1.0, gain=gain, out=out)
+        plain = self.v_freq is None and out is None and gain == 1.0
+        return hy.attn_bias(q, kc, vc, ctx.slot0, self.scale, sink=self.sink, chunk=self.chunk, head_scale=self.temp, out=out,
+                            turn=None if plain else (ctx.positions, self.v_freq, -1.0, gain))
 
     def __call__(self, h, ctx: StepContext) -> torch.Tensor:
         return hy.linear(self.features(h, ctx), self.w_o)

@@ -1073,7 +1073,7 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
               sink: Optional[torch.Tensor] = None, chunk: int = 0,
               head_scale: Optional[torch.Tensor] = None, window: int = 0, keep_first: int = 0,
               gate: Optional[torch.Tensor] = None, vdim: Optional[int] = None, gate_cols: bool = False,
-              out: Optional[torch.Tensor] = None, diff: Optional[DiffMaps] = None) -> torch.Tensor:
+              out: Optional[torch.Tensor] = None, diff: Optional[DiffMaps] = None, turn: Optional[tuple] = None) -> torch.Tensor:
     """Causal attention of ``q [B, S, H, dim]`` (queries at cache slots ``slot + s``) over ``[B, G, T, .]`` caches:
     ``score = q.k * scale``; ``softcap * tanh(score / softcap)`` if ``softcap > 0``; ``+ bias[min(i - j, last), h]``;
     softmax over ``j <= i``, with ``exp(sink[h])`` added to the denominator when ``sink [H]`` is given (a slot without
@@ -1086,13 +1086,18 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
     column ``c`` by ``sigmoid(gate[m, h * vdim + c])``. ``kc`` and ``vc`` may be one tensor (latent
     attention); ``vdim``: the values are the first ``vdim`` columns of ``vc``'s rows. ``diff``: differential heads, ``q
     [B, S, 2 H, dim]`` and ``kc [B, G, T, 2 dim]`` hold the two maps of a head side by side (``sink``, ``head_scale`` and the
-    columns of ``bias`` then count per query head, ``2 h + map``). Returns fp32 ``[B*S, H*vdim]``, or ``out``, a column slice
+    columns of ``bias`` then count per query head, ``2 h + map``). ``turn = (positions, freq, sign, gain)``: the result goes
+    through ``rotate_heads`` (in the same launches for one query per row). Returns fp32 ``[B*S, H*vdim]``, or ``out``, a column slice
     of a wider fp32 or bf16 buffer."""
     b, s, qh, dim = q.shape
     maps = 2 if diff is not None else 1
     h = qh // maps
     g = kc.shape[1]
     vdim = vc.shape[3] if vdim is None else int(vdim)
+    if turn is not None and (s != 1 or maps != 1 or not _gpu(q) or (out is not None and out.dtype != F32)):
+        a = attn_bias(q, kc, vc, slot, scale, softcap, bias, max_kv, sink, chunk, head_scale, window, keep_first, gate, vdim,
+                      gate_cols, None, diff)
+        return rotate_heads(a, turn[0], turn[1], h, sign=turn[2], gain=turn[3], out=out)
     if chunk and window:
         raise ValueError("attn_bias: a block-local mask and a sliding window exclude each other")
     if not _gpu(q):
@@ -1150,7 +1155,9 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
             vt = torch.empty(nb // 2, dtype=BF16, device=q.device)
     e.attn_bias(q.contiguous(), kc, vc, _slot_tensor(slot, q.device), float(scale), float(softcap or 0.0), bias, out,
                 t_cap, ws, splits, vt, sink, int(chunk or 0), head_scale, int(window or 0), int(keep_first or 0), gate,
-                vdim, bool(gate_cols), maps, *((diff.lam, diff.eps, diff.gain) if diff is not None else ()))
+                vdim, bool(gate_cols), maps, *((diff.lam, diff.eps, diff.gain) if diff is not None else (0.0, 0.0, 1.0)),
+                *((turn[0].reshape(-1).to(torch.int32).contiguous(), turn[1], float(turn[2]), float(turn[3])) if turn is not None
+                  else ()))
     return out
 
 

@@ -683,3 +683,23 @@ def test_token_shift_with_its_norm(b, d, n):
     got = hy.token_shift(hy.RmsInput(x.to(DEV), gw.to(DEV), 1e-6), pg, mu.to(DEV), b, 1)
     _close(got, ref, 2e-6, "mixes")
     _close(pg, prev, 2e-6, "previous token")
+
+
+@pytest.mark.parametrize("vdim,half,t,b", [(64, 32, 100, 1), (128, 64, 2100, 2), (80, 10, 70, 1), (128, 0, 40, 3), (40, 20, 5000, 1), (512, 256, 65, 1)])
+def test_decode_attention_turned_by_its_position(vdim, half, t, b):
+    """One query per row: the merge of the splits turns the heads itself; the same sums as the separate launch, turned by the
+    same angles."""
+    h, g, dim = 4, 2, 64
+    q, kc, vc = _rand(b, 1, h, dim), _rand(b, g, t + 3, dim), _rand(b, g, t + 3, vdim)
+    pos = torch.arange(b, dtype=torch.int32) * 1000 + t - 1
+    freq = torch.rand(half, dtype=torch.float64) if half else None
+    slot = torch.tensor([t - 1], dtype=torch.int32)
+    ref = hy.attn_bias(q, kc, vc, slot, 0.2, turn=(pos, freq, -1.0, 0.5))
+    dev = [x.to(DEV) for x in (q, kc, vc, slot)]
+    wide = torch.zeros(b, h * vdim + 4, device=DEV)
+    fg = freq.to(DEV) if half else None
+    hy.attn_bias(*dev, 0.2, out=wide[:, 4:], turn=(pos.to(DEV), fg, -1.0, 0.5))
+    _close(wide[:, 4:], ref, 2e-5, "turned")
+    sep = hy.rotate_heads(hy.attn_bias(*dev, 0.2), pos.to(DEV), fg, h, sign=-1.0, gain=0.5)
+    _close(wide[:, 4:], sep, 1e-6, "turned against the separate launch")
+    assert float(wide[:, :4].abs().max()) == 0.0
