@@ -162,8 +162,15 @@ void set_residual(jla::RowLinear& p, const Tensor& a, const OptT& y, int64_t nsu
 // too), then normed with gain a_norm_w where that is given; f = act, then with ids gelu_tanh * table[ids, col0 ..]. False: not a call of that kernel, nothing was launched.
 bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc, OptT res_w, double eps, OptT x_out, OptT ids,
                 OptT table, int64_t col0, OptT a_norm_w, double a_norm_eps, int64_t act, double act_limit) {
+  const bool one = a_norm_w.has_value() && a_norm_w->numel() == 1 && w.size(-1) != 1;
   jla::RowLinear p = row_linear(a, c10::nullopt, w, out, c10::nullopt, c10::nullopt, c10::nullopt, a.size(0), act, act_limit, 1.0,
-                                c10::nullopt, a_norm_w, a_norm_eps, 0, false);
+                                c10::nullopt, one ? OptT() : a_norm_w, a_norm_eps, 0, false);
+  if (one) {
+    check(!p.a_bf16, "rows_fused: a normed row is float32");
+    p.a_norm_w = f32(*a_norm_w, "a_norm_w");
+    p.a_norm_eps = a_norm_eps;
+    p.a_norm_one = 1;
+  }
   check(act != jla::HY_ACT_SOFTCAP || act_limit > 0, "rows_fused: softcap");
   set_residual(p, a, y, nsum, ysc, res_w, eps, x_out);
   if (ids.has_value()) {
@@ -174,7 +181,7 @@ bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc
     p.mul_V = table->size(0); p.mul_ld = table->size(1); p.mul_col0 = col0;
     check(p.mul_V >= 1, "rows_fused: empty table");
   }
-  if (p.R == 0 || p.N < 1 || !(p.res_y ? jla::hy_rows_gemv_takes_residual(p) : jla::hy_rows_gemv_takes(p))) return false;
+  if (p.R == 0 || p.N < 1 || !(p.res_y || one ? jla::hy_rows_gemv_takes_residual(p) : jla::hy_rows_gemv_takes(p))) return false;
   rc(jla::hy_rows_gemv(p, stream()), "rows_fused");
   return true;
 }

@@ -54,6 +54,7 @@ struct RowLinear {
   float act_alpha;
   int add_out;           // out += act(...) instead of out = (fp32 outputs): a residual add in the epilogue
   // the rest: hy_rows_gemv only
+  int a_norm_one;        // a_norm_w is one number (where hy_rows_gemv_takes_residual)
   int a_div;             // > 1: activation row of linear row r is r / a_div
   const int32_t* tab;    // optional: expert of linear row r = tab[tab_ids[r / tab_top] * tab_top + r % tab_top] ([tab_V, tab_top])
   const int32_t* tab_ids;

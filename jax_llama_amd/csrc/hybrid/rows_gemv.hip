@@ -256,7 +256,14 @@ struct RvRow {
     }
     if (p.a_norm_w) {
 #pragma unroll
-      for (int u = 0; u < V; ++u) g[u] = *reinterpret_cast<const f32x4*>(p.a_norm_w + k[u]);
+      for (int u = 0; u < V; ++u) {
+        if (p.a_norm_one) {
+          const float w0 = p.a_norm_w[0];
+          g[u] = f32x4{w0, w0, w0, w0};
+        } else {
+          g[u] = *reinterpret_cast<const f32x4*>(p.a_norm_w + k[u]);
+        }
+      }
     }
     if (p.res_y) {
       const float* yp = p.res_y + (size_t)src * p.res_nsum * K;
@@ -416,7 +423,7 @@ bool hy_rows_gemv_takes(const RowLinear& p) {
   return p.wbf16 && !p.a_bf16 && !p.out_bf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
          (p.offs || p.row_expert || p.tab || p.E == 1) && p.K % 8 == 0 &&
          p.K >= (p.R > 2 ? 64 : 256) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
-         (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && aligned(p.a_norm_w)));
+         (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && (p.a_norm_one || aligned(p.a_norm_w))));
 }
 
 // One or two normed rows, or with a pending residual add, walk: the plain form would read them twice, the norm ahead of the
@@ -446,6 +453,7 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // rows of a pass: a dense batch's count rounded up; an expert's share of the sorted rows, twice the mean (at least 4)
   const int even = p.offs && p.even_rows > 0 ? p.even_rows : 0;
   const int rows = each ? 1 : (p.offs ? (even ? even : (p.R < 2 * ((p.R + p.E - 1) / p.E) ? p.R : 2 * ((p.R + p.E - 1) / p.E))) : p.R);
+  if (p.a_norm_one && !rv_walks(p, rows)) return -10;
   if (rv_walks(p, rows)) {
     // two tiles per step from a few workgroups for every compute unit on; as many workgroups as are resident (four of 88
     // registers per unit, or two of 156, K > 2048), with equally many steps each

@@ -290,9 +290,9 @@ def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
     pending add and the norm in the product's launch."""
     act, r = ACT_SOFTCAP if cap > 0 else ACT_NONE, x if isinstance(x, Residual) else None
     xv = r.x if r is not None else x
-    if norms_free(xv.shape[0], w) and gain.numel() == xv.shape[1] and xv.is_contiguous():
+    if norms_free(xv.shape[0], w) and gain.numel() in (1, xv.shape[1]) and xv.is_contiguous():
         out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
-        norm = dict(a_norm_w=gain, a_norm_eps=float(eps), act=act, act_limit=float(cap))
+        norm = dict(a_norm_w=gain.reshape(-1), a_norm_eps=float(eps), act=act, act_limit=float(cap))
         if r is not None and r.fusable():
             new = torch.empty_like(xv)
             if ext().rows_fused(xv, w, out, *r.pending, new, **norm):

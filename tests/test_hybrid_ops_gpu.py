@@ -655,7 +655,7 @@ def _rand_fixed(m, d):
 def test_head_with_its_norm(m, k, n, cap):
     """The final norm (behind a pending residual add or not) in the head's launch; more rows and odd sizes: the separate ops."""
     w, gw = _rand(n, k, dt=torch.bfloat16, std=k ** -0.5), torch.rand(k) + 0.5
-    for pending in (False, True):
+    for pending, gw in ((False, gw), (True, gw), (False, gw[:1]), (True, gw[:1])):
         out = []
         for dev in ("cpu", DEV):
             r = _residual(m, k, 1, dev, vector=True)
@@ -703,3 +703,17 @@ def test_decode_attention_turned_by_its_position(vdim, half, t, b):
     sep = hy.rotate_heads(hy.attn_bias(*dev, 0.2), pos.to(DEV), fg, h, sign=-1.0, gain=0.5)
     _close(wide[:, 4:], sep, 1e-6, "turned against the separate launch")
     assert float(wide[:, :4].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("d", [1, 255, 256, 260, 1024, 1028, 2048, 2052, 4096, 4097, 4100, 8192, 8196])
+@pytest.mark.parametrize("off", [0, 1])
+def test_norm_residual_widths(d, off):
+    """The widths at which the row kernel's form changes, and rows that are not 16-byte aligned."""
+    m, nsum = 3, 2
+    flat, x, extra = _rand(m * nsum * d + 1), _rand(m, d), _rand(m, d)
+    y = flat[off:off + m * nsum * d].view(m * nsum, d)
+    yg = flat.to(DEV)[off:off + m * nsum * d].view(m * nsum, d)
+    for w in (torch.tensor([0.7]), torch.rand(d) + 0.5):
+        got = hy.norm_residual_(x.clone().to(DEV), yg, w.to(DEV), 1e-6, nsum, 0.5, extra.to(DEV))
+        _close(got, hy.norm_residual_(x.clone(), y, w, 1e-6, nsum, 0.5, extra), 1e-5, "norm_residual")
+        _close(hy.rms_rows(yg, w.to(DEV), 1e-6), hy.rms_rows(y, w, 1e-6), 1e-5, "rms_rows")
