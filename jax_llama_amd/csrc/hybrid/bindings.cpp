@@ -954,6 +954,13 @@ void lin_scan(int64_t mode, Tensor q, Tensor k, Tensor v, Tensor decay, OptT wri
   p.o = f32w(o, "o");
   p.B = B; p.S = S; p.H = H; p.dim = dim; p.vdim = vdim;
   p.q_scale = q_scale;
+  p.nseg = nseg > INT32_MAX ? INT32_MAX : nseg;
+  const long long floats = jla::hy_scalar_chunk_floats(p);
+  if (floats > 0) {  // (a prompt with scalar gates: chunks on the matrix cores)
+    Tensor ws = torch::empty({floats}, q.options());
+    rc(jla::hy_scalar_chunk(p, reinterpret_cast<float*>(ws.data_ptr()), stream()), "lin_scan");
+    return;
+  }
   check(nseg >= 1 && seg_len >= 1 && nseg * seg_len >= S && (nseg - 1) * seg_len < S, "lin_scan: segments cover the tokens");
   p.nseg = nseg;
   p.seg_len = seg_len;

@@ -1,4 +1,4 @@
-// The gated delta rule of a prompt in chunks of 32 tokens, everything fp32, on v_mfma_f32_16x16x4_f32.
+// The gated delta rule and the scalar-gated memory of a prompt in chunks of 32 tokens, everything fp32, on v_mfma_f32_16x16x4_f32.
 //
 // With P(t, i) the product of the decays of tokens i + 1 .. t of a chunk, G_t = P(t, chunk start) and S0 the state the chunk
 // starts from, the recurrence of delta_rule.hip (S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q) unrolls to
@@ -12,8 +12,8 @@
 //     r = v - G (K S), u = T' r, o = G (Q S) + M u, S = G_last S + K^T (P(last, .) u).
 // What bounds it: (2) is a chain of chunks at the fp32 matrix rate of one SIMD (416 + 64 multiply-adds per token and column:
 // 216 MFMAs of 32 cycles per chunk at dim 128). The token-by-token kernel spends 0.93 us per token on lane exchanges
-// whatever the batch: 2048 tokens of one row, 16 heads of 128 x 128, 1.94 ms -> 0.32; 8 rows of 1500 tokens,
-// 32 heads, 3.50 -> 0.58.
+// whatever the batch: 2048 tokens of one row, 16 heads of 128 x 128, 1.94 ms -> 0.22 (split walk below); 8 rows of 1500
+// tokens, 32 heads, 3.50 -> 0.60. Error of o against 64 bits 1.04e-7 -> 1.15e-7 (split walk; whole 1.3e-7), of the state 7e-8 -> 8e-8.
 // The state stays in the accumulator layout and never leaves its registers: the lane that holds S[16 mb + 4 (l >> 4) + r][l &
 // 15] hands it to the next product as the B operand of k-step r, whose A operand is then column 4 (l >> 4) + r of a 16-wide
 // block: four k-steps per 16-byte LDS read. Likewise r and u. K, Q, T' and M of a chunk go through LDS once per workgroup (64
@@ -26,6 +26,7 @@ namespace jla {
 
 constexpr int DC = 32;                       // tokens of a chunk
 constexpr int DC_WS = 2 * DC * DC + 2 * DC;  // floats per (chunk, head, row): T', M, G, P(last, .)
+constexpr int DC_WS_SCALAR = DC * DC + 2 * DC + 4;  // scalar gates: M, G, P(last, .) write, G_last
 
 JLA_DEV f32x4 mma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -36,7 +37,7 @@ JLA_DEV f32x4 dc_load4(const float* p, bool in) {
 // grid (ceil(chunks / 4), H, B), a wave per chunk. DB = dim / 16.
 template <int DB>
 __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws, int chunks) {
-  __shared__ __attribute__((aligned(16))) float lp[4][DC][DC + 1];  // P(t, i); column DC: G
+  __shared__ __attribute__((aligned(16))) double lp[4][DC][DC + 1];  // P(t, i); column DC: G
   __shared__ __attribute__((aligned(16))) float la[4][DC][DC + 4];  // A
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ch = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
@@ -46,9 +47,12 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
   float* out = ws + (((size_t)b * p.H + h) * chunks + ch) * DC_WS;
 
   // Gram products: token rows as both operands, 16 x 16 blocks on and below the diagonal
-  f32x4 kk[3], qk[3];
+  // (eight short chains per block: a long one would lose a bit to the token-by-token form)
+  f32x4 kk[3], qk[3], kp_[3][8], qp_[3][8];
 #pragma unroll
-  for (int x = 0; x < 3; ++x) kk[x] = qk[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int a = 0; a < 8; ++a) kp_[x][a] = qp_[x][a] = f32x4{0.f, 0.f, 0.f, 0.f};
   const bool in0 = t0 + c < p.S, in1 = t0 + 16 + c < p.S;
   const size_t row0 = ((m0 + c) * p.G + kh) * (16 * DB) + 4 * q, row1 = row0 + (size_t)16 * p.G * (16 * DB);
 #pragma unroll
@@ -57,25 +61,32 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
     const f32x4 q0 = dc_load4(p.qn + row0 + 16 * kb, in0), q1 = dc_load4(p.qn + row1 + 16 * kb, in1);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      kk[0] = mma_f32(k0[r], k0[r], kk[0]);
-      kk[1] = mma_f32(k1[r], k0[r], kk[1]);
-      kk[2] = mma_f32(k1[r], k1[r], kk[2]);
-      qk[0] = mma_f32(q0[r], k0[r], qk[0]);
-      qk[1] = mma_f32(q1[r], k0[r], qk[1]);
-      qk[2] = mma_f32(q1[r], k1[r], qk[2]);
+      const int a = 4 * (kb & 1) + r;
+      kp_[0][a] = mma_f32(k0[r], k0[r], kp_[0][a]);
+      kp_[1][a] = mma_f32(k1[r], k0[r], kp_[1][a]);
+      kp_[2][a] = mma_f32(k1[r], k1[r], kp_[2][a]);
+      qp_[0][a] = mma_f32(q0[r], k0[r], qp_[0][a]);
+      qp_[1][a] = mma_f32(q1[r], k0[r], qp_[1][a]);
+      qp_[2][a] = mma_f32(q1[r], k1[r], qp_[2][a]);
     }
+  }
+  auto total = [](const f32x4 (&v)[8]) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    kk[x] = total(kp_[x]);
+    qk[x] = total(qp_[x]);
   }
   // lane i: the running products from token i on (lane DC: from the chunk's start); tokens past the end keep (decay 1) and
   // write nothing (beta 0)
   const bool mine = lane < DC && t0 + lane < p.S;
   const float g = mine ? p.decay[(m0 + lane) * p.H + h] : 1.f, beta = mine ? p.beta[(m0 + lane) * p.H + h] : 0.f;
   {
-    float run = 1.f;
+    double run = 1.0;  // (64 bits: an error here would be common to a whole token's part of the state)
 #pragma unroll
     for (int t = 0; t < DC; ++t) {
       const float gt = __shfl(g, t, 64);
-      run = (lane < t || lane == DC) ? run * gt : 1.f;
-      if (lane <= DC) lp[wave][t][lane] = lane <= t || lane == DC ? run : 0.f;
+      run = (lane < t || lane == DC) ? run * gt : 1.0;
+      if (lane <= DC) lp[wave][t][lane] = lane <= t || lane == DC ? run : 0.0;
     }
   }
   __builtin_amdgcn_wave_barrier();  // (LDS is the wave's own and in order)
@@ -86,15 +97,16 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = rb + 4 * q + r, i = cb + c;
-      const float pr = lp[wave][t][i], bt = __shfl(beta, t, 64);  // (every lane takes part in the exchange)
-      la[wave][t][i] = i < t ? bt * pr * kk[x][r] : 0.f;
-      out[DC * DC + t * DC + i] = pr * qk[x][r];  // (P is 0 above the diagonal)
+      const double pr = lp[wave][t][i];
+      const float bt = __shfl(beta, t, 64);  // (every lane takes part in the exchange)
+      la[wave][t][i] = i < t ? (float)(pr * bt * kk[x][r]) : 0.f;
+      out[DC * DC + t * DC + i] = (float)(pr * qk[x][r]);  // (P is 0 above the diagonal)
     }
   }
   __builtin_amdgcn_wave_barrier();
   if (lane < DC) {
-    out[2 * DC * DC + lane] = lp[wave][lane][DC];
-    out[2 * DC * DC + DC + lane] = lp[wave][DC - 1][lane];
+    out[2 * DC * DC + lane] = (float)lp[wave][lane][DC];
+    out[2 * DC * DC + DC + lane] = (float)lp[wave][DC - 1][lane];
     // column `lane` of the inverse: x_t = [t == lane] - sum_{i < t} A(t, i) x_i
     float x[DC];
 #pragma unroll
@@ -113,15 +125,15 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
   }
 }
 
-// grid (ceil(vdim / 64), H, B), wave w: value columns 64 blockIdx.x + 16 w ..
+// grid (H, ceil(vdim / 64), B), wave w: value columns 64 blockIdx.y + 16 w ..
 template <int DB>
 __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const float* ws, int chunks) {
   constexpr int D = 16 * DB, LK = D + 4, LT = DC + 4;  // LDS row pitches: the 16 rows of a read fall on all banks
   constexpr int NK = DC * D / 4 / 256;                 // 16-byte pieces of K (and of Q) per thread
   __shared__ __attribute__((aligned(16))) float Ks[DC * LK], Qs[DC * LK], Ts[2 * DC * LT], Gs[2 * DC];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
-  const int h = blockIdx.y, b = blockIdx.z, kh = h / (p.H / p.G);
-  const int j0 = blockIdx.x * 64 + 16 * wave;
+  const int h = blockIdx.x, b = blockIdx.z, kh = h / (p.H / p.G);
+  const int j0 = blockIdx.y * 64 + 16 * wave;
   const bool live = j0 < p.vdim;  // (a wave without columns still stages)
   const int j = live ? j0 + c : 0;
   const float* wsp = ws + ((size_t)b * p.H + h) * chunks * DC_WS;
@@ -200,15 +212,12 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
           qs[mt] = mma_f32(qa[mt][r], S[kb][r], qs[mt]);
         }
     }
-    f32x4 u[2], r_[2];
+    f32x4 u[2], r_[2], g_[2];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
-      const f32x4 gt = *reinterpret_cast<const f32x4*>(&Gs[16 * mt + 4 * q]);
+      g_[mt] = *reinterpret_cast<const f32x4*>(&Gs[16 * mt + 4 * q]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        r_[mt][r] = fmaf(-gt[r], ks[mt][r], v[mt][r]);
-        qs[mt][r] *= gt[r];
-      }
+      for (int r = 0; r < 4; ++r) r_[mt][r] = fmaf(-g_[mt][r], ks[mt][r], v[mt][r]);
       u[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
@@ -220,13 +229,17 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
         for (int r = 0; r < 4; ++r) u[mt] = mma_f32(a[r], r_[kb][r], u[mt]);
       }
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < 2; ++mt) {
+      f32x4 in[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int kb = 0; kb <= mt; ++kb) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(&Ts[(DC + 16 * mt + c) * LT + 16 * kb + 4 * q]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) qs[mt] = mma_f32(a[r], u[kb][r], qs[mt]);
+        for (int r = 0; r < 4; ++r) in[kb] = mma_f32(a[r], u[kb][r], in[kb]);
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) qs[mt][r] = fmaf(qs[mt][r], g_[mt][r], in[0][r] + in[1][r]);
+    }
     const int t0 = ch * DC;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -259,6 +272,298 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
     for (int r = 0; r < 4; ++r) sp[(size_t)(16 * mb + 4 * q + r) * p.vdim] = S[mb][r];
 }
 
+// What a walk of chunks reads and writes, for the delta rule and for scalar gates (mlstm): token m, head h at x + m * ldx + hx *
+// dim, hx the key head.
+struct ChunkWalk {
+  const float* q;
+  int ldq;
+  const float* k;
+  int ldk;
+  const float* v;  // token m, head h at v + m * ldv + h * vdim; a column vdim (ncols = vdim + 1) is 1
+  int ldv;
+  const float* ws;
+  float* state;  // [B, H, dim, ncols]
+  float* o;      // [M, H, ncols]
+  int S, H, heads_per_key, vdim, ncols, chunks;
+  float o_scale;
+};
+
+// The walk where its waves would leave SIMDs idle: the four waves of a workgroup share 16 value columns, each holds a quarter of
+// the key rows of their state (DBW 16-row blocks), and the two products that sum over the key rows (K S and Q S) meet in LDS
+// once per chunk. Operands come straight from memory, a chunk ahead. A chunk's chain per wave at dim 128 is 76 MFMAs instead
+// of 216; 2048 tokens of one row, 16 heads of 128 x 128: 316 -> 218 us with the delta rule's first launch.
+// grid (H, ceil(ncols / 16), B): workgroups go round the XCDs by their id, so a head's columns mostly share one L2.
+// DELTA 0 (scalar gates): u = v, no K S.
+template <int DBW, int DELTA>
+__global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
+  constexpr int D = 64 * DBW, NP = DELTA ? 4 : 2, WS = DELTA ? DC_WS : DC_WS_SCALAR, OFF_M = DELTA ? DC * DC : 0,
+                OFF_G = OFF_M + DC * DC;
+  __shared__ f32x4 red[2][4][NP][64];  // [buffer][wave][Q S of both token tiles, K S of both][lane]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q = lane >> 4;
+  const int h = blockIdx.x, b = blockIdx.z, kh = h / p.heads_per_key;
+  const int j = 16 * blockIdx.y + c, jv = min(j, p.vdim - 1), js = min(j, p.ncols - 1);
+  const int d0 = 16 * DBW * wave;  // this wave's key rows
+  float* sp = p.state + ((size_t)b * p.H + h) * D * p.ncols + js;
+  f32x4 S[DBW];
+#pragma unroll
+  for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[mb][r] = sp[(size_t)(d0 + 16 * mb + 4 * q + r) * p.ncols];
+
+  // a chunk's first rows and workspace (uniform), and this lane's places behind them: only the uniform part moves
+  const float* qp = p.q + (size_t)b * p.S * p.ldq + (size_t)kh * D + d0;
+  const float* kp = p.k + (size_t)b * p.S * p.ldk + (size_t)kh * D + d0;
+  const float* vp = p.v + (size_t)b * p.S * p.ldv + (size_t)h * p.vdim;
+  const float* wp = p.ws + ((size_t)b * p.H + h) * p.chunks * WS;
+  const int mt_o = wave & 1;  // the token tile whose output waves 0 and 1 finish
+  unsigned oq[2], oa[2], ok[2][4], ov[2][4];
+  auto places = [&](int left) {  // rows of a chunk with `left` tokens (further ones repeat the last: their u is 0)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      const int m = min(16 * mt + c, left - 1);
+      oq[mt] = (unsigned)(m * p.ldq + 4 * q);
+      oa[mt] = (unsigned)(m * p.ldk + 4 * q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = min(16 * mt + 4 * q + r, left - 1);
+        ok[mt][r] = (unsigned)(t * p.ldk + c);
+        ov[mt][r] = (unsigned)(t * p.ldv + jv);
+      }
+    }
+  };
+  struct Operands {
+    f32x4 ka[DELTA ? DBW : 1][2], qa[DBW][2], ta[DELTA ? 3 : 1], ma[2], ga[2], wa[2];
+    float kt[DBW][2][4], va[2][4], glast;
+  };
+  const unsigned row = (unsigned)(c * DC + 4 * q);
+  auto fetch = [&](Operands& x, int ch) {  // chunk ch (called in order) on its way to registers
+    if (ch == 0 || (ch + 1) * DC > p.S) places(min(p.S - ch * DC, DC));
+#pragma unroll
+    for (int kb = 0; kb < DBW; ++kb)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        if (DELTA) x.ka[kb][mt] = *reinterpret_cast<const f32x4*>(kp + oa[mt] + 16 * kb);
+        x.qa[kb][mt] = *reinterpret_cast<const f32x4*>(qp + oq[mt] + 16 * kb);
+      }
+    if (DELTA) {
+      x.ta[0] = *reinterpret_cast<const f32x4*>(wp + row);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) x.ta[DELTA ? 1 + kb : 0] = *reinterpret_cast<const f32x4*>(wp + row + 16 * DC + 16 * kb);
+    }
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) x.ma[kb] = *reinterpret_cast<const f32x4*>(wp + OFF_M + 16 * mt_o * DC + row + 16 * kb);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      x.ga[mt] = *reinterpret_cast<const f32x4*>(wp + (unsigned)(4 * q) + OFF_G + 16 * mt);
+      x.wa[mt] = *reinterpret_cast<const f32x4*>(wp + (unsigned)(4 * q) + OFF_G + DC + 16 * mt);
+    }
+    x.glast = DELTA ? wp[OFF_G + DC - 1] : wp[OFF_G + 2 * DC];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x.va[mt][r] = vp[ov[mt][r]];
+#pragma unroll
+        for (int mb = 0; mb < DBW; ++mb) x.kt[mb][mt][r] = kp[ok[mt][r] + 16 * mb];
+      }
+    qp += (size_t)DC * p.ldq;
+    kp += (size_t)DC * p.ldk;
+    vp += (size_t)DC * p.ldv;
+    wp += WS;
+  };
+  auto step = [&](const Operands& x, int ch, int buf) {
+    f32x4 qs[2][4], ks[2][4];  // (short chains)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) qs[mt][a] = ks[mt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < DBW; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          if (DELTA) ks[mt][r] = mma_f32(x.ka[kb][mt][r], S[kb][r], ks[mt][r]);
+          qs[mt][r] = mma_f32(x.qa[kb][mt][r], S[kb][r], qs[mt][r]);
+        }
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      red[buf][wave][mt][lane] = (qs[mt][0] + qs[mt][1]) + (qs[mt][2] + qs[mt][3]);
+      if (DELTA) red[buf][wave][DELTA ? 2 + mt : 0][lane] = (ks[mt][0] + ks[mt][1]) + (ks[mt][2] + ks[mt][3]);
+    }
+    __syncthreads();  // (one per chunk: the other buffer's readers are past it)
+    f32x4 u[2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[mt][r] = ch * DC + 16 * mt + 4 * q + r < p.S ? (j < p.vdim ? x.va[mt][r] : 1.f) : 0.f;
+    if (DELTA) {
+      f32x4 r_[2];
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        constexpr int K0 = DELTA ? 2 : 0;
+        const f32x4 k = (red[buf][0][K0 + mt][lane] + red[buf][1][K0 + mt][lane]) + (red[buf][2][K0 + mt][lane] + red[buf][3][K0 + mt][lane]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) r_[mt][r] = fmaf(-x.ga[mt][r], k[r], u[mt][r]);
+        u[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        u[0] = mma_f32(x.ta[0][r], r_[0][r], u[0]);
+        u[1] = mma_f32(x.ta[DELTA ? 1 : 0][r], r_[0][r], u[1]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[1] = mma_f32(x.ta[DELTA ? 2 : 0][r], r_[1][r], u[1]);
+    }
+    if (wave < 2) {  // o of token tile mt_o
+      f32x4 o = (red[buf][0][mt_o][lane] + red[buf][1][mt_o][lane]) + (red[buf][2][mt_o][lane] + red[buf][3][mt_o][lane]);
+      const f32x4 g = mt_o ? x.ga[1] : x.ga[0];
+      f32x4 in[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) in[r] = mma_f32(x.ma[0][r], u[0][r], f32x4{0.f, 0.f, 0.f, 0.f});
+      if (mt_o) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) in[r] = mma_f32(x.ma[1][r], u[1][r], in[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = fmaf(o[r], g[r], (in[0][r] + in[1][r]) + (in[2][r] + in[3][r]));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = ch * DC + 16 * mt_o + 4 * q + r;
+        if (t < p.S && j < p.ncols) p.o[(((size_t)b * p.S + t) * p.H + h) * p.ncols + j] = DELTA ? o[r] : o[r] * p.o_scale;
+      }
+    }
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[mt][r] *= x.wa[mt][r];
+#pragma unroll
+    for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[mb][r] *= x.glast;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int mb = 0; mb < DBW; ++mb) S[mb] = mma_f32(x.kt[mb][tb][r], u[tb][r], S[mb]);
+  };
+  // two sets of operands in turn: moved from one set to another, a chunk's loads would be waited for at the end of each step
+  Operands x0, x1;
+  fetch(x0, 0);
+  if (p.chunks > 1) fetch(x1, 1);
+  for (int ch = 0; ch < p.chunks; ch += 2) {
+    step(x0, ch, 0);
+    if (ch + 2 < p.chunks) fetch(x0, ch + 2);
+    if (ch + 1 < p.chunks) {
+      step(x1, ch + 1, 1);
+      if (ch + 3 < p.chunks) fetch(x1, ch + 3);
+    }
+  }
+  if (j < p.ncols) {
+#pragma unroll
+    for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sp[(size_t)(d0 + 16 * mb + 4 * q + r) * p.ncols] = S[mb][r];
+  }
+}
+
+// Scalar gates, step (1): one wave per (chunk, head, row). With keep_t and write_t of a token and P(t, i) the product of the keeps
+// of i + 1 .. t:  o_t = (G_t S0^T q_t + sum_{i <= t} P(t, i) write_i (q_t . k_i) v_i) q_scale,  S = G_last S0 + sum_i P(last, i)
+// write_i k_i v_i^T.
+template <int DB>
+__global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws, int chunks) {
+  __shared__ __attribute__((aligned(16))) double lp[4][DC][DC + 1];  // P(t, i) write_i
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ch = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
+  if (ch >= chunks) return;  // (no barrier below: waves share nothing)
+  const int t0 = ch * DC, c = lane & 15, q = lane >> 4;
+  const size_t m0 = (size_t)b * p.S + t0;
+  float* out = ws + (((size_t)b * p.H + h) * chunks + ch) * DC_WS_SCALAR;
+  f32x4 qk[3], part[3][8];  // (eight short chains per block: a long one would lose a bit to the token-by-token form)
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) part[x][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool in0 = t0 + c < p.S, in1 = t0 + 16 + c < p.S;
+  const size_t r0 = m0 + (in0 ? c : 0), r1 = m0 + (in1 ? 16 + c : 0);
+  const int at = h * 16 * DB + 4 * q;
+#pragma unroll
+  for (int kb = 0; kb < DB; ++kb) {
+    const f32x4 k0 = dc_load4(p.k + r0 * p.ldk + at + 16 * kb, in0), k1 = dc_load4(p.k + r1 * p.ldk + at + 16 * kb, in1);
+    const f32x4 q0 = dc_load4(p.q + r0 * p.ldq + at + 16 * kb, in0), q1 = dc_load4(p.q + r1 * p.ldq + at + 16 * kb, in1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int a = 4 * (kb & 1) + r;
+      part[0][a] = mma_f32(q0[r], k0[r], part[0][a]);
+      part[1][a] = mma_f32(q1[r], k0[r], part[1][a]);
+      part[2][a] = mma_f32(q1[r], k1[r], part[2][a]);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < 3; ++x) qk[x] = ((part[x][0] + part[x][1]) + (part[x][2] + part[x][3])) + ((part[x][4] + part[x][5]) + (part[x][6] + part[x][7]));
+  // lane i: the running products behind token i (lane DC: from the chunk's start)
+  const bool mine = lane < DC && t0 + lane < p.S;
+  const size_t mr = m0 + (mine ? lane : 0);
+  const float keep = mine ? p.decay[mr * p.H + h] : 1.f, write = mine ? p.write[mr * p.H + h] : 0.f;
+  const double first = lane < DC ? write : 1.f;
+  double run = first;
+#pragma unroll
+  for (int t = 0; t < DC; ++t) {
+    const float kt = __shfl(keep, t, 64);
+    run = (lane < t || lane == DC) ? run * kt : first;
+    if (lane < DC) lp[wave][t][lane] = lane <= t ? run : 0.0;
+    else if (lane == DC) out[DC * DC + t] = (float)run;
+  }
+  if (lane < DC) out[DC * DC + DC + lane] = (float)run;  // P(last, i) write_i
+  if (lane == DC) out[DC * DC + 2 * DC] = (float)run;    // G_last
+  __builtin_amdgcn_wave_barrier();  // (LDS is the wave's own and in order)
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {  // (block 3, above the diagonal: zeros)
+    const int rb = x == 1 || x == 2 ? 16 : 0, cb = x >= 2 ? 16 : 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = rb + 4 * q + r, i = cb + c;
+      out[t * DC + i] = x < 3 ? (float)(lp[wave][t][i] * qk[x < 3 ? x : 0][r]) : 0.f;
+    }
+  }
+}
+
+// Waves (16 value columns each) from which the walk that keeps a whole column in one wave fills the SIMDs
+constexpr long long DC_WHOLE_WAVES = 1024;
+static bool dc_splits(int B, int H, int ncols) { return (long long)B * H * ((ncols + 15) / 16) < DC_WHOLE_WAVES; }
+
+// Scalar gates in chunks win over the token-by-token scan from a chunk on (16 heads of 128 x 128, one row, us: 32 tokens 28.4 -> 14.5,
+// 777 192 -> 62, 2048 467 -> 139; 8 rows of 2048 2633 -> 746), as long as the scan cannot cut the sequence into many more
+// segments side by side than a walk can make up for (4 heads of 64 x 64, 4096 tokens, 64 segments: 102 -> 206; two passes of
+// 0.7 us per token against 2.1 us per chunk meet at about 21 segments).
+constexpr int DC_SCALAR_MIN_TOKENS = 32, DC_SCALAR_MAX_SEGMENTS = 16;
+
+long long hy_scalar_chunk_floats(const LinScan& p) {
+  auto ok = [](const float* x, int ld) { return ((uintptr_t)x & 15) == 0 && ld % 4 == 0; };
+  if (p.mode != 0 || p.nseg > DC_SCALAR_MAX_SEGMENTS || p.B < 1 || p.S < DC_SCALAR_MIN_TOKENS || p.H < 1 || (p.dim != 64 && p.dim != 128) || p.vdim < 1 || p.H > 65535 ||
+      p.B > 65535 || !p.write || p.ldq < p.H * p.dim || p.ldk < p.H * p.dim || p.ldv < p.H * p.vdim || !ok(p.q, p.ldq) || !ok(p.k, p.ldk))
+    return 0;
+  return (long long)p.B * p.H * ((p.S + DC - 1) / DC) * DC_WS_SCALAR;
+}
+
+int hy_scalar_chunk(const LinScan& p, float* ws, hipStream_t s) {
+  if (hy_scalar_chunk_floats(p) == 0) return -1;
+  if ((uintptr_t)ws & 15) return -2;
+  const int chunks = (p.S + DC - 1) / DC, ncols = p.vdim + 1;
+  const ChunkWalk w{p.q, p.ldq, p.k, p.ldk, p.v, p.ldv, ws, p.state, p.o, p.S, p.H, 1, p.vdim, ncols, chunks, p.q_scale};
+  const dim3 g1((chunks + 3) / 4, p.H, p.B), g2(p.H, (ncols + 15) / 16, p.B);
+  if (p.dim == 128) {
+    scalar_chunk_kernel<8><<<g1, 256, 0, s>>>(p, ws, chunks);
+    chunk_walk_split_kernel<2, 0><<<g2, 256, 0, s>>>(w);
+  } else {
+    scalar_chunk_kernel<4><<<g1, 256, 0, s>>>(p, ws, chunks);
+    chunk_walk_split_kernel<1, 0><<<g2, 256, 0, s>>>(w);
+  }
+  JLA_CHECK_LAUNCH();
+  return 0;
+}
+
 // Tokens from which the chunks win over the token-by-token kernel (two launches and whole chunks against 0.93 us per token)
 constexpr int DC_MIN_TOKENS = 20;  // (16 heads of 128 x 128, one row: 20 tokens 23.6 -> 18.7 us, 64 tokens 55 -> 23)
 
@@ -273,13 +578,17 @@ int hy_delta_chunk(const DeltaScan& p, float* ws, hipStream_t s) {
   if (hy_delta_chunk_floats(p) == 0) return -1;
   if (((uintptr_t)p.kn | (uintptr_t)p.qn | (uintptr_t)ws) & 15) return -2;
   const int chunks = (p.S + DC - 1) / DC;
-  const dim3 g1((chunks + 3) / 4, p.H, p.B), g2((p.vdim + 63) / 64, p.H, p.B);
-  if (p.dim == 128) {
-    delta_chunk_kernel<8><<<g1, 256, 0, s>>>(p, ws, chunks);
-    delta_walk_kernel<8><<<g2, 256, 0, s>>>(p, ws, chunks);
+  const dim3 g1((chunks + 3) / 4, p.H, p.B), g2(p.H, (p.vdim + 63) / 64, p.B);
+  if (p.dim == 128) delta_chunk_kernel<8><<<g1, 256, 0, s>>>(p, ws, chunks);
+  else delta_chunk_kernel<4><<<g1, 256, 0, s>>>(p, ws, chunks);
+  if (dc_splits(p.B, p.H, p.vdim)) {
+    const ChunkWalk w{p.qn, p.G * p.dim, p.kn, p.G * p.dim, p.v, p.H * p.vdim, ws, p.state, p.o, p.S, p.H, p.H / p.G, p.vdim, p.vdim, chunks, 1.f};
+    const dim3 g3(p.H, p.vdim / 16, p.B);
+    if (p.dim == 128) chunk_walk_split_kernel<2, 1><<<g3, 256, 0, s>>>(w);
+    else chunk_walk_split_kernel<1, 1><<<g3, 256, 0, s>>>(w);
   } else {
-    delta_chunk_kernel<4><<<g1, 256, 0, s>>>(p, ws, chunks);
-    delta_walk_kernel<4><<<g2, 256, 0, s>>>(p, ws, chunks);
+    if (p.dim == 128) delta_walk_kernel<8><<<g2, 256, 0, s>>>(p, ws, chunks);
+    else delta_walk_kernel<4><<<g2, 256, 0, s>>>(p, ws, chunks);
   }
   JLA_CHECK_LAUNCH();
   return 0;

@@ -473,6 +473,9 @@ struct LinScan {
   float* seg_decay;
 };
 int hy_lin_scan(const LinScan& p, hipStream_t s);
+// mode 0 in chunks on the matrix cores (delta_chunk.hip): floats of scratch it needs, 0 where it does not apply
+long long hy_scalar_chunk_floats(const LinScan& p);
+int hy_scalar_chunk(const LinScan& p, float* ws, hipStream_t s);
 
 // One token of a matrix-state recurrence with its gates and its gated head norm (rec_step.hip). mode 0: exponential gates
 // (state [B, H, dim, vdim + 1], mstate advanced), 1: time mix, 2: running memory, 3: delta rule. Row b, head h at x + b * ldx +

@@ -129,6 +129,7 @@ def test_attention(dt, shape, own_kv):
                                    dict(b=2, s=20, h=2, g=1, dim=64, vdim=16, taps=4),
                                    dict(b=1, s=64, h=4, g=2, dim=128, vdim=128, taps=4),
                                    dict(b=3, s=97, h=2, g=2, dim=128, vdim=80, taps=4),
+                                   dict(b=8, s=33, h=32, g=4, dim=64, vdim=64, taps=2),  # (whole columns per wave)
                                    dict(b=1, s=321, h=2, g=1, dim=64, vdim=48, taps=2),
                                    dict(b=2, s=9, h=2, g=2, dim=16, vdim=130, taps=1)])
 def test_delta_rule(shape):
@@ -717,3 +718,29 @@ def test_norm_residual_widths(d, off):
         got = hy.norm_residual_(x.clone().to(DEV), yg, w.to(DEV), 1e-6, nsum, 0.5, extra.to(DEV))
         _close(got, hy.norm_residual_(x.clone(), y, w, 1e-6, nsum, 0.5, extra), 1e-5, "norm_residual")
         _close(hy.rms_rows(yg, w.to(DEV), 1e-6), hy.rms_rows(y, w, 1e-6), 1e-5, "rms_rows")
+
+
+@pytest.mark.parametrize("b,s,h,dim,vdim", [(1, 31, 2, 64, 16), (1, 32, 2, 64, 16), (2, 33, 3, 64, 15), (1, 64, 2, 128, 128), (2, 97, 2, 128, 130),
+                                            (1, 300, 4, 64, 1), (1, 65, 2, 96, 40), (1, 1200, 1, 64, 64)])
+def test_scalar_gated_scan_in_chunks(b, s, h, dim, vdim):
+    """The chunked form (and the sizes on both sides of it) against the token loop, and against 64 bits from the same operands:
+    an error of a few fp32 roundings, as the token loop's."""
+    m = b * s
+    proj = _rand(m, 2 * h * dim + h * vdim + 4 - h * vdim % 4)
+    q, k = (proj[:, i * h * dim:(i + 1) * h * dim].unflatten(1, (h, dim)) for i in (0, 1))
+    v = proj[:, 2 * h * dim:2 * h * dim + h * vdim].unflatten(1, (h, vdim))
+    keep, write = torch.rand(m, h) ** 0.1, torch.rand(m, h)
+    state = _rand(b, h, dim, vdim + 1, std=0.3)
+    pg, st_g = proj.to(DEV), state.clone().to(DEV)
+    st, o64 = state.double(), torch.empty(b, s, h, vdim + 1, dtype=torch.float64)
+    q64, k64 = (x.double().reshape(b, s, h, dim) for x in (q, k))
+    v64 = torch.cat([v.double().reshape(b, s, h, vdim), torch.ones(b, s, h, 1, dtype=torch.float64)], -1)
+    for t in range(s):
+        ke, wr = (x.double().reshape(b, s, h)[:, t, :, None, None] for x in (keep, write))
+        st = st * ke + wr * k64[:, t, :, :, None] * v64[:, t, :, None]
+        o64[:, t] = (st * q64[:, t, :, :, None]).sum(2) * 0.25
+    gq, gk = (pg[:, i * h * dim:(i + 1) * h * dim].unflatten(1, (h, dim)) for i in (0, 1))
+    gv = pg[:, 2 * h * dim:2 * h * dim + h * vdim].unflatten(1, (h, vdim))
+    o = hy.mlstm_scan(gq, gk, gv, keep.to(DEV), write.to(DEV), st_g, b, s, 0.25)
+    assert float((o.cpu().double().reshape(o64.shape) - o64).norm() / o64.norm()) < 5e-7
+    assert float((st_g.cpu().double() - st).norm() / st.norm()) < 5e-7
