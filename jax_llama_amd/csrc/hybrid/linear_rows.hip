@@ -505,16 +505,26 @@ JLA_DEV void rt_sort(int* cnt, int* cur, int R, int top, int E, const int32_t* r
     offs[E] = run;
   }
   __syncthreads();
-  for (int r = threadIdx.x; r < R; r += blockDim.x) {
-    const int e = row_expert[r];
-    const int pos = atomicAdd(&cur[e], 1);
-    sort_tok[pos] = r / top;
-    sort_dst[pos] = r;
-    if (sort_w) sort_w[pos] = row_w[r];
+  constexpr int U = 4;  // rows in flight per thread
+  for (int r0 = threadIdx.x; r0 < R; r0 += U * blockDim.x) {
+    int e[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = row_expert[min(r0 + u * (int)blockDim.x, R - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int r = r0 + u * (int)blockDim.x;
+      if (r >= R) break;
+      const int pos = atomicAdd(&cur[e[u]], 1);
+      sort_tok[pos] = r / top;
+      sort_dst[pos] = r;
+      if (sort_w) sort_w[pos] = row_w[r];
+    }
   }
 }
 
-__global__ void __launch_bounds__(256) route_table_kernel(const int32_t* ids, const int32_t* table, int V, int M, int top,
+// One workgroup: up to 1024 threads, four rows in flight each. Us, 256 threads with one row -> now: 32768 rows 77 -> 35, 4096
+// rows 11 -> 6.2, 16384 rows of 64 experts 43 -> 21.
+__global__ void __launch_bounds__(1024) route_table_kernel(const int32_t* ids, const int32_t* table, int V, int M, int top,
                                                           int E, int32_t* row_expert, int32_t* row_tok,
                                                           int32_t* sort_tok, int32_t* sort_dst, int32_t* offs) {
   __shared__ int cnt[RT_MAX_E + 1];
@@ -522,15 +532,25 @@ __global__ void __launch_bounds__(256) route_table_kernel(const int32_t* ids, co
   const int R = M * top;
   for (int e = threadIdx.x; e <= E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int r = threadIdx.x; r < R; r += blockDim.x) {
-    const int m = r / top, c = r - m * top;
-    int id = ids[m];
-    id = id < 0 || id >= V ? 0 : id;
-    int e = table[(size_t)id * top + c];
-    e = e < 0 || e >= E ? 0 : e;
-    row_expert[r] = e;
-    row_tok[r] = m;
-    atomicAdd(&cnt[e], 1);
+  constexpr int U = 4;
+  for (int r0 = threadIdx.x; r0 < R; r0 += U * blockDim.x) {
+    int id[U], e[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      id[u] = ids[min(r0 + u * (int)blockDim.x, R - 1) / top];
+      id[u] = id[u] < 0 || id[u] >= V ? 0 : id[u];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = table[(size_t)id[u] * top + min(r0 + u * (int)blockDim.x, R - 1) % top];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int r = r0 + u * (int)blockDim.x;
+      if (r >= R) break;
+      e[u] = e[u] < 0 || e[u] >= E ? 0 : e[u];
+      row_expert[r] = e[u];
+      row_tok[r] = r / top;
+      atomicAdd(&cnt[e[u]], 1);
+    }
   }
   rt_sort(cnt, cur, R, top, E, row_expert, nullptr, sort_tok, sort_dst, nullptr, offs);
 }
@@ -539,7 +559,7 @@ int hy_route_table(const int32_t* ids, const int32_t* table, int V, int M, int t
                    int32_t* row_tok, int32_t* sort_tok, int32_t* sort_dst, int32_t* offs, hipStream_t s) {
   if (M < 0 || top < 1 || E < 1 || E > RT_MAX_E || V < 1) return -1;
   if (M == 0) return 0;
-  route_table_kernel<<<1, 256, 0, s>>>(ids, table, V, M, top, E, row_expert, row_tok, sort_tok, sort_dst, offs);
+  route_table_kernel<<<1, (long long)M * top > 256 ? 1024 : 256, 0, s>>>(ids, table, V, M, top, E, row_expert, row_tok, sort_tok, sort_dst, offs);
   JLA_CHECK_LAUNCH();
   return 0;
 }

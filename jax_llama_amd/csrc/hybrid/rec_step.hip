@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
       lc[t] = keep * qs;
       e[0] = wk * qs;
       e[1] = keep * zs * qs;
-      st[(size_t)t * ncols + vdim] = fmaf(keep, zs, wk);  // (this thread is its only reader)
+      st[(size_t)t * ncols + vdim] = fmaf(keep, zs, wk);  // (no other thread uses what it holds)
     }
   } else if (MODE == RS_TIMEMIX) {
     const float pre = p.pre[(size_t)b * p.ldpre + (size_t)h * dim + td];
