@@ -744,3 +744,21 @@ def test_scalar_gated_scan_in_chunks(b, s, h, dim, vdim):
     o = hy.mlstm_scan(gq, gk, gv, keep.to(DEV), write.to(DEV), st_g, b, s, 0.25)
     assert float((o.cpu().double().reshape(o64.shape) - o64).norm() / o64.norm()) < 5e-7
     assert float((st_g.cpu().double() - st).norm() / st.norm()) < 5e-7
+
+
+@pytest.mark.parametrize("b,s,h,g,dim,vdim", [(17, 31, 2, 1, 64, 64), (16, 32, 2, 1, 128, 128), (16, 33, 6, 3, 64, 128), (2, 257, 4, 2, 128, 64),
+                                              (1, 511, 2, 2, 64, 64), (1, 527, 2, 2, 64, 64), (8, 64, 2, 1, 80, 64)])
+def test_delta_preparation_in_runs(b, s, h, g, dim, vdim):
+    """Convolutions, unit norms and gates of a prompt in runs of tokens (and on both sides of that form) against the CPU op, the
+    tail of the call before included."""
+    c, taps = 2 * g * dim + h * vdim, 4
+    proj = _rand(b * s, c + h * vdim + 2 * h + 4)
+    conv_w, tail = _rand(c, taps, std=0.6), _rand(b, c, taps - 1)
+    a_log, dt_bias = torch.rand(h) - 1.0, torch.randn(h)
+    tail_g = tail.clone().to(DEV)
+    width = c + h * vdim + 2 * h
+    ref = hy.delta_prep(proj[:, :width], b, s, h, g, dim, vdim, conv_w, tail, a_log, dt_bias)
+    got = hy.delta_prep(proj.to(DEV)[:, :width], b, s, h, g, dim, vdim, conv_w.to(DEV), tail_g, a_log.to(DEV), dt_bias.to(DEV))
+    for r, x, name in zip(ref, got, ("q", "k", "v", "beta", "decay")):
+        _close(x, r, 2e-5, name)
+    _close(tail_g, tail, 0.0, "conv tail")
