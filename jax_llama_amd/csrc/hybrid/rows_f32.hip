@@ -1,8 +1,8 @@
 // The fp32 form of a prompt's row-gathered, expert-grouped linears: split products on the bf16 matrix cores
 // (kernels/gemm_f32x3.h) with the epilogues of a row linear. Us, exact-f32 MFMA tiles (lr_gemm_kernel) -> here, rows x K x N:
-// 9 x 2048 x 8224 89 -> 29; 200 x 2048 x 8224 145 -> 72; 400 x 5632 x 2048 358 -> 74; 400 x 2048 x 5632 gated 248 -> 171; 4000 x
-// 5632 x 2048 824 -> 484 (191 TFLOP/s). Relative error against 64 bits at K 2048: 8.1e-7 -> 7.0e-7 (in one split), 2.5e-7 to
-// 4e-7 where K is split.
+// 9 x 2048 x 8224 89 -> 31; 200 x 2048 x 8224 145 -> 71; 400 x 5632 x 2048 358 -> 77; 400 x 2048 x 5632 gated 248 -> 165; 4000 x
+// 5632 x 2048 824 -> 478 (193 TFLOP/s). Relative error against 64 bits, 400 x 5632 x 2048: 1.34e-6 -> 4.1e-7, of positive
+// numbers 1.13e-6 -> 1.2e-7 (K split).
 #include "../kernels/gemm_f32x3.h"
 #include "hy_util.h"
 #include "hybrid.h"

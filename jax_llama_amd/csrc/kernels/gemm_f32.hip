@@ -2,8 +2,8 @@
 // `precision`, jax_test.py:433 runs the parity harness with precision='highest').
 //
 // y[M, N] = x[M, K] @ W[N, K]^T with fp32 inputs, fp32 accumulation and fp32 output. Rows of whole 16-byte pieces run as
-// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 146, 100 567 -> 222,
-// 600 1780 -> 1028, 6000 15484 -> 8514); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
+// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 163, 100 567 -> 209,
+// 600 1780 -> 925, 6000 15484 -> 8211); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
 // k-ordered fmaf chain, no xf32 shortcut on gfx950): 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64
 // (2 x 2 MFMA tiles), K staged 32 deep through LDS in k-major images ([k][row]) so a lane's fragment element (row l & 31, k
 // l >> 5) is one conflict-free ds_read_b32.

@@ -1,16 +1,24 @@
-// fp32 products on the bf16 matrix cores: every operand is the sum of three bf16 numbers (8 + 8 + 8 mantissa bits, cut, not
-// rounded, so the split is exact), and a product is the six largest of the nine partial products, smallest first,
+// fp32 products on the bf16 matrix cores: every operand is the sum of three bf16 numbers, each the nearest to what the ones
+// before it leave (8 bits each, so the split is exact), and a product is the six largest of the nine partial products, smallest
+// first,
 //     a w = lo hi + hi lo + mid mid + mid hi + hi mid + hi hi,
-// in one fp32 accumulator. What is left out is below 2^-23 of each product, and an accumulator is rounded 6 times per 32
-// products where the fp32 matrix instruction rounds it once per 2: against 64 bits the result is the closer one (600 x
-// 32000 x 4096: 1.15e-6 -> 0.71e-6). v_mfma_f32_16x16x32_bf16 does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle, so six of them
-// are 2.7 times its rate.
+// in one fp32 accumulator. |mid| is below 2^-8 and |lo| below 2^-17 of the operand, so what is left out (mid lo, lo mid, lo lo)
+// is below 2^-24 of the product, half an fp32 rounding, and of either sign: parts that are cut instead of rounded all have the
+// operand's sign, and a sum of products of one sign comes out low (1 x 32000 x 4096, positive numbers, error against 64 bits:
+// exact-f32 MFMA 9.9e-7, cut parts 3.2e-6, all of it one-sided, nearest parts 3.2e-7). v_mfma_f32_16x16x32_bf16 adds 8
+// products at a time to the accumulator, rounded to nearest: 24 roundings per 32 products here, 5 of 6 of them of a small
+// addend, where the fp32 matrix instruction rounds once per product (600 x 4000 x 4096, either sign: 1.14e-6 -> 0.57e-6; 70 x
+// 512 x 8: 5.3e-8 -> 3.1e-8). It does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle, so six of them are 2.7 times
+// its rate.
 //
 // One workgroup: BM x 128 outputs, four waves of BM / 2 x 64; K advances 32 per step. The operands are split on their way
-// from registers to LDS (5.5 vector instructions per number, beside the products of the step before), so memory holds plain
+// from registers to LDS (6 vector instructions per number, beside the products of the step before), so memory holds plain
 // fp32 and nothing is prepared ahead; loads are two steps ahead. LDS: per operand and part [rows][4 cells of
 // 16 B], cell c of row r at c ^ ((r >> 2) & 3): the 16 lanes of a fragment read fall on all 64 banks.
-// An infinity or NaN makes its remainder NaN: the workgroup notices and computes its tile again with plain fp32 FMAs.
+// Where the split does not hold, the workgroup computes its tile again on the fp32 matrix instruction (600 x 4000 x 4096 with
+// a NaN in every tile: 138 -> 285 us). An infinity or NaN among the operands, or a number that rounds up to an infinity,
+// makes its remainder NaN and so every result it enters (a sum past the largest number shows there too); a piece of a row
+// whose numbers are all below 2^-95 would have parts that bf16's smallest step of 2^-133 cuts.
 #pragma once
 #include "common.h"
 #include "row_tiles.h"
@@ -36,28 +44,23 @@ struct F3Rows {
 constexpr int F3_BN = 128, F3_BK = 32;
 constexpr int F3_RESIDENT = 512;  // workgroups resident at once: two per compute unit
 
+constexpr unsigned F3_EXP = 0x70000000u;  // set in some number of a row piece unless all of them are below 2^-95
+
 struct F3Part {
   u32x4 hi, mid, lo;
 };
 
-// 8 numbers -> their three parts, packed; bad: whether one of them is no number
-JLA_DEV F3Part f3_split(const f32x4 x, const f32x4 y, bool& bad) {
-  unsigned h[8], m[8], l[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float v = i < 4 ? x[i & 3] : y[i & 3];
-    h[i] = __float_as_uint(v) & 0xffff0000u;
-    const float r = v - __uint_as_float(h[i]);
-    bad |= r != r;
-    m[i] = __float_as_uint(r) & 0xffff0000u;
-    l[i] = __float_as_uint(r - __uint_as_float(m[i]));
-  }
+// 8 numbers -> their three parts, packed; any: the bits that some number so far has
+JLA_DEV F3Part f3_split(const f32x4 x, const f32x4 y, unsigned& any) {
   F3Part p;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {  // bytes 2, 3 of each pair
-    p.hi[i] = __builtin_amdgcn_perm(h[2 * i + 1], h[2 * i], 0x07060302u);
-    p.mid[i] = __builtin_amdgcn_perm(m[2 * i + 1], m[2 * i], 0x07060302u);
-    p.lo[i] = __builtin_amdgcn_perm(l[2 * i + 1], l[2 * i], 0x07060302u);
+  for (int i = 0; i < 4; ++i) {
+    const float v0 = i < 2 ? x[2 * (i & 1)] : y[2 * (i & 1)], v1 = i < 2 ? x[2 * (i & 1) + 1] : y[2 * (i & 1) + 1];
+    any |= __float_as_uint(v0) | __float_as_uint(v1);
+    p.hi[i] = pack2bf(v0, v1);
+    const float r0 = v0 - __uint_as_float(p.hi[i] << 16), r1 = v1 - __uint_as_float(p.hi[i] & 0xffff0000u);
+    p.mid[i] = pack2bf(r0, r1);
+    p.lo[i] = pack2bf(r0 - __uint_as_float(p.mid[i] << 16), r1 - __uint_as_float(p.mid[i] & 0xffff0000u));
   }
   return p;
 }
@@ -108,7 +111,11 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
   u32x4* const lw = lds + 3 * AU;
   const int cell = sch ^ ((srow >> 2) & 3);  // (64 u does not change it)
   const int rcell = q ^ ((c >> 2) & 3);
-  bool bad = false;
+  unsigned ta[NA], tw[NW];  // bits of this thread's row pieces
+#pragma unroll
+  for (int u = 0; u < NA; ++u) ta[u] = 0;
+#pragma unroll
+  for (int u = 0; u < NW; ++u) tw[u] = 0;
   struct Step {
     f32x4 a[NA][2], w[NW][2];
   };
@@ -128,7 +135,7 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
   auto stage = [&](const Step& f, int buf) {  // split and into LDS
 #pragma unroll
     for (int u = 0; u < NA; ++u) {
-      const F3Part s = f3_split(f.a[u][0] * sc[u], f.a[u][1] * sc[u], bad);
+      const F3Part s = f3_split(f.a[u][0] * sc[u], f.a[u][1] * sc[u], ta[u]);
       u32x4* d = la + buf * F3_BUF + (64 * u + srow) * 4 + cell;
       d[0] = s.hi;
       d[AU] = s.mid;
@@ -136,7 +143,7 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
     }
 #pragma unroll
     for (int u = 0; u < NW; ++u) {
-      const F3Part s = f3_split(f.w[u][0], f.w[u][1], bad);
+      const F3Part s = f3_split(f.w[u][0], f.w[u][1], tw[u]);
       u32x4* d = lw + buf * F3_BUF + (64 * u + srow) * 4 + cell;
       d[0] = s.hi;
       d[WU] = s.mid;
@@ -201,27 +208,48 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
     }
   }
   // lane: rows 16 i + c of the wave's BM / 2, columns (weight tile rows) 16 j + 4 q + 0..3
-  if (__syncthreads_or(bad)) {
-    const float* ar[MT];
+  bool again = false;
+#pragma unroll
+  for (int u = 0; u < NA; ++u) again |= (ta[u] & 0x7fffffffu) && !(ta[u] & F3_EXP);
+#pragma unroll
+  for (int u = 0; u < NW; ++u) again |= (tw[u] & 0x7fffffffu) && !(tw[u] & F3_EXP);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) again |= !(fabsf(acc[j][i][r]) < INFINITY);
+  if (__syncthreads_or(again)) {
+    const float *ar[MT], *wr_[4];
     float as[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      ar[i] = arow(wr * (BM / 2) + 16 * i + c);
+      ar[i] = arow(wr * (BM / 2) + 16 * i + c) + 4 * q;
       as[i] = ascale(wr * (BM / 2) + 16 * i + c);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      wr_[j] = wrow(64 * wc + 16 * j + c) + 4 * q;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* wv = wrow(64 * wc + 16 * j + 4 * q + r);
-        for (int k = F3_BK * t0; k < min(K, F3_BK * t1); ++k) {
-          const float b = wv[k];
+      for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int k1 = min(K, F3_BK * t1);
+#pragma unroll 2
+    for (int k = F3_BK * t0; k < k1; k += 16) {  // lane group q: numbers k + 4 q .. + 3 of both operands, one per instruction
+      const bool in = k + 4 * q < K;
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      f32x4 a[MT], w[4];
 #pragma unroll
-          for (int i = 0; i < MT; ++i) acc[j][i][r] = fmaf(ar[i][k] * as[i], b, acc[j][i][r]);
-        }
-      }
+      for (int j = 0; j < 4; ++j) w[j] = in ? *reinterpret_cast<const f32x4*>(wr_[j] + k) : z;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[i] = in ? *reinterpret_cast<const f32x4*>(ar[i] + k) * as[i] : z;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][r], a[i][r], acc[j][i], 0, 0, 0);
+    }
   }
   // results leave through the wave's own LDS, 32 rows x 64 accumulator columns at a time: the activation is one small loop
   // and rows leave in whole lines. 16-byte chunk x of row r lies at x ^ (r & 15)

@@ -520,7 +520,7 @@ def test_few_rows_on_the_matrix_cores(r, k, n, act):
 def test_fp32_rows_as_split_products(counts, k, n, act):
     """fp32 tiles on the bf16 matrix cores: both row tiles, one and several K splits, K that ends inside a step, ragged and
     empty experts, gathered, scaled and scattered rows, the add into the output. Against 64 bits: every product is exact to
-    2^-23 and the fp32 sum of k of them rounds like any other (5e-6 of the summed magnitudes, as for the exact-f32 path)."""
+    2^-24 and the fp32 sum of k of them rounds like any other (5e-6 of the summed magnitudes, as for the exact-f32 path)."""
     e, r = len(counts), sum(counts)
     gated = hy.act_gated(act)
     g = torch.Generator().manual_seed(k + n + act + r)
@@ -545,6 +545,36 @@ def test_fp32_rows_as_split_products(counts, k, n, act):
                              0.0, 0, add)
         got = out.double() - (0.5 if add else 0.0)
         assert float((got - ref).abs().max() / ref.abs().max()) < 5e-6
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 512, 8), (70, 512, 64), (600, 4000, 256), (600, 4000, 4096)])
+def test_fp32_split_products_are_not_one_sided(m, n, k):
+    """fp32 products on the bf16 matrix cores against 64 bits. A product loses less than 2^-24 of itself, of either sign, and
+    sums round to nearest: products of one sign must not come out low on average (parts cut instead of rounded lose 4.7e-7 at
+    k 8 and 8e-7 at k 4096), and no error grows past sqrt(roundings) / 3 of half a step, 3 k / 4 of them (a chain of fp32
+    FMAs has k). Operands far below 1 keep their bits: rows of 2^-118 as rows of 1."""
+    from jax_llama_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(k)
+    a, b = torch.randn(m, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    hard = lambda bits: torch.tensor(bits, dtype=torch.int32, device=DEV).view(torch.float32)  # noqa: E731
+    bound = 2.0 ** -24 * (1.0 + (0.75 * k) ** 0.5 / 3 ** 0.5)
+    forms = [ops.linear_f32] + ([hy.linear] if k >= 256 else [])
+    for f in forms:
+        for x, w in ((a.abs(), b.abs()), (a.abs() * 2.0 ** -118, b.abs()), (a.abs(), b.abs() * 2.0 ** -118)):
+            y, ref = f(x, w).double(), x.double() @ w.double().t()
+            assert float((y - ref).norm() / ref.norm()) < bound
+            assert abs(float(((y - ref) / ref).mean())) < 1.5e-7
+        for bits in (0x3F80FFFF, 0x3F807FC0):  # the numbers whose cut (rounded) parts leave out most: k equal products
+            if k > 8:
+                continue
+            x, w = (hard(bits).expand(r, k).contiguous() for r in (m, n))
+            ref = k * float(hard(bits)) ** 2
+            assert float((f(x, w).double() - ref).abs().max()) / ref < 1.3e-7  # (2^-24 left out, 2^-24 rounded)
+    x, w = a.clone(), b * 1e-3
+    x[3, 2] = x[m - 1, k - 1] = 3.4e38  # rounds up to an infinity in bf16
+    for f in forms:
+        y, ref = f(x, w).double(), x.double() @ w.double().t()
+        assert float(((y - ref).abs() / (x.double().abs() @ w.double().abs().t())).max()) < 1e-6 * k ** 0.5
 
 
 def test_fp32_split_products_keep_infinities():
