@@ -8,7 +8,11 @@
 // rows the instruction's 16 A rows are G output columns times 16 / G neighbouring K ranges and its 16 B columns the G
 // activation rows times the same ranges: the diagonal blocks of the product hold the sums, a load covers G rows x 1024 / G
 // contiguous bytes, and a workgroup needs only G columns -- enough workgroups for every compute unit from 1024 columns on.
-// The waves of a workgroup deal the K steps among themselves, U in flight each, and sum their blocks through LDS.
+// The waves of a workgroup deal the K steps among themselves, U in flight each, and sum their blocks through LDS. The sums
+// of four MFMAs, and then the waves', are added in 64 bits: the matrix instruction cuts the small ones of the 8 products that it adds at a
+// time at 24 bits of the largest, and that already is the error of the vector unit's six lane exchanges (against 64 bits, one row
+// of K 2048 | 7168: vector unit 7.5e-8 | 9.5e-8; one chain per wave and the waves one by one 9.7e-8 | 13.9e-8; now 6.4e-8 |
+// 6.9e-8; 64 rows of 8 experts, K 7168: 9.5e-8, 25.4e-8, 7.0e-8).
 // Us before -> after, weights in no cache, 1 | 8 | 33 rows: K 2048 x N 5152 11.1 -> 7.7 | 27.4 -> 10.7 | 54 -> 21; 4096 x 10304 42.6 ->
 // 19.1 | 62.6 -> 26.6 | 108 -> 59; 2048 x 32000 49.6 -> 24.3 (5.4 TB/s) | 99 -> 29.4 | 67 -> 63; gated 2048 x 5632 17.2 -> 12.4 |
 // 44.8 -> 16.0 | 82 -> 34; both products of 2 of 8 experts (4096 x 7168) for 1 | 8 tokens 105 -> 68 | 403 -> 230. With one output element
@@ -55,6 +59,19 @@ JLA_DEV float rv_table(const RowLinear& p, int r, int col) {
   return p.mul_bf16 ? bf2f(reinterpret_cast<const bf16_t*>(p.mul_table)[at]) : reinterpret_cast<const float*>(p.mul_table)[at];
 }
 
+// The sum of N partial sums, rounded once
+template <int N>
+JLA_DEV float rv_sum(const float (&f)[N]) {
+  double s[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) s[i] = f[i];
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) s[i] += s[i + n];
+  return (float)s[0];
+}
+
 // output column col of linear row r from its accumulators
 JLA_DEV void rv_store(const RowLinear& p, int r, int col, float g, float v) {
   float* dst = reinterpret_cast<float*>(p.out) + (size_t)(p.dst_idx ? p.dst_idx[r] : r) * p.ldo + col;
@@ -72,6 +89,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   constexpr int SEG = 16 / G;                // neighbouring K ranges of one MFMA
   constexpr int H = G == 16 ? 2 : 1;         // MFMAs of a K step (G = 16: the two halves of a 128-byte line)
   constexpr int STEP = 32 * SEG * H;         // K of a step
+  constexpr int RUN = 4 / H;                 // steps (four MFMAs) whose sums share an fp32 accumulator
   constexpr int ROWS = G * MT;               // rows of a pass
   __shared__ f32x4 red[WAVES][NT * MT][64];
   __shared__ float stat[NORM ? WAVES : 1][16];
@@ -135,11 +153,13 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
       for (int w = 0; w < WAVES; ++w) ss += stat[w][c % G];
       xs[0] = 1.f / sqrtf(ss / (float)K + p.a_norm_eps);
     }
-    f32x4 acc[NT][MT];
+    double acc[NT][MT][4];  // (64 bits cost nothing beside the stream: 8 rows, K 7168 x N 4096: 16.7 -> 17.0 us)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][m][i] = 0.0;
 
     for (int s0 = wave; s0 < steps; s0 += WAVES * U) {
       u32x4 wf[U][H][NT];
@@ -158,46 +178,62 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
           }
         }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int s = s0 + WAVES * u;
-        if (s >= steps) break;  // (wave-uniform)
+      for (int u0 = 0; u0 < U; u0 += RUN) {
+        if (s0 + WAVES * u0 >= steps) break;  // (wave-uniform)
+        f32x4 part[NT][MT];  // this run's own sums
 #pragma unroll
-        for (int h = 0; h < H; ++h) {
-          const bool ragged = STEP * s + 32 * (h + 1) * SEG > K;  // (wave-uniform: some lane's range ends before K does)
-          const bool in = STEP * s + 32 * h + k0 < K;
-          if (ragged) {
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int t = 0; t < NT; ++t) wf[u][h][t] = in ? wf[u][h][t] : u32x4{0, 0, 0, 0};
-          }
+          for (int m = 0; m < MT; ++m) part[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            f32x4 a = xa[u][h][m], b = xb[u][h][m];
+        for (int u = u0; u < (u0 + RUN < U ? u0 + RUN : U); ++u) {
+          const int s = s0 + WAVES * u;
+          if (s >= steps) break;  // (wave-uniform)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              a[i] *= xs[m];
-              b[i] *= xs[m];
+          for (int h = 0; h < H; ++h) {
+            const bool ragged = STEP * s + 32 * (h + 1) * SEG > K;  // (wave-uniform: some lane's range ends before K does)
+            const bool in = STEP * s + 32 * h + k0 < K;
+            if (ragged) {
+#pragma unroll
+              for (int t = 0; t < NT; ++t) wf[u][h][t] = in ? wf[u][h][t] : u32x4{0, 0, 0, 0};
             }
-            if (NORM) {
-              const float* gw = p.a_norm_w + at(s, h);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+              f32x4 a = xa[u][h][m], b = xb[u][h][m];
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
-                a[i] *= gw[i];
-                b[i] *= gw[4 + i];
+                a[i] *= xs[m];
+                b[i] *= xs[m];
               }
-            }
-            u32x4 x = rv_round8(a, b);
-            if (ragged) x = in ? x : u32x4{0, 0, 0, 0};
+              if (NORM) {
+                const float* gw = p.a_norm_w + at(s, h);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) acc[t][m] = mfma16x16x32(wf[u][h][t], x, acc[t][m]);
+                for (int i = 0; i < 4; ++i) {
+                  a[i] *= gw[i];
+                  b[i] *= gw[4 + i];
+                }
+              }
+              u32x4 x = rv_round8(a, b);
+              if (ragged) x = in ? x : u32x4{0, 0, 0, 0};
+#pragma unroll
+              for (int t = 0; t < NT; ++t) part[t][m] = mfma16x16x32(wf[u][h][t], x, part[t][m]);
+            }
           }
         }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t][m][i] += part[t][m][i];
       }
     }
     // lane: row (B column) c, columns (A rows) 4 q + 0..3 of tile t
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) red[wave][t * MT + m][lane] = acc[t][m];
+      for (int m = 0; m < MT; ++m)
+        red[wave][t * MT + m][lane] = f32x4{(float)acc[t][m][0], (float)acc[t][m][1], (float)acc[t][m][2], (float)acc[t][m][3]};
     __syncthreads();
     // one output element per thread: the epilogue's code, which a short launch has to fetch, stays small
     constexpr int PER = G * G;  // (column, row) pairs of a tile
@@ -207,21 +243,17 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
       const int row = 16 * m + x, col = G * (blockIdx.x * (gated ? NT / 2 : NT) + to) + y;
       if (row >= nr || col >= N) continue;
       const int slot = (gated ? 2 * to : to) * MT + m;
-      float g = 0.f, v = 0.f;
+      auto total = [&](int at) {
+        float f[SEG * WAVES];
 #pragma unroll
-      for (int sg = 0; sg < SEG; ++sg) {  // the diagonal block of range sg
-        const int l = 16 * (G / 4 * sg + y / 4) + G * sg + x;
+        for (int sg = 0; sg < SEG; ++sg) {  // the diagonal block of range sg
+          const int l = 16 * (G / 4 * sg + y / 4) + G * sg + x;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-          g += red[w][slot][l][y % 4];
+          for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[w][at][l][y % 4];
         }
-      }
-      if (gated) {
-#pragma unroll
-        for (int sg = 0; sg < SEG; ++sg)
-#pragma unroll
-          for (int w = 0; w < WAVES; ++w) v += red[w][slot + MT][16 * (G / 4 * sg + y / 4) + G * sg + x][y % 4];
-      }
+        return rv_sum(f);
+      };
+      const float g = total(slot), v = gated ? total(slot + MT) : 0.f;
       rv_store(p, r0 + row, col, g, v);
     }
     __syncthreads();
@@ -394,21 +426,15 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
     if (tid < outs) {
       const int y = tid % G, to = tid / G / nr, x = tid / G - to * nr, slot = gated ? 2 * to : to;
       const int col = G * (tg * (gated ? NT / 2 : NT) + to) + y;
-      float g = 0.f, v = 0.f;
+      auto total = [&](int at) {
+        float f[4 * WAVES];
 #pragma unroll
-      for (int sg = 0; sg < 4; ++sg) {  // the diagonal block of K range sg
-        const int l = 20 * sg + x;
+        for (int sg = 0; sg < 4; ++sg)  // the diagonal block of K range sg
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-          g += red[buf][w][slot][l][y];
-        }
-      }
-      if (gated) {
-#pragma unroll
-        for (int sg = 0; sg < 4; ++sg)
-#pragma unroll
-          for (int w = 0; w < WAVES; ++w) v += red[buf][w][slot + 1][20 * sg + x][y];
-      }
+          for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[buf][w][at][20 * sg + x][y];
+        return rv_sum(f);
+      };
+      const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
       if (col < N) rv_store(p, r0 + x, col, g, v);
     }
   }
