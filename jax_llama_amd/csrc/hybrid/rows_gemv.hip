@@ -441,13 +441,14 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 }
 
 // up to 64 rows, and up to 32 of a wide output, whose tiles fill the chip (64 rows x 32000 columns, K 2048: 70 us on the
-// tiles, 82 here); one or two rows of a short K are over before the waves' sum pays (K 64: 3.2 against 3.6 us)
-constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 16;
+// tiles, 82 here); one or two rows of a short K are over before the waves' sum pays (K 64: 3.2 against 3.6 us). Rows with an
+// expert of their own and no offsets: as many as the vector unit's form takes.
+constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 2;
 
 bool hy_rows_gemv_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return p.wbf16 && !p.a_bf16 && !p.out_bf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
-         (p.offs || p.row_expert || p.tab || p.E == 1) && p.K % 8 == 0 &&
+         (p.offs || p.tab || (p.row_expert ? p.R <= HY_GEMV_MAX_R : p.E == 1)) && p.K % 8 == 0 &&
          p.K >= (p.R > 2 ? 64 : 256) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
          (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && (p.a_norm_one || aligned(p.a_norm_w))));
 }
@@ -521,24 +522,20 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
     else if (nt == 2) RV_RUN(G, 2, 1, 2, NORM); \
     else RV_RUN(G, 4, 1, 2, NORM);      \
   } while (0)
-#define RV_G(NORM)                \
-  do {                            \
-    if (G == 4) RV_NT(4, NORM);   \
-    else if (G == 8) RV_NT(8, NORM); \
-    else RV_NT(16, NORM);         \
-  } while (0)
   if (mt == 4) {
     if (nt == 2) RV_RUN(16, 2, 4, 1, 0);
     else RV_RUN(16, 4, 4, 1, 0);
   } else if (mt == 2) {
     if (nt == 2) RV_RUN(16, 2, 2, 2, 0);
     else RV_RUN(16, 4, 2, 1, 0);
-  } else if (p.a_norm_w) {
-    RV_G(1);
+  } else if (G == 4) {
+    if (p.a_norm_w) RV_NT(4, 1);  // (at most two rows)
+    else RV_NT(4, 0);
+  } else if (G == 8) {
+    RV_NT(8, 0);
   } else {
-    RV_G(0);
+    RV_NT(16, 0);
   }
-#undef RV_G
 #undef RV_NT
 #undef RV_RUN
   JLA_CHECK_LAUNCH();

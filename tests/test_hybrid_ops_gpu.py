@@ -514,6 +514,28 @@ def test_few_rows_on_the_matrix_cores(r, k, n, act):
     _close(run(w, new(), dst_=idx, offs_=offs, a_idx=idx), per, 2e-5, "expert-sorted")
 
 
+def test_few_rows_refuse_what_the_vector_unit_refuses():
+    """A norm on the way in for more than two rows, an expert per row for more than GEMV_MAX_R rows without offsets: refused on
+    the host before any launch; the row counts below are taken."""
+    most, k, n = hy.ext().GEMV_MAX_R, 512, 64
+    w, gain = _rand(3, n, k, dt=torch.bfloat16).to(DEV), torch.ones(k, device=DEV)
+
+    def call(r, wt, row_expert=None, norm=None):
+        x, out = torch.randn(r, k, device=DEV), torch.empty(r, n, device=DEV)
+        ex = torch.zeros(r, dtype=torch.int32, device=DEV) if row_expert else None
+        hy.ext().linear_rows(x, None, wt, out, None, None, ex, r, 0, 0.0, 1.0, None, norm, 1e-5, 0, False)
+
+    for r in (1, 2):
+        call(r, w[0], norm=gain)
+    call(most, w, row_expert=True)
+    for r in (3, 8, 9, 16, 17):
+        with pytest.raises(RuntimeError):
+            call(r, w[0], norm=gain)
+    for r in (most + 1, 64):
+        with pytest.raises(RuntimeError):
+            call(r, w, row_expert=True)
+
+
 @pytest.mark.parametrize("k,n", [(2048, 1030), (4104, 516), (7168, 516)])
 def test_few_rows_sum_as_exactly_as_the_vector_unit(k, n):
     """Products of bf16 numbers are exact in fp32, so a row's error against 64 bits is its summation's alone. On the vector unit
