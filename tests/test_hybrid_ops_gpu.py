@@ -680,6 +680,38 @@ def test_one_token_recurrence(kind, b, h, dim, vdim):
         _close(x, r, 2e-5, name)
 
 
+@pytest.mark.parametrize("kind,bound", [("timemix", 1.11e-7), ("running", 8.95e-8), ("delta", 1.11e-7)])
+def test_one_token_recurrence_as_exact_as_the_scans(kind, bound):
+    """The read-out of one token and its norm against 64 bits. The bounds are what the scan and the norm kernel lose on the same
+    operands (two chains of 8 key rows per lane, three lane exchanges, the norm): the one-launch form may lose no more."""
+    b, h, dim = 8, 16, 128
+    g = torch.Generator(device=DEV).manual_seed(1)
+    R = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    S, gate, w = R(b, h, dim, dim) * 0.3, R(b, h * dim), torch.rand(h * dim, generator=g, device=DEV) + 0.5
+    q, k, v, pre = (R(b, h, dim) for _ in range(4))
+    w0, u = R(h * dim) - 2.0, R(h * dim) * 0.3
+    S64, q64, k64, v64 = S.double(), q.double(), k.double(), v.double()
+    if kind == "timemix":
+        y = hy.timemix_memory(q, k, v, pre, w0, u, S, b, 1, gate, w, 1e-6)
+        o = ((S64 + u.double().reshape(h, dim, 1) * k64[..., None] * v64[:, :, None]) * q64[..., None]).sum(2)
+    elif kind == "running":
+        fb, room = w0 + 4.0, torch.rand(h * dim, generator=g, device=DEV)
+        y = hy.running_memory(q, v, pre, fb, room, S, b, 1, w, 1e-6)
+        wr = (room.double() * torch.sigmoid(-(pre.double().reshape(b, -1) + fb.double()))).reshape(b, h, dim, 1)
+        o = ((S64 * (1.0 - wr) + wr * v64[:, :, None]) * torch.nn.functional.silu(q64)[..., None]).sum(2)
+    else:
+        unit = lambda x: x / x.norm(dim=-1, keepdim=True)  # noqa: E731
+        q, k, w = unit(q) * dim ** -0.5, unit(k), w[:dim].contiguous()
+        q64, k64, beta, decay = q.double(), k.double(), torch.sigmoid(R(b, h)), torch.sigmoid(R(b, h) + 2.0)
+        y = hy.delta_memory(q, k, v, beta, decay, S, b, 1, gate, w, 1e-6)
+        S64 = S64 * decay.double()[..., None, None]
+        S64 = S64 + k64[..., None] * (beta.double()[..., None] * (v64 - (S64 * k64[..., None]).sum(2)))[:, :, None]
+        o = (S64 * q64[..., None]).sum(2)
+    o = o / (o.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt() * w.double().reshape(-1, dim)
+    o = o.reshape(b, -1) * (torch.nn.functional.silu(gate.double()) if kind != "running" else 1.0)
+    assert float((y.double() - o).norm() / o.norm()) < bound
+
+
 def _residual(m, d, nsum, dev, seed=5, vector=False):
     g = torch.Generator().manual_seed(seed)
     x, y = torch.randn(m, d, generator=g), torch.randn(m * nsum, d, generator=g) * 3.0
