@@ -12,8 +12,13 @@
 //     r = v - G (K S), u = T' r, o = G (Q S) + M u, S = G_last S + K^T (P(last, .) u).
 // What bounds it: (2) is a chain of chunks at the fp32 matrix rate of one SIMD (416 + 64 multiply-adds per token and column:
 // 216 MFMAs of 32 cycles per chunk at dim 128). The token-by-token kernel spends 0.93 us per token on lane exchanges
-// whatever the batch: 2048 tokens of one row, 16 heads of 128 x 128, 1.94 ms -> 0.22 (split walk below); 8 rows of 1500
-// tokens, 32 heads, 3.50 -> 0.60. Error of o against 64 bits 1.04e-7 -> 1.15e-7 (split walk; whole 1.3e-7), of the state 7e-8 -> 8e-8.
+// whatever the batch: 2048 tokens of one row, 16 heads of 128 x 128, 1.94 ms -> 0.24 (split walk below); 8 rows of 1500
+// tokens, 32 heads, 3.50 -> 0.60.
+// Error against 64 bits, output | state, token by token -> here: those two 1.05e-7 -> 1.02e-7 | 7.4e-8 -> 6.9e-8 and 1.05e-7 ->
+// 1.03e-7 | 7.2e-8 -> 6.9e-8; scalar gates, 777 tokens 1.07e-7 -> 1.02e-7 | 7.1e-8 -> 6.6e-8. It takes short chains: sums over key
+// rows in blocks of 16, what a chunk's tokens add to the state in four parts, the diagonal of T' after everything below it, Gram
+// products and decays in 64 bits (one chain each, as the products fall, gave 1.32e-7 | 8.2e-8; the walk with scalar gates pays 8 %
+// for it, the delta rule's nothing).
 // The state stays in the accumulator layout and never leaves its registers: the lane that holds S[16 mb + 4 (l >> 4) + r][l &
 // 15] hands it to the next product as the B operand of k-step r, whose A operand is then column 4 (l >> 4) + r of a 16-wide
 // block: four k-steps per 16-byte LDS read. Likewise r and u. K, Q, T' and M of a chunk go through LDS once per workgroup (64
@@ -25,10 +30,18 @@
 namespace jla {
 
 constexpr int DC = 32;                       // tokens of a chunk
-constexpr int DC_WS = 2 * DC * DC + 2 * DC;  // floats per (chunk, head, row): T', M, G, P(last, .)
+constexpr int DC_WS = 2 * DC * DC + 3 * DC;  // floats per (chunk, head, row): T' below its diagonal, M, G, P(last, .), beta
 constexpr int DC_WS_SCALAR = DC * DC + 2 * DC + 4;  // scalar gates: M, G, P(last, .) write, G_last
 
 JLA_DEV f32x4 mma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// element r of the sum of eight chains
+JLA_DEV double dc_total(const f32x4 (&v)[8], int r) {
+  double s[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = (double)v[i][r] + v[i + 4][r];
+  return (s[0] + s[1]) + (s[2] + s[3]);
+}
 
 JLA_DEV f32x4 dc_load4(const float* p, bool in) {
   return in ? *reinterpret_cast<const f32x4*>(p) : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -48,7 +61,7 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
 
   // Gram products: token rows as both operands, 16 x 16 blocks on and below the diagonal
   // (eight short chains per block: a long one would lose a bit to the token-by-token form)
-  f32x4 kk[3], qk[3], kp_[3][8], qp_[3][8];
+  f32x4 kp_[3][8], qp_[3][8];
 #pragma unroll
   for (int x = 0; x < 3; ++x)
 #pragma unroll
@@ -69,12 +82,6 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
       qp_[1][a] = mma_f32(q1[r], k0[r], qp_[1][a]);
       qp_[2][a] = mma_f32(q1[r], k1[r], qp_[2][a]);
     }
-  }
-  auto total = [](const f32x4 (&v)[8]) { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); };
-#pragma unroll
-  for (int x = 0; x < 3; ++x) {
-    kk[x] = total(kp_[x]);
-    qk[x] = total(qp_[x]);
   }
   // lane i: the running products from token i on (lane DC: from the chunk's start); tokens past the end keep (decay 1) and
   // write nothing (beta 0)
@@ -99,14 +106,16 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
       const int t = rb + 4 * q + r, i = cb + c;
       const double pr = lp[wave][t][i];
       const float bt = __shfl(beta, t, 64);  // (every lane takes part in the exchange)
-      la[wave][t][i] = i < t ? (float)(pr * bt * kk[x][r]) : 0.f;
-      out[DC * DC + t * DC + i] = (float)(pr * qk[x][r]);  // (P is 0 above the diagonal)
+      const double kk = dc_total(kp_[x], r), qk = dc_total(qp_[x], r);
+      la[wave][t][i] = i < t ? (float)(pr * bt * kk) : 0.f;
+      out[DC * DC + t * DC + i] = (float)(pr * qk);  // (P is 0 above the diagonal)
     }
   }
   __builtin_amdgcn_wave_barrier();
   if (lane < DC) {
     out[2 * DC * DC + lane] = (float)lp[wave][lane][DC];
     out[2 * DC * DC + DC + lane] = (float)lp[wave][DC - 1][lane];
+    out[2 * DC * DC + 2 * DC + lane] = beta;
     // column `lane` of the inverse: x_t = [t == lane] - sum_{i < t} A(t, i) x_i
     float x[DC];
 #pragma unroll
@@ -120,7 +129,7 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
           if (i + u < t) s[u] = fmaf(-a[u], x[i + u], s[u]);
       }
       x[t] = (s[0] + s[1]) + (s[2] + s[3]);
-      out[t * DC + lane] = x[t] * beta;
+      out[t * DC + lane] = lane < t ? x[t] * beta : 0.f;
     }
   }
 }
@@ -130,45 +139,49 @@ template <int DB>
 __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const float* ws, int chunks) {
   constexpr int D = 16 * DB, LK = D + 4, LT = DC + 4;  // LDS row pitches: the 16 rows of a read fall on all banks
   constexpr int NK = DC * D / 4 / 256;                 // 16-byte pieces of K (and of Q) per thread
-  __shared__ __attribute__((aligned(16))) float Ks[DC * LK], Qs[DC * LK], Ts[2 * DC * LT], Gs[2 * DC];
+  __shared__ __attribute__((aligned(16))) float Ks[DC * LK], Qs[DC * LK], Ts[2 * DC * LT], Gs[3 * DC];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
   const int h = blockIdx.x, b = blockIdx.z, kh = h / (p.H / p.G);
   const int j0 = blockIdx.y * 64 + 16 * wave;
   const bool live = j0 < p.vdim;  // (a wave without columns still stages)
   const int j = live ? j0 + c : 0;
   const float* wsp = ws + ((size_t)b * p.H + h) * chunks * DC_WS;
-  float* sp = p.state + ((size_t)b * p.H + h) * D * p.vdim + j;
+  float* const sp = p.state + ((size_t)b * p.H + h) * D * p.vdim;
+  const unsigned at_s = (unsigned)(4 * q * p.vdim + j);  // (this lane's place; the rows of a block differ by uniform steps)
 
   f32x4 S[DB];
 #pragma unroll
   for (int mb = 0; mb < DB; ++mb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[mb][r] = sp[(size_t)(16 * mb + 4 * q + r) * p.vdim];
+    for (int r = 0; r < 4; ++r) S[mb][r] = (sp + (size_t)(16 * mb + r) * p.vdim)[at_s];
 
+  // a lane's places behind a chunk's first rows (uniform)
+  const int krow = tid / (D / 4);  // piece u of a thread: row krow + 1024 / D u
+  const unsigned at_k = (unsigned)(krow * p.G * D + 4 * (tid % (D / 4))), at_v = (unsigned)(4 * q * p.H * p.vdim + j);
+  const size_t kstep = (size_t)(1024 / D) * p.G * D, vstep = (size_t)p.H * p.vdim;
+  const float* const kbase = p.kn + ((size_t)b * p.S * p.G + kh) * D;
+  const float* const qbase = p.qn + ((size_t)b * p.S * p.G + kh) * D;
+  const float* const vbase = p.v + ((size_t)b * p.S * p.H + h) * p.vdim;
+  float* const obase = p.o + ((size_t)b * p.S * p.H + h) * p.vdim;
   f32x4 pk[NK], pq[NK], pt[2];
   float pg = 0.f, pv[2][4];
   auto fetch = [&](int ch) {  // chunk ch on its way to registers
-    const int t0 = ch * DC;
-    const size_t m0 = (size_t)b * p.S + t0;
+    const int left = p.S - ch * DC;
 #pragma unroll
     for (int u = 0; u < NK; ++u) {
-      const int e = u * 256 + tid, row = e / (D / 4), c4 = e % (D / 4);
-      const bool in = t0 + row < p.S;
-      const size_t at = ((m0 + row) * p.G + kh) * D + 4 * c4;
-      pk[u] = dc_load4(p.kn + at, in);
-      pq[u] = dc_load4(p.qn + at, in);
+      const size_t up = (size_t)ch * DC * p.G * D + u * kstep;
+      pk[u] = dc_load4(kbase + up + at_k, krow + 1024 / D * u < left);
+      pq[u] = dc_load4(qbase + up + at_k, krow + 1024 / D * u < left);
     }
     const float* w = wsp + (size_t)ch * DC_WS;
 #pragma unroll
     for (int u = 0; u < 2; ++u) pt[u] = *reinterpret_cast<const f32x4*>(w + 4 * (u * 256 + tid));
-    if (tid < 2 * DC) pg = w[2 * DC * DC + tid];
+    if (tid < 3 * DC) pg = w[2 * DC * DC + tid];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * mt + 4 * q + r;
-        pv[mt][r] = t0 + t < p.S ? p.v[((m0 + t) * p.H + h) * p.vdim + j] : 0.f;
-      }
+      for (int r = 0; r < 4; ++r)
+        pv[mt][r] = 16 * mt + 4 * q + r < left ? (vbase + ((size_t)ch * DC + 16 * mt + r) * vstep)[at_v] : 0.f;
   };
   fetch(0);
   for (int ch = 0; ch < chunks; ++ch) {
@@ -184,7 +197,7 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
       const int e = 4 * (u * 256 + tid), row = e / DC, col = e % DC;  // rows 0 .. 31: T', 32 .. 63: M
       *reinterpret_cast<f32x4*>(&Ts[row * LT + col]) = pt[u];
     }
-    if (tid < 2 * DC) Gs[tid] = pg;
+    if (tid < 3 * DC) Gs[tid] = pg;
     float v[2][4];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -193,31 +206,31 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
     __syncthreads();
     if (ch + 1 < chunks) fetch(ch + 1);
     if (!live) continue;
-    f32x4 ks[2], qs[2];
+    // X S of both token tiles, X = K or Q: each block of key rows a chain of its own
+    auto times_state = [&](const float* X, f32x4 (&xs)[2]) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) ks[mt] = qs[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < DB; ++kb) {
-      f32x4 ka[2], qa[2];
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        ka[mt] = *reinterpret_cast<const f32x4*>(&Ks[(16 * mt + c) * LK + 16 * kb + 4 * q]);
-        qa[mt] = *reinterpret_cast<const f32x4*>(&Qs[(16 * mt + c) * LK + 16 * kb + 4 * q]);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int kb = 0; kb < DB; ++kb) {
+        f32x4 a[2], blk[2];
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-          ks[mt] = mma_f32(ka[mt][r], S[kb][r], ks[mt]);
-          qs[mt] = mma_f32(qa[mt][r], S[kb][r], qs[mt]);
+          a[mt] = *reinterpret_cast<const f32x4*>(&X[(16 * mt + c) * LK + 16 * kb + 4 * q]);
+          blk[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-    }
-    f32x4 u[2], r_[2], g_[2];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) blk[mt] = mma_f32(a[mt][r], S[kb][r], blk[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) xs[mt] = kb ? xs[mt] + blk[mt] : blk[mt];
+      }
+    };
+    f32x4 u[2], r_[2];
+    times_state(Ks, r_);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
-      g_[mt] = *reinterpret_cast<const f32x4*>(&Gs[16 * mt + 4 * q]);
+      const f32x4 g = *reinterpret_cast<const f32x4*>(&Gs[16 * mt + 4 * q]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) r_[mt][r] = fmaf(-g_[mt][r], ks[mt][r], v[mt][r]);
+      for (int r = 0; r < 4; ++r) r_[mt][r] = fmaf(-g[r], r_[mt][r], v[mt][r]);
       u[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
@@ -228,26 +241,32 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
 #pragma unroll
         for (int r = 0; r < 4; ++r) u[mt] = mma_f32(a[r], r_[kb][r], u[mt]);
       }
+    // (the diagonal of T', beta, last: what the earlier tokens take away is small beside it)
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
-      f32x4 in[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      const f32x4 bt = *reinterpret_cast<const f32x4*>(&Gs[2 * DC + 16 * mt + 4 * q]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[mt][r] = fmaf(bt[r], r_[mt][r], u[mt][r]);
+    }
+    const int t0 = ch * DC;
+    f32x4 qs[2];
+    times_state(Qs, qs);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      const f32x4 g = *reinterpret_cast<const f32x4*>(&Gs[16 * mt + 4 * q]);
+      f32x4 in[4];
 #pragma unroll
       for (int kb = 0; kb <= mt; ++kb) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(&Ts[(DC + 16 * mt + c) * LT + 16 * kb + 4 * q]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) in[kb] = mma_f32(a[r], u[kb][r], in[kb]);
+        for (int r = 0; r < 4; ++r) in[r] = mma_f32(a[r], u[kb][r], kb ? in[r] : f32x4{0.f, 0.f, 0.f, 0.f});
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) qs[mt][r] = fmaf(qs[mt][r], g_[mt][r], in[0][r] + in[1][r]);
-    }
-    const int t0 = ch * DC;
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int t = t0 + 16 * mt + 4 * q + r;
-        if (t < p.S) p.o[(((size_t)b * p.S + t) * p.H + h) * p.vdim + j] = qs[mt][r];
+        const float o = fmaf(qs[mt][r], g[r], (in[0][r] + in[1][r]) + (in[2][r] + in[3][r]));
+        if (t0 + 16 * mt + 4 * q + r < p.S) (obase + ((size_t)t0 + 16 * mt + r) * vstep)[at_v] = o;
       }
+    }
     const float glast = Gs[DC - 1];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
@@ -257,19 +276,23 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
     }
 #pragma unroll
     for (int mb = 0; mb < DB; ++mb) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[mb][r] *= glast;
+      f32x4 add[4];  // what the tokens add, four short chains: one onto S itself would round S at every token
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[mb] = mma_f32(Ks[(16 * tb + 4 * q + r) * LK + 16 * mb + c], u[tb][r], S[mb]);
+        for (int r = 0; r < 4; ++r)
+          add[r] = mma_f32(Ks[(16 * tb + 4 * q + r) * LK + 16 * mb + c], u[tb][r], tb ? add[r] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[mb][r] = fmaf(S[mb][r], glast, (add[0][r] + add[1][r]) + (add[2][r] + add[3][r]));
     }
   }
   if (!live) return;
+  float* to = sp;
+  asm volatile("" : "+s"(to));  // (the addresses are formed again: kept through the walk they would take 64 registers)
 #pragma unroll
   for (int mb = 0; mb < DB; ++mb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sp[(size_t)(16 * mb + 4 * q + r) * p.vdim] = S[mb][r];
+    for (int r = 0; r < 4; ++r) (to + (size_t)(16 * mb + r) * p.vdim)[at_s] = S[mb][r];
 }
 
 // What a walk of chunks reads and writes, for the delta rule and for scalar gates (mlstm): token m, head h at x + m * ldx + hx *
@@ -332,7 +355,7 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     }
   };
   struct Operands {
-    f32x4 ka[DELTA ? DBW : 1][2], qa[DBW][2], ta[DELTA ? 3 : 1], ma[2], ga[2], wa[2];
+    f32x4 ka[DELTA ? DBW : 1][2], qa[DBW][2], ta[DELTA ? 3 : 1], ma[2], ga[2], wa[2], ba[DELTA ? 2 : 1];
     float kt[DBW][2][4], va[2][4], glast;
   };
   const unsigned row = (unsigned)(c * DC + 4 * q);
@@ -356,6 +379,7 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     for (int mt = 0; mt < 2; ++mt) {
       x.ga[mt] = *reinterpret_cast<const f32x4*>(wp + (unsigned)(4 * q) + OFF_G + 16 * mt);
       x.wa[mt] = *reinterpret_cast<const f32x4*>(wp + (unsigned)(4 * q) + OFF_G + DC + 16 * mt);
+      if (DELTA) x.ba[DELTA ? mt : 0] = *reinterpret_cast<const f32x4*>(wp + (unsigned)(4 * q) + OFF_G + 2 * DC + 16 * mt);
     }
     x.glast = DELTA ? wp[OFF_G + DC - 1] : wp[OFF_G + 2 * DC];
 #pragma unroll
@@ -414,6 +438,11 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) u[1] = mma_f32(x.ta[DELTA ? 2 : 0][r], r_[1][r], u[1]);
+      // (the diagonal of T', beta, last: what the earlier tokens take away is small beside it)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[mt][r] = fmaf(x.ba[DELTA ? mt : 0][r], r_[mt][r], u[mt][r]);
     }
     if (wave < 2) {  // o of token tile mt_o
       f32x4 o = (red[buf][0][mt_o][lane] + red[buf][1][mt_o][lane]) + (red[buf][2][mt_o][lane] + red[buf][3][mt_o][lane]);
@@ -437,16 +466,18 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) u[mt][r] *= x.wa[mt][r];
-#pragma unroll
-    for (int mb = 0; mb < DBW; ++mb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[mb][r] *= x.glast;
+    f32x4 add[DBW][4];  // what the tokens add, four short chains: one onto S itself would round S at every token
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int mb = 0; mb < DBW; ++mb)
 #pragma unroll
-        for (int mb = 0; mb < DBW; ++mb) S[mb] = mma_f32(x.kt[mb][tb][r], u[tb][r], S[mb]);
+        for (int r = 0; r < 4; ++r) add[mb][r] = mma_f32(x.kt[mb][tb][r], u[tb][r], tb ? add[mb][r] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        S[mb][r] = fmaf(S[mb][r], x.glast, (add[mb][0][r] + add[mb][1][r]) + (add[mb][2][r] + add[mb][3][r]));
   };
   // two sets of operands in turn: moved from one set to another, a chunk's loads would be waited for at the end of each step
   Operands x0, x1;
@@ -472,7 +503,7 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
 // of i + 1 .. t:  o_t = (G_t S0^T q_t + sum_{i <= t} P(t, i) write_i (q_t . k_i) v_i) q_scale,  S = G_last S0 + sum_i P(last, i)
 // write_i k_i v_i^T.
 template <int DB>
-__global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws, int chunks) {
+__global__ void __launch_bounds__(256, 2) scalar_chunk_kernel(LinScan p, float* ws, int chunks) {
   __shared__ __attribute__((aligned(16))) double lp[4][DC][DC + 1];  // P(t, i) write_i
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ch = blockIdx.x * 4 + wave, h = blockIdx.y, b = blockIdx.z;
@@ -480,7 +511,7 @@ __global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws,
   const int t0 = ch * DC, c = lane & 15, q = lane >> 4;
   const size_t m0 = (size_t)b * p.S + t0;
   float* out = ws + (((size_t)b * p.H + h) * chunks + ch) * DC_WS_SCALAR;
-  f32x4 qk[3], part[3][8];  // (eight short chains per block: a long one would lose a bit to the token-by-token form)
+  f32x4 part[3][8];  // (eight short chains per block: a long one would lose a bit to the token-by-token form)
 #pragma unroll
   for (int x = 0; x < 3; ++x)
 #pragma unroll
@@ -500,8 +531,6 @@ __global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws,
       part[2][a] = mma_f32(q1[r], k1[r], part[2][a]);
     }
   }
-#pragma unroll
-  for (int x = 0; x < 3; ++x) qk[x] = ((part[x][0] + part[x][1]) + (part[x][2] + part[x][3])) + ((part[x][4] + part[x][5]) + (part[x][6] + part[x][7]));
   // lane i: the running products behind token i (lane DC: from the chunk's start)
   const bool mine = lane < DC && t0 + lane < p.S;
   const size_t mr = m0 + (mine ? lane : 0);
@@ -515,8 +544,7 @@ __global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws,
     if (lane < DC) lp[wave][t][lane] = lane <= t ? run : 0.0;
     else if (lane == DC) out[DC * DC + t] = (float)run;
   }
-  if (lane < DC) out[DC * DC + DC + lane] = (float)run;  // P(last, i) write_i
-  if (lane == DC) out[DC * DC + 2 * DC] = (float)run;    // G_last
+  if (lane == DC) out[DC * DC + 2 * DC] = (float)run;  // G_last
   __builtin_amdgcn_wave_barrier();  // (LDS is the wave's own and in order)
 #pragma unroll
   for (int x = 0; x < 4; ++x) {  // (block 3, above the diagonal: zeros)
@@ -524,9 +552,11 @@ __global__ void __launch_bounds__(256) scalar_chunk_kernel(LinScan p, float* ws,
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = rb + 4 * q + r, i = cb + c;
-      out[t * DC + i] = x < 3 ? (float)(lp[wave][t][i] * qk[x < 3 ? x : 0][r]) : 0.f;
+      const double qk = x < 3 ? dc_total(part[x < 3 ? x : 0], r) : 0.0;
+      out[t * DC + i] = x < 3 ? (float)(lp[wave][t][i] * qk) : 0.f;
     }
   }
+  if (lane < DC) out[DC * DC + DC + lane] = (float)run;  // P(last, i) write_i
 }
 
 // Waves (16 value columns each) from which the walk that keeps a whole column in one wave fills the SIMDs

@@ -856,6 +856,52 @@ def test_scalar_gated_scan_in_chunks(b, s, h, dim, vdim):
     assert float((st_g.cpu().double() - st).norm() / st.norm()) < 5e-7
 
 
+def _delta_inputs(b, s, h, g, dim, vdim, seed):
+    gen = torch.Generator().manual_seed(seed)
+    R = lambda *x: torch.randn(*x, generator=gen)  # noqa: E731
+    m = b * s
+    q, k = (x / x.norm(dim=-1, keepdim=True) for x in (R(m, g, dim), R(m, g, dim)))
+    decay = torch.exp(-torch.exp(torch.rand(h, generator=gen) * 2.5 - 2.0) * torch.nn.functional.softplus(R(m, h)))
+    return [q * dim ** -0.5, k, torch.nn.functional.silu(R(m, h, vdim)), torch.sigmoid(R(m, h)), decay], R(b, h, dim, vdim) * 0.1
+
+
+def _mlstm_inputs(b, s, h, dim, vdim, seed):
+    gen = torch.Generator().manual_seed(seed)
+    R = lambda *x: torch.randn(*x, generator=gen)  # noqa: E731
+    m = b * s
+    return [R(m, h, dim), R(m, h, dim), R(m, h, vdim), torch.sigmoid(R(m, h) + 2.5), torch.sigmoid(R(m, h))], R(b, h, dim, vdim + 1) * 0.1
+
+
+@pytest.mark.parametrize("kind,b,s,h,dim,vdim", [("delta", 1, 64, 16, 128, 128), ("delta", 3, 333, 16, 64, 64), ("delta", 16, 200, 32, 64, 64),
+                                                 ("delta", 8, 70, 32, 128, 128), ("mlstm", 1, 32, 16, 128, 128), ("mlstm", 3, 333, 16, 64, 64)])
+def test_chunks_as_exact_as_token_by_token(kind, b, s, h, dim, vdim):
+    """Read-outs and state of the chunked forms (split walk, whole walk, scalar gates) against 64 bits. The bounds are what the
+    token-by-token kernels lose on the same operands (read-out 1.0e-7 to 1.05e-7, state 7.3e-8 to 7.5e-8 with the delta rule, 6.9e-8
+    to 7.3e-8 with scalar gates): the chunks may lose no more."""
+    if kind == "delta":
+        x, st = _delta_inputs(b, s, h, h // 4, dim, vdim, 1)
+    else:
+        x, st = _mlstm_inputs(b, s, h, dim, vdim, 1)
+    x, S = [t.to(DEV) for t in x], st.to(DEV)
+    S64 = S.double()
+    o = hy.delta_scan(*x, S, b, s) if kind == "delta" else hy.mlstm_scan(*x, S, b, s, dim ** -0.5)
+    q, k = (t.double().reshape(b, s, -1, dim).repeat_interleave(h // t.shape[1], 2) for t in x[:2])
+    v = x[2].double().reshape(b, s, h, vdim)
+    v = torch.cat([v, torch.ones_like(v[..., :1])], -1) if kind == "mlstm" else v
+    c, d = (t.double().reshape(b, s, h, 1) for t in x[3:])
+    ref = torch.empty_like(v)
+    for t in range(s):
+        if kind == "delta":
+            S64 = S64 * d[:, t, :, :, None]
+            u = c[:, t] * (v[:, t] - (S64 * k[:, t, :, :, None]).sum(2))
+        else:
+            S64, u = S64 * c[:, t, :, :, None], d[:, t] * v[:, t]
+        S64 = S64 + k[:, t, :, :, None] * u[:, :, None]
+        ref[:, t] = (S64 * q[:, t, :, :, None]).sum(2) * (1.0 if kind == "delta" else dim ** -0.5)
+    assert float((o.double().reshape(ref.shape) - ref).norm() / ref.norm()) < 1.04e-7
+    assert float((S.double() - S64).norm() / S64.norm()) < (7.4e-8 if kind == "delta" else 7.1e-8)
+
+
 @pytest.mark.parametrize("b,s,h,g,dim,vdim", [(17, 31, 2, 1, 64, 64), (16, 32, 2, 1, 128, 128), (16, 33, 6, 3, 64, 128), (2, 257, 4, 2, 128, 64),
                                               (1, 511, 2, 2, 64, 64), (1, 527, 2, 2, 64, 64), (8, 64, 2, 1, 80, 64)])
 def test_delta_preparation_in_runs(b, s, h, g, dim, vdim):
