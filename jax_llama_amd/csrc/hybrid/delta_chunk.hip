@@ -23,7 +23,9 @@
 // 15] hands it to the next product as the B operand of k-step r, whose A operand is then column 4 (l >> 4) + r of a 16-wide
 // block: four k-steps per 16-byte LDS read. Likewise r and u. K, Q, T' and M of a chunk go through LDS once per workgroup (64
 // columns); the next chunk's loads are in flight meanwhile.
-// A token that is not a number spoils the outputs of its whole chunk (masked products are 0 x NaN), not only later ones.
+// A number that is none (in a key, query, value or gate, or by overflow) would spoil every token of its chunk, as masked products
+// are 0 x NaN: such a chunk is walked token by token, and only the tokens from that one on see it (the check and the walk's
+// registers cost 5 %: 2048 tokens of 16 heads 209 -> 220 us).
 #include "hy_util.h"
 #include "hybrid.h"
 
@@ -98,6 +100,7 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
   }
   __builtin_amdgcn_wave_barrier();  // (LDS is the wave's own and in order)
   // A in LDS, M to the workspace; lane holds row (token) 4 q + r, column (token) c of each block
+  bool whole = true;  // (a number that is none in a token's key or query shows in its own products)
 #pragma unroll
   for (int x = 0; x < 3; ++x) {
     const int rb = x ? 16 : 0, cb = x == 2 ? 16 : 0;
@@ -107,15 +110,18 @@ __global__ void __launch_bounds__(256) delta_chunk_kernel(DeltaScan p, float* ws
       const double pr = lp[wave][t][i];
       const float bt = __shfl(beta, t, 64);  // (every lane takes part in the exchange)
       const double kk = dc_total(kp_[x], r), qk = dc_total(qp_[x], r);
+      whole &= isfinite(kk) && isfinite(qk);
       la[wave][t][i] = i < t ? (float)(pr * bt * kk) : 0.f;
       out[DC * DC + t * DC + i] = (float)(pr * qk);  // (P is 0 above the diagonal)
     }
   }
+  whole &= isfinite(g) && isfinite(beta);
+  const bool spoiled = __any(!whole);
   __builtin_amdgcn_wave_barrier();
   if (lane < DC) {
     out[2 * DC * DC + lane] = (float)lp[wave][lane][DC];
     out[2 * DC * DC + DC + lane] = (float)lp[wave][DC - 1][lane];
-    out[2 * DC * DC + 2 * DC + lane] = beta;
+    out[2 * DC * DC + 2 * DC + lane] = spoiled ? NAN : beta;  // (the walk then takes this chunk token by token)
     // column `lane` of the inverse: x_t = [t == lane] - sum_{i < t} A(t, i) x_i
     float x[DC];
 #pragma unroll
@@ -242,13 +248,52 @@ __global__ void __launch_bounds__(256, 2) delta_walk_kernel(DeltaScan p, const f
         for (int r = 0; r < 4; ++r) u[mt] = mma_f32(a[r], r_[kb][r], u[mt]);
       }
     // (the diagonal of T', beta, last: what the earlier tokens take away is small beside it)
+    bool whole = true;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const f32x4 bt = *reinterpret_cast<const f32x4*>(&Gs[2 * DC + 16 * mt + 4 * q]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[mt][r] = fmaf(bt[r], r_[mt][r], u[mt][r]);
+      for (int r = 0; r < 4; ++r) {
+        u[mt][r] = fmaf(bt[r], r_[mt][r], u[mt][r]);
+        whole &= isfinite(u[mt][r]);
+      }
     }
     const int t0 = ch * DC;
+    if (__any(!whole)) {  // a number that is none spoils the tokens from its own on, not those before it
+      const int n = min(p.S - t0, DC);
+#pragma unroll 1
+      for (int t = 0; t < n; ++t) {
+        const size_t m = ((size_t)b * p.S + t0 + t) * p.H + h;
+        const float g = p.decay[m];
+        float sk = 0.f, oq = 0.f;
+#pragma unroll
+        for (int mb = 0; mb < DB; ++mb) {
+          const f32x4 k = *reinterpret_cast<const f32x4*>(&Ks[t * LK + 16 * mb + 4 * q]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            S[mb][r] *= g;
+            sk = fmaf(S[mb][r], k[r], sk);
+          }
+        }
+        sk += __shfl_xor(sk, 16, 64);
+        sk += __shfl_xor(sk, 32, 64);
+        const float ut = p.beta[m] * (p.v[m * p.vdim + j] - sk);
+#pragma unroll
+        for (int mb = 0; mb < DB; ++mb) {
+          const f32x4 k = *reinterpret_cast<const f32x4*>(&Ks[t * LK + 16 * mb + 4 * q]);
+          const f32x4 x = *reinterpret_cast<const f32x4*>(&Qs[t * LK + 16 * mb + 4 * q]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            S[mb][r] = fmaf(k[r], ut, S[mb][r]);
+            oq = fmaf(S[mb][r], x[r], oq);
+          }
+        }
+        oq += __shfl_xor(oq, 16, 64);
+        oq += __shfl_xor(oq, 32, 64);
+        if (q == 0) p.o[m * p.vdim + j] = oq;
+      }
+      continue;
+    }
     f32x4 qs[2];
     times_state(Qs, qs);
 #pragma unroll
@@ -305,6 +350,8 @@ struct ChunkWalk {
   const float* v;  // token m, head h at v + m * ldv + h * vdim; a column vdim (ncols = vdim + 1) is 1
   int ldv;
   const float* ws;
+  const float* decay;  // [B * S, H]
+  const float* write;  // [B * S, H]: beta, or the scalar gates' write factors
   float* state;  // [B, H, dim, ncols]
   float* o;      // [M, H, ncols]
   int S, H, heads_per_key, vdim, ncols, chunks;
@@ -395,6 +442,53 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     vp += (size_t)DC * p.ldv;
     wp += WS;
   };
+  // chunk ch token by token: a number that is none spoils the tokens from its own on, not those before it. Every wave of the
+  // workgroup comes here together.
+  auto by_token = [&](int ch) {
+    __syncthreads();  // (the chunk's exchange has been read)
+    float* const ex = reinterpret_cast<float*>(red);  // [2][4 waves][16 columns] read-outs, then the same of S^T k
+    const int end = min(p.S, (ch + 1) * DC);
+#pragma unroll 1
+    for (int t = ch * DC; t < end; ++t) {
+      const size_t m = (size_t)b * p.S + t, mh = m * p.H + h;
+      const float* kr = p.k + m * p.ldk + (size_t)kh * D + d0 + 4 * q;
+      const float* qr = p.q + m * p.ldq + (size_t)kh * D + d0 + 4 * q;
+      const float g = p.decay[mh], v = j < p.vdim ? p.v[m * p.ldv + (size_t)h * p.vdim + j] : 1.f;
+      float sk = 0.f, oq = 0.f, u = p.write[mh];
+#pragma unroll
+      for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[mb][r] *= g;
+          if (DELTA) sk = fmaf(S[mb][r], kr[16 * mb + r], sk);
+        }
+      if (DELTA) {
+        sk += __shfl_xor(sk, 16, 64);
+        sk += __shfl_xor(sk, 32, 64);
+        if (q == 0) ex[128 + 16 * wave + c] = sk;
+        __syncthreads();
+        sk = (ex[128 + c] + ex[144 + c]) + (ex[160 + c] + ex[176 + c]);
+        u *= v - sk;
+      } else {
+        u *= v;
+      }
+#pragma unroll
+      for (int mb = 0; mb < DBW; ++mb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[mb][r] = fmaf(kr[16 * mb + r], u, S[mb][r]);
+          oq = fmaf(S[mb][r], qr[16 * mb + r], oq);
+        }
+      oq += __shfl_xor(oq, 16, 64);
+      oq += __shfl_xor(oq, 32, 64);
+      float* const eo = ex + 64 * (t & 1);
+      if (q == 0) eo[16 * wave + c] = oq;
+      __syncthreads();
+      if (wave == 0 && q == 0 && j < p.ncols)
+        p.o[mh * p.ncols + j] = ((eo[c] + eo[16 + c]) + (eo[32 + c] + eo[48 + c])) * (DELTA ? 1.f : p.o_scale);
+    }
+    __syncthreads();
+  };
   auto step = [&](const Operands& x, int ch, int buf) {
     f32x4 qs[2][4], ks[2][4];  // (short chains)
 #pragma unroll
@@ -444,6 +538,12 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) u[mt][r] = fmaf(x.ba[DELTA ? mt : 0][r], r_[mt][r], u[mt][r]);
     }
+    bool whole = DELTA || isfinite(x.wa[0][0]);  // (all waves hold the same u and the same gates)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) whole &= isfinite(u[mt][r]);
+    if (__any(!whole)) return by_token(ch);
     if (wave < 2) {  // o of token tile mt_o
       f32x4 o = (red[buf][0][mt_o][lane] + red[buf][1][mt_o][lane]) + (red[buf][2][mt_o][lane] + red[buf][3][mt_o][lane]);
       const f32x4 g = mt_o ? x.ga[1] : x.ga[0];
@@ -546,6 +646,7 @@ __global__ void __launch_bounds__(256, 2) scalar_chunk_kernel(LinScan p, float* 
   }
   if (lane == DC) out[DC * DC + 2 * DC] = (float)run;  // G_last
   __builtin_amdgcn_wave_barrier();  // (LDS is the wave's own and in order)
+  bool whole = isfinite(keep) && isfinite(write);  // (a number that is none in a token's key or query shows in its own products)
 #pragma unroll
   for (int x = 0; x < 4; ++x) {  // (block 3, above the diagonal: zeros)
     const int rb = x == 1 || x == 2 ? 16 : 0, cb = x >= 2 ? 16 : 0;
@@ -553,10 +654,12 @@ __global__ void __launch_bounds__(256, 2) scalar_chunk_kernel(LinScan p, float* 
     for (int r = 0; r < 4; ++r) {
       const int t = rb + 4 * q + r, i = cb + c;
       const double qk = x < 3 ? dc_total(part[x < 3 ? x : 0], r) : 0.0;
+      whole &= isfinite(qk);
       out[t * DC + i] = x < 3 ? (float)(lp[wave][t][i] * qk) : 0.f;
     }
   }
-  if (lane < DC) out[DC * DC + DC + lane] = (float)run;  // P(last, i) write_i
+  const bool spoiled = __any(!whole);
+  if (lane < DC) out[DC * DC + DC + lane] = spoiled ? NAN : (float)run;  // P(last, i) write_i; the walk takes a spoiled chunk by token
 }
 
 // Waves (16 value columns each) from which the walk that keeps a whole column in one wave fills the SIMDs
@@ -581,7 +684,7 @@ int hy_scalar_chunk(const LinScan& p, float* ws, hipStream_t s) {
   if (hy_scalar_chunk_floats(p) == 0) return -1;
   if ((uintptr_t)ws & 15) return -2;
   const int chunks = (p.S + DC - 1) / DC, ncols = p.vdim + 1;
-  const ChunkWalk w{p.q, p.ldq, p.k, p.ldk, p.v, p.ldv, ws, p.state, p.o, p.S, p.H, 1, p.vdim, ncols, chunks, p.q_scale};
+  const ChunkWalk w{p.q, p.ldq, p.k, p.ldk, p.v, p.ldv, ws, p.decay, p.write, p.state, p.o, p.S, p.H, 1, p.vdim, ncols, chunks, p.q_scale};
   const dim3 g1((chunks + 3) / 4, p.H, p.B), g2(p.H, (ncols + 15) / 16, p.B);
   if (p.dim == 128) {
     scalar_chunk_kernel<8><<<g1, 256, 0, s>>>(p, ws, chunks);
@@ -612,7 +715,7 @@ int hy_delta_chunk(const DeltaScan& p, float* ws, hipStream_t s) {
   if (p.dim == 128) delta_chunk_kernel<8><<<g1, 256, 0, s>>>(p, ws, chunks);
   else delta_chunk_kernel<4><<<g1, 256, 0, s>>>(p, ws, chunks);
   if (dc_splits(p.B, p.H, p.vdim)) {
-    const ChunkWalk w{p.qn, p.G * p.dim, p.kn, p.G * p.dim, p.v, p.H * p.vdim, ws, p.state, p.o, p.S, p.H, p.H / p.G, p.vdim, p.vdim, chunks, 1.f};
+    const ChunkWalk w{p.qn, p.G * p.dim, p.kn, p.G * p.dim, p.v, p.H * p.vdim, ws, p.decay, p.beta, p.state, p.o, p.S, p.H, p.H / p.G, p.vdim, p.vdim, chunks, 1.f};
     const dim3 g3(p.H, p.vdim / 16, p.B);
     if (p.dim == 128) chunk_walk_split_kernel<2, 1><<<g3, 256, 0, s>>>(w);
     else chunk_walk_split_kernel<1, 1><<<g3, 256, 0, s>>>(w);

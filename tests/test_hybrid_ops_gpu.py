@@ -902,6 +902,26 @@ def test_chunks_as_exact_as_token_by_token(kind, b, s, h, dim, vdim):
     assert float((S.double() - S64).norm() / S64.norm()) < (7.4e-8 if kind == "delta" else 7.1e-8)
 
 
+@pytest.mark.parametrize("kind,b,s,h,dim,vdim", [("delta", 1, 70, 4, 128, 32), ("delta", 2, 45, 2, 64, 16), ("delta", 16, 40, 32, 64, 32),
+                                                 ("mlstm", 1, 70, 2, 128, 20), ("mlstm", 2, 45, 2, 64, 16)])
+@pytest.mark.parametrize("operand", range(5))
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_chunks_keep_tokens_before_a_number_that_is_none(kind, b, s, h, dim, vdim, operand, bad):
+    """A NaN or infinity at one token of a chunk (in its query, key, value or one of its gates) reaches that token and those behind
+    it, as token by token on the CPU; the tokens before it, and the other heads and rows, keep their values."""
+    x, st = _delta_inputs(b, s, h, h // 2, dim, vdim, 3) if kind == "delta" else _mlstm_inputs(b, s, h, dim, vdim, 3)
+    at = (b - 1) * s + 37  # the last row's token 37: the sixth of its second chunk
+    x[operand].reshape(b * s, -1)[at, 0] = bad
+    S_g = st.clone().to(DEV)
+    scan = lambda y, S: hy.delta_scan(*y, S, b, s) if kind == "delta" else hy.mlstm_scan(*y, S, b, s, 0.3)  # noqa: E731
+    want, got = scan(x, st), scan([t.to(DEV) for t in x], S_g).cpu()
+    assert torch.isfinite(want.reshape(b, s, -1)[:, :37]).all() and not torch.isfinite(want.reshape(b, s, -1)[-1, 37]).all()
+    for w, y in ((want, got), (st, S_g.cpu())):
+        ok = torch.isfinite(w)
+        assert torch.equal(torch.isfinite(y), ok)
+        assert float((y - w)[ok].abs().max()) < 2e-5 * float(w[ok].abs().max())
+
+
 @pytest.mark.parametrize("b,s,h,g,dim,vdim", [(17, 31, 2, 1, 64, 64), (16, 32, 2, 1, 128, 128), (16, 33, 6, 3, 64, 128), (2, 257, 4, 2, 128, 64),
                                               (1, 511, 2, 2, 64, 64), (1, 527, 2, 2, 64, 64), (8, 64, 2, 1, 80, 64)])
 def test_delta_preparation_in_runs(b, s, h, g, dim, vdim):
