@@ -1496,20 +1496,18 @@ SCAN_SEG_MIN = 64
 SCAN_TARGET_BLOCKS = int(os.environ.get("JLA_HY_SCAN_BLOCKS", "512"))
 
 
-def _scan_segments(b: int, s: int, heads: int, dim: int, cols: int, device):
-    """``(nseg, seg_len, workspace)`` of a scan over ``s`` tokens of ``b`` rows (csrc/hybrid/recurrent.hip: a thread
-    holds 16 key rows of a state column, 256 threads a workgroup)."""
+def _scan_segments(b: int, s: int, heads: int, dim: int, cols: int, device=None):
+    """``(nseg, seg_len)`` of a scan over ``s`` tokens of ``b`` rows (csrc/hybrid/recurrent.hip: a thread holds 16 key rows of a
+    state column, 256 threads a workgroup), the same on every device."""
     lanes = 1
     while lanes * 16 < dim:
         lanes *= 2
     blocks = b * heads * ((cols * lanes + 255) // 256)
     nseg = min(s // SCAN_SEG_MIN, SCAN_TARGET_BLOCKS // max(1, blocks))
     if nseg < 2:
-        return 1, max(s, 1), None
+        return 1, max(s, 1)
     seg_len = (s + nseg - 1) // nseg
-    nseg = (s + seg_len - 1) // seg_len
-    ws = torch.empty(b * nseg * heads * dim * (cols + 1), dtype=F32, device=device)
-    return nseg, seg_len, ws
+    return (s + seg_len - 1) // seg_len, seg_len
 
 
 def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, keep: torch.Tensor, write: torch.Tensor,
@@ -1532,8 +1530,8 @@ def mlstm_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, keep: torch.Te
             o[:, t] = torch.einsum("bhdv,bhd->bhv", state, qq[:, t])
         return o.reshape(m, h, vdim + 1)
     o = torch.empty(m, h, vdim + 1, dtype=F32, device=q.device)
-    nseg, seg_len, ws = _scan_segments(b, s, h, dim, vdim + 1, q.device)
-    ext().lin_scan(0, q, k, v, keep, write, None, None, state, o, b, s, float(q_scale), nseg, seg_len, ws)
+    nseg, seg_len = _scan_segments(b, s, h, dim, vdim + 1)
+    ext().lin_scan(0, q, k, v, keep, write, None, None, state, o, b, s, float(q_scale), nseg, seg_len)
     return o
 
 
@@ -1558,8 +1556,8 @@ def timemix_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre: torch.
             state.add_(kv)
         return o.reshape(m, h, vdim)
     o = torch.empty(m, h, vdim, dtype=F32, device=r.device)
-    nseg, seg_len, ws = _scan_segments(b, s, h, dim, vdim, r.device)
-    ext().lin_scan(1, r, k, v, wpre, None, w0.reshape(h, dim), u.reshape(h, dim), state, o, b, s, 1.0, nseg, seg_len, ws)
+    nseg, seg_len = _scan_segments(b, s, h, dim, vdim)
+    ext().lin_scan(1, r, k, v, wpre, None, w0.reshape(h, dim), u.reshape(h, dim), state, o, b, s, 1.0, nseg, seg_len)
     return o
 
 
@@ -1581,9 +1579,9 @@ def gated_running_scan(q: torch.Tensor, v: torch.Tensor, fpre: torch.Tensor, f_b
             o[:, t] = torch.einsum("bhdv,bhd->bhv", state, qq[:, t])
         return o.reshape(m, h, vdim)
     o = torch.empty(m, h, vdim, dtype=F32, device=q.device)
-    nseg, seg_len, ws = _scan_segments(b, s, h, dim, vdim, q.device)
+    nseg, seg_len = _scan_segments(b, s, h, dim, vdim)
     ext().lin_scan(2, q, fpre, v, fpre, None, f_bias.reshape(h, dim), room.reshape(h, dim), state, o, b, s, 1.0, nseg,
-                   seg_len, ws)
+                   seg_len)
     return o
 
 

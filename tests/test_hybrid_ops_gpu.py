@@ -856,6 +856,31 @@ def test_scalar_gated_scan_in_chunks(b, s, h, dim, vdim):
     assert float((st_g.cpu().double() - st).norm() / st.norm()) < 5e-7
 
 
+@pytest.mark.parametrize("nseg,seg_len", [(2, 20), (3, 40), (0, 64)])
+def test_scan_refuses_segments_that_miss_the_tokens(nseg, seg_len):
+    """... whichever form the sizes then take (64 tokens of 64 x 64 heads: the chunks)."""
+    x, st = _mlstm_inputs(1, 64, 2, 64, 64, 5)
+    o, st = torch.empty(64, 2, 65, device=DEV), st.to(DEV)
+    with pytest.raises(RuntimeError):
+        hy.ext().lin_scan(0, *[t.to(DEV) for t in x], None, None, st, o, 1, 64, 1.0, nseg, seg_len)
+
+
+def test_scan_takes_only_the_scratch_of_its_form():
+    """A prompt that runs in chunks allocates the chunks' scratch, not the segments' too."""
+    b, s, h, dim = 1, 2048, 16, 128
+    x, st = _mlstm_inputs(b, s, h, dim, dim, 5)
+    x, st = [t.to(DEV) for t in x], st.to(DEV)
+    assert hy._scan_segments(b, s, h, dim, dim + 1)[0] > 1
+    hy.mlstm_scan(*x, st, b, s)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    hy.mlstm_scan(*x, st, b, s)
+    taken = torch.cuda.max_memory_allocated() - base
+    out, chunks = b * s * h * (dim + 1) * 4, b * h * (s // 32) * 1092 * 4  # (1092 numbers per chunk)
+    assert taken <= out + chunks + 4096
+
+
 def _delta_inputs(b, s, h, g, dim, vdim, seed):
     gen = torch.Generator().manual_seed(seed)
     R = lambda *x: torch.randn(*x, generator=gen)  # noqa: E731
