@@ -261,7 +261,7 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
     take the pending residual add and the gate in the product's launch; else the separate ops."""
     r = x if isinstance(x, Residual) else None
     ids = ids.reshape(-1).to(torch.int32).contiguous() if ids is not None else None
-    if r is not None and r.fusable():
+    if r is not None and r.fusable() and w.dtype == BF16:
         out = torch.empty(r.x.shape[0], w.shape[0], dtype=F32, device=r.x.device)
         new = torch.empty_like(r.x)
         if ext().rows_fused(r.x, w, out, *r.pending, new, ids, table, int(col0)):
@@ -270,7 +270,7 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
     xv = r.value() if r is not None else x
     if ids is None:
         return linear(xv, w)
-    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and xv.dtype == F32:
+    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and xv.dtype == F32 and w.dtype == BF16:
         out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, ids, table, int(col0)):
             return out

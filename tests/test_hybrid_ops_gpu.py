@@ -741,6 +741,22 @@ def test_pending_residual_in_the_product(m, k, n, nsum):
     _close(got, hy.linear(hy.RmsInput(x, gw, 1e-6), w), 2e-3, "normed product")
 
 
+@pytest.mark.parametrize("pending", [True, False])
+def test_fp32_weights_are_not_offered_to_the_bf16_product(pending, monkeypatch):
+    """fp32 weights run the separate ops without a fused call, and its buffers, first; the result is theirs."""
+    class Watch:
+        def __getattr__(self, name):
+            assert name != "rows_fused"
+            return getattr(real, name)
+
+    real, n = hy.ext(), 64
+    w, gate, ids = _rand(n, 512).to(DEV), _rand(9, n).to(DEV), torch.tensor([3, 8], dtype=torch.int32, device=DEV)
+    monkeypatch.setattr(hy, "ext", lambda: Watch())
+    out = [hy.linear_rows_gated(r if pending else r.value(), w, ids, gate) for r in (_residual(2, 512, 1, DEV), _residual(2, 512, 1, DEV))]
+    sep = hy.gelu_gate_rows(hy.linear(_residual(2, 512, 1, DEV).value(), w), ids, gate, 0)
+    assert torch.equal(out[0], sep) and torch.equal(out[1], sep)
+
+
 @pytest.mark.parametrize("m,top,e,d,f", [(1, 2, 8, 256, 96), (2, 2, 8, 2048, 704), (4, 2, 3, 64, 72), (1, 1, 4, 256, 264), (3, 3, 5, 128, 64),
                                          (1, 2, 4, 130, 64)])
 def test_table_experts_without_a_routing_launch(m, top, e, d, f):
