@@ -200,6 +200,8 @@ int hy_norm_residual(const float* y, int nsum, float ysc, const float* w, int w_
   norm_residual_kernel<NU><<<M, 256, 0, s>>>(y, nsum, ysc, w, w_vec, eps, x, out, D, extra, extra_gate, ldg)
   const int nu = (D + 255) / 256;
   if (nu <= 1) NR_LAUNCH(1);
+  else if (nu <= 2) NR_LAUNCH(2);
+  else if (nu <= 4) NR_LAUNCH(4);
   else if (nu <= 8) NR_LAUNCH(8);
   else if (nu <= 16) NR_LAUNCH(16);
   else NR_LAUNCH(0);
