@@ -56,12 +56,15 @@ __global__ void __launch_bounds__(256) rows_f32_sum_kernel(RowLinear p, const fl
   *o = p.add_out ? *o + v : v;
 }
 
-// (a K of a few steps is over before the pipeline is filled: 64 x 2048 x K 64 6.6 us on lr_gemm_kernel's tiles, 7.2 here)
-constexpr int RF_MIN_K = 256;
+// A K of a few steps is over before the pipeline is filled: 64 x 2048 x K 64 6.6 us on lr_gemm_kernel's tiles, 7.2 here; 130 rows of
+// K 256 | 384 13.2 | 17.5, 15.0 | 19.7 here (K 512, cut in two: 25.7, 18.4). From 256 rows per expert on those tiles are of 128
+// rows and it turns earlier: 300 rows of K 256 20.7, 16.6 here.
+constexpr int RF_MIN_K = 512, RF_MIN_K_MANY = 256, RF_MANY_ROWS = 256;
 
 bool hy_rows_f32_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  return !p.wbf16 && !p.a_bf16 && !p.out_bf16 && !p.a_norm_w && (p.offs || p.E == 1) && p.K % 8 == 0 && p.K >= RF_MIN_K && p.lda % 4 == 0 &&
+  return !p.wbf16 && !p.a_bf16 && !p.out_bf16 && !p.a_norm_w && (p.offs || p.E == 1) && p.K % 8 == 0 &&
+         p.K >= (p.R / (p.offs ? p.E : 1) >= RF_MANY_ROWS ? RF_MIN_K_MANY : RF_MIN_K) && p.lda % 4 == 0 &&
          p.N % 4 == 0 && p.ldo % 4 == 0 && p.w_stride % 4 == 0 && aligned(p.a) && aligned(p.w) && aligned(p.out);
 }
 
