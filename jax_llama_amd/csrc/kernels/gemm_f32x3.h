@@ -213,12 +213,14 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
   for (int u = 0; u < NA; ++u) again |= (ta[u] & 0x7fffffffu) && !(ta[u] & F3_EXP);
 #pragma unroll
   for (int u = 0; u < NW; ++u) again |= (tw[u] & 0x7fffffffu) && !(tw[u] & F3_EXP);
+  float none[4] = {0.f, 0.f, 0.f, 0.f};  // (0 x an infinity or NaN)
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) again |= !(fabsf(acc[j][i][r]) < INFINITY);
+      for (int r = 0; r < 4; ++r) none[r] = fmaf(acc[j][i][r], 0.f, none[r]);
+  again |= !((none[0] + none[1]) + (none[2] + none[3]) == 0.f);
   if (__syncthreads_or(again)) {
     const float *ar[MT], *wr_[4];
     float as[MT];
