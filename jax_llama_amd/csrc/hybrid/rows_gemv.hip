@@ -59,10 +59,10 @@ JLA_DEV float rv_table(const RowLinear& p, int r, int col) {
   return p.mul_bf16 ? bf2f(reinterpret_cast<const bf16_t*>(p.mul_table)[at]) : reinterpret_cast<const float*>(p.mul_table)[at];
 }
 
-// The sum of N partial sums, rounded once
-template <int N>
+// The sum of N partial sums in type T
+template <class T, int N>
 JLA_DEV float rv_sum(const float (&f)[N]) {
-  double s[N];
+  T s[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) s[i] = f[i];
 #pragma unroll
@@ -82,14 +82,15 @@ JLA_DEV void rv_store(const RowLinear& p, int r, int col, float g, float v) {
 
 // G: output columns of a tile, and rows of a pass per 16 MT / (16 / G); NT: tiles of a workgroup (gated: gate and up tiles
 // alternate); MT: 16-row tiles (G = 16); U: K steps in flight per wave. NORM 1 (MT = 1): rows are RMS-normed with a gain
-// first, in the order (a * scale) * gain of the norm kernel.
-template <int G, int NT, int MT, int WAVES, int U, int NORM>
+// first, in the order (a * scale) * gain of the norm kernel. SUM: the type that the MFMAs' sums are added in.
+template <int G, int NT, int MT, int WAVES, int U, int NORM, class SUM>
 __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int rows_per_group, int gated) {
   static_assert(G == 16 || MT == 1, "several row tiles: whole 16-column tiles");
   constexpr int SEG = 16 / G;                // neighbouring K ranges of one MFMA
   constexpr int H = G == 16 ? 2 : 1;         // MFMAs of a K step (G = 16: the two halves of a 128-byte line)
   constexpr int STEP = 32 * SEG * H;         // K of a step
-  constexpr int RUN = 4 / H;                 // steps (four MFMAs) whose sums share an fp32 accumulator
+  constexpr bool WIDE = sizeof(SUM) > sizeof(float);
+  constexpr int RUN = WIDE ? 4 / H : U;      // steps (four MFMAs) whose sums share an fp32 accumulator; SUM float: all of them do
   constexpr int ROWS = G * MT;               // rows of a pass
   __shared__ f32x4 red[WAVES][NT * MT][64];
   __shared__ float stat[NORM ? WAVES : 1][16];
@@ -153,13 +154,16 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
       for (int w = 0; w < WAVES; ++w) ss += stat[w][c % G];
       xs[0] = 1.f / sqrtf(ss / (float)K + p.a_norm_eps);
     }
-    double acc[NT][MT][4];  // (64 bits cost nothing beside the stream: 8 rows, K 7168 x N 4096: 16.7 -> 17.0 us)
+    SUM acc[NT][MT][4];  // (64 bits cost little beside the stream: 8 rows, K 7168 x N 4096: 16.7 -> 17.0 us)
+    f32x4 part[NT][MT];  // a run's own sums
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
+      for (int m = 0; m < MT; ++m) {
+        part[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][m][i] = 0.0;
+        for (int i = 0; i < 4; ++i) acc[t][m][i] = 0;
+      }
 
     for (int s0 = wave; s0 < steps; s0 += WAVES * U) {
       u32x4 wf[U][H][NT];
@@ -180,11 +184,12 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
 #pragma unroll
       for (int u0 = 0; u0 < U; u0 += RUN) {
         if (s0 + WAVES * u0 >= steps) break;  // (wave-uniform)
-        f32x4 part[NT][MT];  // this run's own sums
+        if (WIDE) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+          for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) part[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MT; ++m) part[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int u = u0; u < (u0 + RUN < U ? u0 + RUN : U); ++u) {
           const int s = s0 + WAVES * u;
@@ -220,12 +225,14 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
             }
           }
         }
+        if (WIDE) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+          for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[t][m][i] += part[t][m][i];
+              for (int i = 0; i < 4; ++i) acc[t][m][i] += part[t][m][i];
+        }
       }
     }
     // lane: row (B column) c, columns (A rows) 4 q + 0..3 of tile t
@@ -233,7 +240,8 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        red[wave][t * MT + m][lane] = f32x4{(float)acc[t][m][0], (float)acc[t][m][1], (float)acc[t][m][2], (float)acc[t][m][3]};
+        red[wave][t * MT + m][lane] = WIDE ? f32x4{(float)acc[t][m][0], (float)acc[t][m][1], (float)acc[t][m][2], (float)acc[t][m][3]}
+                                           : part[t][m];
     __syncthreads();
     // one output element per thread: the epilogue's code, which a short launch has to fetch, stays small
     constexpr int PER = G * G;  // (column, row) pairs of a tile
@@ -251,7 +259,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
 #pragma unroll
           for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[w][at][l][y % 4];
         }
-        return rv_sum(f);
+        return rv_sum<SUM>(f);
       };
       const float g = total(slot), v = gated ? total(slot + MT) : 0.f;
       rv_store(p, r0 + row, col, g, v);
@@ -432,7 +440,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
         for (int sg = 0; sg < 4; ++sg)  // the diagonal block of K range sg
 #pragma unroll
           for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[buf][w][at][20 * sg + x][y];
-        return rv_sum(f);
+        return rv_sum<double>(f);
       };
       const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
       if (col < N) rv_store(p, r0 + x, col, g, v);
@@ -441,15 +449,15 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 }
 
 // up to 64 rows, and up to 32 of a wide output, whose tiles fill the chip (64 rows x 32000 columns, K 2048: 70 us on the
-// tiles, 82 here); one or two rows of a short K are over before the waves' sum pays (K 64: 3.2 against 3.6 us). Rows with an
-// expert of their own and no offsets: as many as the vector unit's form takes.
+// tiles, 82 here); a short K is over before the waves' sum pays (K 64: one row 3.2 us on the vector unit, 3.6 here, 64 rows
+// 4.8 on the tiles, 5.4 here). Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
 constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 2;
 
 bool hy_rows_gemv_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return p.wbf16 && !p.a_bf16 && !p.out_bf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
          (p.offs || p.tab || (p.row_expert ? p.R <= HY_GEMV_MAX_R : p.E == 1)) && p.K % 8 == 0 &&
-         p.K >= (p.R > 2 ? 64 : 256) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
+         p.K >= (p.R <= 2 ? 256 : (p.R <= 32 ? 64 : 128)) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
          (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && (p.a_norm_one || aligned(p.a_norm_w))));
 }
 
@@ -515,27 +523,39 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   const long long wgs = (tiles + nt - 1) / nt;
   if (wgs > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)wgs, groups);
-#define RV_RUN(G, NT, MT, U, NORM) rows_gemv_kernel<G, NT, MT, 4, U, NORM><<<grid, 256, 0, s>>>(q, rpg, gated)
-#define RV_NT(G, NORM)                  \
-  do {                                  \
-    if (nt == 1) RV_RUN(G, 1, 1, 4, NORM); \
-    else if (nt == 2) RV_RUN(G, 2, 1, 2, NORM); \
-    else RV_RUN(G, 4, 1, 2, NORM);      \
+#define RV_RUN(G, NT, MT, U, NORM, T) rows_gemv_kernel<G, NT, MT, 4, U, NORM, T><<<grid, 256, 0, s>>>(q, rpg, gated)
+#define RV_NT(G, NORM, T)                     \
+  do {                                        \
+    if (nt == 1) RV_RUN(G, 1, 1, 4, NORM, T);  \
+    else if (nt == 2) RV_RUN(G, 2, 1, 2, NORM, T); \
+    else RV_RUN(G, 4, 1, 2, NORM, T);         \
   } while (0)
-  if (mt == 4) {
-    if (nt == 2) RV_RUN(16, 2, 4, 1, 0);
-    else RV_RUN(16, 4, 4, 1, 0);
-  } else if (mt == 2) {
-    if (nt == 2) RV_RUN(16, 2, 2, 2, 0);
-    else RV_RUN(16, 4, 2, 1, 0);
-  } else if (G == 4) {
-    if (p.a_norm_w) RV_NT(4, 1);  // (at most two rows)
-    else RV_NT(4, 0);
+#define RV_16(T)                         \
+  do {                                   \
+    if (mt == 4) {                       \
+      if (nt == 2) RV_RUN(16, 2, 4, 1, 0, T); \
+      else RV_RUN(16, 4, 4, 1, 0, T);    \
+    } else if (mt == 2) {                \
+      if (nt == 2) RV_RUN(16, 2, 2, 2, 0, T); \
+      else RV_RUN(16, 4, 2, 1, 0, T);    \
+    } else {                             \
+      RV_NT(16, 0, T);                   \
+    }                                    \
+  } while (0)
+  // (rows that had the vector unit's form are added in 64 bits, to lose no more than it did; more than eight dense rows had the
+  // tiles' one fp32 chain over all of K, 2.7e-7 at K 2048, here 1.3e-7 in one chain per wave: 33 rows of 4096 x 10304 60.5 us,
+  // 64.5 in 64 bits)
+  if (G == 4) {
+    if (p.a_norm_w) RV_NT(4, 1, double);  // (at most two rows)
+    else RV_NT(4, 0, double);
   } else if (G == 8) {
-    RV_NT(8, 0);
+    RV_NT(8, 0, double);
+  } else if (p.offs) {
+    RV_16(double);
   } else {
-    RV_NT(16, 0);
+    RV_16(float);
   }
+#undef RV_16
 #undef RV_NT
 #undef RV_RUN
   JLA_CHECK_LAUNCH();
