@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256) rows_f32_sum_kernel(RowLinear p, const fl
 }
 
 // A K of a few steps is over before the pipeline is filled: 64 x 2048 x K 64 6.6 us on lr_gemm_kernel's tiles, 7.2 here; 130 rows of
-// K 256 | 384 13.2 | 17.5, 15.0 | 19.7 here (K 512, cut in two: 25.7, 18.4). From 256 rows per expert on those tiles are of 128
+// K 256 | 384 13.2 | 17.5, 15.0 | 19.7 here (K 512, cut in two: 23.5, 18.6). From 256 rows per expert on those tiles are of 128
 // rows and it turns earlier: 300 rows of K 256 20.7, 16.6 here.
 constexpr int RF_MIN_K = 512, RF_MIN_K_MANY = 256, RF_MANY_ROWS = 256;
 

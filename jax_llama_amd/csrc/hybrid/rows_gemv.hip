@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 
 // up to 64 rows, and up to 32 of a wide output, whose tiles fill the chip (64 rows x 32000 columns, K 2048: 70 us on the
 // tiles, 82 here); a short K is over before the waves' sum pays (K 64: one row 3.2 us on the vector unit, 3.6 here, 64 rows
-// 4.8 on the tiles, 5.4 here). Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
+// 4.8 on the tiles, 5.3 here). Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
 constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 2;
 
 bool hy_rows_gemv_takes(const RowLinear& p) {

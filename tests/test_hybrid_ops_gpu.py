@@ -473,9 +473,9 @@ def test_rows_on_the_large_tiles(counts, k, n, act):
 @pytest.mark.parametrize("k,n", [(264, 20), (2048, 130), (1096, 4100), (448, 2)])
 @pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_SWIGLU, hy.ACT_SOFTCAP])
 def test_few_rows_on_the_matrix_cores(r, k, n, act):
-    """A few rows on bf16 weights: every rows-per-pass form and tile count, K that ends inside a step, ragged columns; dense
-    (strided rows, per-row scale, add into the output, scattered results), a norm on the way in, one expert per row and
-    expert-sorted rows. Sums of k products differ from the reference's by their order."""
+    """A few rows on bf16 weights: every rows-per-pass form (the tile counts of wide outputs: the next test), K that ends inside
+    a step, ragged columns; dense (strided rows, per-row scale, add into the output, scattered results), a norm on the way in,
+    one expert per row and expert-sorted rows. Sums of k products differ from the reference's by their order."""
     gated = hy.act_gated(act)
     g = torch.Generator().manual_seed(r * 1000 + k + n + act)
     e = 3
@@ -512,6 +512,47 @@ def test_few_rows_on_the_matrix_cores(r, k, n, act):
         _close(run(w, new(), row_expert=ex.to(DEV)), per, 2e-5, "an expert per row")
     idx = order.to(torch.int32).to(DEV)
     _close(run(w, new(), dst_=idx, offs_=offs, a_idx=idx), per, 2e-5, "expert-sorted")
+
+
+@pytest.mark.parametrize("r,k,n,e,gated", [(9, 264, 16388, 0, True), (17, 264, 16388, 0, True), (32, 264, 16388, 0, True),
+                                           (16, 264, 32772, 0, False), (40, 264, 16372, 0, True), (64, 264, 16372, 0, True),
+                                           (40, 264, 2052, 8, True), (64, 264, 3284, 5, True), (64, 264, 5468, 3, True),
+                                           (20, 520, 2052, 8, True), (5, 264, 8196, 0, True), (8, 264, 16388, 0, False)])
+def test_few_rows_on_wide_outputs(r, k, n, e, gated):
+    """Two and four column tiles per workgroup at 1, 2 and 4 row tiles, dense and expert-sorted (``e`` experts): the outputs wide
+    enough for them, with a ragged last tile. Sums of k products differ from the reference's by their order."""
+    g = torch.Generator(device=DEV).manual_seed(r + n)
+    act = hy.ACT_SWIGLU if gated else hy.ACT_NONE
+    w = (torch.randn(max(e, 1), 2 * n if gated else n, k, generator=g, device=DEV) * k ** -0.5).to(torch.bfloat16)
+    x = torch.randn(r, k, generator=g, device=DEV)
+    ex = torch.randint(0, max(e, 1), (r,), generator=g, device=DEV).to(torch.int32)
+    idx = torch.argsort(ex, stable=True).to(torch.int32)
+    offs = torch.tensor([int((ex < i).sum()) for i in range(e + 1)], dtype=torch.int32, device=DEV)
+    ref = torch.empty(r, n, device=DEV)
+    for i in range(max(e, 1)):
+        sel = (ex == i).nonzero().squeeze(1)
+        ref[sel] = hy._act_cpu(x[sel].to(torch.bfloat16).float() @ w[i].float().t(), act, 0.0, 1.0)
+    out = torch.full((r, n + 4), 0.25, device=DEV)
+    if e:
+        hy.ext().linear_rows(x, idx, w, out[:, :n], idx, offs, None, r, act, 0.0, 1.0, None, None, 0.0, 0, False)
+    else:
+        hy.ext().linear_rows(x, None, w[0], out[:, :n], None, None, None, r, act, 0.0, 1.0, None, None, 0.0, 0, False)
+    _close(out[:, :n], ref, 2e-5, "wide output")
+    assert bool((out[:, n:] == 0.25).all())
+
+
+@pytest.mark.parametrize("r", [1, 2])
+@pytest.mark.parametrize("k,n,gated", [(4104, 516, False), (4104, 4100, False), (4104, 49156, False), (4104, 2052, True), (4104, 4100, True)])
+def test_normed_rows_too_long_to_walk(r, k, n, gated):
+    """One and two rows longer than the walking form holds, normed on the way in: one, two and four column tiles per workgroup.
+    (The norm's own sum differs by its order, which can round an operand to the neighbouring bf16.)"""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    act = hy.ACT_SWIGLU if gated else hy.ACT_NONE
+    w = (torch.randn(2 * n if gated else n, k, generator=g, device=DEV) * k ** -0.5).to(torch.bfloat16)
+    x, gain = torch.randn(r, k, generator=g, device=DEV), torch.rand(k, generator=g, device=DEV) + 0.5
+    normed = (x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5)) * gain
+    ref = hy._act_cpu(normed.to(torch.bfloat16).float() @ w.float().t(), act, 0.0, 1.0)
+    _close(hy.linear(hy.RmsInput(x, gain, 1e-5), w, act=act), ref, 3e-3, "normed")
 
 
 def test_few_rows_refuse_what_the_vector_unit_refuses():
