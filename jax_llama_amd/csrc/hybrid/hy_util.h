@@ -28,6 +28,7 @@ JLA_DEV float hy_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
 JLA_DEV float hy_gelu_tanh(float z) {
   return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
+JLA_DEV float hy_logsigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 JLA_DEV float hy_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 }  // namespace jla

@@ -5,7 +5,7 @@
 // Every launcher returns 0 on success, <0 on a shape/argument error, >0 for a hipError_t.
 //
 // Activations between kernels are fp32 in both number formats. "wbf16" selects the weight / cache element type: bf16
-// (matrix operands rounded to bf16, fp32 accumulation) or fp32 (exact-f32 MFMA, fp32 caches).
+// (matrix operands rounded to bf16, fp32 accumulation) or fp32 (fp32 products, fp32 caches).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -74,8 +74,8 @@ struct RowLinear {
 inline bool hy_act_gated(int act) {
   return act == HY_ACT_SWIGLU || act == HY_ACT_CLAMP_GLU || act == HY_ACT_GELU_GLU;
 }
-// R <= HY_GEMV_MAX_R and (offs == nullptr or row_expert != nullptr): one wave per output column (weights streamed once
-// per row group); else the 64 x 64 MFMA tiles (offs: expert-grouped).
+// rows up to which the vector GEMV takes a dense batch or rows with an expert each (one wave per output column, weights
+// streamed once per row group); linear_rows.hip lists the forms of hy_linear_rows in their order
 constexpr int HY_GEMV_MAX_R = 8;
 // the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, and the launch
 bool hy_rows_gemm_takes(const RowLinear& p);

@@ -1,22 +1,28 @@
 // Row-gathered, expert-grouped linear on row-major weights of any shape (no N % 16 / K % 32 packing constraint):
 //   out[dst(r), :] = act(A[src(r), :] @ W[expert(r)]^T)
-// A is fp32 in memory. With bf16 weights the A tile is rounded to bf16 while it is staged (v_mfma_f32_32x32x16_bf16,
-// fp32 accumulation); with fp32 weights everything stays fp32 on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32).
+// The dispatch of every such product (hy_linear_rows), and the forms that take what no other does. In this order:
+//   a handful of output columns (a router), any rows            the vector GEMV below
+//   one to 64 rows on bf16 weights, 16-byte rows                rows_gemv.hip, on the matrix cores
+//   up to 8 rows, or 64 sorted by expert, otherwise             the vector GEMV below (fp32 weights, odd or short K)
+//   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, 256-row tiles
+//   fp32 weights, 16-byte rows, K >= 512 (256 with many rows)   rows_f32.hip, split products on the bf16 matrix cores
+//   the rest                                                    the tiles below
+// The tiles round an fp32 A to bf16 while it is staged where the weights are bf16 (v_mfma_f32_32x32x16_bf16, fp32
+// accumulation); with fp32 weights everything stays fp32 (v_mfma_f32_32x32x2_f32).
 //
 //  * tiles: 64 x 64 or (with rows to fill them) 128 x 64 outputs per 256-thread workgroup, four waves of 32 x 32 /
 //    64 x 32, K staged 32 deep through LDS (several workgroups per CU hide each other's staging; a 128 x 128 tile with
-//    register prefetch and a 64-deep K stage measured slower). A prompt's bf16 rows with K >= 1024 run the 256-row tiles
-//    of rows_gemm.hip instead; these are for few rows per expert, short or odd K, fp32 and scaled activations. The activations may be a bf16 copy and the output bf16
+//    register prefetch and a 64-deep K stage measured slower). The activations may be a bf16 copy and the output bf16
 //    (the expert pair of a prompt: x -> bf16 once, hidden kept bf16), which halves the activation traffic. With an
 //    expert offset table the m-tiles of the launch are dealt to the experts in order (a workgroup finds its expert by
 //    walking the table; surplus workgroups exit), so one launch covers every expert of a token-sorted batch.
-//  * few rows (decode): a wave streams one or four weight rows once and dots them with up to 8 activation rows.
+//  * vector GEMV: a wave streams one or four weight rows once and dots them with up to 8 activation rows.
 //  * epilogues (RowAct): squared ReLU on one accumulator; gated forms accumulate the gate and the up rows of a column
 //    side by side: silu(g) * u, gelu_tanh(g) * u, or the clamped form g' sigmoid(alpha g') (u' + 1) with
 //    g' = min(g, limit), u' = clamp(u).
 //  * an optional per-row scale multiplies the activation row while it is staged (before the operand is rounded): the
 //    input-weighted experts of a score-routed mixture.
-//  * two linears of a few rows can share a launch (a mixture's experts beside its shared expert).
+//  * two linears of a few rows can share a launch of the vector GEMV (a mixture's experts beside its shared expert).
 // The table router's counting sort is here too.
 #include "hy_util.h"
 #include "hybrid.h"
@@ -351,6 +357,10 @@ static int lr_pass_rows(const RowLinear& p) {
   return want > 4 ? HY_GEMV_MAX_R : (want > 2 ? 4 : (want > 1 ? 2 : 1));
 }
 
+// The joint launch was measured against two launches of the vector GEMV. With bf16 weights two launches of rows_gemv.hip are now the
+// faster ones from two tokens on, and for one token on wide experts (us, joint | two; one token, top 2 of 8 experts beside a shared
+// one: gated 2048 x 1408 13.9 | 14.4, 4096 x 2048 33.2 | 25.6; two tokens 26.7 | 18.4, 66.7 | 36.9; four 38.9 | 26.0, 86.0 | 58.1):
+// the rule does not look at that yet.
 int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, float* ws, hipStream_t s) {
   auto plain = [](const RowLinear& x) {  // what the one-launch form takes
     return x.R > 0 && x.N > 0 && x.K > 0 && x.lda >= x.K && x.ldo >= x.N && x.E >= 1 && x.E <= 65535 && x.N < 8192 &&

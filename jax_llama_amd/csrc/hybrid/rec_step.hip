@@ -21,8 +21,6 @@ namespace jla {
 constexpr int RS_THREADS = 1024, RS_MAX = 256;
 enum { RS_MLSTM = 0, RS_TIMEMIX = 1, RS_RUNNING = 2, RS_DELTA = 3 };
 
-JLA_DEV float rs_logsigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
-
 // Sums of N numbers per thread over the first `nw` waves of the block; red holds 16 N floats. Every thread gets them.
 template <int N>
 JLA_DEV void rs_sum(float (&v)[N], int nw, float* red) {
@@ -69,7 +67,7 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
     const float xi = p.gate_i[(size_t)b * p.ldgate + h], xf = p.gate_f[(size_t)b * p.ldgate + h];
     const float zs = st[(size_t)td * ncols + vdim], m = p.mstate[(size_t)b * p.H + h];
     const float a = p.cap * tanhf((xi + p.gate_bias[h]) * (1.f / p.cap));
-    const float f = rs_logsigmoid(p.cap * tanhf((xf + p.gate_bias[p.H + h]) * (1.f / p.cap)));
+    const float f = hy_logsigmoid(p.cap * tanhf((xf + p.gate_bias[p.H + h]) * (1.f / p.cap)));
     m_new = fmaxf(f + m, a);
     const float keep = expf(f + m - m_new), write = expf(a - m_new), qs = q * p.q_scale, wk = write * k;
     floor_ = expf(-m_new);

@@ -80,7 +80,6 @@ int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* o
 JLA_DEV float rc_uniform(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-JLA_DEV float rc_logsigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
 // grid (H, B), one wave
 __global__ void __launch_bounds__(64) mlstm_prep_kernel(MlstmPrep p) {
@@ -104,7 +103,7 @@ __global__ void __launch_bounds__(64) mlstm_prep_kernel(MlstmPrep p) {
     if (t0 + 64 < p.S) gates(t0 + 64, xi_next, xf_next);  // (in flight behind this chunk's chain)
     // (a token past the end keeps m: f = 0, a = -inf)
     const float a = on ? p.cap * tanhf((xi + bi) * inv_cap) : -INFINITY;
-    const float f = on ? rc_logsigmoid(p.cap * tanhf((xf + bf) * inv_cap)) : 0.f;
+    const float f = on ? hy_logsigmoid(p.cap * tanhf((xf + bf) * inv_cap)) : 0.f;
     float m_before = 0.f, m_after = 0.f;
 #pragma unroll
     for (int l = 0; l < 64; ++l) {

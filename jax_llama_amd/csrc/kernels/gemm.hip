@@ -1001,7 +1001,7 @@ __global__ void __launch_bounds__(256, 1)
   const int tiles = tiles_m * tiles_n;
   const int split = wgid / tiles, pid = wgid - split * tiles;
   int tm, tn;
-  g4_tile_coords(pid, tiles_m, tiles_n, tm, tn, group_m);
+  row_tile_coords(pid, tiles_m, tiles_n, group_m, tm, tn);
   const int m0 = tm * G4_BM, n0 = tn * (32 * NJ);
   const int t0 = split * kc, KT = min(K >> 6, t0 + kc) - t0;
 
@@ -1043,7 +1043,7 @@ __global__ void __launch_bounds__(256, 1)
   const G4Epi ep{out, M, N, K, accumulate, out_f32, mirror, tiles_n, rms_eps, nullptr, rms_inv};
   for (int pid = wg; pid < tiles; pid += nwg) {
     int tm, tn;
-    g4_tile_coords(pid, tiles_m, tiles_n, tm, tn, group_m);
+    row_tile_coords(pid, tiles_m, tiles_n, group_m, tm, tn);
     const int m0 = tm * G4_BM, n0 = tn * G4_BN;
     // the lane index laundered once per tile: the lane-dependent address math of the main loop and the unrolled
     // epilogue would otherwise be hoisted out of the tile loop and kept live (spills)
@@ -1324,7 +1324,7 @@ static bool use_g4(int tile, int M, int K) {
          (tile == G4_TILE || tile == G4P_TILE || tile == G4D_TILE || (tile == 0 && g_g4_default && M > 128));
 }
 
-// Tile rasterisation: the launch order walks groups of gm m-tiles across every n-tile (g4_tile_coords), so the 32
+// Tile rasterisation: the launch order walks groups of gm m-tiles across every n-tile (row_tile_coords), so the 32
 // workgroups an XCD runs at once cover gm m-tiles x 32 / gm n-tiles. gm = 4 (4 x 8 tiles per XCD) beat 8 (the
 // round-4 order), 1, 2 and 16 on every Llama-3-8B projection at M = 2048 and 32768: qkv -7 / -9 %, o -3 / -8 %,
 // gate_up -5 / 0 %, down -5 / -6 % (profiles/r5_gemm4_group_m.jsonl). gemm_set_g4_group pins another (tools).

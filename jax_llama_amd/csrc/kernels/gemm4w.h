@@ -23,6 +23,7 @@
 // Reference ops: jax_llama/model.py:210 (q/k/v projections), :294 (wo), :338 (SwiGLU MLP), :736 (lm_head).
 #pragma once
 #include "common.h"
+#include "row_tiles.h"
 
 namespace jla {
 
@@ -30,15 +31,6 @@ constexpr int G4_BM = 256, G4_BN = 256, G4_BK = 64, G4_GROUP_M = 8;
 constexpr int G4_A_U4 = G4_BM * G4_BK * 2 / 16;  // 2048 u32x4 = 32 KiB
 constexpr int G4_B_U4 = G4_BN * G4_BK * 2 / 16;  // 2048 u32x4 = 32 KiB
 constexpr int G4_SLOT_U4 = G4_A_U4 + G4_B_U4;    // 64 KiB
-
-// launch-order tile index -> (m tile, n tile), M-grouped by gm so consecutive workgroups share W columns
-JLA_DEV void g4_tile_coords(int pid, int tiles_m, int tiles_n, int& tm, int& tn, int gm = G4_GROUP_M) {
-  const int in_group = gm * tiles_n;
-  const int first_m = (pid / in_group) * gm;
-  const int gsz = min(tiles_m - first_m, gm);
-  tm = first_m + (pid % in_group) % gsz;
-  tn = (pid % in_group) / gsz;
-}
 
 // The accumulators are pinned to AGPRs through inline asm: with the intrinsic, hipcc (ROCm 7.2) splits the 256
 // loop-carried accumulators between the two register files and shuffles them with v_accvgpr moves around every

@@ -1,4 +1,4 @@
-// Launch order of a tiled product over rows that may be sorted by expert.
+// Launch order of a tiled product, over rows that may be sorted by expert.
 #pragma once
 #include "common.h"
 

@@ -135,8 +135,8 @@ def prefetch(t: torch.Tensor) -> None:
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x [M, K] @ w [N, K]^T`` with fp32 inputs, accumulation and output (precision='highest' lm_head; GPU: the
-    exact-f32 MFMA kernel, csrc/kernels/gemm_f32.hip)."""
+    """``x [M, K] @ w [N, K]^T`` with fp32 inputs, accumulation and output (precision='highest' lm_head; GPU:
+    csrc/kernels/gemm_f32.hip, split products on the bf16 matrix cores, each exact to 2^-24 of itself)."""
     if not _is_gpu(x):
         return x.float() @ w.float().t()
     y = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)

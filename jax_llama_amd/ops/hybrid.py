@@ -4,7 +4,8 @@ Same dispatch rule as the rest of ``ops``: GPU tensors run the hand-written gfx9
 raises), CPU tensors run the PyTorch implementation below (the test / oracle path of the framework).
 
 Conventions: activations between ops are fp32 in both number formats. A weight (or cache) tensor's dtype selects the
-arithmetic: bf16 weights -> operands rounded to bf16, fp32 accumulation; fp32 weights -> exact fp32 products.
+arithmetic: bf16 weights -> operands rounded to bf16, fp32 accumulation; fp32 weights -> fp32 products (each exact to
+2^-24 of itself) and sums.
 
 Mechanisms (each with its constants as arguments, usable by any model of the registry):
   * ``linear`` / ``moe_table``: row-major weights of any shape; a token-id -> experts table routes a mixture of SwiGLU
@@ -189,8 +190,9 @@ class RmsInput:
         return self._value
 
 
-# rows up to which a GEMV norms its input itself: every wave repeats the row statistic, which beats a launch of the norm
-# kernel for one or two rows and loses to it from eight (measured on a 2048-wide stack: 8 rows 8 % slower fused)
+# rows up to which a product norms its input itself: every workgroup repeats the row statistic (the walking form once, the
+# vector GEMV in every wave), which beats a launch of the norm kernel for one or two rows and loses to it from eight (vector
+# GEMV, 2048-wide stack: 8 rows 8 % slower fused)
 FUSE_NORM_MAX_ROWS = 2
 
 
