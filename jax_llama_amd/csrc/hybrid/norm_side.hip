@@ -150,6 +150,21 @@ __global__ void __launch_bounds__(256) norm_residual_kernel(const float* y, int 
   }
 }
 
+// The sum over a block of T threads, the waves' sums in pairs: one behind the other, eight of them lose more than the four of 256
+// threads did (rows of 4096, error against 64 bits: 256 threads 5.95e-8, 512 one by one 6.05e-8, in pairs 5.92e-8). For one use
+// of red per launch.
+template <int T>
+JLA_DEV float ns_block_sum(float v, float* red) {
+  const int lane = threadIdx.x & 63;
+  v = wave_sum(v);
+  if (lane == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = red[lane & (T / 64 - 1)];
+#pragma unroll
+  for (int o = T / 128; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
 // The same with 16-byte accesses (D a multiple of 4, aligned rows): one workgroup brings a whole row in, so the instructions
 // between its loads show. Us before -> after: 1 x 2048 3.5 -> 2.5, 8 x 4096 with two summands 6.4 -> 3.0, 16384 x 4096 with two
 // summands 322 -> 199 (5.4 TB/s). T: about one 16-byte column group per thread (256 threads of a 4096-column row: 3.3 us).
@@ -187,7 +202,7 @@ __global__ void __launch_bounds__(T) norm_residual_vec_kernel(const float* y, in
       ss = 4 * ((int)threadIdx.x + T * u) < D ? fmaf(v[u][i], v[u][i], ss) : ss;
     }
   }
-  const float sc = 1.f / sqrtf(block_sum(ss, red) / (float)D + eps);
+  const float sc = 1.f / sqrtf(ns_block_sum<T>(ss, red) / (float)D + eps);
   float* to = (x ? x : out) + (size_t)m * D;
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
