@@ -15,8 +15,7 @@ JLA_DEV float ns_ld(const float* p) { return *p; }
 JLA_DEV float ns_ld(const bf16_t* p) { return bf2f(*p); }
 
 // One workgroup per row; with a gain w the row is RMS-normed (the row is read a second time, from the cache). W: consecutive
-// elements of a thread: 8 where that keeps every thread busy (rows of 2048 and more, 16 bytes per load), else 1 (5000 rows of
-// 64 | 257 | 1000 elements: 8 each 4.1 | 7.2 | 9.0 us, one each 3.2 | 4.7 | 7.9).
+// elements of a thread: 8 where that keeps every thread busy and every access is of 16 bytes, else 1 (hy_embed_rows).
 template <typename WT, int W, int NORM>
 __global__ void __launch_bounds__(256) embed_rows_kernel(const int32_t* ids, const WT* table, int V, int ld, int col0,
                                                          float scale, float* out, int D, int copies, const float* w, float eps) {
@@ -73,11 +72,20 @@ int hy_embed_rows(const int32_t* ids, const void* table, int wbf16, int V, int l
     if (w) EMBED_N(WT, W, 1);     \
     else EMBED_N(WT, W, 0);       \
   } while (0)
+  // Eight elements per thread from 2048 columns on (5000 rows of 64 | 257 | 1000 elements: 8 each 4.1 | 7.2 | 9.0 us, one each 3.2 |
+  // 4.7 | 7.9; 4000 bf16 rows of 4096: 16.4, 18.4) and only with 16-byte rows on both sides: otherwise eight neighbouring
+  // accesses of every thread fall on different lines (4000 bf16 rows of 2050 | 4100: 26.7 | 20.9, one each 11.2 | 18.6). Several
+  // copies are bound by their stores, whole lines of which one element each writes at once (two copies of 4000 bf16 rows of 2048:
+  // 16.4, 14.3), until the row is long (8192: 45, 47).
+  const int vec = wbf16 ? 8 : 4;
+  auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  const bool wide = D >= (copies == 1 ? 2048 : 8192) && D % 4 == 0 && ld % vec == 0 && col0 % vec == 0 && aligned(table) &&
+                    aligned(out) && (!w || aligned(w));
   if (wbf16) {
-    if (D >= 2048) EMBED(bf16_t, 8);
+    if (wide) EMBED(bf16_t, 8);
     else EMBED(bf16_t, 1);
   } else {
-    if (D >= 2048) EMBED(float, 8);
+    if (wide) EMBED(float, 8);
     else EMBED(float, 1);
   }
 #undef EMBED

@@ -843,6 +843,18 @@ def test_embedding_with_its_norm(d, ld, col0):
             _close(got, ref, 0.0 if norm is None else 2e-6, "embedding")
 
 
+@pytest.mark.parametrize("d,ld,col0", [(2048, 2048, 0), (2052, 2060, 4), (2050, 2050, 0), (2051, 2064, 8), (8192, 8192, 0), (8196, 8200, 0)])
+@pytest.mark.parametrize("copies", [1, 2])
+def test_embedding_rows_of_any_alignment(d, ld, col0, copies):
+    for dt in DTYPES:
+        table, ids, gw = _rand(9, ld, dt=dt), torch.tensor([0, 8, 7, 1], dtype=torch.int32), torch.rand(d) + 0.5
+        for norm in (None, gw):
+            args = dict(col0=col0, ncols=d, scale=0.5, copies=copies, eps=1e-6)
+            ref = hy.embed_rows(ids, table, norm=norm, **args)
+            got = hy.embed_rows(ids.to(DEV), table.to(DEV), norm=norm.to(DEV) if norm is not None else None, **args)
+            _close(got, ref, 0.0 if norm is None else 2e-6, "embedding")
+
+
 @pytest.mark.parametrize("b,d,n", [(1, 2048, 5), (2, 4096, 5), (3, 40, 2), (1, 4100, 1), (2, 257, 3)])
 def test_token_shift_with_its_norm(b, d, n):
     x, gw, prev, mu = _rand(b, d), torch.rand(d) + 0.5, _rand(b, d), torch.rand(n, d)
