@@ -450,14 +450,19 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 
 // up to 64 rows, and up to 32 of a wide output, whose tiles fill the chip (64 rows x 32000 columns, K 2048: 70 us on the
 // tiles, 82 here); a short K is over before the waves' sum pays (K 64: one row 3.2 us on the vector unit, 3.6 here, 64 rows
-// 4.8 on the tiles, 5.3 here). Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
+// 4.8 on the tiles, 5.3 here), and with very many columns the tiles stream it as fast (9 | 17 | 32 rows of K 256 x N 32000: weights in
+// no cache 9.9 | 14.3 | 16.5 us here, 10.6 | 11.3 | 12.4 on the tiles, in a cache 9.3 | 13.0 | 15.5 and 6.8 | 7.5 | 8.7; N 16384, no
+// cache: 6.4 | 8.3 | 9.8 here, 8.7 | 9.5 | 10.4 there; K 512 x N 32000: 10.8 | 15.5 | 17.6, 17.7 | 18.8 | 19.8).
+// Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
 constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 2;
+constexpr int RV_SHORT_K = 512, RV_SHORT_WIDE = 20480;
 
 bool hy_rows_gemv_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return p.wbf16 && !p.a_bf16 && !p.out_bf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
          (p.offs || p.tab || (p.row_expert ? p.R <= HY_GEMV_MAX_R : p.E == 1)) && p.K % 8 == 0 &&
-         p.K >= (p.R <= 2 ? 256 : (p.R <= 32 ? 64 : 128)) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
+         p.K >= (p.R <= 2 ? 256 : (p.R <= 32 ? 64 : 128)) &&
+         !(p.R > HY_GEMV_MAX_R && p.E == 1 && !p.offs && p.K < RV_SHORT_K && p.N >= RV_SHORT_WIDE) && p.lda % 4 == 0 && p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) &&
          (!p.a_norm_w || (p.R <= RV_MAX_NORM_ROWS && !p.a_scale && !p.offs && !p.row_expert && (p.a_norm_one || aligned(p.a_norm_w))));
 }
 

@@ -517,10 +517,13 @@ def test_few_rows_on_the_matrix_cores(r, k, n, act):
 @pytest.mark.parametrize("r,k,n,e,gated", [(9, 264, 16388, 0, True), (17, 264, 16388, 0, True), (32, 264, 16388, 0, True),
                                            (16, 264, 32772, 0, False), (40, 264, 16372, 0, True), (64, 264, 16372, 0, True),
                                            (40, 264, 2052, 8, True), (64, 264, 3284, 5, True), (64, 264, 5468, 3, True),
-                                           (20, 520, 2052, 8, True), (5, 264, 8196, 0, True), (8, 264, 16388, 0, False)])
+                                           (20, 520, 2052, 8, True), (5, 264, 8196, 0, True), (8, 264, 16388, 0, False),
+                                           (1, 264, 1021, 0, False), (2, 1024, 1030, 0, False), (3, 72, 1022, 0, False), (4, 1024, 2050, 0, False),
+                                           (4, 1032, 2050, 0, False), (2, 520, 602, 2, False), (9, 504, 20484, 0, False),
+                                           (32, 256, 20482, 0, False), (9, 512, 20484, 0, False), (32, 512, 20482, 0, False)])
 def test_few_rows_on_wide_outputs(r, k, n, e, gated):
     """Two and four column tiles per workgroup at 1, 2 and 4 row tiles, dense and expert-sorted (``e`` experts): the outputs wide
-    enough for them, with a ragged last tile. Sums of k products differ from the reference's by their order."""
+    enough for them, with a ragged last tile; short K on both sides of the tiles' line. Sums of k products differ from the reference's by their order."""
     g = torch.Generator(device=DEV).manual_seed(r + n)
     act = hy.ACT_SWIGLU if gated else hy.ACT_NONE
     w = (torch.randn(max(e, 1), 2 * n if gated else n, k, generator=g, device=DEV) * k ** -0.5).to(torch.bfloat16)
