@@ -456,6 +456,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 // Rows with an expert of their own and no offsets: as many as the vector unit's form takes.
 constexpr int RV_MAX_ROWS = 64, RV_MAX_WIDE_ROWS = 32, RV_WIDE = 16384, RV_MAX_NORM_ROWS = 2;
 constexpr int RV_SHORT_K = 512, RV_SHORT_WIDE = 20480;
+constexpr int RV_PAIR_K = 1024;
 
 bool hy_rows_gemv_takes(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
@@ -521,9 +522,11 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   const long long tiles = (gated ? 2LL : 1LL) * ((p.N + G - 1) / G);
   // one tile per workgroup until there are a few workgroups for every compute unit; then tiles share the workgroup's
   // activation reads, which weigh more the more rows there are (8 rows, K 4096 x N 4096: 1 / 2 / 4 tiles 15.0 / 12.3 / 14.8
-  // us; K 2048 x N 32000: 46 / 35 / 29; one row 27.9 / 24.5 / 27.6)
+  // us; K 2048 x N 32000: 46 / 35 / 29; one row 27.9 / 24.5 / 27.6). Up to K 1024, where each wave has one batch of loads, two
+  // tiles pay from one workgroup per compute unit on: K 1024 x N 2048, weights in no cache, one row 4.1 -> 3.4 us (vector
+  // unit 4.6), four rows 5.5 -> 3.6; weights in a cache, one row 4.3 -> 3.3 (3.5); K 4096 5.9 -> 6.8.
   const long long all = tiles * groups;
-  int nt = gated || mt > 1 || all >= (G == 4 ? 1024 : 512) ? 2 : 1;
+  int nt = gated || mt > 1 || all >= (G == 4 ? (p.K <= RV_PAIR_K ? 256 : 1024) : 512) ? 2 : 1;
   if (all >= (G > 4 ? 2048 : (gated ? 2048 : 12288))) nt = 4;
   const long long wgs = (tiles + nt - 1) / nt;
   if (wgs > 0x7fffffffLL) return -4;
