@@ -139,11 +139,13 @@ __global__ void __launch_bounds__(256) delta_prep_run_kernel(DeltaPrep p) {
   }
 }
 
-// (with fewer tokens the runs leave the chip empty: 64 tokens 8.0 -> 11.3 us, 600 tokens 11.3 -> 9.3)
-constexpr int DP_MIN_TOKENS = 512;
+// With fewer tokens, or with few heads, the runs leave the chip empty: 64 tokens 8.0 -> 11.3 us, 600 tokens 11.3 -> 9.3; 513 tokens of
+// 2 | 4 | 8 heads (66 | 99 | 165 workgroups) 5.4 -> 6.6 | 6.0 -> 7.0 | 7.5 -> 7.1.
+constexpr int DP_MIN_TOKENS = 512, DP_MIN_WORKGROUPS = 160;
 static bool dp_runs(const DeltaPrep& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  return p.S >= 2 * DP_SPAN && p.B * (long long)p.S >= DP_MIN_TOKENS && p.taps == 4 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.ld % 4 == 0 &&
+  return p.S >= 2 * DP_SPAN && p.B * (long long)p.S >= DP_MIN_TOKENS &&
+         (long long)((p.S + DP_SPAN - 1) / DP_SPAN) * ((2 * p.G + p.H + 4) / 4) * p.B >= DP_MIN_WORKGROUPS && p.taps == 4 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.ld % 4 == 0 &&
          p.B <= 65535 && aligned(p.proj) && aligned(p.conv_w) && aligned(p.qn) && aligned(p.kn) && aligned(p.vc);
 }
 

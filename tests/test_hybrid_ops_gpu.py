@@ -1034,7 +1034,8 @@ def test_chunks_keep_tokens_before_a_number_that_is_none(kind, b, s, h, dim, vdi
 
 
 @pytest.mark.parametrize("b,s,h,g,dim,vdim", [(17, 31, 2, 1, 64, 64), (16, 32, 2, 1, 128, 128), (16, 33, 6, 3, 64, 128), (2, 257, 4, 2, 128, 64),
-                                              (1, 511, 2, 2, 64, 64), (1, 527, 2, 2, 64, 64), (8, 64, 2, 1, 80, 64)])
+                                              (1, 511, 2, 2, 64, 64), (1, 527, 2, 2, 64, 64), (8, 64, 2, 1, 80, 64),
+                                              (40, 32, 2, 1, 128, 128), (39, 32, 2, 1, 64, 128), (2, 257, 10, 5, 128, 64), (1, 527, 14, 7, 64, 64)])
 def test_delta_preparation_in_runs(b, s, h, g, dim, vdim):
     """Convolutions, unit norms and gates of a prompt in runs of tokens (and on both sides of that form) against the CPU op, the
     tail of the call before included."""
