@@ -102,10 +102,11 @@ __global__ void __launch_bounds__(256) argmax_splits_kernel(const float2* __rest
   }
 }
 
-// workgroups per row: about 1024 in all, at most 64 and at least 2048 columns each; a row that one workgroup reads in two
-// rounds does not pay for the second launch (1 | 500 rows of 5000 columns: two workgroups 5.5 | 6.8 us, one 3.6 | 4.4)
+// workgroups per row: about 1024 in all, at most 64 and at least 2048 columns each; a row that one workgroup reads in three
+// rounds does not pay for the second launch (1 | 500 rows of 5000 columns: two workgroups 5.5 | 6.8 us, one 3.6 | 4.4; 200 rows of
+// 12001 columns: 6.2, 5.5)
 static int argmax_splits(int B, int V) {
-  if (B <= 0 || V < 8192) return 1;
+  if (B <= 0 || V < 12288) return 1;
   const int want = (1024 + B - 1) / B, most = V / 2048;
   return max(1, min(min(want, most), 64));
 }
