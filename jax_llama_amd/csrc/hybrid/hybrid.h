@@ -77,8 +77,10 @@ inline bool hy_act_gated(int act) {
 // rows up to which the vector GEMV takes a dense batch or rows with an expert each (one wave per output column, weights
 // streamed once per row group); linear_rows.hip lists the forms of hy_linear_rows in their order
 constexpr int HY_GEMV_MAX_R = 8;
-// the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, and the launch
+// the large-tile form of a prompt's bf16 rows (rows_gemm.hip): whether it takes a call, whether rounding fp32 rows for it pays,
+// and the launch
 bool hy_rows_gemm_takes(const RowLinear& p);
+bool hy_rows_gemm_pays(const RowLinear& p);
 // the fp32 tiles as split products on the bf16 matrix cores (rows_f32.hip)
 bool hy_rows_f32_takes(const RowLinear& p);
 long long hy_rows_f32_floats(const RowLinear& p);  // scratch of its split-K form (0: none)

@@ -194,6 +194,18 @@ bool hy_rows_gemm_takes(const RowLinear& p) {
          wrows * p.K * 2 < 0x100000000LL;  // (32-bit offsets into an expert's weights)
 }
 
+// For a caller who has yet to round its rows to bf16: a dense gated matrix of a short K whose 64-row tiles of fp32 rows all run at
+// once is faster there. Us, 64-row tiles | here with the rounding: K 1024, gated N 1024, 300 | 512 | 700 rows 27.9 | 29.6, 27.7 |
+// 30.2, 32.9 | 30.6; N 512, 700 | 1000 rows 28.0 | 31.0, 38.3 | 32.1; N 1376, 256 rows 39.7 | 29.7; K 1152, 512 rows of N 512 |
+// 1024 31.1 | 33.0, 31.2 | 32.3; K 1280 even.
+constexpr int RG_GATED_K = 1152, RG_GATED_N = 1024, RG_GATED_ROWS = 704, RG_GATED_TILES = 128;
+
+bool hy_rows_gemm_pays(const RowLinear& p) {
+  const bool few = hy_act_gated(p.act) && !p.offs && p.K <= RG_GATED_K && p.N <= RG_GATED_N && p.R <= RG_GATED_ROWS &&
+                   (p.R + 63) / 64 * ((p.N + 63) / 64) <= RG_GATED_TILES;
+  return hy_rows_gemm_takes(p) && !few;
+}
+
 int hy_rows_gemm(const RowLinear& p, hipStream_t s) {
   const int gated = hy_act_gated(p.act), E = p.offs ? p.E : 1;
   const long long wrows = gated ? 2LL * p.N : p.N;

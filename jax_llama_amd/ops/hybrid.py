@@ -328,7 +328,7 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     if act == ACT_NONE and norm_w is None and _use_packed_gemm(x, w):
         from . import linear as packed_linear
         return packed_linear(_bf16_rows(x), _packed_weight(w), out_dtype=F32)
-    if act_gated(act) and norm_w is None and x.shape[0] >= PACKED_GEMM_MIN_M and ext().rows_gemm_takes(x.shape[0], w, int(act)):
+    if act_gated(act) and norm_w is None and x.shape[0] >= PACKED_GEMM_MIN_M and ext().rows_gemm_pays(x.shape[0], w, int(act)):
         # a prompt's gated product: bf16 rows (the operands they would be rounded to anyway) on the large tiles
         xb = _bf16_rows(x) if x.is_contiguous() and x.numel() % 8 == 0 else x.to(BF16).contiguous()
         out = torch.empty(x.shape[0], n, dtype=out_dtype, device=x.device)

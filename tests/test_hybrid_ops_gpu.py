@@ -441,7 +441,7 @@ def test_moe_grouped_and_the_stream_update(dt, m, experts, identity, top):
     _close(hy.ff_dense(x.to(DEV), s_up.to(DEV), s_down.to(DEV)), hy.ff_dense(x, s_up, s_down), 2e-5, "one-accumulator FF")
 
 
-@pytest.mark.parametrize("counts", [[300], [255, 0, 257, 1, 512], [128] * 7 + [0, 33]])
+@pytest.mark.parametrize("counts", [[300], [800], [255, 0, 257, 1, 512], [128] * 7 + [0, 33]])
 @pytest.mark.parametrize("k,n", [(1024, 260), (1088, 516), (1024, 8192 + 4)])
 @pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_RELU2, hy.ACT_SWIGLU, hy.ACT_CLAMP_GLU, hy.ACT_GELU_GLU])
 def test_rows_on_the_large_tiles(counts, k, n, act):
