@@ -96,7 +96,7 @@ def embedding(ids: torch.Tensor, table: torch.Tensor, mirror: Optional[torch.Ten
             mirror.copy_(out.to(BF16))
         return out
     out = torch.empty(ids.numel(), table.shape[1], dtype=torch.float32, device=table.device)
-    ext().embedding(ids.reshape(-1).to(torch.int32), table, out, mirror)
+    ext().embedding(ids.reshape(-1).to(torch.int32).contiguous(), table, out, mirror)  # (a column of a batch has a stride)
     return out
 
 

@@ -58,6 +58,19 @@ def test_greedy_generation_gpu_matches_cpu_path(batch):
     assert torch.equal(got[:, :11], toks)
 
 
+def test_next_tokens_as_a_column_of_a_batch():
+    cfg = gpu_config()
+    _, gpu, _ = _pair(cfg)
+    ids = torch.randint(3, cfg.vocab_size, (3, 8), generator=torch.Generator().manual_seed(1), dtype=torch.int32).cuda()
+    pos = torch.arange(8, dtype=torch.int32, device="cuda").expand(3, 8).contiguous()
+    got = []
+    for column in (lambda t, i: t[:, i:i + 1], lambda t, i: t[:, i:i + 1].contiguous()):
+        cache = gpu.init_cache(3, 8)
+        gpu(ids[:, :5].contiguous(), position_ids=pos[:, :5], past_key_values=cache)
+        got.append([gpu(column(ids, i), position_ids=column(pos, i), past_key_values=cache).logits for i in range(5, 8)])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 def test_graph_replay_matches_eager():
     cfg = gpu_config()
     _, gpu, _ = _pair(cfg, seed=5)
