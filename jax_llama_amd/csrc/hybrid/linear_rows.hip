@@ -2,6 +2,7 @@
 //   out[dst(r), :] = act(A[src(r), :] @ W[expert(r)]^T)
 // The dispatch of every such product (hy_linear_rows), and the forms that take what no other does. In this order:
 //   a handful of output columns (a router), any rows            the vector GEMV below
+//   one or two normed rows, K <= 512, N <= 2048                 the vector GEMV below
 //   one to 64 rows on bf16 weights, 16-byte rows                rows_gemv.hip, on the matrix cores
 //   up to 8 rows, or 64 sorted by expert, otherwise             the vector GEMV below (fp32 weights, odd or short K)
 //   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, 256-row tiles
@@ -410,6 +411,14 @@ long long hy_linear_rows_floats(const RowLinear& p) {
   return hy_rows_f32_floats(p);
 }
 
+// One or two normed rows of a short K and few columns are a launch and little else, and the walking form stages its rows first: K 512,
+// weights in no cache, one | two rows of N 130 3.1 | 3.9 us on the vector unit, 3.75 | 4.6 walking, N 1000 3.9 | 4.65 and 4.4 | 5.3, N 2048
+// 4.2 | 5.1 and 4.4 | 5.5. From N 5152, or K 640 (N 256: 4.6 | 5.5 and 4.2 | 5.1), walking is the faster one.
+constexpr int HY_NORMED_GEMV_MAX_K = 512, HY_NORMED_GEMV_MAX_N = 2048;
+static bool lr_short_normed(const RowLinear& p) {
+  return p.a_norm_w && !p.a_norm_one && p.K <= HY_NORMED_GEMV_MAX_K && p.N <= HY_NORMED_GEMV_MAX_N;
+}
+
 int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s) {
   if (p.R < 0 || p.N <= 0 || p.K <= 0 || p.lda < p.K || p.ldo < p.N || p.E < 1) return -1;
   if (p.act < HY_ACT_NONE || p.act > HY_ACT_GELU_GLU) return -8;
@@ -421,7 +430,7 @@ int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s) {
   if (p.offs && p.E > 65535) return -2;
   const bool grouped = lr_grouped(p);
   const bool small = hy_linear_rows_is_gemv(p);
-  if (!lr_skinny(p) && hy_rows_gemv_takes(p)) return hy_rows_gemv(p, s);
+  if (!lr_skinny(p) && !lr_short_normed(p) && hy_rows_gemv_takes(p)) return hy_rows_gemv(p, s);
   if (p.a_norm_w && (!small || p.a_bf16)) return -10;  // (the tiles take a normed activation, they do not norm it)
   if (small) {
     if (p.a_bf16 || p.out_bf16) return -7;  // (the GEMV reads and writes fp32)

@@ -308,6 +308,16 @@ def test_linear_norms_its_input(dt, m, n):
     _close(got, ref, 2e-5 if dt == torch.float32 else 4e-3, "fused input norm")
 
 
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("n,k", [(2048, 512), (2052, 512), (2048, 520), (40, 256), (17, 504)])
+def test_linear_norms_a_short_row(m, n, k):
+    """Both sides of the line between the vector GEMV and the walking form."""
+    x, gain, w = _rand(m, k, std=3.0), torch.rand(k) + 0.5, _rand(n, k, dt=torch.bfloat16, std=k ** -0.5)
+    ref = hy.linear(hy.RmsInput(x, gain, 1e-5), w)
+    # (a normed operand that differs in its last fp32 bit can round to the neighbouring bf16)
+    _close(hy.linear(hy.RmsInput(x.to(DEV), gain.to(DEV), 1e-5), w.to(DEV)), ref, 4e-3, "fused input norm")
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("m,top", [(1, 2), (4, 2), (5, 2)])
 def test_moe_routed_norms_its_input(dt, m, top):
