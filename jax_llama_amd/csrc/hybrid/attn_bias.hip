@@ -27,8 +27,7 @@
 // bias column) are indexed by it. Prefill: one wave runs both maps of its query (plain), or a pair of waves runs one map
 // each over the same 32 queries and joins them through LDS (MFMA). Decode: the splits of both maps side by side, joined by
 // the merge.
-#include "hy_util.h"
-#include "hybrid.h"
+#include "attn_span.h"
 
 namespace jla {
 
@@ -100,37 +99,6 @@ constexpr int AB_MAX_DIM = 1024;  // q head held in LDS per wave (keys may be wi
                                   // with a rotated part behind the latent)
 constexpr int AB_MAX_VREG = 8;    // value columns per lane: vdim <= 512
 
-// The keys a query at slot qi sees: slots [0, kf) (kept first keys, only beside a window) and [lo, qi], numbered
-// 0 .. n - 1 in that order.
-struct AbSpan {
-  int kf, lo, n;
-};
-JLA_DEV AbSpan ab_span(const AttnBias& p, int qi) {
-  AbSpan sp;
-  sp.lo = p.chunk > 0 ? qi / p.chunk * p.chunk : (p.window > 0 ? max(0, qi - p.window + 1) : 0);
-  sp.kf = p.window > 0 ? min(p.keep_first, sp.lo) : 0;
-  sp.n = sp.kf + qi + 1 - sp.lo;
-  return sp;
-}
-// query head vh = map vh % maps of output head vh / maps: its key / value head, and its keys' offset within a key row
-struct AbMap {
-  int g, koff;
-};
-JLA_DEV AbMap ab_map(const AttnBias& p, int vh) {
-  const int h = vh / p.maps;
-  return {h / (p.H / p.G), (vh - h * p.maps) * p.dim};
-}
-JLA_DEV int ab_key(const AbSpan& sp, int v) { return v < sp.kf ? v : sp.lo + (v - sp.kf); }
-// gate of column c of head h: one per head, or one per column
-JLA_DEV float ab_gate(const AttnBias& p, size_t m, int h, int c) {
-  return p.gate ? hy_sigmoid(p.gate[m * p.ldg + (p.gate_cols ? h * p.vdim + c : h)]) : 1.f;
-}
-JLA_DEV void ab_out(const AttnBias& p, size_t m, int h, int c, float v) {
-  const size_t at = m * p.ldo + (size_t)h * p.vdim + c;
-  if (p.out_bf16) reinterpret_cast<bf16_t*>(p.out)[at] = f2bf(v);
-  else reinterpret_cast<float*>(p.out)[at] = v;
-}
-
 // One wave: visible keys number [j_lo, j_hi) of query (b, query head h) at slot qi (span); returns the running max m, sum l and
 // unnormalised acc. with_sink: the wave whose keys start the row also counts the head's sink.
 template <typename CT, int VREG>  // VREG: value columns per lane (vdim <= 64 VREG)
@@ -200,14 +168,6 @@ JLA_DEV void ab_wave(const AttnBias& p, const float* qs, int b, int h, int qi, c
       }
     }
   }
-}
-
-// visible keys number [j_lo, j_hi) of decode split sp: the query's n visible keys dealt to the splits in runs of 64
-JLA_DEV void ab_split_range(const AttnBias& p, const AbSpan& span, int sp, int& j_lo, int& j_hi) {
-  const int n = span.n;
-  const int per = ((n + p.splits - 1) / p.splits + 63) / 64 * 64;
-  j_lo = min(n, sp * per);
-  j_hi = min(n, j_lo + per);
 }
 
 // prefill of differential heads: grid (ceil(S / 4), H, B), one wave per query, its two maps one after the other

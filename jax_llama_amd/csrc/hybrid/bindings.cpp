@@ -661,6 +661,81 @@ void attn_bias(Tensor q, Tensor kc, Tensor vc, Tensor slot, double scale, double
   rc(jla::hy_attn_bias(p, stream()), "attn_bias");
 }
 
+// One token of an attention layer in one launch; false (nothing done) where its shapes are not the kernel's.
+bool attn_step(Tensor proj, Tensor kc, Tensor vc, Tensor slot, Tensor positions, int64_t H, bool own, Tensor tickets, double scale,
+               double softcap, OptT bias, Tensor out, int64_t seen, OptT sink, int64_t chunk, OptT head_scale, bool rope,
+               double eps, double temp_coef, int64_t temp_every, OptT q_w, OptT k_w, bool norm_v, OptT col_bias, OptT qk_freq,
+               OptT v_freq, bool turn, double turn_sign, double turn_gain) {
+  jla::AttnStep p{};
+  jla::AttnBias& a = p.a;
+  check(kc.dim() == 4 && vc.dim() == 4 && kc.size(0) == vc.size(0) && kc.size(1) == vc.size(1) && kc.size(2) == vc.size(2),
+        "attn_step: cache shapes");
+  a.cbf16 = wtype(kc, "k cache");
+  check(wtype(vc, "v cache") == a.cbf16, "attn_step: cache dtypes differ");
+  a.B = kc.size(0); a.G = kc.size(1); a.T = kc.size(2); a.dim = a.ldk = kc.size(3); a.vdim = a.ldv = vc.size(3);
+  a.S = 1; a.H = H; a.maps = 1;
+  check(H >= 1 && H % a.G == 0, "attn_step: heads");
+  a.kc = kc.data_ptr();
+  a.vc = vc.data_ptr();
+  a.splits = jla::hy_attn_decode_splits(a.B, a.H, std::max<int64_t>(1, std::min<int64_t>(seen, a.T)));
+  if (!jla::hy_attn_step_takes(p) || tickets.numel() < (int64_t)a.B * H * jla::AS_TICKET) return false;
+  const int64_t cols = H * a.dim + (own ? (int64_t)a.G * (a.dim + a.vdim) : 0);
+  check(proj.dim() == 2 && proj.size(0) == a.B, "attn_step: proj rows");
+  p.proj = rows2d(proj, "proj", cols, &p.ld);
+  p.own = own;
+  p.positions = i32(positions, "positions", a.B);
+  a.slot = i32(slot, "slot", 1);
+  a.scale = scale;
+  a.softcap = softcap;
+  if (bias.has_value()) {
+    check(bias->dim() == 2 && bias->size(1) == H, "attn_step: bias is [distances, heads]");
+    a.bias = f32(*bias, "bias");
+    a.nbias = bias->size(0);
+  }
+  if (sink.has_value()) {
+    check(sink->numel() == H, "attn_step: one sink per head");
+    a.sink = f32(*sink, "sink");
+  }
+  check(chunk >= 0 && chunk <= INT32_MAX, "attn_step: chunk");
+  a.chunk = chunk;
+  if (head_scale.has_value()) {
+    check(head_scale->numel() == H, "attn_step: one factor per head");
+    a.head_scale = f32(*head_scale, "head_scale");
+  }
+  a.out = slice2d_any(out, "out", a.B, (int64_t)H * a.vdim, &a.ldo, &a.out_bf16);
+  p.rope = rope;
+  p.eps = eps; p.temp_coef = temp_coef; p.temp_every = temp_every; p.norm_v = norm_v;
+  if (q_w.has_value()) {
+    check(q_w->numel() == a.dim, "attn_step: q_w is [dim]");
+    p.q_w = f32(*q_w, "q_w");
+  }
+  if (k_w.has_value()) {
+    check(k_w->numel() == a.dim, "attn_step: k_w is [dim]");
+    p.k_w = f32(*k_w, "k_w");
+  }
+  if (col_bias.has_value()) {
+    check(col_bias->numel() == H * a.dim + (int64_t)a.G * (a.dim + a.vdim), "attn_step: one bias per projection column");
+    p.col_bias = f32(*col_bias, "col_bias");
+  }
+  if (qk_freq.has_value() && qk_freq->numel() > 0) {
+    p.qk_half = qk_freq->numel();
+    check(2 * p.qk_half <= a.dim, "attn_step: more rotated numbers than a head holds");
+    p.qk_freq = f64(*qk_freq, "qk_freq");
+  }
+  if (v_freq.has_value() && v_freq->numel() > 0) {
+    p.v_half = v_freq->numel();
+    check(2 * p.v_half <= a.vdim, "attn_step: more rotated numbers than a value head holds");
+    p.v_freq = f64(*v_freq, "v_freq");
+  }
+  p.turn = turn;
+  p.turn_sign = turn_sign; p.turn_gain = turn_gain;
+  p.tickets = i32w(tickets, "tickets", (int64_t)a.B * H * jla::AS_TICKET);
+  const Tensor ws = torch::empty({(int64_t)a.B * H * a.splits * (a.vdim + 2)}, out.options().dtype(torch::kFloat32));
+  a.ws = f32w(ws, "ws");
+  rc(jla::hy_attn_step(p, stream()), "attn_step");
+  return true;
+}
+
 jla::DeltaPrep delta_args(const Tensor& proj, int64_t B, int64_t S, int64_t H, int64_t G, int64_t dim, int64_t vdim,
                           const Tensor& conv_w, const Tensor& conv_state) {
   jla::DeltaPrep p{};
@@ -1080,6 +1155,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("gate_cols") = false, py::arg("maps") = 1, py::arg("diff_lambda") = 0.0, py::arg("diff_eps") = 0.0,
         py::arg("diff_gain") = 1.0, py::arg("turn_pos") = py::none(), py::arg("turn_freq") = py::none(),
         py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
+  m.def("attn_step", &attn_step, py::arg("proj"), py::arg("kc"), py::arg("vc"), py::arg("slot"), py::arg("positions"), py::arg("H"),
+        py::arg("own"), py::arg("tickets"), py::arg("scale"), py::arg("softcap"), py::arg("bias"), py::arg("out"), py::arg("seen"),
+        py::arg("sink") = py::none(), py::arg("chunk") = 0, py::arg("head_scale") = py::none(), py::arg("rope") = false,
+        py::arg("eps") = 0.0, py::arg("temp_coef") = 0.0, py::arg("temp_every") = 1, py::arg("q_w") = py::none(),
+        py::arg("k_w") = py::none(), py::arg("norm_v") = true, py::arg("col_bias") = py::none(), py::arg("qk_freq") = py::none(),
+        py::arg("v_freq") = py::none(), py::arg("turn") = false, py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);

@@ -311,6 +311,33 @@ int hy_attn_bias(const AttnBias& p, hipStream_t s);
 long long hy_attn_prefill_ws_bytes(int B, int S, int G, int dim, int vdim, int T, int cbf16);
 int hy_attn_decode_splits(int B, int H, int t_cap);
 
+constexpr int AS_TICKET = 32;  // int32s from a head's ticket to the next: counts on one line of memory go one behind the other
+
+// One token per row: hy_attn_prep or (rope) hy_rope_prep, the cache write, hy_attn_bias and its merge in one launch
+// (attn_step.hip). a: the arguments of hy_attn_bias without q and turn_*.
+struct AttnStep {
+  AttnBias a;
+  const float* proj;  // [B, ld]: q heads at column 0, then (own) k heads, then v heads
+  int ld;
+  int own;            // the layer brings its own keys and values, which go to the cache at the slot
+  const int32_t* positions;  // [B]
+  int rope;
+  float eps, temp_coef;  // norms (rope = 0), as AttnPrep
+  int temp_every, norm_v;
+  const float* q_w;
+  const float* k_w;
+  const float* col_bias;  // rotations (rope = 1), as RopePrep
+  const double* qk_freq;
+  int qk_half;
+  const double* v_freq;
+  int v_half;
+  int turn;  // the output turned by turn_sign times the position over v_freq, then times turn_gain
+  float turn_sign, turn_gain;
+  int32_t* tickets;  // [B * H * AS_TICKET] zeros, left as zeros: not shared between launches that may run at the same time
+};
+bool hy_attn_step_takes(const AttnStep& p);
+int hy_attn_step(const AttnStep& p, hipStream_t s);
+
 struct DeltaPrep {
   const float* proj;  // [M, ld]: q (G * dim), k (G * dim), v (H * vdim), gate (H * vdim), b (H), a (H)
   int ld;

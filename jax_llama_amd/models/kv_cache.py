@@ -95,6 +95,9 @@ class KVCacheRows:
         return self.parent.k[i, self.b0:self.b1], self.parent.v[i, self.b0:self.b1]
 
 
+TICKET_INTS = 64 * 32  # tickets of a cache row: 64 heads, each on a line of its own (csrc: AS_TICKET)
+
+
 class HybridCache:
     """Per-layer sequence state of a stack that mixes attention and recurrent layers, pre-allocated.
 
@@ -131,6 +134,9 @@ class HybridCache:
         self._device = device
         self.index = 0
         self.index_t = torch.zeros(1, dtype=torch.int32, device=device)
+        # counters of the one-launch decode attention (ops.hybrid.attn_step), which leaves them at zero: one per row and head, part
+        # of the cache because two steps on one cache are never in flight at once
+        self.tickets = torch.zeros(batch_size * TICKET_INTS, dtype=torch.int32, device=device)
 
     @staticmethod
     def parts(sp) -> list:
@@ -209,6 +215,7 @@ class HybridCache:
     def clear(self) -> None:
         """``reset`` and zero the keys and values too (after a failed step may have left non-finite rows)."""
         self.reset()
+        self.tickets.zero_()
         for t in {id(t): t for t in list(self._k.values()) + list(self._v.values())}.values():
             t.zero_()
 
@@ -263,6 +270,10 @@ class HybridCacheRows:
     @property
     def index_t(self):
         return self.parent.index_t
+
+    @property
+    def tickets(self):
+        return self.parent.tickets[self.b0 * TICKET_INTS:self.b1 * TICKET_INTS]
 
     def layer(self, i: int):
         k, v = self.parent.layer(i)

@@ -84,6 +84,10 @@ class StepContext:
     every_row: bool = False
     v_first: Optional[torch.Tensor] = None  # values [M, G vdim] of the first value-mixing layer of this step
 
+    @property
+    def tickets(self) -> Optional[torch.Tensor]:
+        return getattr(self.cache, "tickets", None)
+
 
 class BiasedAttention:
     def __init__(self, layer_idx: int, spec, eps: float, w_in: torch.Tensor, w_o: torch.Tensor,
@@ -100,6 +104,11 @@ class BiasedAttention:
         proj = hy.linear(x, self.w_in)
         kc, vc = ctx.cache.layer(self.i)
         own = sp.kv_from is None
+        if ctx.s == 1:
+            a = hy.attn_step(proj, ctx.positions, ctx.slot0, ctx.tickets, sp.heads, own, kc, vc, sp.scale, sp.softcap, self.bias,
+                             norm=(self.eps, sp.q_temp_coef, sp.q_temp_every))
+            if a is not None:
+                return hy.linear(a, self.w_o)
         q = hy.attn_prep(proj, ctx.positions, ctx.slot0, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim,
                          kc if own else None, vc if own else None, self.eps, sp.q_temp_coef, sp.q_temp_every)
         a = hy.attn_bias(q, kc, vc, ctx.slot0, sp.scale, sp.softcap, self.bias)
@@ -328,6 +337,11 @@ class RotaryChunkAttention:
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
         proj = hy.linear(h, self.w_in)
         kc, vc = ctx.cache.layer(self.i)
+        if ctx.s == 1:
+            a = hy.attn_step(proj, ctx.positions, ctx.slot0, ctx.tickets, self.heads, True, kc, vc, self.scale, sink=self.sink,
+                             chunk=self.chunk, head_scale=self.temp, out=out, rope=(self.bias, self.qk_freq, self.v_freq, gain))
+            if a is not None:
+                return a
         q = hy.rope_prep(proj, self.bias, ctx.positions, ctx.slot0, ctx.b, ctx.s, self.heads, self.kv_heads, self.dim,
                          self.vdim, kc, vc, self.qk_freq, self.v_freq)
         plain = self.v_freq is None and out is None and gain == 1.0

@@ -1163,6 +1163,31 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
     return out
 
 
+def attn_step(proj: torch.Tensor, positions: torch.Tensor, slot, tickets: Optional[torch.Tensor], heads: int, own: bool,
+              kc: torch.Tensor, vc: torch.Tensor, scale: float, softcap: float = 0.0, bias: Optional[torch.Tensor] = None,
+              sink: Optional[torch.Tensor] = None, chunk: int = 0, head_scale: Optional[torch.Tensor] = None,
+              out: Optional[torch.Tensor] = None, norm: Optional[tuple] = None, rope: Optional[tuple] = None
+              ) -> Optional[torch.Tensor]:
+    """One token per row, from the fused projection to the heads' output in one launch: ``attn_prep`` (``norm = (eps, temp_coef,
+    temp_every)``) or ``rope_prep`` (``rope = (col_bias, qk_freq, v_freq, gain)``: with ``v_freq`` or ``gain`` other than 1 the result
+    is ``rotate_heads(., positions, v_freq, sign=-1, gain)``), then ``attn_bias``. ``own``: the projection brings keys and values for
+    the cache. ``tickets``: zeros that no concurrent step uses (the cache's). None where only the separate ops apply."""
+    if not _gpu(proj) or tickets is None or kc.dtype != BF16 or (out is not None and out.dtype != F32):
+        return None
+    b, vdim = kc.shape[0], vc.shape[3]
+    dst = torch.empty(b, heads * vdim, dtype=F32, device=proj.device) if out is None else out
+    seen = min(kc.shape[2], chunk) if chunk and chunk > 0 else kc.shape[2]
+    args = (proj, kc, vc, _slot_tensor(slot, proj.device), positions, heads, own, tickets, float(scale), float(softcap or 0.0), bias,
+            dst, seen, sink, int(chunk or 0), head_scale)
+    if rope is not None:
+        col_bias, qk_freq, v_freq, gain = rope
+        done = ext().attn_step(*args, rope=True, col_bias=col_bias, qk_freq=qk_freq, v_freq=v_freq,
+                               turn=v_freq is not None or gain != 1.0, turn_sign=-1.0, turn_gain=float(gain))
+    else:
+        done = ext().attn_step(*args, eps=float(norm[0]), temp_coef=float(norm[1]), temp_every=int(norm[2]))
+    return dst if done else None
+
+
 # ------------------------------------------------------------------------------------------------ gated delta rule
 def delta_prep(proj: torch.Tensor, b: int, s: int, heads: int, kv_heads: int, dim: int, vdim: int,
                conv_w: torch.Tensor, conv_state: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor

@@ -1,0 +1,86 @@
+"""One token per row through the kernels that fuse a decode step's launches (csrc/hybrid/attn_step.hip), against the separate ops
+on the CPU, at the edges of their key splits and caches."""
+import pytest
+import torch
+
+from jax_llama_amd.ops import hybrid as hy
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF16 = torch.bfloat16
+
+
+def _rand(*shape, dt=torch.float32, std=1.0):
+    return (torch.randn(*shape) * std).to(dt)
+
+
+def _close(a, b, tol, what):
+    a, b = a.float().cpu(), b.float().cpu()
+    assert a.shape == b.shape, what
+    err = float((a - b).abs().max() / b.abs().max().clamp_min(1e-6))
+    assert err <= tol, f"{what}: relative error {err:.3e} > {tol:.1e}"
+
+
+def _to(x):
+    return None if x is None else x.to(DEV)
+
+
+SHAPES = [  # rows, heads, key heads, key width, value width, cache length, slot
+    (1, 4, 2, 64, 64, 40, 0), (1, 4, 1, 128, 128, 200, 63), (2, 4, 2, 128, 64, 200, 64), (3, 2, 2, 64, 128, 200, 65),
+    (1, 16, 4, 128, 128, 2112, 2080), (1, 8, 2, 128, 128, 2112, 2111), (1, 2, 1, 128, 128, 1100, 1023), (1, 2, 1, 64, 64, 1100, 1024),
+    (5, 4, 4, 128, 128, 64, 1), (1, 2, 1, 64, 64, 1, 0), (60, 4, 2, 64, 64, 130, 100), (1, 30, 10, 64, 128, 2600, 2570), (2, 2, 1, 128, 128, 90, 90)]
+
+
+@pytest.mark.parametrize("b,h,g,dim,vdim,t,slot", SHAPES)
+@pytest.mark.parametrize("kind", ["norm", "norm-shared", "rope", "rope-chunk", "rope-sink"])
+def test_attention_of_one_token(b, h, g, dim, vdim, t, slot, kind):
+    """Projection to head output, and the cache row written (none when the cache is full: slot == t), as the separate ops; the
+    tickets are back at zero, so that a second step on the same buffers gives the same."""
+    own = kind != "norm-shared"
+    if not own and slot >= t:
+        slot = t - 1
+    cols = h * dim + (g * (dim + vdim) if own else 0)
+    proj = _rand(b, cols + 8)[:, :cols]
+    kc, vc = _rand(b, g, t, dim, dt=BF16), _rand(b, g, t, vdim, dt=BF16)
+    pos = torch.full((b,), slot, dtype=torch.int32) + torch.arange(b, dtype=torch.int32)
+    slot_t, full = torch.tensor([slot], dtype=torch.int32), slot >= t
+    scale, kr, vr = dim ** -0.5, kc.clone(), vc.clone()
+    args = dict(softcap=0.0, bias=None, sink=None, chunk=0, head_scale=None)
+    out = None
+    if kind.startswith("norm"):
+        args.update(softcap=20.0, bias=_rand(50, h))
+        q = hy.attn_prep(proj, pos, min(slot, t - 1), b, 1, h, g, dim, vdim, kr if own else None, vr if own else None, 1e-5, 0.1, 7)
+        how = dict(norm=(1e-5, 0.1, 7))
+    else:
+        freq, vf = hy.rotary_freqs(1e4, dim // 2, "cpu"), (None if kind == "rope-sink" else hy.rotary_freqs(1e4, vdim, "cpu"))
+        cb = _rand(cols)
+        args.update(head_scale=torch.rand(h) + 0.5, chunk=64 if kind == "rope-chunk" else 0, sink=_rand(h) if kind == "rope-sink" else None)
+        q = hy.rope_prep(proj, cb, pos, min(slot, t - 1), b, 1, h, g, dim, vdim, kr, vr, freq, vf)
+        out = torch.zeros(b, h * vdim + 24, device=DEV)[:, 8:8 + h * vdim]
+        how = dict(rope=(cb.to(DEV), freq.to(DEV), _to(vf), 0.7))
+    if full:
+        kr, vr = kc.clone(), vc.clone()  # the token's own key is dropped
+    kd, vd, tickets = kc.to(DEV), vc.to(DEV), torch.zeros(b * h * 32, dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        kd.copy_(kc), vd.copy_(vc)
+        got = hy.attn_step(proj.to(DEV).as_strided((b, cols), (cols, 1)) if proj.is_contiguous() else _strided(proj), pos.to(DEV),
+                           slot_t.to(DEV), tickets, h, own, kd, vd, scale, **{k: _to(v) if torch.is_tensor(v) else v for k, v in args.items()},
+                           out=out, **how)
+        assert got is not None
+        # the output over the cache as this step left it: the last bit of a prepared key in 32 bits may round it to either of two
+        # neighbouring bf16 numbers
+        a = hy.attn_bias(q, kd.cpu(), vd.cpu(), min(slot, t - 1), scale, args["softcap"], args["bias"], sink=args["sink"],
+                         chunk=args["chunk"], head_scale=args["head_scale"])
+        if not kind.startswith("norm"):
+            a = hy.rotate_heads(a, pos, vf, h, sign=-1.0, gain=0.7)
+        _close(got, a, 2e-5, "output")
+        _close(kd, kr, 2.0 ** -7 if own else 0.0, "keys"), _close(vd, vr, 2.0 ** -7 if own else 0.0, "values")
+        keep = torch.arange(t) != slot
+        assert torch.equal(kd.cpu()[:, :, keep], kc[:, :, keep]) and torch.equal(vd.cpu()[:, :, keep], vc[:, :, keep])
+        assert not tickets.any()
+
+
+def _strided(x):
+    big = torch.zeros(x.shape[0], x.shape[1] + 8, device=DEV)
+    big[:, :x.shape[1]] = x.to(DEV)
+    return big[:, :x.shape[1]]
