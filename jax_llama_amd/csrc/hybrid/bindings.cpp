@@ -1003,6 +1003,43 @@ void mlstm_prep(Tensor proj, int64_t col_i, int64_t col_f, Tensor gate_bias, dou
   rc(jla::hy_mlstm_prep(p, stream()), "mlstm_prep");
 }
 
+void timemix_run(const jla::TimeMixChunk& t, const Tensor& like) {
+  Tensor ws;  // scratch of this call, from the allocator of the stream that uses it
+  const long long floats = jla::hy_timemix_chunk_floats(t);
+  if (floats > 0) ws = torch::empty({floats}, like.options());
+  rc(jla::hy_timemix_chunk(t, floats > 0 ? reinterpret_cast<float*>(ws.data_ptr()) : nullptr, stream()), "timemix_chunk");
+}
+
+// A prompt's time-mix memory with its gated head norm; false (nothing done) where the chunked kernel does not apply.
+bool timemix_norm(Tensor r, Tensor k, Tensor v, Tensor pre, Tensor w0, Tensor u, Tensor state, int64_t B, int64_t S, Tensor gate, Tensor w,
+                  double eps, double gain, Tensor out) {
+  check(r.dim() == 3 && v.dim() == 3, "timemix_norm: r, k are [M, H, dim], v is [M, H, vdim]");
+  const int64_t M = B * S, H = r.size(1), dim = r.size(2), vdim = v.size(2);
+  jla::TimeMixChunk t{};
+  jla::LinScan& p = t.s;
+  p.mode = 1;
+  p.q = heads3d(r, "r", M, H, dim, &p.ldq);
+  p.k = heads3d(k, "k", M, H, dim, &p.ldk);
+  p.v = heads3d(v, "v", M, H, vdim, &p.ldv);
+  p.decay = heads3d(pre, "pre", M, H, dim, &p.ldd);
+  check(w0.numel() == H * dim && u.numel() == H * dim, "timemix_norm: w0, u are [H, dim]");
+  p.w0 = f32(w0, "w0");
+  p.u = f32(u, "u");
+  check(state.numel() == B * H * dim * vdim, "timemix_norm: state");
+  p.state = f32w(state, "state");
+  p.B = B; p.S = S; p.H = H; p.dim = dim; p.vdim = vdim;
+  t.norm = 1;
+  check(gate.dim() == 2 && gate.size(0) == M && (w.numel() == vdim || w.numel() == H * vdim), "timemix_norm: gate, w");
+  t.gate = rows2d(gate, "gate", H * vdim, &t.ldg);
+  t.w = f32(w, "w");
+  t.w_heads = w.numel() != vdim || H == 1;
+  t.eps = eps; t.gain = gain;
+  t.out = slice2d_any(out, "out", M, H * vdim, &t.ldo, &t.out_bf16);
+  if (M == 0 || !jla::hy_timemix_chunk_takes(t)) return false;
+  timemix_run(t, r);
+  return true;
+}
+
 void lin_scan(int64_t mode, Tensor q, Tensor k, Tensor v, Tensor decay, OptT write, OptT w0, OptT u, Tensor state,
               Tensor o, int64_t B, int64_t S, double q_scale, int64_t nseg, int64_t seg_len) {
   jla::LinScan p{};
@@ -1030,6 +1067,9 @@ void lin_scan(int64_t mode, Tensor q, Tensor k, Tensor v, Tensor decay, OptT wri
   p.B = B; p.S = S; p.H = H; p.dim = dim; p.vdim = vdim;
   p.q_scale = q_scale;
   check(nseg >= 1 && seg_len >= 1 && nseg * seg_len >= S && (nseg - 1) * seg_len < S, "lin_scan: segments cover the tokens");
+  jla::TimeMixChunk t{};
+  t.s = p;
+  if (jla::hy_timemix_chunk_takes(t)) return timemix_run(t, q);
   p.nseg = nseg;
   p.seg_len = seg_len;
   Tensor ws;  // scratch of this call, from the allocator of the stream that uses it
@@ -1162,6 +1202,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("k_w") = py::none(), py::arg("norm_v") = true, py::arg("col_bias") = py::none(), py::arg("qk_freq") = py::none(),
         py::arg("v_freq") = py::none(), py::arg("turn") = false, py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
+  m.def("timemix_norm", &timemix_norm);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
   m.def("delta_scan", &delta_scan);

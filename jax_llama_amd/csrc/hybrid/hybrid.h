@@ -506,6 +506,23 @@ int hy_lin_scan(const LinScan& p, hipStream_t s);
 long long hy_scalar_chunk_floats(const LinScan& p);
 int hy_scalar_chunk(const LinScan& p, float* ws, hipStream_t s);
 
+// mode 1 in chunks on the matrix cores (timemix_chunk.hip), with the gated head norm (GatedNorm with silu) behind it or not (norm 0:
+// s.o is written). s.nseg, s.seg_len and the segment arrays are not read: the scratch is floats() numbers, segments are chosen here.
+struct TimeMixChunk {
+  LinScan s;
+  int norm;
+  const float* gate;
+  int ldg;
+  const float* w;
+  int w_heads;
+  float eps, gain;
+  void* out;
+  int ldo, out_bf16;
+};
+bool hy_timemix_chunk_takes(const TimeMixChunk& p);
+long long hy_timemix_chunk_floats(const TimeMixChunk& p);
+int hy_timemix_chunk(const TimeMixChunk& p, float* ws, hipStream_t s);
+
 // One token of a matrix-state recurrence with its gates and its gated head norm (rec_step.hip). mode 0: exponential gates
 // (state [B, H, dim, vdim + 1], mstate advanced), 1: time mix, 2: running memory, 3: delta rule. Row b, head h at x + b * ldx +
 // h * dim (or vdim; mode 3: q and k by key head, h / (H / G)). out[b * ldo + h * vdim + j] as hy_gated_rmsnorm gives it.

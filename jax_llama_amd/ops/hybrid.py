@@ -1638,6 +1638,10 @@ def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre: torc
     """``gated_rmsnorm(timemix_scan(...), gate, w, eps, GATE_SILU, gain=gain, out=out)``."""
     h, dim, vdim = r.shape[1], r.shape[2], v.shape[2]
     to = _step_out(r, h * vdim, dim, vdim, s, out)
+    if to is None and _gpu(r) and s > 1:  # (heads of 64: recurrence and norm of a prompt together)
+        y = torch.empty(b * s, h * vdim, dtype=F32, device=r.device) if out is None else out
+        if ext().timemix_norm(r, k, v, wpre, w0.reshape(h, dim), u.reshape(h, dim), state, b, s, gate, w, float(eps), float(gain), y):
+            return y
     if to is None:
         return gated_rmsnorm(timemix_scan(r, k, v, wpre, w0, u, state, b, s), gate, w, eps, GATE_SILU, gain=gain, out=out)
     ext().rec_step(1, r, k, v, pre=wpre, w0=w0.reshape(h, dim), u=u.reshape(h, dim), state=state, gate=gate, w=w, eps=float(eps),
