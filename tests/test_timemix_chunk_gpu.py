@@ -74,3 +74,16 @@ def test_a_number_that_is_none_reaches_no_token_before_it(b, s, operand, bad):
     for w, y in ((want, got), (st, S.cpu())):
         ok = torch.isfinite(w)
         assert torch.equal(torch.isfinite(y), ok) and float((y - w)[ok].abs().max()) < 2e-5 * float(w[ok].abs().max())
+
+
+@pytest.mark.parametrize("b,s", [(1, 1), (2, 63), (1, 64), (1, 65), (3, 130), (1, 1023), (2, 1024), (1, 1025), (1, 2113)])
+def test_gates_of_the_exponential_memory(b, s):
+    """The running maximum over blocks of 64 and 1024 tokens: every token's factors and the carried maximum as the CPU's chain."""
+    h, cap = 3, 15.0
+    proj, bias, m = torch.randn(b * s, 2 * h + 5) * 6.0, torch.randn(2 * h), torch.rand(b, h) * 8.0
+    m_dev = m.to(DEV)
+    got = hy.mlstm_prep(proj.to(DEV), 1, h + 2, bias.to(DEV), cap, m_dev, b, s, h)
+    want = hy.mlstm_prep(proj, 1, h + 2, bias, cap, m, b, s, h)
+    for x, y in zip(got, want):  # (tanh, exp and log of the two sides: a few units in the last place of exponents up to 15)
+        assert float(((x.cpu() - y).abs() / y.abs().clamp_min(1e-12)).max()) < 2e-5
+    assert float((m_dev.cpu() - m).abs().max()) < 15.0 * 2.0 ** -21
