@@ -887,6 +887,7 @@ int hy_attn_bias(const AttnBias& p, hipStream_t s) {
 #undef AM_CASE
     return -9;
   }
+  if (hy_attn_f32_takes(p)) return hy_attn_f32(p, s);
   dim3 grid((p.S + 3) / 4, p.H, p.B);
   if (p.maps == 2) AB_BY_VREG(attn_diff_prefill_kernel, grid, 256);
   else AB_BY_VREG(attn_bias_prefill_kernel, grid, 256);

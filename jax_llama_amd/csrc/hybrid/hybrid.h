@@ -308,6 +308,9 @@ struct AttnBias {
   float turn_sign, turn_gain;
 };
 int hy_attn_bias(const AttnBias& p, hipStream_t s);
+// its prompt form over fp32 caches on the matrix cores (attn_f32.hip)
+bool hy_attn_f32_takes(const AttnBias& p);
+int hy_attn_f32(const AttnBias& p, hipStream_t s);
 long long hy_attn_prefill_ws_bytes(int B, int S, int G, int dim, int vdim, int T, int cbf16);
 int hy_attn_decode_splits(int B, int H, int t_cap);
 
