@@ -16,6 +16,11 @@
 namespace jla {
 
 JLA_DEV void as_put(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// a number as a cache of that type holds it
+JLA_DEV void as_held(bf16_t& d, float v) { d = f2bf(v); }
+JLA_DEV void as_held(float& d, float v) { d = v; }
+JLA_DEV float as_number(bf16_t v) { return bf2f(v); }
+JLA_DEV float as_number(float v) { return v; }
 JLA_DEV float as_get(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // LDS that only this wave uses: its accesses stay in program order
@@ -97,7 +102,7 @@ JLA_DEV void as_merge(const float* w, int splits, int lane, float (&o)[VREG]) {
 }
 
 // dim = 8 DK8, vdim = 64 VREG; ROPE: biases and rotations, else norms and the query temperature
-template <int DK8, int VREG, int ROPE, int WAVES>
+template <typename CT, int DK8, int VREG, int ROPE, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   constexpr int dim = 8 * DK8, vdim = 64 * VREG, ND = dim / 64;
   __shared__ float qs_[WAVES][dim], row_[WAVES][dim > vdim ? dim : vdim], cs_[WAVES][2][64], sn_[WAVES][2][64];
@@ -127,20 +132,30 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   if (own) --span.n;  // (the token's own key comes from the projection)
   int j_lo, j_hi;
   ab_split_range(a, span, sp, j_lo, j_hi);
-  const bf16_t* kbase = reinterpret_cast<const bf16_t*>(a.kc) + ((size_t)b * a.G + g) * a.T * dim;
-  const bf16_t* vbase = reinterpret_cast<const bf16_t*>(a.vc) + ((size_t)b * a.G + g) * a.T * vdim + VREG * lane;
-  u32x4 kf[DK8];
-  uint32_t vv[64];
+  constexpr bool WIDE = sizeof(CT) == 4;
+  constexpr int KL = dim * sizeof(CT) / 16;
+  const CT* kbase = reinterpret_cast<const CT*>(a.kc) + ((size_t)b * a.G + g) * a.T * dim;
+  const CT* vbase = reinterpret_cast<const CT*>(a.vc) + ((size_t)b * a.G + g) * a.T * vdim + VREG * lane;
+  u32x4 kf[KL];
+  uint32_t vv[64][WIDE ? VREG : 1];
   float bl = 0.f;
   auto fetch = [&](int j0) {
     const int jc = ab_key(span, min(j0 + lane, j_hi - 1));
 #pragma unroll
-    for (int u = 0; u < DK8; ++u) kf[u] = *reinterpret_cast<const u32x4*>(kbase + (size_t)jc * dim + 8 * u);
+    for (int u = 0; u < KL; ++u) kf[u] = reinterpret_cast<const u32x4*>(kbase + (size_t)jc * dim)[u];
     bl = a.bias ? a.bias[(size_t)min(qi - jc, a.nbias - 1) * a.H + h] : 0.f;
 #pragma unroll
     for (int jj = 0; jj < 64; ++jj) {
-      const bf16_t* vr = vbase + (size_t)ab_key(span, min(j0 + jj, j_hi - 1)) * vdim;
-      vv[jj] = VREG == 2 ? *reinterpret_cast<const uint32_t*>(vr) : *vr;
+      const CT* vr = vbase + (size_t)ab_key(span, min(j0 + jj, j_hi - 1)) * vdim;
+      if constexpr (WIDE && VREG == 2) {
+        const u32x2 t = *reinterpret_cast<const u32x2*>(vr);
+        vv[jj][0] = t[0];
+        vv[jj][VREG - 1] = t[1];
+      } else if constexpr (WIDE || VREG == 2) {
+        vv[jj][0] = *reinterpret_cast<const uint32_t*>(vr);
+      } else {
+        vv[jj][0] = *reinterpret_cast<const bf16_t*>(vr);
+      }
     }
   };
   const bool any = j_lo < j_hi;
@@ -200,7 +215,15 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
 #pragma unroll
     for (int u = 0; u < DK8; ++u) {
       float f[8];
-      unpack8(kf[u], f);
+      if constexpr (WIDE) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f[i] = __uint_as_float(kf[2 * u][i]);
+          f[4 + i] = __uint_as_float(kf[2 * u + 1][i]);
+        }
+      } else {
+        unpack8(kf[u], f);
+      }
 #pragma unroll
       for (int i = 0; i < 8; i += 2) {
         d0 = fmaf(qs[8 * u + i], f[i], d0);
@@ -222,27 +245,27 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
 #pragma unroll
     for (int jj = 0; jj < 64; ++jj) {
       const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pw), jj));  // (0 past the split)
-      acc[0] = fmaf(pj, __uint_as_float(vv[jj] << 16), acc[0]);
-      if (VREG == 2) acc[VREG - 1] = fmaf(pj, __uint_as_float(vv[jj] & 0xffff0000u), acc[VREG - 1]);
+      acc[0] = fmaf(pj, __uint_as_float(WIDE ? vv[jj][0] : vv[jj][0] << 16), acc[0]);
+      if (VREG == 2) acc[VREG - 1] = fmaf(pj, __uint_as_float(WIDE ? vv[jj][WIDE ? VREG - 1 : 0] : vv[jj][0] & 0xffff0000u), acc[VREG - 1]);
     }
   }
   if (own && tail) {  // the token's own key, as the cache holds it
-    bf16_t kb[ND], vb[VREG];
+    CT kb[ND], vb[VREG];
     float dot = 0.f;
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
-      kb[i] = f2bf(kx[i]);
-      dot = fmaf(qv[i], bf2f(kb[i]), dot);
+      as_held(kb[i], kx[i]);
+      dot = fmaf(qv[i], as_number(kb[i]), dot);
     }
     as_order();  // (row: the rotations are done)
 #pragma unroll
     for (int i = 0; i < VREG; ++i) {
-      vb[i] = f2bf(vx[i]);
-      row[lane + 64 * i] = bf2f(vb[i]);
+      as_held(vb[i], vx[i]);
+      row[lane + 64 * i] = as_number(vb[i]);
     }
     if (h % (a.H / a.G) == 0) {
-      bf16_t* kd = const_cast<bf16_t*>(reinterpret_cast<const bf16_t*>(a.kc)) + (((size_t)b * a.G + g) * a.T + slot) * dim;
-      bf16_t* vd = const_cast<bf16_t*>(reinterpret_cast<const bf16_t*>(a.vc)) + (((size_t)b * a.G + g) * a.T + slot) * vdim;
+      CT* kd = const_cast<CT*>(reinterpret_cast<const CT*>(a.kc)) + (((size_t)b * a.G + g) * a.T + slot) * dim;
+      CT* vd = const_cast<CT*>(reinterpret_cast<const CT*>(a.vc)) + (((size_t)b * a.G + g) * a.T + slot) * vdim;
 #pragma unroll
       for (int i = 0; i < ND; ++i) kd[lane + 64 * i] = kb[i];
 #pragma unroll
@@ -331,7 +354,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   for (int i = 0; i < VREG; ++i) ab_out(a, b, h, VREG * lane + i, o[i]);
 }
 
-// bf16 caches with heads of 64 or 128 numbers, up to about a wave per SIMD: more waves share a SIMD, and then the preparation in
+// Heads of 64 or 128 numbers, up to about a wave per SIMD: more waves share a SIMD, and then the preparation in
 // each of them costs what the launches did. Us in turn, separate launches | here, heads of 128, rows x heads x splits: norms, 1 x 16
 // x 2 11.1 | 7.2, 3 x 16 x 17 16.0 | 11.8, 1 x 16 x 33 15.0 | 11.5, 2 x 16 x 33 18.2 | 17.1, 6 x 16 x 17 19.8 | 19.2, 13 x 16 x 9
 // 19.9 | 20.6, 8 x 32 x 8 34.4 | 38.7; rotations, 1 x 16 x 13 12.0 | 9.0, 2 x 32 x 16 14.1 | 11.0, 6 x 16 x 17 16.8 | 17.4, 4 x 32 x 16
@@ -340,7 +363,7 @@ constexpr long long AS_MAX_WAVES = 1280;
 
 bool hy_attn_step_takes(const AttnStep& p) {
   const AttnBias& a = p.a;
-  return a.S == 1 && a.maps == 1 && a.cbf16 && (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128) &&
+  return a.S == 1 && a.maps == 1 && (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128) &&
          a.ldk == a.dim && a.ldv == a.vdim && ((uintptr_t)a.kc & 15) == 0 && ((uintptr_t)a.vc & 15) == 0 && a.splits >= 1 &&
          a.splits <= 64 && (long long)a.B * a.H * a.splits <= AS_MAX_WAVES;
 }
@@ -362,8 +385,10 @@ int hy_attn_step(const AttnStep& p, hipStream_t s) {
   const dim3 grid((a.splits + waves - 1) / waves, a.H, a.B);
 #define AS_ONE(DK8, VREG, ROPE)                                                                      \
   do {                                                                                               \
-    if (waves == 2) attn_step_kernel<DK8, VREG, ROPE, 2><<<grid, 128, 0, s>>>(p);                    \
-    else attn_step_kernel<DK8, VREG, ROPE, 1><<<grid, 64, 0, s>>>(p);                                \
+    if (!a.cbf16 && waves == 2) attn_step_kernel<float, DK8, VREG, ROPE, 2><<<grid, 128, 0, s>>>(p); \
+    else if (!a.cbf16) attn_step_kernel<float, DK8, VREG, ROPE, 1><<<grid, 64, 0, s>>>(p);           \
+    else if (waves == 2) attn_step_kernel<bf16_t, DK8, VREG, ROPE, 2><<<grid, 128, 0, s>>>(p);       \
+    else attn_step_kernel<bf16_t, DK8, VREG, ROPE, 1><<<grid, 64, 0, s>>>(p);                        \
   } while (0)
 #define AS_RUN(DK8, VREG)              \
   do {                                 \

@@ -1172,7 +1172,7 @@ def attn_step(proj: torch.Tensor, positions: torch.Tensor, slot, tickets: Option
     temp_every)``) or ``rope_prep`` (``rope = (col_bias, qk_freq, v_freq, gain)``: with ``v_freq`` or ``gain`` other than 1 the result
     is ``rotate_heads(., positions, v_freq, sign=-1, gain)``), then ``attn_bias``. ``own``: the projection brings keys and values for
     the cache. ``tickets``: zeros that no concurrent step uses (the cache's). None where only the separate ops apply."""
-    if not _gpu(proj) or tickets is None or kc.dtype != BF16 or (out is not None and out.dtype != F32):
+    if not _gpu(proj) or tickets is None or (out is not None and out.dtype != F32):
         return None
     b, vdim = kc.shape[0], vc.shape[3]
     dst = torch.empty(b, heads * vdim, dtype=F32, device=proj.device) if out is None else out

@@ -33,7 +33,8 @@ SHAPES = [  # rows, heads, key heads, key width, value width, cache length, slot
 
 @pytest.mark.parametrize("b,h,g,dim,vdim,t,slot", SHAPES)
 @pytest.mark.parametrize("kind", ["norm", "norm-shared", "rope", "rope-chunk", "rope-sink"])
-def test_attention_of_one_token(b, h, g, dim, vdim, t, slot, kind):
+@pytest.mark.parametrize("dt", [BF16, torch.float32])
+def test_attention_of_one_token(b, h, g, dim, vdim, t, slot, kind, dt):
     """Projection to head output, and the cache row written (none when the cache is full: slot == t), as the separate ops; the
     tickets are back at zero, so that a second step on the same buffers gives the same."""
     own = kind != "norm-shared"
@@ -41,7 +42,7 @@ def test_attention_of_one_token(b, h, g, dim, vdim, t, slot, kind):
         slot = t - 1
     cols = h * dim + (g * (dim + vdim) if own else 0)
     proj = _rand(b, cols + 8)[:, :cols]
-    kc, vc = _rand(b, g, t, dim, dt=BF16), _rand(b, g, t, vdim, dt=BF16)
+    kc, vc = _rand(b, g, t, dim, dt=dt), _rand(b, g, t, vdim, dt=dt)
     pos = torch.full((b,), slot, dtype=torch.int32) + torch.arange(b, dtype=torch.int32)
     slot_t, full = torch.tensor([slot], dtype=torch.int32), slot >= t
     scale, kr, vr = dim ** -0.5, kc.clone(), vc.clone()
@@ -74,7 +75,8 @@ def test_attention_of_one_token(b, h, g, dim, vdim, t, slot, kind):
         if not kind.startswith("norm"):
             a = hy.rotate_heads(a, pos, vf, h, sign=-1.0, gain=0.7)
         _close(got, a, 2e-5, "output")
-        _close(kd, kr, 2.0 ** -7 if own else 0.0, "keys"), _close(vd, vr, 2.0 ** -7 if own else 0.0, "values")
+        tol = (2.0 ** -7 if dt == BF16 else 2e-6) if own else 0.0
+        _close(kd, kr, tol, "keys"), _close(vd, vr, tol, "values")
         keep = torch.arange(t) != slot
         assert torch.equal(kd.cpu()[:, :, keep], kc[:, :, keep]) and torch.equal(vd.cpu()[:, :, keep], vc[:, :, keep])
         assert not tickets.any()
