@@ -186,6 +186,41 @@ bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc
   return true;
 }
 
+// Several matrices on one or two normed rows, blended or not, in one launch: out[i] = ws[i] v_i, v = rms_norm(x) gain, blended v + (prev -
+// v) mu[mix[i]] for mix[i] >= 0, capped (cap[i] > 0); row <- v. False: not a call of that kernel, nothing was launched.
+bool rows_parts(Tensor x, Tensor gain, double eps, Tensor prev, Tensor mu, std::vector<Tensor> ws, std::vector<int64_t> mix,
+                std::vector<double> cap, std::vector<Tensor> outs, Tensor row) {
+  const int64_t R = x.size(0), K = x.size(1);
+  check(x.dim() == 2 && mu.dim() == 2 && mu.size(1) == K && gain.numel() == K && prev.numel() == R * K && row.numel() == R * K,
+        "rows_parts: rows of x, prev, row; mu and gain of its width");
+  check(ws.size() == mix.size() && ws.size() == cap.size() && ws.size() == outs.size(), "rows_parts: parts");
+  if (ws.empty() || ws.size() > (size_t)jla::RV_MAX_PARTS) return false;
+  jla::RowLinear p{};
+  p.a = rows2d(x, "x", K, &p.lda);
+  p.K = K; p.R = R; p.E = 1;
+  p.wbf16 = 1;
+  p.a_norm_w = f32(gain, "gain");
+  p.a_norm_eps = eps;
+  jla::RowParts t{};
+  t.n = ws.size();
+  t.prev = f32(prev, "prev");
+  t.mu = f32(mu, "mu");
+  t.row = f32w(row, "row");
+  for (int i = 0; i < t.n; ++i) {
+    if (!wtype(ws[i], "w")) return false;
+    check(ws[i].dim() == 2 && ws[i].size(1) == K && mix[i] < mu.size(0), "rows_parts: w is [N, K], mix a row of mu");
+    t.w[i] = ws[i].data_ptr();
+    t.N[i] = ws[i].size(0);
+    t.out[i] = const_cast<float*>(rows2d(outs[i], "out", t.N[i], &t.ldo[i]));
+    check(outs[i].size(0) == R, "rows_parts: out rows");
+    t.mix[i] = std::max<int64_t>(mix[i], -1);
+    t.cap[i] = cap[i];
+  }
+  if (!jla::hy_rows_parts_takes(p, t)) return false;
+  rc(jla::hy_rows_parts(p, t, stream()), "rows_parts");
+  return true;
+}
+
 // Both products of a few tokens' table-chosen SwiGLU experts, the table read by the products: h [M * top, F], out [M * top, D] in
 // (token, choice) order. False: not a call of that kernel, nothing was launched.
 bool table_rows(Tensor a, Tensor ids, Tensor table, Tensor w_gu, Tensor w_down, Tensor h, Tensor out, OptT y, int64_t nsum,
@@ -1095,7 +1130,7 @@ bool rec_step_takes(int64_t dim, int64_t vdim) {
 // gates: mode 0: (projection [B, .], column of the input gates, column of the forget gates, biases, running maximum [B, H])
 void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT u, OptT beta, OptT decay, OptT proj, int64_t col_i,
               int64_t col_f, OptT gate_bias, double cap, OptT mstate, double q_scale, Tensor state, OptT gate, Tensor w,
-              double eps, int64_t gate_act, double gain, Tensor out) {
+              double eps, int64_t gate_act, double gain, Tensor out, OptT pre_x, OptT pre_w, OptT prev, OptT row) {
   jla::RecStep p{};
   check(mode >= 0 && mode <= 3, "rec_step: mode");
   check(q.dim() == 3 && v.dim() == 3, "rec_step: q is [B, H (mode 3: G), dim], v is [B, H, vdim]");
@@ -1123,9 +1158,28 @@ void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT 
     p.beta = f32(*beta, "beta");
     p.decay = f32(*decay, "decay");
   } else {
-    check(pre.has_value() && w0.has_value() && u.has_value() && w0->numel() == H * dim && u->numel() == H * dim,
+    check((pre.has_value() || (mode == 1 && pre_x.has_value())) && w0.has_value() && u.has_value() && w0->numel() == H * dim &&
+              u->numel() == H * dim,
           "rec_step: pre, w0, u");
-    p.pre = heads3d(*pre, "pre", B, H, dim, &p.ldpre);
+    if (pre_x.has_value()) {
+      check(mode == 1 && !pre.has_value() && pre_w.has_value() && pre_w->dim() == 2 && pre_w->size(0) == H * dim &&
+                pre_x->dim() == 2 && pre_x->size(0) == B && pre_x->size(1) == pre_w->size(1) && pre_w->size(1) % 4 == 0,
+            "rec_step: low-rank gate product");
+      p.pre_x = f32(*pre_x, "pre_x");
+      p.pre_bf16 = wtype(*pre_w, "pre_w");
+      p.pre_w = pre_w->data_ptr();
+      p.rank = pre_w->size(1);
+      check(((uintptr_t)p.pre_x & 15) == 0 && ((uintptr_t)p.pre_w & 15) == 0, "rec_step: alignment");
+      check(prev.has_value() == row.has_value(), "rec_step: prev and row");
+      if (row.has_value()) {
+        check(prev->numel() == row->numel() && row->numel() % B == 0, "rec_step: prev and row are [B, width]");
+        p.prev = f32w(*prev, "prev");
+        p.row = f32(*row, "row");
+        p.width = row->numel() / B;
+      }
+    } else {
+      p.pre = heads3d(*pre, "pre", B, H, dim, &p.ldpre);
+    }
     p.w0 = f32(*w0, "w0");
     p.u = f32(*u, "u");
   }
@@ -1203,6 +1257,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("v_freq") = py::none(), py::arg("turn") = false, py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("timemix_norm", &timemix_norm);
+  m.def("rows_parts", &rows_parts);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
   m.def("delta_scan", &delta_scan);
@@ -1216,7 +1271,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("w0") = py::none(), py::arg("u") = py::none(), py::arg("beta") = py::none(), py::arg("decay") = py::none(),
         py::arg("proj") = py::none(), py::arg("col_i") = 0, py::arg("col_f") = 0, py::arg("gate_bias") = py::none(),
         py::arg("cap") = 1.0, py::arg("mstate") = py::none(), py::arg("q_scale") = 1.0, py::arg("state"), py::arg("gate"),
-        py::arg("w"), py::arg("eps"), py::arg("gate_act"), py::arg("gain"), py::arg("out"));
+        py::arg("w"), py::arg("eps"), py::arg("gate_act"), py::arg("gain"), py::arg("out"), py::arg("pre_x") = py::none(),
+        py::arg("pre_w") = py::none(), py::arg("prev") = py::none(), py::arg("row") = py::none());
   m.def("gated_rmsnorm", &gated_rmsnorm, py::arg("o"), py::arg("gate"), py::arg("w"), py::arg("eps"), py::arg("out"),
         py::arg("H"), py::arg("vdim"), py::arg("gate_act") = 0, py::arg("denom_floor") = py::none(),
         py::arg("gain") = 1.0);

@@ -71,6 +71,24 @@ struct RowLinear {
   int res_w_vec;
   float* res_out;
 };
+// Several bf16 matrices [N, K] that read the same one or two rows: a normed row v, or blended with the row before it, v + (prev - v)
+// mu[mix] (rows_gemv.hip). first, tgroups: filled in by the launch.
+constexpr int RV_MAX_PARTS = 6;
+struct RowParts {
+  int n;
+  const void* w[RV_MAX_PARTS];
+  int N[RV_MAX_PARTS];
+  float* out[RV_MAX_PARTS];  // [R, ldo]
+  int ldo[RV_MAX_PARTS];
+  int mix[RV_MAX_PARTS];     // row of mu, or -1: the normed row itself
+  float cap[RV_MAX_PARTS];   // > 0: cap * tanh(. / cap)
+  const float* prev;         // [R, K]
+  const float* mu;           // [*, K]
+  float* row;                // [R, K]: the normed rows
+  int first[RV_MAX_PARTS + 1], tgroups[RV_MAX_PARTS];
+};
+bool hy_rows_parts_takes(const RowLinear& p, const RowParts& t);  // p: a, lda, K, R, a_norm_w, a_norm_eps
+int hy_rows_parts(const RowLinear& p, const RowParts& t, hipStream_t s);
 inline bool hy_act_gated(int act) {
   return act == HY_ACT_SWIGLU || act == HY_ACT_CLAMP_GLU || act == HY_ACT_GELU_GLU;
 }
@@ -539,6 +557,12 @@ struct RecStep {
   int ldv;
   const float* pre;  // modes 1, 2: gate pre-activations
   int ldpre;
+  const float* pre_x;  // mode 1, in pre's place: pre = pre_w [H dim, rank] pre_x [B, rank] (bf16 weights: pre_x rounded to bf16)
+  const void* pre_w;
+  int rank, pre_bf16;
+  float* prev;         // with pre_x, optional: prev [B, width] <- row [B, width]
+  const float* row;
+  int width;
   const float* w0;   // modes 1, 2: [H, dim]
   const float* u;
   const float* beta; // mode 3: [B, H]

@@ -40,6 +40,28 @@ JLA_DEV void rs_sum(float (&v)[N], int nw, float* red) {
   }
 }
 
+// sum_r w[d, r] x[r] of key row d = t / lanes, over lanes (a power of two up to 64) adjacent threads; every one of them gets it
+JLA_DEV float rs_low_rank(const RecStep& p, int b, size_t d, int lane, int lanes) {
+  const float* x = p.pre_x + (size_t)b * p.rank;
+  float s = 0.f;
+  for (int r = 4 * lane; r < p.rank; r += 4 * lanes) {
+    const f32x4 xv = *reinterpret_cast<const f32x4*>(x + r);
+    if (p.pre_bf16) {
+      const u32x2 wv = *reinterpret_cast<const u32x2*>(reinterpret_cast<const bf16_t*>(p.pre_w) + d * p.rank + r);
+      s = fmaf(bf2f(f2bf(xv[0])), __uint_as_float(wv[0] << 16), s);
+      s = fmaf(bf2f(f2bf(xv[1])), __uint_as_float(wv[0] & 0xffff0000u), s);
+      s = fmaf(bf2f(f2bf(xv[2])), __uint_as_float(wv[1] << 16), s);
+      s = fmaf(bf2f(f2bf(xv[3])), __uint_as_float(wv[1] & 0xffff0000u), s);
+    } else {
+      const f32x4 wv = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(p.pre_w) + d * p.rank + r);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s = fmaf(xv[i], wv[i], s);
+    }
+  }
+  for (int o = 1; o < lanes; o <<= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
 // grid (H, B). Thread -> value column j = t % cw, key rows [RPT s, RPT s + RPT) of slice s = t / cw (cw: vdim rounded up to
 // whole waves).
 template <int MODE, int RPT>
@@ -80,8 +102,20 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
       st[(size_t)t * ncols + vdim] = fmaf(keep, zs, wk);  // (no other thread uses what it holds)
     }
   } else if (MODE == RS_TIMEMIX) {
-    const float pre = p.pre[(size_t)b * p.ldpre + (size_t)h * dim + td];
     const float w0 = p.w0[(size_t)h * dim + td], u = p.u[(size_t)h * dim + td];
+    float pre;
+    if (p.pre_x) {  // (uniform) the decay's low-rank product here, all threads on it; the carried token row beside it
+      const int lanes = 1024 / (dim <= 64 ? 64 : (dim <= 128 ? 128 : 256)), d = t / lanes;
+      const float s = rs_low_rank(p, b, (size_t)h * dim + min(d, dim - 1), t % lanes, lanes);
+      if (t % lanes == 0 && d < dim) lw[d] = s;
+      if (p.row) {
+        for (int i = h * RS_THREADS + t; i < p.width; i += p.H * RS_THREADS) p.prev[(size_t)b * p.width + i] = p.row[(size_t)b * p.width + i];
+      }
+      __syncthreads();
+      pre = lw[td];
+    } else {
+      pre = p.pre[(size_t)b * p.ldpre + (size_t)h * dim + td];
+    }
     if (key) {
       la[t] = expf(-expf(pre + w0));
       lb[t] = k;
@@ -167,6 +201,7 @@ int hy_rec_step(const RecStep& p, hipStream_t s) {
   if (p.mode < 0 || p.mode > 3 || p.B < 0 || p.H < 1 || !hy_rec_step_takes(p.dim, p.vdim)) return -1;
   if (p.mode == RS_DELTA && (p.G < 1 || p.H % p.G)) return -2;
   if (p.gate_act < 0 || p.gate_act > 2 || (p.gate_act != 2 && !p.gate)) return -3;
+  if (p.pre_x && (p.mode != RS_TIMEMIX || p.rank < 4 || p.rank % 4 || !p.pre_w)) return -5;
   if (p.B == 0) return 0;
   if (p.B > 65535) return -4;
   const int cw = (p.vdim + 63) / 64 * 64, slices = RS_THREADS / cw;

@@ -279,10 +279,32 @@ JLA_DEV float rv_block_sum(float v, float (*stat)[16]) {
   __syncthreads();
   return stat[0][0] + stat[1][0] + stat[2][0] + stat[3][0];
 }
-template <int V>
+// MIX: the normed row is then blended with the row before it (RowParts), row 0 of the launch's parts also stored as it was.
+template <int V, int MIX>
 struct RvRow {
-  f32x4 x[V], y[V], g[V], w[V];
+  f32x4 x[V], y[V], g[V], w[V], before[MIX ? V : 1], mu[MIX ? V : 1];
   float scale;
+  JLA_DEV void load_mix(const RowParts& t, int part, int r, int K, int tid) {
+    if constexpr (MIX) {
+      const float* m = t.mu + (size_t)max(t.mix[part], 0) * K;
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const int k = 4 * tid + 1024 * u < K ? 4 * tid + 1024 * u : 0;
+        before[u] = *reinterpret_cast<const f32x4*>(t.prev + (size_t)r * K + k);
+        mu[u] = *reinterpret_cast<const f32x4*>(m + k);
+      }
+    }
+  }
+  JLA_DEV f32x4 mixed(const RowParts& t, int part, f32x4 v, int u, int r, int K, int k) const {
+    if constexpr (MIX) {
+      if (blockIdx.x == 0 && k < K) *reinterpret_cast<f32x4*>(t.row + (size_t)r * K + k) = v;
+      if (t.mix[part] >= 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = fmaf(before[u][j] - v[j], mu[u][j], v[j]);
+      }
+    }
+    return v;
+  }
   JLA_DEV void load(const RowLinear& p, int r, int K, int tid) {
     const int src = p.a_idx ? p.a_idx[r] : (p.a_div > 1 ? r / p.a_div : r);
     const float* xp = reinterpret_cast<const float*>(p.a) + (size_t)src * p.lda;
@@ -323,7 +345,7 @@ struct RvRow {
       }
     }
   }
-  JLA_DEV void stage(const RowLinear& p, int r, int i, int K, int tid, float (*stat)[16], f32x4* staged) {
+  JLA_DEV void stage(const RowLinear& p, int r, int i, int K, int tid, float (*stat)[16], f32x4* staged, const RowParts& t, int part) {
     if (p.res_y) {
       float ss = 0.f;
 #pragma unroll
@@ -358,6 +380,7 @@ struct RvRow {
       const int k = 4 * tid + 1024 * u;
       f32x4 v = x[u] * scale;
       if (p.a_norm_w) v *= g[u];
+      v = mixed(t, part, v, u, r, K, k);
       if (k < K) staged[((size_t)i * K + k) / 4] = v;
     }
   }
@@ -366,15 +389,30 @@ struct RvRow {
 // One or two rows, K <= 128 WAVES U: a wave's share of K is U steps, so the rows' operands stay in its registers, and a
 // workgroup walks over groups of NT tiles with the next group's weights issued as this one's are consumed. The rows pass
 // through LDS once per workgroup, where a pending residual add (res_y) and the norm are applied behind the first weights.
-// grid (workgroups, linear rows with their own expert, else 1).
-template <int NT, int U, int V>
-__global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups) {
+// grid (workgroups, linear rows with their own expert, else 1). PARTS: several matrices (RowParts) that read the same rows, each with
+// a run of the workgroups, the rows blended for it as they are staged.
+template <int NT, int U, int V, int PARTS>
+__global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
   constexpr int G = 4, WAVES = 4, STEP = 128;
   extern __shared__ f32x4 staged[];  // [rows][K]
   __shared__ f32x4 red[2][WAVES][NT][64];
   __shared__ float stat[WAVES][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
-  rv_arguments(p);
+  int part = 0, tg = blockIdx.x, walk = gridDim.x;  // this workgroup's first group of tiles, and from one to its next
+  if constexpr (PARTS) {
+    while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
+    tg -= parts.first[part];
+    walk = parts.first[part + 1] - parts.first[part];
+    tgroups = parts.tgroups[part];
+    p.w = parts.w[part];
+    p.N = parts.N[part];
+    p.out = parts.out[part];
+    p.ldo = parts.ldo[part];
+    p.act = parts.cap[part] > 0.f ? HY_ACT_SOFTCAP : HY_ACT_NONE;
+    p.act_limit = parts.cap[part];
+  } else {
+    rv_arguments(p);
+  }
   const int r0 = blockIdx.y * rows_per_group, nr = min(rows_per_group, p.R - r0);
   const int e = rv_expert(p, r0);
   if (e < 0) return;  // (the whole workgroup)
@@ -390,19 +428,20 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
     const int T = tg * NT + t, col = min(G * (gated ? T >> 1 : T) + c % G, N - 1);
     return wbase + (size_t)(gated && (T & 1) ? N + col : col) * K;
   };
-  RvRow<V> row;
+  RvRow<V, PARTS> row;
   row.load(p, r0, K, tid);
-  int tg = blockIdx.x;
+  row.load_mix(parts, part, r0, K, tid);
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const bf16_t* w = weight_row(tg, t);
 #pragma unroll
     for (int u = 0; u < U; ++u) wf[u][t] = load_nt(reinterpret_cast<const u32x4*>(w + at(u)));
   }
-  row.stage(p, r0, 0, K, tid, stat, staged);
+  row.stage(p, r0, 0, K, tid, stat, staged, parts, part);
   if (nr > 1) {
     row.load(p, r0 + 1, K, tid);
-    row.stage(p, r0 + 1, 1, K, tid, stat, staged);
+    row.load_mix(parts, part, r0 + 1, K, tid);
+    row.stage(p, r0 + 1, 1, K, tid, stat, staged, parts, part);
   }
   __syncthreads();
   u32x4 xr[U];
@@ -411,8 +450,8 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
     const f32x4* x = staged + ((size_t)min(c % G, nr - 1) * K + at(u)) / 4;
     xr[u] = STEP * (wave + WAVES * u) + k0 < K ? rv_round8(x[0], x[1]) : u32x4{0, 0, 0, 0};
   }
-  for (int buf = 0; tg < tgroups; tg += gridDim.x, buf ^= 1) {
-    const int next = tg + (int)gridDim.x;
+  for (int buf = 0; tg < tgroups; tg += walk, buf ^= 1) {
+    const int next = tg + walk;
     const bool more = next < tgroups;  // (workgroup-uniform)
     f32x4 acc[NT];
 #pragma unroll
@@ -483,6 +522,32 @@ bool hy_rows_gemv_takes_residual(const RowLinear& p) {
          aligned(p.res_y) && aligned(p.res_out) && (!p.res_w_vec || aligned(p.res_w));
 }
 
+bool hy_rows_parts_takes(const RowLinear& p, const RowParts& t) {
+  auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  bool ok = p.R >= 1 && p.R <= RV_WALK_ROWS && p.a_norm_w && p.K % 8 == 0 && p.K >= 256 && p.K <= RV_WALK_K && p.lda % 4 == 0 && aligned(p.a) &&
+            aligned(p.a_norm_w) && aligned(t.prev) && aligned(t.mu) && aligned(t.row) && t.n >= 1 && t.n <= RV_MAX_PARTS;
+  for (int i = 0; ok && i < t.n; ++i) ok = t.N[i] >= 1 && aligned(t.w[i]);
+  return ok;
+}
+
+// What the launch saves: the norm and blend of one row, four products of its blends, a low-rank product of the fifth and a product of
+// the row itself (K 2048; N 4 x 2048, 64, 3072) were four launches.
+int hy_rows_parts(const RowLinear& p, const RowParts& parts, hipStream_t s) {
+  if (!hy_rows_parts_takes(p, parts)) return -1;
+  RowParts t = parts;
+  const int occ = p.K <= 2048 ? 4 : 2;
+  long long all = 0;
+  for (int i = 0; i < t.n; ++i) all += t.tgroups[i] = ((t.N[i] + 3) / 4 + 1) / 2;
+  const int rounds = (int)((all + 256 * occ - 1) / (256 * occ));
+  t.first[0] = 0;
+  for (int i = 0; i < t.n; ++i) t.first[i + 1] = t.first[i] + (t.tgroups[i] + rounds - 1) / rounds;
+  const unsigned lds = (unsigned)(p.R * p.K * sizeof(float));
+  if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1><<<dim3(t.first[t.n], 1), 256, lds, s>>>(p, p.R, 0, 0, t);
+  else rows_gemv_walk_kernel<2, 8, 4, 1><<<dim3(t.first[t.n], 1), 256, lds, s>>>(p, p.R, 0, 0, t);
+  JLA_CHECK_LAUNCH();
+  return 0;
+}
+
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   const int gated = hy_act_gated(p.act);
   RowLinear q = p;
@@ -506,7 +571,7 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
     const long long room = 256LL * occ / groups > 0 ? 256LL * occ / groups : 1, rounds = (tg + room - 1) / room;
     const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
     const unsigned lds = (unsigned)(rows * p.K * sizeof(float));
-#define RV_WALK(NT, U, V) rows_gemv_walk_kernel<NT, U, V><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg)
+#define RV_WALK(NT, U, V) rows_gemv_walk_kernel<NT, U, V, 0><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
     if (p.K <= 2048) {
       if (wnt == 1) RV_WALK(1, 4, 2);
       else RV_WALK(2, 4, 2);

@@ -334,8 +334,11 @@ class RotaryChunkAttention:
         self.w_o = w_o          # [D, H vdim]
         self.width = heads * vdim
 
-    def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
-        proj = hy.linear(h, self.w_in)
+    def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0,
+                 proj: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """``proj``: ``linear(h, w_in)`` where another launch has computed it."""
+        if proj is None:
+            proj = hy.linear(h, self.w_in)
         kc, vc = ctx.cache.layer(self.i)
         if ctx.s == 1:
             a = hy.attn_step(proj, ctx.positions, ctx.slot0, ctx.tickets, self.heads, True, kc, vc, self.scale, sink=self.sink,
@@ -398,18 +401,31 @@ class TimeMix:
         self.w_o = w_o        # [D, H dim]
         self.width = heads * dim
 
-    def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
+    def inputs(self, h, ctx: StepContext, w_also: torch.Tensor):
+        """One token per row: this mixer's five projections and ``linear(h, w_also)`` from one launch, ``(that, what features()
+        takes as its inputs)``; None where they are launches of their own."""
+        _, prev = ctx.cache.recurrent(self.i)
+        got = hy.shifted_linears(h, prev, self.mu, [(w_also, -1, 0.0)] + [(w, j, 0.0) for j, w in enumerate(self.w_each)] +
+                                 [(self.w_d1, 4, 1.0)])
+        return None if got is None else (got[0][0], (got[0][1:], got[1]))
+
+    def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0, inputs=None) -> torch.Tensor:
         nh, dim, m = self.heads, self.dim, ctx.b * ctx.s
         state, prev = ctx.cache.recurrent(self.i)
-        mixes = hy.token_shift(h, prev, self.mu, ctx.b, ctx.s)
-        if 4 * m <= hy.STACKED_MAX_ROWS:  # a few tokens: the four same-shaped projections as one grouped launch
-            r, k, v, g = hy.stacked_linear(mixes[:4], self.w_rkvg).unbind(0)
+        carry = None
+        if inputs is not None:
+            (r, k, v, g, z), row = inputs
+            carry = (prev, row)
         else:
-            r, k, v, g = (hy.linear(mixes[j], self.w_each[j]) for j in range(4))
-        wpre = hy.linear(hy.linear_softcap(mixes[4], self.w_d1, 1.0), self.w_d2)
+            mixes = hy.token_shift(h, prev, self.mu, ctx.b, ctx.s)
+            if 4 * m <= hy.STACKED_MAX_ROWS:  # a few tokens: the four same-shaped projections as one grouped launch
+                r, k, v, g = hy.stacked_linear(mixes[:4], self.w_rkvg).unbind(0)
+            else:
+                r, k, v, g = (hy.linear(mixes[j], self.w_each[j]) for j in range(4))
+            z = hy.linear_softcap(mixes[4], self.w_d1, 1.0)
         hd = (nh, dim)
-        return hy.timemix_memory(r.unflatten(1, hd), k.unflatten(1, hd), v.unflatten(1, hd), wpre.unflatten(1, hd), self.w0,
-                                 self.u, state, ctx.b, ctx.s, g, self.norm_w, self.eps, gain, out)
+        return hy.timemix_memory(r.unflatten(1, hd), k.unflatten(1, hd), v.unflatten(1, hd), (z, self.w_d2), self.w0,
+                                 self.u, state, ctx.b, ctx.s, g, self.norm_w, self.eps, gain, out, carry)
 
     def __call__(self, h, ctx: StepContext) -> torch.Tensor:
         return hy.linear(self.features(h, ctx), self.w_o)
@@ -431,9 +447,13 @@ class SideBySide:
         hv = h if ctx.s == 1 and isinstance(h, hy.RmsInput) and hy.norms_free(m, self.w_o, h.x.shape[1]) else _value(h)
         if out is None:
             out = torch.empty(m, self.width, dtype=torch.float32, device=hv.device if torch.is_tensor(hv) else hv.x.device)
+        # one token: an attention beside a time mix read their inputs in one launch
+        kinds = [type(mm) for mm in self.members]
+        both = self.members[1].inputs(hv, ctx, self.members[0].w_in) if ctx.s == 1 and kinds == [RotaryChunkAttention, TimeMix] else None
         c = 0
-        for mm, sc in zip(self.members, self.scales):
-            mm.features(hv, ctx, out=out[:, c:c + mm.width], gain=gain * sc)
+        for n, (mm, sc) in enumerate(zip(self.members, self.scales)):
+            given = {} if both is None else {("proj", "inputs")[n]: both[n]}
+            mm.features(hv, ctx, out=out[:, c:c + mm.width], gain=gain * sc, **given)
             c += mm.width
         return out
 

@@ -1488,6 +1488,27 @@ def token_shift(h, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int) -> torc
     return out
 
 
+def shifted_linears(h, prev: torch.Tensor, mu: torch.Tensor, parts) -> Optional[tuple]:
+    """One token per row: ``(outs, row)`` with ``outs[i] = v_i @ w_i^T`` for every ``(w_i, mix, cap)`` of ``parts``, in one launch: ``v_i``
+    the normed row of the ``RmsInput`` ``h``, or with ``mix >= 0`` its blend ``token_shift(h, prev, mu)[mix]``; ``cap > 0``: ``cap *
+    tanh(. / cap)``. ``row``: the normed rows, which ``prev`` is to hold when this token is done (``timemix_memory``). None where the
+    separate ops run."""
+    if not isinstance(h, RmsInput) or not _gpu(h.x) or h._value is not None or h.x.shape[0] > RESIDUAL_MAX_ROWS \
+            or any(w.dtype != BF16 for w, _, _ in parts) or not h.x.is_contiguous() or h.gain.numel() != h.x.shape[1]:
+        return None
+    m = h.x.shape[0]
+    flat = torch.empty(m * sum(w.shape[0] for w, _, _ in parts), dtype=F32, device=h.x.device)
+    outs, at = [], 0
+    for w, _, _ in parts:
+        outs.append(flat[at:at + m * w.shape[0]].view(m, w.shape[0]))
+        at += m * w.shape[0]
+    row = torch.empty_like(h.x)
+    if ext().rows_parts(h.x, h.gain, h.eps, prev, mu, [w for w, _, _ in parts], [int(j) for _, j, _ in parts],
+                        [float(c) for _, _, c in parts], outs, row):
+        return outs, row
+    return None
+
+
 def mlstm_prep(proj: torch.Tensor, col_i: int, col_f: int, gate_bias: torch.Tensor, cap: float, mstate: torch.Tensor,
                b: int, s: int, heads: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Gates of the stabilised exponential-gate memory from columns of ``proj [B*S, .]``: per head
@@ -1632,20 +1653,28 @@ def mlstm_memory(proj: torch.Tensor, heads: int, dim: int, vdim: int, gate_bias:
     return gated_rmsnorm(o, gate, w, eps, GATE_SIGMOID, denom_floor=floor, gain=gain, out=out)
 
 
-def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre: torch.Tensor, w0: torch.Tensor, u: torch.Tensor,
+def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre, w0: torch.Tensor, u: torch.Tensor,
                    state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float, gain: float = 1.0,
-                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``gated_rmsnorm(timemix_scan(...), gate, w, eps, GATE_SILU, gain=gain, out=out)``."""
+                   out: Optional[torch.Tensor] = None, carry: Optional[tuple] = None) -> torch.Tensor:
+    """``gated_rmsnorm(timemix_scan(...), gate, w, eps, GATE_SILU, gain=gain, out=out)``. ``wpre`` may be a pair ``(z, w2)``: ``linear(z,
+    w2)``, in the launch of one token. ``carry = (prev, row)``: ``prev`` is set to ``row``."""
     h, dim, vdim = r.shape[1], r.shape[2], v.shape[2]
     to = _step_out(r, h * vdim, dim, vdim, s, out)
+    pair = wpre if isinstance(wpre, tuple) else None
+    low = to is not None and pair is not None and pair[1].shape[1] % 4 == 0
+    if pair is not None and not low:
+        wpre = linear(*pair).unflatten(1, (h, dim))
+    if carry is not None and not low:
+        carry[0].copy_(carry[1])
     if to is None and _gpu(r) and s > 1:  # (heads of 64: recurrence and norm of a prompt together)
         y = torch.empty(b * s, h * vdim, dtype=F32, device=r.device) if out is None else out
         if ext().timemix_norm(r, k, v, wpre, w0.reshape(h, dim), u.reshape(h, dim), state, b, s, gate, w, float(eps), float(gain), y):
             return y
     if to is None:
         return gated_rmsnorm(timemix_scan(r, k, v, wpre, w0, u, state, b, s), gate, w, eps, GATE_SILU, gain=gain, out=out)
-    ext().rec_step(1, r, k, v, pre=wpre, w0=w0.reshape(h, dim), u=u.reshape(h, dim), state=state, gate=gate, w=w, eps=float(eps),
-                   gate_act=GATE_SILU, gain=float(gain), out=to)
+    gates = dict(pre_x=pair[0], pre_w=pair[1], prev=carry[0] if carry else None, row=carry[1] if carry else None) if low else dict(pre=wpre)
+    ext().rec_step(1, r, k, v, w0=w0.reshape(h, dim), u=u.reshape(h, dim), state=state, gate=gate, w=w, eps=float(eps),
+                   gate_act=GATE_SILU, gain=float(gain), out=to, **gates)
     return to
 
 

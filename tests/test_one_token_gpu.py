@@ -86,3 +86,37 @@ def _strided(x):
     big = torch.zeros(x.shape[0], x.shape[1] + 8, device=DEV)
     big[:, :x.shape[1]] = x.to(DEV)
     return big[:, :x.shape[1]]
+
+
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("d", [256, 264, 2048, 2056, 4096])
+def test_inputs_of_a_token_shift_in_one_launch(m, d):
+    """Products of the normed row and of its blends with the row before it, as the norm, the blend and the products one by one; odd
+    widths, a capped part, a part of one column, and more columns than are resident at once."""
+    x, gain, prev, mu = _rand(m, d), torch.rand(d) + 0.5, _rand(m, d), torch.rand(3, d)
+    parts = [(_rand(n, d, dt=BF16, std=d ** -0.5), j, cap) for n, j, cap in ((70, -1, 0.0), (1, 2, 0.0), (8200, 0, 0.0), (33, 1, 1.0), (4, 2, 0.5))]
+    h = hy.RmsInput(x.to(DEV), gain.to(DEV), 1e-5)
+    got = hy.shifted_linears(h, prev.to(DEV), mu.to(DEV), [(w.to(DEV), j, c) for w, j, c in parts])
+    assert got is not None
+    row = hy.rms_rows(x, gain, 1e-5)
+    _close(got[1], row, 2e-6, "row")
+    for y, (w, j, cap) in zip(got[0], parts):
+        v = got[1].cpu() if j < 0 else hy.token_shift(got[1].cpu(), prev.clone(), mu, m, 1)[j]
+        ref = hy.linear(v, w)
+        # (a blend's last bit in 32 bits may round it to either of two bf16 neighbours: one number of d, 2^-8 of it)
+        _close(y, cap * torch.tanh(ref / cap) if cap else ref, 2e-5 + 2.0 ** -8 * d ** -0.5, f"part of {w.shape[0]}")
+
+
+@pytest.mark.parametrize("dt", [BF16, torch.float32])
+@pytest.mark.parametrize("b,h,dim,rank,width", [(1, 3, 64, 64, 200), (2, 2, 64, 4, 64), (1, 4, 128, 36, 5000), (3, 2, 20, 60, 40), (1, 2, 256, 64, 512)])
+def test_time_mix_of_one_token_takes_its_decay_product(dt, b, h, dim, rank, width):
+    hd = (h, dim)
+    r, k, v = (_rand(b, *hd) for _ in range(3))
+    z, w2, w0, u, gate, w = torch.tanh(_rand(b, rank)), _rand(h * dim, rank, dt=dt, std=rank ** -0.5), _rand(*hd) - 2.0, _rand(*hd), _rand(b, h * dim), torch.rand(h * dim)
+    st, prev, row = _rand(b, h, dim, dim), _rand(b, width), _rand(b, width)
+    s_dev, p_dev = st.to(DEV), prev.to(DEV)
+    got = hy.timemix_memory(*(t.to(DEV) for t in (r, k, v)), (z.to(DEV), w2.to(DEV)), w0.to(DEV), u.to(DEV), s_dev, b, 1, gate.to(DEV), w.to(DEV),
+                            1e-5, 0.7, carry=(p_dev, row.to(DEV)))
+    want = hy.timemix_memory(r, k, v, (z, w2), w0, u, st, b, 1, gate, w, 1e-5, 0.7, carry=(prev, row))
+    _close(got, want, 2e-5, "output"), _close(s_dev, st, 2e-5, "state")
+    assert torch.equal(p_dev.cpu(), row) and torch.equal(prev, row)
