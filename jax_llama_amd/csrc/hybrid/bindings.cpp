@@ -1199,6 +1199,35 @@ void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT 
   rc(jla::hy_rec_step(p, stream()), "rec_step");
 }
 
+// The delta rule of one token from its fused projection; false (nothing done) where its shapes are not the kernel's.
+bool delta_step(Tensor proj, int64_t B, int64_t H, int64_t G, int64_t dim, int64_t vdim, Tensor conv_w, Tensor conv_state, Tensor a_log,
+                Tensor dt_bias, Tensor tickets, Tensor state, Tensor w, double eps, Tensor out) {
+  const jla::DeltaPrep d = delta_args(proj, B, 1, H, G, dim, vdim, conv_w, conv_state);
+  if (d.taps != 4 || !rec_step_takes(dim, vdim) || G < 1 || H % G || B > 65535 || tickets.numel() < B * G * 4 * 32 ||
+      ((uintptr_t)d.conv_w & 15) != 0)
+    return false;
+  jla::RecStep p{};
+  p.mode = 4; p.B = B; p.H = H; p.G = G; p.dim = dim; p.vdim = vdim;
+  p.proj = d.proj; p.ldproj = d.ld;
+  p.conv_w = d.conv_w;
+  p.conv_state = d.conv_state;
+  check(a_log.numel() == H && dt_bias.numel() == H, "delta_step: per-head constants");
+  p.a_log = f32(a_log, "a_log");
+  p.dt_bias = f32(dt_bias, "dt_bias");
+  p.tickets = i32w(tickets, "tickets", B * G * 4 * 32);
+  check(state.numel() == B * H * dim * vdim, "delta_step: state");
+  p.state = f32w(state, "state");
+  p.gate = p.proj + 2 * G * dim + H * vdim;
+  p.ldg = p.ldproj;
+  check(w.numel() == vdim || w.numel() == H * vdim, "delta_step: norm gain");
+  p.w = f32(w, "w");
+  p.w_heads = w.numel() != vdim || H == 1;
+  p.eps = eps; p.gate_act = 0; p.gain = 1.f;
+  p.out = slice2d(out, "out", B, H * vdim, &p.ldo);
+  rc(jla::hy_rec_step(p, stream()), "delta_step");
+  return true;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1258,6 +1287,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("timemix_norm", &timemix_norm);
   m.def("rows_parts", &rows_parts);
+  m.def("delta_step", &delta_step);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
   m.def("delta_scan", &delta_scan);

@@ -567,6 +567,14 @@ struct RecStep {
   const float* u;
   const float* beta; // mode 3: [B, H]
   const float* decay;
+  // mode 4: the delta rule from its projection, in the place of q, k, v, beta, decay (DeltaPrep with four taps and its tail)
+  const float* proj;
+  int ldproj;
+  const float* conv_w;
+  float* conv_state;
+  const float* a_log;
+  const float* dt_bias;
+  int32_t* tickets;  // [B * G * 4 * 32] zeros, left as zeros: not shared between launches that may run at the same time
   const float* gate_i;  // mode 0: pre-activations of row b, head h at gate_i[b * ldgate + h]
   const float* gate_f;
   int ldgate;

@@ -19,7 +19,8 @@
 namespace jla {
 
 constexpr int RS_THREADS = 1024, RS_MAX = 256;
-enum { RS_MLSTM = 0, RS_TIMEMIX = 1, RS_RUNNING = 2, RS_DELTA = 3 };
+enum { RS_MLSTM = 0, RS_TIMEMIX = 1, RS_RUNNING = 2, RS_DELTA = 3, RS_CONV = 4 };  // (RS_CONV: the delta rule from its projection)
+constexpr int RS_TAPS = 4;
 
 // Sums of N numbers per thread over the first `nw` waves of the block; red holds 16 N floats. Every thread gets them.
 template <int N>
@@ -62,12 +63,33 @@ JLA_DEV float rs_low_rank(const RecStep& p, int b, size_t d, int lane, int lanes
   return s;
 }
 
+// SiLU of the short convolution of channel c at this token; x: its inputs, the carried ones first
+JLA_DEV float rs_conv(const RecStep& p, int b, int c, float (&x)[RS_TAPS]) {
+  const int C = 2 * p.G * p.dim + p.H * p.vdim;
+  const float* tail = p.conv_state + ((size_t)b * C + c) * (RS_TAPS - 1);
+#pragma unroll
+  for (int i = 0; i < RS_TAPS - 1; ++i) x[i] = tail[i];
+  x[RS_TAPS - 1] = p.proj[(size_t)b * p.ldproj + c];
+  const f32x4 w = *reinterpret_cast<const f32x4*>(p.conv_w + (size_t)c * RS_TAPS);
+  float y = 0.f;
+#pragma unroll
+  for (int i = 0; i < RS_TAPS; ++i) y = fmaf(w[i], x[i], y);
+  return hy_silu(y);
+}
+JLA_DEV void rs_conv_carry(const RecStep& p, int b, int c, const float (&x)[RS_TAPS]) {
+  const int C = 2 * p.G * p.dim + p.H * p.vdim;
+  float* tail = p.conv_state + ((size_t)b * C + c) * (RS_TAPS - 1);
+#pragma unroll
+  for (int i = 0; i < RS_TAPS - 1; ++i) tail[i] = x[i + 1];
+}
+
 // grid (H, B). Thread -> value column j = t % cw, key rows [RPT s, RPT s + RPT) of slice s = t / cw (cw: vdim rounded up to
 // whole waves).
 template <int MODE, int RPT>
 __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw) {
   __shared__ float la[RS_MAX], lb[RS_MAX], lc[RS_MAX], lw[RS_MAX];
-  __shared__ float part[(MODE == RS_DELTA ? 2 : 1) * RS_THREADS];
+  constexpr bool DELTA = MODE == RS_DELTA || MODE == RS_CONV;
+  __shared__ float part[(DELTA ? 2 : 1) * RS_THREADS];
   __shared__ float red[4 * 16];
   const int t = threadIdx.x, h = blockIdx.x, b = blockIdx.y;
   const int dim = p.dim, vdim = p.vdim, ncols = MODE == RS_MLSTM ? vdim + 1 : vdim;
@@ -77,11 +99,29 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
   float S[RPT];
 #pragma unroll
   for (int i = 0; i < RPT; ++i) S[i] = st[(size_t)min(d0 + i, dim - 1) * ncols + (col ? j : 0)];
-  const float v = p.v[(size_t)b * p.ldv + (size_t)h * vdim + (col ? j : 0)];
   const bool key = t < dim;
   const int td = key ? t : 0;
-  const int kh = MODE == RS_DELTA ? h / (p.H / p.G) : h;
-  const float q = p.q[(size_t)b * p.ldq + (size_t)kh * dim + td], k = MODE == RS_RUNNING ? 0.f : p.k[(size_t)b * p.ldk + (size_t)kh * dim + td];
+  const int kh = DELTA ? h / (p.H / p.G) : h;
+  float v = 0.f, q = 0.f, k = 0.f;
+  float xq[RS_TAPS], xk[RS_TAPS];  // RS_CONV: the inputs of this thread's query and key channel, which the key head's heads share
+  int before = 0;                  // ... and how many of those heads have read the carried ones
+  if (MODE == RS_CONV) {
+    const int QK = p.G * dim;
+    if (t < cw) {
+      float xv[RS_TAPS];
+      const int c = 2 * QK + h * vdim + (col ? j : 0);
+      v = rs_conv(p, b, c, xv);
+      if (col) rs_conv_carry(p, b, c, xv);  // (this thread is the channel's only reader)
+    }
+    if (key) {
+      q = rs_conv(p, b, kh * dim + t, xq);
+      k = rs_conv(p, b, QK + kh * dim + t, xk);
+    }
+  } else {
+    v = p.v[(size_t)b * p.ldv + (size_t)h * vdim + (col ? j : 0)];
+    q = p.q[(size_t)b * p.ldq + (size_t)kh * dim + td];
+    k = MODE == RS_RUNNING ? 0.f : p.k[(size_t)b * p.ldk + (size_t)kh * dim + td];
+  }
   // the head's vectors over its key rows, and the sums that need them
   float e[2] = {0.f, 0.f};  // e; exponential gates: the normaliser's read-out
   float floor_ = 0.f, m_new = 0.f, g = 0.f, beta = 0.f;
@@ -131,6 +171,22 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
       lc[t] = (1.f - wr) * qs;
       e[0] = wr * qs;
     }
+  } else if (MODE == RS_CONV) {
+    const float* row = p.proj + (size_t)b * p.ldproj + 2 * p.G * dim + 2 * p.H * vdim;
+    beta = hy_sigmoid(row[h]);
+    g = expf(-expf(p.a_log[h]) * hy_softplus(row[p.H + h] + p.dt_bias[h]));
+    float n[2] = {q * q, k * k};  // (0 past the key rows)
+    rs_sum(n, (dim + 63) / 64, red);
+    // a wave has its carried inputs in registers now: it takes its ticket, whose answer is needed at the end only
+    if ((t & 63) == 0 && key) before = __hip_atomic_fetch_add(p.tickets + (((size_t)b * p.G + kh) * 4 + t / 64) * 32, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    q *= 1.f / sqrtf(n[0] + 1e-6f) * (1.f / sqrtf((float)dim));
+    k *= 1.f / sqrtf(n[1] + 1e-6f);
+    if (key) {
+      lb[t] = k;
+      lc[t] = g * q;
+      e[0] = k * q;
+    }
+    __syncthreads();  // (red is read)
   } else {
     g = p.decay[(size_t)b * p.H + h];
     beta = p.beta[(size_t)b * p.H + h];
@@ -148,11 +204,11 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
   for (int i = 0; i < RPT; ++i) {
     if (d0 + i < dim) {
       o[i & 1] = fmaf(S[i], lc[d0 + i], o[i & 1]);
-      if (MODE == RS_DELTA) sk[i & 1] = fmaf(S[i], lb[d0 + i], sk[i & 1]);
+      if (DELTA) sk[i & 1] = fmaf(S[i], lb[d0 + i], sk[i & 1]);
     }
   }
   part[t] = o[0] + o[1];
-  if (MODE == RS_DELTA) part[RS_THREADS + t] = sk[0] + sk[1];
+  if (DELTA) part[RS_THREADS + t] = sk[0] + sk[1];
   __syncthreads();
   const int slices = RS_THREADS / cw;
   float out = 0.f;
@@ -160,9 +216,9 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
     double so = 0.0, ssk = 0.0;  // (one behind the other in 32 bits they would lose more than the scans' lane exchanges do)
     for (int s = 0; s < slices; ++s) {
       so += part[s * cw + t];
-      if (MODE == RS_DELTA) ssk += part[RS_THREADS + s * cw + t];
+      if (DELTA) ssk += part[RS_THREADS + s * cw + t];
     }
-    const float w = MODE == RS_DELTA ? beta * (float)(v - g * ssk) : v;  // (t < cw: this thread's v is column t's)
+    const float w = DELTA ? beta * (float)(v - g * ssk) : v;  // (t < cw: this thread's v is column t's)
     lw[t] = w;
     out = (float)(so + (double)e[0] * w);
     if (MODE == RS_MLSTM) out *= 1.f / (fmaxf(fabsf(e[0] + e[1]), floor_) + 1e-6f);
@@ -176,7 +232,7 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
     const int d = d0 + i;
     if (d < dim && col) {
       const float n = MODE == RS_RUNNING ? fmaf(lb[d], w - S[i], S[i])
-                      : fmaf(MODE == RS_DELTA ? g : la[d], S[i], lb[d] * w);
+                      : fmaf(DELTA ? g : la[d], S[i], lb[d] * w);
       st[(size_t)d * ncols + j] = n;
     }
   }
@@ -189,6 +245,14 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
     }
     p.out[(size_t)b * p.ldo + (size_t)h * vdim + t] = out * sc * p.w[(p.w_heads ? (size_t)h * vdim : 0) + t] * gate * p.gain;
   }
+  if (MODE == RS_CONV && key) {  // the last of the key head's heads to have read the carried inputs moves them on (nobody waits)
+    const int first = __builtin_amdgcn_readfirstlane(before);
+    if (first == p.H / p.G - 1) {
+      rs_conv_carry(p, b, kh * dim + t, xq);
+      rs_conv_carry(p, b, p.G * dim + kh * dim + t, xk);
+      if ((t & 63) == 0) __hip_atomic_store(p.tickets + (((size_t)b * p.G + kh) * 4 + t / 64) * 32, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 }
 
 bool hy_rec_step_takes(int dim, int vdim) {
@@ -198,10 +262,11 @@ bool hy_rec_step_takes(int dim, int vdim) {
 }
 
 int hy_rec_step(const RecStep& p, hipStream_t s) {
-  if (p.mode < 0 || p.mode > 3 || p.B < 0 || p.H < 1 || !hy_rec_step_takes(p.dim, p.vdim)) return -1;
+  if (p.mode < 0 || p.mode > 4 || p.B < 0 || p.H < 1 || !hy_rec_step_takes(p.dim, p.vdim)) return -1;
   if (p.mode == RS_DELTA && (p.G < 1 || p.H % p.G)) return -2;
   if (p.gate_act < 0 || p.gate_act > 2 || (p.gate_act != 2 && !p.gate)) return -3;
   if (p.pre_x && (p.mode != RS_TIMEMIX || p.rank < 4 || p.rank % 4 || !p.pre_w)) return -5;
+  if (p.mode == RS_CONV && (!p.proj || !p.conv_w || !p.conv_state || !p.a_log || !p.dt_bias || !p.tickets)) return -6;
   if (p.B == 0) return 0;
   if (p.B > 65535) return -4;
   const int cw = (p.vdim + 63) / 64 * 64, slices = RS_THREADS / cw;
@@ -216,6 +281,7 @@ int hy_rec_step(const RecStep& p, hipStream_t s) {
   if (p.mode == RS_MLSTM) RS_RUN(RS_MLSTM);
   else if (p.mode == RS_TIMEMIX) RS_RUN(RS_TIMEMIX);
   else if (p.mode == RS_RUNNING) RS_RUN(RS_RUNNING);
+  else if (p.mode == RS_CONV) RS_RUN(RS_CONV);
   else RS_RUN(RS_DELTA);
 #undef RS_RUN
   JLA_CHECK_LAUNCH();

@@ -95,7 +95,7 @@ class KVCacheRows:
         return self.parent.k[i, self.b0:self.b1], self.parent.v[i, self.b0:self.b1]
 
 
-TICKET_INTS = 64 * 32  # tickets of a cache row: 64 heads, each on a line of its own (csrc: AS_TICKET)
+TICKET_INTS = 64 * 32  # tickets of a cache row: 64, each on a line of its own (csrc: AS_TICKET)
 
 
 class HybridCache:
@@ -134,8 +134,8 @@ class HybridCache:
         self._device = device
         self.index = 0
         self.index_t = torch.zeros(1, dtype=torch.int32, device=device)
-        # counters of the one-launch decode attention (ops.hybrid.attn_step), which leaves them at zero: one per row and head, part
-        # of the cache because two steps on one cache are never in flight at once
+        # counters of the one-launch decode steps (ops.hybrid.attn_step, delta_step), which leave them at zero: part of the cache because
+        # two steps on one cache are never in flight at once
         self.tickets = torch.zeros(batch_size * TICKET_INTS, dtype=torch.int32, device=device)
 
     @staticmethod

@@ -130,6 +130,11 @@ class GatedDeltaMixer:
         sp = self.spec
         proj = hy.linear(x, self.w_in)
         state, tail = ctx.cache.recurrent(self.i)
+        if ctx.s == 1:
+            y = hy.delta_step(proj, ctx.b, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w, tail, self.a_log, self.dt_bias, state,
+                              self.norm_w, self.eps, ctx.tickets)
+            if y is not None:
+                return hy.linear(y, self.w_o)
         q, k, v, beta, decay = hy.delta_prep(proj, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w,
                                              tail, self.a_log, self.dt_bias)
         c = 2 * sp.kv_heads * sp.dim + sp.heads * sp.vdim

@@ -1308,6 +1308,18 @@ def delta_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.
     return out
 
 
+def delta_step(proj: torch.Tensor, b: int, heads: int, kv_heads: int, dim: int, vdim: int, conv_w: torch.Tensor, tail: torch.Tensor,
+               a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, w: torch.Tensor, eps: float,
+               tickets: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``delta_prep`` and ``delta_memory`` (gated by the projection's gate columns) of one token per row in one launch; ``tickets``: zeros
+    that no concurrent step uses (the cache's). None where only the separate ops apply."""
+    if not _gpu(proj) or tickets is None:
+        return None
+    out = torch.empty(b, heads * vdim, dtype=F32, device=proj.device)
+    return out if ext().delta_step(proj, b, heads, kv_heads, dim, vdim, conv_w, tail, a_log, dt_bias, tickets, state, w, float(eps),
+                                   out) else None
+
+
 # ------------------------------------------------------------------------------------------------ rotary positions
 def rotary_freqs(base: float, dims: int, device) -> torch.Tensor:
     """float64 ``[dims / 2]``: ``base^(-2 i / dims)``, the turn per position of pair ``i``. Angles are formed in 64-bit

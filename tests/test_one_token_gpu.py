@@ -120,3 +120,22 @@ def test_time_mix_of_one_token_takes_its_decay_product(dt, b, h, dim, rank, widt
     want = hy.timemix_memory(r, k, v, (z, w2), w0, u, st, b, 1, gate, w, 1e-5, 0.7, carry=(prev, row))
     _close(got, want, 2e-5, "output"), _close(s_dev, st, 2e-5, "state")
     assert torch.equal(p_dev.cpu(), row) and torch.equal(prev, row)
+
+
+@pytest.mark.parametrize("b,h,g,dim,vdim", [(1, 4, 1, 128, 128), (2, 4, 2, 64, 64), (3, 3, 3, 40, 20), (1, 16, 4, 128, 128), (2, 6, 2, 200, 64),
+                                            (1, 2, 1, 64, 256), (1, 2, 1, 256, 64), (70, 4, 2, 64, 64)])
+def test_delta_rule_of_one_token_from_its_projection(b, h, g, dim, vdim):
+    """Three tokens one after the other (the carried convolution inputs move on once per token, whichever head comes last) as the
+    separate ops on the CPU; the tickets are back at zero."""
+    c = 2 * g * dim + h * vdim
+    conv_w, tail, st = _rand(c, 4, std=0.6), _rand(b, c, 3), _rand(b, h, dim, vdim)
+    a_log, dt, w = torch.rand(h) - 1.0, _rand(h), torch.rand(vdim) + 0.5
+    s_dev, t_dev, tickets = st.to(DEV), tail.to(DEV), torch.zeros(b * g * 128, dtype=torch.int32, device=DEV)
+    for _ in range(3):
+        proj = _rand(b, c + h * vdim + 2 * h)
+        got = hy.delta_step(proj.to(DEV), b, h, g, dim, vdim, conv_w.to(DEV), t_dev, a_log.to(DEV), dt.to(DEV), s_dev, w.to(DEV), 1e-5, tickets)
+        q, k, v, beta, decay = hy.delta_prep(proj, b, 1, h, g, dim, vdim, conv_w, tail, a_log, dt)
+        want = hy.delta_memory(q, k, v, beta, decay, st, b, 1, proj[:, c:c + h * vdim], w, 1e-5)
+        assert got is not None
+        _close(got, want, 2e-5, "output"), _close(s_dev, st, 2e-5, "state")
+        assert torch.equal(t_dev.cpu(), tail) and not tickets.any()
