@@ -221,7 +221,7 @@ void linear_skinny(Tensor x, Tensor w, int64_t n, int64_t k, Tensor out, int64_t
 // greedy lm_head at decode M (<= 64): GEMV with a first-max epilogue -> [M][N / 16] (value, index) partials in
 // `part`, then one wave per row picks the first maximum (the fp32 logits are never written)
 void linear_skinny_argmax(Tensor x, Tensor w, int64_t n, int64_t k, double rms_eps, int64_t variant, Tensor part,
-                          Tensor idx, Tensor val) {
+                          c10::optional<Tensor> idx, c10::optional<Tensor> val) {
   check_gpu(x, "x");
   check_packed(w, n, k);
   check(x.dim() == 2 && x.size(1) == k && (x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16),
@@ -232,16 +232,20 @@ void linear_skinny_argmax(Tensor x, Tensor w, int64_t n, int64_t k, double rms_e
         "argmax: GEMV variants only (row-major x)");
   check_gpu(part, "part");
   check(part.scalar_type() == torch::kFloat32 && part.numel() >= m * (n / 16) * 2, "argmax partials too small");
-  check_gpu(idx, "idx");
-  check_gpu(val, "val");
-  check(idx.scalar_type() == torch::kInt32 && val.scalar_type() == torch::kFloat32 && idx.numel() == m &&
-            val.numel() == m,
-        "argmax outputs");
+  check(idx.has_value() == val.has_value(), "argmax outputs together");  // (absent: the partials are the result)
+  if (idx.has_value()) {
+    check_gpu(*idx, "idx");
+    check_gpu(*val, "val");
+    check(idx->scalar_type() == torch::kInt32 && val->scalar_type() == torch::kFloat32 && idx->numel() == m &&
+              val->numel() == m,
+          "argmax outputs");
+  }
   jla::QKVArgs qa{};
   rc(jla::linear_skinny(x.data_ptr(), x.scalar_type() == torch::kFloat32, w.data_ptr(), part.data_ptr(), m, n, k,
                         MODE_ARGMAX_ID, (float)rms_eps, 0, 1, &qa, variant, stream()),
      "linear_skinny_argmax");
-  rc(jla::argmax_partials(ptr<float>(part), n / 16, m, ptr<int32_t>(idx), ptr<float>(val), stream()), "argmax_partials");
+  if (idx.has_value())
+    rc(jla::argmax_partials(ptr<float>(part), n / 16, m, ptr<int32_t>(*idx), ptr<float>(*val), stream()), "argmax_partials");
 }
 
 // the decode workspace of the split-K GEMV variants (16 / 18 / 26): partial slabs + tickets
@@ -632,6 +636,34 @@ void topk_merge(Tensor cv, Tensor ci, int64_t k, int64_t mode, c10::optional<Ten
      "topk_merge");
 }
 
+// Partials [B, n, 2] of the greedy choice over logits in memory
+Tensor argmax_parts(Tensor logits) {
+  check_gpu(logits, "logits");
+  check(logits.scalar_type() == torch::kFloat32 && logits.dim() == 2 && logits.size(0) >= 1 && logits.size(0) <= 256,
+        "logits must be fp32 [B <= 256, V]");
+  const int64_t b = logits.size(0), v = logits.size(1);
+  Tensor part = torch::empty({b, (int64_t)jla::argmax_part_count(b, v), 2}, logits.options());
+  rc(jla::argmax_parts(ptr<float>(logits), b, v, ptr<float>(part), stream()), "argmax_parts");
+  return part;
+}
+
+void argmax_next(Tensor part, Tensor finished, Tensor sequences, Tensor cur_len, Tensor tokens, Tensor positions, Tensor slot,
+                 int64_t pad, int64_t eos) {
+  check_gpu(part, "part");
+  check(part.scalar_type() == torch::kFloat32 && part.dim() == 3 && part.size(2) == 2 && part.size(1) >= 1, "argmax_next: part is fp32 [B, n, 2]");
+  for (auto* t : {&finished, &sequences, &cur_len, &tokens, &positions, &slot}) {
+    check_gpu(*t, "argmax_next arg");
+    check(t->scalar_type() == torch::kInt32, "argmax_next: int32 tensors");
+  }
+  const int64_t b = part.size(0);
+  check(b >= 1 && b <= 256 && finished.numel() == b && tokens.numel() == b && positions.numel() == b && sequences.dim() == 2 &&
+            sequences.size(0) == b && cur_len.numel() >= 1 && slot.numel() >= 1,
+        "argmax_next shapes");
+  rc(jla::argmax_next(ptr<float>(part), part.size(1), ptr<int32_t>(finished), ptr<int32_t>(sequences), ptr<int32_t>(cur_len),
+                      ptr<int32_t>(tokens), ptr<int32_t>(positions), ptr<int32_t>(slot), b, sequences.size(1), pad, eos, stream()),
+     "argmax_next");
+}
+
 void decode_update(Tensor nxt, Tensor finished, Tensor sequences, Tensor cur_len, Tensor tokens, Tensor positions,
                    Tensor slot, int64_t pad, int64_t eos) {
   for (auto* t : {&nxt, &finished, &sequences, &cur_len, &tokens, &positions, &slot}) {
@@ -870,7 +902,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_dbg for the bounds-chec
   }, py::arg("m"), py::arg("rep"), py::arg("spl") = 1, py::arg("o_groups") = 0);
   m.def("attn_decode_packs", &jla::attn_decode_packs);
   m.def("skinny_workspace", &skinny_workspace);
-  m.def("linear_skinny_argmax", &linear_skinny_argmax);
+  m.def("linear_skinny_argmax", &linear_skinny_argmax, py::arg("x"), py::arg("w"), py::arg("n"), py::arg("k"), py::arg("rms_eps"),
+        py::arg("variant"), py::arg("part"), py::arg("idx") = py::none(), py::arg("val") = py::none());
   m.def("gemm_tp_residual", &gemm_tp_residual, py::arg("state"), py::arg("x"), py::arg("w"), py::arg("n"), py::arg("k"),
         py::arg("h"), py::arg("hb"), py::arg("ksplit"), py::arg("ws"), py::arg("tile"));
   m.def("gemm_tp_groups", [](int64_t m, int64_t n) { return (int64_t)jla::gemm_tp_groups((int)m, (int)n); });
@@ -936,6 +969,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_dbg for the bounds-chec
         py::arg("kv_start"), py::arg("key_mask").none(true), py::arg("out"));
   m.def("attn_prefill_set_impl", [](int64_t impl) { jla::attn_prefill_set_impl((int)impl); });
   m.def("argmax", &argmax);
+  m.def("argmax_parts", &argmax_parts);
+  m.def("argmax_next", &argmax_next);
   m.def("topk_chunks", [](int64_t v) { return jla::topk_chunks(v); });
   m.def("car_alloc", &car_alloc);
   m.def("car_init", &car_init);

@@ -186,6 +186,34 @@ bool rows_fused(Tensor a, Tensor w, Tensor out, OptT y, int64_t nsum, double ysc
   return true;
 }
 
+// The largest of the (softcapped) products of one or two normed rows, the pending residual add included, per workgroup: [R, n, 2] (value,
+// column bits). None: not a call of that kernel, nothing was launched.
+OptT rows_best(Tensor a, Tensor w, OptT y, int64_t nsum, double ysc, OptT res_w, double eps, OptT x_out, Tensor a_norm_w,
+               double a_norm_eps, double cap) {
+  const bool one = a_norm_w.numel() == 1 && w.size(-1) != 1;
+  jla::RowLinear p{};
+  check(a.dim() == 2 && w.dim() == 2 && w.size(1) == a.size(1), "rows_best: a [R, K], w [N, K]");
+  p.wbf16 = wtype(w, "w");
+  p.E = 1; p.K = a.size(1); p.N = w.size(0); p.R = a.size(0);
+  p.w = w.data_ptr();
+  p.w_stride = (long long)p.N * p.K;
+  p.a = rows2d(a, "a", p.K, &p.lda);
+  p.act = cap > 0 ? jla::HY_ACT_SOFTCAP : jla::HY_ACT_NONE;
+  p.act_limit = cap;
+  p.a_norm_w = f32(a_norm_w, "a_norm_w");
+  check(one || a_norm_w.numel() == p.K, "rows_best: norm gain");
+  p.a_norm_one = one;
+  p.a_norm_eps = a_norm_eps;
+  set_residual(p, a, y, nsum, ysc, res_w, eps, x_out);
+  if (p.R == 0 || p.N < 1 || !(p.res_y || one ? jla::hy_rows_gemv_takes_residual(p) : jla::hy_rows_gemv_takes(p))) return c10::nullopt;
+  const int groups = jla::hy_rows_walk_groups(p);
+  if (groups < 1) return c10::nullopt;
+  Tensor best = torch::empty({(int64_t)p.R, (int64_t)groups, 2}, a.options());
+  p.best = reinterpret_cast<float2*>(best.data_ptr());
+  rc(jla::hy_rows_gemv(p, stream()), "rows_best");
+  return best;
+}
+
 // Several matrices on one or two normed rows, blended or not, in one launch: out[i] = ws[i] v_i, v = rms_norm(x) gain, blended v + (prev -
 // v) mu[mix[i]] for mix[i] >= 0, capped (cap[i] > 0); row <- v. False: not a call of that kernel, nothing was launched.
 bool rows_parts(Tensor x, Tensor gain, double eps, Tensor prev, Tensor mu, std::vector<Tensor> ws, std::vector<int64_t> mix,
@@ -1287,6 +1315,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("timemix_norm", &timemix_norm);
   m.def("rows_parts", &rows_parts);
+  m.def("rows_best", &rows_best);
   m.def("delta_step", &delta_step);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);

@@ -70,7 +70,11 @@ struct RowLinear {
   const float* res_w;
   int res_w_vec;
   float* res_out;
+  // optional, the walking form: instead of the products, the largest of every workgroup's (ties to the lowest column, a NaN never):
+  // best [R][hy_rows_walk_groups(p)] (value, column bits); column 0x7fffffff: none
+  float2* best;
 };
+int hy_rows_walk_groups(const RowLinear& p);
 // Several bf16 matrices [N, K] that read the same one or two rows: a normed row v, or blended with the row before it, v + (prev - v)
 // mu[mix] (rows_gemv.hip). first, tgroups: filled in by the launch.
 constexpr int RV_MAX_PARTS = 6;

@@ -59,6 +59,8 @@ JLA_DEV float rv_table(const RowLinear& p, int r, int col) {
   return p.mul_bf16 ? bf2f(reinterpret_cast<const bf16_t*>(p.mul_table)[at]) : reinterpret_cast<const float*>(p.mul_table)[at];
 }
 
+constexpr int RV_WALK_ROWS = 2;
+
 // The sum of N partial sums in type T
 template <class T, int N>
 JLA_DEV float rv_sum(const float (&f)[N]) {
@@ -70,6 +72,14 @@ JLA_DEV float rv_sum(const float (&f)[N]) {
 #pragma unroll
     for (int i = 0; i < n; ++i) s[i] += s[i + n];
   return (float)s[0];
+}
+
+// the better of two candidates of a maximum: the larger, ties to the lower index, a NaN never
+JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
+  if (v > bv || (v == bv && i < bi)) {
+    bv = v;
+    bi = i;
+  }
 }
 
 // output column col of linear row r from its accumulators
@@ -391,13 +401,16 @@ struct RvRow {
 // through LDS once per workgroup, where a pending residual add (res_y) and the norm are applied behind the first weights.
 // grid (workgroups, linear rows with their own expert, else 1). PARTS: several matrices (RowParts) that read the same rows, each with
 // a run of the workgroups, the rows blended for it as they are staged.
-template <int NT, int U, int V, int PARTS>
+template <int NT, int U, int V, int PARTS, int BEST = 0>
 __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
   constexpr int G = 4, WAVES = 4, STEP = 128;
   extern __shared__ f32x4 staged[];  // [rows][K]
   __shared__ f32x4 red[2][WAVES][NT][64];
   __shared__ float stat[WAVES][16];
+  __shared__ float2 cand[BEST ? NT * 4 * RV_WALK_ROWS : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
+  float bv = -INFINITY;  // BEST: this thread's candidate
+  int bi = 0x7fffffff;
   int part = 0, tg = blockIdx.x, walk = gridDim.x;  // this workgroup's first group of tiles, and from one to its next
   if constexpr (PARTS) {
     while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
@@ -482,7 +495,31 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
         return rv_sum<double>(f);
       };
       const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
-      if (col < N) rv_store(p, r0 + x, col, g, v);
+      if constexpr (BEST) {
+        const float val = lr_act(p, g, v);
+        if (col < N && val > bv) {  // (a thread's columns ascend; -inf, as a NaN, is never chosen)
+          bv = val;
+          bi = col;
+        }
+      } else {
+        if (col < N) rv_store(p, r0 + x, col, g, v);
+      }
+    }
+  }
+  if constexpr (BEST) {  // (threads below NT nr G hold candidates, row (tid / G) % nr)
+    const int outs = NT * nr * G;
+    __syncthreads();
+    if (tid < outs) cand[tid] = make_float2(bv, __int_as_float(bi));
+    __syncthreads();
+    if (tid < nr) {
+      float2 best = make_float2(-INFINITY, __int_as_float(0x7fffffff));
+      for (int i = 0; i < outs; ++i) {
+        if (i / G % nr != tid) continue;
+        int at = __float_as_int(best.y);
+        rv_better(best.x, at, cand[i].x, __float_as_int(cand[i].y));
+        best.y = __int_as_float(at);
+      }
+      p.best[(size_t)(r0 + tid) * gridDim.x + blockIdx.x] = best;
     }
   }
 }
@@ -510,7 +547,7 @@ bool hy_rows_gemv_takes(const RowLinear& p) {
 // first weight (RMS norm and product, K 2048 x N 2048 | 5152 | 8224 | 32000 | gated 5632: 6.1 | 9.5 | 12.3 | 34.6 | 13.5 us in the
 // plain form, 5.3 | 7.5 | 9.7 | 23.0 | 10.8 walking; K 4096 x 10304: 26.1 -> 17.8). Rows as they are gain nothing from it (4.7 | 7.2 |
 // 9.3 | 22.7 | 11.5 plain, 5.2 | 7.5 | 9.8 | 22.7 | 11.0 walking). Further rows would not fit the registers.
-constexpr int RV_WALK_K = 4096, RV_WALK_ROWS = 2;
+constexpr int RV_WALK_K = 4096;
 static bool rv_walks(const RowLinear& p, int rows) {
   return (p.a_norm_w || p.res_y) && !p.offs && rows <= RV_WALK_ROWS && p.K <= RV_WALK_K;
 }
@@ -548,6 +585,25 @@ int hy_rows_parts(const RowLinear& p, const RowParts& parts, hipStream_t s) {
   return 0;
 }
 
+// workgroups of the walking form over the columns (of one expert), and the groups of tiles they walk
+static bool rv_walk_grid(const RowLinear& p, int groups, int& wnt, long long& tg, long long& wgs) {
+  // two tiles per step from a few workgroups for every compute unit on; as many workgroups as are resident (four of 88
+  // registers per unit, or two of 156, K > 2048), with equally many steps each
+  const int gated = hy_act_gated(p.act), occ = p.K <= 2048 ? 4 : 2;
+  const long long tiles = (gated ? 2LL : 1LL) * ((p.N + 3) / 4);
+  wnt = gated || tiles * groups >= 1024 ? 2 : 1;
+  tg = (tiles + wnt - 1) / wnt;
+  const long long room = 256LL * occ / groups > 0 ? 256LL * occ / groups : 1, rounds = (tg + room - 1) / room;
+  wgs = (tg + rounds - 1) / rounds;
+  return tg <= 0x7fffffffLL;
+}
+
+int hy_rows_walk_groups(const RowLinear& p) {
+  int wnt;
+  long long tg, wgs;
+  return hy_rows_gemv_takes(p) && rv_walks(p, p.R) && !p.row_expert && !p.tab && rv_walk_grid(p, 1, wnt, tg, wgs) && wnt == 2 ? (int)wgs : 0;
+}
+
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   const int gated = hy_act_gated(p.act);
   RowLinear q = p;
@@ -559,20 +615,19 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // rows of a pass: a dense batch's count rounded up; an expert's share of the sorted rows, twice the mean (at least 4)
   const int even = p.offs && p.even_rows > 0 ? p.even_rows : 0;
   const int rows = each ? 1 : (p.offs ? (even ? even : (p.R < 2 * ((p.R + p.E - 1) / p.E) ? p.R : 2 * ((p.R + p.E - 1) / p.E))) : p.R);
-  if (p.a_norm_one && !rv_walks(p, rows)) return -10;
+  if ((p.a_norm_one || p.best) && !rv_walks(p, rows)) return -10;
   if (rv_walks(p, rows)) {
-    // two tiles per step from a few workgroups for every compute unit on; as many workgroups as are resident (four of 88
-    // registers per unit, or two of 156, K > 2048), with equally many steps each
-    const int occ = p.K <= 2048 ? 4 : 2;
-    const long long tiles = (gated ? 2LL : 1LL) * ((p.N + 3) / 4);
-    const int wnt = gated || tiles * groups >= 1024 ? 2 : 1;
-    const long long tg = (tiles + wnt - 1) / wnt;
-    if (tg > 0x7fffffffLL) return -4;
-    const long long room = 256LL * occ / groups > 0 ? 256LL * occ / groups : 1, rounds = (tg + room - 1) / room;
-    const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
+    int wnt;
+    long long tg, wgs;
+    if (!rv_walk_grid(p, groups, wnt, tg, wgs)) return -4;
+    const dim3 grid((unsigned)wgs, groups);
     const unsigned lds = (unsigned)(rows * p.K * sizeof(float));
 #define RV_WALK(NT, U, V) rows_gemv_walk_kernel<NT, U, V, 0><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
-    if (p.K <= 2048) {
+    if (p.best) {
+      if (wnt != 2 || groups != 1 || gated) return -11;
+      if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 0, 1><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{});
+      else rows_gemv_walk_kernel<2, 8, 4, 0, 1><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{});
+    } else if (p.K <= 2048) {
       if (wnt == 1) RV_WALK(1, 4, 2);
       else RV_WALK(2, 4, 2);
     } else {

@@ -168,6 +168,12 @@ long long car_max_bytes(void* state);
 int car_world(void* state);
 int car_set_grid(void* state, int grid);  // collective blocks per launch (0: the maximum; same on every rank, before first use)
 void car_destroy(void* state);
+// the two halves of greedy choice and bookkeeping (at most 256 rows): partials [B][count] (value, index) of logits in memory; the choice
+// over any such partials with decode_update behind it
+int argmax_part_count(int B, int V);
+int argmax_parts(const float* logits, int B, int V, float* part, hipStream_t s);
+int argmax_next(const float* part, int n, int32_t* finished, int32_t* sequences, int32_t* cur_len, int32_t* tokens, int32_t* positions,
+                int32_t* slot, int B, int L, int pad, int eos, hipStream_t s);
 int decode_update(const int32_t* nxt, int32_t* finished, int32_t* sequences, int32_t* cur_len, int32_t* tokens,
                   int32_t* positions, int32_t* slot, int B, int L, int pad, int eos, hipStream_t s);
 // CU placement (placement.hip): CU-masked streams and a census of where a launch's workgroups run

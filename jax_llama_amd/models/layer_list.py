@@ -22,6 +22,7 @@ from .mixers import StepContext
 
 BF16 = torch.bfloat16
 F32 = torch.float32
+GREEDY_MODES = ("last", "argmax", "argmax_parts")  # logits of every row's last token
 
 
 class LayerListLM:
@@ -119,7 +120,7 @@ class LayerListLM:
                        logit_rows: Optional[torch.Tensor] = None):
         """Run all layers for ``ids [B, S]`` placed at cache slots ``slot0 .. slot0 + S - 1`` (``slot0``: int or a
         device int32[1]); keys / values and recurrent state of ``cache`` advance. Returns ``(logits, x, hidden, [])``:
-        fp32 logits ``[B, V]`` ("last" / "argmax": the sampler reduces them), ``[B*S, V]`` ("all"), the rows
+        fp32 logits ``[B, V]`` ("last" / "argmax": the sampler reduces them; "argmax_parts": or an ``ops.ArgmaxParts``), ``[B*S, V]`` ("all"), the rows
         ``logit_rows`` of the flattened ``[B*S]`` tokens ("rows"), or None ("none"). ``hidden`` (``collect_hidden``):
         the residual stream after every layer. Recurrent layers carry no padding mask: every row's tokens must be
         real (``kv_start`` all zero, no ``key_mask``)."""
@@ -147,7 +148,7 @@ class LayerListLM:
             ctx.hist = torch.empty(len(self.blocks) + 1, b * s, d, dtype=F32, device=self.device)
             x = hy.embed_rows(idf, self.embed, scale=self.embed_scale, out=ctx.hist[0])
             ctx.act_dtype = BF16 if hy.prompt_bf16(b * s, d, self.param_dtype) else F32
-            ctx.every_row = logits_mode == "all" or (s == 1 and logits_mode in ("last", "argmax"))
+            ctx.every_row = logits_mode == "all" or (s == 1 and logits_mode in GREEDY_MODES)
             if self.blocks:
                 ctx.h = hy.squash_rows(x, self.blocks[0].norm, ctx.act_dtype)
                 x = torch.empty_like(x)
@@ -158,7 +159,7 @@ class LayerListLM:
         elif self.chained_norms:
             x = hy.embed_rows(idf, self.embed, scale=self.embed_scale)
             ctx.act_dtype = BF16 if hy.prompt_bf16(b * s, d, self.param_dtype) else F32
-            ctx.every_row = logits_mode == "all" or (s == 1 and logits_mode in ("last", "argmax"))
+            ctx.every_row = logits_mode == "all" or (s == 1 and logits_mode in GREEDY_MODES)
             if self.blocks:
                 ctx.h = hy.sandwich_update_(x, None, None, self.eps, pre=self.blocks[0].pre1, h_dtype=ctx.act_dtype)
             for blk in self.blocks:
@@ -171,13 +172,17 @@ class LayerListLM:
                 blk(r if getattr(blk, "takes_residual", False) else r.value(), ctx)
                 if collect_hidden:
                     hidden.append(r.value().reshape(b, s, d).clone())
-            if s == 1 and logits_mode in ("last", "argmax", "all") and not isinstance(self.final_norm, hy.SquashNorm):
+            if s == 1 and logits_mode == "argmax_parts" and not isinstance(self.final_norm, hy.SquashNorm):
+                parts = hy.head_argmax(r, self.final_norm, self.eps, self.head, float(self.logit_softcap or 0.0))
+                if parts is not None:
+                    return parts, r.x, hidden, []
+            if s == 1 and logits_mode in (*GREEDY_MODES, "all") and not isinstance(self.final_norm, hy.SquashNorm):
                 logits = hy.head_linear(r, self.final_norm, self.eps, self.head, float(self.logit_softcap or 0.0))
                 return logits, r.value(), hidden, []
             x = r.value()
         if logits_mode == "none":
             return None, x, hidden, []
-        if logits_mode in ("last", "argmax"):
+        if logits_mode in GREEDY_MODES:
             xl = x.reshape(b, s, d)[:, -1].contiguous()
         elif logits_mode == "rows":
             xl = x.index_select(0, logit_rows.to(self.device, torch.long))

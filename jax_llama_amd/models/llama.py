@@ -355,7 +355,8 @@ class LLaMAForCausalLM:
         ``slot0``: int or device int32[1] tensor (graph capture). Returns
         ``(logits_local, h, hidden_states, attentions)`` where logits are this rank's
         vocab shard: ``[B, V/tp]`` ("last"), ``[B*S, V/tp]`` ("all"), None ("none"), or the
-        shard's greedy ``(idx int32[B], val fp32[B])`` of the last position ("argmax")."""
+        shard's greedy ``(idx int32[B], val fp32[B])`` of the last position ("argmax"; "argmax_parts": or an
+        ``ops.ArgmaxParts``)."""
         with ops.autotune.tp_scope(self.comm):  # TP: rank 0 picks the kernel plans for every rank
             return self._forward_tokens(ids, positions, cache, slot0, kv_start, key_mask, logits_mode,
                                         collect_hidden, collect_attn)
@@ -376,10 +377,11 @@ class LLaMAForCausalLM:
         elif self.precision == "highest":  # fp32 lm_head weights + fp32 GEMM (reference model.py:698-736)
             hl = h if logits_mode == "all" else h.reshape(b, s, d)[:, -1].contiguous()
             logits = ops.linear_f32(self.final_norm(hl), self.lm_head_f32)
-            if logits_mode == "argmax":
+            if logits_mode in ("argmax", "argmax_parts"):
                 logits = ops.argmax(logits.contiguous())
-        elif logits_mode == "argmax":  # greedy: (idx, val) of this rank's vocab shard, argmax fused in the GEMM
-            logits = ops.linear_argmax(hb.reshape(b, s, d)[:, -1].contiguous(), self.lm_head, rms_eps=self.eps)
+        elif logits_mode in ("argmax", "argmax_parts"):  # greedy: (idx, val) of this rank's vocab shard, argmax fused in the GEMM
+            logits = ops.linear_argmax(hb.reshape(b, s, d)[:, -1].contiguous(), self.lm_head, rms_eps=self.eps,
+                                       parts=logits_mode == "argmax_parts")
         else:
             hl = hb if logits_mode == "all" else hb.reshape(b, s, d)[:, -1].contiguous()
             logits = ops.linear(hl, self.lm_head, rms_eps=self.eps, out_dtype=torch.float32)

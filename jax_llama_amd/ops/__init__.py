@@ -663,16 +663,31 @@ def argmax(logits: torch.Tensor):
     return idx, val
 
 
+class ArgmaxParts:
+    """A step's greedy choice before its last reduction: ``part`` fp32 ``[B, n, 2]`` (value, index bits) on the GPU."""
+
+    MAX_ROWS = 256  # csrc AN_ROWS
+
+    def __init__(self, part: torch.Tensor):
+        self.part = part
+
+    @staticmethod
+    def of(logits: torch.Tensor) -> Optional["ArgmaxParts"]:
+        """Of fp32 logits ``[B, V]`` in memory; None for more rows than one workgroup finishes."""
+        return ArgmaxParts(ext().argmax_parts(logits)) if 1 <= logits.shape[0] <= ArgmaxParts.MAX_ROWS else None
+
+
 ARGMAX_FUSED_MIN_M = 256  # one 256-row tile or more: the tiled GEMM is the lm_head kernel anyway
 # decode M <= 64: the argmax runs in the lm_head GEMV's epilogue (per-16-column partials); JLA_SKINNY_ARGMAX=0 off
 SKINNY_ARGMAX = os.environ.get("JLA_SKINNY_ARGMAX", "1") != "0"
 
 
-def linear_argmax(x: torch.Tensor, w, rms_eps: Optional[float] = None):
+def linear_argmax(x: torch.Tensor, w, rms_eps: Optional[float] = None, parts: bool = False):
     """Greedy token of ``[inv_rms(x) *] x @ W^T`` (the lm_head): ``(idx int32[M], val fp32[M])``, first
     max like ``jnp.argmax``. On the GPU the argmax runs in the GEMM epilogue and the fp32 logits never
     reach HBM: in the decode GEMV's (M <= 64, ``linear_skinny_argmax``) or in the tiled GEMM's (from
-    ARGMAX_FUSED_MIN_M rows, ``gemm_argmax``); in between ``linear`` + ``argmax``."""
+    ARGMAX_FUSED_MIN_M rows, ``gemm_argmax``); in between ``linear`` + ``argmax``. ``parts``: one row's may be left to the caller's
+    last reduction (``ArgmaxParts``)."""
     m = x.shape[0]
     if not _is_gpu(x):
         return argmax(linear(x, w, rms_eps, out_dtype=torch.float32))
@@ -681,6 +696,10 @@ def linear_argmax(x: torch.Tensor, w, rms_eps: Optional[float] = None):
         v = _variant(e, x, w, MODE_STORE, no_split=True)  # the logits GEMV's main loop: its tuned variant applies
         if v in (1, 2, 3, 5, 6, 8, 9, 20):
             part = workspace.get("skinny_argmax", m * (w.n // 16) * 2, torch.float32, x.device)
+            if parts and m == 1:  # (several rows of thousands of partials are for several workgroups)
+                part = part[:w.n // 16 * 2].view(1, w.n // 16, 2)
+                e.linear_skinny_argmax(x, w.weight, w.n, w.k, -1.0 if rms_eps is None else float(rms_eps), v, part)
+                return ArgmaxParts(part)
             idx = torch.empty(m, dtype=torch.int32, device=x.device)
             val = torch.empty(m, dtype=torch.float32, device=x.device)
             e.linear_skinny_argmax(x, w.weight, w.n, w.k, -1.0 if rms_eps is None else float(rms_eps), v, part, idx,

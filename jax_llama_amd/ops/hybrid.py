@@ -306,6 +306,25 @@ def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
     return linear(rms_rows(r.value() if r is not None else x, gain, eps), w, act=act, limit=cap)
 
 
+def head_argmax(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float = 0.0):
+    """The greedy choice over ``head_linear(x, gain, eps, w, cap)`` as an ``ops.ArgmaxParts``, the logits never written; None where
+    that is not one launch (more than two rows, fp32 weights, a short output)."""
+    from . import ArgmaxParts
+    r = x if isinstance(x, Residual) else Residual(x)
+    xv = r.x
+    if not (norms_free(xv.shape[0], w) and gain.numel() in (1, xv.shape[1]) and xv.is_contiguous() and xv.dtype == F32):
+        return None
+    if r.pending is not None and not r.fusable():
+        r.value()
+    new = torch.empty_like(xv) if r.pending is not None else None
+    part = ext().rows_best(xv, w, *(r.pending or (None, 1, 1.0, None, 0.0)), new, gain.reshape(-1), float(eps), float(cap))
+    if part is None:
+        return None
+    if new is not None:
+        r.x, r.pending = new, None
+    return ArgmaxParts(part)
+
+
 def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit: float = 0.0,
            alpha: float = 1.0, out_dtype=F32) -> torch.Tensor:
     """``act(x [M, K] (fp32, or an ``RmsInput``) @ w^T)`` -> fp32 ``[M, N]``. ``act``: none, ``ACT_RELU2`` (``max(y, 0)^2``),

@@ -183,8 +183,17 @@ class DecodeEngine:
         return "argmax" if _fused_greedy() and not self.gc.do_sample else "last"
 
     def _decode_step(self):
+        mode = self._logits_mode()
+        # greedy on one GPU: the choice's last reduction and the bookkeeping are one launch
+        joint = mode == "argmax" and self.device.type == "cuda" and self.model.comm.size == 1
         logits, *_ = self.model.forward_tokens(self.tokens, self.positions, self.cache, self.cache.index_t,
-                                               self.kv_start, self.key_mask, logits_mode=self._logits_mode())
+                                               self.kv_start, self.key_mask, logits_mode="argmax_parts" if joint else mode)
+        if joint and torch.is_tensor(logits):
+            logits = ops.ArgmaxParts.of(logits) or logits
+        if isinstance(logits, ops.ArgmaxParts):
+            ops.ext().argmax_next(logits.part, self.finished, self.sequences, self.cur_len, self.tokens, self.positions,
+                                  self.cache.index_t, int(self.gc.pad_token_id), int(self.gc.eos_token_id))
+            return
         self._update(self._next_token(logits))
 
     # ---------------------------------------------------------------------------------

@@ -139,3 +139,48 @@ def test_delta_rule_of_one_token_from_its_projection(b, h, g, dim, vdim):
         assert got is not None
         _close(got, want, 2e-5, "output"), _close(s_dev, st, 2e-5, "state")
         assert torch.equal(t_dev.cpu(), tail) and not tickets.any()
+
+
+@pytest.mark.parametrize("b,v", [(1, 1), (2, 63), (17, 5000), (1, 12288), (3, 32001), (64, 20000), (65, 13000), (256, 12289), (1, 128256)])
+def test_greedy_choice_and_bookkeeping_in_one_launch(b, v):
+    """Partials of logits with ties, infinities and rows of NaN, the choice over them and the loop's state, as the two launches."""
+    from jax_llama_amd import ops
+    logits = torch.randint(-3, 4, (b, v)).float()
+    logits[0, v // 2:] = float("nan")
+    if b > 2:
+        logits[1], logits[2] = float("nan"), float("-inf")
+        logits[2, v - 1] = float("inf")
+    lg = logits.to(DEV)
+    length, cl, eos, pad = 9, 6, 2, 77
+    state = lambda: dict(finished=(torch.arange(b) % 5 == 3).int().to(DEV), sequences=torch.zeros(b, length, dtype=torch.int32, device=DEV),  # noqa: E731
+                         cur_len=torch.tensor([cl], dtype=torch.int32, device=DEV), tokens=torch.zeros(b, 1, dtype=torch.int32, device=DEV),
+                         positions=torch.arange(b, dtype=torch.int32, device=DEV), slot=torch.tensor([11], dtype=torch.int32, device=DEV))
+    one, two = state(), state()
+    ops.ext().decode_update(ops.argmax(lg)[0], *two.values(), pad, eos)
+    part = ops.ArgmaxParts.of(lg).part
+    for p in (part, torch.cat([part, torch.tensor([float("-inf"), 0.0], device=DEV).expand(b, 70, 2)], 1).contiguous()):  # (a wave, the workgroup)
+        one = state()
+        ops.ext().argmax_next(p, *one.values(), pad, eos)
+        assert all(torch.equal(one[k], two[k]) for k in one)
+    assert ops.ArgmaxParts.of(torch.zeros(257, 8, device=DEV)) is None
+
+
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("d,v", [(256, 4096), (264, 4101), (2048, 32000), (4096, 5000)])
+@pytest.mark.parametrize("pending,cap", [(True, 0.0), (False, 3.0), (True, 3.0)])
+def test_greedy_choice_inside_the_output_product(m, d, v, pending, cap):
+    """The same token, and the same residual stream, as the product written out and its argmax (a cap that ties many columns too)."""
+    from jax_llama_amd import ops
+    w, gain, x, y = _rand(v, d, dt=BF16).to(DEV), (torch.rand(d) + 0.5).to(DEV), _rand(m, d).to(DEV), _rand(2 * m, d).to(DEV)
+    res = []
+    for _ in range(2):
+        r = hy.Residual(x.clone())
+        if pending:
+            r.add(y, gain, 1e-5, nsum=2, ysc=0.5)
+        res.append(r)
+    logits = hy.head_linear(res[0], gain, 1e-5, w, cap)
+    got = hy.head_argmax(res[1], gain, 1e-5, w, cap)
+    part = got.part.cpu()
+    best = [max(((float(a), -int(i)) for a, i in zip(part[r, :, 0], part[r, :, 1].view(torch.int32)))) for r in range(m)]
+    assert [-i for _, i in best] == ops.argmax(logits)[0].tolist()
+    assert torch.equal(torch.tensor([a for a, _ in best]), logits.max(1).values.cpu()) and torch.equal(res[0].x, res[1].x)
