@@ -555,7 +555,7 @@ __global__ void __launch_bounds__(64 * AB_MAX_VREG) attn_diff_merge_kernel(AttnB
 }
 
 // ---- MFMA flash prefill (bf16 caches) ----------------------------------------------------------------------------------
-// One wave = 32 queries of one head, no LDS and no barriers. Keys go by in tiles of 32:
+// One wave = 32 queries of one head. Keys go by in tiles of 32:
 //   S^T = K Q^T on v_mfma_f32_32x32x16_bf16 with the QUERY on the lane (lane l: query l & 31; its 16 accumulators are 16
 //   of the tile's keys, the other half-wave holds the other 16), so scale, soft cap, bias, mask and the online softmax
 //   are lane-local plus one exchange with lane ^ 32. The key rows are fed in an order (bits 2 and 3 of the row index
@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(64 * AB_MAX_VREG) attn_diff_merge_kernel(AttnB
 //   of the B operand of O^T += V^T P^T, so P is used in place. V^T comes from a transposed bf16 copy of the values
 //   (attn_vt_kernel, zero past the last key), 16-byte loads along the keys.
 //   The softmax weights stay 32-bit: P is split into a bf16 high part and a bf16 remainder, two MFMAs per value tile.
-//   Scores of the fast path use exp-based tanh and v_exp_f32; the fp32 format keeps the exact kernel above.
+//   Scores of the fast path use exp-based tanh and v_exp_f32; fp32 caches: attn_f32.hip or the exact kernel above.
 constexpr int AM_Q = 32, AM_K = 32;
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 
@@ -589,154 +589,264 @@ JLA_DEV float am_tanh(float x) {  // 1 - 2 / (e^(2x) + 1), saturating cleanly fo
   return 1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f);
 }
 
-// MAPS = 2 (differential heads): waves 2 t and 2 t + 1 of a workgroup run the two maps of query tile t; the second hands its
-// normalised output to the first through LDS, which subtracts, norms and stores.
-template <int DK, int VT, int MAPS>  // dim = 16 DK, vdim = 32 VT
-__global__ void __launch_bounds__(256) attn_bias_mma_kernel(AttnBias p, const bf16_t* __restrict__ vt, int Tp) {
-  constexpr int TILES = 4 / MAPS;  // query tiles per workgroup
-  __shared__ float joined[MAPS == 2 ? TILES * VT * 16 * 64 : 1];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int map = wave % MAPS;
-  const int ql = lane & 31, hi = lane >> 5;
-  // Workgroups go round the 8 XCDs by their id: where the heads divide evenly, each XCD gets whole runs of neighbouring
-  // heads (which share their keys in grouped-query attention), so that a head's keys and values pass through one L2.
-  const int nq = (p.S + TILES * AM_Q - 1) / (TILES * AM_Q), heads = p.H * p.B;
-  int hb, blk;
-  if (heads % 8 == 0) {
-    const int r = blockIdx.x >> 3, hl = r / nq;
-    hb = (int)(blockIdx.x & 7) * (heads >> 3) + hl;
-    blk = r - hl * nq;
-  } else {
-    hb = blockIdx.x / nq;
-    blk = blockIdx.x - hb * nq;
-  }
-  const int qblk = (nq - 1 - blk) * TILES + wave / MAPS;  // long rows first
-  const int s0 = qblk * AM_Q;
-  const bool live = s0 < p.S;
-  if (MAPS == 1 && !live) return;  // (a pair of waves without queries stays for the workgroup's barrier)
-  const int b = hb / p.H, h = hb - b * p.H;
-  const int g = h / (p.H / p.G), vh = h * MAPS + map;
-  const int slot = *p.slot;
-  const int q0 = slot + s0;                 // cache slot of this wave's first query
-  const int sq = min(s0 + ql, p.S - 1);     // (surplus lanes repeat the last query; never stored)
-  const int qi = slot + sq;
-  constexpr int dim = 16 * DK, vdim = 32 * VT;
-  // Q as the B operand: query ql, k-slots 16 kk + 8 hi + e
-  bf16x8_t qf[DK];
-  {
-    const float* q = p.q + (((size_t)b * p.S + sq) * (p.H * MAPS) + vh) * dim + 8 * hi;
+// What a wave keeps of its 32 queries
+template <int DK, int VT>
+struct AmRow {
+  bf16x8_t q[DK];  // the B operand: query lane & 31, k-slots 16 kk + 8 (lane >> 5) + e
+  f32x16 o[VT];
+  float m, l;      // (l: this half-wave's part of the sum)
+  int q0, qi, lo_q, lo_last, kfirst, vh, heads;
+  float scale, inv_cap;
+};
+
+// The tile of 32 keys from slot j0 on. keys(kk), values(c, v): operand fragments; behind(): what is issued behind the scores' products.
+template <int DK, int VT, class Keys, class Values, class Behind>
+JLA_DEV void am_tile(const AttnBias& p, AmRow<DK, VT>& w, int j0, Keys keys, Values values, Behind behind) {
+  const int lane = threadIdx.x & 63, ql = lane & 31, hi = lane >> 5;
+  // scores: rows = keys (fed permuted), columns = queries
+  f32x16 sacc;
 #pragma unroll
-    for (int kk = 0; kk < DK; ++kk) {
-      float f[8];
-      hy_load8(q + 16 * kk, 8, f);
-      qf[kk] = __builtin_bit_cast(bf16x8_t, pack8(f));
+  for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < DK; ++kk)
+    sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, keys(kk)), w.q[kk], sacc, 0, 0, 0);
+  // bias of this tile's 63 distances, one per lane: lane t holds distance q0 - j0 - 31 + t
+  float bl = 0.f;
+  const int dbase = w.q0 - j0 - (AM_K - 1);
+  if (p.bias) bl = p.bias[(size_t)min(max(dbase + lane, 0), p.nbias - 1) * w.heads + w.vh];
+  behind();
+  // key of accumulator r within the tile: 16 (r >> 3) + 8 hi + (r & 7)
+#pragma unroll
+  for (int r = 0; r < 16; ++r) sacc[r] *= w.scale;
+  if (p.softcap > 0.f) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sacc[r] = p.softcap * am_tanh(sacc[r] * w.inv_cap);
+  }
+  if (p.bias) {
+    if (dbase >= p.nbias - 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sacc[r] += bl;
+    } else {
+      float bk[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bk[r] = __shfl(bl, ql - (16 * (r >> 3) + 8 * hi + (r & 7)) + (AM_K - 1), 64);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sacc[r] += bk[r];
     }
   }
-  const bf16_t* kbase = reinterpret_cast<const bf16_t*>(p.kc) + ((size_t)b * p.G + g) * p.T * p.ldk + map * dim;
-  const bf16_t* vbase = vt + ((size_t)b * p.G + g) * vdim * Tp;
-  const int krow = (ql & 0x13) | ((ql & 4) << 1) | ((ql & 8) >> 1);  // bits 2 and 3 swapped
-  f32x16 o[VT];
+  // some (query, key) of the tile is masked
+  if (j0 + AM_K - 1 > w.q0 || (j0 < w.lo_last && j0 + AM_K - 1 >= w.kfirst)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int j = j0 + 16 * (r >> 3) + 8 * hi + (r & 7);
+      sacc[r] = j > w.qi || (j < w.lo_q && j >= w.kfirst) ? -INFINITY : sacc[r];
+    }
+  }
+  float tmax = sacc[0];
+#pragma unroll
+  for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
+  tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+  const float m_new = fmaxf(w.m, tmax);
+  // (a query without a sink may have no visible key in a tile it shares with its neighbours' earlier blocks)
+  const float m_use = m_new == -INFINITY ? 0.f : m_new;
+  const float corr = __expf(w.m - m_use);
+  w.m = m_new;
+  float psum = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    sacc[r] = __expf(sacc[r] - m_use);
+    psum += sacc[r];
+  }
+  w.l = w.l * corr + psum;    // (the halves are added at the end)
+  if (__any(corr != 1.f)) {  // (wave-uniform)
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w.o[v][r] *= corr;
+  }
+  // O^T += V^T P^T, P = high bf16 part + bf16 remainder
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    float ph[8], pl[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      ph[e] = bf2f(f2bf(sacc[8 * c + e]));
+      pl[e] = sacc[8 * c + e] - ph[e];
+    }
+    const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, pack8(ph)), bo = __builtin_bit_cast(bf16x8_t, pack8(pl));
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const bf16x8_t vv = __builtin_bit_cast(bf16x8_t, values(c, v));
+      w.o[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, bh, w.o[v], 0, 0, 0);
+      w.o[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, bo, w.o[v], 0, 0, 0);
+    }
+  }
+}
+
+// a lane's columns of its query's output, times inv and the gates per column
+template <int VT>
+JLA_DEV void am_store(const AttnBias& p, const f32x16 (&o)[VT], size_t m, int h, int hi, float inv) {
+  const size_t at = m * p.ldo + (size_t)h * (32 * VT);
+  const float* gt = p.gate && p.gate_cols ? p.gate + m * p.ldg + (size_t)h * (32 * VT) : nullptr;
 #pragma unroll
   for (int v = 0; v < VT; ++v)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[v][r] = 0.f;
-  // (l_run holds this half-wave's part of the sum: the sink counts once, in the lower half)
-  float m_run = p.sink ? p.sink[vh] : -INFINITY, l_run = p.sink && hi == 0 ? 1.f : 0.f;
-  const int q_last = live ? min(q0 + AM_Q - 1, slot + p.S - 1) : -1;  // (no tile is walked without queries)
-  const float inv_cap = p.softcap > 0.f ? 1.f / p.softcap : 0.f;
-  const float hs = p.head_scale ? p.head_scale[vh] : 1.f;
-  // block-local mask: this query's first key, the last query's (the largest of the wave), and the tile the walk starts at
-  const int lo_q = ab_span(p, qi).lo, lo_last = ab_span(p, q_last).lo;
-  const int j_begin = ab_span(p, q0).lo / AM_K * AM_K;
-  // kept first keys (beside a window): their tiles [0, kf_end) come first, then the walk jumps to the window's tiles
-  const int kfirst = p.window > 0 ? p.keep_first : 0;
-  const int kf_end = min((kfirst + AM_K - 1) / AM_K * AM_K, j_begin);
-  auto next_tile = [&](int j0) { return j0 + AM_K == kf_end ? j_begin : j0 + AM_K; };
-  // the next tile's key and value fragments are loaded while the current tile is computed (one wave per SIMD at small
-  // batch: nothing else hides the loads)
-  u32x4 kn[DK], vn[2][VT];
-  auto fetch = [&](int j0) {
-    const bf16_t* kr = kbase + (size_t)min(j0 + krow, p.T - 1) * p.ldk + 8 * hi;
+    for (int r = 0; r < 16; r += 4) {  // rows (value columns) (r & 3) + 8 (r >> 2) + 4 hi: runs of four
+      const int c = 32 * v + 8 * (r >> 2) + 4 * hi;
+      float f[4];
 #pragma unroll
-    for (int kk = 0; kk < DK; ++kk) kn[kk] = *reinterpret_cast<const u32x4*>(kr + 16 * kk);
+      for (int k = 0; k < 4; ++k) f[k] = o[v][r + k] * inv * (gt ? hy_sigmoid(gt[c + k]) : 1.f);
+      if (p.out_bf16)
+        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.out) + at + c) = uint2{pack2bf(f[0], f[1]), pack2bf(f[2], f[3])};
+      else
+        *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + at + c) = float4{f[0], f[1], f[2], f[3]};
+    }
+}
+
+// head and block of query tiles of this workgroup (nq blocks per head). Workgroups go round the 8 XCDs by their id: where the heads
+// divide evenly, each XCD gets whole runs of neighbouring heads (which share their keys in grouped-query attention), so that a
+// head's keys and values pass through one L2. Long rows come first.
+JLA_DEV void am_place(const AttnBias& p, int nq, int& hb, int& blk) {
+  const int heads = p.H * p.B;
+  if (heads % 8 == 0) {
+    const int r = blockIdx.x >> 3, hl = r / nq;
+    hb = (int)(blockIdx.x & 7) * (heads >> 3) + hl;
+    blk = nq - 1 - (r - hl * nq);
+  } else {
+    hb = blockIdx.x / nq;
+    blk = nq - 1 - (blockIdx.x - hb * nq);
+  }
+}
+
+// the row of query tile s0 before its first key
+template <int DK, int VT>
+JLA_DEV void am_start(const AttnBias& p, AmRow<DK, VT>& w, int b, int vh, int maps, int s0, int slot, bool sunk) {
+  const int lane = threadIdx.x & 63, ql = lane & 31, hi = lane >> 5;
+  const int sq = min(s0 + ql, p.S - 1);  // (surplus lanes repeat the last query; never stored)
+  const float* q = p.q + (((size_t)b * p.S + sq) * (p.H * maps) + vh) * (16 * DK) + 8 * hi;
+#pragma unroll
+  for (int kk = 0; kk < DK; ++kk) {
+    float f[8];
+    hy_load8(q + 16 * kk, 8, f);
+    w.q[kk] = __builtin_bit_cast(bf16x8_t, pack8(f));
+  }
+#pragma unroll
+  for (int v = 0; v < VT; ++v)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) w.o[v][r] = 0.f;
+  w.m = sunk ? p.sink[vh] : -INFINITY;
+  w.l = sunk && hi == 0 ? 1.f : 0.f;  // (the sink counts once, in the lower half)
+  w.q0 = slot + s0;
+  w.qi = slot + sq;
+  w.vh = vh;
+  w.heads = p.H * maps;
+  w.scale = p.scale * (p.head_scale ? p.head_scale[vh] : 1.f);
+  w.inv_cap = p.softcap > 0.f ? 1.f / p.softcap : 0.f;
+  w.lo_q = ab_span(p, w.qi).lo;
+  w.lo_last = ab_span(p, min(w.q0 + AM_Q - 1, slot + p.S - 1)).lo;  // (the largest of the wave)
+  w.kfirst = p.window > 0 ? p.keep_first : 0;
+}
+
+// MAPS = 2 (differential heads): waves 2 t and 2 t + 1 of a workgroup run the two maps of query tile t; the second hands its
+// normalised output to the first through LDS, which subtracts, norms and stores.
+// KS = 4 (few queries): the four waves of a workgroup take one query tile and every fourth key tile each, joined through LDS; KS = 1: a
+// query tile per wave.
+// What bounds it: the vector unit, about 2.5 k cycles per tile of 32 x 32 (scores, their exponentials, the split weights) beside 24
+// matrix instructions, and the operand loads (below). So the tile has no branch and no wait per score: the options are taken for all
+// 16 at once, the accumulators are rescaled only where a maximum grew, and a tile's values are loaded behind its scores' products, the
+// next one's keys behind its softmax. Us before -> after, 16 heads of 128: 300 tokens, soft cap and bias, 38.8 -> 16.0; 777 tokens in
+// blocks of 1024 54.5 -> 27.9; 64 tokens behind 900 62 -> 21.
+template <int DK, int VT, int MAPS, int KS>  // dim = 16 DK, vdim = 32 VT
+__global__ void __launch_bounds__(256, DK <= 8 ? 2 : 1) attn_bias_mma_kernel(AttnBias p, const bf16_t* __restrict__ vt, int Tp) {
+  static_assert(MAPS == 1 || KS == 1, "differential heads: a map per wave");
+  constexpr int TILES = 4 / (MAPS * KS);  // query tiles per workgroup
+  constexpr int dim = 16 * DK, vdim = 32 * VT, PITCH = vdim + 4;
+  __shared__ float joined[MAPS == 2 ? TILES * VT * 16 * 64 : (KS > 1 ? KS * AM_Q * PITCH : 1)];
+  __shared__ float jm[KS > 1 ? KS : 1][AM_Q], jl[KS > 1 ? KS : 1][AM_Q];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int map = wave % MAPS;
+  const int ql = lane & 31, hi = lane >> 5;
+  const int nq = (p.S + TILES * AM_Q - 1) / (TILES * AM_Q);
+  int hb, blk;
+  am_place(p, nq, hb, blk);
+  const int s0 = (blk * TILES + (KS > 1 ? 0 : wave / MAPS)) * AM_Q;
+  const bool live = s0 < p.S;
+  if (MAPS == 1 && KS == 1 && !live) return;  // (a pair of waves without queries stays for the workgroup's barrier)
+  const int b = hb / p.H, h = hb - b * p.H;
+  const int g = h / (p.H / p.G), slot = *p.slot;
+  AmRow<DK, VT> w;
+  am_start<DK, VT>(p, w, b, h * MAPS + map, MAPS, s0, slot, p.sink && (KS == 1 || wave == 0));
+  const bf16_t* kbase = reinterpret_cast<const bf16_t*>(p.kc) + ((size_t)b * p.G + g) * p.T * p.ldk + map * dim + 8 * hi;
+  const bf16_t* vbase = vt + (((size_t)b * p.G + g) * vdim + ql) * Tp + 8 * hi;
+  const int krow = (ql & 0x13) | ((ql & 4) << 1) | ((ql & 8) >> 1);  // bits 2 and 3 swapped
+  const int q_last = live ? min(w.q0 + AM_Q - 1, slot + p.S - 1) : -1;
+  const int j_begin = ab_span(p, w.q0).lo / AM_K * AM_K;  // the tile that the walk starts at
+  // kept first keys (beside a window): their tiles come first, then the walk jumps to the window's tiles
+  const int kf_tiles = min((w.kfirst + AM_K - 1) / AM_K, j_begin / AM_K);
+  const int tiles = live ? kf_tiles + (q_last - j_begin) / AM_K + 1 : 0;  // (no tile is walked without queries)
+  auto tile_key = [&](int t) { return t < kf_tiles ? t * AM_K : j_begin + (t - kf_tiles) * AM_K; };
+  u32x4 kf[DK], vf[2][VT];
+  auto fetch_keys = [&](int t) {  // (past the last tile: it again, unused)
+    const bf16_t* kr = kbase + (size_t)min(tile_key(min(t, max(tiles, 1) - 1)) + krow, p.T - 1) * p.ldk;
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk) kf[kk] = *reinterpret_cast<const u32x4*>(kr + 16 * kk);
+  };
+  const int t_first = KS > 1 ? wave : 0;
+  fetch_keys(t_first);
+  for (int t = t_first; t < tiles; t += KS) {
+    const int j0 = tile_key(t);
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int v = 0; v < VT; ++v)
-        vn[c][v] = *reinterpret_cast<const u32x4*>(vbase + (size_t)(32 * v + ql) * Tp + min(j0, Tp - AM_K) + 16 * c + 8 * hi);
-  };
-  const int j_first = kf_end > 0 ? 0 : j_begin;
-  fetch(j_first);
-  for (int j0 = j_first; j0 <= q_last; j0 = next_tile(j0)) {
-    u32x4 kc_[DK], vc_[2][VT];
+        vf[c][v] = *reinterpret_cast<const u32x4*>(vbase + (size_t)(32 * v) * Tp + min(j0, Tp - AM_K) + 16 * c);
+    am_tile<DK, VT>(p, w, j0, [&](int kk) { return kf[kk]; }, [&](int c, int v) { return vf[c][v]; }, [&]() { fetch_keys(t + KS); });
+  }
+  float l_run = w.l;
+  const float m_run = w.m;
+  auto& o = w.o;
+  l_run += __shfl_xor(l_run, 32, 64);
+  if constexpr (KS > 1) {  // the waves' parts of the row; then 8 threads per query, 16 columns' worth of steps each
+    if (hi == 0) jm[wave][ql] = m_run;
+    __syncthreads();
+    float m_all = jm[0][ql];
 #pragma unroll
-    for (int kk = 0; kk < DK; ++kk) kc_[kk] = kn[kk];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int v = 0; v < VT; ++v) vc_[c][v] = vn[c][v];
-    fetch(next_tile(j0));  // (past the last tile: clamped addresses, never used)
-    // scores: rows = keys (fed permuted), columns = queries
-    f32x16 sacc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < DK; ++kk)
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kc_[kk]), qf[kk], sacc, 0, 0, 0);
-    // bias of this tile's 63 distances, one per lane: lane t holds distance q0 - j0 - 31 + t
-    float bl = 0.f;
-    const int dbase = q0 - j0 - (AM_K - 1);
-    const bool far = p.bias && dbase >= p.nbias - 1;
-    if (p.bias) bl = p.bias[(size_t)min(max(dbase + lane, 0), p.nbias - 1) * (p.H * MAPS) + vh];
-    // some (query, key) of the tile is masked
-    const bool diag = j0 + AM_K - 1 > q0 || (j0 < lo_last && j0 + AM_K - 1 >= kfirst);
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kl = 16 * (r >> 3) + 8 * hi + (r & 7);  // key of accumulator r within the tile
-      float sc = sacc[r] * p.scale * hs;
-      if (p.softcap > 0.f) sc = p.softcap * am_tanh(sc * inv_cap);
-      if (p.bias) sc += far ? bl : __shfl(bl, ql - kl + (AM_K - 1), 64);
-      if (diag && (j0 + kl > qi || (j0 + kl < lo_q && j0 + kl >= kfirst))) sc = -INFINITY;
-      sacc[r] = sc;
-      tmax = fmaxf(tmax, sc);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m_run, tmax);
-    // (a query without a sink may have no visible key in a tile it shares with its neighbours' earlier blocks)
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float corr = __expf(m_run - m_use);
-    m_run = m_new;
-    float psum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      sacc[r] = __expf(sacc[r] - m_use);
-      psum += sacc[r];
-    }
-    l_run = l_run * corr + psum;  // (this half-wave's keys; the halves are added at the end)
+    for (int w = 1; w < KS; ++w) m_all = fmaxf(m_all, jm[w][ql]);
+    const float wt = m_run == -INFINITY ? 0.f : __expf(m_run - m_all);  // (a wave without keys of this query: zeros)
+    if (hi == 0) jl[wave][ql] = l_run * wt;
+    float* mine = joined + ((size_t)wave * AM_Q + ql) * PITCH + 4 * hi;
 #pragma unroll
     for (int v = 0; v < VT; ++v)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[v][r] *= corr;
-    // O^T += V^T P^T, P = high bf16 part + bf16 remainder
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4*>(mine + 32 * v + 2 * r) =
+            float4{o[v][r] * wt, o[v][r + 1] * wt, o[v][r + 2] * wt, o[v][r + 3] * wt};
+    __syncthreads();
+    const int qt = threadIdx.x >> 3;
+    if (s0 + qt >= p.S) return;
+    float l = 0.f;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      float ph[8], pl[8];
+    for (int w = 0; w < KS; ++w) l += jl[w][qt];
+    const size_t m = (size_t)b * p.S + s0 + qt, at = m * p.ldo + (size_t)h * vdim;
+    float inv = 1.f / l;
+    if (p.gate && !p.gate_cols) inv *= ab_gate(p, m, h, 0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ph[e] = bf2f(f2bf(sacc[8 * c + e]));
-        pl[e] = sacc[8 * c + e] - ph[e];
+    for (int c = 4 * (threadIdx.x & 7); c < vdim; c += 32) {
+      float f[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < KS; ++w) {
+        const float4 x = *reinterpret_cast<const float4*>(joined + ((size_t)w * AM_Q + qt) * PITCH + c);
+        f[0] += x.x; f[1] += x.y; f[2] += x.z; f[3] += x.w;
       }
-      const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, pack8(ph)), bo = __builtin_bit_cast(bf16x8_t, pack8(pl));
 #pragma unroll
-      for (int v = 0; v < VT; ++v) {
-        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, vc_[c][v]);
-        o[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bh, o[v], 0, 0, 0);
-        o[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bo, o[v], 0, 0, 0);
-      }
+      for (int k = 0; k < 4; ++k) f[k] *= inv * (p.gate && p.gate_cols ? ab_gate(p, m, h, c + k) : 1.f);
+      if (p.out_bf16)
+        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.out) + at + c) = uint2{pack2bf(f[0], f[1]), pack2bf(f[2], f[3])};
+      else
+        *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + at + c) = float4{f[0], f[1], f[2], f[3]};
     }
+    return;
   }
-  l_run += __shfl_xor(l_run, 32, 64);
   const size_t m = (size_t)b * p.S + s0 + ql;
   float inv = 1.f / l_run;
   if constexpr (MAPS == 2) {
@@ -762,23 +872,107 @@ __global__ void __launch_bounds__(256) attn_bias_mma_kernel(AttnBias p, const bf
   }
   if (s0 + ql >= p.S) return;
   if (p.gate && !p.gate_cols) inv *= ab_gate(p, m, h, 0);
-  const size_t at = m * p.ldo + (size_t)h * vdim;
-  const float* gt = p.gate && p.gate_cols ? p.gate + m * p.ldg + (size_t)h * vdim : nullptr;
-#pragma unroll
-  for (int v = 0; v < VT; ++v)
-#pragma unroll
-    for (int r = 0; r < 16; r += 4) {  // rows (value columns) (r & 3) + 8 (r >> 2) + 4 hi: runs of four
-      const int c = 32 * v + 8 * (r >> 2) + 4 * hi;
-      float f[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) f[k] = o[v][r + k] * inv * (gt ? hy_sigmoid(gt[c + k]) : 1.f);
-      if (p.out_bf16)
-        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.out) + at + c) =
-            uint2{(uint32_t)f2bf(f[0]) | (uint32_t)f2bf(f[1]) << 16, (uint32_t)f2bf(f[2]) | (uint32_t)f2bf(f[3]) << 16};
-      else
-        *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.out) + at + c) = float4{f[0], f[1], f[2], f[3]};
-    }
+  am_store<VT>(p, o, m, h, hi, inv);
 }
+
+// Key widths of 64 and 128, more than a few queries: four waves with neighbouring query tiles of a head share its key tiles, 64 keys at a time, staged by LDS-DMA into one
+// of two buffers while the other is used. Straight from the caches (the kernel above) a wave's operand load touches 32 lines for 32
+// bytes each, which is what bounds it once every SIMD has waves: 512 line accesses per tile and wave; staged, a line is fetched once
+// per workgroup. Images: key rows of 16 DK numbers, chunk c (16 bytes) of row r at c ^ swizzle(r), value rows (64 keys) likewise.
+constexpr int AL_KEYS = 64;
+template <int DK, int VT, int KS>
+__global__ void __launch_bounds__(256 * KS, 2) attn_bias_lds_kernel(AttnBias p, const bf16_t* __restrict__ vt, int Tp) {
+  static_assert(DK == 4 || DK == 8, "power-of-two key rows");
+  constexpr int dim = 16 * DK, vdim = 32 * VT;
+  constexpr int KC = 2 * DK, KU = AL_KEYS * KC, VU = vdim * 8, STAGE = KU + VU;  // 16-byte chunks: of a key row, of the images
+  constexpr int PARTS = KS == 2 ? 4 * VT * 16 * 64 / 4 : 0;  // (16-byte units)
+  __shared__ u32x4 lds[2 * STAGE > PARTS ? 2 * STAGE : PARTS];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ql = lane & 31, hi = lane >> 5;
+  const int nq = (p.S + 4 * AM_Q - 1) / (4 * AM_Q);
+  int hb, blk;
+  am_place(p, nq, hb, blk);
+  const int s_first = blk * 4 * AM_Q, s0 = s_first + (wave & 3) * AM_Q;
+  const int b = hb / p.H, h = hb - b * p.H;
+  const int g = h / (p.H / p.G), slot = *p.slot;
+  AmRow<DK, VT> w;
+  am_start<DK, VT>(p, w, b, h, 1, min(s0, p.S - 1), slot, p.sink && wave < 4);  // (a wave without queries walks along)
+  const bf16_t* kbase = reinterpret_cast<const bf16_t*>(p.kc) + ((size_t)b * p.G + g) * p.T * p.ldk;
+  const bf16_t* vbase = vt + ((size_t)b * p.G + g) * vdim * Tp;
+  const int q_last = min(w.q0 + AM_Q - 1, slot + p.S - 1), q_end = min(slot + s_first + 4 * AM_Q, slot + p.S) - 1;
+  const int lo_own = ab_span(p, w.q0).lo;
+  const int j_begin = ab_span(p, slot + s_first).lo / AL_KEYS * AL_KEYS;
+  const int kf_steps = min((w.kfirst + AL_KEYS - 1) / AL_KEYS, j_begin / AL_KEYS);
+  const int steps = kf_steps + (q_end - j_begin) / AL_KEYS + 1;
+  auto step_key = [&](int t) { return t < kf_steps ? t * AL_KEYS : j_begin + (t - kf_steps) * AL_KEYS; };
+  // chunk position of chunk c in row r: the 16 rows of a fragment's half fall on all banks
+  auto kpos = [](int r, int c) { return DK == 8 ? c ^ (r & 15) : c ^ ((r >> 1) & 7); };
+  auto vpos = [](int r, int c) { return c ^ ((r >> 1) & 7); };
+  auto stage = [&](int t) {
+    const int j0 = step_key(t);
+    u32x4* const buf = lds + (t & 1) * STAGE;
+#pragma unroll
+    for (int i = 0; i < KU / (256 * KS); ++i) {
+      const int first = 64 * (4 * KS * i + wave), at = first + lane, r = at / KC, c = kpos(r, at % KC);  // (the swizzle is its own inverse)
+      glds16_asm(kbase + (size_t)min(j0 + r, p.T - 1) * p.ldk + 8 * c, buf + first);
+    }
+#pragma unroll
+    for (int i = 0; i < VU / (256 * KS); ++i) {
+      const int first = 64 * (4 * KS * i + wave), at = first + lane, r = at / 8, c = vpos(r, at % 8);
+      glds16_asm(vbase + (size_t)r * Tp + min(j0 + 8 * c, Tp - 8), buf + KU + first);
+    }
+  };
+  const int krow = (ql & 0x13) | ((ql & 4) << 1) | ((ql & 8) >> 1);  // bits 2 and 3 swapped
+  stage(0);
+  for (int t = 0; t < steps; ++t) {
+    wait_vmcnt<0>();  // this wave's part of step t has landed; then every wave's has, and step t - 1 is read
+    __syncthreads();
+    if (t + 1 < steps) stage(t + 1);
+    const u32x4* const buf = lds + (t & 1) * STAGE;
+#pragma unroll 1
+    for (int half = KS == 2 ? wave >> 2 : 0; half < (KS == 2 ? (wave >> 2) + 1 : 2); ++half) {
+      const int j0 = step_key(t) + AM_K * half;
+      if (s0 >= p.S || j0 > q_last || (j0 + AM_K <= lo_own && j0 >= w.kfirst)) continue;  // (wave-uniform: nothing to see)
+      const int kr = AM_K * half + krow;
+      am_tile<DK, VT>(
+          p, w, j0, [&](int kk) { return buf[kr * KC + kpos(kr, 2 * kk + hi)]; },
+          [&](int c, int v) { return buf[KU + (32 * v + ql) * 8 + vpos(32 * v + ql, 4 * half + 2 * c + hi)]; }, []() {});
+    }
+  }
+  float l = w.l + __shfl_xor(w.l, 32, 64);
+  if constexpr (KS == 2) {  // the waves of the second halves hand their part over, through the images' memory
+    __shared__ float jm[4][AM_Q], jl[4][AM_Q];
+    float* const part = reinterpret_cast<float*>(lds) + (size_t)(wave & 3) * VT * 16 * 64 + lane;
+    __syncthreads();
+    if (wave >= 4) {
+      if (hi == 0) jm[wave & 3][ql] = w.m, jl[wave & 3][ql] = l;
+#pragma unroll
+      for (int v = 0; v < VT; ++v)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[(v * 16 + r) * 64] = w.o[v][r];
+    }
+    __syncthreads();
+    if (wave >= 4) return;
+    const float m2 = jm[wave][ql], m_all = fmaxf(w.m, m2);
+    const float w1 = w.m == -INFINITY ? 0.f : __expf(w.m - m_all), w2 = m2 == -INFINITY ? 0.f : __expf(m2 - m_all);
+    l = l * w1 + jl[wave][ql] * w2;
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w.o[v][r] = w.o[v][r] * w1 + part[(v * 16 + r) * 64] * w2;
+  }
+  if (s0 + ql >= p.S) return;
+  const size_t m = (size_t)b * p.S + s0 + ql;
+  float inv = 1.f / l;
+  if (p.gate && !p.gate_cols) inv *= ab_gate(p, m, h, 0);
+  am_store<VT>(p, w.o, m, h, hi, inv);
+}
+
+// Query tiles up to which they share the chip by their keys: four ways (measured us, four ways / two ways / one: 400 tiles 28 / 33 / 37,
+// 768 tiles 38 / 29 / 30, 1024 tiles 105 / 91 / 119), then two ways (2048 tiles 115 / 95 / 92, 4096 tiles 254 / 165 / 165,
+// 6032 tiles 305 / 238 / 203). Key widths that are not staged (measured on heads of 128
+// without the staging, four ways / one): 105 / 135 at 1024 tiles, 254 / 236 at 4096.
+constexpr long long AM_SPLIT4 = 512, AM_SPLIT2 = 1536, AM_SPLIT4_DIRECT = 1024;
 
 template <int DK, int VT>
 static int am_launch(const AttnBias& p, bf16_t* vt, int Tp, hipStream_t s) {
@@ -786,8 +980,14 @@ static int am_launch(const AttnBias& p, bf16_t* vt, int Tp, hipStream_t s) {
                                                                      p.S, p.T, Tp, p.vdim);
   JLA_CHECK_LAUNCH();
   const long long hb = (long long)p.H * p.B;
-  if (p.maps == 2) attn_bias_mma_kernel<DK, VT, 2><<<(unsigned)((p.S + 63) / 64 * hb), 256, 0, s>>>(p, vt, Tp);
-  else attn_bias_mma_kernel<DK, VT, 1><<<(unsigned)((p.S + 127) / 128 * hb), 256, 0, s>>>(p, vt, Tp);
+  const long long tiles = (p.S + AM_Q - 1) / AM_Q * hb;
+  constexpr bool staged = DK == 4 || DK == 8;
+  const unsigned g4 = (unsigned)((p.S + 4 * AM_Q - 1) / (4 * AM_Q) * hb);
+  if (p.maps == 2) attn_bias_mma_kernel<DK, VT, 2, 1><<<(unsigned)((p.S + 63) / 64 * hb), 256, 0, s>>>(p, vt, Tp);
+  else if (tiles <= (staged ? AM_SPLIT4 : AM_SPLIT4_DIRECT)) attn_bias_mma_kernel<DK, VT, 1, 4><<<(unsigned)tiles, 256, 0, s>>>(p, vt, Tp);
+  else if constexpr (!staged) attn_bias_mma_kernel<DK, VT, 1, 1><<<g4, 256, 0, s>>>(p, vt, Tp);
+  else if (tiles <= AM_SPLIT2) attn_bias_lds_kernel<DK, VT, 2><<<g4, 512, 0, s>>>(p, vt, Tp);
+  else attn_bias_lds_kernel<DK, VT, 1><<<g4, 256, 0, s>>>(p, vt, Tp);
   JLA_CHECK_LAUNCH();
   return 0;
 }
