@@ -1,8 +1,7 @@
 // The fp32 form of a prompt's row-gathered, expert-grouped linears: split products on the bf16 matrix cores
 // (kernels/gemm_f32x3.h) with the epilogues of a row linear. Us, exact-f32 MFMA tiles (lr_gemm_kernel) -> here, rows x K x N:
-// 9 x 2048 x 8224 89 -> 31; 200 x 2048 x 8224 145 -> 71; 400 x 5632 x 2048 358 -> 77; 400 x 2048 x 5632 gated 248 -> 165; 4000 x
-// 5632 x 2048 824 -> 478 (193 TFLOP/s). Relative error against 64 bits, 400 x 5632 x 2048: 1.34e-6 -> 4.1e-7, of positive
-// numbers 1.13e-6 -> 1.2e-7 (K split).
+// 16 x 2048 x 8224 89 -> 24; 400 x 5632 x 2048 358 -> 68; 400 x 2048 x 5632 gated 248 -> 138. Relative error against 64 bits,
+// 400 x 5632 x 2048: 1.34e-6 -> 1.4e-7 (K split).
 #include "../kernels/gemm_f32x3.h"
 #include "hy_util.h"
 #include "hybrid.h"
@@ -10,10 +9,10 @@
 
 namespace jla {
 
-template <int BM, int GATED>
-__global__ void __launch_bounds__(256, 2) rows_f32x3_kernel(F3Rows p, RowLinear act, int tiles_n) {
-  __shared__ u32x4 lds[f3_lds<BM>()];
-  f3_tile<BM, GATED>(p, tiles_n, 0, (p.K + F3_BK - 1) / F3_BK, lds, [&](const f32x4 g, const f32x4 u) {
+template <int MT, int GATED, bool SCALED>
+__global__ void __launch_bounds__(64 * MT, 2) rows_f32x3_kernel(F3Rows p, RowLinear act, int tiles_n) {
+  __shared__ u32x4 lds[f3_lds<MT>()];
+  f3_tile<MT, MT, GATED, SCALED>(p, tiles_n, 0, (p.K + F3_BK - 1) / F3_BK, lds, [&](const f32x4 g, const f32x4 u) {
     f32x4 v = g;
     if (act.act != HY_ACT_NONE) {
 #pragma unroll
@@ -24,12 +23,12 @@ __global__ void __launch_bounds__(256, 2) rows_f32x3_kernel(F3Rows p, RowLinear 
 }
 
 // K over gridDim.y workgroups per tile: partial sums of every weight row (gate and up side by side) into their slabs
-template <int BM>
-__global__ void __launch_bounds__(256, 2) rows_f32x3_split_kernel(F3Rows p, int tiles_n, int steps) {
-  __shared__ u32x4 lds[f3_lds<BM>()];
+template <int MT, bool SCALED>
+__global__ void __launch_bounds__(64 * MT, 2) rows_f32x3_split_kernel(F3Rows p, int tiles_n, int steps) {
+  __shared__ u32x4 lds[f3_lds<MT>()];
   const int t0 = blockIdx.y * steps;
   p.out += (size_t)blockIdx.y * p.R * p.ldo;
-  f3_tile<BM, 0>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
+  f3_tile<MT, MT, 0, SCALED>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
                  [](const f32x4 g, const f32x4) { return g; });
 }
 
@@ -70,9 +69,8 @@ bool hy_rows_f32_takes(const RowLinear& p) {
 
 static F3Plan rows_f32_plan(const RowLinear& p) {
   const int E = p.offs ? p.E : 1;
-  const long long tn = ((hy_act_gated(p.act) ? 2LL : 1LL) * p.N + F3_BN - 1) / F3_BN;
   auto tiles = [&](int bm) { return E == 1 ? (p.R + bm - 1LL) / bm : (p.R + bm / 2LL * E) / bm; };  // (on average)
-  return f3_plan(tiles(128), tiles(64), tn, p.K);
+  return f3_plan(tiles, p.R, (hy_act_gated(p.act) ? 2LL : 1LL) * p.N, p.K);
 }
 
 long long hy_rows_f32_floats(const RowLinear& p) {
@@ -85,7 +83,7 @@ int hy_rows_f32(const RowLinear& p, float* ws, hipStream_t s) {
   const F3Plan pl = rows_f32_plan(p);
   F3Rows f{reinterpret_cast<const float*>(p.a), p.lda, p.a_idx, p.a_scale, reinterpret_cast<const float*>(p.w),
            p.w_stride, p.N, p.K, reinterpret_cast<float*>(p.out), p.ldo, p.dst_idx, p.add_out, p.offs, p.E, p.R};
-  const long long tn = ((gated ? 2LL : 1LL) * p.N + F3_BN - 1) / F3_BN;
+  const long long tn = ((gated ? 2LL : 1LL) * p.N + pl.bn - 1) / pl.bn;
   const long long grid = ((p.R / pl.bm + (long long)E) * tn + 7) / 8 * 8;
   if (grid > 0x7fffffffLL) return -4;
   if (pl.splits > 1) {
@@ -95,21 +93,32 @@ int hy_rows_f32(const RowLinear& p, float* ws, hipStream_t s) {
     f.dst_idx = nullptr;
     f.add = 0;
     const dim3 g((unsigned)grid, pl.splits);
-    if (pl.bm == 64) rows_f32x3_split_kernel<64><<<g, 256, 0, s>>>(f, (int)tn, pl.steps);
-    else rows_f32x3_split_kernel<128><<<g, 256, 0, s>>>(f, (int)tn, pl.steps);
+#define RF_SPLIT(MT, SC) rows_f32x3_split_kernel<MT, SC><<<g, 64 * MT, 0, s>>>(f, (int)tn, pl.steps)
+    if (pl.bm == 64) {
+      if (f.a_scale) RF_SPLIT(4, true);
+      else RF_SPLIT(4, false);
+    } else {
+      if (f.a_scale) RF_SPLIT(8, true);
+      else RF_SPLIT(8, false);
+    }
+#undef RF_SPLIT
     JLA_CHECK_LAUNCH();
     const long long n = (long long)p.R * (p.N / 4);
     rows_f32_sum_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(p, ws, pl.splits, gated);
     JLA_CHECK_LAUNCH();
     return 0;
   }
-#define RF_RUN(BM, G) rows_f32x3_kernel<BM, G><<<(unsigned)grid, 256, 0, s>>>(f, p, (int)tn)
+#define RF_RUN(MT, G)                                                                                     \
+  do {                                                                                                    \
+    if (f.a_scale) rows_f32x3_kernel<MT, G, true><<<(unsigned)grid, 64 * MT, 0, s>>>(f, p, (int)tn);       \
+    else rows_f32x3_kernel<MT, G, false><<<(unsigned)grid, 64 * MT, 0, s>>>(f, p, (int)tn);                \
+  } while (0)
   if (pl.bm == 64) {
-    if (gated) RF_RUN(64, 1);
-    else RF_RUN(64, 0);
+    if (gated) RF_RUN(4, 1);
+    else RF_RUN(4, 0);
   } else {
-    if (gated) RF_RUN(128, 1);
-    else RF_RUN(128, 0);
+    if (gated) RF_RUN(8, 1);
+    else RF_RUN(8, 0);
   }
 #undef RF_RUN
   JLA_CHECK_LAUNCH();

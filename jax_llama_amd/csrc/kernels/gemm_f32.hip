@@ -2,8 +2,8 @@
 // `precision`, jax_test.py:433 runs the parity harness with precision='highest').
 //
 // y[M, N] = x[M, K] @ W[N, K]^T with fp32 inputs, fp32 accumulation and fp32 output. Rows of whole 16-byte pieces run as
-// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 163, 100 567 -> 209,
-// 600 1780 -> 925, 6000 15484 -> 8211); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
+// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 163,
+// 128 567 -> 196, 600 1780 -> 856, 1500 2162 (with 128 x 128 tiles) -> 1890); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
 // k-ordered fmaf chain, no xf32 shortcut on gfx950): 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64
 // (2 x 2 MFMA tiles), K staged 32 deep through LDS in k-major images ([k][row]) so a lane's fragment element (row l & 31, k
 // l >> 5) is one conflict-free ds_read_b32.
@@ -95,12 +95,12 @@ __global__ void __launch_bounds__(GF_THREADS)
     }
 }
 
-template <int BM>
-__global__ void __launch_bounds__(256, 2) gemm_f32x3_kernel(F3Rows p, int tiles_n, int steps) {
-  __shared__ u32x4 lds[f3_lds<BM>()];
+template <int MT>  // (MT waves)
+__global__ void __launch_bounds__(64 * MT, 2) gemm_f32x3_kernel(F3Rows p, int tiles_n, int steps) {
+  __shared__ u32x4 lds[f3_lds<MT>()];
   const int t0 = blockIdx.y * steps;
   p.out += (size_t)blockIdx.y * p.R * p.ldo;
-  f3_tile<BM, 0>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
+  f3_tile<MT, MT, 0, false>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
                  [](const f32x4 g, const f32x4) { return g; });
 }
 
@@ -116,7 +116,7 @@ static bool f32x3_takes(const float* x, const float* w, const float* y, int M, i
   return M > 0 && N > 0 && K > 0 && K % 8 == 0 && N % 4 == 0 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0;
 }
 static F3Plan f32x3_plan(int M, int N, int K) {
-  return f3_plan((M + 127) / 128, (M + 63) / 64, (N + F3_BN - 1) / F3_BN, K);
+  return f3_plan([&](int bm) { return (long long)(M + bm - 1) / bm; }, M, N, K);
 }
 
 long long gemm_f32_workspace(const float* x, const float* w, const float* y, int M, int N, int K) {
@@ -131,11 +131,11 @@ int gemm_f32(const float* x, const float* w, float* y, int M, int N, int K, floa
     const F3Plan pl = f32x3_plan(M, N, K);
     if (pl.splits > 1 && (!ws || ((uintptr_t)ws & 15))) return -3;
     const F3Rows p{x, K, nullptr, nullptr, w, (long long)N * K, N, K, pl.splits > 1 ? ws : y, N, nullptr, 0, nullptr, 1, M};
-    const long long tn = (N + F3_BN - 1) / F3_BN, tiles = ((M + pl.bm - 1) / pl.bm * tn + 7) / 8 * 8;
+    const long long tn = (N + pl.bn - 1) / pl.bn, tiles = ((M + pl.bm - 1) / pl.bm * tn + 7) / 8 * 8;
     if (tiles > 0x7fffffffLL) return -2;
     const dim3 grid((unsigned)tiles, pl.splits);
-    if (pl.bm == 64) gemm_f32x3_kernel<64><<<grid, 256, 0, s>>>(p, (int)tn, pl.steps);
-    else gemm_f32x3_kernel<128><<<grid, 256, 0, s>>>(p, (int)tn, pl.steps);
+    if (pl.bm == 64) gemm_f32x3_kernel<4><<<grid, 256, 0, s>>>(p, (int)tn, pl.steps);
+    else gemm_f32x3_kernel<8><<<grid, 512, 0, s>>>(p, (int)tn, pl.steps);
     JLA_CHECK_LAUNCH();
     if (pl.splits > 1) {
       const size_t n = (size_t)M * N / 4;

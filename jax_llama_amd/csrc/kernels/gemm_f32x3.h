@@ -2,24 +2,29 @@
 // before it leave (8 bits each, so the split is exact), and a product is the six largest of the nine partial products, smallest
 // first,
 //     a w = lo hi + hi lo + mid mid + mid hi + hi mid + hi hi,
-// in one fp32 accumulator. |mid| is below 2^-8 and |lo| below 2^-17 of the operand, so what is left out (mid lo, lo mid, lo lo)
+// in fp32, the sum of a step of 32 from zero and then into the running sum. |mid| is below 2^-8 and |lo| below 2^-17 of the operand, so what is left out (mid lo, lo mid, lo lo)
 // is below 2^-24 of the product, half an fp32 rounding, and of either sign: parts that are cut instead of rounded all have the
 // operand's sign, and a sum of products of one sign comes out low (1 x 32000 x 4096, positive numbers, error against 64 bits:
 // exact-f32 MFMA 9.9e-7, cut parts 3.2e-6, all of it one-sided, nearest parts 3.2e-7). v_mfma_f32_16x16x32_bf16 adds 8
-// products at a time to the accumulator, rounded to nearest: 24 roundings per 32 products here, 5 of 6 of them of a small
-// addend, where the fp32 matrix instruction rounds once per product (600 x 4000 x 4096, either sign: 1.14e-6 -> 0.57e-6; 70 x
-// 512 x 8: 5.3e-8 -> 3.1e-8). It does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle, so six of them are 2.7 times
+// products at a time to the accumulator, rounded to nearest: 24 roundings per 32 products, of the step's sum, and one of the running
+// sum, where the fp32 matrix instruction rounds the running sum once per product (70 x 512 x 8: 5.3e-8 -> 3.1e-8). It does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle, so six of them are 2.7 times
 // its rate.
 //
-// One workgroup: BM x 128 outputs, four waves of BM / 2 x 64; K advances 32 per step. The operands are split on their way
-// from registers to LDS (6 vector instructions per number, beside the products of the step before), so memory holds plain
-// fp32 and nothing is prepared ahead; loads are two steps ahead. LDS: per operand and part [rows][4 cells of
-// 16 B], cell c of row r at c ^ ((r >> 2) & 3): the 16 lanes of a fragment read fall on all 64 banks.
-// Where the split does not hold, the workgroup computes its tile again on the fp32 matrix instruction (600 x 4000 x 4096 with
-// a NaN in every tile: 138 -> 285 us). An infinity or NaN among the operands, or a number that rounds up to an infinity,
-// makes its remainder NaN and so every result it enters (a sum past the largest number shows there too); a piece of a row
-// whose numbers are all below 2^-95 would have parts that bf16's smallest step of 2^-133 cuts.
+// One workgroup: 128 x 256 outputs in eight waves (two per SIMD) or 64 x 128 in four; a wave has all rows and 32 columns. K advances
+// 32 per step. The operands are split on their way (6 vector instructions per number), so memory holds plain fp32 and nothing is
+// prepared ahead: the activations through LDS, in two images, a wave's own weights straight into the layout of the matrix
+// instruction. LDS: per part [rows][4 cells of 16 B], cell c of row r at c ^ (r & 8 ? 3 : 0): a read of 16 bytes per lane takes lanes
+// 0-3, 12-15, 20-23, 24-27 together (then 4-11, 16-19, 28-31, and so above 32), which fall on all 64 banks (c ^ ((r >> 2) & 3): half of
+// the reads' cycles were conflicts).
+// What bounds it: the matrix cores at 70 % of their cycles and a clock held at 1.95 GHz by power. Each product is followed by the few
+// vector instructions that fit beside it, the one barrier of a step lies where the next products' operands are on their way, and a
+// step's six products start from zero, so that the running sums are rounded once per step and not 24 times (4 vector additions per
+// tile, 5 % of the time; relative error of normal numbers, K 4096 in one chain 1.0e-6 -> 2.2e-7, K 2048 7.0e-7 -> 1.6e-7). Before,
+// 128 x 128 outputs in four waves, both operands through LDS, splits and products in turn: us of the product of M x N x K, before ->
+// here, 600 x 32000 x 4096 935 -> 856, 1500 2162 -> 1890, 128 248 -> 196, 400 x 14600 x 2048 172 -> 150, 200 x 11264 x 2048 91 -> 77, 64 x
+// 2048 x 2048 19 -> 16. Both operands through LDS in this order: 5 % slower.
 #pragma once
+#include <type_traits>
 #include "common.h"
 #include "row_tiles.h"
 
@@ -41,8 +46,7 @@ struct F3Rows {
   int E, R;
 };
 
-constexpr int F3_BN = 128, F3_BK = 32;
-constexpr int F3_RESIDENT = 512;  // workgroups resident at once: two per compute unit
+constexpr int F3_BK = 32;
 
 constexpr unsigned F3_EXP = 0x70000000u;  // set in some number of a row piece unless all of them are below 2^-95
 
@@ -65,218 +69,213 @@ JLA_DEV F3Part f3_split(const f32x4 x, const f32x4 y, unsigned& any) {
   return p;
 }
 
+using F3Global = __attribute__((address_space(1))) f32x4;
+// (what a row piece past the tile's last number reads)
+__device__ const f32x4 f3_zeros[2] = {};
+
 // K steps [t0, t1). act(gate accumulators, up accumulators) -> outputs of 4 neighbouring columns
-template <int BM, int GATED, class Act>
+template <int MT, int WV, int GATED, bool SCALED, class Act>
 JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, const Act& act) {
-  constexpr int MT = BM / 32;                       // 16-row tiles of a wave
-  constexpr int NA = BM * 4 / 256, NW = F3_BN * 4 / 256;  // 8-number pieces per thread and step
-  constexpr int AU = BM * 4, WU = F3_BN * 4;        // u32x4 of one part
-  constexpr int F3_BUF = 3 * (AU + WU);             // ... of one staged step
+  constexpr int BM = 16 * MT, BN = 32 * WV;
+  static_assert(BM == 16 * WV && MT % 4 == 0, "a row piece per thread and step");
+  constexpr int AU = BM * 4;  // u32x4 of one part of the staged rows
+  constexpr int BUF = 3 * AU;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 1, wc = wave & 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int e = 0, r0 = 0, rend = 0, tn = 0;
   if (!row_tile<BM>(p.offs, p.E, p.R, tiles_n, lane, e, r0, rend, tn)) return;
   const int K = p.K, N = p.N;
-  constexpr int COLS = GATED ? F3_BN / 2 : F3_BN;
+  constexpr int COLS = GATED ? BN / 2 : BN;
   const int n0 = tn * COLS;
   const float* const wbase = p.w + (size_t)e * p.w_stride;
-  // row x of the weight tile: 16 gate rows and 16 up rows in turn for a gated product
-  auto wrow = [&](int x) {
-    const int jt = x >> 4, col = min(n0 + (GATED ? 16 * (jt >> 1) + (x & 15) : x), N - 1);
-    return wbase + (size_t)(GATED && (jt & 1) ? N + col : col) * K;
+  // weight row of lane c, column tile j of this wave: 16 gate rows and 16 up rows for a gated product
+  auto wrow = [&](int j) {
+    const int col = min(GATED ? n0 + 16 * wave + c : n0 + 32 * wave + 16 * j + c, N - 1);
+    return wbase + (size_t)(GATED && j ? N + col : col) * K;
   };
   auto arow = [&](int x) {
     const int row = min(r0 + x, rend - 1);  // (rows past the end repeat the last one)
     return p.a + (size_t)(p.a_idx ? p.a_idx[row] : row) * p.lda;
   };
-  auto ascale = [&](int x) { return p.a_scale ? p.a_scale[min(r0 + x, rend - 1)] : 1.f; };
-  const int sch = tid & 3, srow = tid >> 2;  // staging: piece u is k-chunk sch of row 64 u + srow
-  const float* pa[NA];
-  float sc[NA];
-  const float* pw[NW];
-#pragma unroll
-  for (int u = 0; u < NA; ++u) {
-    pa[u] = arow(64 * u + srow) + 8 * sch;
-    sc[u] = ascale(64 * u + srow);
-  }
-#pragma unroll
-  for (int u = 0; u < NW; ++u) pw[u] = wrow(64 * u + srow) + 8 * sch;
+  auto ascale = [&](int x) { return SCALED ? p.a_scale[min(r0 + x, rend - 1)] : 1.f; };
+  // pieces of 8 numbers: one of the activations (k-chunk sch of row srow, for all waves), two of this wave's own weights (k-chunk q)
+  const int sch = tid & 3, srow = tid >> 2;
+  const float* const src[3] = {arow(srow) + 8 * sch, wrow(0) + 8 * q, wrow(1) + 8 * q};
+  const float sc = ascale(srow);
+  const int kend = min(K, F3_BK * t1);
 
-  f32x4 acc[4][MT];
+  f32x4 acc[2][MT];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4* const la = lds;
-  u32x4* const lw = lds + 3 * AU;
-  const int cell = sch ^ ((srow >> 2) & 3);  // (64 u does not change it)
-  const int rcell = q ^ ((c >> 2) & 3);
-  unsigned ta[NA], tw[NW];  // bits of this thread's row pieces
-#pragma unroll
-  for (int u = 0; u < NA; ++u) ta[u] = 0;
-#pragma unroll
-  for (int u = 0; u < NW; ++u) tw[u] = 0;
-  struct Step {
-    f32x4 a[NA][2], w[NW][2];
-  };
-  auto fetch = [&](Step& f, int t) {  // step t on its way to registers
+  u32x4* const st = lds + srow * 4 + (sch ^ (srow & 8 ? 3 : 0));
+  const u32x4* const ra = lds + c * 4 + (q ^ (c & 8 ? 3 : 0));
+  unsigned bits[3] = {0, 0, 0};  // bits of this thread's row pieces
+  f32x4 f[3][2];                 // a step on its way
+  auto fetch = [&](int t, int n) {
     const int k0 = F3_BK * t;
-    const bool in = k0 + 8 * sch < K;  // (K is a multiple of 8)
-    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < NA; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) f.a[u][h] = in ? *reinterpret_cast<const f32x4*>(pa[u] + k0 + 4 * h) : z;
-#pragma unroll
-    for (int u = 0; u < NW; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) f.w[u][h] = in ? *reinterpret_cast<const f32x4*>(pw[u] + k0 + 4 * h) : z;
+    const float* from = k0 + 8 * (n ? q : sch) < kend ? src[n] + k0 : reinterpret_cast<const float*>(f3_zeros);  // (K: a multiple of 8)
+    const F3Global* at = reinterpret_cast<const F3Global*>(reinterpret_cast<uintptr_t>(from));
+    f[n][0] = at[0];
+    f[n][1] = at[1];
   };
-  auto stage = [&](const Step& f, int buf) {  // split and into LDS
-#pragma unroll
-    for (int u = 0; u < NA; ++u) {
-      const F3Part s = f3_split(f.a[u][0] * sc[u], f.a[u][1] * sc[u], ta[u]);
-      u32x4* d = la + buf * F3_BUF + (64 * u + srow) * 4 + cell;
-      d[0] = s.hi;
-      d[AU] = s.mid;
-      d[2 * AU] = s.lo;
-    }
-#pragma unroll
-    for (int u = 0; u < NW; ++u) {
-      const F3Part s = f3_split(f.w[u][0], f.w[u][1], tw[u]);
-      u32x4* d = lw + buf * F3_BUF + (64 * u + srow) * 4 + cell;
-      d[0] = s.hi;
-      d[WU] = s.mid;
-      d[2 * WU] = s.lo;
-    }
+  auto stage = [&](int buf) {  // the activations split and into LDS
+    const F3Part s = SCALED ? f3_split(f[0][0] * sc, f[0][1] * sc, bits[0]) : f3_split(f[0][0], f[0][1], bits[0]);
+    u32x4* d = st + buf * BUF;
+    d[0] = s.hi;
+    d[AU] = s.mid;
+    d[2 * AU] = s.lo;
   };
-  auto products = [&](int buf) {
-    u32x4 w[3][4];
-#pragma unroll
-    for (int x = 0; x < 3; ++x)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[x][j] = lw[buf * F3_BUF + x * WU + (64 * wc + 16 * j + c) * 4 + rcell];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      u32x4 a[3];
-#pragma unroll
-      for (int x = 0; x < 3; ++x) a[x] = la[buf * F3_BUF + x * AU + (wr * (BM / 2) + 16 * i + c) * 4 + rcell];
-      constexpr int PW[6] = {2, 0, 1, 1, 0, 0}, PA[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-      for (int x = 0; x < 6; ++x)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j][i] = mfma16x16x32(w[PW[x]][j], a[PA[x]], acc[j][i]);
-    }
+  u32x4 w[2][2][3], a[4][3];  // two steps' weights; four row tiles, two of them on their way
+  auto weights = [&](int set, int j) {
+    const F3Part s = f3_split(f[1 + j][0], f[1 + j][1], bits[1 + j]);
+    w[set][j][0] = s.hi;
+    w[set][j][1] = s.mid;
+    w[set][j][2] = s.lo;
   };
-  Step f0, f1;  // two steps on their way
-  fetch(f0, t0);
-  if (t0 + 1 < t1) fetch(f1, t0 + 1);
-  if constexpr (BM == 64) {  // two steps in LDS: one barrier per step, a step's products beside the split of the next
-    stage(f0, 0);
-    if (t0 + 2 < t1) fetch(f0, t0 + 2);
-    __syncthreads();
-    for (int t = t0; t < t1; t += 2) {
-      products(0);
-      if (t + 1 < t1) {
-        stage(f1, 1);
-        if (t + 3 < t1) fetch(f1, t + 3);
+  auto read = [&](int buf, int i) {
+#pragma unroll
+    for (int x = 0; x < 3; ++x) a[i & 3][x] = ra[buf * BUF + x * AU + i * 64];
+  };
+  auto products = [&](int set, int i) {
+    constexpr int PW[6] = {2, 0, 1, 1, 0, 0}, PA[6] = {0, 2, 1, 0, 1, 0};
+    f32x4 sum[2] = {};  // (of the step: the running sums are rounded once per step)
+#pragma unroll
+    for (int x = 0; x < 6; ++x)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) sum[j] = mfma16x16x32(w[set][j][PW[x]], a[i & 3][PA[x]], sum[j]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[j][i][r] += sum[j][r];
+  };
+  // Round u of parity P reads step u's image, writes step u + 1's and multiplies the last two row tiles of step u - 1 (not in the
+  // first round) and all but the last two of step u: the one barrier at its end finds every read of the image behind it and none of
+  // the operands that the next products need.
+  auto round = [&](auto first, auto parity, int u) {
+    constexpr int P = parity.value;
+#pragma unroll
+    for (int jj = 0; jj < MT; ++jj) {
+      const int i = (MT - 2 + jj) % MT;
+      read(P, (i + 2) % MT);
+      if (jj == 0) {
+        stage(P ^ 1);
+        fetch(u + 2, 0);
       }
-      __syncthreads();
-      if (t + 1 < t1) {
-        products(1);
-        if (t + 2 < t1) {
-          stage(f0, 0);
-          if (t + 4 < t1) fetch(f0, t + 4);
+      if (jj == 2 || jj == (MT > 4 ? 4 : 3)) {
+        weights(P ^ 1, jj == 2 ? 0 : 1);
+        fetch(u + 2, jj == 2 ? 1 : 2);
+      }
+      if (!first.value || jj > 1) products(jj < 2 ? P ^ 1 : P, i);
+      if (jj % 2) {  // the order of two row tiles' work: a few vector instructions behind every product
+#pragma unroll
+        for (int m = 0; m < 24; ++m) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                 // MFMA
+          if (m % 4 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+          __builtin_amdgcn_sched_group_barrier(0x002, MT == 4 ? 6 : 3, 0);   // vector
+          if (m % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+          if (m > 18) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);     // load
         }
-        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  } else {  // one step in LDS, so that two workgroups fit a compute unit (two steps and one workgroup: 137 against 157 TFLOP/s)
-    for (int t = t0; t < t1; t += 2) {
-      __syncthreads();
-      stage(f0, 0);
-      if (t + 2 < t1) fetch(f0, t + 2);
-      __syncthreads();
-      products(0);
-      if (t + 1 < t1) {
-        __syncthreads();
-        stage(f1, 0);
-        if (t + 3 < t1) fetch(f1, t + 3);
-        __syncthreads();
-        products(0);
-      }
-    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's reads and writes; loads stay on their way
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int n = 0; n < 3; ++n) fetch(t0, n);
+  stage(0);
+  weights(0, 0);
+  weights(0, 1);
+#pragma unroll
+  for (int n = 0; n < 3; ++n) fetch(t0 + 1, n);
+  __syncthreads();
+  using Even = std::integral_constant<int, 0>;
+  using Odd = std::integral_constant<int, 1>;
+  round(std::true_type{}, Even{}, t0);
+  int t = t0 + 1;
+#pragma unroll 1
+  for (; t + 1 < t1; t += 2) {
+    round(std::false_type{}, Odd{}, t);
+    round(std::false_type{}, Even{}, t + 1);
   }
-  // lane: rows 16 i + c of the wave's BM / 2, columns (weight tile rows) 16 j + 4 q + 0..3
+  if (t < t1) {
+    round(std::false_type{}, Odd{}, t);
+    products(1, MT - 2);
+    products(1, MT - 1);
+  } else {
+    products(0, MT - 2);
+    products(0, MT - 1);
+  }
+  // lane: rows 16 i + c, columns (weight tile rows) 16 j + 4 q + 0..3 of the wave's 32
   bool again = false;
 #pragma unroll
-  for (int u = 0; u < NA; ++u) again |= (ta[u] & 0x7fffffffu) && !(ta[u] & F3_EXP);
-#pragma unroll
-  for (int u = 0; u < NW; ++u) again |= (tw[u] & 0x7fffffffu) && !(tw[u] & F3_EXP);
+  for (int n = 0; n < 3; ++n) again |= (bits[n] & 0x7fffffffu) && !(bits[n] & F3_EXP);
   float none[4] = {0.f, 0.f, 0.f, 0.f};  // (0 x an infinity or NaN)
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) none[r] = fmaf(acc[j][i][r], 0.f, none[r]);
   again |= !((none[0] + none[1]) + (none[2] + none[3]) == 0.f);
   if (__syncthreads_or(again)) {
-    const float *ar[MT], *wr_[4];
+    const float *ar[MT], *wr[2];
     float as[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      ar[i] = arow(wr * (BM / 2) + 16 * i + c) + 4 * q;
-      as[i] = ascale(wr * (BM / 2) + 16 * i + c);
+      ar[i] = arow(16 * i + c) + 4 * q;
+      as[i] = ascale(16 * i + c);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      wr_[j] = wrow(64 * wc + 16 * j + c) + 4 * q;
+    for (int j = 0; j < 2; ++j) {
+      wr[j] = wrow(j) + 4 * q;
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const int k1 = min(K, F3_BK * t1);
 #pragma unroll 2
-    for (int k = F3_BK * t0; k < k1; k += 16) {  // lane group q: numbers k + 4 q .. + 3 of both operands, one per instruction
+    for (int k = F3_BK * t0; k < kend; k += 16) {  // lane group q: numbers k + 4 q .. + 3 of both operands, one per instruction
       const bool in = k + 4 * q < K;
       const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      f32x4 a[MT], w[4];
+      f32x4 x[MT], y[2];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = in ? *reinterpret_cast<const f32x4*>(wr_[j] + k) : z;
+      for (int j = 0; j < 2; ++j) y[j] = in ? *reinterpret_cast<const f32x4*>(wr[j] + k) : z;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) a[i] = in ? *reinterpret_cast<const f32x4*>(ar[i] + k) * as[i] : z;
+      for (int i = 0; i < MT; ++i) x[i] = in ? *reinterpret_cast<const f32x4*>(ar[i] + k) * as[i] : z;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][r], a[i][r], acc[j][i], 0, 0, 0);
+          for (int j = 0; j < 2; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j][r], x[i][r], acc[j][i], 0, 0, 0);
     }
   }
-  // results leave through the wave's own LDS, 32 rows x 64 accumulator columns at a time: the activation is one small loop
-  // and rows leave in whole lines. 16-byte chunk x of row r lies at x ^ (r & 15)
-  f32x4* const st = reinterpret_cast<f32x4*>(lds) + wave * 512;
-  constexpr int OCH = GATED ? 8 : 16;  // output chunks of a row
+  // results leave through the wave's own LDS, 32 rows x 32 accumulator columns at a time: the activation is one small loop
+  // and rows leave in whole lines. 16-byte chunk x of row r lies at x ^ (r & 7)
+  f32x4* const out = reinterpret_cast<f32x4*>(lds) + wave * 256;
+  constexpr int OCH = GATED ? 4 : 8;  // output chunks of a row
   const int rr0 = lane / OCH, oc = lane % OCH;
-  const int gch = GATED ? 8 * (oc >> 2) + (oc & 3) : oc;
-  const int col = n0 + wc * (COLS / 2) + 4 * oc;
+  const int col = n0 + wave * (COLS / WV) + 4 * oc;
 #pragma unroll
-  for (int half = 0; half < MT / 2; ++half) {
+  for (int part = 0; part < MT / 2; ++part) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) st[(16 * i + c) * 16 + ((4 * j + q) ^ c)] = acc[j][2 * half + i];
-    const int rbase = r0 + wr * (BM / 2) + 32 * half;
+      for (int j = 0; j < 2; ++j) out[(16 * i + c) * 8 + ((4 * j + q) ^ (c & 7))] = acc[j][2 * part + i];
+    const int rbase = r0 + 32 * part;
     int drow = rbase + (lane & 31);
     drow = drow < rend ? (p.dst_idx ? p.dst_idx[drow] : drow) : -1;
 #pragma unroll 2
     for (int s = 0; s < 32; s += 64 / OCH) {
       const int rr = s + rr0;
       const int d = __shfl(drow, rr, 64);
-      const f32x4 g = st[rr * 16 + (gch ^ (rr & 15))];
-      const f32x4 u = GATED ? st[rr * 16 + ((gch + 4) ^ (rr & 15))] : g;
+      const f32x4 g = out[rr * 8 + (oc ^ (rr & 7))];
+      const f32x4 v0 = GATED ? out[rr * 8 + ((oc + 4) ^ (rr & 7))] : g;
       if (d >= 0 && col < N) {
-        const f32x4 v = act(g, u);
+        const f32x4 v = act(g, v0);
         f32x4* o = reinterpret_cast<f32x4*>(p.out + (size_t)d * p.ldo + col);
         *o = p.add ? *o + v : v;
       }
@@ -284,31 +283,34 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
   }
 }
 
-// u32x4 of LDS: two staged steps of 64 rows, one of 128 (and both hold the epilogue's 32 KiB)
-template <int BM>
+// u32x4 of LDS: two staged steps
+template <int MT>
 constexpr int f3_lds() {
-  return (BM == 64 ? 2 : 1) * 3 * 4 * (BM + F3_BN);
+  return 2 * 3 * 4 * 16 * MT;
 }
 
-// How a launch cuts its work: 64- or 128-row tiles (a step of 512 resident workgroups takes about 1.8 and 2.6 us) and K over
-// `splits` workgroups per tile, at least 8 steps each, whose partial sums go through slabs [split][R][N] that the caller's
-// second kernel adds in order (about 4 us and the slabs' traffic).
+// How a launch cuts its work: the tile and K over `splits` workgroups per tile, at least 8 steps each, whose partial sums go through
+// slabs [split][rows][cols] that the caller's second kernel adds in order. Measured: a step of 256 resident 128 x 256 tiles takes 2.05 us
+// and 5 once, one of 512 resident 64 x 128 tiles 1.33 us (0.75 if at most 256 run) and 4; the second kernel 4 us and the slabs' traffic.
 struct F3Plan {
-  int bm, splits, steps;  // steps per split
+  int bm, bn, splits, steps;  // steps per split
 };
-inline F3Plan f3_plan(long long mt128, long long mt64, long long tn, int K) {
+template <class Tiles>  // (int height) -> row tiles
+inline F3Plan f3_plan(const Tiles& row_tiles, long long rows, long long cols, int K) {
   const int total = (K + F3_BK - 1) / F3_BK;
-  F3Plan best{128, 1, total};
+  F3Plan best{128, 256, 1, total};
   double least = 1e30;
   for (int bm = 64; bm <= 128; bm += 64) {
-    const long long tiles = (bm == 64 ? mt64 : mt128) * tn;
+    const bool small = bm == 64;
+    const long long tiles = row_tiles(bm) * ((cols + 2 * bm - 1) / (2 * bm));
     for (int splits = 1; splits <= 16 && (splits == 1 || total / splits >= 8); ++splits) {
       const int steps = (total + splits - 1) / splits;
-      const double slab_us = splits == 1 ? 0. : 4. + (double)tiles * bm * F3_BN * 4 * (splits + 0.5) * 2 / 5e6;
-      const double us = (double)((tiles * splits + F3_RESIDENT - 1) / F3_RESIDENT) * steps * (bm == 64 ? 1.8 : 2.6) + slab_us;
-      if (us < 0.95 * least) {
+      const long long n = tiles * splits, resident = small ? 512 : 256;
+      const double slab_us = splits == 1 ? 0. : 4. + (double)rows * cols * 4 * (2 * splits + 1) / 5e6;
+      const double us = (double)((n + resident - 1) / resident) * (steps * (small ? (n <= 256 ? 0.75 : 1.33) : 2.05) + (small ? 4. : 5.)) + slab_us;
+      if (us < 0.97 * least) {
         least = us;
-        best = {bm, (total + steps - 1) / steps, steps};
+        best = {bm, 2 * bm, (total + steps - 1) / steps, steps};
       }
     }
   }
