@@ -354,12 +354,52 @@ __global__ void __launch_bounds__(256) gated_rmsnorm_kernel(GatedNorm p) {
   }
 }
 
+// The same with 16-byte accesses, 64 / L heads per wave (12000 tokens, 32 heads of 128: 222 -> 99 us, 5.9 TB/s).
+template <typename OT, int L>
+__global__ void __launch_bounds__(256) gated_rmsnorm_vec_kernel(GatedNorm p) {
+  const int d = 4 * (threadIdx.x % L);
+  const long long item = (long long)blockIdx.x * (256 / L) + threadIdx.x / L;
+  const long long m = item / p.H;
+  const int h = (int)(item - m * p.H);
+  const bool on = m < p.M && d < p.vdim;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f}, g = {1.f, 1.f, 1.f, 1.f}, w = v;
+  if (on) {
+    v = *reinterpret_cast<const f32x4*>(p.o + item * p.vdim + d);
+    if (p.gate_act != 2) g = *reinterpret_cast<const f32x4*>(p.gate + m * p.ldg + (size_t)h * p.vdim + d);
+    w = *reinterpret_cast<const f32x4*>(p.w + (p.w_heads ? (size_t)h * p.vdim : 0) + d);
+  }
+  const float sc = 1.f / sqrtf(hy_head_squares<L>(v) / (float)p.vdim + p.eps);
+  if (!on) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = p.gate_act == 2 ? 1.f : (p.gate_act == 1 ? hy_sigmoid(g[i]) : hy_silu(g[i]));
+    v[i] = v[i] * sc * w[i] * a * p.gain;
+  }
+  hy_store4(reinterpret_cast<OT*>(p.out) + m * p.ldo + (size_t)h * p.vdim + d, v);
+}
+
+template <typename OT>
+static void gated_rmsnorm_vec(const GatedNorm& p, int L, hipStream_t s) {
+  const unsigned grid = (unsigned)(((long long)p.M * p.H + 256 / L - 1) / (256 / L));
+  if (L == 16) gated_rmsnorm_vec_kernel<OT, 16><<<grid, 256, 0, s>>>(p);
+  else if (L == 32) gated_rmsnorm_vec_kernel<OT, 32><<<grid, 256, 0, s>>>(p);
+  else gated_rmsnorm_vec_kernel<OT, 64><<<grid, 256, 0, s>>>(p);
+}
+
 int hy_gated_rmsnorm(const GatedNorm& p, hipStream_t s) {
   if (p.M < 0 || p.H < 1 || p.vdim < 1 || p.ldo < p.H * p.vdim) return -1;
   if (p.gate_act < 0 || p.gate_act > 2) return -3;
   if (p.gate_act != 2 && (!p.gate || p.ldg < p.H * p.vdim)) return -1;
   if (p.M == 0) return 0;
   if ((p.H + 3) / 4 > 65535) return -2;
+  const int L = p.denom_floor || p.ldo % 4 || (p.gate_act != 2 && p.ldg % 4) ? 0 : hy_head_lanes(p.vdim);
+  const uintptr_t at = (uintptr_t)p.o | (uintptr_t)p.w | (uintptr_t)(p.gate_act != 2 ? p.gate : nullptr);
+  if (L && !(at & 15) && !((uintptr_t)p.out & (p.out_bf16 ? 7 : 15)) && (long long)p.M * p.H <= 0x7fffffffLL) {
+    if (p.out_bf16) gated_rmsnorm_vec<bf16_t>(p, L, s);
+    else gated_rmsnorm_vec<float>(p, L, s);
+    JLA_CHECK_LAUNCH();
+    return 0;
+  }
   gated_rmsnorm_kernel<<<dim3(p.M, (p.H + 3) / 4), 256, 0, s>>>(p);
   JLA_CHECK_LAUNCH();
   return 0;

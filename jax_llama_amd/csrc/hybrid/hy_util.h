@@ -31,4 +31,17 @@ JLA_DEV float hy_gelu_tanh(float z) {
 JLA_DEV float hy_logsigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 JLA_DEV float hy_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
+// Heads of up to 4 L numbers in groups of L lanes, four neighbouring numbers per lane: the sum of squares of the group's head
+template <int L>
+JLA_DEV float hy_head_squares(const f32x4 v) {
+  float ss = fmaf(v[0], v[0], v[1] * v[1]) + fmaf(v[2], v[2], v[3] * v[3]);
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  return ss;
+}
+// ... whether heads of n numbers run in such groups, and L (0: they do not)
+inline int hy_head_lanes(int n) { return n % 4 || n > 256 ? 0 : (n <= 64 ? 16 : (n <= 128 ? 32 : 64)); }
+JLA_DEV void hy_store4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+JLA_DEV void hy_store4(bf16_t* p, const f32x4 v) { *reinterpret_cast<u32x2*>(p) = u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])}; }
+
 }  // namespace jla

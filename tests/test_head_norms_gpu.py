@@ -1,0 +1,51 @@
+"""Per-head norms in groups of lanes (attn_prep in csrc/hybrid/attn_bias.hip, gated_rmsnorm in delta_rule.hip) against the CPU ops, at
+the edges of the groups and where the separate kernel runs (odd sizes, unaligned rows)."""
+import pytest
+import torch
+
+from jax_llama_amd.ops import hybrid as hy
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# a norm's statistic, root and three products round by 2^-24 each, the sum of n squares by at most log2(n) + 2 of it
+TOL = 16 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dim,vdim", [(4, 4), (60, 64), (64, 64), (68, 128), (128, 64), (128, 128), (132, 256), (256, 4), (256, 260), (66, 64)])
+@pytest.mark.parametrize("h,g,pad", [(1, 1, 0), (6, 2, 4), (5, 5, 3)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("own", [True, False])
+def test_attn_prep(dim, vdim, h, g, pad, dt, own):
+    b, s, s0, t = 2, 7, 3, 9  # (the last token of a row has no slot left)
+    gen = torch.Generator().manual_seed(dim * h)
+    proj = torch.randn(b * s, h * dim + g * (dim + vdim) + pad, generator=gen)
+    pos = torch.arange(b * s, dtype=torch.int32) * 400
+    kw = dict(temp_coef=0.1, temp_every=512, q_w=torch.randn(dim, generator=gen), k_w=torch.randn(dim, generator=gen), norm_v=h != 5)
+    out = []
+    for dev in ("cpu", DEV):
+        n = s if dev == DEV else s - 1
+        kc, vc = torch.zeros(b, g, t, dim, dtype=dt, device=dev), torch.zeros(b, g, t, vdim, dtype=dt, device=dev)
+        rows = torch.arange(b * s).reshape(b, s)[:, :n].reshape(-1)
+        cols = h * dim + (g * (dim + vdim) if own else 0)
+        q = hy.attn_prep(proj[rows].to(dev)[:, :cols], pos[rows].to(dev), torch.tensor([s0], dtype=torch.int32, device=dev), b, n, h, g, dim, vdim,
+                         kc if own else None, vc if own else None, 1e-5, **{k: v.to(dev) if torch.is_tensor(v) else v for k, v in kw.items()})
+        out.append([x.float().cpu() for x in (q[:, :s - 1], kc, vc)])
+    for want, got in zip(*out):
+        assert float(((got - want).abs() / want.abs().clamp_min(1e-6)).max()) <= (TOL if want is out[0][0] or dt == torch.float32 else 2.0 ** -7)
+
+
+@pytest.mark.parametrize("vdim", [4, 64, 68, 128, 200, 256, 260, 66])
+@pytest.mark.parametrize("m,h", [(1, 1), (5, 3), (300, 6)])
+@pytest.mark.parametrize("act", [hy.GATE_SILU, hy.GATE_SIGMOID, hy.GATE_NONE])
+@pytest.mark.parametrize("dt,col", [(torch.float32, 0), (torch.bfloat16, 4), (torch.float32, 3)])
+def test_gated_rmsnorm(vdim, m, h, act, dt, col):
+    gen = torch.Generator().manual_seed(vdim + m)
+    o, gate = torch.randn(m, h, vdim, generator=gen), torch.randn(m, h * vdim + 8, generator=gen)[:, col:col + h * vdim]
+    w = torch.randn(h * vdim if m == 5 else vdim, generator=gen)
+    want = hy.gated_rmsnorm(o, None if act == hy.GATE_NONE else gate, w, 1e-5, act, gain=0.5)
+    wide = torch.full((m, h * vdim + 8), 7.0, dtype=dt, device=DEV)
+    hy.gated_rmsnorm(o.to(DEV), None if act == hy.GATE_NONE else gate.to(DEV), w.to(DEV), 1e-5, act, gain=0.5, out=wide[:, col:col + h * vdim])
+    got = wide.float().cpu()
+    assert bool((got[:, :col] == 7).all()) and bool((got[:, col + h * vdim:] == 7).all())
+    got = got[:, col:col + h * vdim]
+    assert float(((got - want).abs() / want.abs().clamp_min(1e-6)).max()) <= (TOL if dt == torch.float32 else 2.0 ** -8 + TOL)
