@@ -403,7 +403,7 @@ void hc_update(Tensor xs, OptT mix, OptT out_w, OptT y, int64_t nsum, OptT row_w
 }
 
 void norm_residual(Tensor y, int64_t nsum, double ysc, Tensor w, double eps, OptT x, OptT out, OptT extra,
-                   OptT extra_gate) {
+                   OptT extra_gate, OptT rounded) {
   check(y.dim() == 2 && nsum >= 1 && y.size(0) % nsum == 0, "norm_residual: y is [M * nsum, D]");
   const int M = y.size(0) / nsum, D = y.size(1);
   check(w.numel() == 1 || w.numel() == D, "norm_residual: w has 1 or D elements");
@@ -429,8 +429,15 @@ void norm_residual(Tensor y, int64_t nsum, double ysc, Tensor w, double eps, Opt
     check(ep && extra_gate->dim() == 2 && extra_gate->size(0) == M, "norm_residual: extra_gate is [M, 1] beside extra");
     gp = rows2d(*extra_gate, "extra_gate", 1, &ldg);
   }
+  jla::bf16_t* rp = nullptr;
+  if (rounded.has_value()) {
+    gpu(*rounded, "rounded");
+    check(rounded->scalar_type() == torch::kBFloat16 && rounded->is_contiguous() && rounded->numel() == (int64_t)M * D && D % 8 == 0,
+          "norm_residual: rounded is bf16 [M, D], D a multiple of 8");
+    rp = reinterpret_cast<jla::bf16_t*>(rounded->data_ptr());
+  }
   rc(jla::hy_norm_residual(f32(y, "y"), nsum, (float)ysc, f32(w, "w"), w.numel() > 1 || D == 1, (float)eps, xp, op, M,
-                           D, ep, gp, ldg, stream()),
+                           D, ep, gp, ldg, rp, stream()),
      "norm_residual");
 }
 
@@ -1290,7 +1297,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("ACT_RELU2") = (int)jla::HY_ACT_RELU2;
   m.attr("ACT_SWIGLU") = (int)jla::HY_ACT_SWIGLU;
   m.attr("ACT_CLAMP_GLU") = (int)jla::HY_ACT_CLAMP_GLU;
-  m.def("norm_residual", &norm_residual);
+  m.def("norm_residual", &norm_residual, py::arg("y"), py::arg("nsum"), py::arg("ysc"), py::arg("w"), py::arg("eps"), py::arg("x"),
+        py::arg("out"), py::arg("extra"), py::arg("extra_gate"), py::arg("rounded") = py::none());
   m.def("gelu_gate_rows", &gelu_gate_rows);
   m.def("cast_bf16", &cast_bf16, py::arg("x"), py::arg("y"), py::arg("act") = 0);
   m.def("softcap", &softcap);

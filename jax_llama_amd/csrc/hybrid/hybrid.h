@@ -174,16 +174,17 @@ struct HyperUpdate {
 };
 int hy_hc_update(const HyperUpdate& p, hipStream_t s);
 
+typedef uint16_t bf16_t;
+
 // x[m, :] += (sum_{c < nsum} y[m * nsum + c, :]) * ysc / sqrt(mean(.^2) + eps) * w   (w: one number, or D numbers).
 // x == nullptr: out-of-place into `out` without the add (a plain RMS norm).
 // extra (optional, [M, D]): sigmoid(extra_gate[m * ldg]) * extra[m, :] joins the sum before the norm (extra_gate ==
-// nullptr: weight 1).
+// nullptr: weight 1). rounded (optional, D a multiple of 8): the result also in bf16, the operand of the next product.
 int hy_norm_residual(const float* y, int nsum, float ysc, const float* w, int w_vec, float eps, float* x, float* out,
-                     int M, int D, const float* extra, const float* extra_gate, int ldg, hipStream_t s);
+                     int M, int D, const float* extra, const float* extra_gate, int ldg, bf16_t* rounded, hipStream_t s);
 
 // y (bf16) = act(x (fp32)), n a multiple of 8; act: HY_ACT_NONE or HY_ACT_RELU2 (the activation of a feed-forward whose two
 // products run on the packed GEMM, applied while the hidden activation is rounded for the second)
-typedef uint16_t bf16_t;
 int hy_cast_bf16(const float* x, bf16_t* y, long long n, int act, hipStream_t s);
 
 // out[m * ldo + c] = act(gu[m * ldg + c], gu[m * ldg + F + c]) for c < F: the gated epilogue of a product [M, >= 2F] that ran

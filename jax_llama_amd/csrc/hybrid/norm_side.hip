@@ -175,11 +175,12 @@ JLA_DEV float ns_block_sum(float v, float* red) {
 
 // The same with 16-byte accesses (D a multiple of 4, aligned rows): one workgroup brings a whole row in, so the instructions
 // between its loads show. Us before -> after: 1 x 2048 3.5 -> 2.5, 8 x 4096 with two summands 6.4 -> 3.0, 16384 x 4096 with two
-// summands 322 -> 199 (5.4 TB/s). T: about one 16-byte column group per thread (256 threads of a 4096-column row: 3.3 us).
+// summands 322 -> 199 (5.4 TB/s). rounded: the result also in bf16 for a prompt's next product, whose own pass took 49 us of 12000 x 4096 (a
+// prompt of that size with 11 of them and 4 bf16 features 25.0 -> 24.6 ms). T: about one 16-byte column group per thread (256 threads of a 4096-column row: 3.3 us).
 template <int T, int NV>
 __global__ void __launch_bounds__(T) norm_residual_vec_kernel(const float* y, int nsum, float ysc, const float* w, int w_vec,
                                                               float eps, float* x, float* out, int D, const float* extra,
-                                                              const float* extra_gate, int ldg) {
+                                                              const float* extra_gate, int ldg, bf16_t* rounded) {
   __shared__ float red[16];
   const int m = blockIdx.x;
   const float* yr = y + (size_t)m * nsum * D;
@@ -218,16 +219,17 @@ __global__ void __launch_bounds__(T) norm_residual_vec_kernel(const float* y, in
 #pragma unroll
     for (int i = 0; i < 4; ++i) xv[u][i] += v[u][i] * sc * wv[u][i];
     if (d < D) *reinterpret_cast<f32x4*>(to + d) = xv[u];
+    if (rounded && d < D) hy_store4(rounded + (size_t)m * D + d, xv[u]);
   }
 }
 
 int hy_norm_residual(const float* y, int nsum, float ysc, const float* w, int w_vec, float eps, float* x, float* out,
-                     int M, int D, const float* extra, const float* extra_gate, int ldg, hipStream_t s) {
-  if (M < 0 || D < 1 || nsum < 1 || (!x && !out) || (extra_gate && (!extra || ldg < 1))) return -1;
+                     int M, int D, const float* extra, const float* extra_gate, int ldg, bf16_t* rounded, hipStream_t s) {
+  if (M < 0 || D < 1 || nsum < 1 || (!x && !out) || (extra_gate && (!extra || ldg < 1)) || (rounded && D % 8)) return -1;
   if (M == 0) return 0;
   auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  if (D % 4 == 0 && D > 256 && D <= 8192 && aligned(y) && aligned(x) && aligned(out) && aligned(extra) && (!w_vec || aligned(w))) {
-#define NR_VEC(T, NV) norm_residual_vec_kernel<T, NV><<<M, T, 0, s>>>(y, nsum, ysc, w, w_vec, eps, x, out, D, extra, extra_gate, ldg)
+  if (D % 4 == 0 && D > 256 && D <= 8192 && aligned(y) && aligned(x) && aligned(out) && aligned(extra) && (!w_vec || aligned(w)) && aligned(rounded)) {
+#define NR_VEC(T, NV) norm_residual_vec_kernel<T, NV><<<M, T, 0, s>>>(y, nsum, ysc, w, w_vec, eps, x, out, D, extra, extra_gate, ldg, rounded)
     if (D <= 1024) NR_VEC(256, 1);
     else if (D <= 2048) NR_VEC(512, 1);
     else if (D <= 4096) NR_VEC(512, 2);
@@ -247,7 +249,7 @@ int hy_norm_residual(const float* y, int nsum, float ysc, const float* w, int w_
   else NR_LAUNCH(0);
 #undef NR_LAUNCH
   JLA_CHECK_LAUNCH();
-  return 0;
+  return rounded ? hy_cast_bf16(x ? x : out, rounded, (long long)M * D, HY_ACT_NONE, s) : 0;
 }
 
 // bf16 copy of an fp32 activation (the A operand of the packed MFMA GEMMs), 8 elements per thread

@@ -111,7 +111,7 @@ class BiasedAttention:
                 return hy.linear(a, self.w_o)
         q = hy.attn_prep(proj, ctx.positions, ctx.slot0, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim,
                          kc if own else None, vc if own else None, self.eps, sp.q_temp_coef, sp.q_temp_every)
-        a = hy.attn_bias(q, kc, vc, ctx.slot0, sp.scale, sp.softcap, self.bias)
+        a = hy.attn_bias(q, kc, vc, ctx.slot0, sp.scale, sp.softcap, self.bias, out=hy.operand_rows(ctx.b * ctx.s, self.w_o))
         return hy.linear(a, self.w_o)
 
 
@@ -139,7 +139,8 @@ class GatedDeltaMixer:
                                              tail, self.a_log, self.dt_bias)
         c = 2 * sp.kv_heads * sp.dim + sp.heads * sp.vdim
         gate = proj[:, c:c + sp.heads * sp.vdim]
-        return hy.linear(hy.delta_memory(q, k, v, beta, decay, state, ctx.b, ctx.s, gate, self.norm_w, self.eps), self.w_o)
+        rows = hy.operand_rows(ctx.b * ctx.s, self.w_o) if ctx.s > 1 else None
+        return hy.linear(hy.delta_memory(q, k, v, beta, decay, state, ctx.b, ctx.s, gate, self.norm_w, self.eps, rows), self.w_o)
 
 
 class TableMoE:

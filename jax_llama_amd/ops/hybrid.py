@@ -231,12 +231,13 @@ def _act_cpu(y: torch.Tensor, act: int, limit: float, alpha: float) -> torch.Ten
 
 class Residual:
     """A step's residual stream ``x [M, D]`` with its last sublayer's result not added yet (``norm_residual_``'s arguments): the
-    product that reads the stream next adds it where it has few rows (``rows_gemv.hip``), ``value()`` everywhere else."""
+    product that reads the stream next adds it where it has few rows (``rows_gemv.hip``), ``value()`` everywhere else. ``rows``:
+    the stream in bf16, once a prompt's product has asked for it (``operand``)."""
 
-    __slots__ = ("x", "pending")
+    __slots__ = ("x", "pending", "rows")
 
     def __init__(self, x: torch.Tensor):
-        self.x, self.pending = x, None
+        self.x, self.pending, self.rows = x, None, None
 
     def add(self, y: torch.Tensor, w: torch.Tensor, eps: float, nsum: int = 1, ysc: float = 1.0) -> None:
         self.value()
@@ -244,9 +245,22 @@ class Residual:
 
     def value(self) -> torch.Tensor:
         if self.pending is not None:
-            (y, nsum, ysc, w, eps), self.pending = self.pending, None
+            (y, nsum, ysc, w, eps), self.pending, self.rows = self.pending, None, None
             norm_residual_(self.x, y, w, eps, nsum, ysc)
         return self.x
+
+    def operand(self, wdtype) -> torch.Tensor:
+        """``value()`` for a product with weights of ``wdtype``: a prompt's rows rounded to bf16 by the kernel that adds, others fp32."""
+        x = self.x
+        if not (_gpu(x) and x.is_contiguous() and prompt_bf16(x.shape[0], x.shape[1], wdtype)):
+            return self.value()
+        if self.pending is not None:
+            (y, nsum, ysc, w, eps), self.pending = self.pending, None
+            self.rows = torch.empty(x.shape, dtype=BF16, device=x.device)
+            norm_residual_(x, y, w, eps, nsum, ysc, rounded=self.rows)
+        elif self.rows is None:
+            self.rows = _bf16_rows(x)
+        return self.rows
 
     def fusable(self) -> bool:
         return (self.pending is not None and _gpu(self.x) and self.x.shape[0] <= RESIDUAL_MAX_ROWS and self.x.is_contiguous()
@@ -267,9 +281,12 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
         out = torch.empty(r.x.shape[0], w.shape[0], dtype=F32, device=r.x.device)
         new = torch.empty_like(r.x)
         if ext().rows_fused(r.x, w, out, *r.pending, new, ids, table, int(col0)):
-            r.x, r.pending = new, None
+            r.x, r.pending, r.rows = new, None, None
             return out
-    xv = r.value() if r is not None else x
+    if r is not None and _use_packed_gemm(r.x, w):  # (a prompt)
+        xv = r.operand(w.dtype)
+    else:
+        xv = r.value() if r is not None else x
     if ids is None:
         return linear(xv, w)
     if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and xv.dtype == F32 and w.dtype == BF16:
@@ -298,7 +315,7 @@ def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
         if r is not None and r.fusable():
             new = torch.empty_like(xv)
             if ext().rows_fused(xv, w, out, *r.pending, new, **norm):
-                r.x, r.pending = new, None
+                r.x, r.pending, r.rows = new, None, None
                 return out
         xv = r.value() if r is not None else x
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, **norm):
@@ -321,7 +338,7 @@ def head_argmax(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
     if part is None:
         return None
     if new is not None:
-        r.x, r.pending = new, None
+        r.x, r.pending, r.rows = new, None, None
     return ArgmaxParts(part)
 
 
@@ -337,7 +354,7 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     if isinstance(x, Residual):
         if act == ACT_NONE and not swiglu and x.fusable() and w.shape[0] > SKINNY_MAX_N:
             return linear_rows_gated(x, w)
-        x = x.value()
+        x = x.operand(w.dtype) if act == ACT_NONE and not swiglu and _use_packed_gemm(x.x, w) else x.value()
     if swiglu:
         act = ACT_SWIGLU
     n = w.shape[0] // 2 if act_gated(act) else w.shape[0]
@@ -372,6 +389,15 @@ def prompt_bf16(m: int, cols: int, wdtype) -> bool:
     """Whether a step of ``m`` rows keeps a sublayer's input and features in bf16 (the matrix operands they would be
     rounded to anyway, half the traffic): prompt-sized batches with bf16 weights. Fewer rows run GEMVs, which read fp32."""
     return wdtype == BF16 and m >= PACKED_GEMM_MIN_M and cols % 8 == 0
+
+
+def operand_rows(m: int, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """Where the kernel before a product with ``w [N, K]`` writes ``m`` rows for it: bf16 ``[m, K]`` of a prompt on the packed GEMM
+    (the operand they would be rounded to anyway), else None."""
+    if not _gpu(w) or w.dim() != 2 or not prompt_bf16(m, w.shape[1], w.dtype):
+        return None
+    rows = torch.empty(m, w.shape[1], dtype=BF16, device=w.device)
+    return rows if _use_packed_gemm(rows, w) else None
 
 
 def glu_rows(gu: torch.Tensor, act: int, out: torch.Tensor, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
@@ -546,13 +572,13 @@ def moe_table(x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, w_gu: tor
         if res is not None and res.fusable():
             new = torch.empty_like(x)
             if ext().table_rows(x, *args, *res.pending, new):
-                res.x, res.pending = new, None
+                res.x, res.pending, res.rows = new, None, None
                 return y
         x = res.value() if res is not None else x
         if ext().table_rows(x, *args, None, 1, 1.0, None, 0.0, None):
             return y
     if res is not None:
-        x = res.value()
+        x = res.operand(w_gu.dtype) if r > GROUPED_GEMV_MAX_R and w_down.dtype == BF16 else res.value()
     if not _gpu(x):
         ex = table[ids.long()].reshape(-1).long()  # [R]
         xr = _round_like(x, w_gu).repeat_interleave(top, 0)
@@ -578,8 +604,7 @@ def moe_table(x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, w_gu: tor
     elif bf16_pair:
         # prompt-sized, bf16: the tiles read a bf16 copy of x and keep the hidden activation bf16 (the operands they
         # would round to anyway), which halves the activation traffic of both products
-        xb = torch.empty(x.shape, dtype=BF16, device=dev)
-        e.cast_bf16(x, xb)
+        xb = _bf16_rows(x)
         hb = torch.empty(r, w_gu.shape[1] // 2, dtype=BF16, device=dev)
         e.linear_rows(xb, sort_tok, w_gu, hb, None, offs, None, r, ACT_SWIGLU, 0.0, 1.0, None, None, 0.0)
         e.linear_rows(hb, None, w_down, y, sort_dst, offs, None, r, ACT_NONE, 0.0, 1.0, None, None, 0.0)
@@ -877,17 +902,19 @@ def sandwich_update_(x: torch.Tensor, y: Optional[torch.Tensor], post: Optional[
 
 
 def norm_residual_(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, eps: float, nsum: int = 1, ysc: float = 1.0,
-                   extra: Optional[torch.Tensor] = None, extra_gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   extra: Optional[torch.Tensor] = None, extra_gate: Optional[torch.Tensor] = None,
+                   rounded: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``x += rms_norm(ysc * sum of each token's nsum rows of y [+ sigmoid(extra_gate) * extra]) * w`` in place; ``w``
     one number or ``[D]``. ``extra [M, D]``: one more summand per token (a shared expert's output) with the logit of
-    its gate in ``extra_gate [M, 1]`` (a column view is fine; absent: weight 1)."""
+    its gate in ``extra_gate [M, 1]`` (a column view is fine; absent: weight 1). ``rounded [M, D]`` bf16 (on the GPU): the new ``x``
+    as a product's operand."""
     if not _gpu(x):
         v = y.float().reshape(x.shape[0], nsum, -1).sum(1) * ysc
         if extra is not None:
             v = v + (torch.sigmoid(extra_gate.float()) * extra.float() if extra_gate is not None else extra.float())
         x.add_(v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps) * w.float().reshape(-1))
         return x
-    ext().norm_residual(y, int(nsum), float(ysc), w.reshape(-1), float(eps), x, None, extra, extra_gate)
+    ext().norm_residual(y, int(nsum), float(ysc), w.reshape(-1), float(eps), x, None, extra, extra_gate, rounded)
     return x
 
 
@@ -1316,12 +1343,13 @@ def _step_out(x: torch.Tensor, width: int, dim: int, vdim: int, s: int, out: Opt
 
 
 def delta_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor,
-                 state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
-    """``gated_rmsnorm(delta_scan(...), gate, w, eps)``."""
+                 state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float,
+                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``gated_rmsnorm(delta_scan(...), gate, w, eps)``; ``rows``: what it writes where the separate ops run (a product's operand)."""
     h, vdim = v.shape[1], v.shape[2]
-    out = _step_out(q, h * vdim, q.shape[2], vdim, s, None)
+    out = _step_out(q, h * vdim, q.shape[2], vdim, s, None) if rows is None else None
     if out is None:
-        return gated_rmsnorm(delta_scan(q, k, v, beta, decay, state, b, s), gate, w, eps)
+        return gated_rmsnorm(delta_scan(q, k, v, beta, decay, state, b, s), gate, w, eps, out=rows)
     ext().rec_step(3, q, k, v, beta=beta, decay=decay, state=state, gate=gate, w=w, eps=float(eps), gate_act=GATE_SILU, gain=1.0,
                    out=out)
     return out

@@ -49,3 +49,20 @@ def test_gated_rmsnorm(vdim, m, h, act, dt, col):
     assert bool((got[:, :col] == 7).all()) and bool((got[:, col + h * vdim:] == 7).all())
     got = got[:, col:col + h * vdim]
     assert float(((got - want).abs() / want.abs().clamp_min(1e-6)).max()) <= (TOL if dt == torch.float32 else 2.0 ** -8 + TOL)
+
+
+@pytest.mark.parametrize("m,d", [(256, 264), (300, 1024), (256, 4096), (257, 8200), (256, 200)])
+@pytest.mark.parametrize("nsum", [1, 2])
+def test_residual_as_an_operand(m, d, nsum):
+    """The stream rounded by the kernel that adds to it: what rounding it afterwards gives, again after another addition."""
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    r, plain = (hy.Residual(torch.ones(m, d, device=DEV)) for _ in range(2))
+    assert torch.equal(r.operand(torch.bfloat16), r.x.bfloat16())
+    for _ in range(2):
+        y, w = torch.randn(m * nsum, d, generator=gen, device=DEV), torch.randn(d, generator=gen, device=DEV)
+        r.add(y, w, 1e-5, nsum, 0.5)
+        plain.add(y, w, 1e-5, nsum, 0.5)
+        rows = r.operand(torch.bfloat16)
+        assert rows.dtype == torch.bfloat16 and torch.equal(rows, plain.value().bfloat16()) and torch.equal(r.value(), plain.x)
+        assert r.operand(torch.bfloat16) is rows and r.operand(torch.float32).dtype == torch.float32
+    assert hy.Residual(torch.ones(3, 8, device=DEV)).operand(torch.bfloat16).dtype == torch.float32
