@@ -647,7 +647,9 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // unit 4.6), four rows 5.5 -> 3.6; weights in a cache, one row 4.3 -> 3.3 (3.5); K 4096 5.9 -> 6.8.
   const long long all = tiles * groups;
   int nt = gated || mt > 1 || all >= (G == 4 ? (p.K <= RV_PAIR_K ? 256 : 1024) : 512) ? 2 : 1;
-  if (all >= (G > 4 ? 2048 : (gated ? 2048 : 12288))) nt = 4;
+  // Rows by expert, four tiles from 2048 on (us, two | four tiles: 16 rows, 8 experts, K 7168 x N 4096 84 | 76, 3 rows 34 | 30, K 2816 x
+  // N 2048 16 rows 22.4 | 19.0, 3 rows 9.7 | 10.4).
+  if (all >= (G > 4 || gated || p.offs ? 2048 : 12288)) nt = 4;
   const long long wgs = (tiles + nt - 1) / nt;
   if (wgs > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)wgs, groups);
