@@ -1495,6 +1495,25 @@ static int num_cus() {
   return g_num_cus;
 }
 
+// The rows behind the whole rounds of 256 x 256 tiles, where they fill at most half of another one: how many (0: none) and the K split
+// that fills the chip with them, at least four 64-deep K-tiles each. It has to take enough off the chain of one tile for its partial
+// sums' way through memory and its second launch. Us without -> with, M x 4096 x K, residual: 12800 x 14336 1365 -> 1125, x 4096
+// 445 -> 387, x 2048 265 -> 250 (x 1024 157 -> 174: not); 8704 x 14336 1000 -> 787; 14336 x 4096 447 -> 425 (2 ways). Stored:
+// 12800 x 4096 385 -> 360, 13312 x 4096 (4 ways) 375 -> 373, 14336 x 14336 (2 ways) 1371 -> 1255 (x 4096 399 -> 408, 12800 x 2048
+// 209 -> 207: not).
+int gemm_tail_rows(int M, int N, int K, int residual, int* ksplit) {
+  const int tm = (M + G4_BM - 1) / G4_BM, tn = (N + G4_BN - 1) / G4_BN, cus = num_cus();
+  *ksplit = 1;
+  if ((K & 63) || M <= 0 || N <= 0 || (long long)tm * tn > 0x7fffffffLL) return 0;
+  const int whole = tm * tn / cus * cus / tn;  // tile rows of the whole rounds
+  const int rest = (tm - whole) * tn;
+  if (whole == 0 || rest == 0 || 2 * rest > cus) return 0;
+  const int ks = min(cus / rest, (K >> 6) / 4);
+  if (ks < 2 || (long long)K * (ks - 1) < (residual ? 1536LL : 3072LL) * ks) return 0;
+  *ksplit = ks;
+  return M - whole * G4_BM;
+}
+
 // the split-K reduce + epilogue launch over [ksplit][M][N] partial slabs (+ [ksplit][M] sums of squares, fused norm)
 static int launch_reduce(const float* ws, int ksplit, void* out, int M, int N, int K, int mode, int accumulate,
                          int out_f32, bf16_t* mirror, const QKVArgs* qkv, const float* ssq, float rms_eps,

@@ -73,6 +73,7 @@ inline bool gemv_xp_variant(int v) { return v == 12 || v == 15 || v == 18 || v =
 // 128x128-tile MFMA GEMM (gemm.hip). ksplit > 1 splits K over gridDim.z into fp32 partials
 // (ws >= gemm_workspace_floats) reduced in fixed order by an epilogue kernel; MODE_QKV needs ksplit > 1.
 int gemm_ksplit(int M, int N, int K);
+int gemm_tail_rows(int M, int N, int K, int residual, int* ksplit);
 int gemm_qkv_direct_ok(int M, int tile, int K);  // qkv without a K split: the direct RoPE / KV-write GEMM epilogue applies
 // gemm4 (the 4-wave 256 x 256 kernel, tile config 7) as the tile-0 default for M > 128, K % 64 == 0 (on by default)
 void gemm_set_g4_default(int on);

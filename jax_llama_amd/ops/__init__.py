@@ -330,6 +330,7 @@ def _tiled_input(x, rms_eps, fused=False):
     return x if x.dtype == BF16 else x.to(BF16)
 
 
+G4D_TILE = 14  # gemm4 with the weights three K-tiles deep
 G5_TILES = (11, 12)  # gemm5 weight-streaming split-K (csrc/kernels/gemm5ws.h): 256- / 128-column workgroups
 
 
@@ -360,6 +361,13 @@ def _tiled(e, x, weight, n, k, out, mode, rms_eps, accumulate, mirror=None, pack
     fused = _fused_rms(e, mode, rms_eps)
     xb = _tiled_input(x, rms_eps, fused)
     ks, tm, ws = _gemm_ws(e, x.shape[0], n, k, x.device, mode, fused)
+    if ks == 1 and tm == 0 and not fused and mode in (MODE_STORE, MODE_RESIDUAL):  # (a prompt past the tuned sizes)
+        rest, split = e.gemm_tail(x.shape[0], n, k, mode == MODE_RESIDUAL)
+        if rest:  # its last rows, whose tiles would leave most of the chip idle, with K split over the chip
+            m0 = x.shape[0] - rest
+            e.gemm(xb[m0:], weight, n, k, out[m0:], mode, bool(accumulate), mirror[m0:] if mirror is not None else None, split,
+                   workspace.get("gemm_ws", split * rest * (n + 1), torch.float32, x.device), -1.0, G4D_TILE, None, None)
+            xb, out, mirror = xb[:m0], out[:m0], mirror[:m0] if mirror is not None else None
     e.gemm(xb, weight, n, k, out, mode, bool(accumulate), mirror, ks, ws, float(rms_eps) if fused else -1.0, tm,
            pack_out, _rms_ws(x, fused, ks))
 
