@@ -232,7 +232,7 @@ def _act_cpu(y: torch.Tensor, act: int, limit: float, alpha: float) -> torch.Ten
 class Residual:
     """A step's residual stream ``x [M, D]`` with its last sublayer's result not added yet (``norm_residual_``'s arguments): the
     product that reads the stream next adds it where it has few rows (``rows_gemv.hip``), ``value()`` everywhere else. ``rows``:
-    the stream in bf16, once a prompt's product has asked for it (``operand``)."""
+    the stream in bf16, once a prompt's product has asked for it (``operand``) and until the stream itself is handed out."""
 
     __slots__ = ("x", "pending", "rows")
 
@@ -244,8 +244,9 @@ class Residual:
         self.pending = (y, int(nsum), float(ysc), w.reshape(-1), float(eps))
 
     def value(self) -> torch.Tensor:
+        self.rows = None  # (who takes the tensor may write to it)
         if self.pending is not None:
-            (y, nsum, ysc, w, eps), self.pending, self.rows = self.pending, None, None
+            (y, nsum, ysc, w, eps), self.pending = self.pending, None
             norm_residual_(self.x, y, w, eps, nsum, ysc)
         return self.x
 

@@ -63,6 +63,9 @@ def test_residual_as_an_operand(m, d, nsum):
         r.add(y, w, 1e-5, nsum, 0.5)
         plain.add(y, w, 1e-5, nsum, 0.5)
         rows = r.operand(torch.bfloat16)
-        assert rows.dtype == torch.bfloat16 and torch.equal(rows, plain.value().bfloat16()) and torch.equal(r.value(), plain.x)
-        assert r.operand(torch.bfloat16) is rows and r.operand(torch.float32).dtype == torch.float32
+        assert rows.dtype == torch.bfloat16 and torch.equal(rows, plain.value().bfloat16()) and r.operand(torch.bfloat16) is rows
+        assert torch.equal(r.value(), plain.x) and r.operand(torch.float32).dtype == torch.float32
+        for x in (r, plain):
+            x.value().mul_(0.5)  # (a block that adds to the stream in place)
+        assert torch.equal(r.operand(torch.bfloat16), plain.x.bfloat16())
     assert hy.Residual(torch.ones(3, 8, device=DEV)).operand(torch.bfloat16).dtype == torch.float32
