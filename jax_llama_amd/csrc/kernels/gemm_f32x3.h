@@ -1,28 +1,29 @@
 // fp32 products on the bf16 matrix cores: every operand is the sum of three bf16 numbers, each the nearest to what the ones
-// before it leave (8 bits each, so the split is exact), and a product is the six largest of the nine partial products, smallest
-// first,
+// before it leave (8 bits each, so the split is exact), and a product is the six largest of the nine partial products,
+// smallest first,
 //     a w = lo hi + hi lo + mid mid + mid hi + hi mid + hi hi,
-// in fp32, the sum of a step of 32 from zero and then into the running sum. |mid| is below 2^-8 and |lo| below 2^-17 of the operand, so what is left out (mid lo, lo mid, lo lo)
-// is below 2^-24 of the product, half an fp32 rounding, and of either sign: parts that are cut instead of rounded all have the
-// operand's sign, and a sum of products of one sign comes out low (1 x 32000 x 4096, positive numbers, error against 64 bits:
-// exact-f32 MFMA 9.9e-7, cut parts 3.2e-6, all of it one-sided, nearest parts 3.2e-7). v_mfma_f32_16x16x32_bf16 adds 8
-// products at a time to the accumulator, rounded to nearest: 24 roundings per 32 products, of the step's sum, and one of the running
-// sum, where the fp32 matrix instruction rounds the running sum once per product (70 x 512 x 8: 5.3e-8 -> 3.1e-8). It does 16 times the work of v_mfma_f32_16x16x4_f32 per cycle, so six of them are 2.7 times
-// its rate.
+// in fp32, the sum of a step of 32 from zero and then into the running sum. |mid| is below 2^-8 and |lo| below 2^-17 of the
+// operand, so what is left out (mid lo, lo mid, lo lo) is below 2^-24 of the product, half an fp32 rounding, and of either
+// sign: parts that are cut instead of rounded all have the operand's sign, and a sum of products of one sign comes out low (1
+// x 32000 x 4096, positive numbers, error against 64 bits: exact-f32 MFMA 9.9e-7, cut parts 3.2e-6, all of it one-sided,
+// nearest parts 3.2e-7). v_mfma_f32_16x16x32_bf16 adds 8 products at a time to the accumulator, rounded to nearest: 24
+// roundings per 32 products, of the step's sum, and one of the running sum, where the fp32 matrix instruction rounds the
+// running sum once per product (70 x 512 x 8: 5.3e-8 -> 3.1e-8). It does 16 times the work of v_mfma_f32_16x16x4_f32 per
+// cycle, so six of them are 2.7 times its rate.
 //
-// One workgroup: 128 x 256 outputs in eight waves (two per SIMD) or 64 x 128 in four; a wave has all rows and 32 columns. K advances
-// 32 per step. The operands are split on their way (6 vector instructions per number), so memory holds plain fp32 and nothing is
-// prepared ahead: the activations through LDS, in two images, a wave's own weights straight into the layout of the matrix
-// instruction. LDS: per part [rows][4 cells of 16 B], cell c of row r at c ^ (r & 8 ? 3 : 0): a read of 16 bytes per lane takes lanes
-// 0-3, 12-15, 20-23, 24-27 together (then 4-11, 16-19, 28-31, and so above 32), which fall on all 64 banks (c ^ ((r >> 2) & 3): half of
-// the reads' cycles were conflicts).
-// What bounds it: the matrix cores at 70 % of their cycles and a clock held at 1.95 GHz by power. Each product is followed by the few
-// vector instructions that fit beside it, the one barrier of a step lies where the next products' operands are on their way, and a
-// step's six products start from zero, so that the running sums are rounded once per step and not 24 times (4 vector additions per
-// tile, 5 % of the time; relative error of normal numbers, K 4096 in one chain 1.0e-6 -> 2.2e-7, K 2048 7.0e-7 -> 1.6e-7). Before,
-// 128 x 128 outputs in four waves, both operands through LDS, splits and products in turn: us of the product of M x N x K, before ->
-// here, 600 x 32000 x 4096 935 -> 856, 1500 2162 -> 1890, 128 248 -> 196, 400 x 14600 x 2048 172 -> 150, 200 x 11264 x 2048 91 -> 77, 64 x
-// 2048 x 2048 19 -> 16. Both operands through LDS in this order: 5 % slower.
+// One workgroup: 128 x 256 outputs in eight waves (two per SIMD) or 64 x 128 in four; a wave has all rows and 32 columns. K
+// advances 32 per step. The operands are split on their way (6 vector instructions per number), so memory holds plain fp32 and
+// nothing is prepared ahead: the activations through LDS, in two images, a wave's own weights straight into the layout of the
+// matrix instruction. LDS: per part [rows][4 cells of 16 B], cell c of row r at c ^ (r & 8 ? 3 : 0): a read of 16 bytes per
+// lane takes lanes 0-3, 12-15, 20-23, 24-27 together (then 4-11, 16-19, 28-31, and so above 32), which fall on all 64 banks (c
+// ^ ((r >> 2) & 3): half of the reads' cycles were conflicts). What bounds it: the matrix cores at 70 % of their cycles and a
+// clock held at 1.95 GHz by power. Each product is followed by the few vector instructions that fit beside it, the one barrier
+// of a step lies where the next products' operands are on their way, and a step's six products start from zero, so that the
+// running sums are rounded once per step and not 24 times (4 vector additions per tile, 5 % of the time; relative error of
+// normal numbers, K 4096 in one chain 1.0e-6 -> 2.2e-7, K 2048 7.0e-7 -> 1.6e-7). Before, 128 x 128 outputs in four waves,
+// both operands through LDS, splits and products in turn: us of the product of M x N x K, before -> here, 600 x 32000 x 4096
+// 935 -> 856, 1500 2162 -> 1890, 128 248 -> 196, 400 x 14600 x 2048 172 -> 150, 200 x 11264 x 2048 91 -> 77, 64 x 2048 x 2048
+// 19 -> 16. Both operands through LDS in this order: 5 % slower.
 #pragma once
 #include <type_traits>
 #include "common.h"
