@@ -214,7 +214,7 @@ static void tc_segments(const LinScan& p, int& nseg, int& len) {
 bool hy_timemix_chunk_takes(const TimeMixChunk& p) {
   const LinScan& q = p.s;
   auto rows = [](const void* x, int ld) { return ((uintptr_t)x & 15) == 0 && ld % 4 == 0; };
-  return q.mode == 1 && q.dim == TC_D && q.vdim == TC_D && q.S > 1 && q.B <= 65535 && q.H <= 65535 && rows(q.q, q.ldq) && rows(q.k, q.ldk) &&
+  return q.mode == 1 && q.dim == TC_D && q.vdim == TC_D && q.S > 1 && q.B >= 1 && q.H >= 1 && q.B <= 65535 && q.H <= 65535 && rows(q.q, q.ldq) && rows(q.k, q.ldk) &&
          rows(q.v, q.ldv) && rows(q.decay, q.ldd) && rows(q.w0, 0) && rows(q.u, 0) && rows(q.state, 0) &&
          (p.norm ? rows(p.gate, p.ldg) && rows(p.w, 0) && p.ldo % 4 == 0 && ((uintptr_t)p.out & (p.out_bf16 ? 7 : 15)) == 0 : rows(q.o, 0));
 }

@@ -38,6 +38,13 @@ def test_chunks_as_token_by_token(b, s, h, shift):
         assert got is out and _rel(got, ref) < tol and _rel(dev_st, ref_st) < 2e-5
 
 
+def test_no_rows():
+    """An empty batch of a prompt gives an empty result (there are no heads to deal segments to)."""
+    x, st = _inputs(0, 5, 2)
+    got = hy.timemix_scan(*[t.to(DEV) for t in x], st.to(DEV), 0, 5)
+    assert got.shape == (0, 2, 64) and got.is_cuda
+
+
 @pytest.mark.parametrize("b,s,shift", [(1, 777, -3.0), (2, 130, -3.0), (1, 17, 0.0), (3, 64, 1.0), (1, 400, -5.0), (1, 1000, -2.0)])
 def test_no_less_exact_than_the_scan(b, s, shift):
     """Relative errors (2-norm) against 64 bits beside those of the token-by-token scan, which rows off 16 bytes still take. Both are
