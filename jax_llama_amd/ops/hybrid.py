@@ -1557,11 +1557,12 @@ def shifted_linears(h, prev: torch.Tensor, mu: torch.Tensor, parts) -> Optional[
             or any(w.dtype != BF16 for w, _, _ in parts) or not h.x.is_contiguous() or h.gain.numel() != h.x.shape[1]:
         return None
     m = h.x.shape[0]
-    flat = torch.empty(m * sum(w.shape[0] for w, _, _ in parts), dtype=F32, device=h.x.device)
+    sizes = [m * w.shape[0] for w, _, _ in parts]
+    flat = torch.empty(sum((n + 3) // 4 * 4 for n in sizes), dtype=F32, device=h.x.device)
     outs, at = [], 0
-    for w, _, _ in parts:
-        outs.append(flat[at:at + m * w.shape[0]].view(m, w.shape[0]))
-        at += m * w.shape[0]
+    for (w, _, _), n in zip(parts, sizes):
+        outs.append(flat[at:at + n].view(m, w.shape[0]))
+        at += (n + 3) // 4 * 4  # (every part starts on 16 bytes, whatever the widths before it)
     row = torch.empty_like(h.x)
     if ext().rows_parts(h.x, h.gain, h.eps, prev, mu, [w for w, _, _ in parts], [int(j) for _, j, _ in parts],
                         [float(c) for _, _, c in parts], outs, row):
@@ -1721,7 +1722,7 @@ def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre, w0: 
     h, dim, vdim = r.shape[1], r.shape[2], v.shape[2]
     to = _step_out(r, h * vdim, dim, vdim, s, out)
     pair = wpre if isinstance(wpre, tuple) else None
-    low = to is not None and pair is not None and pair[1].shape[1] % 4 == 0
+    low = to is not None and pair is not None and pair[1].shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in pair)
     if pair is not None and not low:
         wpre = linear(*pair).unflatten(1, (h, dim))
     if carry is not None and not low:

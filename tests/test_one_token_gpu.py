@@ -122,6 +122,28 @@ def test_time_mix_of_one_token_takes_its_decay_product(dt, b, h, dim, rank, widt
     assert torch.equal(p_dev.cpu(), row) and torch.equal(prev, row)
 
 
+@pytest.mark.parametrize("m,before", [(1, 194), (1, 1), (2, 67), (1, 64)])
+@pytest.mark.parametrize("moved", [False, True])
+def test_time_mix_behind_a_part_of_any_width(m, before, moved):
+    """The decay product's input from the joint launch behind a matrix whose row count is no multiple of four, and as a view that
+    does not start on 16 bytes: the same as from memory of its own."""
+    d, hd, rank = 256, (2, 64), 64
+    x, gain, prev, mu = _rand(m, d), torch.rand(d) + 0.5, _rand(m, d), torch.rand(2, d)
+    w_also, w1, w2 = _rand(before, d, dt=BF16), _rand(rank, d, dt=BF16, std=d ** -0.5), _rand(128, rank, dt=BF16, std=rank ** -0.5)
+    outs, _ = hy.shifted_linears(hy.RmsInput(x.to(DEV), gain.to(DEV), 1e-5), prev.to(DEV), mu.to(DEV),
+                                 [(w_also.to(DEV), -1, 0.0), (w1.to(DEV), 1, 1.0)])
+    z = outs[1]
+    if moved:
+        z = torch.zeros(m * rank + 2, device=DEV)[2:].view(m, rank).copy_(z)
+    r, k, v, w0, u, gate, w = _rand(m, *hd), _rand(m, *hd), _rand(m, *hd), _rand(*hd) - 2.0, _rand(*hd), _rand(m, 128), torch.rand(128)
+    st = _rand(m, 2, 64, 64)
+    s_dev, s_own = st.to(DEV), st.to(DEV)
+    args = [t.to(DEV) for t in (w0, u)]
+    got = hy.timemix_memory(*(t.to(DEV) for t in (r, k, v)), (z, w2.to(DEV)), *args, s_dev, m, 1, gate.to(DEV), w.to(DEV), 1e-5)
+    want = hy.timemix_memory(*(t.to(DEV) for t in (r, k, v)), (z.clone(), w2.to(DEV)), *args, s_own, m, 1, gate.to(DEV), w.to(DEV), 1e-5)
+    _close(got, want.cpu(), 2e-5, "output"), _close(s_dev, s_own.cpu(), 2e-5, "state")
+
+
 @pytest.mark.parametrize("b,h,g,dim,vdim", [(1, 4, 1, 128, 128), (2, 4, 2, 64, 64), (3, 3, 3, 40, 20), (1, 16, 4, 128, 128), (2, 6, 2, 200, 64),
                                             (1, 2, 1, 64, 256), (1, 2, 1, 256, 64), (70, 4, 2, 64, 64)])
 def test_delta_rule_of_one_token_from_its_projection(b, h, g, dim, vdim):
