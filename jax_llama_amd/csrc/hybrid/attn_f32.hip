@@ -6,8 +6,8 @@
 // 16-byte loads and step r of v_mfma_f32_16x16x4_f32 takes the numbers 16 i + 4 (lane >> 4) + r of both. Its result, keys
 // 4 (lane >> 4) + r of query lane & 15, is in place the B operand of O^T += V^T P^T with the keys in that order; value tile
 // (jj, e) holds the columns 64 jj + 4 row + e, so that values too come and go in 16-byte pieces.
-// Masked keys have weight 0; where a masked tile holds a value that is none, the value takes no part in the product and only the
-// queries that see its key get NaN in its column.
+// Masked keys have weight 0; where a masked tile holds a value that is not finite, the value takes no part in the product, and only
+// the queries that see its key get in its column what the product would give them: an infinity, or NaN.
 // What bounds it: the chain of a tile (32 + 32 matrix instructions, the softmax between them) over the keys / 64 tiles of a wave.
 // One wave per query that read every key for itself took 138 us for 400 tokens and 173 us for 200 tokens behind 400 (16 heads of 128).
 #include "attn_span.h"
@@ -126,15 +126,24 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(AttnBias p) {
       for (int j = 0; j < VT; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          f32x4 bad = {0.f, 0.f, 0.f, 0.f};  // keys without a number in this column that the query sees
+          f32x4 up = {0.f, 0.f, 0.f, 0.f}, down = up, none = up;  // how many such keys of this column the query sees
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const bool ok = isfinite(vc[j][r][e]);
-            bad = __builtin_amdgcn_mfma_f32_16x16x4f32(ok ? 0.f : 1.f, seen[r] ? 1.f : 0.f, bad, 0, 0, 0);
-            if (!ok) vc[j][r][e] = 0.f;
+            const float v = vc[j][r][e];
+            const bool inf = isinf(v);
+            const float weighed = sc[r] > 0.f ? 1.f : 0.f, lost = seen[r] && !(sc[r] > 0.f) ? 1.f : 0.f;  // (0 x an infinity)
+            up = __builtin_amdgcn_mfma_f32_16x16x4f32(inf && v > 0.f ? 1.f : 0.f, weighed, up, 0, 0, 0);
+            down = __builtin_amdgcn_mfma_f32_16x16x4f32(inf && v < 0.f ? 1.f : 0.f, weighed, down, 0, 0, 0);
+            none = __builtin_amdgcn_mfma_f32_16x16x4f32(inf ? 1.f : 0.f, lost, none, 0, 0, 0);
+            none = __builtin_amdgcn_mfma_f32_16x16x4f32(isnan(v) ? 1.f : 0.f, seen[r] ? 1.f : 0.f, none, 0, 0, 0);
+            if (!isfinite(v)) vc[j][r][e] = 0.f;
           }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[j][e][r] = bad[r] > 0.f ? NAN : o[j][e][r];
+          for (int r = 0; r < 4; ++r) {
+            o[j][e][r] += up[r] > 0.f ? INFINITY : 0.f;
+            o[j][e][r] += down[r] > 0.f ? -INFINITY : 0.f;
+            o[j][e][r] = none[r] > 0.f ? NAN : o[j][e][r];
+          }
         }
     }
 #pragma unroll

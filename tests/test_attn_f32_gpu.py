@@ -48,3 +48,28 @@ def test_a_number_that_is_none_reaches_no_query_before_it(where, bad):
         got, want = _both(q, kc, vc, 0, 0.125)
         ok = torch.isfinite(want)
     assert torch.equal(torch.isfinite(got), ok) and float((got - want)[ok].abs().max()) < 2e-5 * float(want[ok].abs().max())
+
+
+@pytest.mark.parametrize("at", [5, 37, 69])
+@pytest.mark.parametrize("bad", [(float("inf"), float("inf")), (float("-inf"), float("inf")), (float("nan"), float("inf"))])
+@pytest.mark.parametrize("window", [0, 20])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_a_value_without_end_is_the_same_in_every_tile(at, bad, window, dim):
+    """What a query gets that sees one or both of two keys whose values are not finite in a column: the infinity, NaN where they
+    are of both signs or one is NaN, wherever the keys lie in tiles of 16 with and without hidden keys. Queries that see neither,
+    and the other columns, as without them."""
+    s, h = 90, 2
+    q, kc, vc = torch.randn(1, s, h, dim) * 0.1, torch.randn(1, 1, s, dim), torch.randn(1, 1, s, dim)
+    held = vc.clone()
+    for j, x in zip((at, at + 7), bad):
+        held[0, 0, j, 3], vc[0, 0, j, 3] = x, 0.0
+    kw = dict(window=window) if window else {}
+    want = hy.attn_bias(q, kc, vc, 0, dim ** -0.5, **kw).view(s, h, dim)
+    for i in range(s):
+        seen = [x for j, x in zip((at, at + 7), bad) if j <= i and (not window or i - j < window)]
+        if seen:
+            want[i, :, 3] = sum(seen)
+    got = _both(q, kc, held, 0, dim ** -0.5, **kw)[0].view(s, h, dim)
+    ok = torch.isfinite(want)
+    assert torch.equal(torch.nan_to_num(got, 7e30, 8e30, 9e30)[~ok], torch.nan_to_num(want, 7e30, 8e30, 9e30)[~ok])
+    assert torch.equal(torch.isfinite(got), ok) and float((got - want)[ok].abs().max()) < 2e-5 * float(want[ok].abs().max())
