@@ -10,6 +10,9 @@
 // the queries that see its key get in its column what the product would give them: an infinity, or NaN.
 // What bounds it: the chain of a tile (32 + 32 matrix instructions, the softmax between them) over the keys / 64 tiles of a wave.
 // One wave per query that read every key for itself took 138 us for 400 tokens and 173 us for 200 tokens behind 400 (16 heads of 128).
+// Two workgroups share a compute unit (208 registers at 128 x 128). The column that counts in a masked tile keeps two sums and not a
+// count of its own per kind: with three the kernel took 255 and one workgroup, 13 rows x 32 heads x 64 tokens behind 400 129 us
+// instead of 101, 200 tokens behind 400 of one row x 32 heads 44 instead of 38.
 #include "attn_span.h"
 
 namespace jla {
@@ -126,23 +129,23 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(AttnBias p) {
       for (int j = 0; j < VT; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          f32x4 up = {0.f, 0.f, 0.f, 0.f}, down = up, none = up;  // how many such keys of this column the query sees
+          // of this column the query sees: infinities (those below in units of 32, a tile has 16 keys), and products that are none
+          f32x4 ends = {0.f, 0.f, 0.f, 0.f}, none = ends;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float v = vc[j][r][e];
-            const bool inf = isinf(v);
-            const float weighed = sc[r] > 0.f ? 1.f : 0.f, lost = seen[r] && !(sc[r] > 0.f) ? 1.f : 0.f;  // (0 x an infinity)
-            up = __builtin_amdgcn_mfma_f32_16x16x4f32(inf && v > 0.f ? 1.f : 0.f, weighed, up, 0, 0, 0);
-            down = __builtin_amdgcn_mfma_f32_16x16x4f32(inf && v < 0.f ? 1.f : 0.f, weighed, down, 0, 0, 0);
-            none = __builtin_amdgcn_mfma_f32_16x16x4f32(inf ? 1.f : 0.f, lost, none, 0, 0, 0);
+            const float v = vc[j][r][e], end = isinf(v) ? (v > 0.f ? 1.f : 32.f) : 0.f;
+            const bool weighed = sc[r] > 0.f;
+            ends = __builtin_amdgcn_mfma_f32_16x16x4f32(end, weighed ? 1.f : 0.f, ends, 0, 0, 0);
             none = __builtin_amdgcn_mfma_f32_16x16x4f32(isnan(v) ? 1.f : 0.f, seen[r] ? 1.f : 0.f, none, 0, 0, 0);
+            none = __builtin_amdgcn_mfma_f32_16x16x4f32(end, seen[r] && !weighed ? 1.f : 0.f, none, 0, 0, 0);  // (0 x an infinity)
             if (!isfinite(v)) vc[j][r][e] = 0.f;
           }
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            o[j][e][r] += up[r] > 0.f ? INFINITY : 0.f;
-            o[j][e][r] += down[r] > 0.f ? -INFINITY : 0.f;
-            o[j][e][r] = none[r] > 0.f ? NAN : o[j][e][r];
+            const int n = (int)ends[r];
+            if (n & 31) o[j][e][r] += INFINITY;
+            if (n >> 5) o[j][e][r] -= INFINITY;
+            if (none[r] > 0.f) o[j][e][r] = NAN;
           }
         }
     }
