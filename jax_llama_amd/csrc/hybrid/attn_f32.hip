@@ -10,9 +10,10 @@
 // the queries that see its key get in its column what the product would give them: an infinity, or NaN.
 // What bounds it: the chain of a tile (32 + 32 matrix instructions, the softmax between them) over the keys / 64 tiles of a wave.
 // One wave per query that read every key for itself took 138 us for 400 tokens and 173 us for 200 tokens behind 400 (16 heads of 128).
-// Two workgroups share a compute unit (208 registers at 128 x 128). The column that counts in a masked tile keeps two sums and not a
-// count of its own per kind: with three the kernel took 255 and one workgroup, 13 rows x 32 heads x 64 tokens behind 400 129 us
-// instead of 101, 200 tokens behind 400 of one row x 32 heads 44 instead of 38.
+// Two workgroups share a compute unit (three at 64 x 64), with their accumulators among the vector unit's registers, which rescale
+// them (231 at 128 x 128): a column that counts in a masked tile keeps two sums and not one per kind. With three sums the kernel took
+// 254 and half of its accumulators, one workgroup: 13 rows x 32 heads x 64 tokens behind 400 129 us, 101 without bounds on the
+// registers; over 2 to 400 tokens behind 0 to 1500 of one row x 16 heads of 128 9 % and 6 % more time than here, 32 x 32 36 % and 1 %.
 #include "attn_span.h"
 
 namespace jla {
@@ -20,7 +21,7 @@ namespace jla {
 constexpr int AF_Q = 16, AF_K = 16;
 
 template <int DK, int VT>  // dim = 16 DK, vdim = 64 VT
-__global__ void __launch_bounds__(256) attn_f32_kernel(AttnBias p) {
+__global__ void __launch_bounds__(256, DK == 4 && VT == 1 ? 3 : 2) attn_f32_kernel(AttnBias p) {
   constexpr int dim = 16 * DK, vdim = 64 * VT, PITCH = vdim + 4;
   __shared__ __attribute__((aligned(16))) float os[4][AF_Q][PITCH];
   __shared__ float ms[4][AF_Q], ls[4][AF_Q];
