@@ -184,9 +184,20 @@ __global__ void __launch_bounds__(256, DK == 4 && VT == 1 ? 3 : 2) attn_f32_kern
   }
 }
 
+// Two to four queries per row over a few keys leave most of a 16 x 16 tile idle; where the workgroups take more than a round (two per
+// compute unit, three at 64 x 64) they stay with a wave per query. Us, that | here, heads of 128, soft cap and bias (without), rows x heads:
+// 13 x 32, 2 queries over 2 keys 6.5 | 6.8 (6.4 | 6.3); 64 x 32, 2 queries over 2 | 32 | 62 | 122 keys 9.4 | 18 | 30 | 56, here 24 | 31 | 41 |
+// 67 (9.3 | 18 | 29 | 55, 22 | 26 | 33 | 49); 4 over 4 | 34 | 64 15 | 32 | 46, 25 | 36 | 41; 6 over 6 28 | 26, 8 over 8 30 | 27. Heads of
+// 64: 24 x 32, 4 over 4 6.3 | 5.9; 64 x 32, 2 over 2 | 62 6.8 | 17, 13 | 24. How many keys there are is known where the host knows the
+// slot.
+static bool af_few(const AttnBias& p) {
+  const long long most = (long long)p.S * p.t_cap, round = p.dim == 64 && p.vdim == 64 ? 768 : 512;
+  return p.S <= 4 && (long long)p.B * p.H > round && p.t_cap > 0 && most <= (p.bias && p.S == 2 ? 250 : 128);
+}
+
 bool hy_attn_f32_takes(const AttnBias& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  return !p.cbf16 && p.S > 1 && p.maps == 1 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.ldk == p.dim &&
+  return !p.cbf16 && p.S > 1 && !af_few(p) && p.maps == 1 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.ldk == p.dim &&
          p.ldv == p.vdim && aligned(p.q) && aligned(p.kc) && aligned(p.vc);
 }
 

@@ -1194,6 +1194,8 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
     e = ext()
     t_cap = int(max_kv) if max_kv is not None else kc.shape[2]
     ws, splits, vt = None, 1, None
+    if s > 1 and max_kv is None and not torch.is_tensor(slot):
+        t_cap = min(t_cap, int(slot) + s)  # (a slot that the host knows: so many keys at most)
     if s == 1:
         seen = min(t_cap, chunk) if chunk and chunk > 0 else (min(t_cap, window + keep_first) if window > 0 else t_cap)
         splits = int(e.attn_decode_splits(b, qh, seen))

@@ -73,3 +73,17 @@ def test_a_value_without_end_is_the_same_in_every_tile(at, bad, window, dim):
     ok = torch.isfinite(want)
     assert torch.equal(torch.nan_to_num(got, 7e30, 8e30, 9e30)[~ok], torch.nan_to_num(want, 7e30, 8e30, 9e30)[~ok])
     assert torch.equal(torch.isfinite(got), ok) and float((got - want)[ok].abs().max()) < 2e-5 * float(want[ok].abs().max())
+
+
+@pytest.mark.parametrize("s,s0,bias,dim", [(2, 62, False, 128), (2, 63, False, 128), (2, 123, True, 64), (2, 124, True, 64), (4, 28, False, 64), (4, 29, True, 128)])
+def test_a_few_queries_of_many_rows_in_either_form(s, s0, bias, dim):
+    """Slots that the host knows choose the form for a few queries over few keys, slots on the device never do: the same from both,
+    on either side of the rule's line, and as the CPU op."""
+    b, h, g = 200, 4, 2
+    q, kc, vc = torch.randn(b, s, h, dim), torch.randn(b, g, s0 + s + 3, dim), torch.randn(b, g, s0 + s + 3, dim)
+    kw = dict(softcap=20.0, bias=torch.randn(40, h)) if bias else {}
+    dev = {k: v.to(DEV) if torch.is_tensor(v) else v for k, v in kw.items()}
+    got = hy.attn_bias(q.to(DEV), kc.to(DEV), vc.to(DEV), s0, dim ** -0.5, **dev).cpu()
+    tiles, want = _both(q, kc, vc, s0, dim ** -0.5, **kw)
+    for y in (got, tiles):
+        assert float((y - want).abs().max() / want.abs().max()) < 2e-5
