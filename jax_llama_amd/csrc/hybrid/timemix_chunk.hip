@@ -17,6 +17,8 @@
 // segment on its staging and its lane exchanges. Errors against 64 bits, scan | here, output and state: 777 tokens, decays near
 // exp(-0.05) 1.12e-7, 9.0e-8 | 9.6e-8, 7.9e-8; 64 tokens near exp(-2.7) 8.2e-8, 3.7e-8 | 7.3e-8, 2.9e-8 (with 32-bit running
 // products, one chain per sum and 32-bit joins 1.32e-7, 1.0e-7 and 8.6e-8, 2.9e-8).
+// Two workgroups per compute unit: without that bound the form with the norm took 181 registers and as many accumulators as held it to
+// one, and 200 rows x 32 heads x 2 tokens took 153 us where the scan had taken 147; with it 101 (1500 tokens of 8 rows 575 -> 465).
 #include "hy_util.h"
 #include "hybrid.h"
 
@@ -32,7 +34,7 @@ JLA_DEV float tc_dot(const f32x4 a, const f32x4 b) { return fmaf(a[0], b[0], a[1
 
 // grid (segments, H, B); NORM: the gated head norm is applied and p.out written, else the read-out to p.s.o
 template <int STATE_ONLY, int NORM>
-__global__ void __launch_bounds__(256) timemix_chunk_kernel(TimeMixChunk p, const float* s_init, float* s_final, float* seg_decay) {
+__global__ void __launch_bounds__(256, 2) timemix_chunk_kernel(TimeMixChunk p, const float* s_init, float* s_final, float* seg_decay) {
   __shared__ __attribute__((aligned(16))) float R[TC_C][TC_P], V[TC_C][TC_Q], W[TC_C][TC_P], RT[TC_C][TC_P], KT[TC_C][TC_Q],
       O[TC_C][TC_P], PM[TC_C][20], all[TC_D];
   const LinScan& q = p.s;
@@ -197,9 +199,10 @@ __global__ void __launch_bounds__(256) timemix_combine_kernel(const f32x4* state
   }
 }
 
-// Segments of at least a chunk, up to two workgroups per compute unit. Us, scan | here: 1 x 32 heads, 777 | 400 | 200 | 100 tokens 118 |
-// 55, 117 | 35, 114 | 26, 83 | 23 (segments of at least 32 tokens: 55, 39, 31, 30); 2500 tokens 260 | 118; 8 rows x 64 heads of 1500
-// tokens, one segment each, 1207 | 634.
+// Segments of at least a chunk, up to two workgroups per compute unit (segments of at least 32 tokens: 777 | 400 | 200 | 100 tokens of one row
+// x 32 heads 55 | 39 | 31 | 30 us, here 55 | 35 | 25 | 23). Us with the norm behind it, scan | here: 1 x 32 heads, 2 | 16 | 32 | 200 | 777 | 1500 tokens
+// 14 | 25 | 36 | 119 | 127 | 181, 8 | 8 | 15 | 25 | 55 | 77; 8 x 32, one segment from 512 workgroups on, 2 | 32 | 1500 tokens 15 | 38 | 1234, 8 | 25 | 465;
+// 200 x 32, 2 | 3 | 16 | 32 tokens 147 | 154 | 307 | 490, 101 | 101 | 102 | 181. So every prompt of two tokens and more is taken.
 constexpr int TC_TARGET = 512, TC_SEG_MIN = 16;
 
 static void tc_segments(const LinScan& p, int& nseg, int& len) {
