@@ -392,7 +392,10 @@ int hy_gated_rmsnorm(const GatedNorm& p, hipStream_t s) {
   if (p.gate_act != 2 && (!p.gate || p.ldg < p.H * p.vdim)) return -1;
   if (p.M == 0) return 0;
   if ((p.H + 3) / 4 > 65535) return -2;
-  const int L = p.denom_floor || p.ldo % 4 || (p.gate_act != 2 && p.ldg % 4) ? 0 : hy_head_lanes(p.vdim);
+  int L = p.denom_floor || p.ldo % 4 || (p.gate_act != 2 && p.ldg % 4) ? 0 : hy_head_lanes(p.vdim);
+  // (few heads of up to 64 numbers are over before the wider accesses pay: us, a wave per head | here, heads of 64, 32 of them 2.2 | 2.5, 256 2.4 |
+  // 2.6, 2048 2.5 | 2.7, 4096 2.8 | 2.8, 8192 3.8 | 3.0; heads of 128 from the first on, 4 of them 2.5 | 2.4)
+  if (L == 16 && (long long)p.M * p.H < 4096) L = 0;
   const uintptr_t at = (uintptr_t)p.o | (uintptr_t)p.w | (uintptr_t)(p.gate_act != 2 ? p.gate : nullptr);
   if (L && !(at & 15) && !((uintptr_t)p.out & (p.out_bf16 ? 7 : 15)) && (long long)p.M * p.H <= 0x7fffffffLL) {
     if (p.out_bf16) gated_rmsnorm_vec<bf16_t>(p, L, s);

@@ -51,6 +51,13 @@ def test_gated_rmsnorm(vdim, m, h, act, dt, col):
     assert float(((got - want).abs() / want.abs().clamp_min(1e-6)).max()) <= (TOL if dt == torch.float32 else 2.0 ** -8 + TOL)
 
 
+@pytest.mark.parametrize("vdim,m,h", [(64, 1365, 3), (64, 1366, 3), (60, 4096, 1), (4, 820, 5)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_gated_rmsnorm_of_many_narrow_heads(vdim, m, h, dt):
+    """Heads of up to 64 numbers on either side of the 4096 heads from which they run in groups of lanes."""
+    test_gated_rmsnorm(vdim, m, h, hy.GATE_SILU, dt, 4)
+
+
 @pytest.mark.parametrize("m,d", [(256, 264), (300, 1024), (256, 4096), (257, 8200), (256, 200)])
 @pytest.mark.parametrize("nsum", [1, 2])
 def test_residual_as_an_operand(m, d, nsum):
