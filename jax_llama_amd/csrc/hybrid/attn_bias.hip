@@ -920,7 +920,7 @@ __global__ void __launch_bounds__(256, DK <= 8 ? 2 : 1) attn_bias_mma_kernel(Att
   am_store<VT>(p, o, m, h, hi, inv);
 }
 
-// Key widths of 64 and 128, more than a few queries: four waves with neighbouring query tiles of a head share its key tiles, 64 keys at a time, staged by LDS-DMA into one
+// Key widths of 64 and 128, more queries than one tile per head: four waves with neighbouring query tiles of a head share its key tiles, 64 keys at a time, staged by LDS-DMA into one
 // of two buffers while the other is used. Straight from the caches (the kernel above) a wave's operand load touches 32 lines for 32
 // bytes each, which is what bounds it once every SIMD has waves: 512 line accesses per tile and wave; staged, a line is fetched once
 // per workgroup. Images: key rows of 16 DK numbers, chunk c (16 bytes) of row r at c ^ swizzle(r), value rows (64 keys) likewise.
@@ -1015,9 +1015,20 @@ __global__ void __launch_bounds__(256 * KS, 2) attn_bias_lds_kernel(AttnBias p, 
 
 // Query tiles up to which they share the chip by their keys: four ways (measured us, four ways / two ways / one: 400 tiles 28 / 33 / 37,
 // 768 tiles 38 / 29 / 30, 1024 tiles 105 / 91 / 119), then two ways (2048 tiles 115 / 95 / 92, 4096 tiles 254 / 165 / 165,
-// 6032 tiles 305 / 238 / 203). Key widths that are not staged (measured on heads of 128
-// without the staging, four ways / one): 105 / 135 at 1024 tiles, 254 / 236 at 4096.
-constexpr long long AM_SPLIT4 = 512, AM_SPLIT2 = 1536, AM_SPLIT4_DIRECT = 1024;
+// 6032 tiles 305 / 238 / 203). Heads of 64 x 64 have half the bytes to stage and gain nothing from two ways: rows x heads x queries
+// behind 0 | 400 | 1500 keys, 9 x 32 x 64 13 | 26 | 59 four ways, 16 | 43 | 105 two ways, 9 x 32 x 128 (1152 tiles) 21 | 39 | 88, 24 | 52 | 115
+// and one way 19 | 48 | 116; the kernel before these 14 | 53 | 156 and 23 | 64 | 166; keys of a single staged step one way (9 x 32 x 64 behind
+// none 12, four ways 13). Key widths that are not staged (measured on heads of
+// 128 without the staging, four ways / one): 105 / 135 at 1024 tiles, 254 / 236 at 4096.
+constexpr long long AM_SPLIT4 = 512, AM_SPLIT2 = 1536, AM_SPLIT4_NARROW = 1024, AM_SPLIT4_DIRECT = 1024;
+// A head of one query tile has nobody to share staged keys with, three of four waves would walk along: over few keys a wave takes its
+// tile directly, over many, or as many as the host does not know, four waves share it by its keys. Us, directly | four ways | two ways (one
+// way from 2048 tiles on) | before, soft cap and bias, 2 queries behind 0 | 60 | 400 | 1500 keys: 18 x 32 heads of 128 12, 14, 39, 120 | 15, 17,
+// 38, 109 | 27, 29, 71, 193 | 26, 35, 130, 439; 64 x 32 25, 33, 98, 458 | 32, 38, 91, 425 | 38, 46, 135, 507 | 69, 93, 347, 1355; 30 x 32
+// heads of 64 10, 13, 37, 107 | 12, 14, 32, 84 | 22, 24, 69, 196 | 12, 16, 53, 167; 9 x 32 heads of 64, 32 queries 9, 11 | 11, 12 | - | 10, 16;
+// 20 x 32 of 80 x 64, 32 queries behind none 12 | 14 | - | 12.
+constexpr long long AM_ALONE = 256;
+constexpr int AM_ALONE_KEYS = 256;
 
 template <int DK, int VT>
 static int am_launch(const AttnBias& p, bf16_t* vt, int Tp, hipStream_t s) {
@@ -1026,12 +1037,15 @@ static int am_launch(const AttnBias& p, bf16_t* vt, int Tp, hipStream_t s) {
   JLA_CHECK_LAUNCH();
   const long long hb = (long long)p.H * p.B;
   const long long tiles = (p.S + AM_Q - 1) / AM_Q * hb;
-  constexpr bool staged = DK == 4 || DK == 8;
+  constexpr bool staged = DK == 4 || DK == 8, narrow = DK == 4 && VT == 2;
   const unsigned g4 = (unsigned)((p.S + 4 * AM_Q - 1) / (4 * AM_Q) * hb);
   if (p.maps == 2) attn_bias_mma_kernel<DK, VT, 2, 1><<<(unsigned)((p.S + 63) / 64 * hb), 256, 0, s>>>(p, vt, Tp);
-  else if (tiles <= (staged ? AM_SPLIT4 : AM_SPLIT4_DIRECT)) attn_bias_mma_kernel<DK, VT, 1, 4><<<(unsigned)tiles, 256, 0, s>>>(p, vt, Tp);
+  else if (p.S <= AM_Q && tiles > AM_ALONE && p.t_cap <= AM_ALONE_KEYS)
+    attn_bias_mma_kernel<DK, VT, 1, 1><<<g4, 256, 0, s>>>(p, vt, Tp);
+  else if (tiles <= (narrow && p.t_cap > AL_KEYS ? AM_SPLIT4_NARROW : (staged ? AM_SPLIT4 : AM_SPLIT4_DIRECT)) || (staged && p.S <= AM_Q))
+    attn_bias_mma_kernel<DK, VT, 1, 4><<<(unsigned)tiles, 256, 0, s>>>(p, vt, Tp);
   else if constexpr (!staged) attn_bias_mma_kernel<DK, VT, 1, 1><<<g4, 256, 0, s>>>(p, vt, Tp);
-  else if (tiles <= AM_SPLIT2) attn_bias_lds_kernel<DK, VT, 2><<<g4, 512, 0, s>>>(p, vt, Tp);
+  else if (!narrow && tiles <= AM_SPLIT2) attn_bias_lds_kernel<DK, VT, 2><<<g4, 512, 0, s>>>(p, vt, Tp);
   else attn_bias_lds_kernel<DK, VT, 1><<<g4, 256, 0, s>>>(p, vt, Tp);
   JLA_CHECK_LAUNCH();
   return 0;

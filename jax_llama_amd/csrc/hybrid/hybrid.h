@@ -308,7 +308,7 @@ struct AttnBias {
   void* out;   // [B * S, H * vdim] fp32, or (out_bf16) bf16; rows ldo apart
   int ldo;
   int out_bf16;
-  int t_cap;   // keys the launch may have to cover (the form of a prompt over fp32 caches); <= T
+  int t_cap;   // keys the launch may have to cover (which form a prompt takes); <= T
   float* ws;   // decode split partials: B * H * splits * (vdim + 2) floats
   int splits;
   void* vt_ws;  // prefill: hy_attn_prefill_ws_bytes(...) bytes for the transposed values (nullptr: the plain kernel)
