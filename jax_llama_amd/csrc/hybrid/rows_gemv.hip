@@ -647,9 +647,16 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // unit 4.6), four rows 5.5 -> 3.6; weights in a cache, one row 4.3 -> 3.3 (3.5); K 4096 5.9 -> 6.8.
   const long long all = tiles * groups;
   int nt = gated || mt > 1 || all >= (G == 4 ? (p.K <= RV_PAIR_K ? 256 : 1024) : 512) ? 2 : 1;
-  // Rows by expert, four tiles from 2048 on (us, two | four tiles: 16 rows, 8 experts, K 7168 x N 4096 84 | 76, 3 rows 34 | 30, K 2816 x
-  // N 2048 16 rows 22.4 | 19.0, 3 rows 9.7 | 10.4).
-  if (all >= (G > 4 || gated || p.offs ? 2048 : 12288)) nt = 4;
+  // Rows by expert, up to four per expert: four tiles from 4096 on where the experts have rows (two per expert on average or as many each; one
+  // on average from 512 tiles per expert on), with two per expert and K from 2560 on from 2048; not on weights 4 KiB apart (8 KiB: with two),
+  // which share their memory channels. Fewer rows leave too many experts, and workgroups, without work. Us, two | four tiles, 8 experts: 16
+  // rows, K 1024 | 2816 | 7168 x N 2048 10.3 | 21.5 | 44, 8.8 | 18.6 | 39, N 1024 6.4 | 12.8 | 24.1, 6.3 | 11.5 | 22.4, K 2048 16.0 | 16.4 and 9.2 | 9.9;
+  // 8 rows, K 1024 | 2048 | 2816 | 7168 x N 2048 8.1 | 11.9 | 16.0 | 33.2, 7.3 | 13.2 | 15.2 | 30.5; 16 of 16 experts, K 2816 x N 1024 16.6 | 17.2; one
+  // row each, K 128 | 512 x N 2048 5.7 | 8.8, 4.3 | 7.4, N 1024 3.7 | 5.4, 3.7 | 5.5; 3 rows in all, K 2816 | 7168 x N 2048 9.2 | 17.4, 10.1 | 19.8, 4
+  // rows x N 1024 7.2 | 12.6, 9.8 | 18.2. 16 rows, K 7168 x N 4096 84 | 75.
+  const bool pairs = p.R >= 2LL * p.E, wide = p.K % 2048 != 0 && (even > 0 || (p.R >= p.E && tiles >= 512));
+  const bool filled = p.offs && ((all >= 4096 && (wide || (pairs && p.K != 2048))) || (all >= 2048 && pairs && p.K >= 2560));
+  if (all >= (G > 4 || gated ? 2048 : 12288) || filled) nt = 4;
   const long long wgs = (tiles + nt - 1) / nt;
   if (wgs > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)wgs, groups);

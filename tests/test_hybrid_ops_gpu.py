@@ -554,6 +554,23 @@ def test_few_rows_on_wide_outputs(r, k, n, e, gated):
     assert bool((out[:, n:] == 0.25).all())
 
 
+@pytest.mark.parametrize("r,e,k,n,even", [(16, 8, 264, 2050, 0), (16, 8, 264, 2044, 0), (8, 8, 264, 2050, 0), (7, 8, 264, 2050, 0), (8, 8, 2048, 2050, 0), (16, 8, 2560, 1027, 0), (16, 8, 2552, 1027, 0),
+                                          (8, 8, 136, 2049, 1), (8, 8, 136, 2044, 1), (32, 8, 72, 2051, 4), (4, 2, 264, 8197, 0)])
+def test_a_few_rows_of_every_expert(r, e, k, n, even):
+    """Up to four rows per expert: four column tiles per workgroup on both sides of the rule's lines (tiles in all, one and two rows
+    per expert on average, K, as many rows each), ragged last tiles."""
+    g = torch.Generator(device=DEV).manual_seed(r + n)
+    w = (torch.randn(e, n, k, generator=g, device=DEV) * k ** -0.5).to(torch.bfloat16)
+    x = torch.randn(r, k, generator=g, device=DEV)
+    ex = torch.arange(r, device=DEV) // even if even else torch.randint(0, e, (r,), generator=g, device=DEV).sort().values
+    offs = torch.tensor([int((ex < i).sum()) for i in range(e + 1)], dtype=torch.int32, device=DEV)
+    ref = torch.stack([x[i].to(torch.bfloat16).float() @ w[int(ex[i])].float().t() for i in range(r)])
+    out = torch.full((r, n + 4), 0.25, device=DEV)
+    hy.ext().linear_rows(x, None, w, out[:, :n], None, offs, None, r, hy.ACT_NONE, 0.0, 1.0, None, None, 0.0, even, False)
+    _close(out[:, :n], ref, 2e-5, "rows by expert")
+    assert bool((out[:, n:] == 0.25).all())
+
+
 @pytest.mark.parametrize("r", [1, 2])
 @pytest.mark.parametrize("k,n,gated", [(4104, 516, False), (4104, 4100, False), (4104, 49156, False), (4104, 2052, True), (4104, 4100, True)])
 def test_normed_rows_too_long_to_walk(r, k, n, gated):
