@@ -95,7 +95,7 @@ class KVCacheRows:
         return self.parent.k[i, self.b0:self.b1], self.parent.v[i, self.b0:self.b1]
 
 
-TICKET_INTS = 64 * 32  # tickets of a cache row: 64, each on a line of its own (csrc: AS_TICKET)
+TICKET_INTS = 64 * 32  # tickets of a cache row that has some: 64, each on a line of its own (csrc: AS_TICKET)
 
 
 class HybridCache:
@@ -135,8 +135,17 @@ class HybridCache:
         self.index = 0
         self.index_t = torch.zeros(1, dtype=torch.int32, device=device)
         # counters of the one-launch decode steps (ops.hybrid.attn_step, delta_step), which leave them at zero: part of the cache because
-        # two steps on one cache are never in flight at once
-        self.tickets = torch.zeros(batch_size * TICKET_INTS, dtype=torch.int32, device=device)
+        # two steps on one cache are never in flight at once. None where no layer takes those steps
+        self._row_tickets = self.tickets_per_row(self.specs)
+        self.tickets = torch.zeros(batch_size * self._row_tickets, dtype=torch.int32, device=device) if self._row_tickets else None
+
+    @staticmethod
+    def tickets_per_row(specs) -> int:
+        """Counters (int32) of a cache row: for key / value heads of 64 or 128 numbers and delta rules of four taps, else none."""
+        sizes = (64, 128)
+        some = any(sp[0] == "kv" and sp[2] in sizes and sp[3] in sizes or sp[0] == "delta" and sp[5] == 4
+                   for layer in specs for sp in HybridCache.parts(layer))
+        return TICKET_INTS if some else 0
 
     @staticmethod
     def parts(sp) -> list:
@@ -215,7 +224,8 @@ class HybridCache:
     def clear(self) -> None:
         """``reset`` and zero the keys and values too (after a failed step may have left non-finite rows)."""
         self.reset()
-        self.tickets.zero_()
+        if self.tickets is not None:
+            self.tickets.zero_()
         for t in {id(t): t for t in list(self._k.values()) + list(self._v.values())}.values():
             t.zero_()
 
@@ -224,13 +234,13 @@ class HybridCache:
 
     def nbytes(self) -> int:
         seen = {id(t): t for d in (self._k, self._v, self._state, self._conv) for t in d.values()}
-        return sum(t.numel() * t.element_size() for t in seen.values())
+        return sum(t.numel() * t.element_size() for t in seen.values()) + 4 * self.batch_size * self._row_tickets
 
     @staticmethod
     def bytes_per(specs, batch_size: int, max_length: int, dtype=torch.bfloat16) -> int:
         """Bytes a cache of this geometry takes (without allocating it)."""
         es = torch.empty(0, dtype=dtype).element_size()
-        n = 0
+        n = 4 * batch_size * HybridCache.tickets_per_row(specs)
         for layer in specs:
             for sp in HybridCache.parts(layer):
                 if sp[0] == "kv":
@@ -273,7 +283,8 @@ class HybridCacheRows:
 
     @property
     def tickets(self):
-        return self.parent.tickets[self.b0 * TICKET_INTS:self.b1 * TICKET_INTS]
+        per = self.parent._row_tickets
+        return self.parent.tickets[self.b0 * per:self.b1 * per] if per else None
 
     def layer(self, i: int):
         k, v = self.parent.layer(i)

@@ -608,3 +608,22 @@ def test_longer_prompts_at_the_kernel_shapes(dtype):
     assert e.mean() < (5e-5 if dtype == F32 else 1.5e-2), e.mean()
     whole = run_portions(model, t, [600])
     assert err(whole, got) < (2e-5 if dtype == F32 else 2e-2)
+
+
+@pytest.mark.parametrize("specs,counters", [([("kv", 2, 128, 64), ("mlstm", 2, 64, 64)], True), ([None, ("delta", 4, 2, 24, 24, 4)], True),
+                                            ([("delta", 4, 2, 24, 24, 3), ("latent", 40)], False),
+                                            ([("kv", 2, 64, 64), ("kv_from", 0)], True),
+                                            ([("multi", ("kv", 2, 64, 64), ("timemix", 3, 8, 8, 48))], True), ([("kv", 2, 12, 64)], False)])
+def test_a_cache_counts_all_that_it_holds(specs, counters):
+    """The bytes of a cache, held and foretold, with the counters of its one-launch steps, which exist where some layer takes them."""
+    cache = HybridCache(specs, 3, 10, "cpu", BF16)
+    held = {t.data_ptr(): t for v in vars(cache).values() for t in (v.values() if isinstance(v, dict) else [v]) if torch.is_tensor(t)}
+    n = sum(t.numel() * t.element_size() for t in held.values()) - 4  # (the slot index)
+    assert cache.nbytes() == HybridCache.bytes_per(specs, 3, 10, BF16) == n
+    assert (cache.tickets is not None) == counters and (cache.rows(1, 3).tickets is not None) == counters
+    if counters:
+        cache.tickets[:] = torch.arange(cache.tickets.numel())
+        per = cache.tickets.numel() // 3
+        assert torch.equal(cache.rows(1, 3).tickets, cache.tickets[per:])
+        cache.clear()
+        assert not cache.tickets.any()
