@@ -192,11 +192,11 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
     float sc = as_norm<ND>(qv, p.eps);
     if (p.temp_coef != 0.f) sc *= 1.f + p.temp_coef * logf((float)((pos + 1) / p.temp_every) + 1.f);
 #pragma unroll
-    for (int i = 0; i < ND; ++i) qv[i] = qv[i] * sc * (p.q_w ? p.q_w[lane + 64 * i] : 1.f);
+    for (int i = 0; i < ND; ++i) qv[i] *= sc;
     if (own && tail) {
-      const float sk = as_norm<ND>(kx, p.eps), sv = p.norm_v ? as_norm<VREG>(vx, p.eps) : 1.f;
+      const float sk = as_norm<ND>(kx, p.eps), sv = as_norm<VREG>(vx, p.eps);
 #pragma unroll
-      for (int i = 0; i < ND; ++i) kx[i] = kx[i] * sk * (p.k_w ? p.k_w[lane + 64 * i] : 1.f);
+      for (int i = 0; i < ND; ++i) kx[i] *= sk;
 #pragma unroll
       for (int i = 0; i < VREG; ++i) vx[i] *= sv;
     }
@@ -325,16 +325,13 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
     if (__builtin_amdgcn_readfirstlane(before) != groups - 1) return;
     asm volatile("" ::: "memory");
     if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // (one branch for all of it, as in ab_merge)
-    if (64 / WAVES > 32 && groups > 32) as_merge<64, VREG>(head, groups, lane, o);
-    else if (64 / WAVES > 16 && groups > 16) as_merge<32, VREG>(head, groups, lane, o);
+    // (one branch for all of it, as in ab_merge; one wave per workgroup: at most 16 splits, two: 64)
+    if (WAVES > 1 && groups > 16) as_merge<32, VREG>(head, groups, lane, o);
     else as_merge<16, VREG>(head, groups, lane, o);
   } else {
 #pragma unroll
     for (int i = 0; i < VREG; ++i) o[i] = acc[i] / l_run;
   }
-#pragma unroll
-  for (int i = 0; i < VREG; ++i) o[i] *= ab_gate(a, b, h, VREG * lane + i);
   if (ROPE && p.turn) {  // the summed values turned back by the query's position
     as_order();
 #pragma unroll
@@ -351,7 +348,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < VREG; ++i) ab_out(a, b, h, VREG * lane + i, o[i]);
+  for (int i = 0; i < VREG; ++i) reinterpret_cast<float*>(a.out)[(size_t)b * a.ldo + (size_t)h * vdim + VREG * lane + i] = o[i];
 }
 
 // Heads of 64 or 128 numbers, up to about a wave per SIMD: more waves share a SIMD, and then the preparation in
@@ -360,6 +357,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
 // 19.9 | 20.6, 8 x 32 x 8 34.4 | 38.7; rotations, 1 x 16 x 13 12.0 | 9.0, 2 x 32 x 16 14.1 | 11.0, 6 x 16 x 17 16.8 | 17.4, 4 x 32 x 16
 // 17.5 | 20.0.
 constexpr long long AS_MAX_WAVES = 1280;
+constexpr int AS_PAIR_SPLITS = 16;  // more of them: two per workgroup (hy_attn_step)
 
 bool hy_attn_step_takes(const AttnStep& p) {
   const AttnBias& a = p.a;
@@ -373,7 +371,7 @@ int hy_attn_step(const AttnStep& p, hipStream_t s) {
   if (a.B < 0 || a.H < 1 || a.G < 1 || a.H % a.G || a.T < 1 || !hy_attn_step_takes(p)) return -1;
   if (a.bias && a.nbias < 1) return -3;
   if (a.chunk < 0 || a.window < 0 || a.keep_first < 0 || (a.chunk > 0 && a.window > 0)) return -7;
-  if ((a.gate && a.ldg < (a.gate_cols ? a.H * a.vdim : a.H)) || a.ldo < a.H * a.vdim) return -8;
+  if (a.gate || a.out_bf16 || a.ldo < a.H * a.vdim) return -8;
   if (p.rope && (p.qk_half < 0 || 2 * p.qk_half > a.dim || p.v_half < 0 || 2 * p.v_half > a.vdim || !p.positions)) return -2;
   if (!p.rope && p.temp_coef != 0.f && (p.temp_every < 1 || !p.positions)) return -2;
   if (p.ld < a.H * a.dim + (p.own ? a.G * (a.dim + a.vdim) : 0)) return -4;
@@ -381,7 +379,7 @@ int hy_attn_step(const AttnStep& p, hipStream_t s) {
   if (a.B == 0) return 0;
   // Two splits per workgroup halve what a head publishes, from 17 splits on (33 splits, keys in no cache: a decode step with two of
   // these launches 241.8 -> 236.2 us; 2 splits alone 7.2 -> 8.7).
-  const int waves = a.splits > 16 ? 2 : 1;
+  const int waves = a.splits > AS_PAIR_SPLITS ? 2 : 1;
   const dim3 grid((a.splits + waves - 1) / waves, a.H, a.B);
 #define AS_ONE(DK8, VREG, ROPE)                                                                      \
   do {                                                                                               \

@@ -461,6 +461,7 @@ void gelu_gate_rows(Tensor gp, Tensor ids, Tensor table, int64_t col0, Tensor g)
 }
 
 void* slice2d_any(const Tensor& t, const char* name, int64_t rows, int64_t cols, int* ld, int* bf);
+float* slice2d(const Tensor& t, const char* name, int64_t rows, int64_t cols, int* ld);
 
 void glu_rows(Tensor gu, Tensor out, int64_t act, double limit, double alpha) {
   check(gu.dim() == 2 && out.dim() == 2 && gu.size(1) >= 2 * out.size(1) && jla::hy_act_gated(act),
@@ -734,8 +735,8 @@ void attn_bias(Tensor q, Tensor kc, Tensor vc, Tensor slot, double scale, double
 // One token of an attention layer in one launch; false (nothing done) where its shapes are not the kernel's.
 bool attn_step(Tensor proj, Tensor kc, Tensor vc, Tensor slot, Tensor positions, int64_t H, bool own, Tensor tickets, double scale,
                double softcap, OptT bias, Tensor out, int64_t seen, OptT sink, int64_t chunk, OptT head_scale, bool rope,
-               double eps, double temp_coef, int64_t temp_every, OptT q_w, OptT k_w, bool norm_v, OptT col_bias, OptT qk_freq,
-               OptT v_freq, bool turn, double turn_sign, double turn_gain) {
+               double eps, double temp_coef, int64_t temp_every, OptT col_bias, OptT qk_freq, OptT v_freq, bool turn,
+               double turn_sign, double turn_gain) {
   jla::AttnStep p{};
   jla::AttnBias& a = p.a;
   check(kc.dim() == 4 && vc.dim() == 4 && kc.size(0) == vc.size(0) && kc.size(1) == vc.size(1) && kc.size(2) == vc.size(2),
@@ -772,17 +773,9 @@ bool attn_step(Tensor proj, Tensor kc, Tensor vc, Tensor slot, Tensor positions,
     check(head_scale->numel() == H, "attn_step: one factor per head");
     a.head_scale = f32(*head_scale, "head_scale");
   }
-  a.out = slice2d_any(out, "out", a.B, (int64_t)H * a.vdim, &a.ldo, &a.out_bf16);
+  a.out = slice2d(out, "out", a.B, (int64_t)H * a.vdim, &a.ldo);
   p.rope = rope;
-  p.eps = eps; p.temp_coef = temp_coef; p.temp_every = temp_every; p.norm_v = norm_v;
-  if (q_w.has_value()) {
-    check(q_w->numel() == a.dim, "attn_step: q_w is [dim]");
-    p.q_w = f32(*q_w, "q_w");
-  }
-  if (k_w.has_value()) {
-    check(k_w->numel() == a.dim, "attn_step: k_w is [dim]");
-    p.k_w = f32(*k_w, "k_w");
-  }
+  p.eps = eps; p.temp_coef = temp_coef; p.temp_every = temp_every;
   if (col_bias.has_value()) {
     check(col_bias->numel() == H * a.dim + (int64_t)a.G * (a.dim + a.vdim), "attn_step: one bias per projection column");
     p.col_bias = f32(*col_bias, "col_bias");
@@ -1317,9 +1310,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_step", &attn_step, py::arg("proj"), py::arg("kc"), py::arg("vc"), py::arg("slot"), py::arg("positions"), py::arg("H"),
         py::arg("own"), py::arg("tickets"), py::arg("scale"), py::arg("softcap"), py::arg("bias"), py::arg("out"), py::arg("seen"),
         py::arg("sink") = py::none(), py::arg("chunk") = 0, py::arg("head_scale") = py::none(), py::arg("rope") = false,
-        py::arg("eps") = 0.0, py::arg("temp_coef") = 0.0, py::arg("temp_every") = 1, py::arg("q_w") = py::none(),
-        py::arg("k_w") = py::none(), py::arg("norm_v") = true, py::arg("col_bias") = py::none(), py::arg("qk_freq") = py::none(),
-        py::arg("v_freq") = py::none(), py::arg("turn") = false, py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
+        py::arg("eps") = 0.0, py::arg("temp_coef") = 0.0, py::arg("temp_every") = 1, py::arg("col_bias") = py::none(),
+        py::arg("qk_freq") = py::none(), py::arg("v_freq") = py::none(), py::arg("turn") = false, py::arg("turn_sign") = 1.0, py::arg("turn_gain") = 1.0);
   m.def("attn_prefill_ws_bytes", &attn_prefill_ws_bytes);
   m.def("timemix_norm", &timemix_norm);
   m.def("rows_parts", &rows_parts);

@@ -340,7 +340,7 @@ int hy_attn_decode_splits(int B, int H, int t_cap);
 constexpr int AS_TICKET = 32;  // int32s from a head's ticket to the next: counts on one line of memory go one behind the other
 
 // One token per row: hy_attn_prep or (rope) hy_rope_prep, the cache write, hy_attn_bias and its merge in one launch
-// (attn_step.hip). a: the arguments of hy_attn_bias without q and turn_*.
+// (attn_step.hip). a: the arguments of hy_attn_bias without q, gate and turn_*, fp32 out.
 struct AttnStep {
   AttnBias a;
   const float* proj;  // [B, ld]: q heads at column 0, then (own) k heads, then v heads
@@ -348,10 +348,8 @@ struct AttnStep {
   int own;            // the layer brings its own keys and values, which go to the cache at the slot
   const int32_t* positions;  // [B]
   int rope;
-  float eps, temp_coef;  // norms (rope = 0), as AttnPrep
-  int temp_every, norm_v;
-  const float* q_w;
-  const float* k_w;
+  float eps, temp_coef;  // norms of queries, keys and values (rope = 0), as AttnPrep without gains
+  int temp_every;
   const float* col_bias;  // rotations (rope = 1), as RopePrep
   const double* qk_freq;
   int qk_half;
