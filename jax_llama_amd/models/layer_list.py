@@ -172,7 +172,7 @@ class LayerListLM:
                 blk(r if getattr(blk, "takes_residual", False) else r.value(), ctx)
                 if collect_hidden:
                     hidden.append(r.value().reshape(b, s, d).clone())
-            if s == 1 and logits_mode == "argmax_parts" and not isinstance(self.final_norm, hy.SquashNorm):
+            if s == 1 and logits_mode == "argmax_parts" and not isinstance(self.final_norm, hy.SquashNorm) and hy.head_argmax_pays(b, self.head):
                 parts = hy.head_argmax(r, self.final_norm, self.eps, self.head, float(self.logit_softcap or 0.0))
                 if parts is not None:
                     return parts, r.x, hidden, []

@@ -681,7 +681,7 @@ class ArgmaxParts:
 
     @staticmethod
     def of(logits: torch.Tensor) -> Optional["ArgmaxParts"]:
-        """Of fp32 logits ``[B, V]`` in memory; None for more rows than one workgroup finishes."""
+        """Of fp32 logits ``[B, V]`` in memory, to finish like a product's; None for more rows than one workgroup finishes."""
         return ArgmaxParts(ext().argmax_parts(logits)) if 1 <= logits.shape[0] <= ArgmaxParts.MAX_ROWS else None
 
 

@@ -324,6 +324,13 @@ def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
     return linear(rms_rows(r.value() if r is not None else x, gain, eps), w, act=act, limit=cap)
 
 
+def head_argmax_pays(rows: int, w: torch.Tensor) -> bool:
+    """Whether ``head_argmax`` and its last reduction are faster than ``head_linear``, argmax and update. Us, logits written | not, K 2048: one
+    row x 8192 14.6 | 15.2, 16000 20.2 | 18.9, 32000 29.7 | 27.5, 128256 89.3 | 84.8; two rows x 4096 13.1 | 15.0, 32000 31.7 | 32.5, 128256
+    92.3 | 88.4 (the last reduction takes one row after the other)."""
+    return rows <= RESIDUAL_MAX_ROWS and w.shape[0] >= (12288 if rows == 1 else 65536)
+
+
 def head_argmax(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float = 0.0):
     """The greedy choice over ``head_linear(x, gain, eps, w, cap)`` as an ``ops.ArgmaxParts``, the logits never written; None where
     that is not one launch (more than two rows, fp32 weights, a short output)."""

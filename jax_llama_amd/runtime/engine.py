@@ -184,12 +184,11 @@ class DecodeEngine:
 
     def _decode_step(self):
         mode = self._logits_mode()
-        # greedy on one GPU: the choice's last reduction and the bookkeeping are one launch
+        # greedy on one GPU: a choice that a product left as partials is reduced by the launch that does the bookkeeping (logits in
+        # memory are not: their argmax and the update take 8.1 us for 1 x 32000, 12 for 256 x 32000, partials and that launch 8.6 and 22)
         joint = mode == "argmax" and self.device.type == "cuda" and self.model.comm.size == 1
         logits, *_ = self.model.forward_tokens(self.tokens, self.positions, self.cache, self.cache.index_t,
                                                self.kv_start, self.key_mask, logits_mode="argmax_parts" if joint else mode)
-        if joint and torch.is_tensor(logits):
-            logits = ops.ArgmaxParts.of(logits) or logits
         if isinstance(logits, ops.ArgmaxParts):
             ops.ext().argmax_next(logits.part, self.finished, self.sequences, self.cur_len, self.tokens, self.positions,
                                   self.cache.index_t, int(self.gc.pad_token_id), int(self.gc.eos_token_id))
