@@ -1723,6 +1723,12 @@ def mlstm_memory(proj: torch.Tensor, heads: int, dim: int, vdim: int, gate_bias:
     return gated_rmsnorm(o, gate, w, eps, GATE_SIGMOID, denom_floor=floor, gain=gain, out=out)
 
 
+# (row, head) pairs up to which a token's time mix takes its decay product into its own launch, a workgroup per pair: us, separate | inside,
+# heads of 64, rank 64, rows x heads 1 x 32 7.3 | 5.4, 20 x 32 13.0 | 11.2, 64 x 32 24.7 | 24.2, 64 x 64 38 | 42, 200 x 32 53 | 63; rank 256, 64 x 16
+# 18.0 | 15.4, 200 x 16 37 | 42
+TIMEMIX_LOW_PAIRS = 2048
+
+
 def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre, w0: torch.Tensor, u: torch.Tensor,
                    state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float, gain: float = 1.0,
                    out: Optional[torch.Tensor] = None, carry: Optional[tuple] = None) -> torch.Tensor:
@@ -1731,7 +1737,8 @@ def timemix_memory(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, wpre, w0: 
     h, dim, vdim = r.shape[1], r.shape[2], v.shape[2]
     to = _step_out(r, h * vdim, dim, vdim, s, out)
     pair = wpre if isinstance(wpre, tuple) else None
-    low = to is not None and pair is not None and pair[1].shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in pair)
+    low = to is not None and pair is not None and pair[1].shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in pair) \
+        and b * h <= TIMEMIX_LOW_PAIRS
     if pair is not None and not low:
         wpre = linear(*pair).unflatten(1, (h, dim))
     if carry is not None and not low:

@@ -206,3 +206,9 @@ def test_greedy_choice_inside_the_output_product(m, d, v, pending, cap):
     best = [max(((float(a), -int(i)) for a, i in zip(part[r, :, 0], part[r, :, 1].view(torch.int32)))) for r in range(m)]
     assert [-i for _, i in best] == ops.argmax(logits)[0].tolist()
     assert torch.equal(torch.tensor([a for a, _ in best]), logits.max(1).values.cpu()) and torch.equal(res[0].x, res[1].x)
+
+
+@pytest.mark.parametrize("b", [32, 33])
+def test_time_mix_of_many_rows_takes_its_decay_product_apart(b):
+    """On either side of the pairs from which the decay product is a launch of its own."""
+    test_time_mix_of_one_token_takes_its_decay_product(BF16, b, 64, 20, 12, 24)
