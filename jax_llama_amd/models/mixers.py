@@ -130,7 +130,7 @@ class GatedDeltaMixer:
         sp = self.spec
         proj = hy.linear(x, self.w_in)
         state, tail = ctx.cache.recurrent(self.i)
-        if ctx.s == 1:
+        if ctx.s == 1 and ctx.b * sp.heads <= hy.DELTA_STEP_PAIRS:
             y = hy.delta_step(proj, ctx.b, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w, tail, self.a_log, self.dt_bias, state,
                               self.norm_w, self.eps, ctx.tickets)
             if y is not None:

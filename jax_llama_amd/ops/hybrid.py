@@ -1365,6 +1365,13 @@ def delta_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.
     return out
 
 
+# (row, head) pairs up to which delta_step is faster than delta_prep and delta_memory, a workgroup per pair and compute unit: every head of a
+# key head prepares that head's keys again. Us, separate | one launch, heads of 128, four per key head, rows x heads 1 x 16 10.3 | 8.1, 8 x 32
+# 13.2 | 10.8, 20 x 16 15.2 | 16.5, 64 x 16 31 | 40, 200 x 32 180 | 251; own key heads 20 x 8 11.9 | 9.3, 64 x 8 19.2 | 19.5; heads of 64, two
+# per key head 64 x 4 8.7 | 7.6, 200 x 4 14.7 | 16.8
+DELTA_STEP_PAIRS = 256
+
+
 def delta_step(proj: torch.Tensor, b: int, heads: int, kv_heads: int, dim: int, vdim: int, conv_w: torch.Tensor, tail: torch.Tensor,
                a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, w: torch.Tensor, eps: float,
                tickets: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
