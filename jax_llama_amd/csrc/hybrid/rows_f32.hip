@@ -69,8 +69,12 @@ bool hy_rows_f32_takes(const RowLinear& p) {
 
 static F3Plan rows_f32_plan(const RowLinear& p) {
   const int E = p.offs ? p.E : 1;
-  auto tiles = [&](int bm) { return E == 1 ? (p.R + bm - 1LL) / bm : (p.R + bm / 2LL * E) / bm; };  // (on average)
-  return f3_plan(tiles, p.R, (hy_act_gated(p.act) ? 2LL : 1LL) * p.N, p.K);
+  auto tiles = [&](int bm) {  // (experts: on average, at least one each while there are rows)
+    if (E == 1) return (p.R + bm - 1LL) / bm;
+    const long long mean = (p.R + bm / 2LL * E) / bm, least = E < p.R ? E : p.R;
+    return mean > least ? mean : least;
+  };
+  return f3_plan(tiles, p.R, (hy_act_gated(p.act) ? 2LL : 1LL) * p.N, p.K, E < p.R ? E : p.R);
 }
 
 long long hy_rows_f32_floats(const RowLinear& p) {

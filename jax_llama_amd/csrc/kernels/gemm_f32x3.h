@@ -291,27 +291,34 @@ constexpr int f3_lds() {
 }
 
 // How a launch cuts its work: the tile and K over `splits` workgroups per tile, at least 8 steps each, whose partial sums go through
-// slabs [split][rows][cols] that the caller's second kernel adds in order. Measured: a step of 256 resident 128 x 256 tiles takes 2.05 us
-// and 5 once, one of 512 resident 64 x 128 tiles 1.33 us (0.75 if at most 256 run) and 4; the second kernel 4 us and the slabs' traffic.
+// slabs [split][rows][cols] that the caller's second kernel adds in order. The times are fitted to 3000 launches of 8 to 1500 rows, cols x K
+// from 64 x 2048 to 32000 x 4096, and choose within 0.2 % of the fastest on average: a step of up to 256 resident 64 x 128 tiles takes 1 us,
+// of up to 512 1.45 (1.36 in whole rounds), 3 once; of 256 128 x 256 tiles 2.04 and 5 once; the operands come at 4.6 TB/s at most, 3.2 with one
+// workgroup per compute unit; the second kernel 4.5 us and the slabs' traffic at 6.6 TB/s. (With 0.75 and 1.33 for the small tiles and no rate
+// of the operands 2.9 %: 777 x 2048 x 2048 61 us, here 52, 8 x 32000 x 4096 158 and 118.)
 struct F3Plan {
   int bm, bn, splits, steps;  // steps per split
 };
-template <class Tiles>  // (int height) -> row tiles
-inline F3Plan f3_plan(const Tiles& row_tiles, long long rows, long long cols, int K) {
+template <class Tiles>  // (int height) -> row tiles; matrices: of cols x K each
+inline F3Plan f3_plan(const Tiles& row_tiles, long long rows, long long cols, int K, int matrices = 1) {
   const int total = (K + F3_BK - 1) / F3_BK;
   F3Plan best{128, 256, 1, total};
   double least = 1e30;
   for (int bm = 64; bm <= 128; bm += 64) {
     const bool small = bm == 64;
-    const long long tiles = row_tiles(bm) * ((cols + 2 * bm - 1) / (2 * bm));
-    for (int splits = 1; splits <= 16 && (splits == 1 || total / splits >= 8); ++splits) {
-      const int steps = (total + splits - 1) / splits;
-      const long long n = tiles * splits, resident = small ? 512 : 256;
-      const double slab_us = splits == 1 ? 0. : 4. + (double)rows * cols * 4 * (2 * splits + 1) / 5e6;
-      const double us = (double)((n + resident - 1) / resident) * (steps * (small ? (n <= 256 ? 0.75 : 1.33) : 2.05) + (small ? 4. : 5.)) + slab_us;
-      if (us < 0.97 * least) {
+    // (of the launch: a multiple of 8 per split, and one without work that falls among the others' splits costs as much as one with)
+    const long long tiles = (row_tiles(bm) * ((cols + 2 * bm - 1) / (2 * bm)) + 7) / 8 * 8;
+    for (int cut = 1; cut <= 16 && (cut == 1 || total / cut >= 8); ++cut) {
+      const int steps = (total + cut - 1) / cut, splits = (total + steps - 1) / steps;
+      const long long n = tiles * splits, rest = n % 512;
+      double us = small ? (double)(n / 512) * (steps * 1.36 + 3.) + (rest ? steps * (rest <= 256 ? 1. : 1.45) + 3. : 0.)
+                        : (double)((n + 255) / 256) * (steps * 2.04 + 5.);
+      const double rate = small && n <= 256 ? 3.2e6 : 4.6e6, bytes = 4. * K * ((double)cols * matrices + (double)rows);
+      if (us < bytes / rate) us = bytes / rate;
+      if (splits > 1) us += 4.5 + (double)rows * cols * 4 * (2 * splits + 1) / 6.6e6;
+      if (us < 0.99 * least) {
         least = us;
-        best = {bm, 2 * bm, (total + steps - 1) / steps, steps};
+        best = {bm, 2 * bm, splits, steps};
       }
     }
   }
