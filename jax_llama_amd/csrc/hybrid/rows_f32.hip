@@ -1,7 +1,7 @@
 // The fp32 form of a prompt's row-gathered, expert-grouped linears: split products on the bf16 matrix cores
 // (kernels/gemm_f32x3.h) with the epilogues of a row linear. Us, exact-f32 MFMA tiles (lr_gemm_kernel) -> here, rows x K x N:
-// 16 x 2048 x 8224 89 -> 24; 400 x 5632 x 2048 358 -> 68; 400 x 2048 x 5632 gated 248 -> 138. Relative error against 64 bits,
-// 400 x 5632 x 2048: 1.34e-6 -> 1.4e-7 (K split).
+// 16 x 2048 x 8224 91 -> 29; 400 x 5632 x 2048 363 -> 74; 400 x 2048 x 5632 gated 246 -> 136. Relative error against 64 bits,
+// 400 x 5632 x 2048: 1.35e-6 -> 1.4e-7 (K split).
 #include "../kernels/gemm_f32x3.h"
 #include "hy_util.h"
 #include "hybrid.h"
@@ -12,7 +12,7 @@ namespace jla {
 template <int MT, int GATED, bool SCALED>
 __global__ void __launch_bounds__(64 * MT, 2) rows_f32x3_kernel(F3Rows p, RowLinear act, int tiles_n) {
   __shared__ u32x4 lds[f3_lds<MT>()];
-  f3_tile<MT, MT, GATED, SCALED>(p, tiles_n, 0, (p.K + F3_BK - 1) / F3_BK, lds, [&](const f32x4 g, const f32x4 u) {
+  f3_tile<MT, GATED, SCALED>(p, tiles_n, 0, (p.K + F3_BK - 1) / F3_BK, lds, [&](const f32x4 g, const f32x4 u) {
     f32x4 v = g;
     if (act.act != HY_ACT_NONE) {
 #pragma unroll
@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(64 * MT, 2) rows_f32x3_split_kernel(F3Rows p, 
   __shared__ u32x4 lds[f3_lds<MT>()];
   const int t0 = blockIdx.y * steps;
   p.out += (size_t)blockIdx.y * p.R * p.ldo;
-  f3_tile<MT, MT, 0, SCALED>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
+  f3_tile<MT, 0, SCALED>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
                  [](const f32x4 g, const f32x4) { return g; });
 }
 

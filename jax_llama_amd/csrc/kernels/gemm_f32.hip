@@ -2,8 +2,8 @@
 // `precision`, jax_test.py:433 runs the parity harness with precision='highest').
 //
 // y[M, N] = x[M, K] @ W[N, K]^T with fp32 inputs, fp32 accumulation and fp32 output. Rows of whole 16-byte pieces run as
-// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, before -> after: 1 554 -> 163,
-// 128 567 -> 196, 600 1780 -> 856, 1500 2162 (with 128 x 128 tiles) -> 1890); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
+// split products on the bf16 matrix cores (gemm_f32x3.h; us at M x 32000 x 4096, exact-f32 MFMA -> here: 1 555 -> 134, 100 565 -> 200,
+// 128 570 -> 204, 600 1785 -> 859, 1500 4182 -> 1918); any other K or N on the exact-f32 MFMA (v_mfma_f32_32x32x2_f32: a
 // k-ordered fmaf chain, no xf32 shortcut on gfx950): 128 x 128 output tile per 256-thread workgroup, four waves of 64 x 64
 // (2 x 2 MFMA tiles), K staged 32 deep through LDS in k-major images ([k][row]) so a lane's fragment element (row l & 31, k
 // l >> 5) is one conflict-free ds_read_b32.
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(64 * MT, 2) gemm_f32x3_kernel(F3Rows p, int ti
   __shared__ u32x4 lds[f3_lds<MT>()];
   const int t0 = blockIdx.y * steps;
   p.out += (size_t)blockIdx.y * p.R * p.ldo;
-  f3_tile<MT, MT, 0, false>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
+  f3_tile<MT, 0, false>(p, tiles_n, t0, min(t0 + steps, (p.K + F3_BK - 1) / F3_BK), lds,
                  [](const f32x4 g, const f32x4) { return g; });
 }
 

@@ -22,8 +22,13 @@
 // running sums are rounded once per step and not 24 times (4 vector additions per tile, 5 % of the time; relative error of
 // normal numbers, K 4096 in one chain 1.0e-6 -> 2.2e-7, K 2048 7.0e-7 -> 1.6e-7). Before, 128 x 128 outputs in four waves,
 // both operands through LDS, splits and products in turn: us of the product of M x N x K, before -> here, 600 x 32000 x 4096
-// 935 -> 856, 1500 2162 -> 1890, 128 248 -> 196, 400 x 14600 x 2048 172 -> 150, 200 x 11264 x 2048 91 -> 77, 64 x 2048 x 2048
-// 19 -> 16. Both operands through LDS in this order: 5 % slower.
+// 945 -> 859, 1500 2211 -> 1918, 128 224 -> 195, 400 x 14600 x 2048 177 -> 155, 200 x 11264 x 2048 93 -> 82, 64 x 2048 x 2048
+// 20 -> 18. Both operands through LDS in this order: 5 % slower.
+// Where the split does not hold, the workgroup computes its tile again on the fp32 matrix instruction (600 x 4000 x 4096 with a NaN
+// in every tile: 125 -> 338 us). An infinity or NaN among the
+// operands, or a number that rounds up to an infinity, makes its remainder NaN and so every result it enters (a sum past the largest
+// number shows there too): the results are looked through at the end. A piece of a row whose numbers are all below 2^-95 would have
+// parts that bf16's smallest step of 2^-133 cuts: the bits of the exponents are gathered as the pieces are split.
 #pragma once
 #include <type_traits>
 #include "common.h"
@@ -75,10 +80,10 @@ using F3Global = __attribute__((address_space(1))) f32x4;
 __device__ const f32x4 f3_zeros[2] = {};
 
 // K steps [t0, t1). act(gate accumulators, up accumulators) -> outputs of 4 neighbouring columns
-template <int MT, int WV, int GATED, bool SCALED, class Act>
+template <int MT, int GATED, bool SCALED, class Act>  // MT waves, 16 MT rows
 JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, const Act& act) {
-  constexpr int BM = 16 * MT, BN = 32 * WV;
-  static_assert(BM == 16 * WV && MT % 4 == 0, "a row piece per thread and step");
+  constexpr int BM = 16 * MT, BN = 32 * MT;  // (so that a thread has a row piece per step)
+  static_assert(MT % 4 == 0, "row tiles in fours");
   constexpr int AU = BM * 4;  // u32x4 of one part of the staged rows
   constexpr int BUF = 3 * AU;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
@@ -259,7 +264,7 @@ JLA_DEV void f3_tile(const F3Rows& p, int tiles_n, int t0, int t1, u32x4* lds, c
   f32x4* const out = reinterpret_cast<f32x4*>(lds) + wave * 256;
   constexpr int OCH = GATED ? 4 : 8;  // output chunks of a row
   const int rr0 = lane / OCH, oc = lane % OCH;
-  const int col = n0 + wave * (COLS / WV) + 4 * oc;
+  const int col = n0 + wave * (COLS / MT) + 4 * oc;
 #pragma unroll
   for (int part = 0; part < MT / 2; ++part) {
 #pragma unroll
