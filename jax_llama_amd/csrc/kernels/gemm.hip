@@ -1500,7 +1500,7 @@ static int num_cus() {
 // sums' way through memory and its second launch. Us without -> with, M x 4096 x K, residual: 12800 x 14336 1365 -> 1125, x 4096
 // 445 -> 387, x 2048 265 -> 250 (x 1024 157 -> 174: not); 8704 x 14336 1000 -> 787; 14336 x 4096 447 -> 425 (2 ways). Stored:
 // 12800 x 4096 385 -> 360, 13312 x 4096 (4 ways) 375 -> 373, 14336 x 14336 (2 ways) 1371 -> 1255 (x 4096 399 -> 408, 12800 x 2048
-// 209 -> 207: not).
+// 209 -> 207: not). The sums of many tiles weigh too: 18432 x 2048 x 2048, 64 tiles 4 ways, residual 177 -> 184 (17000, 32 tiles 175 -> 162).
 int gemm_tail_rows(int M, int N, int K, int residual, int* ksplit) {
   const int tm = (M + G4_BM - 1) / G4_BM, tn = (N + G4_BN - 1) / G4_BN, cus = num_cus();
   *ksplit = 1;
@@ -1509,7 +1509,7 @@ int gemm_tail_rows(int M, int N, int K, int residual, int* ksplit) {
   const int rest = (tm - whole) * tn;
   if (whole == 0 || rest == 0 || 2 * rest > cus) return 0;
   const int ks = min(cus / rest, (K >> 6) / 4);
-  if (ks < 2 || (long long)K * (ks - 1) < (residual ? 1536LL : 3072LL) * ks) return 0;
+  if (ks < 2 || (long long)K * (ks - 1) < (residual ? 1536LL + max(rest - 32, 0) : 3072LL) * ks) return 0;
   *ksplit = ks;
   return M - whole * G4_BM;
 }

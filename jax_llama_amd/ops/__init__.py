@@ -363,7 +363,8 @@ def _tiled(e, x, weight, n, k, out, mode, rms_eps, accumulate, mirror=None, pack
     ks, tm, ws = _gemm_ws(e, x.shape[0], n, k, x.device, mode, fused)
     if ks == 1 and tm == 0 and not fused and mode in (MODE_STORE, MODE_RESIDUAL):  # (a prompt past the tuned sizes)
         rest, split = e.gemm_tail(x.shape[0], n, k, mode == MODE_RESIDUAL)
-        if rest:  # its last rows, whose tiles would leave most of the chip idle, with K split over the chip
+        if rest:  # its last rows, whose tiles would leave most of the chip idle, with K split over the chip (their sums are added in
+            # another order than the first rows': equal prompts of one batch may differ in the last bits)
             m0 = x.shape[0] - rest
             e.gemm(xb[m0:], weight, n, k, out[m0:], mode, bool(accumulate), mirror[m0:] if mirror is not None else None, split,
                    workspace.get("gemm_ws", split * rest * (n + 1), torch.float32, x.device), -1.0, G4D_TILE, None, None)

@@ -20,7 +20,7 @@ def test_narrow_output(m, n, k, splits):
 
 
 @pytest.mark.parametrize("m,n,k,rest,split", [(4352, 4096, 2048, 256, 8), (4353, 4096, 4096, 257, 8), (8192 + 1, 4096, 1792, 1, 7), (4608, 4112, 14336, 768, 256 // (3 * 17)),
-                                              (4097, 4096, 1024, 0, 1), (8192, 4096, 4096, 0, 1), (6656, 4096, 4096, 0, 1)])
+                                              (4097, 4096, 1024, 0, 1), (18432, 2048, 2048, 0, 1), (17000, 2048, 2048, 616, 8), (8192, 4096, 4096, 0, 1), (6656, 4096, 4096, 0, 1)])
 @pytest.mark.parametrize("mirrored", [True, False])
 def test_rows_behind_the_whole_rounds(m, n, k, rest, split, mirrored):
     """The rows whose tiles start a mostly empty round have K split, in a launch of their own; all rows against 64 bits."""
