@@ -26,6 +26,7 @@ from __future__ import annotations
 import os
 import socket
 
+import numpy as np
 import torch
 import torch.distributed as dist
 
@@ -154,10 +155,16 @@ class CustomAllReduce:
     LITMUS_ROUNDS = int(os.environ.get("JLA_CAR_LITMUS_ROUNDS", "8"))
 
     @staticmethod
-    def _pattern(n: int, rank: int, rnd: int) -> torch.Tensor:
+    def _period(rank: int, rnd: int) -> np.ndarray:
+        return ((np.arange(97) * (2 * rnd + 1) + 31 * rank + rnd) % 97 + 1).astype(np.float32)
+
+    @classmethod
+    def _pattern(cls, n: int, rank: int, rnd: int) -> torch.Tensor:
         """Rank- and round-dependent integers in [1, 97]: exact in bf16 and fp32, and so are their sums over <= 8
-        ranks -- every rank can compute every peer's data and the exact expected result on the host."""
-        return ((torch.arange(n, dtype=torch.int64) * (2 * rnd + 1) + 31 * rank + rnd) % 97 + 1).to(torch.float32)
+        ranks -- every rank can compute every peer's data and the exact expected result on the host. They repeat
+        after 97 numbers, so only those are computed: the threads of several ranks' tensor operations wait for each
+        other on a shared host (8 ranks on 16 CPUs started in 181 s with every number computed, now in 69 s)."""
+        return torch.from_numpy(np.resize(cls._period(rank, rnd), n))
 
     def self_test(self, kind: str = "collective", rounds=None) -> bool:
         """Litmus test on the real links before the instance is declared usable (a wrong protocol on some fabric
@@ -173,7 +180,7 @@ class CustomAllReduce:
         ok = True
 
         def want_sum(n, rnd):
-            return sum(self._pattern(n, r, rnd) for r in range(world))
+            return torch.from_numpy(np.resize(sum(self._period(r, rnd) for r in range(world)), n))
 
         for rnd in range(rounds):
             if kind == "fused":
@@ -221,7 +228,7 @@ class CustomAllReduce:
             for name, n in (("granule_resid_bf16", 8 * 1024), ("flag_resid_bf16", 256 * 1024)):
                 if n * 2 > self.max_bytes:
                     continue
-                h0 = (torch.arange(n, dtype=torch.float32) % 13)
+                h0 = torch.from_numpy(np.resize(np.arange(13, dtype=np.float32), n))
                 h = h0.cuda()
                 hb = torch.empty(n, dtype=torch.bfloat16, device="cuda")
                 self.all_reduce_residual_(self._pattern(n, rank, rnd).to(torch.bfloat16).cuda(), h, hb)

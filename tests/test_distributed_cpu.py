@@ -186,3 +186,14 @@ def test_fused_row_parallel_routing():
     assert TPComm(size=1, rank=0, group=None).fused_o_state(X(1), W()) == 0
     assert TPComm(size=8, rank=0, group=None, custom=None, reduce_dtype=torch.bfloat16,
                   fused=None).fused_o_state(X(1), W()) is None
+
+
+@pytest.mark.parametrize("n", [1, 96, 97, 98, 8 * 1024, 192 * 1024])
+def test_litmus_pattern_repeats(n):
+    """The collectives' test data: the period laid out again and again is the formula at every index."""
+    from jax_llama_amd.parallel.custom_allreduce import CustomAllReduce
+
+    for rank, rnd in ((0, 0), (1, 1), (7, 7), (3, 254)):
+        want = (torch.arange(n, dtype=torch.int64) * (2 * rnd + 1) + 31 * rank + rnd) % 97 + 1
+        got = CustomAllReduce._pattern(n, rank, rnd)
+        assert got.dtype == torch.float32 and torch.equal(got, want.to(torch.float32))
