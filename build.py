@@ -172,7 +172,7 @@ def build_hybrid(jobs: int, force: bool) -> Path:
     """``_C_hybrid``: csrc/hybrid/*.hip + csrc/hybrid/bindings.cpp (its own module, so a hybrid model runs without
     compiling the LLaMA kernels)."""
     hdir = CSRC / "hybrid"
-    headers = sorted(hdir.glob("*.h")) + [CSRC / "kernels" / h for h in ("common.h", "gemm4w.h", "row_tiles.h", "gemm_f32x3.h")]
+    headers = sorted(hdir.glob("*.h")) + [CSRC / "kernels" / h for h in ("common.h", "gemm4w.h", "row_tiles.h", "gemm_f32x3.h", "mid_tile.h")]
     srcs = sorted(hdir.glob("*.hip"))
     odir = BUILD / "C_hybrid"
     objs = [odir / (s.stem + ".o") for s in srcs]

@@ -293,17 +293,28 @@ bool dense_is_gemv(int64_t rows, int64_t n) {
   return jla::hy_linear_rows_is_gemv(p);
 }
 
-// whether a dense linear of `rows` contiguous rows on `w` is best rounded to bf16 for the large tiles (rows_gemm.hip)
-bool rows_gemm_pays(int64_t rows, const Tensor& w, int64_t act) {
+// a dense linear of `rows` contiguous bf16 rows on `w`, for the questions below; false: there is none
+static bool bf16_rows_linear(int64_t rows, const Tensor& w, int64_t act, jla::RowLinear& p) {
   if (w.dim() != 2 || !w.is_contiguous() || w.scalar_type() != at::kBFloat16) return false;
   if (act < jla::HY_ACT_NONE || act > jla::HY_ACT_GELU_GLU || rows < 0 || rows > 0x7fffffff) return false;
   const bool gated = jla::hy_act_gated(act);
   if (gated && w.size(0) % 2) return false;
-  jla::RowLinear p{};
   p.R = rows; p.N = gated ? w.size(0) / 2 : w.size(0); p.K = w.size(1); p.E = 1;
   p.lda = p.K; p.ldo = p.N; p.a_bf16 = p.wbf16 = 1; p.act = act;
   p.w = w.data_ptr(); p.w_stride = w.numel();
-  return jla::hy_rows_gemm_pays(p);
+  return true;
+}
+
+// whether it is best rounded to bf16 for the large tiles (rows_gemm.hip)
+bool rows_gemm_pays(int64_t rows, const Tensor& w, int64_t act) {
+  jla::RowLinear p{};
+  return bf16_rows_linear(rows, w, act, p) && jla::hy_rows_gemm_pays(p);
+}
+
+// whether it runs on the tiles for some ten to a few hundred rows (rows_mid.hip)
+bool rows_mid_takes(int64_t rows, const Tensor& w, int64_t act) {
+  jla::RowLinear p{};
+  return bf16_rows_linear(rows, w, act, p) && jla::hy_rows_mid_takes(p);
 }
 
 void route_table(Tensor ids, Tensor table, int64_t E, Tensor row_expert, Tensor row_tok, Tensor sort_tok, Tensor sort_dst,
@@ -1282,6 +1293,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("route_topk", &route_topk);
   m.def("dense_is_gemv", &dense_is_gemv);
   m.def("rows_gemm_pays", &rows_gemm_pays);
+  m.def("rows_mid_takes", &rows_mid_takes);
   m.def("latent_prep", &latent_prep, py::arg("proj"), py::arg("col0"), py::arg("w"), py::arg("slot"), py::arg("B"),
         py::arg("S"), py::arg("cache"), py::arg("eps"), py::arg("q"), py::arg("q_col0") = 0,
         py::arg("q_norm_w") = py::none(), py::arg("rot_freq") = py::none(), py::arg("positions") = py::none(),

@@ -112,6 +112,9 @@ bool hy_rows_gemv_takes(const RowLinear& p);
 bool hy_rows_gemv_takes_residual(const RowLinear& p);
 int hy_rows_gemv(const RowLinear& p, hipStream_t s);
 int hy_rows_gemm(const RowLinear& p, hipStream_t s);
+bool hy_rows_mid_takes(const RowLinear& p);
+long long hy_rows_mid_floats(const RowLinear& p);
+int hy_rows_mid(const RowLinear& p, float* ws, hipStream_t s);
 // ws: hy_linear_rows_floats() floats of scratch, 16-byte aligned (0: none needed)
 long long hy_linear_rows_floats(const RowLinear& p);
 int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s);

@@ -3,7 +3,8 @@
 // The dispatch of every such product (hy_linear_rows), and the forms that take what no other does. In this order:
 //   a handful of output columns (a router), any rows            the vector GEMV below
 //   one or two normed rows, K <= 512, N <= 2048                 the vector GEMV below
-//   one to 64 rows on bf16 weights, 16-byte rows                rows_gemv.hip, on the matrix cores
+//   nine to some hundred rows on bf16 weights, K a multiple of 64  rows_mid.hip, tiles of 16 to 128 rows
+//   one to 64 rows on bf16 weights otherwise, 16-byte rows      rows_gemv.hip, on the matrix cores
 //   up to 8 rows, or 64 sorted by expert, otherwise             the vector GEMV below (fp32 weights, odd or short K)
 //   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, 256-row tiles
 //   fp32 weights, 16-byte rows, K >= 512 (256 with many rows)   rows_f32.hip, split products on the bf16 matrix cores
@@ -405,6 +406,7 @@ int hy_linear_rows_pair(const RowLinear& p, const RowLinear& q, float* ws, hipSt
 }
 
 long long hy_linear_rows_floats(const RowLinear& p) {
+  if (p.R > 0 && p.N > 0 && p.K > 0 && !lr_skinny(p) && hy_rows_mid_takes(p)) return hy_rows_mid_floats(p);
   if (p.R <= 0 || p.N <= 0 || p.K <= 0 || hy_linear_rows_is_gemv(p) || hy_rows_gemv_takes(p) || hy_rows_gemm_takes(p) ||
       !hy_rows_f32_takes(p))
     return 0;
@@ -430,6 +432,7 @@ int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s) {
   if (p.offs && p.E > 65535) return -2;
   const bool grouped = lr_grouped(p);
   const bool small = hy_linear_rows_is_gemv(p);
+  if (!lr_skinny(p) && hy_rows_mid_takes(p)) return hy_rows_mid(p, ws, s);
   if (!lr_skinny(p) && !lr_short_normed(p) && hy_rows_gemv_takes(p)) return hy_rows_gemv(p, s);
   if (p.a_norm_w && (!small || p.a_bf16)) return -10;  // (the tiles take a normed activation, they do not norm it)
   if (small) {

@@ -1,0 +1,210 @@
+// Some ten to a few hundred rows on row-major bf16 weights: out[dst(r), :] = act(A[src(r), :] @ W[expert(r)]^T), dense or with some
+// rows per expert, the rows bf16 or fp32 (rounded as a fragment is read). kernels/mid_tile.h says what bounds it and why the tile is
+// as it is; here are its forms, the choice among them, and the epilogue.
+// Us, weights in no cache, 16 | 64 | 128 | 255 rows, the forms before (rows_gemv.hip to 64 rows, lr_gemm_kernel's tiles) -> here, from 65 rows on
+// with the rounding of the rows: 2048 x 2048 9.5 | 23.8 | 41 | 41 -> 7.3 | 10.0 | 12.4 | 16.6; 2048 x 5632 20.7 | 55 | 157 | 157 -> 14 | 17 | 20 | 25;
+// 4096 x 4096 16.4 | 42 | 108 | 103 -> 13.5 | 19 | 23 | 28; 4096 x 14336 50 | 132 | 392 | 392 -> 29 | 35 | 46 | 55; gated 5632 x 2048 20 | 41 | 87 | 87 ->
+// 17 | 22 | 26 | 39. A mixture of 8 experts of 2816 x 2048 (7168 x 4096), two per token, both products, 33 | 100 | 256 tokens: 165 | 172 | 133 -> 77 |
+// 80 | 88 (452 | 473 | 425 -> 257 | 289 | 297; its weights 237 at 5.95 TB/s).
+#include "../kernels/mid_tile.h"
+#include "../kernels/row_tiles.h"
+#include "hy_util.h"
+#include "hybrid.h"
+#include "row_act.h"
+
+namespace jla {
+
+JLA_DEV void rm_store(const RowLinear& p, int d, int col, f32x4 v) {
+  if (p.out_bf16) {
+    *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + (size_t)d * p.ldo + col) = u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
+  } else {
+    f32x4* o = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + (size_t)d * p.ldo + col);
+    *o = p.add_out ? *o + v : v;
+  }
+}
+
+// grid: tiles x splits, rounded up to 8; slabs (several splits): [splits][R][weight rows] partial sums instead of the output.
+// gated: the 16-column tiles of a wave are gate and up tiles in turn (NT even).
+template <int MT, int NT, int WN, int WK, int S, int XB>
+__global__ void __launch_bounds__(64 * WN * WK) rows_mid_kernel(RowLinear p, int gated, int tiles_n, int splits, int steps, float* slabs) {
+  using H = MidShape<MT, NT, WN, WK, S, XB>;
+  __shared__ u32x4 lds[H::LDS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+  int e = 0, r0 = 0, rend = 0, tn = 0, split = 0;
+  if (!row_tile<H::BM>(p.offs, p.E, p.R, tiles_n, lane, e, r0, rend, tn, splits, split)) return;
+  const int K = p.K, N = p.N, t0 = split * steps, t1 = min(K >> 6, t0 + steps);
+  const int n0 = tn * (gated ? H::BN / 2 : H::BN);
+  const char* const wbase = reinterpret_cast<const char*>(reinterpret_cast<const bf16_t*>(p.w) + (size_t)e * p.w_stride);
+  auto xrow = [&](int r) {  // (rows past the end repeat the last one)
+    const int row = min(r0 + r, rend - 1);
+    return reinterpret_cast<const char*>(p.a) + (size_t)(p.a_idx ? p.a_idx[row] : row) * p.lda * XB;
+  };
+  auto wrow = [&](int r) {
+    const int j = r >> 4, col = min(n0 + (gated ? 16 * (j >> 1) + (r & 15) : r), N - 1);
+    return wbase + (size_t)(gated && (j & 1) ? N + col : col) * K * 2;
+  };
+  f32x4 acc[NT][MT];
+  mid_tile<MT, NT, WN, WK, S, XB, false>(lds, xrow, wrow, t0, t1, acc, [](int, const u32x4 (&)[MT]) {});
+  if (wave >= WN) return;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = r0 + 16 * m + c;
+    if (row >= rend) continue;
+    const int d = slabs ? row : (p.dst_idx ? p.dst_idx[row] : row);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int j = wave * NT + t, col = n0 + 16 * (gated ? j >> 1 : j) + 4 * q;
+      if (col >= N) continue;
+      if (slabs) {
+        const int nw = gated ? 2 * N : N;
+        *reinterpret_cast<f32x4*>(slabs + ((size_t)split * p.R + row) * nw + (gated && (t & 1) ? N : 0) + col) = acc[t][m];
+      } else if (!gated || !(t & 1)) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = lr_act(p, acc[t][m][i], gated ? acc[t + 1 < NT ? t + 1 : t][m][i] : 0.f);
+        rm_store(p, d, col, v);
+      }
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256) rows_mid_sum_kernel(RowLinear p, const float* __restrict__ ws, int splits, int gated) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int n4 = p.N / 4;
+  const long long r = i / n4;
+  if (r >= p.R) return;
+  const int col = 4 * (int)(i - r * n4), nw = gated ? 2 * p.N : p.N;
+  const float* at = ws + r * nw + col;
+  f32x4 g = *reinterpret_cast<const f32x4*>(at), u = gated ? *reinterpret_cast<const f32x4*>(at + p.N) : f32x4{0.f, 0.f, 0.f, 0.f}, v;
+  for (int s = 1; s < splits; ++s) {
+    const float* more = at + (size_t)s * p.R * nw;
+    g += *reinterpret_cast<const f32x4*>(more);
+    if (gated) u += *reinterpret_cast<const f32x4*>(more + p.N);
+  }
+#pragma unroll
+  for (int x = 0; x < 4; ++x) v[x] = lr_act(p, g[x], u[x]);
+  rm_store(p, p.dst_idx ? p.dst_idx[r] : (int)r, col, v);
+}
+
+// A form's measured times, us: launch and fill; a stage; a stage's rise with every further workgroup of a compute unit; a split's second
+// launch, and a megabyte through the slabs (write and read)
+struct RmForm {
+  int mt, nt, wn, wk, xb;
+  float fill, stage, more, sum, mb;
+  void (*run)(unsigned, hipStream_t, const RowLinear&, int, int, int, int, float*);
+};
+template <int MT, int NT, int WN, int WK, int S, int XB>
+static void rm_launch(unsigned grid, hipStream_t s, const RowLinear& p, int gated, int tiles_n, int splits, int steps, float* slabs) {
+  rows_mid_kernel<MT, NT, WN, WK, S, XB><<<grid, 64 * WN * WK, 0, s>>>(p, gated, tiles_n, splits, steps, slabs);
+}
+#define RM_FORM(MT, NT, WN, WK, S, XB, ...) {MT, NT, WN, WK, XB, __VA_ARGS__, rm_launch<MT, NT, WN, WK, S, XB>}
+static const RmForm RM_FORMS[] = {
+    RM_FORM(1, 1, 1, 4, 4, 2, 4.14f, 0.342f, 0.462f, 1.53f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 2, 3.36f, 0.243f, 0.716f, 2.81f, 0.438f),
+    RM_FORM(1, 2, 4, 1, 8, 2, 3.06f, 0.413f, 0.977f, 3.35f, 0.814f), RM_FORM(2, 1, 1, 4, 3, 2, 4.64f, 0.481f, 0.411f, 1.23f, 0.706f),
+    RM_FORM(2, 1, 4, 1, 6, 2, 4.61f, 0.285f, 0.658f, 1.79f, 0.301f), RM_FORM(2, 2, 4, 1, 6, 2, 6.37f, 0.374f, 1.12f, 0.381f, 0.523f),
+    RM_FORM(4, 1, 1, 4, 3, 2, 6.64f, 0.577f, 1.5f, 0.0f, 0.793f), RM_FORM(4, 1, 4, 1, 4, 2, 6.18f, 0.344f, 0.666f, 0.701f, 0.247f),
+    RM_FORM(4, 2, 4, 1, 4, 2, 7.42f, 0.446f, 1.2f, 0.0f, 0.311f), RM_FORM(6, 2, 4, 1, 4, 2, 8.0f, 0.586f, 1.17f, 0.104f, 0.283f),
+    RM_FORM(8, 2, 4, 1, 4, 2, 8.0f, 0.787f, 1.14f, 0.84f, 0.236f), RM_FORM(8, 2, 8, 1, 3, 2, 8.0f, 1.06f, 1.0f, 1.52f, 0.198f),
+    RM_FORM(1, 1, 1, 4, 4, 4, 4.63f, 0.422f, 1.28f, 1.74f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 4, 3.73f, 0.307f, 0.912f, 2.31f, 1.0f),
+    RM_FORM(1, 2, 4, 1, 8, 4, 3.24f, 0.438f, 0.957f, 3.29f, 0.886f), RM_FORM(2, 1, 1, 4, 3, 4, 5.43f, 0.63f, 1.33f, 1.33f, 1.0f),
+    RM_FORM(2, 1, 4, 1, 6, 4, 6.23f, 0.346f, 0.967f, 0.0f, 0.8f), RM_FORM(2, 2, 4, 1, 6, 4, 6.95f, 0.457f, 1.02f, 0.0f, 0.625f),
+    RM_FORM(4, 1, 4, 1, 4, 4, 6.81f, 0.48f, 0.998f, 0.0f, 0.513f), RM_FORM(4, 2, 4, 1, 4, 4, 7.62f, 0.641f, 1.0f, 0.0f, 0.4f),
+};
+#undef RM_FORM
+constexpr int RM_MAX_SPLITS = 16;
+
+struct RmPlan {
+  const RmForm* form = nullptr;
+  int splits = 1, steps = 0;
+  float us = 1e30f;
+};
+
+// ... of rows: with experts, whose counts only the device knows, a standard deviation above the mean each
+static long long rm_row_tiles(const RowLinear& p, int bm) {
+  if (!p.offs) return (p.R + bm - 1LL) / bm;
+  const int E = p.E < p.R ? p.E : p.R;
+  const float mean = (float)p.R / (float)E, most = p.even_rows > 0 ? mean : mean + sqrtf(mean);
+  return E * (long long)ceilf(most / (float)bm);
+}
+
+// The form and split with the least time by the figures above: on average 1.9 % above the best of all that were measured (467 shapes: one
+// matrix, 8 and 32 experts, N 64 to 32000, K 512 to 14336, 9 to 1000 rows)
+static RmPlan rm_plan(const RowLinear& p) {
+  const int gated = hy_act_gated(p.act), T = p.K >> 6, xb = p.a_bf16 ? 2 : 4, E = p.offs ? (p.E < p.R ? p.E : p.R) : 1;
+  const long long nw = gated ? 2LL * p.N : p.N;
+  const float stream = (float)E * (float)nw * (float)p.K * 2 / 5.4e6f;  // the weights themselves
+  RmPlan best;
+  for (const RmForm& f : RM_FORMS) {
+    if (f.xb != xb || (gated && f.nt % 2)) continue;
+    const long long tiles = rm_row_tiles(p, 16 * f.mt) * ((nw + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
+    int last = 0;
+    for (int want = 1; want <= RM_MAX_SPLITS && want <= T; ++want) {
+      const int steps = (T + want - 1) / want, splits = (T + steps - 1) / steps;
+      if (splits == last || (want > 1 && (steps < 2 * f.wk || tiles * splits > 700))) continue;
+      last = splits;
+      const float load = (float)(tiles * splits) / 256.f, deep = load > 2.f ? load + .3f : (load > 1.f ? 2.f : 1.f);
+      float us = f.fill + f.stage * (float)((steps + f.wk - 1) / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
+      if (us < 3.5f + stream) us = 3.5f + stream;
+      if (splits > 1) us += f.sum + .15f * (float)splits + f.mb * (float)p.R * (float)nw * (float)splits * 8e-6f;
+      if (f.wk > 1 && load > 2.f) us *= 3.f;  // (16 columns a workgroup: x over and over)
+      if (us < best.us) best = RmPlan{&f, splits, steps, us};
+    }
+  }
+  return best;
+}
+
+// The range, and what is faster outside of it:
+//  * fp32 rows of one matrix, 9 to 64 (more: the caller rounds them first; their bytes are x's twice). Up to 24 rows of K below 1024
+//    rows_gemv.hip: 512 x 512, 16 rows 4.7 us there, 5.5 here; 1024 x 1024 6.1 both.
+//  * bf16 rows of one matrix: to 255; from 256 on a prompt's rows have the 256-row tiles (us here | there, weights in no cache: 2048 x 2048,
+//    255 | 777 rows 16 | 18, 27 | 25 with its sums; 4096 x 4096, 255 | 300 24.6 | 25.5, 29.9 | 27.7; 8224 x 2048, 300 33.2 | 31.4).
+//  * rows by expert: more than 64 up to 112 per expert on average (8 experts, gated 2816 x 2048 and down, 96 | 320 | 800 rows 50 | 98, 49 | 92,
+//    54 | 75 and 20 | 63, 22 | 50, 31 | 52; 128 per expert 80 | 78 and 39 | 54, 32 experts 241 | 267 and 135 | 109), of K below 256
+//    to 64 (16 per-head matrices of 512 x 128, 64 | 80 rows each 7.0 | 8.1, 10.9 | 8.1). Up to 64 rows in all rows_gemv.hip, unless there
+//    are five per expert on large matrices (8 experts, 56 rows: gated 7168 x 4096 171 | 213, 4096 x 7168 82 | 106; gated 2816 x 2048 51 | 48, gated 512 x 1024 11 | 8).
+constexpr int RM_MIN_ROWS = 9, RM_F32_ROWS = 64, RM_FEW_ROWS = 24, RM_FEW_K = 1024, RM_ROWS = 255;
+constexpr long long RM_SORTED_WORK = 20000000;
+constexpr int RM_EXPERT_ROWS = 112, RM_SORTED_ROWS = 64, RM_SHORT_K = 256, RM_SHORT_ROWS = 64;
+
+bool hy_rows_mid_takes(const RowLinear& p) {
+  auto aligned = [](const void* x, size_t n) { return ((uintptr_t)x & (n - 1)) == 0; };
+  if (!p.wbf16 || p.a_scale || p.a_norm_w || p.tab || p.R < RM_MIN_ROWS || !(p.offs || (p.E == 1 && !p.row_expert)) || p.K % 64 || p.K < 128 ||
+      p.lda % (p.a_bf16 ? 8 : 4) || p.N % 4 || p.ldo % 4 || p.w_stride % 8 || (p.add_out && p.out_bf16) || !aligned(p.a, 16) || !aligned(p.w, 16) ||
+      !aligned(p.out, p.out_bf16 ? 8 : 16))
+    return false;
+  const long long nw = hy_act_gated(p.act) ? 2LL * p.N : p.N;
+  if (p.offs) {
+    if (p.R > RM_SORTED_ROWS) return p.R <= (long long)(p.K < RM_SHORT_K ? RM_SHORT_ROWS : RM_EXPERT_ROWS) * p.E;
+    return !p.a_bf16 && p.R >= 5LL * p.E && nw >= 4096 && nw * p.K >= RM_SORTED_WORK;
+  }
+  if (!p.a_bf16) return p.R <= RM_F32_ROWS && !(p.R <= RM_FEW_ROWS && p.K < RM_FEW_K);
+  return p.R <= RM_ROWS;
+}
+
+long long hy_rows_mid_floats(const RowLinear& p) {
+  const RmPlan pl = rm_plan(p);
+  return pl.splits > 1 ? (long long)pl.splits * p.R * (hy_act_gated(p.act) ? 2 : 1) * p.N : 0;
+}
+
+int hy_rows_mid(const RowLinear& p, float* ws, hipStream_t s) {
+  const int gated = hy_act_gated(p.act), E = p.offs ? p.E : 1;
+  const RmPlan pl = rm_plan(p);
+  if (!pl.form) return -13;
+  const int bm = 16 * pl.form->mt, bn = 16 * pl.form->nt * pl.form->wn;
+  const long long tn = ((gated ? 2LL : 1LL) * p.N + bn - 1) / bn;
+  const long long grid = ((p.offs ? p.R / bm + (long long)E : (p.R + bm - 1LL) / bm) * tn * pl.splits + 7) / 8 * 8;
+  if (grid > 0x7fffffffLL) return -4;
+  if (pl.splits > 1 && (!ws || ((uintptr_t)ws & 15))) return -12;
+  RowLinear q = p;
+  q.row_expert = nullptr;
+  pl.form->run((unsigned)grid, s, q, gated, (int)tn, pl.splits, pl.steps, pl.splits > 1 ? ws : nullptr);
+  JLA_CHECK_LAUNCH();
+  if (pl.splits > 1) {
+    const long long n = (long long)p.R * (p.N / 4);
+    rows_mid_sum_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(q, ws, pl.splits, gated);
+    JLA_CHECK_LAUNCH();
+  }
+  return 0;
+}
+
+}  // namespace jla

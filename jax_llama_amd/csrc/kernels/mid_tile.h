@@ -1,0 +1,136 @@
+// The tile of the products of some ten to a few hundred rows, x [M, K] times W [N, K] with bf16 weights (rows_mid.hip: row-major
+// weights; linear_mid.hip: packed ones).
+//
+// What bounds it: bytes through a compute unit's vector memory path. W comes from HBM once (about 24 bytes per ns and unit with
+// every unit pulling), x from L2, and the two do not overlap there: a unit keeps about 32 KB outstanding whatever it asks for,
+// so time is the sum of W's and x's bytes at their latencies (64 rows of 4096 x 4096, operands straight to registers: W alone 9.2
+// us, x alone 8.7, both 15.8, at any depth of prefetch). So: every weight byte is asked for by as few workgroups as can be, whole
+// 128-byte lines of both operands (a fragment that a wave loads from 16 rows at once costs twice the path's time: 26 us instead of
+// 15.8 at 64 rows), and x shared by the workgroup's columns through LDS. Both operands come by LDS-DMA, S stages of 64 WK deep in a ring, one
+// barrier a stage. WN groups of waves deal the columns (16 NT each), WK groups the K of a stage: WN = 1 keeps a workgroup at 16
+// columns, which is what fills the chip with N 2048 without a split of K over workgroups; WN = 4 shares x four times as often.
+#pragma once
+#include "common.h"
+
+namespace jla {
+
+template <int MT, int NT, int WN, int WK, int S, int XB>  // XB: bytes of an x number (2: bf16, 4: fp32, rounded as it is read)
+struct MidShape {
+  static constexpr int WAVES = WN * WK, BM = 16 * MT, BN = 16 * NT * WN;
+  static constexpr int XP = BM / 8 * (XB / 2), WP = BN / 8, PIECES = (XP + WP) * WK;  // 1 KiB DMA pieces of a K slice of 64; of a stage
+  static constexpr int OPS = (PIECES + WAVES - 1) / WAVES;                            // ... of a wave (surplus ones repeat the last piece)
+  static constexpr int SLICE = (XP + WP) * 64, SLOT = SLICE * WK;                     // u32x4
+  static constexpr int LDS = SLOT * S;
+  static_assert(S >= 3 && LDS * 16 <= 160 * 1024, "ring");
+  static_assert(WK * NT * MT * WN / 2 * 64 <= LDS, "the waves' sums reuse the ring");
+};
+
+// 16-byte cell of chunk x of row r in its 128-byte line of LDS: the 16 lanes that a fragment read serves at a time (rows 0-3 and 12-15
+// of one quarter, 4-11 of the next) fall on all 64 banks; fp32 rows, whose quarter is two chunks, need another order for that
+JLA_DEV int mid_cell(int x, int r, int xb) {
+  const int s = (r >> 1) & 7;
+  return x ^ (xb == 4 ? (int)(0x32765410u >> (4 * s)) & 7 : s);
+}
+
+// acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 m + c of the tile at weight columns 4 q .. + 3 of this wave's 16-column
+// tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64; t0 < t1. xrow(r), wrow(r): the address of row r of the
+// tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py pack_frag16x32).
+// SS: squares(row fragment) is called once for every x fragment of the stages, by one wave each: (m, fragment).
+template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, class XRow, class WRow, class Squares>
+JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], Squares squares) {
+  using H = MidShape<MT, NT, WN, WK, S, XB>;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, q = lane >> 4;
+  const int wn = wave % WN, wk = wave / WN, ns = (t1 - t0 + WK - 1) / WK;
+  const char* src[H::OPS];
+#pragma unroll
+  for (int i = 0; i < H::OPS; ++i) {
+    const int p = min(wave + H::WAVES * i, H::PIECES - 1) % (H::XP + H::WP);
+    if (p < H::XP) {  // 8 rows x 128 bytes; fp32: the first halves of all rows, then the second
+      const int row = p % (H::BM / 8) * 8 + (lane >> 3), half = p / (H::BM / 8);
+      src[i] = xrow(row) + 128 * half + 16 * mid_cell(lane & 7, row, XB);
+    } else {
+      const int w = p - H::XP;
+      if constexpr (PACKED) {
+        src[i] = wrow(16 * (w >> 1)) + 1024 * (w & 1) + 16 * lane;  // fragment w & 1 of tile w >> 1
+      } else {
+        const int row = w * 8 + (lane >> 3);
+        src[i] = wrow(row) + 16 * mid_cell(lane & 7, row, 2);
+      }
+    }
+  }
+  auto issue = [&](int st, int slot) {
+#pragma unroll
+    for (int i = 0; i < H::OPS; ++i) {
+      const int p = min(wave + H::WAVES * i, H::PIECES - 1), sl = p / (H::XP + H::WP);
+      const bool xs = p % (H::XP + H::WP) < H::XP;
+      const int t = min(t0 + st * WK + sl, t1 - 1);  // (past the end: the last step again, unused)
+      glds16_asm(src[i] + (size_t)t * (xs ? 64 * XB : (PACKED ? 2048 : 128)), lds + slot * H::SLOT + p * 64);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s) issue(s, s);
+  int slot = 0, fill = S - 1;
+  for (int st = 0; st < ns; ++st) {
+    // this wave's pieces of stage st have landed, then every wave's; and every wave is past the slot that is filled next
+    wait_vmcnt<(S - 2) * H::OPS>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(st + S - 1, fill);
+    if (t0 + st * WK + wk < t1) {  // (wave-uniform)
+      const u32x4* xs = lds + slot * H::SLOT + wk * H::SLICE;
+      const u32x4* ws = xs + H::XP * 64 + wn * NT * 128;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        u32x4 wf[NT], xf[MT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) wf[t] = ws[PACKED ? (2 * t + h) * 64 + lane : (16 * t + c) * 8 + mid_cell(4 * h + q, c, 2)];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          if constexpr (XB == 2) {
+            xf[m] = xs[(16 * m + c) * 8 + mid_cell(4 * h + q, c, 2)];
+          } else {
+            const u32x4* at = xs + (h * H::BM + 16 * m + c) * 8;
+            const f32x4 a = __builtin_bit_cast(f32x4, at[mid_cell(2 * q, c, 4)]), b = __builtin_bit_cast(f32x4, at[mid_cell(2 * q + 1, c, 4)]);
+            const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+            xf[m] = pack8(f);
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[t][m] = mfma16x16x32(wf[t], xf[m], acc[t][m]);
+        squares(wn, xf);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    slot = slot + 1 == S ? 0 : slot + 1;
+    fill = fill + 1 == S ? 0 : fill + 1;
+  }
+  wait_vmcnt<0>();
+  if constexpr (WK > 1) {  // the K groups' sums
+    f32x4* red = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int half = WK / 2; half > 0; half /= 2) {
+      __syncthreads();
+      if (wk >= half && wk < 2 * half) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) red[((((wk - half) * WN + wn) * NT + t) * MT + m) * 64 + lane] = acc[t][m];
+      }
+      __syncthreads();
+      if (wk < half) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[t][m] += red[(((wk * WN + wn) * NT + t) * MT + m) * 64 + lane];
+      }
+    }
+  }
+}
+
+}  // namespace jla

@@ -17,9 +17,12 @@ JLA_DEV void row_tile_coords(int pid, int tiles_m, int tiles_n, int gm, int& tm,
 // matrix) bounds the experts' rows. Workgroups are dealt round robin to the 8 XCDs, so XCD x takes the x-th eighth of the
 // order (expert by expert, groups of 4 m-tiles across every column tile): the tiles that run side by side behind one L2
 // share weight columns and activation rows. Every wave computes the same answer: lane l looks at experts l, l + 64, ...
-// The grid is a multiple of 8 and at least the number of tiles.
+// The grid is a multiple of 8 and at least the number of tiles. With splits, every tile is there that many times, one split after the
+// other in the order, so that an XCD's share of all of them is even (81 tiles in three splits: 31 workgroups at most behind an XCD,
+// where three launches' eighths of 81 would put 33 on its 32 units).
 template <int BM>
-JLA_DEV bool row_tile(const int32_t* offs, int experts, int R, int tiles_n, int lane, int& e, int& r0, int& rend, int& tn) {
+JLA_DEV bool row_tile(const int32_t* offs, int experts, int R, int tiles_n, int lane, int& e, int& r0, int& rend, int& tn, int splits,
+                      int& split) {
   const int E = offs ? experts : 1;
   auto rows = [&](int x) { return x < E ? (offs ? offs[x + 1] - offs[x] : R) : 0; };
   int total = 0;
@@ -30,9 +33,11 @@ JLA_DEV bool row_tile(const int32_t* offs, int experts, int R, int tiles_n, int 
     total += n;
   }
   total *= tiles_n;
-  const int per = (total + 7) / 8, at = blockIdx.x >> 3;
-  const int pid = (int)(blockIdx.x & 7) * per + at;
-  if (at >= per || pid >= total) return false;
+  const int per = (total * splits + 7) / 8, at = blockIdx.x >> 3;
+  int pid = (int)(blockIdx.x & 7) * per + at;
+  if (at >= per || pid >= total * splits) return false;
+  split = pid / max(total, 1);
+  pid -= split * total;
   int before = 0;  // m-tiles of the experts passed
   for (int b = 0; b < E; b += 64) {
     const int n = (rows(b + lane) + BM - 1) / BM;
@@ -57,6 +62,11 @@ JLA_DEV bool row_tile(const int32_t* offs, int experts, int R, int tiles_n, int 
     before += __builtin_amdgcn_readlane(inc, 63);
   }
   return false;
+}
+template <int BM>
+JLA_DEV bool row_tile(const int32_t* offs, int experts, int R, int tiles_n, int lane, int& e, int& r0, int& rend, int& tn) {
+  int split;
+  return row_tile<BM>(offs, experts, R, tiles_n, lane, e, r0, rend, tn, 1, split);
 }
 
 }  // namespace jla

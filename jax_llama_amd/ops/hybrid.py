@@ -369,14 +369,17 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], n)
     if not _gpu(x):
         return _act_cpu(_round_like(x, w) @ w.float().t(), act, limit, alpha)
+    if norm_w is None and _mid_rows(x, w, act):
+        out = torch.empty(x.shape[0], n, dtype=out_dtype, device=x.device)
+        ext().linear_rows(_bf16_operand(x), None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, None, 0.0)
+        return out
     if act == ACT_NONE and norm_w is None and _use_packed_gemm(x, w):
         from . import linear as packed_linear
         return packed_linear(_bf16_rows(x), _packed_weight(w), out_dtype=F32)
     if act_gated(act) and norm_w is None and x.shape[0] >= PACKED_GEMM_MIN_M and ext().rows_gemm_pays(x.shape[0], w, int(act)):
         # a prompt's gated product: bf16 rows (the operands they would be rounded to anyway) on the large tiles
-        xb = _bf16_rows(x) if x.is_contiguous() and x.numel() % 8 == 0 else x.to(BF16).contiguous()
         out = torch.empty(x.shape[0], n, dtype=out_dtype, device=x.device)
-        ext().linear_rows(xb, None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, None, 0.0)
+        ext().linear_rows(_bf16_operand(x), None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, None, 0.0)
         return out
     out = torch.empty(x.shape[0], n, dtype=F32, device=x.device)
     ext().linear_rows(x, None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, norm_w,
@@ -391,6 +394,17 @@ def _bf16_rows(x: torch.Tensor) -> torch.Tensor:
     xb = torch.empty(x.shape, dtype=BF16, device=x.device)
     ext().cast_bf16(x, xb)
     return xb
+
+
+def _bf16_operand(x: torch.Tensor) -> torch.Tensor:
+    """``x`` as contiguous bf16 rows, whatever its strides and size."""
+    return _bf16_rows(x) if x.is_contiguous() and x.numel() % 8 == 0 else x.to(BF16).contiguous()
+
+
+def _mid_rows(x: torch.Tensor, w: torch.Tensor, act: int = ACT_NONE) -> bool:
+    """Whether the rows ``x`` of a dense product on ``w`` are rounded to bf16 (the operand they would be rounded to anyway) for the
+    tiles for some ten to a few hundred rows (csrc: rows_mid.hip, which takes up to ``FEW_ROWS`` as they are)."""
+    return x.shape[0] > FEW_ROWS and w.dtype == BF16 and ext().rows_mid_takes(x.shape[0], w, int(act))
 
 
 def prompt_bf16(m: int, cols: int, wdtype) -> bool:
@@ -471,6 +485,9 @@ def linear_add_(res: torch.Tensor, x, w: torch.Tensor) -> torch.Tensor:
     x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], w.shape[0])
     if not _gpu(x):
         return res.add_(_round_like(x, w) @ w.float().t())
+    if norm_w is None and res.is_contiguous() and _mid_rows(x, w):
+        ext().linear_rows(_bf16_operand(x), None, w, res, None, None, None, x.shape[0], ACT_NONE, 0.0, 1.0, None, None, 0.0, 0, True)
+        return res
     if norm_w is None and res.is_contiguous() and _use_packed_gemm(x, w):
         from . import linear_residual as packed_linear_residual
         return packed_linear_residual(_bf16_rows(x), _packed_weight(w), res)
