@@ -420,7 +420,8 @@ void gemm(Tensor x, Tensor w, int64_t n, int64_t k, Tensor out, int64_t mode, bo
   if (pack_out.has_value()) {
     check(m <= SKINNY_MAX_M && (mode == 1 || mode == 2) && (mode != 1 || mir), "gemm pack_out: decode M, residual "
           "(with its mirror) or SwiGLU");
-    check(ksplit > 1 || tile == 11 || tile == 12, "gemm pack_out: the split-K reduce-kernel path only");
+    check(ksplit > 1 || tile == 11 || tile == 12 || jla::linear_mid_tile((int)tile), "gemm pack_out: the split-K reduce-kernel path, or "
+          "the tiles of mid-sized batches, only");
     pqa.pack = packed_ptr(pack_out, m, mode == 2 ? n / 2 : n, "pack_out");
   }
   if (tile == 11 || tile == 12) {  // gemm5 (weight-streaming) partial slabs + the reduce kernel's epilogue, any split
@@ -786,7 +787,7 @@ void gemm_tp_residual(int64_t state, Tensor x, Tensor w, int64_t n, int64_t k, T
   const int64_t groups = jla::gemm_tp_groups((int)m, (int)n);
   check(groups <= jla::CAR_WG_COUNTERS && groups * jla::TPRES_REGION <= jla::car_max_bytes(st),
         "gemm_tp_residual: the output does not fit the fused exchange buffer");
-  const bool g5 = tile == 11 || tile == 12;
+  const bool g5 = tile == 11 || tile == 12 || jla::linear_mid_tile((int)tile);  // (slabs at any split)
   check(g5 || ksplit > 1, "gemm_tp_residual: a split-K plan (the exchange lives in the reduce)");
   if (g5)
     check_g5_ws(ws, k, ksplit, m, n, false);
@@ -918,7 +919,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_dbg for the bounds-chec
   m.def("bounds_error", [](bool reset) {
     const int r = reset ? 1 : 0;
     return (int64_t)(jla::jla_bounds_norm_embed(r) | jla::jla_bounds_rope_kv(r) | jla::jla_bounds_sample(r) |
-                     jla::jla_bounds_gemm(r) | jla::jla_bounds_gemv(r) |
+                     jla::jla_bounds_gemm(r) | jla::jla_bounds_linear_mid(r) | jla::jla_bounds_gemv(r) |
                      jla::jla_bounds_attn_decode(r) | jla::jla_bounds_attn_prefill(r));
   }, "OR of the bounds-checked debug build's error words (JLA_BOUNDS_* bits); always 0 in a release build",
         py::arg("reset") = false);
@@ -962,6 +963,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_dbg for the bounds-chec
        "clock_probe");
   });
   m.def("gemm5_set_diag", [](int64_t d) { jla::gemm5_set_diag((int)d); });
+  m.def("linear_mid_plan", [](int64_t mm, int64_t n, int64_t k) {  // (K split, tile config; 0: none takes the sizes)
+    int ks = 1;
+    const int tile = mm > 0x7fffffff ? 0 : jla::linear_mid_plan((int)mm, (int)n, (int)k, &ks);
+    return std::make_pair(ks, tile);
+  });
+  m.attr("LINEAR_MID_TILE") = jla::LINEAR_MID_TILE;
+  m.attr("LINEAR_MID_MAX_M") = jla::LINEAR_MID_MAX_M;
   m.def("gemm5_ksplit", [](int64_t k, int64_t ks) { return jla::gemm5_ksplit((int)k, (int)ks); });
   m.def("attn_set_v6", [](int64_t mode) { jla::attn_set_v6((int)mode); });
   m.def("attn_set_v6_wpp", [](int64_t wpp) { jla::attn_set_v6_wpp((int)wpp); });

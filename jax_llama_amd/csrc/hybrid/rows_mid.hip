@@ -26,7 +26,7 @@ JLA_DEV void rm_store(const RowLinear& p, int d, int col, f32x4 v) {
 // grid: tiles x splits, rounded up to 8; slabs (several splits): [splits][R][weight rows] partial sums instead of the output.
 // gated: the 16-column tiles of a wave are gate and up tiles in turn (NT even).
 template <int MT, int NT, int WN, int WK, int S, int XB>
-__global__ void __launch_bounds__(64 * WN * WK) rows_mid_kernel(RowLinear p, int gated, int tiles_n, int splits, int steps, float* slabs) {
+__global__ void __launch_bounds__(64 * WN * WK, 2) rows_mid_kernel(RowLinear p, int gated, int tiles_n, int splits, int steps, float* slabs) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
   __shared__ u32x4 lds[H::LDS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
@@ -44,7 +44,8 @@ __global__ void __launch_bounds__(64 * WN * WK) rows_mid_kernel(RowLinear p, int
     return wbase + (size_t)(gated && (j & 1) ? N + col : col) * K * 2;
   };
   f32x4 acc[NT][MT];
-  mid_tile<MT, NT, WN, WK, S, XB, false>(lds, xrow, wrow, t0, t1, acc, [](int, const u32x4 (&)[MT]) {});
+  float none[1];
+  mid_tile<MT, NT, WN, WK, S, XB, false, false>(lds, xrow, wrow, t0, t1, acc, none);
   if (wave >= WN) return;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -99,16 +100,15 @@ static void rm_launch(unsigned grid, hipStream_t s, const RowLinear& p, int gate
 }
 #define RM_FORM(MT, NT, WN, WK, S, XB, ...) {MT, NT, WN, WK, XB, __VA_ARGS__, rm_launch<MT, NT, WN, WK, S, XB>}
 static const RmForm RM_FORMS[] = {
-    RM_FORM(1, 1, 1, 4, 4, 2, 4.14f, 0.342f, 0.462f, 1.53f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 2, 3.36f, 0.243f, 0.716f, 2.81f, 0.438f),
-    RM_FORM(1, 2, 4, 1, 8, 2, 3.06f, 0.413f, 0.977f, 3.35f, 0.814f), RM_FORM(2, 1, 1, 4, 3, 2, 4.64f, 0.481f, 0.411f, 1.23f, 0.706f),
-    RM_FORM(2, 1, 4, 1, 6, 2, 4.61f, 0.285f, 0.658f, 1.79f, 0.301f), RM_FORM(2, 2, 4, 1, 6, 2, 6.37f, 0.374f, 1.12f, 0.381f, 0.523f),
-    RM_FORM(4, 1, 1, 4, 3, 2, 6.64f, 0.577f, 1.5f, 0.0f, 0.793f), RM_FORM(4, 1, 4, 1, 4, 2, 6.18f, 0.344f, 0.666f, 0.701f, 0.247f),
-    RM_FORM(4, 2, 4, 1, 4, 2, 7.42f, 0.446f, 1.2f, 0.0f, 0.311f), RM_FORM(6, 2, 4, 1, 4, 2, 8.0f, 0.586f, 1.17f, 0.104f, 0.283f),
-    RM_FORM(8, 2, 4, 1, 4, 2, 8.0f, 0.787f, 1.14f, 0.84f, 0.236f), RM_FORM(8, 2, 8, 1, 3, 2, 8.0f, 1.06f, 1.0f, 1.52f, 0.198f),
-    RM_FORM(1, 1, 1, 4, 4, 4, 4.63f, 0.422f, 1.28f, 1.74f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 4, 3.73f, 0.307f, 0.912f, 2.31f, 1.0f),
-    RM_FORM(1, 2, 4, 1, 8, 4, 3.24f, 0.438f, 0.957f, 3.29f, 0.886f), RM_FORM(2, 1, 1, 4, 3, 4, 5.43f, 0.63f, 1.33f, 1.33f, 1.0f),
-    RM_FORM(2, 1, 4, 1, 6, 4, 6.23f, 0.346f, 0.967f, 0.0f, 0.8f), RM_FORM(2, 2, 4, 1, 6, 4, 6.95f, 0.457f, 1.02f, 0.0f, 0.625f),
-    RM_FORM(4, 1, 4, 1, 4, 4, 6.81f, 0.48f, 0.998f, 0.0f, 0.513f), RM_FORM(4, 2, 4, 1, 4, 4, 7.62f, 0.641f, 1.0f, 0.0f, 0.4f),
+    RM_FORM(1, 1, 1, 4, 4, 2, 3.83f, 0.416f, 0.231f, 1.64f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 2, 2.99f, 0.214f, 0.768f, 2.94f, 0.395f),
+    RM_FORM(1, 2, 4, 1, 8, 2, 3.36f, 0.352f, 1.03f, 2.77f, 0.753f), RM_FORM(2, 1, 1, 4, 3, 2, 3.92f, 0.73f, 0.1f, 1.23f, 0.926f),
+    RM_FORM(2, 1, 4, 1, 6, 2, 3.69f, 0.225f, 0.851f, 2.55f, 0.284f), RM_FORM(2, 2, 4, 1, 6, 2, 4.93f, 0.352f, 1.2f, 1.54f, 0.474f),
+    RM_FORM(4, 1, 4, 1, 4, 2, 3.14f, 0.345f, 0.73f, 3.08f, 0.224f), RM_FORM(4, 2, 4, 1, 4, 2, 6.92f, 0.43f, 1.28f, 0.0f, 0.323f),
+    RM_FORM(6, 2, 4, 1, 4, 2, 7.82f, 0.472f, 1.32f, 0.0f, 0.282f), RM_FORM(8, 2, 4, 1, 4, 2, 8.0f, 0.672f, 1.25f, 0.233f, 0.222f),
+    RM_FORM(1, 1, 1, 4, 4, 4, 4.58f, 0.455f, 1.24f, 1.84f, 1.0f), RM_FORM(1, 1, 4, 1, 8, 4, 4.02f, 0.232f, 0.932f, 1.99f, 1.0f),
+    RM_FORM(1, 2, 4, 1, 8, 4, 3.74f, 0.389f, 0.983f, 2.47f, 0.83f), RM_FORM(2, 1, 1, 4, 3, 4, 4.7f, 0.882f, 1.29f, 1.48f, 1.0f),
+    RM_FORM(2, 1, 4, 1, 6, 4, 5.62f, 0.312f, 0.963f, 0.618f, 0.779f), RM_FORM(2, 2, 4, 1, 6, 4, 6.8f, 0.434f, 1.06f, 0.0f, 0.595f),
+    RM_FORM(4, 1, 4, 1, 4, 4, 6.66f, 0.436f, 1.02f, 0.0f, 0.484f), RM_FORM(4, 2, 4, 1, 4, 4, 7.55f, 0.601f, 1.09f, 0.0f, 0.382f),
 };
 #undef RM_FORM
 constexpr int RM_MAX_SPLITS = 16;
@@ -119,31 +119,31 @@ struct RmPlan {
   float us = 1e30f;
 };
 
-// ... of rows: with experts, whose counts only the device knows, a standard deviation above the mean each
+// ... of rows: with experts, whose counts only the device knows, one and a half standard deviations above the mean each
 static long long rm_row_tiles(const RowLinear& p, int bm) {
   if (!p.offs) return (p.R + bm - 1LL) / bm;
   const int E = p.E < p.R ? p.E : p.R;
-  const float mean = (float)p.R / (float)E, most = p.even_rows > 0 ? mean : mean + sqrtf(mean);
+  const float mean = (float)p.R / (float)E, most = p.even_rows > 0 ? mean : mean + 1.5f * sqrtf(mean);
   return E * (long long)ceilf(most / (float)bm);
 }
 
-// The form and split with the least time by the figures above: on average 1.9 % above the best of all that were measured (467 shapes: one
-// matrix, 8 and 32 experts, N 64 to 32000, K 512 to 14336, 9 to 1000 rows)
+// The form and split with the least time by the figures above: on average 2.0 % above the best of all that were measured (384 shapes: one
+// matrix, 8 and 32 experts, N 64 to 32000, K 512 to 14336, 9 to 3200 rows)
 static RmPlan rm_plan(const RowLinear& p) {
   const int gated = hy_act_gated(p.act), T = p.K >> 6, xb = p.a_bf16 ? 2 : 4, E = p.offs ? (p.E < p.R ? p.E : p.R) : 1;
   const long long nw = gated ? 2LL * p.N : p.N;
   const float stream = (float)E * (float)nw * (float)p.K * 2 / 5.4e6f;  // the weights themselves
   RmPlan best;
   for (const RmForm& f : RM_FORMS) {
-    if (f.xb != xb || (gated && f.nt % 2)) continue;
+    if (f.xb != xb || (gated && f.nt % 2) || T % f.wk) continue;
     const long long tiles = rm_row_tiles(p, 16 * f.mt) * ((nw + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
     int last = 0;
     for (int want = 1; want <= RM_MAX_SPLITS && want <= T; ++want) {
-      const int steps = (T + want - 1) / want, splits = (T + steps - 1) / steps;
+      const int steps = ((T + want - 1) / want + f.wk - 1) / f.wk * f.wk, splits = (T + steps - 1) / steps;
       if (splits == last || (want > 1 && (steps < 2 * f.wk || tiles * splits > 700))) continue;
       last = splits;
       const float load = (float)(tiles * splits) / 256.f, deep = load > 2.f ? load + .3f : (load > 1.f ? 2.f : 1.f);
-      float us = f.fill + f.stage * (float)((steps + f.wk - 1) / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
+      float us = f.fill + f.stage * (float)(steps / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
       if (us < 3.5f + stream) us = 3.5f + stream;
       if (splits > 1) us += f.sum + .15f * (float)splits + f.mb * (float)p.R * (float)nw * (float)splits * 8e-6f;
       if (f.wk > 1 && load > 2.f) us *= 3.f;  // (16 columns a workgroup: x over and over)
@@ -157,12 +157,14 @@ static RmPlan rm_plan(const RowLinear& p) {
 //  * fp32 rows of one matrix, 9 to 64 (more: the caller rounds them first; their bytes are x's twice). Up to 24 rows of K below 1024
 //    rows_gemv.hip: 512 x 512, 16 rows 4.7 us there, 5.5 here; 1024 x 1024 6.1 both.
 //  * bf16 rows of one matrix: to 255; from 256 on a prompt's rows have the 256-row tiles (us here | there, weights in no cache: 2048 x 2048,
-//    255 | 777 rows 16 | 18, 27 | 25 with its sums; 4096 x 4096, 255 | 300 24.6 | 25.5, 29.9 | 27.7; 8224 x 2048, 300 33.2 | 31.4).
+//    255 | 777 rows 16 | 18, 27 | 25 with its sums; 4096 x 4096, 255 | 300 24.6 | 25.5, 29.9 | 27.7; 8224 x 2048, 300 33.2 | 31.4), and
+//    wide outputs from 129 (32000 x 2048, 128 | 200 rows 48.5 | 47.4, 59 | 49; gated 14336 x 4096, 200 92 | 87).
 //  * rows by expert: more than 64 up to 112 per expert on average (8 experts, gated 2816 x 2048 and down, 96 | 320 | 800 rows 50 | 98, 49 | 92,
-//    54 | 75 and 20 | 63, 22 | 50, 31 | 52; 128 per expert 80 | 78 and 39 | 54, 32 experts 241 | 267 and 135 | 109), of K below 256
+//    66 | 75 and 22 | 63, 26 | 50, 31 | 52; 128 per expert 80 | 78 and 39 | 54, 32 experts 241 | 267 and 135 | 109), of K below 256
 //    to 64 (16 per-head matrices of 512 x 128, 64 | 80 rows each 7.0 | 8.1, 10.9 | 8.1). Up to 64 rows in all rows_gemv.hip, unless there
 //    are five per expert on large matrices (8 experts, 56 rows: gated 7168 x 4096 171 | 213, 4096 x 7168 82 | 106; gated 2816 x 2048 51 | 48, gated 512 x 1024 11 | 8).
 constexpr int RM_MIN_ROWS = 9, RM_F32_ROWS = 64, RM_FEW_ROWS = 24, RM_FEW_K = 1024, RM_ROWS = 255;
+constexpr int RM_WIDE = 16384, RM_WIDE_ROWS = 128;
 constexpr long long RM_SORTED_WORK = 20000000;
 constexpr int RM_EXPERT_ROWS = 112, RM_SORTED_ROWS = 64, RM_SHORT_K = 256, RM_SHORT_ROWS = 64;
 
@@ -178,7 +180,7 @@ bool hy_rows_mid_takes(const RowLinear& p) {
     return !p.a_bf16 && p.R >= 5LL * p.E && nw >= 4096 && nw * p.K >= RM_SORTED_WORK;
   }
   if (!p.a_bf16) return p.R <= RM_F32_ROWS && !(p.R <= RM_FEW_ROWS && p.K < RM_FEW_K);
-  return p.R <= RM_ROWS;
+  return p.R <= (nw > RM_WIDE ? RM_WIDE_ROWS : RM_ROWS);
 }
 
 long long hy_rows_mid_floats(const RowLinear& p) {

@@ -20,6 +20,7 @@
 #include "common.h"
 #include "gemm4w.h"
 #include "gemm5ws.h"
+#include "gemm_out.h"
 #include "launchers.h"
 #include "ring.h"
 
@@ -1113,74 +1114,18 @@ __global__ void __launch_bounds__(256)
     v.z *= rs;
     v.w *= rs;
   }
-  float vv[4] = {v.x, v.y, v.z, v.w};
+  const float vv[4] = {v.x, v.y, v.z, v.w};
   if constexpr (MODE == MODE_SWIGLU) {
     // gate tile t = 2p holds columns [32p, 32p+16), the up tile the next 16: pair the two halves
-    const int tile = col >> 4, c0 = col & 15;  // tile is even: the gate half of the pair
     float4 u = sum_splits(ws, ksplit, slab4, e4 + 4);
     u.x *= rs;
     u.y *= rs;
     u.z *= rs;
     u.w *= rs;
     const float uu[4] = {u.x, u.y, u.z, u.w};
-    bf16_t* o = static_cast<bf16_t*>(out) + (size_t)m * (N >> 1) + (tile >> 1) * 16 + c0;
-    const uint2 pk = make_uint2(pack2bf(silu(vv[0]) * uu[0], silu(vv[1]) * uu[1]),
-                                pack2bf(silu(vv[2]) * uu[2], silu(vv[3]) * uu[3]));
-    *reinterpret_cast<uint2*>(o) = pk;
-    // decode M: also the packed copy (common.h pack_off) the next projection's packed-x GEMV reads
-    if (qa.pack) *reinterpret_cast<uint2*>(qa.pack + pack_off(m, (tile >> 1) * 16 + c0, N >> 1)) = pk;
-  } else if constexpr (MODE == MODE_RESIDUAL) {
-    float4* o = reinterpret_cast<float4*>(static_cast<float*>(out) + idx);
-    float4 r = *o;
-    if (accumulate) {
-      r.x += vv[0];
-      r.y += vv[1];
-      r.z += vv[2];
-      r.w += vv[3];
-    } else {
-      r = make_float4(vv[0], vv[1], vv[2], vv[3]);
-    }
-    *o = r;
-    if (mirror) {
-      const uint2 pk = make_uint2(pack2bf(r.x, r.y), pack2bf(r.z, r.w));
-      *reinterpret_cast<uint2*>(mirror + idx) = pk;
-      if (qa.pack) *reinterpret_cast<uint2*>(qa.pack + pack_off(m, col, N)) = pk;  // packed copy of the mirror
-    }
-  } else if constexpr (MODE == MODE_QKV) {
-    const int head = col / qa.Dh, d0 = col - head * qa.Dh;
-    const int b = m / qa.S, sq = m - b * qa.S;
-    if (head < qa.H + qa.Hkv) {
-      int pos = qa.positions[m];
-      if (pos < 0 || pos >= qa.table_len) JLA_FLAG(JLA_BOUNDS_ROPE_POS);
-      pos = pos < 0 ? 0 : (pos >= qa.table_len ? qa.table_len - 1 : pos);
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const float2 cs = qa.table[(size_t)pos * (qa.Dh >> 1) + (d0 >> 1) + p];
-        const float xr = vv[2 * p], xi = vv[2 * p + 1];
-        vv[2 * p] = xr * cs.x - xi * cs.y;
-        vv[2 * p + 1] = xr * cs.y + xi * cs.x;
-      }
-    }
-    const uint2 packed = make_uint2(pack2bf(vv[0], vv[1]), pack2bf(vv[2], vv[3]));
-    if (head < qa.H) {
-      *reinterpret_cast<uint2*>(qa.q + ((size_t)m * qa.H + head) * qa.Dh + d0) = packed;
-    } else {
-      const int slot = qa.slot[0] + sq;
-      if (slot < qa.T) {
-        const bool is_k = head < qa.H + qa.Hkv;
-        const int kh = is_k ? head - qa.H : head - qa.H - qa.Hkv;
-        bf16_t* cache = is_k ? qa.kc : qa.vc;
-        *reinterpret_cast<uint2*>(cache + (((size_t)b * qa.Hkv + kh) * qa.T + slot) * qa.Dh + d0) = packed;
-      } else {
-        JLA_FLAG(JLA_BOUNDS_KV_SLOT);
-      }
-    }
+    gemm_out4<MODE>(vv, uu, m, col, N, out, accumulate, out_f32, mirror, qa);
   } else {
-    if (out_f32)
-      *reinterpret_cast<float4*>(static_cast<float*>(out) + idx) = make_float4(vv[0], vv[1], vv[2], vv[3]);
-    else
-      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out) + idx) =
-          make_uint2(pack2bf(vv[0], vv[1]), pack2bf(vv[2], vv[3]));
+    gemm_out4<MODE>(vv, vv, m, col, N, out, accumulate, out_f32, mirror, qa);
   }
 }
 
@@ -1307,7 +1252,7 @@ static bool use_g4(int tile, int M, int K);
 constexpr int G4N6D_TILE = 16;  // 256 x 192 tiles (g4n_mainloop<6, W3>)
 constexpr int G4ND_TILE = 17;   // 256 x 128 tiles (g4n_mainloop<4, W3>)
 int gemm_qkv_direct_ok(int M, int tile, int K) {
-  return ((tile == 0 || tile == 1) && tile_cfg(tile, M) == 1) || use_g4(tile, M, K) ||
+  return linear_mid_tile(tile) || ((tile == 0 || tile == 1) && tile_cfg(tile, M) == 1) || use_g4(tile, M, K) ||
          (tile == G4N6D_TILE && (K & 63) == 0);
 }
 
@@ -1589,9 +1534,29 @@ static int launch_g5(const bf16_t* x, const u32x4* w, void* out, int M, int N, i
   return launch_reduce(ws, ksplit, out, M, N, K, mode, accumulate, out_f32, mirror, qkv, ssq, rms_eps, s);
 }
 
+// the tiles for mid-sized batches (linear_mid.hip): the epilogue in their launch, or behind slabs in the reduce kernel
+static int launch_mid(const bf16_t* x, const void* w, void* out, int M, int N, int K, int mode, int accumulate, int out_f32,
+                      bf16_t* mirror, const QKVArgs* qkv, float* ws, size_t ws_floats, int ksplit, float rms_eps, int tile,
+                      hipStream_t s) {
+  if (M <= 0) return 0;
+  if ((mode == MODE_SWIGLU && (N & 31)) || (mode == MODE_QKV && !qkv) || mode == MODE_ARGMAX) return -1;
+  if (rms_eps >= 0.f && (mode == MODE_RESIDUAL || mode == MODE_TPRESID)) return -5;  // caller pre-scales x instead
+  ksplit = gemm5_ksplit(K, ksplit);
+  if (ksplit == 1 && mode != MODE_TPRESID)
+    return linear_mid(x, w, out, M, N, K, mode, accumulate, out_f32, mirror, qkv, nullptr, nullptr, 1, rms_eps, tile, s);
+  const bool rms = rms_eps >= 0.f;
+  const size_t need = (size_t)ksplit * M * N + (rms ? (size_t)ksplit * M : 0);
+  if (ws == nullptr || ws_floats < need) return -3;
+  float* ssq = rms ? ws + (size_t)ksplit * M * N : nullptr;
+  const int r = linear_mid(x, w, nullptr, M, N, K, MODE_STORE, 0, 1, nullptr, nullptr, ws, ssq, ksplit, rms_eps, tile, s);
+  return r ? r : launch_reduce(ws, ksplit, out, M, N, K, mode, accumulate, out_f32, mirror, qkv, ssq, rms_eps, s);
+}
+
 int gemm(const bf16_t* x, const void* W, void* out, int M, int N, int K, int mode, int accumulate, int out_f32,
          bf16_t* mirror, const QKVArgs* qkv, float* ws, size_t ws_floats, int ksplit, hipStream_t s,
          float rms_eps, int tile, float* rms_ws, size_t rms_ws_floats) {
+  if (linear_mid_tile(tile))
+    return launch_mid(x, W, out, M, N, K, mode, accumulate, out_f32, mirror, qkv, ws, ws_floats, ksplit, rms_eps, tile, s);
   if (tile == G5_TILE || tile == G5_TILE + 1) {
     if (mode == MODE_ARGMAX || (rms_eps >= 0.f && (mode == MODE_RESIDUAL || mode == MODE_TPRESID))) return -1;
     return launch_g5(x, static_cast<const u32x4*>(W), out, M, N, K, mode, accumulate, out_f32, mirror, qkv, ws,

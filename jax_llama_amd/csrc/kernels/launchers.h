@@ -79,6 +79,13 @@ int gemm_qkv_direct_ok(int M, int tile, int K);  // qkv without a K split: the d
 void gemm_set_g4_default(int on);
 void gemm_set_g4_group(int gm);
 int gemm5_ksplit(int K, int ksplit);
+// Tiles of 32 to 128 rows for mid-sized batches and short prompts (linear_mid.hip), tile configs LINEAR_MID_TILE + form: the form and K split
+// with the least expected time (0: none takes the sizes); the product of one, or its partial sums (slabs, ssq as gemm5's)
+constexpr int LINEAR_MID_TILE = 32, LINEAR_MID_MIN_M = 17, LINEAR_MID_MAX_M = 256;
+bool linear_mid_tile(int tile);
+int linear_mid_plan(int M, int N, int K, int* ksplit);
+int linear_mid(const bf16_t* x, const void* W, void* out, int M, int N, int K, int mode, int accumulate, int out_f32, bf16_t* mirror,
+               const QKVArgs* qkv, float* slabs, float* ssq, int ksplit, float rms_eps, int tile, hipStream_t s);
 int clock_probe(int iters, int grid, unsigned long long* out, hipStream_t s);  // [cycles, 100 MHz ticks]
 void gemm5_set_diag(int d);  // tools only: gemm5 ablations (wrong results)  // gemm5 (tiles 11 / 12): the effective split over 64-deep K-stages
 size_t gemm_workspace_floats(int M, int N, int K);
@@ -118,6 +125,7 @@ unsigned jla_bounds_norm_embed(int reset);
 unsigned jla_bounds_rope_kv(int reset);
 unsigned jla_bounds_sample(int reset);
 unsigned jla_bounds_gemm(int reset);
+unsigned jla_bounds_linear_mid(int reset);
 unsigned jla_bounds_gemv(int reset);
 unsigned jla_bounds_attn_decode(int reset);
 unsigned jla_bounds_attn_prefill(int reset);

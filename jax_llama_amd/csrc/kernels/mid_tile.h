@@ -32,15 +32,35 @@ JLA_DEV int mid_cell(int x, int r, int xb) {
   return x ^ (xb == 4 ? (int)(0x32765410u >> (4 * s)) & 7 : s);
 }
 
-// acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 m + c of the tile at weight columns 4 q .. + 3 of this wave's 16-column
-// tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64; t0 < t1. xrow(r), wrow(r): the address of row r of the
-// tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py pack_frag16x32).
-// SS: squares(row fragment) is called once for every x fragment of the stages, by one wave each: (m, fragment).
-template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, class XRow, class WRow, class Squares>
-JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], Squares squares) {
+// Row tiles whose squares a wave sums (SS below), and the row tile that accumulator m of wave wn of a K group belongs to: with SS each
+// wave starts with those that are its own.
+template <int MT, int WN>
+constexpr int MID_SQ = (MT + WN - 1) / WN;
+template <int MT, int WN, bool SS>
+JLA_DEV int mid_row_tile(int m, int wn) {
+  return SS ? (m + wn * MID_SQ<MT, WN>) % MT : m;
+}
+
+// The sums are pinned to the matrix unit's own registers: with one wave per SIMD, and registers to spare, the compiler copied them there
+// and back at the loop's edge. PAD: an operand comes from the vector unit, whose writes a product may read two states later (those from
+// LDS are waited for).
+template <bool PAD>
+JLA_DEV void mid_mfma(f32x4& acc, const u32x4& w, const u32x4& x) {
+  if constexpr (PAD) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
+}
+
+// acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 mid_row_tile(m) + c of the tile at weight columns 4 q .. + 3 of this wave's
+// 16-column tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64, a positive multiple of WK. xrow(r), wrow(r): the address of row r
+// of the tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py
+// pack_frag16x32). SS (bf16 rows): ss[m] is this lane's share of the squares of row 16 mid_row_tile(m) + c, over quarters q and K groups
+// (the row tiles beyond MT, counted from wn MID_SQ on, are another wave's). The waves deal the row tiles, without a branch, which would
+// keep a stage's reads and products apart.
+template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, bool SS, class XRow, class WRow>
+JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], float (&ss)[SS ? MID_SQ<MT, WN> : 1]) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, q = lane >> 4;
-  const int wn = wave % WN, wk = wave / WN, ns = (t1 - t0 + WK - 1) / WK;
+  const int wn = wave % WN, wk = wave / WN, ns = (t1 - t0) / WK;
   const char* src[H::OPS];
 #pragma unroll
   for (int i = 0; i < H::OPS; ++i) {
@@ -70,47 +90,85 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) {
+      acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[t][m]));
+    }
+#pragma unroll
+  for (int m = 0; m < (SS ? MID_SQ<MT, WN> : 1); ++m) ss[m] = 0.f;
+  int xat[MT];  // where accumulator m's rows start in a slice (wave-uniform)
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xat[m] = 128 * mid_row_tile<MT, WN, SS>(m, wn);
+  constexpr int XR = XB / 2;  // 16-byte reads of an x fragment
+  auto read_w = [&](u32x4& w, int slot, int h, int t) {
+    const u32x4* ws = lds + slot * H::SLOT + wk * H::SLICE + H::XP * 64 + wn * NT * 128;
+    w = ws[PACKED ? (2 * t + h) * 64 + lane : (16 * t + c) * 8 + mid_cell(4 * h + q, c, 2)];
+  };
+  auto read_x = [&](u32x4 (&x)[XR], int slot, int h, int m) {
+    const u32x4* xs = lds + slot * H::SLOT + wk * H::SLICE + xat[m] + c * 8;
+    if constexpr (XB == 2) {
+      x[0] = xs[mid_cell(4 * h + q, c, 2)];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) x[i] = xs[h * H::BM * 8 + mid_cell(2 * q + i, c, 4)];
+    }
+  };
+  // the products of half a stage, with the reads of the next half (of slot, h) between them
+  auto half = [&](u32x4 (&w)[NT], u32x4 (&x)[MT][XR], u32x4 (&wnext)[NT], u32x4 (&xnext)[MT][XR], int slot, int h) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) read_w(wnext[t], slot, h, t);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      u32x4 f = x[m][0];
+      if constexpr (XB == 4) {
+        const f32x4 a = __builtin_bit_cast(f32x4, x[m][0]), b = __builtin_bit_cast(f32x4, x[m][1]);
+        const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        f = pack8(v);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) mid_mfma<XB == 4>(acc[t][m], w[t], f);
+      if constexpr (SS) {
+        if (m < MID_SQ<MT, WN>) {  // (plain FMAs: a dot product beside the products costs them more)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float lo = __uint_as_float(f[i] << 16), hi = __uint_as_float(f[i] & 0xffff0000u);
+            ss[m] = fmaf(lo, lo, ss[m]);
+            ss[m] = fmaf(hi, hi, ss[m]);
+          }
+        }
+      }
+      read_x(xnext[m], slot, h, m);
+    }
+  };
+  u32x4 w0[NT], w1[NT], x0[MT][XR], x1[MT][XR];
 #pragma unroll
   for (int s = 0; s < S - 1; ++s) issue(s, s);
+  wait_vmcnt<(S - 2) * H::OPS>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < NT; ++t) read_w(w0[t], 0, 0, t);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) read_x(x0[m], 0, 0, m);
   int slot = 0, fill = S - 1;
   for (int st = 0; st < ns; ++st) {
-    // this wave's pieces of stage st have landed, then every wave's; and every wave is past the slot that is filled next
-    wait_vmcnt<(S - 2) * H::OPS>();
+    half(w0, x0, w1, x1, slot, 1);
+    // this wave's pieces of stage st + 1 have landed, then every wave's; and every wave is past the slot that is filled next (its
+    // reads of stage st - 1 were behind the products before this barrier)
+    wait_vmcnt<(S - 3) * H::OPS>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     issue(st + S - 1, fill);
-    if (t0 + st * WK + wk < t1) {  // (wave-uniform)
-      const u32x4* xs = lds + slot * H::SLOT + wk * H::SLICE;
-      const u32x4* ws = xs + H::XP * 64 + wn * NT * 128;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        u32x4 wf[NT], xf[MT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) wf[t] = ws[PACKED ? (2 * t + h) * 64 + lane : (16 * t + c) * 8 + mid_cell(4 * h + q, c, 2)];
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          if constexpr (XB == 2) {
-            xf[m] = xs[(16 * m + c) * 8 + mid_cell(4 * h + q, c, 2)];
-          } else {
-            const u32x4* at = xs + (h * H::BM + 16 * m + c) * 8;
-            const f32x4 a = __builtin_bit_cast(f32x4, at[mid_cell(2 * q, c, 4)]), b = __builtin_bit_cast(f32x4, at[mid_cell(2 * q + 1, c, 4)]);
-            const float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-            xf[m] = pack8(f);
-          }
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int t = 0; t < NT; ++t) acc[t][m] = mfma16x16x32(wf[t], xf[m], acc[t][m]);
-        squares(wn, xf);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     slot = slot + 1 == S ? 0 : slot + 1;
     fill = fill + 1 == S ? 0 : fill + 1;
+    half(w1, x1, w0, x0, slot, 0);  // (behind the last stage: reads that nothing uses)
   }
   wait_vmcnt<0>();
+  asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // the last products, before their sums are read
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) asm volatile("" : "+a"(acc[t][m]));
   if constexpr (WK > 1) {  // the K groups' sums
     f32x4* red = reinterpret_cast<f32x4*>(lds);
 #pragma unroll

@@ -303,9 +303,11 @@ def tiled_tp_residual(x: torch.Tensor, w, h: torch.Tensor, hb: torch.Tensor, sta
     m = x.shape[0]
     assert x.dtype == BF16 and x.is_contiguous(), (x.dtype, x.shape)
     ks, tm = autotune.choose_gemm_plan(e, m, w.n, w.k, x.device, MODE_STORE, False)
-    if tm not in G5_TILES and ks <= 1:
+    if not _slab_tile(tm) and ks <= 1:
         return False
     ks, tm, ws = _gemm_ws(e, m, w.n, w.k, x.device, MODE_STORE, False)
+    if ws is None:
+        ws = workspace.get("gemm_ws", m * (w.n + 1), torch.float32, x.device)
     e.gemm_tp_residual(state, x, w.weight, w.n, w.k, h, hb, ks, ws, tm)
     return True
 
@@ -332,6 +334,12 @@ def _tiled_input(x, rms_eps, fused=False):
 
 G4D_TILE = 14  # gemm4 with the weights three K-tiles deep
 G5_TILES = (11, 12)  # gemm5 weight-streaming split-K (csrc/kernels/gemm5ws.h): 256- / 128-column workgroups
+
+
+def _slab_tile(tm) -> bool:
+    """Tile configs whose partial sums can go through the reduce kernel without a K split too: gemm5, and the tiles of
+    mid-sized batches (csrc/kernels/linear_mid.hip)."""
+    return tm in G5_TILES or tm in autotune.MID_TILES
 
 
 def _gemm_ws(e, m, n, k, device, mode=MODE_STORE, rms=False):
@@ -375,13 +383,11 @@ def _tiled(e, x, weight, n, k, out, mode, rms_eps, accumulate, mirror=None, pack
 
 def _tiled_packs(e, m, n, k, device, mode, rms_eps) -> bool:
     """Whether the tiled GEMM's tuned plan for this decode shape can write a packed output copy: the plain split-K
-    path, whose reduce kernel runs the epilogue (not ks = 1)."""
+    path, whose reduce kernel runs the epilogue (not ks = 1), and the tiles of mid-sized batches."""
     if e is None or m > SKINNY_M or mode not in (MODE_RESIDUAL, MODE_SWIGLU):
         return False
     ks, tm = autotune.choose_gemm_plan(e, m, n, k, device, mode, _fused_rms(e, mode, rms_eps))
-    if tm in G5_TILES:
-        return True
-    return ks > 1
+    return _slab_tile(tm) or ks > 1
 
 
 def _variant(e, x, w, mode, x_packed=None, pack_out=None, no_split=False) -> int:

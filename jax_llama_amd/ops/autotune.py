@@ -11,7 +11,7 @@ seen during capture fall back to the static heuristic.
 
 Variants: 1 = GEMV 4 waves (1 or 2 tiles/WG), 5 = GEMV 4 tiles/WG, 6 = GEMV 2 tiles/WG, 10 = 2 tiles with a doubled
 register ring (M > 16, bf16 activations), 20 = 2 tiles x 8 waves, 16 = K over 2 workgroups, packed-x 12 / 15 / 18 / 21 /
-22 / 26, 7 = tiled MFMA GEMM with split-K (gemm.hip; a candidate for M > 16, always used for M > 64). ``JLA_GEMV_VARIANT`` pins one; ``JLA_AUTOTUNE=0`` disables tuning.
+22 / 26, 7 = tiled MFMA GEMM with split-K (gemm.hip, to 128 rows linear_mid.hip; a candidate for M > 16, always used for M > 64). ``JLA_GEMV_VARIANT`` pins one; ``JLA_AUTOTUNE=0`` disables tuning.
 
 Shipped picks: ``ops/tune_gfx950.json`` (measured on an MI355X for the bench, latency and tensor-parallel shapes) is
 loaded first, so plans are identical on every box and nothing is measured for those shapes; shapes it lacks are
@@ -82,7 +82,7 @@ def tune_file() -> str:
     return os.path.join(base, "jax_llama_amd", f"tune_{ARCH}.json")
 
 
-TUNE_VERSION = 12  # bumped when a candidate set changes (2: split-K GEMV 16-19; 3: 4-tile split-K 26; 4: gemm4 tile 7; 5: gemm4 stream-K; 6: never-picked GEMV variants removed; 7: gemm4 256 x 128 tiles; 8: gemm5 tiles 11 / 12; 9: gemm4 rasterised in groups of 4 m-tiles; 10: stream-K / hybrid plans replaced by the exchange split; 11: gemm4 with the weights three K-tiles deep, 256 x 192 tiles; 12: the never-picked tiles 8 / 10 / 15 removed), so older persisted picks are re-measured
+TUNE_VERSION = 13  # bumped when a candidate set changes (2: split-K GEMV 16-19; 3: 4-tile split-K 26; 4: gemm4 tile 7; 5: gemm4 stream-K; 6: never-picked GEMV variants removed; 7: gemm4 256 x 128 tiles; 8: gemm5 tiles 11 / 12; 9: gemm4 rasterised in groups of 4 m-tiles; 10: stream-K / hybrid plans replaced by the exchange split; 11: gemm4 with the weights three K-tiles deep, 256 x 192 tiles; 12: the never-picked tiles 8 / 10 / 15 removed; 13: linear_mid's tiles), so older persisted picks are re-measured
 
 
 def _key_str(kind: str, key: Tuple) -> str:
@@ -248,9 +248,6 @@ def _measure(x, w, run, cands) -> int:
     iters = 2 * copies
     graphs = {}
     for v in cands:
-        if v == TILED_VARIANT:  # its plan (and workspace) is chosen per call: timed eagerly (a long kernel anyway)
-            graphs[v] = None
-            continue
         g = torch.cuda.CUDAGraph()
         try:
             with torch.cuda.graph(g):
@@ -304,7 +301,11 @@ KS_CANDIDATES = (1, 2, 3, 4, 6, 8, 12, 16)
 # 256 / 128 columns per workgroup, M <= 256 per tile). What the bench shapes pick (BENCH_r05 gemm_plan_choice):
 #   Llama-3-8B M = 1024 / 2048: qkv 16 / 17, o 17, gate_up 7 / 14 / 16, down 14 / 17 (split 2), lm_head 14;
 #   Llama-3-70B M = 256 (MP 1 and the MP 8 shard): 1 / 3 (split 4 / 12), 11 / 12 (gemm5 splits), 14, 17.
-TILE_CANDIDATES = (1, 2, 3, 7, 11, 12, 14, 16, 17)
+# 32 to 38: the tiles of mid-sized batches (csrc/kernels/linear_mid.hip), the one of them and the split that its model picks. They win on
+#   narrow outputs (M = 200: 8192 x 1024 20.4 -> 13.1 us, 4096 x 4096 residual 23.9 -> 20.8, 1280 x 8192 24.2 -> 19.5) and lose on wide ones
+#   (28672 x 4096 gated 65 -> 79).
+MID_TILES = tuple(range(32, 39))
+TILE_CANDIDATES = (1, 2, 3, 7, 11, 12, 14, 16, 17, *MID_TILES)
 if os.environ.get("JLA_TUNE_TILES"):  # A/B tooling: restrict the tile candidates, e.g. JLA_TUNE_TILES=1,2,3,7,11,12
     TILE_CANDIDATES = tuple(int(v) for v in os.environ["JLA_TUNE_TILES"].split(","))
 # decode-sized M measured per shape (above: the C++ heuristic; prefill-sized M have enough 256 x 256 tiles)
@@ -322,6 +323,10 @@ def choose_gemm_plan(e, m: int, n: int, k: int, device, mode: int = 0, rms: bool
     plan = _KS_CACHE.get(key)
     if plan is not None:
         return plan
+    if m <= 128:  # the tiles of mid-sized batches, by their model (linear_mid.hip has both sides' times)
+        plan = e.linear_mid_plan(m, n, k)
+        if plan[1]:
+            return plan
     heur = e.gemm_ksplit(m, n, k)
     # tuned band: decode-sized M (prefill-sized M has enough 256x256 tiles; tuning it would also need
     # multi-GB scratch outputs)
@@ -361,9 +366,12 @@ def _measure_plan(e, m, n, k, device, heur, mode=0, rms=False) -> Tuple[int, int
         return c * m * (n + 1) * 4 <= TUNE_WS_BYTES
 
     ks_c = sorted({c for c in KS_CANDIDATES if kt // c >= 4 and fits(c)} | ({heur} if fits(heur) else set()) | {1})
-    cands = [(c, tm) for tm in TILE_CANDIDATES for c in ks_c
+    cands = [(c, tm) for tm in TILE_CANDIDATES if tm not in MID_TILES for c in ks_c
              if (tm not in G4N_TILES or (k % 64 == 0 and not (c > 1 and rms and mode != 1)))
              and (tm not in G5_TILES or (k % 64 == 0 and m <= 512))]
+    mid = e.linear_mid_plan(m, n, k)
+    if mid[1] in TILE_CANDIDATES and fits(mid[0]):
+        cands.append(mid)
     if k % 64 == 0 and m <= 512:  # gemm5 also at the deeper splits its 64-deep stages allow (narrow shards, long K)
         cands += [(c, tm) for tm in G5_TILES for c in (24, 32, 48) if (k // 64) // c >= 2 and c not in ks_c and fits(c)]
     nbytes = n * k * 2
