@@ -348,7 +348,11 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < VREG; ++i) reinterpret_cast<float*>(a.out)[(size_t)b * a.ldo + (size_t)h * vdim + VREG * lane + i] = o[i];
+  for (int i = 0; i < VREG; ++i) {
+    const size_t at = (size_t)b * a.ldo + (size_t)h * vdim + VREG * lane + i;
+    if (a.out_bf16) reinterpret_cast<bf16_t*>(a.out)[at] = f2bf(o[i]);
+    else reinterpret_cast<float*>(a.out)[at] = o[i];
+  }
 }
 
 // Heads of 64 or 128 numbers, up to about a wave per SIMD: more waves share a SIMD, and then the preparation in
@@ -371,7 +375,7 @@ int hy_attn_step(const AttnStep& p, hipStream_t s) {
   if (a.B < 0 || a.H < 1 || a.G < 1 || a.H % a.G || a.T < 1 || !hy_attn_step_takes(p)) return -1;
   if (a.bias && a.nbias < 1) return -3;
   if (a.chunk < 0 || a.window < 0 || a.keep_first < 0 || (a.chunk > 0 && a.window > 0)) return -7;
-  if (a.gate || a.out_bf16 || a.ldo < a.H * a.vdim) return -8;
+  if (a.gate || a.ldo < a.H * a.vdim) return -8;
   if (p.rope && (p.qk_half < 0 || 2 * p.qk_half > a.dim || p.v_half < 0 || 2 * p.v_half > a.vdim || !p.positions)) return -2;
   if (!p.rope && p.temp_coef != 0.f && (p.temp_every < 1 || !p.positions)) return -2;
   if (p.ld < a.H * a.dim + (p.own ? a.G * (a.dim + a.vdim) : 0)) return -4;

@@ -317,6 +317,21 @@ bool rows_mid_takes(int64_t rows, const Tensor& w, int64_t act) {
   return bf16_rows_linear(rows, w, act, p) && jla::hy_rows_mid_takes(p);
 }
 
+// whether it runs on one of the kernels for few rows; w [E, N, K]: E of them, `rows` rows each, in one launch
+bool rows_bf16_takes(int64_t rows, const Tensor& w, int64_t act) {
+  jla::RowLinear p{};
+  if (w.dim() == 3 && w.is_contiguous() && w.size(0) >= 1 && rows <= 0x7fffffff / w.size(0)) {
+    if (!bf16_rows_linear(rows, w.select(0, 0), act, p)) return false;
+    static const int32_t any = 0;
+    p.offs = &any;  // (asked of, not read)
+    p.E = w.size(0);
+    p.even_rows = rows;
+    p.R = rows * p.E;
+    return jla::hy_rows_bf16_takes(p);
+  }
+  return bf16_rows_linear(rows, w, act, p) && jla::hy_rows_bf16_takes(p);
+}
+
 void route_table(Tensor ids, Tensor table, int64_t E, Tensor row_expert, Tensor row_tok, Tensor sort_tok, Tensor sort_dst,
                  Tensor offs) {
   check(table.dim() == 2, "route_table: table is [vocab, top]");
@@ -784,7 +799,7 @@ bool attn_step(Tensor proj, Tensor kc, Tensor vc, Tensor slot, Tensor positions,
     check(head_scale->numel() == H, "attn_step: one factor per head");
     a.head_scale = f32(*head_scale, "head_scale");
   }
-  a.out = slice2d(out, "out", a.B, (int64_t)H * a.vdim, &a.ldo);
+  a.out = slice2d_any(out, "out", a.B, (int64_t)H * a.vdim, &a.ldo, &a.out_bf16);
   p.rope = rope;
   p.eps = eps; p.temp_coef = temp_coef; p.temp_every = temp_every;
   if (col_bias.has_value()) {
@@ -1042,11 +1057,12 @@ void rotate_heads(Tensor a, Tensor positions, OptT freq, int64_t H, double sign,
   const int64_t M = a.size(0), n = a.size(1) / H;
   int lda = 0, ldo = 0;
   const float* ap = slice2d(a, "a", M, H * n, &lda);
-  float* op = slice2d(out, "out", M, H * n, &ldo);
+  int bf = 0;
+  void* op = slice2d_any(out, "out", M, H * n, &ldo, &bf);
   const int half = freq.has_value() ? (int)freq->numel() : 0;
   check(offset >= 0 && offset + 2 * half <= n, "rotate_heads: more rotated numbers than a head holds");
   rc(jla::hy_rotate_heads(ap, lda, i32(positions, "positions", M), half ? f64(*freq, "freq") : nullptr, half, M, H, n,
-                          (float)sign, (float)gain, op, ldo, offset, interleaved, stream()),
+                          (float)sign, (float)gain, op, bf, ldo, offset, interleaved, stream()),
      "rotate_heads");
 }
 
@@ -1055,7 +1071,9 @@ void token_shift(Tensor h, Tensor prev, Tensor mu, Tensor out, int64_t B, int64_
   const int64_t n = mu.size(0), D = mu.size(1);
   check(!w.has_value() || w->numel() == D, "token_shift: w is [D]");
   check(h.numel() == B * S * D && prev.numel() == B * D && out.numel() == n * B * S * D, "token_shift shapes");
-  rc(jla::hy_token_shift(f32(h, "h"), f32w(prev, "prev"), f32(mu, "mu"), n, f32w(out, "out"), B, S, D,
+  const int bf = wtype(out, "out");
+  check(out.is_contiguous(), "token_shift: out is contiguous");
+  rc(jla::hy_token_shift(f32(h, "h"), f32w(prev, "prev"), f32(mu, "mu"), n, out.data_ptr(), bf, B, S, D,
                          w.has_value() ? f32(*w, "w") : nullptr, eps, stream()),
      "token_shift");
 }
@@ -1234,7 +1252,7 @@ void rec_step(int64_t mode, Tensor q, OptT k, Tensor v, OptT pre, OptT w0, OptT 
   p.w = f32(w, "w");
   p.w_heads = w.numel() != vdim || H == 1;
   p.eps = eps; p.gate_act = gate_act; p.gain = gain;
-  p.out = slice2d(out, "out", B, H * vdim, &p.ldo);
+  p.out = slice2d_any(out, "out", B, H * vdim, &p.ldo, &p.out_bf16);
   rc(jla::hy_rec_step(p, stream()), "rec_step");
 }
 
@@ -1262,7 +1280,7 @@ bool delta_step(Tensor proj, int64_t B, int64_t H, int64_t G, int64_t dim, int64
   p.w = f32(w, "w");
   p.w_heads = w.numel() != vdim || H == 1;
   p.eps = eps; p.gate_act = 0; p.gain = 1.f;
-  p.out = slice2d(out, "out", B, H * vdim, &p.ldo);
+  p.out = slice2d_any(out, "out", B, H * vdim, &p.ldo, &p.out_bf16);
   rc(jla::hy_rec_step(p, stream()), "delta_step");
   return true;
 }
@@ -1294,6 +1312,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dense_is_gemv", &dense_is_gemv);
   m.def("rows_gemm_pays", &rows_gemm_pays);
   m.def("rows_mid_takes", &rows_mid_takes);
+  m.def("rows_bf16_takes", &rows_bf16_takes);
   m.def("latent_prep", &latent_prep, py::arg("proj"), py::arg("col0"), py::arg("w"), py::arg("slot"), py::arg("B"),
         py::arg("S"), py::arg("cache"), py::arg("eps"), py::arg("q"), py::arg("q_col0") = 0,
         py::arg("q_norm_w") = py::none(), py::arg("rot_freq") = py::none(), py::arg("positions") = py::none(),

@@ -41,6 +41,8 @@ JLA_DEV float hy_head_squares(const f32x4 v) {
 }
 // ... whether heads of n numbers run in such groups, and L (0: they do not)
 inline int hy_head_lanes(int n) { return n % 4 || n > 256 ? 0 : (n <= 64 ? 16 : (n <= 128 ? 32 : 64)); }
+JLA_DEV void hy_store1(float* p, float v) { *p = v; }
+JLA_DEV void hy_store1(bf16_t* p, float v) { *p = f2bf(v); }
 JLA_DEV void hy_store4(float* p, const f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 JLA_DEV void hy_store4(bf16_t* p, const f32x4 v) { *reinterpret_cast<u32x2*>(p) = u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])}; }
 

@@ -117,6 +117,9 @@ long long hy_rows_mid_floats(const RowLinear& p);
 int hy_rows_mid(const RowLinear& p, float* ws, hipStream_t s);
 // ws: hy_linear_rows_floats() floats of scratch, 16-byte aligned (0: none needed)
 long long hy_linear_rows_floats(const RowLinear& p);
+// whether a linear of some rows, contiguous bf16 ones, is one of the kernels for few rows (three and more: one and two take norms and
+// pending adds, in fp32)
+bool hy_rows_bf16_takes(const RowLinear& p);
 int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s);
 // two independent linears; one launch where both run the GEMV with the same kind of epilogue (gated or not) at the row counts
 // of a mixture's experts (p) beside its shared expert (q), else one after the other
@@ -474,13 +477,13 @@ int hy_qkv_prep(const QkvPrep& p, hipStream_t s);
 // every head rotated (freq == nullptr: none, a scaled copy)
 // offset: the rotated numbers start there within each head; interleaved: number 2i pairs with 2i + 1 instead. out may be a.
 int hy_rotate_heads(const float* a, int lda, const int32_t* positions, const double* freq, int half, int M, int H, int n,
-                    float sign, float gain, float* out, int ldo, int offset, int interleaved, hipStream_t s);
+                    float sign, float gain, void* out, int out_bf16, int ldo, int offset, int interleaved, hipStream_t s);
 
 // out[i][m][:] = h[m] + (h[m - 1] - h[m]) * mu[i] for i < n; the row before a sequence's first is prev[b] (then set to
 // the sequence's last row)
 // w: optional [D] gain, h is RMS-normed first (S = 1, D <= 4096)
-int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, const float* w, float eps,
-                   hipStream_t s);
+int hy_token_shift(const float* h, float* prev, const float* mu, int n, void* out, int out_bf16, int B, int S, int D, const float* w,
+                   float eps, hipStream_t s);
 
 struct MlstmPrep {
   const float* proj;  // [M, ld]: input-gate pre-activations at columns [col_i, col_i + H), forget-gate at [col_f, col_f + H)
@@ -594,7 +597,8 @@ struct RecStep {
   const float* w;
   int w_heads, gate_act;
   float eps, gain;
-  float* out;
+  void* out;        // [B, ldo] fp32, or (out_bf16) bf16
+  int out_bf16;
   int ldo;
 };
 bool hy_rec_step_takes(int dim, int vdim);

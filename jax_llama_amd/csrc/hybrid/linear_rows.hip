@@ -421,6 +421,10 @@ static bool lr_short_normed(const RowLinear& p) {
   return p.a_norm_w && !p.a_norm_one && p.K <= HY_NORMED_GEMV_MAX_K && p.N <= HY_NORMED_GEMV_MAX_N;
 }
 
+bool hy_rows_bf16_takes(const RowLinear& p) {
+  return p.a_bf16 && (p.offs ? p.even_rows : p.R) >= 3 && p.N > 0 && (hy_rows_mid_takes(p) || hy_rows_gemv_takes(p));
+}
+
 int hy_linear_rows(const RowLinear& p, float* ws, hipStream_t s) {
   if (p.R < 0 || p.N <= 0 || p.K <= 0 || p.lda < p.K || p.ldo < p.N || p.E < 1) return -1;
   if (p.act < HY_ACT_NONE || p.act > HY_ACT_GELU_GLU) return -8;

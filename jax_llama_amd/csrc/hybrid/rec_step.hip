@@ -243,7 +243,10 @@ __global__ void __launch_bounds__(RS_THREADS) rec_step_kernel(RecStep p, int cw)
       const float z = p.gate[(size_t)b * p.ldg + (size_t)h * vdim + t];
       gate = p.gate_act == 1 ? hy_sigmoid(z) : hy_silu(z);
     }
-    p.out[(size_t)b * p.ldo + (size_t)h * vdim + t] = out * sc * p.w[(p.w_heads ? (size_t)h * vdim : 0) + t] * gate * p.gain;
+    const float y = out * sc * p.w[(p.w_heads ? (size_t)h * vdim : 0) + t] * gate * p.gain;
+    const size_t at = (size_t)b * p.ldo + (size_t)h * vdim + t;
+    if (p.out_bf16) reinterpret_cast<bf16_t*>(p.out)[at] = f2bf(y);
+    else reinterpret_cast<float*>(p.out)[at] = y;
   }
   if (MODE == RS_CONV && key) {  // the last of the key head's heads to have read the carried inputs moves them on (nobody waits)
     const int first = __builtin_amdgcn_readfirstlane(before);

@@ -21,8 +21,9 @@
 namespace jla {
 
 // grid (M, ceil(D / 256)), one thread per (token, column): a one-token step is one round trip, not D / 256 of them
+template <class OT>  // fp32, or bf16 for products' operands
 __global__ void __launch_bounds__(256) token_shift_kernel(const float* __restrict__ h, float* prev,
-                                                          const float* __restrict__ mu, int n, float* __restrict__ out,
+                                                          const float* __restrict__ mu, int n, OT* __restrict__ out,
                                                           int S, int D, size_t MD) {
   const int m = blockIdx.x, d = blockIdx.y * 256 + threadIdx.x;
   if (d >= D) return;
@@ -31,15 +32,16 @@ __global__ void __launch_bounds__(256) token_shift_kernel(const float* __restric
   const float* before = s == 0 ? prev + (size_t)b * D : cur - D;
   const float c = cur[d], diff = before[d] - c;
   const float last = h[((size_t)b * S + S - 1) * D + d];
-  for (int i = 0; i < n; ++i) out[(size_t)i * MD + (size_t)m * D + d] = fmaf(diff, mu[(size_t)i * D + d], c);
+  for (int i = 0; i < n; ++i) hy_store1(out + (size_t)i * MD + (size_t)m * D + d, fmaf(diff, mu[(size_t)i * D + d], c));
   if (s == 0) prev[(size_t)b * D + d] = last;  // (this thread was the only reader of prev[b, d])
 }
 
 // one token per row, the token RMS-normed first (every workgroup of a row repeats its sum, which a launch of the norm would
 // cost more than); prev holds normed tokens
+template <class OT>
 __global__ void __launch_bounds__(256) token_shift_norm_kernel(const float* __restrict__ x, const float* __restrict__ w, float eps,
                                                                float* prev, const float* __restrict__ mu, int n,
-                                                               float* __restrict__ out, int D, size_t MD) {
+                                                               OT* __restrict__ out, int D, size_t MD) {
   __shared__ float red[16];
   const int m = blockIdx.x, d = blockIdx.y * 256 + threadIdx.x;
   const float* row = x + (size_t)m * D;
@@ -54,12 +56,13 @@ __global__ void __launch_bounds__(256) token_shift_norm_kernel(const float* __re
   ss = block_sum(ss, red);
   if (d >= D) return;
   const float c = own * (1.f / sqrtf(ss / (float)D + eps)) * g, diff = before - c;
-  for (int i = 0; i < n; ++i) out[(size_t)i * MD + (size_t)m * D + d] = fmaf(diff, mu[(size_t)i * D + d], c);
+  for (int i = 0; i < n; ++i) hy_store1(out + (size_t)i * MD + (size_t)m * D + d, fmaf(diff, mu[(size_t)i * D + d], c));
   prev[(size_t)m * D + d] = c;  // (this thread is its only reader)
 }
 
-int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* out, int B, int S, int D, const float* w, float eps,
-                   hipStream_t s) {
+template <class OT>
+static int token_shift(const float* h, float* prev, const float* mu, int n, OT* out, int B, int S, int D, const float* w, float eps,
+                       hipStream_t s) {
   if (B < 0 || S < 1 || D < 1 || n < 1) return -1;
   if (B == 0) return 0;
   const long long M = (long long)B * S;
@@ -73,6 +76,12 @@ int hy_token_shift(const float* h, float* prev, const float* mu, int n, float* o
   }
   JLA_CHECK_LAUNCH();
   return 0;
+}
+
+int hy_token_shift(const float* h, float* prev, const float* mu, int n, void* out, int out_bf16, int B, int S, int D, const float* w,
+                   float eps, hipStream_t s) {
+  return out_bf16 ? token_shift(h, prev, mu, n, reinterpret_cast<bf16_t*>(out), B, S, D, w, eps, s)
+                  : token_shift(h, prev, mu, n, reinterpret_cast<float*>(out), B, S, D, w, eps, s);
 }
 
 // grid (H, B). All waves take the gates of up to MP_TOKENS tokens, the first one the chain over them: a lane holds a token, and 64 rounds

@@ -220,40 +220,45 @@ int hy_qkv_prep(const QkvPrep& p, hipStream_t s) {
 }
 
 // grid (M, ceil(H / 4)), one wave per (token, head)
+template <class OT>  // fp32, or bf16 for a product's operand
 __global__ void __launch_bounds__(256) rotate_heads_kernel(const float* a, int lda,
                                                            const int32_t* __restrict__ positions,
                                                            const double* __restrict__ freq, int half, int H, int n,
-                                                           float sign, float gain, float* out, int ldo,
+                                                           float sign, float gain, OT* out, int ldo,
                                                            int offset, int interleaved) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x, h = blockIdx.y * 4 + wave;
   if (h >= H) return;
   // (out may be a: a thread reads both numbers of its pair before it writes them, and no two threads share a number)
   const float* src = a + (size_t)m * lda + (size_t)h * n;
-  float* dst = out + (size_t)m * ldo + (size_t)h * n;
+  OT* dst = out + (size_t)m * ldo + (size_t)h * n;
   const int pos = half > 0 ? positions[m] : 0;
   for (int i = lane; i < half; i += 64) {
     float sn, cs;
     ro_sincos(pos, freq[i], sign, &sn, &cs);
     const int iu = offset + (interleaved ? 2 * i : i), iv = offset + (interleaved ? 2 * i + 1 : i + half);
     const float u = src[iu], v = src[iv];
-    dst[iu] = (u * cs - v * sn) * gain;
-    dst[iv] = (v * cs + u * sn) * gain;
+    hy_store1(dst + iu, (u * cs - v * sn) * gain);
+    hy_store1(dst + iv, (v * cs + u * sn) * gain);
   }
-  if (src != dst || gain != 1.f) {
-    for (int d = lane; d < offset; d += 64) dst[d] = src[d] * gain;
-    for (int d = offset + 2 * half + lane; d < n; d += 64) dst[d] = src[d] * gain;
+  if ((const void*)src != (const void*)dst || gain != 1.f) {
+    for (int d = lane; d < offset; d += 64) hy_store1(dst + d, src[d] * gain);
+    for (int d = offset + 2 * half + lane; d < n; d += 64) hy_store1(dst + d, src[d] * gain);
   }
 }
 
 int hy_rotate_heads(const float* a, int lda, const int32_t* positions, const double* freq, int half, int M, int H, int n,
-                    float sign, float gain, float* out, int ldo, int offset, int interleaved, hipStream_t s) {
+                    float sign, float gain, void* out, int out_bf16, int ldo, int offset, int interleaved, hipStream_t s) {
   if (M < 0 || H < 1 || n < 1 || lda < H * n || ldo < H * n) return -1;
   if (half < 0 || offset < 0 || offset + 2 * half > n || (half > 0 && !freq)) return -2;
   if (M == 0) return 0;
   if ((H + 3) / 4 > 65535) return -4;
-  rotate_heads_kernel<<<dim3(M, (H + 3) / 4), 256, 0, s>>>(a, lda, positions, freq, half, H, n, sign, gain, out, ldo,
-                                                             offset, interleaved);
+  if (out_bf16 && out == a) return -5;  // (in place: of one type)
+  const dim3 grid(M, (H + 3) / 4);
+  if (out_bf16)
+    rotate_heads_kernel<<<grid, 256, 0, s>>>(a, lda, positions, freq, half, H, n, sign, gain, reinterpret_cast<bf16_t*>(out), ldo, offset, interleaved);
+  else
+    rotate_heads_kernel<<<grid, 256, 0, s>>>(a, lda, positions, freq, half, H, n, sign, gain, reinterpret_cast<float*>(out), ldo, offset, interleaved);
   JLA_CHECK_LAUNCH();
   return 0;
 }

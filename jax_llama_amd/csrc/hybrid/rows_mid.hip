@@ -177,7 +177,8 @@ bool hy_rows_mid_takes(const RowLinear& p) {
   const long long nw = hy_act_gated(p.act) ? 2LL * p.N : p.N;
   if (p.offs) {
     if (p.R > RM_SORTED_ROWS) return p.R <= (long long)(p.K < RM_SHORT_K ? RM_SHORT_ROWS : RM_EXPERT_ROWS) * p.E;
-    return !p.a_bf16 && p.R >= 5LL * p.E && nw >= 4096 && nw * p.K >= RM_SORTED_WORK;
+    if (p.a_bf16) return p.even_rows >= RM_MIN_ROWS;
+    return p.R >= 5LL * p.E && nw >= 4096 && nw * p.K >= RM_SORTED_WORK;
   }
   if (!p.a_bf16) return p.R <= RM_F32_ROWS && !(p.R <= RM_FEW_ROWS && p.K < RM_FEW_K);
   return p.R <= (nw > RM_WIDE ? RM_WIDE_ROWS : RM_ROWS);

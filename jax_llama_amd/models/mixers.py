@@ -104,14 +104,15 @@ class BiasedAttention:
         proj = hy.linear(x, self.w_in)
         kc, vc = ctx.cache.layer(self.i)
         own = sp.kv_from is None
+        rows = hy.operand_rows(ctx.b * ctx.s, self.w_o)
         if ctx.s == 1:
             a = hy.attn_step(proj, ctx.positions, ctx.slot0, ctx.tickets, sp.heads, own, kc, vc, sp.scale, sp.softcap, self.bias,
-                             norm=(self.eps, sp.q_temp_coef, sp.q_temp_every))
+                             out=rows, norm=(self.eps, sp.q_temp_coef, sp.q_temp_every))
             if a is not None:
                 return hy.linear(a, self.w_o)
         q = hy.attn_prep(proj, ctx.positions, ctx.slot0, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim,
                          kc if own else None, vc if own else None, self.eps, sp.q_temp_coef, sp.q_temp_every)
-        a = hy.attn_bias(q, kc, vc, ctx.slot0, sp.scale, sp.softcap, self.bias, out=hy.operand_rows(ctx.b * ctx.s, self.w_o))
+        a = hy.attn_bias(q, kc, vc, ctx.slot0, sp.scale, sp.softcap, self.bias, out=rows)
         return hy.linear(a, self.w_o)
 
 
@@ -130,16 +131,16 @@ class GatedDeltaMixer:
         sp = self.spec
         proj = hy.linear(x, self.w_in)
         state, tail = ctx.cache.recurrent(self.i)
+        rows = hy.operand_rows(ctx.b * ctx.s, self.w_o)
         if ctx.s == 1 and ctx.b * sp.heads <= hy.DELTA_STEP_PAIRS:
             y = hy.delta_step(proj, ctx.b, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w, tail, self.a_log, self.dt_bias, state,
-                              self.norm_w, self.eps, ctx.tickets)
+                              self.norm_w, self.eps, ctx.tickets, rows)
             if y is not None:
                 return hy.linear(y, self.w_o)
         q, k, v, beta, decay = hy.delta_prep(proj, ctx.b, ctx.s, sp.heads, sp.kv_heads, sp.dim, sp.vdim, self.conv_w,
                                              tail, self.a_log, self.dt_bias)
         c = 2 * sp.kv_heads * sp.dim + sp.heads * sp.vdim
         gate = proj[:, c:c + sp.heads * sp.vdim]
-        rows = hy.operand_rows(ctx.b * ctx.s, self.w_o) if ctx.s > 1 else None
         return hy.linear(hy.delta_memory(q, k, v, beta, decay, state, ctx.b, ctx.s, gate, self.norm_w, self.eps, rows), self.w_o)
 
 
@@ -423,8 +424,9 @@ class TimeMix:
             (r, k, v, g, z), row = inputs
             carry = (prev, row)
         else:
-            mixes = hy.token_shift(h, prev, self.mu, ctx.b, ctx.s)
-            if 4 * m <= hy.STACKED_MAX_ROWS:  # a few tokens: the four same-shaped projections as one grouped launch
+            stacked = 4 * m <= hy.STACKED_MAX_ROWS  # a few tokens: the four same-shaped projections as one grouped launch
+            mixes = hy.token_shift(h, prev, self.mu, ctx.b, ctx.s, hy.operand_dtype(m, (self.w_rkvg if stacked else self.w_each[0], self.w_d1)))
+            if stacked:
                 r, k, v, g = hy.stacked_linear(mixes[:4], self.w_rkvg).unbind(0)
             else:
                 r, k, v, g = (hy.linear(mixes[j], self.w_each[j]) for j in range(4))
@@ -449,8 +451,15 @@ class SideBySide:
 
     def features(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None, gain: float = 1.0) -> torch.Tensor:
         m = ctx.b * ctx.s
-        # (each member norms its own copy of the input where that costs nothing, else they share one)
-        hv = h if ctx.s == 1 and isinstance(h, hy.RmsInput) and hy.norms_free(m, self.w_o, h.x.shape[1]) else _value(h)
+        # (each member norms its own copy of the input where that costs nothing, else they share one, or a pair of one in fp32 and one for products)
+        hv = h
+        if not (ctx.s == 1 and isinstance(h, hy.RmsInput) and hy.norms_free(m, self.w_o, h.x.shape[1])):
+            w_in = getattr(self.members[0], "w_in", self.w_o)
+            if w_in.dtype == torch.bfloat16 and isinstance(h, hy.RmsInput) and hy.reads_bf16(h.x, w_in):
+                h.rows()
+            else:
+                hv = _value(h)
+        out = hy.operand_rows(m, self.w_o) if out is None else out
         if out is None:
             out = torch.empty(m, self.width, dtype=torch.float32, device=hv.device if torch.is_tensor(hv) else hv.x.device)
         # one token: an attention beside a time mix read their inputs in one launch
@@ -489,7 +498,8 @@ class PreNormBlock:
         self.mixer, self.norm1, self.mlp, self.norm2, self.eps = mixer, norm1, mlp, norm2, eps
 
     def __call__(self, x: torch.Tensor, ctx: StepContext) -> None:
-        hy.linear_add_(x, self.mixer.features(hy.RmsInput(x, self.norm1, self.eps), ctx), self.mixer.w_o)
+        rows = hy.operand_rows(x.shape[0], self.mixer.w_o)
+        hy.linear_add_(x, self.mixer.features(hy.RmsInput(x, self.norm1, self.eps), ctx, out=rows), self.mixer.w_o)
         if self.mlp is not None:
             hy.linear_add_(x, self.mlp.features(hy.RmsInput(x, self.norm2, self.eps), ctx), self.mlp.w_o)
 

@@ -157,9 +157,14 @@ def _packed_weight(w: torch.Tensor):
 
 
 def _use_packed_gemm(x: torch.Tensor, w: torch.Tensor) -> bool:
-    if not PACKED_GEMM or w.dtype != BF16 or w.dim() != 2 or x.shape[0] < PACKED_GEMM_MIN_M:
+    return x.is_contiguous() and packs(x.shape[0], w)
+
+
+def packs(m: int, w: torch.Tensor) -> bool:
+    """Whether a product of ``m`` contiguous rows on ``w`` runs on the packed GEMM."""
+    if not PACKED_GEMM or w.dtype != BF16 or w.dim() != 2 or m < PACKED_GEMM_MIN_M:
         return False
-    if w.shape[0] % 16 or w.shape[1] % 32 or not x.is_contiguous():
+    if w.shape[0] % 16 or w.shape[1] % 32:
         return False
     from . import ext_available as core_available
     return core_available()
@@ -174,11 +179,12 @@ def one_product(x: torch.Tensor, w: torch.Tensor) -> bool:
 class RmsInput:
     """A sublayer's input ``rms_norm(x) * gain`` that is only written out when a consumer needs it in memory: the GEMV
     kernels norm the row they read themselves (``linear`` / ``moe_routed`` take this object in place of a tensor), the
-    tile kernels and the CPU path read ``value()``, computed once."""
+    tile kernels and the CPU path read ``value()`` or, where a product reads bf16, ``rows()``, computed once."""
 
     def __init__(self, x: torch.Tensor, gain: torch.Tensor, eps: float):
         self.x, self.gain, self.eps = x, gain, float(eps)
         self._value: Optional[torch.Tensor] = None
+        self._rows: Optional[torch.Tensor] = None
 
     @property
     def shape(self):
@@ -189,6 +195,16 @@ class RmsInput:
             self._value = rms_rows(self.x, self.gain, self.eps)
         return self._value
 
+    def rows(self) -> torch.Tensor:
+        """``value()`` in bf16 (``reads_bf16``), from the launch that computes it."""
+        if self._rows is None:
+            if self._value is None:
+                self._rows = torch.empty(self.x.shape, dtype=BF16, device=self.x.device)
+                self._value = rms_rows(self.x, self.gain, self.eps, rounded=self._rows)
+            else:
+                self._rows = _bf16_rows(self._value)
+        return self._rows
+
 
 # rows up to which a product norms its input itself: every workgroup repeats the row statistic (the walking form once, the
 # vector GEMV in every wave), which beats a launch of the norm kernel for one or two rows and loses to it from eight (vector
@@ -196,15 +212,15 @@ class RmsInput:
 FUSE_NORM_MAX_ROWS = 2
 
 
-def _fuse_norm(x, rows: int, n: int):
-    """``(tensor, gain, eps)`` a dense linear of ``rows`` rows and ``n`` columns reads: the un-normed rows with the
-    norm's gain when the GEMV will run it on the GPU, else the normed value."""
+def _fuse_norm(x, rows: int, n: int, w: torch.Tensor, act: int = ACT_NONE):
+    """``(tensor, gain, eps)`` a dense linear of ``rows`` rows and ``n`` columns on ``w`` reads: the un-normed rows with the
+    norm's gain when the GEMV will run it on the GPU, else the normed value, in bf16 where the product reads that."""
     if not isinstance(x, RmsInput):
         return x, None, 0.0
     if (_gpu(x.x) and x._value is None and x.gain.numel() == x.x.shape[1] and rows <= FUSE_NORM_MAX_ROWS
             and ext().dense_is_gemv(rows, n)):
         return x.x, x.gain, x.eps
-    return x.value(), None, 0.0
+    return (x.rows() if w.dtype == BF16 and reads_bf16(x.x, w, act) else x.value()), None, 0.0
 
 
 def act_gated(act: int) -> bool:
@@ -251,10 +267,13 @@ class Residual:
         return self.x
 
     def operand(self, wdtype) -> torch.Tensor:
-        """``value()`` for a product with weights of ``wdtype``: a prompt's rows rounded to bf16 by the kernel that adds, others fp32."""
+        """``value()`` for a product that reads bf16 (``reads_bf16``) on weights of ``wdtype``: the rows as rounded by the kernel that adds,
+        where they are more than those that ride in the product's launch; others fp32."""
         x = self.x
-        if not (_gpu(x) and x.is_contiguous() and prompt_bf16(x.shape[0], x.shape[1], wdtype)):
+        if not (_gpu(x) and x.is_contiguous() and x.shape[0] > RESIDUAL_MAX_ROWS and x.shape[1] % 8 == 0 and wdtype == BF16):
             return self.value()
+        if self.pending is None and self.rows is None and x.shape[0] <= FEW_ROWS:
+            return self.value()  # (a launch of its own would cost more than the bytes)
         if self.pending is not None:
             (y, nsum, ysc, w, eps), self.pending = self.pending, None
             self.rows = torch.empty(x.shape, dtype=BF16, device=x.device)
@@ -270,6 +289,7 @@ class Residual:
 
 RESIDUAL_MAX_ROWS = 2  # csrc: RV_WALK_ROWS
 FEW_ROWS = 64          # csrc: RV_MAX_ROWS
+GATE_ROWS16 = 8        # csrc: RV_MAX_ROWS16 (more bf16 rows would leave the gate to a launch of its own)
 
 
 def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, table: Optional[torch.Tensor] = None,
@@ -284,13 +304,13 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
         if ext().rows_fused(r.x, w, out, *r.pending, new, ids, table, int(col0)):
             r.x, r.pending, r.rows = new, None, None
             return out
-    if r is not None and _use_packed_gemm(r.x, w):  # (a prompt)
+    if r is not None and reads_bf16(r.x, w) and (ids is None or not GATE_ROWS16 < r.x.shape[0] <= FEW_ROWS):
         xv = r.operand(w.dtype)
     else:
         xv = r.value() if r is not None else x
     if ids is None:
         return linear(xv, w)
-    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and xv.dtype == F32 and w.dtype == BF16:
+    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and w.dtype == BF16:
         out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, ids, table, int(col0)):
             return out
@@ -321,7 +341,10 @@ def head_linear(x, gain: torch.Tensor, eps: float, w: torch.Tensor, cap: float =
         xv = r.value() if r is not None else x
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, **norm):
             return out
-    return linear(rms_rows(r.value() if r is not None else x, gain, eps), w, act=act, limit=cap)
+    xv = r.value() if r is not None else x
+    if reads_bf16(xv, w, act) and gain.numel() in (1, xv.shape[1]):
+        return linear(RmsInput(xv, gain.reshape(-1), eps).rows(), w, act=act, limit=cap)
+    return linear(rms_rows(xv, gain, eps), w, act=act, limit=cap)
 
 
 def head_argmax_pays(rows: int, w: torch.Tensor) -> bool:
@@ -357,19 +380,20 @@ def linear(x, w: torch.Tensor, swiglu: bool = False, act: int = ACT_NONE, limit:
     form for which ``w`` is ``[2N, K]`` (gate rows, then up rows): ``ACT_SWIGLU`` (``silu(g) * u``; also
     ``swiglu=True``), ``ACT_GELU_GLU`` (``gelu_tanh(g) * u``) or ``ACT_CLAMP_GLU`` (``g' sigmoid(alpha g') (u' + 1)``,
     ``g' = min(g, limit)``, ``u' = clamp(u, -limit, limit)``). ``x`` may be a column-contiguous view with strided rows; with
-    bf16 weights and no activation it may be bf16 already (the operand it would be rounded to anyway). ``out_dtype`` bf16:
-    the result as the next product's operand, where that saves a pass (a prompt on the large tiles); else fp32 all the same."""
+    bf16 weights and no activation it may be bf16 already (the operand it would be rounded to anyway; with one where ``reads_bf16``).
+    ``out_dtype`` bf16: the result as the next product's operand, where that saves a pass (a prompt on the large tiles, a few bf16 rows);
+    else fp32 all the same."""
     if isinstance(x, Residual):
         if act == ACT_NONE and not swiglu and x.fusable() and w.shape[0] > SKINNY_MAX_N:
             return linear_rows_gated(x, w)
-        x = x.operand(w.dtype) if act == ACT_NONE and not swiglu and _use_packed_gemm(x.x, w) else x.value()
+        x = x.operand(w.dtype) if reads_bf16(x.x, w, ACT_SWIGLU if swiglu else act) else x.value()
     if swiglu:
         act = ACT_SWIGLU
     n = w.shape[0] // 2 if act_gated(act) else w.shape[0]
-    x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], n)
+    x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], n, w, act)
     if not _gpu(x):
         return _act_cpu(_round_like(x, w) @ w.float().t(), act, limit, alpha)
-    if norm_w is None and _mid_rows(x, w, act):
+    if norm_w is None and (_mid_rows(x, w, act) or (x.dtype == BF16 and few_bf16(x.shape[0], w, act))):
         out = torch.empty(x.shape[0], n, dtype=out_dtype, device=x.device)
         ext().linear_rows(_bf16_operand(x), None, w, out, None, None, None, x.shape[0], int(act), float(limit), float(alpha), None, None, 0.0)
         return out
@@ -407,19 +431,46 @@ def _mid_rows(x: torch.Tensor, w: torch.Tensor, act: int = ACT_NONE) -> bool:
     return x.shape[0] > FEW_ROWS and w.dtype == BF16 and ext().rows_mid_takes(x.shape[0], w, int(act))
 
 
+def few_bf16(m: int, w: torch.Tensor, act: int = ACT_NONE) -> bool:
+    """Whether a product of ``m`` contiguous rows, three to a few hundred, on ``w [N, K]`` (``[E, N, K]``: of so many on each) reads them
+    as bf16 (the operand they would be rounded to anyway), on the kernels for such rows; one and two rows take norms and pending adds
+    into the launch instead."""
+    return RESIDUAL_MAX_ROWS < m < PACKED_GEMM_MIN_M and w.dtype == BF16 and ext().rows_bf16_takes(m, w, int(act))
+
+
+def reads_bf16(x: torch.Tensor, w: torch.Tensor, act: int = ACT_NONE) -> bool:
+    """Whether the product of the rows ``x`` (their shape and strides count) on ``w`` is best handed them in bf16."""
+    if w.dtype != BF16 or not (_gpu(x) and w.dim() == 2 and x.shape[1] % 8 == 0 and x.is_contiguous()):
+        return False
+    if x.shape[0] < PACKED_GEMM_MIN_M:
+        return few_bf16(x.shape[0], w, act)
+    if act == ACT_NONE:
+        return _use_packed_gemm(x, w)
+    return act_gated(act) and ext().rows_gemm_pays(x.shape[0], w, int(act))
+
+
 def prompt_bf16(m: int, cols: int, wdtype) -> bool:
     """Whether a step of ``m`` rows keeps a sublayer's input and features in bf16 (the matrix operands they would be
     rounded to anyway, half the traffic): prompt-sized batches with bf16 weights. Fewer rows run GEMVs, which read fp32."""
     return wdtype == BF16 and m >= PACKED_GEMM_MIN_M and cols % 8 == 0
 
 
+def operand_dtype(m: int, ws) -> torch.dtype:
+    """The type of ``m`` contiguous rows each for the products with ``ws``, ``[N, K]`` or (one launch) ``[E, N, K]``: bf16 where all read that."""
+    if m <= RESIDUAL_MAX_ROWS or not all(w.dtype == BF16 and _gpu(w) for w in ws):
+        return F32
+    if m < PACKED_GEMM_MIN_M:
+        return BF16 if all(few_bf16(m, w) for w in ws) else F32
+    return BF16 if all(packs(m, w) for w in ws) else F32
+
+
 def operand_rows(m: int, w: torch.Tensor) -> Optional[torch.Tensor]:
-    """Where the kernel before a product with ``w [N, K]`` writes ``m`` rows for it: bf16 ``[m, K]`` of a prompt on the packed GEMM
-    (the operand they would be rounded to anyway), else None."""
-    if not _gpu(w) or w.dim() != 2 or not prompt_bf16(m, w.shape[1], w.dtype):
+    """Where the kernel before a product with ``w [N, K]`` writes ``m`` rows for it: bf16 ``[m, K]`` where it reads that (a prompt on the
+    packed GEMM, a few rows: the operand they would be rounded to anyway), else None."""
+    if m <= RESIDUAL_MAX_ROWS or w.dtype != BF16 or not _gpu(w) or w.dim() != 2:
         return None
     rows = torch.empty(m, w.shape[1], dtype=BF16, device=w.device)
-    return rows if _use_packed_gemm(rows, w) else None
+    return rows if reads_bf16(rows, w) else None
 
 
 def glu_rows(gu: torch.Tensor, act: int, out: torch.Tensor, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
@@ -482,7 +533,7 @@ def ff_dense(x, w_up: torch.Tensor, w_down: torch.Tensor, act: int = ACT_RELU2) 
 def linear_add_(res: torch.Tensor, x, w: torch.Tensor) -> torch.Tensor:
     """``res [M, N] (fp32) += x [M, K] @ w^T`` in place: a sublayer's output projection with the residual add in its
     epilogue."""
-    x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], w.shape[0])
+    x, norm_w, norm_eps = _fuse_norm(x, x.shape[0], w.shape[0], w)
     if not _gpu(x):
         return res.add_(_round_like(x, w) @ w.float().t())
     if norm_w is None and res.is_contiguous() and _mid_rows(x, w):
@@ -555,7 +606,7 @@ _STACK_INDEX = {}
 
 
 def stacked_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """Same-shaped linears of different inputs in one launch: ``x [E, M, K]`` (fp32, contiguous), ``w [E, N, K]`` ->
+    """Same-shaped linears of different inputs in one launch: ``x [E, M, K]`` (contiguous; fp32, or bf16 where ``few_bf16``), ``w [E, N, K]`` ->
     fp32 ``[E, M, N]``, ``out[e] = x[e] @ w[e]^T``. Runs the expert-grouped row linear (member ``e`` = expert ``e``)."""
     e_n, m, k = x.shape
     n = w.shape[1]
@@ -571,7 +622,7 @@ def stacked_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         ar = torch.arange(e_n + 1, dtype=torch.int32)
         idx = _STACK_INDEX[key] = (ar[:e_n].repeat_interleave(m).to(x.device), (ar * m).to(x.device))
     ex = ext()
-    if rows <= ex.GEMV_MAX_R:
+    if rows <= ex.GEMV_MAX_R and x.dtype == F32:
         ex.linear_rows(x.reshape(rows, k), None, w, out, None, None, idx[0], rows, ACT_NONE, 0.0, 1.0, None, None, 0.0)
     else:
         ex.linear_rows(x.reshape(rows, k), None, w, out, None, idx[1], None, rows, ACT_NONE, 0.0, 1.0, None, None, 0.0, m)
@@ -943,13 +994,13 @@ def norm_residual_(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, eps: float
     return x
 
 
-def rms_rows(y: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
-    """``y / sqrt(mean(y^2) + eps) * w`` (fp32), ``w`` one number or ``[D]``."""
+def rms_rows(y: torch.Tensor, w: torch.Tensor, eps: float, rounded: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``y / sqrt(mean(y^2) + eps) * w`` (fp32), ``w`` one number or ``[D]``; on the GPU also in bf16 into ``rounded``."""
     if not _gpu(y):
         v = y.float()
         return v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps) * w.float().reshape(-1)
     out = torch.empty_like(y)
-    ext().norm_residual(y, 1, 1.0, w.reshape(-1), float(eps), None, out, None, None)
+    ext().norm_residual(y, 1, 1.0, w.reshape(-1), float(eps), None, out, None, None, rounded)
     return out
 
 
@@ -1167,7 +1218,7 @@ def attn_bias(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, slot, scale: 
     h = qh // maps
     g = kc.shape[1]
     vdim = vc.shape[3] if vdim is None else int(vdim)
-    if turn is not None and (s != 1 or maps != 1 or not _gpu(q) or (out is not None and out.dtype != F32)):
+    if turn is not None and (s != 1 or maps != 1 or not _gpu(q)):
         a = attn_bias(q, kc, vc, slot, scale, softcap, bias, max_kv, sink, chunk, head_scale, window, keep_first, gate, vdim,
                       gate_cols, None, diff)
         return rotate_heads(a, turn[0], turn[1], h, sign=turn[2], gain=turn[3], out=out)
@@ -1245,7 +1296,7 @@ def attn_step(proj: torch.Tensor, positions: torch.Tensor, slot, tickets: Option
     temp_every)``) or ``rope_prep`` (``rope = (col_bias, qk_freq, v_freq, gain)``: with ``v_freq`` or ``gain`` other than 1 the result
     is ``rotate_heads(., positions, v_freq, sign=-1, gain)``), then ``attn_bias``. ``own``: the projection brings keys and values for
     the cache. ``tickets``: zeros that no concurrent step uses (the cache's). None where only the separate ops apply."""
-    if not _gpu(proj) or tickets is None or (out is not None and out.dtype != F32):
+    if not _gpu(proj) or tickets is None:
         return None
     b, vdim = kc.shape[0], vc.shape[3]
     dst = torch.empty(b, heads * vdim, dtype=F32, device=proj.device) if out is None else out
@@ -1361,10 +1412,9 @@ def gated_rmsnorm(o: torch.Tensor, gate: Optional[torch.Tensor], w: torch.Tensor
 
 def _step_out(x: torch.Tensor, width: int, dim: int, vdim: int, s: int, out: Optional[torch.Tensor]):
     """Where a recurrence's one-token kernel (csrc/hybrid/rec_step.hip: gates, state and gated head norm in one launch) writes,
-    or None where the separate ops run: more tokens, the CPU, head sizes it does not take, a bf16 buffer, more rows than a
+    or None where the separate ops run: more tokens, the CPU, head sizes it does not take, more rows than a
     grid's second axis."""
-    if s != 1 or not _gpu(x) or x.shape[0] > 65535 or (out is not None and out.dtype != F32) or \
-            not ext().rec_step_takes(dim, vdim):
+    if s != 1 or not _gpu(x) or x.shape[0] > 65535 or not ext().rec_step_takes(dim, vdim):
         return None
     return out if out is not None else torch.empty(x.shape[0], width, dtype=F32, device=x.device)
 
@@ -1372,9 +1422,9 @@ def _step_out(x: torch.Tensor, width: int, dim: int, vdim: int, s: int, out: Opt
 def delta_memory(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor,
                  state: torch.Tensor, b: int, s: int, gate: torch.Tensor, w: torch.Tensor, eps: float,
                  rows: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``gated_rmsnorm(delta_scan(...), gate, w, eps)``; ``rows``: what it writes where the separate ops run (a product's operand)."""
+    """``gated_rmsnorm(delta_scan(...), gate, w, eps)``; ``rows``: what it writes (a product's operand)."""
     h, vdim = v.shape[1], v.shape[2]
-    out = _step_out(q, h * vdim, q.shape[2], vdim, s, None) if rows is None else None
+    out = _step_out(q, h * vdim, q.shape[2], vdim, s, rows)
     if out is None:
         return gated_rmsnorm(delta_scan(q, k, v, beta, decay, state, b, s), gate, w, eps, out=rows)
     ext().rec_step(3, q, k, v, beta=beta, decay=decay, state=state, gate=gate, w=w, eps=float(eps), gate_act=GATE_SILU, gain=1.0,
@@ -1391,12 +1441,12 @@ DELTA_STEP_PAIRS = 256
 
 def delta_step(proj: torch.Tensor, b: int, heads: int, kv_heads: int, dim: int, vdim: int, conv_w: torch.Tensor, tail: torch.Tensor,
                a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor, w: torch.Tensor, eps: float,
-               tickets: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+               tickets: Optional[torch.Tensor], rows: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``delta_prep`` and ``delta_memory`` (gated by the projection's gate columns) of one token per row in one launch; ``tickets``: zeros
     that no concurrent step uses (the cache's). None where only the separate ops apply."""
     if not _gpu(proj) or tickets is None:
         return None
-    out = torch.empty(b, heads * vdim, dtype=F32, device=proj.device)
+    out = torch.empty(b, heads * vdim, dtype=F32, device=proj.device) if rows is None else rows
     return out if ext().delta_step(proj, b, heads, kv_heads, dim, vdim, conv_w, tail, a_log, dt_bias, tickets, state, w, float(eps),
                                    out) else None
 
@@ -1559,14 +1609,14 @@ def rotate_heads(a: torch.Tensor, positions: torch.Tensor, freq: Optional[torch.
 
 
 # ------------------------------------------------------------------------------------------------ linear recurrences
-def token_shift(h, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int) -> torch.Tensor:
+def token_shift(h, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int, dtype=F32) -> torch.Tensor:
     """``out[n, m] = h[m] + (h[m - 1] - h[m]) * mu[n]`` for the ``n`` rows of ``mu [n, D]``; the token before a call's
     first comes from ``prev [B, D]`` (zeros at a sequence start), which is then set to the call's last token. fp32
-    ``[n, B*S, D]``. ``h`` may be an ``RmsInput``: one token per row is normed by the same launch."""
+    ``[n, B*S, D]``, on the GPU with ``dtype`` bf16 rounded for the products that read them. ``h`` may be an ``RmsInput``: one token per row is normed by the same launch."""
     n, d = mu.shape
     if isinstance(h, RmsInput):
         if s == 1 and _gpu(h.x) and h._value is None and d <= 4096 and h.gain.numel() == d and h.x.is_contiguous():
-            out = torch.empty(n, b, d, dtype=F32, device=h.x.device)
+            out = torch.empty(n, b, d, dtype=dtype, device=h.x.device)
             ext().token_shift(h.x, prev, mu, out, b, s, h.gain, h.eps)
             return out
         h = h.value()
@@ -1576,7 +1626,7 @@ def token_shift(h, prev: torch.Tensor, mu: torch.Tensor, b: int, s: int) -> torc
         out = hh[None] + (before - hh)[None] * mu.float()[:, None, None, :]
         prev.copy_(hh[:, -1])
         return out.reshape(n, b * s, d).contiguous()
-    out = torch.empty(n, b * s, d, dtype=F32, device=h.device)
+    out = torch.empty(n, b * s, d, dtype=dtype, device=h.device)
     ext().token_shift(h, prev, mu, out, b, s)
     return out
 
