@@ -28,3 +28,14 @@ def slot_tensor(slot, device) -> torch.Tensor:
     if isinstance(slot, HostSlot) and slot.on_device.device == torch.device(device):
         return slot.on_device
     return torch.full((1,), int(slot), dtype=torch.int32, device=device)
+
+
+def device_numbers(values, dtype, device) -> torch.Tensor:
+    """The numbers ``values`` (a sequence of ints) as a device ``[len(values)]``, without a wait for what the stream still has to do: a copy
+    from pageable host memory has one. One number is a fill's argument; more go through pinned memory, which the allocator hands out
+    again only after the copy."""
+    if torch.device(device).type == "cpu":
+        return torch.tensor(list(values), dtype=dtype)
+    if len(values) == 1:
+        return torch.full((1,), int(values[0]), dtype=dtype, device=device)
+    return torch.tensor(list(values), dtype=dtype, pin_memory=True).to(device, non_blocking=True)

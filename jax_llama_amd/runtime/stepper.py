@@ -12,6 +12,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from ..ops.slots import device_numbers
+
 
 class SequenceStepper:
     def __init__(self, model, max_tokens: int):
@@ -55,10 +57,10 @@ class SequenceStepper:
         if any(w < 0 or w >= n for w in want):
             raise ValueError(f"request {rid!r}: wanted place outside the portion")
         dev = self.model.device
-        ids = torch.tensor([list(tokens)], dtype=torch.int32, device=dev)
+        ids = device_numbers(tokens, torch.int32, dev).reshape(1, n)
         pos = torch.arange(s0, s0 + n, dtype=torch.int32, device=dev).reshape(1, n)
         if len(want):
-            rows = torch.tensor(list(want), dtype=torch.long, device=dev)
+            rows = device_numbers(want, torch.long, dev)
             logits, *_ = self.model.forward_tokens(ids, pos, cache, cache.index_t, logits_mode="rows", logit_rows=rows)
         else:
             logits = None
