@@ -112,6 +112,7 @@ bool hy_rows_gemv_takes(const RowLinear& p);
 bool hy_rows_gemv_takes_residual(const RowLinear& p);
 int hy_rows_gemv(const RowLinear& p, hipStream_t s);
 int hy_rows_gemm(const RowLinear& p, hipStream_t s);
+constexpr int RM_TILES_K = 1024;  // K from which rows_gemm.hip's tiles take rows by expert
 bool hy_rows_mid_takes(const RowLinear& p);
 long long hy_rows_mid_floats(const RowLinear& p);
 int hy_rows_mid(const RowLinear& p, float* ws, hipStream_t s);

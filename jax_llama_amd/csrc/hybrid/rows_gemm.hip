@@ -1,13 +1,16 @@
 // Row-gathered, expert-grouped linear of a prompt on row-major bf16 weights and a bf16 activation copy:
 //   out[dst(r), :] = act(A[src(r), :] @ W[expert(r)]^T),   the large form of linear_rows.hip's lr_gemm_kernel.
 //
-// What bounds it: the matrix cores. lr_gemm_kernel (64- or 128-row tiles, one LDS stage, VGPR staging) pulls 11 TB/s from
-// L2 and stops at 300-450 TFLOP/s. Here one wave per SIMD owns a 128 x 16 NJ output block (NJ x 8 accumulators of
-// v_mfma_f32_16x16x32_bf16 in AGPRs), K advances 64 per LDS slot, two slots filled by LDS-DMA, and every fragment read and
+// What bounds it: the matrix cores, and the rows that whole tiles pad. lr_gemm_kernel (64- or 128-row tiles, one LDS stage, VGPR staging)
+// pulls 11 TB/s from L2 and stops at 300-450 TFLOP/s. Here one wave per SIMD owns a 16 MI x 16 NJ output block (NJ x MI accumulators
+// of v_mfma_f32_16x16x32_bf16 in AGPRs), K advances 64 per LDS slot, two slots filled by LDS-DMA, and every fragment read and
 // DMA issue sits between MFMAs -- the schedule of the packed GEMM (kernels/gemm4w.h), with both operands row-major: the
 // activation rows are gathered by per-lane addresses and the weight rows are read as they lie in the checkpoint, so an
-// expert's weights need no second, packed copy. NJ = 8 (256 x 256 tiles) reads 256 B of LDS per MFMA, NJ = 4 (256 x 128)
-// 384 B but makes twice the tiles: it is for launches that would leave the last round of workgroups nearly empty.
+// expert's weights need no second, packed copy. MI = NJ = 8 (256 x 256 tiles) reads 256 B of LDS per MFMA and is for launches of many
+// rounds; 128, 160 or 192 x 128 tiles (NJ = 4) read 384 to 512 B, but two of them share a compute unit, one's products behind
+// the other's waits, and they pad less: 8 experts of 2816 x 2048 (7168 x 4096), both products, us with 256-row tiles -> now, 1000 | 2600 | 5000 | 12000
+// rows 125 | 188 | 271 | 571 -> 95 | 137 | 211 | 444 (416 | 712 | 1025 | 2265 -> 360 | 533 | 939 | 2056); one gated matrix of 5632 x 2048, 600 | 1500 |
+// 3000 rows 65 | 117 | 194 -> 36 | 77 | 136.
 //
 // LDS images of both operands: [rows][8 cells of 16 B] (64 k); cell c of row r holds k-chunk c ^ ((r & 15) >> 1), so the 16
 // lanes of a fragment read fall on all 64 banks. A gated activation interleaves 16 gate rows and 16 up rows of W, which
@@ -22,29 +25,35 @@
 
 namespace jla {
 
-constexpr int RG_BM = 256, RG_BK = 64;
-constexpr int RG_SLOT_U4 = 2 * RG_BM * RG_BK * 2 / 16;  // u32x4 of one slot: A 32 KiB + W 32 KiB (NJ = 4: half of it used)
+constexpr int RG_BK = 64;
 
-template <int NJ>
-__global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gated, int tiles_n) {
-  static_assert(NJ == 4 || NJ == 8, "16-column tiles per wave");
-  constexpr int MPS = NJ / 2;  // MFMAs per slot: 8 NJ in 16 slots
-  __shared__ u32x4 lds[2 * RG_SLOT_U4];
+template <int NJ, int MI>
+constexpr int RG_PER_CU = (32 * MI + 32 * NJ) * RG_BK * 2 * 2 <= 80 * 1024 ? 2 : 1;  // workgroups whose slots fit a compute unit's LDS
+
+// A wave's block: 16 MI rows x 16 NJ columns
+template <int NJ, int MI>
+__global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(RowLinear p, int gated, int tiles_n) {
+  static_assert((NJ == 4 || NJ == 8) && MI >= 4 && MI <= 8, "16-column and 16-row tiles per wave");
+  constexpr int BM = 32 * MI, SLOT = (BM + 32 * NJ) * RG_BK * 2 / 16;  // u32x4 of a slot: A, then W
+  constexpr int T = NJ * MI;      // MFMAs of half a K-tile, in 16 groups
+  constexpr int EG = MI == 8 ? 4 : (MI % 2 ? 1 : 2);  // row tiles that pass through LDS at a time at the end
+  static_assert(2 * SLOT >= 4 * EG * 16 * 4 * NJ, "the epilogue's staging");
+  __shared__ u32x4 lds[2 * SLOT];
   const int lane = threadIdx.x & 63;
   const int wu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wu >> 1, wc = wu & 1;
   int e = 0, r0 = 0, rend = 0, tn = 0;
-  if (!row_tile<RG_BM>(p.offs, p.E, p.R, tiles_n, lane, e, r0, rend, tn)) return;
+  if (!row_tile<BM>(p.offs, p.E, p.R, tiles_n, lane, e, r0, rend, tn)) return;
   const int K = p.K, N = p.N, KT = K / RG_BK;
   const int cols = gated ? 16 * NJ : 32 * NJ;  // output columns of the workgroup
   const int n0 = tn * cols;
 
   // DMA sources: piece P = wu + 4 j is 8 rows of 128 B; lane -> row 8 P + (lane >> 3), LDS cell lane & 7
-  const char* pa[8];
+  const char* pa[MI];
   unsigned ow[NJ];
   const char* const wbase = reinterpret_cast<const char*>(reinterpret_cast<const bf16_t*>(p.w) + (size_t)e * p.w_stride);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < MI; ++j) {
     const int P = wu + 4 * j;
     const int row = min(r0 + 8 * P + (lane >> 3), rend - 1);  // (rows past the expert's end repeat its last one)
     const int chunk = (lane & 7) ^ (4 * (P & 1) + (lane >> 4));
@@ -58,37 +67,34 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
     const int wrow = gated && (jt & 1) ? N + col : col;
     ow[j] = ((unsigned)wrow * (unsigned)K + 8u * (unsigned)chunk) * 2u;
   }
-  auto dma = [&](int t, int j) {  // the j-th of this wave's 8 + NJ DMAs of K-tile t
-    u32x4* slot = lds + (t & 1) * RG_SLOT_U4;
-    if (j < 8) glds16(pa[j] + (size_t)t * 128, slot + (wu + 4 * j) * 64);
-    else glds16(wbase + (size_t)t * 128 + ow[j - 8], slot + RG_BM * 8 + (wu + 4 * (j - 8)) * 64);
+  auto dma = [&](int t, int j) {  // the j-th of this wave's MI + NJ DMAs of K-tile t
+    u32x4* slot = lds + (t & 1) * SLOT;
+    if (j < MI) glds16(pa[j < MI ? j : 0] + (size_t)t * 128, slot + (wu + 4 * j) * 64);
+    else glds16(wbase + (size_t)t * 128 + ow[j < MI ? 0 : j - MI], slot + BM * 8 + (wu + 4 * (j - MI)) * 64);
   };
-  const int xrd = (wr * 128 + (lane & 15)) * 8, wrd = RG_BM * 8 + (wc * 16 * NJ + (lane & 15)) * 8;
+  const int xrd = (wr * 16 * MI + (lane & 15)) * 8, wrd = BM * 8 + (wc * 16 * NJ + (lane & 15)) * 8;
   const int c0 = (0 + (lane >> 4)) ^ ((lane >> 1) & 7), c1 = (4 + (lane >> 4)) ^ ((lane >> 1) & 7);
-  auto rd = [&](u32x4& dst, int slot, int h, int q) {  // q < NJ: W n-tile q; then the 8 m-tiles of A
-    const u32x4* s = lds + slot * RG_SLOT_U4 + (h ? c1 : c0);
+  auto rd = [&](u32x4& dst, int slot, int h, int q) {  // q < NJ: W n-tile q; then the MI m-tiles of A
+    const u32x4* s = lds + slot * SLOT + (h ? c1 : c0);
     dst = q < NJ ? s[wrd + q * 128] : s[xrd + (q - NJ) * 128];
   };
 
-  f32x4 acc[NJ][8];
+  f32x4 acc[NJ][MI];
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 w0[NJ], x0[8], w1[NJ], x1[8];
+    for (int i = 0; i < MI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 w0[NJ], x0[MI], w1[NJ], x1[MI];
 
-  // 8 NJ MFMAs on (wf, xf) with the 8 + NJ fragment reads of the next half tile and the DMAs of tile td between them
-  auto substep = [&](u32x4 (&wf)[NJ], u32x4 (&xf)[8], u32x4 (&wn)[NJ], u32x4 (&xn)[8], bool do_rd, int rslot, int rh,
+  // MI NJ MFMAs on (wf, xf) with the MI + NJ fragment reads of the next half tile and the DMAs of tile td between them
+  auto substep = [&](u32x4 (&wf)[NJ], u32x4 (&xf)[MI], u32x4 (&wn)[NJ], u32x4 (&xn)[MI], bool do_rd, int rslot, int rh,
                      bool do_dma, int td) {
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
 #pragma unroll
-      for (int u = 0; u < MPS; ++u) {
-        const int m = MPS * q + u;
-        g4_mfma(acc[m >> 3][m & 7], wf[m >> 3], xf[m & 7]);
-      }
-      if (q < 8 + NJ) {
-        if (do_rd) rd(q < NJ ? wn[q < NJ ? q : 0] : xn[q < NJ ? 0 : (q - NJ) & 7], rslot, rh, q);
+      for (int m = q * T / 16; m < (q + 1) * T / 16; ++m) g4_mfma(acc[m / MI][m % MI], wf[m / MI], xf[m % MI]);
+      if (q < MI + NJ) {
+        if (do_rd) rd(q < NJ ? wn[q < NJ ? q : 0] : xn[q < NJ ? 0 : (q - NJ) % MI], rslot, rh, q);
         if (do_dma) dma(td, q);
       }
     }
@@ -100,18 +106,18 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
   };
 
 #pragma unroll
-  for (int j = 0; j < 8 + NJ; ++j) dma(0, j);
+  for (int j = 0; j < MI + NJ; ++j) dma(0, j);
   if (KT > 1) {
 #pragma unroll
-    for (int j = 0; j < 8 + NJ; ++j) dma(1, j);
-    wait_vmcnt<8 + NJ>();
+    for (int j = 0; j < MI + NJ; ++j) dma(1, j);
+    wait_vmcnt<MI + NJ>();
   } else {
     wait_vmcnt<0>();
   }
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int q = 0; q < 8 + NJ; ++q) rd(q < NJ ? w0[q < NJ ? q : 0] : x0[q < NJ ? 0 : (q - NJ) & 7], 0, 0, q);
+  for (int q = 0; q < MI + NJ; ++q) rd(q < NJ ? w0[q < NJ ? q : 0] : x0[q < NJ ? 0 : (q - NJ) % MI], 0, 0, q);
 
   int t = 0;
   for (; t + 2 < KT; ++t) {
@@ -130,9 +136,9 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
   g4_acc_fence();
   __syncthreads();  // every wave is past its last fragment read: the slots become the epilogue's staging
 
-  // lane (c = lane & 15, q = lane >> 4) holds row 16 i + c of the wave's 128 at accumulator columns 16 j + 4 q + 0..3
+  // lane (c = lane & 15, q = lane >> 4) holds row 16 i + c of the wave's 16 MI at accumulator columns 16 j + 4 q + 0..3
   constexpr int CH = 4 * NJ;  // 16-byte chunks of a staged row; chunk x of row r lies at x ^ (r & 15)
-  f32x4* const wl = reinterpret_cast<f32x4*>(lds) + wu * 2048;
+  f32x4* const wl = reinterpret_cast<f32x4*>(lds) + wu * (16 * EG * CH);
   const int c = lane & 15, q4 = lane >> 4;
   const int lanes_per_row = gated ? CH / 2 : CH;
   const int rpi = 64 / lanes_per_row;  // rows per step of the store loop
@@ -140,16 +146,16 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
   const int gch = gated ? 8 * (oc >> 2) + (oc & 3) : oc;  // the staged chunk of output chunk oc (gate; up is 4 further)
   const int col = n0 + wc * (cols / 2) + 4 * oc;
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
+  for (int part = 0; part < MI / EG; ++part) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < EG; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) wl[(16 * i + c) * CH + ((4 * j + q4) ^ c)] = g4_take(acc[j][4 * half + i]);
-    const int rbase = r0 + wr * 128 + 64 * half;
-    int drow = rbase + lane;  // lane l: where the half's row l goes (-1: past the expert's rows)
+      for (int j = 0; j < NJ; ++j) wl[(16 * i + c) * CH + ((4 * j + q4) ^ c)] = g4_take(acc[j][EG * part + i]);
+    const int rbase = r0 + wr * 16 * MI + 16 * EG * part;
+    int drow = rbase + (lane & (16 * EG - 1));  // lane l: where the part's row l goes (-1: past the expert's rows)
     drow = drow < rend ? (p.dst_idx ? p.dst_idx[drow] : drow) : -1;
 #pragma unroll 4
-    for (int s = 0; s < 64; s += rpi) {
+    for (int s = 0; s < 16 * EG; s += rpi) {
       const int rr = s + rr0;
       const int d = __shfl(drow, rr, 64);
       const f32x4 g = wl[rr * CH + (gch ^ (rr & 15))];
@@ -175,13 +181,12 @@ __global__ void __launch_bounds__(256, 1) rows_gemm_kernel(RowLinear p, int gate
   }
 }
 
-// Where the large tiles win over lr_gemm_kernel's 64-row ones (MI355X, gate / up of 2816 columns and down, us old -> new):
-// 24000 rows, 8 experts, K 4096, F 7168: 6182 -> 2553, down 2921 -> 1186; 4096 rows, 8 experts, K 2048: 219 -> 139, 139 ->
-// 73; one dense matrix, 777 rows, K 2048, F 5632: 93 -> 69. A tile is padded to 256 rows: with 64 experts of 64 rows the
-// padding costs more than the pipeline gives (477 -> 528; of 80 rows 638 -> 609), unless every tile runs in the first
-// round of workgroups anyway (8 experts of 32 rows, K 4096: 204 -> 138). Below K = 1024 the pipeline's fill and the
-// epilogue outweigh the loop (K 512: 16 -> 21).
-constexpr int RG_MIN_ROWS = 80, RG_MIN_ROWS_ONE_ROUND = 32, RG_MIN_K = 1024;
+// Where they win over lr_gemm_kernel's 64-row tiles (gate / up of 2816 columns and down, us there -> 256-row tiles here): 24000 rows, 8
+// experts, K 4096, F 7168: 6182 -> 2553, down 2921 -> 1186; 4096 rows, 8 experts, K 2048: 219 -> 139, 139 -> 73; one dense matrix, 777 rows,
+// K 2048, F 5632: 93 -> 69. Fewer rows per expert than these minima are rows_mid.hip's, which streams the weights as fast and pads less
+// (48 rows each of 8 experts, 4096 x 7168 99 us there, 126 here). Below K = 1024 the pipeline's fill and the epilogue outweigh the loop (K
+// 512: 16 -> 21).
+constexpr int RG_MIN_ROWS = 65, RG_MIN_ROWS_ONE_ROUND = 32, RG_MIN_K = RM_TILES_K;
 
 bool hy_rows_gemm_takes(const RowLinear& p) {
   const int E = p.offs ? p.E : 1;
@@ -206,18 +211,56 @@ bool hy_rows_gemm_pays(const RowLinear& p) {
   return hy_rows_gemm_takes(p) && !few;
 }
 
+// A form's measured times, us: launch and fill; a 64-deep step of one workgroup; its rise with every further one of a compute unit, whose
+// last round counts as `last` workgroups more
+struct RgForm {
+  int nj, mi;
+  float fill, step, more, last;
+};
+static const RgForm RG_FORMS[] = {{4, 4, 1.0f, 0.644f, 0.833f, 1.0f}, {4, 5, 9.75f, 0.608f, 0.965f, 0.99f}, {4, 6, 5.17f, 0.819f, 0.795f, 0.945f},
+                                  {8, 8, 17.5f, 1.407f, 1.3f, 1.0f}};
+
+// The form with the least time by the figures above: on average 1.8 % above the best of those measured (54 products: 8 experts of 2816 x
+// 2048 and 7168 x 4096 with 1000 to 12000 rows, one matrix of 5632 x 2048 with 300 to 4000, gated and down), where 256-row tiles, 128 or 256
+// wide, took 1.22 times as long. With experts, whose counts only the device knows, the row tiles are a mean over four
+// counts around the average. Eight rounds of 256 x 256 tiles and more: these (8 experts of gated 7168 x 4096, 6000 | 12000 rows 667 | 1295, 192
+// x 128 688 | 1336: fewer bytes cost less power).
+constexpr long long RG_MANY = 8 * 256;
+
+static const RgForm& rg_form(const RowLinear& p) {
+  const int E = p.offs ? p.E : 1;
+  const long long wrows = hy_act_gated(p.act) ? 2LL * p.N : p.N;
+  const float mean = (float)p.R / (float)E, sd = E > 1 && p.even_rows <= 0 ? sqrtf(mean * (1.f - 1.f / (float)E)) : 0.f;
+  const float stream = 3.5f + (float)E * (float)wrows * (float)p.K * 2 / 5.4e6f;  // the weights themselves
+  const RgForm* best = nullptr;
+  float least = 1e30f;
+  for (const RgForm& f : RG_FORMS) {
+    float mt = 0.f;
+    for (int i = 0; i < 4; ++i) mt += ceilf((mean + (0.8f * (float)i - 1.2f) * sd) / (float)(32 * f.mi));
+    const float tiles = mt * .25f * (float)E * (float)((wrows + 32 * f.nj - 1) / (32 * f.nj)), load = tiles / 256.f;
+    if (f.mi == 8 && tiles >= (float)RG_MANY) return f;
+    const float deep = f.mi == 8 ? ceilf(load - .02f) : (load <= 1.f ? 1.f : (load <= 2.f ? 2.f : load + f.last));
+    float us = f.fill + f.step * (float)(p.K / RG_BK) * (1.f + f.more * (deep - 1.f));
+    if (us < stream) us = stream;
+    if (us < least) {
+      least = us;
+      best = &f;
+    }
+  }
+  return *best;
+}
+
 int hy_rows_gemm(const RowLinear& p, hipStream_t s) {
   const int gated = hy_act_gated(p.act), E = p.offs ? p.E : 1;
   const long long wrows = gated ? 2LL * p.N : p.N;
-  const long long mt_max = p.R / RG_BM + E;          // m-tiles at most (every expert's last one ragged)
-  const long long mt = E == 1 ? (p.R + RG_BM - 1) / RG_BM : (p.R + RG_BM / 2LL * E) / RG_BM;  // ... on average
-  const long long t8 = (wrows + 255) / 256, t4 = (wrows + 127) / 128;
-  // whole rounds of 256 workgroups, a 256 x 128 tile at 0.55 of a 256 x 256 one's time
-  const bool narrow = 55 * ((mt * t4 + 255) / 256) < 100 * ((mt * t8 + 255) / 256);
-  const long long tn = narrow ? t4 : t8, grid = (mt_max * tn + 7) / 8 * 8;
+  const RgForm& f = rg_form(p);
+  const long long tn = (wrows + 32 * f.nj - 1) / (32 * f.nj), grid = ((p.R / (32 * f.mi) + (long long)E) * tn + 7) / 8 * 8;
   if (grid > 0x7fffffffLL) return -4;
-  if (narrow) rows_gemm_kernel<4><<<(unsigned)grid, 256, 0, s>>>(p, gated, (int)tn);
-  else rows_gemm_kernel<8><<<(unsigned)grid, 256, 0, s>>>(p, gated, (int)tn);
+  const unsigned g = (unsigned)grid;
+  if (f.mi == 4) rows_gemm_kernel<4, 4><<<g, 256, 0, s>>>(p, gated, (int)tn);
+  else if (f.mi == 5) rows_gemm_kernel<4, 5><<<g, 256, 0, s>>>(p, gated, (int)tn);
+  else if (f.mi == 6) rows_gemm_kernel<4, 6><<<g, 256, 0, s>>>(p, gated, (int)tn);
+  else rows_gemm_kernel<8, 8><<<g, 256, 0, s>>>(p, gated, (int)tn);
   JLA_CHECK_LAUNCH();
   return 0;
 }

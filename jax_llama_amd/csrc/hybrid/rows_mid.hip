@@ -159,14 +159,15 @@ static RmPlan rm_plan(const RowLinear& p) {
 //  * bf16 rows of one matrix: to 255; from 256 on a prompt's rows have the 256-row tiles (us here | there, weights in no cache: 2048 x 2048,
 //    255 | 777 rows 16 | 18, 27 | 25 with its sums; 4096 x 4096, 255 | 300 24.6 | 25.5, 29.9 | 27.7; 8224 x 2048, 300 33.2 | 31.4), and
 //    wide outputs from 129 (32000 x 2048, 128 | 200 rows 48.5 | 47.4, 59 | 49; gated 14336 x 4096, 200 92 | 87).
-//  * rows by expert: more than 64 up to 112 per expert on average (8 experts, gated 2816 x 2048 and down, 96 | 320 | 800 rows 50 | 98, 49 | 92,
-//    66 | 75 and 22 | 63, 26 | 50, 31 | 52; 128 per expert 80 | 78 and 39 | 54, 32 experts 241 | 267 and 135 | 109), of K below 256
-//    to 64 (16 per-head matrices of 512 x 128, 64 | 80 rows each 7.0 | 8.1, 10.9 | 8.1). Up to 64 rows in all rows_gemv.hip, unless there
+//  * rows by expert: more than 64 up to 104 per expert on average, 64 where rows_gemm.hip's 128-row tiles are enough for every compute unit
+//    (us here | there, 8 experts: gated 2816 x 2048, 64 | 80 | 112 rows each 59 | 51, 60 | 51, 67 | 54, gated 7168 x 4096, 80 | 112 213 | 203, 213 |
+//    204; too few tiles: 2048 x 2816, 80 | 96 | 112 25 | 35, 25 | 36, 43 | 36, 4096 x 7168 95 | 120, 116 | 122, 175 | 131; 32 experts, 2048 x 2816, 64 | 80
+//    90 | 81, 113 | 84), of K below 256 to 64 (16 per-head matrices of 512 x 128, 64 | 80 rows each 7.0 | 8.1, 10.9 | 8.1). Up to 64 rows in all rows_gemv.hip, unless there
 //    are five per expert on large matrices (8 experts, 56 rows: gated 7168 x 4096 171 | 213, 4096 x 7168 82 | 106; gated 2816 x 2048 51 | 48, gated 512 x 1024 11 | 8).
 constexpr int RM_MIN_ROWS = 9, RM_F32_ROWS = 64, RM_FEW_ROWS = 24, RM_FEW_K = 1024, RM_ROWS = 255;
 constexpr int RM_WIDE = 16384, RM_WIDE_ROWS = 128;
 constexpr long long RM_SORTED_WORK = 20000000;
-constexpr int RM_EXPERT_ROWS = 112, RM_SORTED_ROWS = 64, RM_SHORT_K = 256, RM_SHORT_ROWS = 64;
+constexpr int RM_EXPERT_ROWS = 104, RM_SORTED_ROWS = 64, RM_SHORT_K = 256, RM_SHORT_ROWS = 64;
 
 bool hy_rows_mid_takes(const RowLinear& p) {
   auto aligned = [](const void* x, size_t n) { return ((uintptr_t)x & (n - 1)) == 0; };
@@ -176,7 +177,10 @@ bool hy_rows_mid_takes(const RowLinear& p) {
     return false;
   const long long nw = hy_act_gated(p.act) ? 2LL * p.N : p.N;
   if (p.offs) {
-    if (p.R > RM_SORTED_ROWS) return p.R <= (long long)(p.K < RM_SHORT_K ? RM_SHORT_ROWS : RM_EXPERT_ROWS) * p.E;
+    if (p.R > RM_SORTED_ROWS) {
+      const bool tiles = p.a_bf16 && p.K >= RM_TILES_K && p.E * ((nw + 127) / 128) >= 256;
+      return p.R <= (long long)(p.K < RM_SHORT_K || tiles ? RM_SHORT_ROWS : RM_EXPERT_ROWS) * p.E;
+    }
     if (p.a_bf16) return p.even_rows >= RM_MIN_ROWS;
     return p.R >= 5LL * p.E && nw >= 4096 && nw * p.K >= RM_SORTED_WORK;
   }
