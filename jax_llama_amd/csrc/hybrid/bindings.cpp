@@ -226,7 +226,7 @@ bool rows_parts(Tensor x, Tensor gain, double eps, Tensor prev, Tensor mu, std::
   jla::RowLinear p{};
   p.a = rows2d(x, "x", K, &p.lda);
   p.K = K; p.R = R; p.E = 1;
-  p.wbf16 = 1;
+  p.wbf16 = wtype(ws[0], "w");
   p.a_norm_w = f32(gain, "gain");
   p.a_norm_eps = eps;
   jla::RowParts t{};
@@ -235,7 +235,7 @@ bool rows_parts(Tensor x, Tensor gain, double eps, Tensor prev, Tensor mu, std::
   t.mu = f32(mu, "mu");
   t.row = f32w(row, "row");
   for (int i = 0; i < t.n; ++i) {
-    if (!wtype(ws[i], "w")) return false;
+    if (wtype(ws[i], "w") != p.wbf16) return false;
     check(ws[i].dim() == 2 && ws[i].size(1) == K && mix[i] < mu.size(0), "rows_parts: w is [N, K], mix a row of mu");
     t.w[i] = ws[i].data_ptr();
     t.N[i] = ws[i].size(0);

@@ -75,7 +75,7 @@ struct RowLinear {
   float2* best;
 };
 int hy_rows_walk_groups(const RowLinear& p);
-// Several bf16 matrices [N, K] that read the same one or two rows: a normed row v, or blended with the row before it, v + (prev - v)
+// Several matrices [N, K] of one type that read the same one or two rows: a normed row v, or blended with the row before it, v + (prev - v)
 // mu[mix] (rows_gemv.hip). first, tgroups: filled in by the launch.
 constexpr int RV_MAX_PARTS = 6;
 struct RowParts {

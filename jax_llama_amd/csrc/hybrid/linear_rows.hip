@@ -5,6 +5,7 @@
 //   one or two normed rows, K <= 512, N <= 2048                 the vector GEMV below
 //   nine to some hundred rows on bf16 weights, K a multiple of 64  rows_mid.hip, tiles of 16 to 128 rows
 //   one to 64 rows on bf16 weights otherwise, 16-byte rows      rows_gemv.hip, on the matrix cores
+//   one or two rows on fp32 weights (up to 8 with an expert each), K 512 (two rows: 1024) to 8192, 16-byte rows   rows_gemv.hip
 //   up to 8 rows, or 64 sorted by expert, otherwise             the vector GEMV below (fp32 weights, odd or short K)
 //   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, 256-row tiles
 //   fp32 weights, 16-byte rows, K >= 512 (256 with many rows)   rows_f32.hip, split products on the bf16 matrix cores

@@ -59,7 +59,7 @@ JLA_DEV float rv_table(const RowLinear& p, int r, int col) {
   return p.mul_bf16 ? bf2f(reinterpret_cast<const bf16_t*>(p.mul_table)[at]) : reinterpret_cast<const float*>(p.mul_table)[at];
 }
 
-constexpr int RV_WALK_ROWS = 2;
+constexpr int RV_WALK_ROWS = 2, RV_WALK_K = 4096;
 
 // The sum of N partial sums in type T
 template <class T, int N>
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   }
 }
 
-// Linear row r as the product reads it, to row i of the staged activations; K <= 1024 V. Every thread of the workgroup (256)
+// Linear row r as the product reads it; K <= 1024 V. Every thread of the workgroup (256)
 // holds columns 4 tid + 1024 u. load() only issues loads: the weights of the first steps are issued behind
 // them, and a wave's loads return in order. With res_y: x + rms(ysc * sum of the row's nsum rows of y) * w, in the
 // norm_residual kernel's order, also written to res_out by the launch's first workgroup.
@@ -470,7 +470,9 @@ struct RvRow {
       }
     }
   }
-  JLA_DEV void stage(const RowLinear& p, int r, int i, int K, int tid, float (*stat)[16], f32x4* staged, const RowParts& t, int part) {
+  // put(u, k, v): this thread's numbers v at columns k, which may be past K
+  template <class Put>
+  JLA_DEV void stage(const RowLinear& p, int r, int K, int tid, float (*stat)[16], const RowParts& t, int part, Put put) {
     if (p.res_y) {
       float ss = 0.f;
 #pragma unroll
@@ -483,13 +485,13 @@ struct RvRow {
       const float sc = 1.f / sqrtf(rv_block_sum(ss, stat) / (float)K + p.res_eps);
       // (with several linear rows of a source row, its first writes)
       const int src = p.a_idx ? p.a_idx[r] : (p.a_div > 1 ? r / p.a_div : r);
-      const bool put = blockIdx.x == 0 && (p.a_div <= 1 || r % p.a_div == 0);
+      const bool keep = blockIdx.x == 0 && (p.a_div <= 1 || r % p.a_div == 0);
 #pragma unroll
       for (int u = 0; u < V; ++u) {
         const int k = 4 * tid + 1024 * u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) x[u][j] += y[u][j] * sc * w[u][j];
-        if (put && k < K) *reinterpret_cast<f32x4*>(p.res_out + (size_t)src * K + k) = x[u];
+        if (keep && k < K) *reinterpret_cast<f32x4*>(p.res_out + (size_t)src * K + k) = x[u];
       }
     }
     if (p.a_norm_w) {
@@ -505,8 +507,7 @@ struct RvRow {
       const int k = 4 * tid + 1024 * u;
       f32x4 v = x[u] * scale;
       if (p.a_norm_w) v *= g[u];
-      v = mixed(t, part, v, u, r, K, k);
-      if (k < K) staged[((size_t)i * K + k) / 4] = v;
+      put(u, k, mixed(t, part, v, u, r, K, k));
     }
   }
 };
@@ -565,11 +566,16 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 #pragma unroll
     for (int u = 0; u < U; ++u) wf[u][t] = load_nt(reinterpret_cast<const u32x4*>(w + at(u)));
   }
-  row.stage(p, r0, 0, K, tid, stat, staged, parts, part);
+  auto to_row = [&](int i) {
+    return [=](int, int k, f32x4 v) {
+      if (k < K) staged[((size_t)i * K + k) / 4] = v;
+    };
+  };
+  row.stage(p, r0, K, tid, stat, parts, part, to_row(0));
   if (nr > 1) {
     row.load(p, r0 + 1, K, tid);
     row.load_mix(parts, part, r0 + 1, K, tid);
-    row.stage(p, r0 + 1, 1, K, tid, stat, staged, parts, part);
+    row.stage(p, r0 + 1, K, tid, stat, parts, part, to_row(1));
   }
   __syncthreads();
   u32x4 xr[U];
@@ -639,6 +645,126 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   }
 }
 
+// One or two rows on fp32 weights, K <= 1024 V, each number multiplied as it is: a thread's numbers of the rows stay in its registers
+// (columns 4 tid + 1024 u, whole lines per wave), a workgroup walks over groups of NT weight rows (gated: gate and up alternate) with the
+// next group's loads issued as this one's are consumed, and the first group's go out ahead of the norm. What bounds it: the weight
+// stream. lr_gemv_kernel, a wave per column or four, reads a row and its norm before the first weight, every wave again. Us there -> here,
+// weights in no cache, one row: 2048 x 2048 6.1 -> 5.6, 2048 x 5632 12.0 -> 10.6, normed 3072 x 2048 8.8 -> 7.2, normed 8224 x 2048 20.9 -> 14.1, gated
+// and normed 5632 x 2048 22.3 -> 18.1, normed 32000 x 2048 53.8 -> 43.6 (6.0 TB/s); errors against 64 bits 1.2e-7 to 1.8e-7 -> 0.8e-7 to 1.2e-7.
+// grid and PARTS as in rows_gemv_walk_kernel; V > 4: rows as they are.
+template <int NT, int V, int RW, int PARTS>
+__global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
+  constexpr int WAVES = 4;
+  __shared__ float red[2][WAVES][NT * RW];
+  __shared__ float stat[WAVES][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int part = 0, tg = blockIdx.x, walk = gridDim.x;
+  if constexpr (PARTS) {
+    while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
+    tg -= parts.first[part];
+    walk = parts.first[part + 1] - parts.first[part];
+    tgroups = parts.tgroups[part];
+    p.w = parts.w[part];
+    p.N = parts.N[part];
+    p.out = parts.out[part];
+    p.ldo = parts.ldo[part];
+    p.act = parts.cap[part] > 0.f ? HY_ACT_SOFTCAP : HY_ACT_NONE;
+    p.act_limit = parts.cap[part];
+  } else {
+    rv_arguments(p);
+  }
+  const int r0 = blockIdx.y * rows_per_group, nr = min(rows_per_group, p.R - r0);
+  const int e = rv_expert(p, r0);
+  if (e < 0) return;  // (the whole workgroup)
+  const int K = p.K, N = p.N;
+  const float* wbase = reinterpret_cast<const float*>(p.w) + (size_t)e * p.w_stride;
+  auto in = [&](int u) { return 4 * tid + 1024 * u < K; };
+  auto weight_row = [&](int tg, int t) {  // this thread's first numbers of it (past the end of K: the row's start, which counts as zero)
+    const int T = tg * NT + t, col = min(gated ? T >> 1 : T, N - 1);
+    return wbase + (size_t)(gated && (T & 1) ? N + col : col) * K;
+  };
+  auto at = [&](int u) { return in(u) ? 4 * tid + 1024 * u : 0; };
+  f32x4 wf[V][NT], x[RW][V];
+  auto weights = [&](int tg) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float* w = weight_row(tg, t);
+#pragma unroll
+      for (int u = 0; u < V; ++u) wf[u][t] = __builtin_bit_cast(f32x4, load_nt(reinterpret_cast<const u32x4*>(w + at(u))));
+    }
+  };
+  if constexpr (V > 4) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const int row = r0 + min(r, nr - 1), src = p.a_idx ? p.a_idx[row] : (p.a_div > 1 ? row / p.a_div : row);
+      const float* xp = reinterpret_cast<const float*>(p.a) + (size_t)src * p.lda;
+#pragma unroll
+      for (int u = 0; u < V; ++u) x[r][u] = *reinterpret_cast<const f32x4*>(xp + at(u));
+    }
+    weights(tg);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const float scale = p.a_scale ? p.a_scale[r0 + min(r, nr - 1)] : 1.f;
+#pragma unroll
+      for (int u = 0; u < V; ++u) x[r][u] = in(u) ? x[r][u] * scale : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  } else {
+    RvRow<V, PARTS> row;
+    row.load(p, r0, K, tid);
+    row.load_mix(parts, part, r0, K, tid);
+    weights(tg);
+    row.stage(p, r0, K, tid, stat, parts, part, [&](int u, int k, f32x4 v) { x[0][u] = k < K ? v : f32x4{0.f, 0.f, 0.f, 0.f}; });
+    if constexpr (RW > 1) {  // (a single row is there twice; the second result is dropped)
+      const int second = r0 + nr - 1;
+      row.load(p, second, K, tid);
+      row.load_mix(parts, part, second, K, tid);
+      row.stage(p, second, K, tid, stat, parts, part, [&](int u, int k, f32x4 v) { x[1][u] = k < K ? v : f32x4{0.f, 0.f, 0.f, 0.f}; });
+    }
+  }
+  for (int buf = 0; tg < tgroups; tg += walk, buf ^= 1) {
+    const int next = tg + walk;
+    const bool more = next < tgroups;  // (workgroup-uniform)
+    float sum[NT * RW];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float* w = more ? weight_row(next, t) : wbase;  // (after the last group: one line, unused)
+      float a[RW][2];  // even and odd numbers
+#pragma unroll
+      for (int r = 0; r < RW; ++r) a[r][0] = a[r][1] = 0.f;
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const f32x4 f = in(u) ? wf[u][t] : f32x4{0.f, 0.f, 0.f, 0.f};  // (an infinite weight must not meet a zero)
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a[r][j & 1] = fmaf(f[j], x[r][u][j], a[r][j & 1]);
+        wf[u][t] = __builtin_bit_cast(f32x4, load_nt(reinterpret_cast<const u32x4*>(w + (more ? at(u) : 0))));
+      }
+#pragma unroll
+      for (int r = 0; r < RW; ++r) sum[t * RW + r] = a[r][0] + a[r][1];
+    }
+#pragma unroll
+    for (int i = 0; i < NT * RW; ++i) sum[i] = wave_sum(sum[i]);
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < NT * RW; ++i) red[buf][wave][i] = sum[i];
+    }
+    __syncthreads();  // (one per group: the other buffer's readers are past the barrier before)
+    const int outs = (gated ? NT / 2 : NT) * RW;
+    if (tid < outs) {
+      const int r = tid % RW, to = tid / RW, slot = gated ? 2 * to : to, col = tg * (gated ? NT / 2 : NT) + to;
+      auto total = [&](int t) {
+        float f[WAVES];
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) f[w] = red[buf][w][t * RW + r];
+        return rv_sum<double>(f);
+      };
+      const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
+      if (r < nr && col < N) rv_store(p, r0 + r, col, g, v);
+    }
+  }
+}
+
 // up to 64 rows, and up to 32 of a wide output, whose tiles fill the chip (64 rows x 32000 columns, K 2048: 70 us on the
 // tiles, 82 here); a short K is over before the waves' sum pays (K 64: one row 3.2 us on the vector unit, 3.6 here, 64 rows
 // 4.8 on the tiles, 5.3 here), and with very many columns the tiles stream it as fast (9 | 17 | 32 rows of K 256 x N 32000: weights in
@@ -661,7 +787,20 @@ static bool rv_takes16(const RowLinear& p) {
          p.w_stride % 8 == 0 && aligned(p.a) && aligned(p.w) && !(p.add_out && p.out_bf16);
 }
 
+// fp32 weights: one or two rows of one matrix, or up to eight with an expert each; with a norm or a pending residual add as far as those
+// stay in registers. A short K ends before the waves' sum pays (us, vector unit | here: one row, K 256 | 512 x N 2048 3.7 | 3.6, 4.1 | 3.7; two
+// rows, K 256 | 512 | 1024 x N 2048 4.3 | 4.4, 4.6 | 4.7, 5.7 | 5.2, K 256 x N 32000 17.0 | 24.1).
+constexpr int RV_F32_MIN_K = 512, RV_F32_MIN_K2 = 1024, RV_F32_MAX_K = 8192;
+static bool rv_takes32(const RowLinear& p) {
+  auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  const bool each = p.tab || p.row_expert;
+  return !p.wbf16 && !p.a_bf16 && !p.out_bf16 && !p.offs && !p.best && (each ? p.R <= HY_GEMV_MAX_R : (p.E == 1 && p.R <= RV_WALK_ROWS)) &&
+         p.K % 4 == 0 && p.K >= (each || p.R == 1 ? RV_F32_MIN_K : RV_F32_MIN_K2) && p.K <= (p.a_norm_w || p.res_y ? RV_WALK_K : RV_F32_MAX_K) && p.lda % 4 == 0 && p.w_stride % 4 == 0 &&
+         aligned(p.a) && aligned(p.w) && (!p.a_norm_w || (!p.a_scale && !each && (p.a_norm_one || aligned(p.a_norm_w))));
+}
+
 bool hy_rows_gemv_takes(const RowLinear& p) {
+  if (!p.wbf16) return rv_takes32(p);
   if (p.a_bf16 || p.out_bf16) return rv_takes16(p);
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
   return p.wbf16 && p.R <= (p.N >= RV_WIDE ? RV_MAX_WIDE_ROWS : RV_MAX_ROWS) &&
@@ -675,7 +814,6 @@ bool hy_rows_gemv_takes(const RowLinear& p) {
 // first weight (RMS norm and product, K 2048 x N 2048 | 5152 | 8224 | 32000 | gated 5632: 6.1 | 9.5 | 12.3 | 34.6 | 13.5 us in the
 // plain form, 5.3 | 7.5 | 9.7 | 23.0 | 10.8 walking; K 4096 x 10304: 26.1 -> 17.8). Rows as they are gain nothing from it (4.7 | 7.2 |
 // 9.3 | 22.7 | 11.5 plain, 5.2 | 7.5 | 9.8 | 22.7 | 11.0 walking). Further rows would not fit the registers.
-constexpr int RV_WALK_K = 4096;
 static bool rv_walks(const RowLinear& p, int rows) {
   return (p.a_norm_w || p.res_y) && !p.offs && rows <= RV_WALK_ROWS && p.K <= RV_WALK_K;
 }
@@ -700,15 +838,28 @@ bool hy_rows_parts_takes(const RowLinear& p, const RowParts& t) {
 int hy_rows_parts(const RowLinear& p, const RowParts& parts, hipStream_t s) {
   if (!hy_rows_parts_takes(p, parts)) return -1;
   RowParts t = parts;
-  const int occ = p.K <= 2048 ? 4 : 2;
+  const int occ = p.K <= 2048 ? 4 : 2, per = p.wbf16 ? 8 : (p.K <= 2048 ? 4 : 2);  // weight rows of a group
   long long all = 0;
-  for (int i = 0; i < t.n; ++i) all += t.tgroups[i] = ((t.N[i] + 3) / 4 + 1) / 2;
+  for (int i = 0; i < t.n; ++i) all += t.tgroups[i] = (t.N[i] + per - 1) / per;
   const int rounds = (int)((all + 256 * occ - 1) / (256 * occ));
   t.first[0] = 0;
   for (int i = 0; i < t.n; ++i) t.first[i + 1] = t.first[i] + (t.tgroups[i] + rounds - 1) / rounds;
+  const dim3 grid(t.first[t.n], 1);
+  if (!p.wbf16) {
+    if (p.K <= 2048) {
+      if (p.R == 1) rows_walk_f32_kernel<4, 2, 1, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+      else rows_walk_f32_kernel<4, 2, 2, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+    } else if (p.R == 1) {
+      rows_walk_f32_kernel<2, 4, 1, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+    } else {
+      rows_walk_f32_kernel<2, 4, 2, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+    }
+    JLA_CHECK_LAUNCH();
+    return 0;
+  }
   const unsigned lds = (unsigned)(p.R * p.K * sizeof(float));
-  if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1><<<dim3(t.first[t.n], 1), 256, lds, s>>>(p, p.R, 0, 0, t);
-  else rows_gemv_walk_kernel<2, 8, 4, 1><<<dim3(t.first[t.n], 1), 256, lds, s>>>(p, p.R, 0, 0, t);
+  if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1><<<grid, 256, lds, s>>>(p, p.R, 0, 0, t);
+  else rows_gemv_walk_kernel<2, 8, 4, 1><<<grid, 256, lds, s>>>(p, p.R, 0, 0, t);
   JLA_CHECK_LAUNCH();
   return 0;
 }
@@ -729,7 +880,7 @@ static bool rv_walk_grid(const RowLinear& p, int groups, int& wnt, long long& tg
 int hy_rows_walk_groups(const RowLinear& p) {
   int wnt;
   long long tg, wgs;
-  return hy_rows_gemv_takes(p) && rv_walks(p, p.R) && !p.row_expert && !p.tab && rv_walk_grid(p, 1, wnt, tg, wgs) && wnt == 2 ? (int)wgs : 0;
+  return p.wbf16 && hy_rows_gemv_takes(p) && rv_walks(p, p.R) && !p.row_expert && !p.tab && rv_walk_grid(p, 1, wnt, tg, wgs) && wnt == 2 ? (int)wgs : 0;
 }
 
 // bf16 rows. Us, weights in no cache, 8 rows, one | two | four tiles per workgroup: 2048 x 2048 5.4 | 6.3 | 8.0, 3072 x 2048 6.7 | 6.6 | 8.3, 2048 x
@@ -757,7 +908,51 @@ static int rv_rows16(const RowLinear& p, int rows, int groups, int gated, hipStr
   return 0;
 }
 
+// Weight rows per group: one from K 2049 on for a single row, whose groups are longer than a trip to memory anyway, two for two rows; up to K 2048
+// four where that leaves whole numbers of groups per compute unit. Us, weights in no cache, one | two | four, one row: 2048 x 2048 5.67 | 6.04 |
+// 5.63, 3072 x 2048 normed 7.04 | 7.25 | 7.82, 8224 x 2048 14.5 | 14.6 | 14.1, 2048 x 5632 10.6 | 11.6 | 11.7, 4096 x 7168 20.9 | 22.0 | 31.0, 10304 x
+// 4096 normed 29.9 | 31.7 | 31.8; two rows: 10304 x 4096 42.1 | 36.0 | 36.1, 4096 x 7168 24.9 | 24.0 | 32.9.
+static int rv_rows32(const RowLinear& p, hipStream_t s) {
+  const int gated = hy_act_gated(p.act);
+  const bool each = p.row_expert || p.tab;
+  const int groups = each ? p.R : 1, rpg = each ? 1 : p.R;
+  const long long rows = gated ? 2LL * p.N : p.N, all = rows * groups;  // weight rows
+  const int nt = p.K > 2048 ? (rpg == 1 && !gated ? 1 : 2) : (all >= 4096 || (all >= 1024 && all <= 2048) ? 4 : 2);
+  const long long tg = (rows + nt - 1) / nt, room = 256LL * 4 / groups, rounds = (tg + room - 1) / room;  // (four workgroups per compute unit)
+  if (tg > 0x7fffffffLL) return -4;
+  const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
+#define RV_RUN32(NT, V, RW) rows_walk_f32_kernel<NT, V, RW, 0><<<grid, 256, 0, s>>>(p, rpg, gated, (int)tg, RowParts{})
+#define RV_SHORT32(V)                   \
+  do {                                  \
+    if (nt == 2) {                      \
+      if (rpg == 1) RV_RUN32(2, V, 1);  \
+      else RV_RUN32(2, V, 2);           \
+    } else if (rpg == 1) {              \
+      RV_RUN32(4, V, 1);                \
+    } else {                            \
+      RV_RUN32(4, V, 2);                \
+    }                                   \
+  } while (0)
+#define RV_LONG32(V)                    \
+  do {                                  \
+    if (nt == 1) RV_RUN32(1, V, 1);     \
+    else if (rpg == 1) RV_RUN32(2, V, 1); \
+    else RV_RUN32(2, V, 2);             \
+  } while (0)
+  if (p.K <= 1024) RV_SHORT32(1);
+  else if (p.K <= 2048) RV_SHORT32(2);
+  else if (p.K <= 4096) RV_LONG32(4);
+  else if (p.K <= 6144) RV_LONG32(6);
+  else RV_LONG32(8);
+#undef RV_LONG32
+#undef RV_SHORT32
+#undef RV_RUN32
+  JLA_CHECK_LAUNCH();
+  return 0;
+}
+
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
+  if (!p.wbf16) return rv_rows32(p, s);
   const int gated = hy_act_gated(p.act);
   RowLinear q = p;
   const bool each = !p.offs && (p.row_expert || p.tab);  // one row, one expert per group

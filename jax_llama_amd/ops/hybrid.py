@@ -298,7 +298,7 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
     take the pending residual add and the gate in the product's launch; else the separate ops."""
     r = x if isinstance(x, Residual) else None
     ids = ids.reshape(-1).to(torch.int32).contiguous() if ids is not None else None
-    if r is not None and r.fusable() and w.dtype == BF16:
+    if r is not None and r.fusable() and _walks(r.x.shape[0], w):
         out = torch.empty(r.x.shape[0], w.shape[0], dtype=F32, device=r.x.device)
         new = torch.empty_like(r.x)
         if ext().rows_fused(r.x, w, out, *r.pending, new, ids, table, int(col0)):
@@ -310,18 +310,24 @@ def linear_rows_gated(x, w: torch.Tensor, ids: Optional[torch.Tensor] = None, ta
         xv = r.value() if r is not None else x
     if ids is None:
         return linear(xv, w)
-    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and w.dtype == BF16:
+    if _gpu(xv) and xv.shape[0] <= FEW_ROWS and w.shape[0] > SKINNY_MAX_N and _walks(xv.shape[0], w):
         out = torch.empty(xv.shape[0], w.shape[0], dtype=F32, device=xv.device)
         if ext().rows_fused(xv, w, out, None, 1, 1.0, None, 0.0, None, ids, table, int(col0)):
             return out
     return gelu_gate_rows(linear(xv, w), ids, table, col0)
 
 
+def _walks(rows: int, w: torch.Tensor) -> bool:
+    """Whether few rows on ``w`` are worth offering to ``rows_gemv.hip``: bf16 weights, or one or two rows on fp32 ones whose rows stay in
+    registers (csrc: rv_takes32)."""
+    return w.dtype == BF16 or (rows <= RESIDUAL_MAX_ROWS and w.shape[-1] % 4 == 0 and (512 if rows == 1 else 1024) <= w.shape[-1] <= 4096)
+
+
 def norms_free(rows: int, w: torch.Tensor, k: Optional[int] = None) -> bool:
     """Whether a product of ``rows`` rows of ``k`` numbers (``w``'s columns) on matrices like ``w`` norms them at no cost (csrc: the
     walking form of rows_gemv.hip)."""
     k = w.shape[1] if k is None else k
-    return (_gpu(w) and w.dtype == BF16 and w.dim() == 2 and rows <= RESIDUAL_MAX_ROWS and w.shape[0] > SKINNY_MAX_N
+    return (_gpu(w) and w.dim() == 2 and rows <= RESIDUAL_MAX_ROWS and w.shape[0] > SKINNY_MAX_N and _walks(rows, w)
             and k % 8 == 0 and 256 <= k <= 4096)
 
 
@@ -640,7 +646,7 @@ def moe_table(x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, w_gu: tor
     m, top, e_n = x.shape[0], table.shape[1], w_gu.shape[0]
     r = m * top
     ids = ids.reshape(-1)
-    if _gpu(x) and 0 < r <= ext().GEMV_MAX_R and x.dtype == F32 and w_gu.dtype == w_down.dtype == BF16:
+    if _gpu(x) and 0 < r <= ext().GEMV_MAX_R and x.dtype == F32 and w_gu.dtype == w_down.dtype:
         # decode: the products read the table themselves, and the first one adds a pending residual
         h = torch.empty(r, w_gu.shape[1] // 2, dtype=F32, device=x.device)
         y = torch.empty(r, w_down.shape[1], dtype=F32, device=x.device)
@@ -1637,7 +1643,7 @@ def shifted_linears(h, prev: torch.Tensor, mu: torch.Tensor, parts) -> Optional[
     tanh(. / cap)``. ``row``: the normed rows, which ``prev`` is to hold when this token is done (``timemix_memory``). None where the
     separate ops run."""
     if not isinstance(h, RmsInput) or not _gpu(h.x) or h._value is not None or h.x.shape[0] > RESIDUAL_MAX_ROWS \
-            or any(w.dtype != BF16 for w, _, _ in parts) or not h.x.is_contiguous() or h.gain.numel() != h.x.shape[1]:
+            or any(w.dtype != parts[0][0].dtype for w, _, _ in parts) or not h.x.is_contiguous() or h.gain.numel() != h.x.shape[1]:
         return None
     m = h.x.shape[0]
     sizes = [m * w.shape[0] for w, _, _ in parts]
