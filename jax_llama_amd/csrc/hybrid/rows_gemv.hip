@@ -645,19 +645,30 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   }
 }
 
+// v plus that of the lane whose number differs in the bits of a DPP control (quad_perm 0xb1: 1, 0x4e: 2; row_half_mirror 0x141 and row_mirror 0x140
+// pair the halves once those hold one sum)
+template <int CTRL>
+JLA_DEV double rw_add(double v) {
+  const u32x2 b = __builtin_bit_cast(u32x2, v);
+  const u32x2 o = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[0], CTRL, 0xf, 0xf, true), (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[1], CTRL, 0xf, 0xf, true)};
+  return v + __builtin_bit_cast(double, o);
+}
+
 // One or two rows on fp32 weights, K <= 1024 V, each number multiplied as it is: a thread's numbers of the rows stay in its registers
 // (columns 4 tid + 1024 u, whole lines per wave), a workgroup walks over groups of NT weight rows (gated: gate and up alternate) with the
 // next group's loads issued as this one's are consumed, and the first group's go out ahead of the norm. What bounds it: the weight
 // stream. lr_gemv_kernel, a wave per column or four, reads a row and its norm before the first weight, every wave again. Us there -> here,
-// weights in no cache, one row: 2048 x 2048 6.1 -> 5.6, 2048 x 5632 12.0 -> 10.6, normed 3072 x 2048 8.8 -> 7.2, normed 8224 x 2048 20.9 -> 14.1, gated
-// and normed 5632 x 2048 22.3 -> 18.1, normed 32000 x 2048 53.8 -> 43.6 (6.0 TB/s); errors against 64 bits 1.2e-7 to 1.8e-7 -> 0.8e-7 to 1.2e-7.
+// weights in no cache, one row: 2048 x 2048 6.1 -> 5.4, 2048 x 5632 12.0 -> 10.5, normed 3072 x 2048 8.8 -> 7.2, normed 8224 x 2048 20.9 -> 13.6, gated
+// and normed 5632 x 2048 22.3 -> 17.6, normed 32000 x 2048 53.8 -> 42.9 (6.1 TB/s); errors against 64 bits 1.2e-7 to 1.8e-7 -> 0.5e-7 to 1.0e-7 (the 256
+// threads' parts added by lane exchanges in 32 bits: 0.8e-7 to 1.2e-7, and 1 to 3 % slower). The same kernel on bf16 weights is as fast as the
+// matrix cores' there, not faster (normed 8224 x 2048 9.6 | 8.8, 2048 x 2048 4.2 | 4.4, 2048 x 5632 7.9 | 8.3).
 // grid and PARTS as in rows_gemv_walk_kernel; V > 4: rows as they are.
 template <int NT, int V, int RW, int PARTS>
 __global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
-  constexpr int WAVES = 4;
-  __shared__ float red[2][WAVES][NT * RW];
-  __shared__ float stat[WAVES][16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  static_assert(NT * RW <= 16, "sixteen threads per sum");
+  __shared__ float red[2][NT * RW][256];
+  __shared__ float stat[4][16];
+  const int tid = threadIdx.x;
   int part = 0, tg = blockIdx.x, walk = gridDim.x;
   if constexpr (PARTS) {
     while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
@@ -690,7 +701,7 @@ __global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int row
     for (int t = 0; t < NT; ++t) {
       const float* w = weight_row(tg, t);
 #pragma unroll
-      for (int u = 0; u < V; ++u) wf[u][t] = __builtin_bit_cast(f32x4, load_nt(reinterpret_cast<const u32x4*>(w + at(u))));
+      for (int u = 0; u < V; ++u) wf[u][t] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w + at(u)));
     }
   };
   if constexpr (V > 4) {
@@ -724,7 +735,6 @@ __global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int row
   for (int buf = 0; tg < tgroups; tg += walk, buf ^= 1) {
     const int next = tg + walk;
     const bool more = next < tgroups;  // (workgroup-uniform)
-    float sum[NT * RW];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const float* w = more ? weight_row(next, t) : wbase;  // (after the last group: one line, unused)
@@ -738,29 +748,32 @@ __global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int row
         for (int r = 0; r < RW; ++r)
 #pragma unroll
           for (int j = 0; j < 4; ++j) a[r][j & 1] = fmaf(f[j], x[r][u][j], a[r][j & 1]);
-        wf[u][t] = __builtin_bit_cast(f32x4, load_nt(reinterpret_cast<const u32x4*>(w + (more ? at(u) : 0))));
+        wf[u][t] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w + (more ? at(u) : 0)));
       }
 #pragma unroll
-      for (int r = 0; r < RW; ++r) sum[t * RW + r] = a[r][0] + a[r][1];
-    }
-#pragma unroll
-    for (int i = 0; i < NT * RW; ++i) sum[i] = wave_sum(sum[i]);
-    if (lane == 0) {
-#pragma unroll
-      for (int i = 0; i < NT * RW; ++i) red[buf][wave][i] = sum[i];
+      for (int r = 0; r < RW; ++r) red[buf][t * RW + r][tid] = a[r][0] + a[r][1];
     }
     __syncthreads();  // (one per group: the other buffer's readers are past the barrier before)
-    const int outs = (gated ? NT / 2 : NT) * RW;
-    if (tid < outs) {
-      const int r = tid % RW, to = tid / RW, slot = gated ? 2 * to : to, col = tg * (gated ? NT / 2 : NT) + to;
-      auto total = [&](int t) {
-        float f[WAVES];
+    // sixteen threads to a sum, its 256 parts added in 64 bits
+    const int i = tid >> 4, sub = tid & 15;
+    if (i < NT * RW) {  // (whole rows of 16 lanes; gated: gate and up are rows 16 RW lanes apart, in one wave)
+      float f[16];
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) f[w] = red[buf][w][t * RW + r];
-        return rv_sum<double>(f);
-      };
-      const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
-      if (r < nr && col < N) rv_store(p, r0 + r, col, g, v);
+      for (int j = 0; j < 16; ++j) f[j] = red[buf][i][16 * j + sub];
+      double d[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) d[j] = f[j];
+#pragma unroll
+      for (int n = 8; n > 0; n /= 2)
+#pragma unroll
+        for (int j = 0; j < n; ++j) d[j] += d[j + n];
+      d[0] = rw_add<0xb1>(d[0]);
+      d[0] = rw_add<0x4e>(d[0]);
+      d[0] = rw_add<0x141>(d[0]);
+      d[0] = rw_add<0x140>(d[0]);
+      const float g = (float)d[0], v = NT > 1 && gated ? __shfl_xor(g, 16 * RW, 64) : 0.f;
+      const int r = i % RW, t = i / RW, col = tg * (gated ? NT / 2 : NT) + (gated ? t >> 1 : t);
+      if (sub == 0 && !(gated && (t & 1)) && r < nr && col < N) rv_store(p, r0 + r, col, g, v);
     }
   }
 }

@@ -7,8 +7,8 @@ from jax_llama_amd.ops import hybrid as hy
 
 pytestmark = pytest.mark.gpu
 DEV, F32, F64 = "cuda", torch.float32, torch.float64
-# up to 16 products one behind the other in each of two chains, six lane exchanges, two joins: roundings of random sign, sqrt(24) 2^-24 = 2.9e-7
-# of the sum's share; a norm or a gate adds a few more of one number
+# up to 16 products one behind the other in each of two chains and their join, the 256 threads' parts added in 64 bits: roundings of random
+# sign, sqrt(17) 2^-24 = 2.5e-7 of the sum's share; a norm or a gate adds a few more of one number
 TOL = 6e-7
 
 
