@@ -25,7 +25,7 @@
 // columns); the next chunk's loads are in flight meanwhile.
 // A number that is none (in a key, query, value or gate, or by overflow) would spoil every token of its chunk, as masked products
 // are 0 x NaN: such a chunk is walked token by token, and only the tokens from that one on see it (the check and the walk's
-// registers cost 5 %: 2048 tokens of 16 heads 209 -> 220 us).
+// registers cost 5 %).
 #include "hy_util.h"
 #include "hybrid.h"
 
@@ -360,8 +360,10 @@ struct ChunkWalk {
 
 // The walk where its waves would leave SIMDs idle: the four waves of a workgroup share 16 value columns, each holds a quarter of
 // the key rows of their state (DBW 16-row blocks), and the two products that sum over the key rows (K S and Q S) meet in LDS
-// once per chunk. Operands come straight from memory, a chunk ahead. A chunk's chain per wave at dim 128 is 76 MFMAs instead
-// of 216; 2048 tokens of one row, 16 heads of 128 x 128: 316 -> 218 us with the delta rule's first launch.
+// once per chunk. Operands come straight from memory, a chunk ahead, their loads between a chunk's first products: 43 of them in one
+// run keep the four waves waiting for the memory path. A chunk's chain per wave at dim 128 is 76 MFMAs instead
+// of 216; 2048 tokens of one row, 16 heads of 128 x 128: 316 -> 218 us with the delta rule's first launch; loads between the products, an output's
+// place formed once and sums in the vector unit's registers (build.py) 233 -> 195 (another day's clock), scalar gates 140 -> 111, 777 tokens 64 -> 53.
 // grid (H, ceil(ncols / 16), B): workgroups go round the XCDs by their id, so a head's columns mostly share one L2.
 // DELTA 0 (scalar gates): u = v, no K S.
 template <int DBW, int DELTA>
@@ -386,6 +388,10 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
   const float* vp = p.v + (size_t)b * p.S * p.ldv + (size_t)h * p.vdim;
   const float* wp = p.ws + ((size_t)b * p.H + h) * p.chunks * WS;
   const int mt_o = wave & 1;  // the token tile whose output waves 0 and 1 finish
+  float* const op = p.o + ((size_t)b * p.S * p.H + h) * p.ncols;
+  unsigned oo[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) oo[r] = (unsigned)(16 * mt_o + 4 * q + r) * (unsigned)p.H * (unsigned)p.ncols + (unsigned)j;
   unsigned oq[2], oa[2], ok[2][4], ov[2][4];
   auto places = [&](int left) {  // rows of a chunk with `left` tokens (further ones repeat the last: their u is 0)
 #pragma unroll
@@ -406,8 +412,7 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     float kt[DBW][2][4], va[2][4], glast;
   };
   const unsigned row = (unsigned)(c * DC + 4 * q);
-  auto fetch = [&](Operands& x, int ch) {  // chunk ch (called in order) on its way to registers
-    if (ch == 0 || (ch + 1) * DC > p.S) places(min(p.S - ch * DC, DC));
+  auto fetch = [&](Operands& x, bool last) {  // a chunk on its way to registers; the pointers go to the next one behind it
 #pragma unroll
     for (int kb = 0; kb < DBW; ++kb)
 #pragma unroll
@@ -437,10 +442,11 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
 #pragma unroll
         for (int mb = 0; mb < DBW; ++mb) x.kt[mb][mt][r] = kp[ok[mt][r] + 16 * mb];
       }
-    qp += (size_t)DC * p.ldq;
-    kp += (size_t)DC * p.ldk;
-    vp += (size_t)DC * p.ldv;
-    wp += WS;
+    const int on = last ? 0 : DC;  // (no branch, which would keep the loads in front of the products)
+    qp += (size_t)(unsigned)on * (unsigned)p.ldq;
+    kp += (size_t)(unsigned)on * (unsigned)p.ldk;
+    vp += (size_t)(unsigned)on * (unsigned)p.ldv;
+    wp += (unsigned)on * (unsigned)(WS / DC) + (on ? (unsigned)(WS % DC) : 0u);
   };
   // chunk ch token by token: a number that is none spoils the tokens from its own on, not those before it. Every wave of the
   // workgroup comes here together.
@@ -489,7 +495,13 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
     }
     __syncthreads();
   };
-  auto step = [&](const Operands& x, int ch, int buf) {
+  // chunk ch, with the loads of the next one between its first products: in front of them the waves would wait for the memory
+  // path to take all of them (behind the last chunk: that one again, unused)
+  constexpr int FIRST = (DELTA ? 16 : 8) * DBW, LOADS = DELTA ? 12 * DBW + 19 : 10 * DBW + 14;
+  auto step = [&](const Operands& x, Operands& xn, int ch, int buf) {
+    const int next = min(ch + 1, p.chunks - 1);
+    if ((next + 1) * DC > p.S) places(p.S - next * DC);
+    fetch(xn, next + 1 == p.chunks);
     f32x4 qs[2][4], ks[2][4];  // (short chains)
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -504,6 +516,11 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
           if (DELTA) ks[mt][r] = mma_f32(x.ka[kb][mt][r], S[kb][r], ks[mt][r]);
           qs[mt][r] = mma_f32(x.qa[kb][mt][r], S[kb][r], qs[mt][r]);
         }
+#pragma unroll
+    for (int i = 0; i < FIRST; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product, then its share of the loads
+      __builtin_amdgcn_sched_group_barrier(0x020, (LOADS + FIRST - 1) / FIRST, 0);
+    }
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       red[buf][wave][mt][lane] = (qs[mt][0] + qs[mt][1]) + (qs[mt][2] + qs[mt][3]);
@@ -556,11 +573,10 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = fmaf(o[r], g[r], (in[0][r] + in[1][r]) + (in[2][r] + in[3][r]));
+      float* const to = op + (size_t)ch * DC * p.H * p.ncols;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = ch * DC + 16 * mt_o + 4 * q + r;
-        if (t < p.S && j < p.ncols) p.o[(((size_t)b * p.S + t) * p.H + h) * p.ncols + j] = DELTA ? o[r] : o[r] * p.o_scale;
-      }
+      for (int r = 0; r < 4; ++r)
+        if (j < p.ncols && ch * DC + 16 * mt_o + 4 * q + r < p.S) to[oo[r]] = DELTA ? o[r] : o[r] * p.o_scale;
     }
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -581,15 +597,11 @@ __global__ void __launch_bounds__(256) chunk_walk_split_kernel(ChunkWalk p) {
   };
   // two sets of operands in turn: moved from one set to another, a chunk's loads would be waited for at the end of each step
   Operands x0, x1;
-  fetch(x0, 0);
-  if (p.chunks > 1) fetch(x1, 1);
+  places(min(p.S, DC));
+  fetch(x0, p.chunks == 1);
   for (int ch = 0; ch < p.chunks; ch += 2) {
-    step(x0, ch, 0);
-    if (ch + 2 < p.chunks) fetch(x0, ch + 2);
-    if (ch + 1 < p.chunks) {
-      step(x1, ch + 1, 1);
-      if (ch + 3 < p.chunks) fetch(x1, ch + 3);
-    }
+    step(x0, x1, ch, 0);
+    if (ch + 1 < p.chunks) step(x1, x0, ch + 1, 1);
   }
   if (j < p.ncols) {
 #pragma unroll
