@@ -123,8 +123,8 @@ __global__ void __launch_bounds__(AD3_WAVES * 64)
       float mx = sc[h][0];
 #pragma unroll
       for (int r = 1; r < KPG; ++r) mx = fmaxf(mx, sc[h][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = lane_max16(mx);
+      mx = lane_max32(mx);
       const float mn = fmaxf(m_h[h], mx);
       if (mn == -INFINITY) continue;  // nothing valid for this wave yet (wave-uniform)
       const float alpha = __expf(m_h[h] - mn);  // m_h = -inf -> 0
@@ -147,13 +147,13 @@ __global__ void __launch_bounds__(AD3_WAVES * 64)
 #pragma unroll
   for (int h = 0; h < REP; ++h) {
     float l = l_h[h];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = lane_sum16(l);
+    l = lane_sum32(l);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       float v = o[h][e];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = lane_sum16(v);
+      v = lane_sum32(v);
       o[h][e] = v;
     }
     if (g == 0) {
@@ -288,8 +288,8 @@ __global__ void __launch_bounds__(AD5_WAVES * 64)
     float mx = sc[h][0];
 #pragma unroll
     for (int r = 1; r < KPG; ++r) mx = fmaxf(mx, sc[h][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_max16(mx);
+    mx = lane_max32(mx);
     float l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (mx != -INFINITY) {  // wave-uniform
 #pragma unroll
@@ -302,12 +302,12 @@ __global__ void __launch_bounds__(AD5_WAVES * 64)
         for (int e = 0; e < 8; ++e) o[e] += p * vf[e];
       }
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = lane_sum16(l);
+    l = lane_sum32(l);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      o[e] += __shfl_xor(o[e], 16, 64);
-      o[e] += __shfl_xor(o[e], 32, 64);
+      o[e] = lane_sum16(o[e]);
+      o[e] = lane_sum32(o[e]);
     }
     if (g == 0) {
 #pragma unroll
@@ -507,8 +507,8 @@ __global__ void __launch_bounds__(64)
         float cm = sc[h][0];
 #pragma unroll
         for (int r = 1; r < KPG; ++r) cm = fmaxf(cm, sc[h][r]);
-        cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-        cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+        cm = lane_max16(cm);
+        cm = lane_max32(cm);
         const float mn = fmaxf(m_h[h], cm);
         const float alpha = (m_h[h] == -INFINITY) ? 0.f : __expf(m_h[h] - mn);
         m_h[h] = mn;
@@ -581,14 +581,14 @@ __global__ void __launch_bounds__(64)
     // across the 4 lane groups: each group summed its own rows (l is the same in its 16 lanes)
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
-      l_h[h] += __shfl_xor(l_h[h], 16, 64);
-      l_h[h] += __shfl_xor(l_h[h], 32, 64);
+      l_h[h] = lane_sum16(l_h[h]);
+      l_h[h] = lane_sum32(l_h[h]);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          o[h][i][e] += __shfl_xor(o[h][i][e], 16, 64);
-          o[h][i][e] += __shfl_xor(o[h][i][e], 32, 64);
+          o[h][i][e] = lane_sum16(o[h][i][e]);
+          o[h][i][e] = lane_sum32(o[h][i][e]);
         }
     }
   }
@@ -749,8 +749,8 @@ __global__ void __launch_bounds__(64)
         float cm = sc[h][0];
 #pragma unroll
         for (int r = 1; r < KPG; ++r) cm = fmaxf(cm, sc[h][r]);
-        cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-        cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+        cm = lane_max16(cm);
+        cm = lane_max32(cm);
         const float mn = fmaxf(m_h[h], cm);
         const float alpha = __builtin_amdgcn_exp2f(m_h[h] - mn);
         m_h[h] = mn;
@@ -804,14 +804,14 @@ __global__ void __launch_bounds__(64)
     // across the 4 lane groups: each group summed its own rows
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
-      l_h[h] += __shfl_xor(l_h[h], 16, 64);
-      l_h[h] += __shfl_xor(l_h[h], 32, 64);
+      l_h[h] = lane_sum16(l_h[h]);
+      l_h[h] = lane_sum32(l_h[h]);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          o[h][i][e] += __shfl_xor(o[h][i][e], 16, 64);
-          o[h][i][e] += __shfl_xor(o[h][i][e], 32, 64);
+          o[h][i][e] = lane_sum16(o[h][i][e]);
+          o[h][i][e] = lane_sum32(o[h][i][e]);
         }
     }
   }

@@ -23,12 +23,11 @@ JLA_DEV void am_better(float& bv, int& bi, float ov, int oi) {
   }
 }
 JLA_DEV void am_wave(float& bv, int& bi) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    am_better(bv, bi, ov, oi);
-  }
+  lane_halves([&](auto j) {
+    constexpr int J = decltype(j)::value;
+    const float ov = __uint_as_float(lane_xor<J>(__float_as_uint(bv)));
+    am_better(bv, bi, ov, (int)lane_xor<J>((uint32_t)bi));
+  });
 }
 
 // grid (splits, rows): columns [c0, c0 + chunk) of row blockIdx.y; VEC: 16-byte aligned rows. part: [rows][splits] (value,

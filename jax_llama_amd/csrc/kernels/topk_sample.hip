@@ -6,7 +6,7 @@
 //   topk_chunk:  grid (ceil(V/4096), B). A 256-thread workgroup holds a 4096-logit chunk in
 //                registers (16 keys per thread, order-preserving uint32 of the fp32 logit) and finds
 //                the chunk's K-th largest key by 4-pass LDS radix select (8 bits per pass, one wave
-//                scans the 256-bin histogram with DPP-free shuffles). It emits exactly K candidates:
+//                scans the 256-bin histogram with lane moves). It emits exactly K candidates:
 //                everything above the threshold plus the lowest-index ties.
 //   topk_merge:  one workgroup per row merges the C = chunks*K candidates the same way, sorts the K
 //                survivors in one wave (64-lane bitonic network on (key, -index)), and either writes
@@ -17,6 +17,8 @@
 //                Gumbel-max with counter-based Philox4x32-10 keyed by (seed, step, row, rank) -- every
 //                TP rank draws the same token from the same candidates without communicating.
 // Ties: lower vocabulary index first (lax.top_k order).
+// What bounds it: dependent steps within a wave (scans of up to eight radix passes, 21 exchanges of the sort). With lane moves in the place of
+// shuffles through LDS a step of seven rows x 128256 columns is 5 us shorter (23 for both kernels before).
 #include "common.h"
 #include "launchers.h"
 
@@ -65,12 +67,7 @@ JLA_DEV void radix_select(const uint32_t (&key)[E], int K, TkShared& sh, uint32_
         c[q] = sh.hist[255 - 4 * l - q];
         s += c[q];
       }
-      uint32_t incl = s;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t t = __shfl_up(incl, o, 64);
-        if (l >= o) incl += t;
-      }
+      const uint32_t incl = wave_scan(s);
       uint32_t above = incl - s;
       if (above < (uint32_t)kr && (uint32_t)kr <= incl) {  // exactly one lane
         for (int q = 0; q < 4; ++q) {
@@ -96,12 +93,7 @@ JLA_DEV void radix_select(const uint32_t (&key)[E], int K, TkShared& sh, uint32_
 // exclusive block scan of one uint32 per thread (256 threads)
 JLA_DEV uint32_t block_excl_scan(uint32_t v, TkShared& sh) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint32_t incl = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
+  const uint32_t incl = wave_scan(v);
   if (lane == 63) sh.wsum[w] = incl;
   __syncthreads();
   uint32_t base = 0;
@@ -251,15 +243,16 @@ __global__ void __launch_bounds__(TK_THREADS)
   uint64_t v = lane < K ? ((uint64_t)sh.sk[lane] << 32) | (uint32_t)(0x7fffffff - sh.si[lane]) : 0ull;
 #pragma unroll
   for (int k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const uint32_t lo = __shfl_xor((uint32_t)v, j, 64), hi = __shfl_xor((uint32_t)(v >> 32), j, 64);
+    lane_halves([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if (j >= k) return;
+      const uint32_t lo = lane_xor<j>((uint32_t)v), hi = lane_xor<j>((uint32_t)(v >> 32));
       const uint64_t o = ((uint64_t)hi << 32) | lo;
       const bool desc = (lane & k) == 0;  // final k = 64: whole wave descending
       const bool lower = (lane & j) == 0;
       const bool take_max = desc == lower;
       v = take_max ? (o > v ? o : v) : (o < v ? o : v);
-    }
+    });
   }
   const float val = lane < K ? kfloat((uint32_t)(v >> 32)) : -INFINITY;
   const int32_t idx = lane < K ? 0x7fffffff - (int32_t)(uint32_t)v : 0x7fffffff;
@@ -274,10 +267,7 @@ __global__ void __launch_bounds__(TK_THREADS)
   const float l = lane < K ? val * inv_temp : -INFINITY;
   const float mx = __shfl(l, 0, 64);  // sorted: lane 0 holds the max
   float p = lane < K ? __expf(l - mx) : 0.f;
-  float tot = p;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
-  p /= tot;
+  p /= wave_sum(p);
   float incl = p;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -292,15 +282,15 @@ __global__ void __launch_bounds__(TK_THREADS)
   const float g = -__logf(-__logf(u));
   float score = keep ? l + g : -INFINITY;
   int best = lane;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float os = __shfl_xor(score, o, 64);
-    const int ob = __shfl_xor(best, o, 64);
+  lane_halves([&](auto j) {
+    constexpr int J = decltype(j)::value;
+    const float os = __uint_as_float(lane_xor<J>(__float_as_uint(score)));
+    const int ob = (int)lane_xor<J>((uint32_t)best);
     if (os > score || (os == score && ob < best)) {
       score = os;
       best = ob;
     }
-  }
+  });
   const int32_t tok = __shfl(idx, best, 64);
   if (lane == 0) nxt[b] = tok;
 }
