@@ -27,6 +27,7 @@
 // bias column) are indexed by it. Prefill: one wave runs both maps of its query (plain), or a pair of waves runs one map
 // each over the same 32 queries and joins them through LDS (MFMA). Decode: the splits of both maps side by side, joined by
 // the merge.
+#include "attn_chunk.h"
 #include "attn_span.h"
 
 namespace jla {
@@ -305,11 +306,12 @@ __global__ void __launch_bounds__(64) attn_bias_decode_kernel(AttnBias p) {
 }
 
 // decode, bf16 caches, dim = 8 DK8 in {64, 128}, vdim = 64 VREG in {64, 128}: the same split as above with every load of
-// a 64-key chunk (the lane's key row, its bias, all 64 value rows) issued before the first use, and q staged into LDS
+// a 64-key chunk (attn_chunk.h, and the biases) issued before the first use, and q staged into LDS
 // behind them: a decode step is a chain of memory round trips, and this form has two.
 template <int DK8, int VREG>
 __global__ void __launch_bounds__(64) attn_bias_decode_fast_kernel(AttnBias p) {
   constexpr int dim = 8 * DK8, vdim = 64 * VREG;
+  using Chunk = KeyChunk<bf16_t, DK8, VREG>;
   __shared__ float qs[dim];
   const int lane = threadIdx.x;
   const int sp = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
@@ -327,41 +329,23 @@ __global__ void __launch_bounds__(64) attn_bias_decode_fast_kernel(AttnBias p) {
   const bf16_t* vbase = reinterpret_cast<const bf16_t*>(p.vc) + ((size_t)b * p.G + mp.g) * p.T * p.ldv;
   const bool sunk = p.sink && sp == 0;
   const float hs = p.head_scale ? p.head_scale[h] : 1.f;
-  float m_run = sunk ? p.sink[h] : -INFINITY, l_run = sunk ? 1.f : 0.f, acc[VREG];
-#pragma unroll
-  for (int i = 0; i < VREG; ++i) acc[i] = 0.f;
+  float m_run = sunk ? p.sink[h] : -INFINITY, l_run = sunk ? 1.f : 0.f, q8[8] = {}, acc8[8] = {};
   bool staged = false;
   for (int j0 = j_lo; j0 < j_hi; j0 += 64) {
-    const int j = j0 + lane, jc = ab_key(span, min(j, j_hi - 1));  // (jc: the cache slot)
-    u32x4 kf[DK8];
-#pragma unroll
-    for (int u = 0; u < DK8; ++u) kf[u] = *reinterpret_cast<const u32x4*>(kbase + (size_t)jc * p.ldk + 8 * u);
-    const float bl = p.bias ? p.bias[(size_t)min(qi - jc, p.nbias - 1) * heads + h] : 0.f;
-    bf16_t vv[64][VREG];
-#pragma unroll
-    for (int jj = 0; jj < 64; ++jj) {
-      const bf16_t* vr = vbase + (size_t)ab_key(span, min(j0 + jj, j_hi - 1)) * p.ldv + lane;
-#pragma unroll
-      for (int i = 0; i < VREG; ++i) vv[jj][i] = vr[64 * i];
-    }
+    auto slot_of = [&](int i) { return ab_key(span, min(j0 + i, j_hi - 1)); };
+    Chunk ch;
+    ch.load(kbase, p.ldk, vbase, p.ldv, lane, slot_of);
+    const int j = j0 + Chunk::key(lane);
+    const float bl = p.bias ? p.bias[(size_t)min(qi - slot_of(Chunk::key(lane)), p.nbias - 1) * heads + h] : 0.f;
     if (!staged) {
 #pragma unroll
       for (int i = 0; i < dim / 64; ++i) qs[lane + 64 * i] = qv[i];
       __syncthreads();
       staged = true;
-    }
-    float d0 = 0.f, d1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < DK8; ++u) {
-      float f[8];
-      unpack8(kf[u], f);
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        d0 = fmaf(qs[8 * u + i], f[i], d0);
-        d1 = fmaf(qs[8 * u + i + 1], f[i + 1], d1);
-      }
+      for (int e = 0; e < 8; ++e) q8[e] = qs[8 * (lane % DK8) + e];
     }
-    float sc = (d0 + d1) * p.scale * hs;
+    float sc = ch.score(q8, lane) * p.scale * hs;
     if (p.softcap > 0.f) sc = p.softcap * tanhf(sc / p.softcap);
     sc += bl;
     if (j >= j_hi) sc = -INFINITY;
@@ -371,21 +355,18 @@ __global__ void __launch_bounds__(64) attn_bias_decode_fast_kernel(AttnBias p) {
     l_run = l_run * corr + wave_sum(pr);
     m_run = m_new;
 #pragma unroll
-    for (int i = 0; i < VREG; ++i) acc[i] *= corr;
-#pragma unroll
-    for (int jj = 0; jj < 64; ++jj) {
-      const float pj = __shfl(pr, jj, 64);  // (0 for keys past the split)
-#pragma unroll
-      for (int i = 0; i < VREG; ++i) acc[i] = fmaf(pj, bf2f(vv[jj][i]), acc[i]);
-    }
+    for (int e = 0; e < 8; ++e) acc8[e] *= corr;
+    ch.add(acc8, pr, lane);  // (0 for keys past the split)
   }
+  float acc[VREG];
+  Chunk::columns(acc8, lane, acc);
   float* w = p.ws + (((size_t)b * heads + h) * p.splits + sp) * (vdim + 2);
   if (lane == 0) {
     w[0] = m_run;
     w[1] = l_run;
   }
 #pragma unroll
-  for (int i = 0; i < VREG; ++i) w[2 + lane + 64 * i] = acc[i];
+  for (int i = 0; i < VREG; ++i) w[2 + VREG * Chunk::vlane(lane) + i] = acc[i];
 }
 
 // decode over a shared latent: keys = values = ONE bf16 cache head (kc == vc, G == 1), rows of 136 to 512 numbers of
@@ -1108,7 +1089,7 @@ int hy_attn_bias(const AttnBias& p, hipStream_t s) {
     if (p.splits > 64) return -6;  // (the merge holds one split per lane)
     dim3 grid(p.splits, p.H * p.maps, p.B);
     if (p.cbf16 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.ldv == p.vdim && p.ldk % 8 == 0 &&
-        ((uintptr_t)p.kc & 15) == 0) {
+        (((uintptr_t)p.kc | (uintptr_t)p.vc) & 15) == 0) {
       if (p.dim == 64 && p.vdim == 64) attn_bias_decode_fast_kernel<8, 1><<<grid, 64, 0, s>>>(p);
       else if (p.dim == 64) attn_bias_decode_fast_kernel<8, 2><<<grid, 64, 0, s>>>(p);
       else if (p.vdim == 64) attn_bias_decode_fast_kernel<16, 1><<<grid, 64, 0, s>>>(p);

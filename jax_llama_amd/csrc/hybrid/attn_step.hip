@@ -8,9 +8,9 @@
 // takes them as one more key behind its own, and the first head of a key head writes them; the other splits deal the keys before
 // them, so nothing is read that this launch writes. A workgroup publishes its maximum, sum and values past the caches and takes its
 // head's ticket; the last one to arrive (nobody waits) merges them in split order and sets the ticket back.
-// What bounds it: two trips to memory (slot, then keys and values), the publication and the merge's trip. Values are read
-// two columns per lane: half the loads of the separate kernel. Tickets lie on lines of their own: counts on one line go one behind
+// What bounds it: two trips to memory (slot, then keys and values), the publication and the merge's trip. Tickets lie on lines of their own: counts on one line go one behind
 // the other (16 heads x 33 splits on two lines: 4 us).
+#include "attn_chunk.h"
 #include "attn_span.h"
 
 namespace jla {
@@ -132,31 +132,16 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   if (own) --span.n;  // (the token's own key comes from the projection)
   int j_lo, j_hi;
   ab_split_range(a, span, sp, j_lo, j_hi);
-  constexpr bool WIDE = sizeof(CT) == 4;
-  constexpr int KL = dim * sizeof(CT) / 16;
+  using Chunk = KeyChunk<CT, DK8, VREG>;
+  const int vlane = Chunk::vlane(lane);
   const CT* kbase = reinterpret_cast<const CT*>(a.kc) + ((size_t)b * a.G + g) * a.T * dim;
-  const CT* vbase = reinterpret_cast<const CT*>(a.vc) + ((size_t)b * a.G + g) * a.T * vdim + VREG * lane;
-  u32x4 kf[KL];
-  uint32_t vv[64][WIDE ? VREG : 1];
+  const CT* vbase = reinterpret_cast<const CT*>(a.vc) + ((size_t)b * a.G + g) * a.T * vdim;
+  Chunk ch;
   float bl = 0.f;
   auto fetch = [&](int j0) {
-    const int jc = ab_key(span, min(j0 + lane, j_hi - 1));
-#pragma unroll
-    for (int u = 0; u < KL; ++u) kf[u] = reinterpret_cast<const u32x4*>(kbase + (size_t)jc * dim)[u];
-    bl = a.bias ? a.bias[(size_t)min(qi - jc, a.nbias - 1) * a.H + h] : 0.f;
-#pragma unroll
-    for (int jj = 0; jj < 64; ++jj) {
-      const CT* vr = vbase + (size_t)ab_key(span, min(j0 + jj, j_hi - 1)) * vdim;
-      if constexpr (WIDE && VREG == 2) {
-        const u32x2 t = *reinterpret_cast<const u32x2*>(vr);
-        vv[jj][0] = t[0];
-        vv[jj][VREG - 1] = t[1];
-      } else if constexpr (WIDE || VREG == 2) {
-        vv[jj][0] = *reinterpret_cast<const uint32_t*>(vr);
-      } else {
-        vv[jj][0] = *reinterpret_cast<const bf16_t*>(vr);
-      }
-    }
+    auto slot_of = [&](int i) { return ab_key(span, min(j0 + i, j_hi - 1)); };
+    ch.load(kbase, dim, vbase, vdim, lane, slot_of);
+    bl = a.bias ? a.bias[(size_t)min(qi - slot_of(Chunk::key(lane)), a.nbias - 1) * a.H + h] : 0.f;
   };
   const bool any = j_lo < j_hi;
   if (any) fetch(j_lo);
@@ -206,49 +191,30 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   as_order();
   const bool sunk = a.sink && sp == 0;
   const float hs = a.head_scale ? a.head_scale[h] : 1.f;
-  float m_run = sunk ? a.sink[h] : -INFINITY, l_run = sunk ? 1.f : 0.f, acc[VREG];  // acc[i]: column VREG lane + i
+  float m_run = sunk ? a.sink[h] : -INFINITY, l_run = sunk ? 1.f : 0.f, acc[VREG];  // acc[i]: column VREG vlane + i
+  float q8[8], acc8[8];
 #pragma unroll
-  for (int i = 0; i < VREG; ++i) acc[i] = 0.f;
+  for (int e = 0; e < 8; ++e) {
+    q8[e] = qs[8 * (lane % DK8) + e];
+    acc8[e] = 0.f;
+  }
   for (int j0 = j_lo; j0 < j_hi; j0 += 64) {
     if (j0 != j_lo) fetch(j0);
-    float d0 = 0.f, d1 = 0.f;
-#pragma unroll
-    for (int u = 0; u < DK8; ++u) {
-      float f[8];
-      if constexpr (WIDE) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          f[i] = __uint_as_float(kf[2 * u][i]);
-          f[4 + i] = __uint_as_float(kf[2 * u + 1][i]);
-        }
-      } else {
-        unpack8(kf[u], f);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        d0 = fmaf(qs[8 * u + i], f[i], d0);
-        d1 = fmaf(qs[8 * u + i + 1], f[i + 1], d1);
-      }
-    }
-    float sc = (d0 + d1) * a.scale * hs;
+    float sc = ch.score(q8, lane) * a.scale * hs;
     if (a.softcap > 0.f) sc = a.softcap * tanhf(sc / a.softcap);
     sc += bl;
-    const bool in = j0 + lane < j_hi;
+    const bool in = j0 + Chunk::key(lane) < j_hi;
     if (!in) sc = -INFINITY;
     const float m_new = fmaxf(m_run, wave_max(sc));
     const float corr = expf(m_run - m_new);
-    const float pw = in ? expf(sc - m_new) : 0.f;
+    const float pw = in ? expf(sc - m_new) : 0.f;  // (0 past the split)
     l_run = l_run * corr + wave_sum(pw);
     m_run = m_new;
 #pragma unroll
-    for (int i = 0; i < VREG; ++i) acc[i] *= corr;
-#pragma unroll
-    for (int jj = 0; jj < 64; ++jj) {
-      const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pw), jj));  // (0 past the split)
-      acc[0] = fmaf(pj, __uint_as_float(WIDE ? vv[jj][0] : vv[jj][0] << 16), acc[0]);
-      if (VREG == 2) acc[VREG - 1] = fmaf(pj, __uint_as_float(WIDE ? vv[jj][WIDE ? VREG - 1 : 0] : vv[jj][0] & 0xffff0000u), acc[VREG - 1]);
-    }
+    for (int e = 0; e < 8; ++e) acc8[e] *= corr;
+    ch.add(acc8, pw, lane);
   }
+  Chunk::columns(acc8, lane, acc);
   if (own && tail) {  // the token's own key, as the cache holds it
     CT kb[ND], vb[VREG];
     float dot = 0.f;
@@ -280,7 +246,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
     m_run = m_new;
     as_order();
 #pragma unroll
-    for (int i = 0; i < VREG; ++i) acc[i] = fmaf(pw, row[VREG * lane + i], acc[i] * corr);
+    for (int i = 0; i < VREG; ++i) acc[i] = fmaf(pw, row[VREG * vlane + i], acc[i] * corr);
   }
   float o[VREG];
   if (WAVES > 1) {  // the workgroup's splits, joined by its first wave
@@ -289,7 +255,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
       join[wave][1] = l_run;
     }
 #pragma unroll
-    for (int i = 0; i < VREG; ++i) join[wave][2 + VREG * lane + i] = acc[i];
+    for (int i = 0; i < VREG; ++i) join[wave][2 + VREG * vlane + i] = acc[i];
     __syncthreads();
     if (wave) return;
     float m = m_run;
@@ -304,11 +270,12 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
       const float wt = join[w][1] > 0.f ? expf(join[w][0] - m) : 0.f;
       l_run = fmaf(join[w][1], wt, l_run);
 #pragma unroll
-      for (int i = 0; i < VREG; ++i) acc[i] = fmaf(join[w][2 + VREG * lane + i], wt, acc[i]);
+      for (int i = 0; i < VREG; ++i) acc[i] = fmaf(join[w][2 + VREG * vlane + i], wt, acc[i]);
     }
     m_run = m;
   }
   const int groups = (a.splits + WAVES - 1) / WAVES;
+  const int at_o = groups > 1 ? lane : vlane;  // o[i]: column VREG at_o + i
   if (groups > 1) {
     constexpr int pitch = vdim + 2;
     float* head = a.ws + ((size_t)b * a.H + h) * a.splits * pitch;
@@ -317,7 +284,7 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
       as_put(w, m_run);
       as_put(w + 1, l_run);
     }
-    as_put_row<VREG>(w + 2 + VREG * lane, acc);
+    as_put_row<VREG>(w + 2 + VREG * vlane, acc);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the split's numbers are out before its ticket is
     int32_t* ticket = p.tickets + ((size_t)b * a.H + h) * AS_TICKET;
     int before = 0;
@@ -335,11 +302,11 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   if (ROPE && p.turn) {  // the summed values turned back by the query's position
     as_order();
 #pragma unroll
-    for (int i = 0; i < VREG; ++i) row[VREG * lane + i] = o[i];
+    for (int i = 0; i < VREG; ++i) row[VREG * at_o + i] = o[i];
     as_order();
 #pragma unroll
     for (int i = 0; i < VREG; ++i) {
-      const int c = VREG * lane + i, half = p.v_half, f = c < half ? c : c - half;
+      const int c = VREG * at_o + i, half = p.v_half, f = c < half ? c : c - half;
       if (c < 2 * half) {
         const float s_ = p.turn_sign * sn[1][f], other = row[c < half ? c + half : f];
         o[i] = c < half ? o[i] * cs[1][f] - other * s_ : o[i] * cs[1][f] + other * s_;
@@ -349,18 +316,17 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   }
 #pragma unroll
   for (int i = 0; i < VREG; ++i) {
-    const size_t at = (size_t)b * a.ldo + (size_t)h * vdim + VREG * lane + i;
+    const size_t at = (size_t)b * a.ldo + (size_t)h * vdim + VREG * at_o + i;
     if (a.out_bf16) reinterpret_cast<bf16_t*>(a.out)[at] = f2bf(o[i]);
     else reinterpret_cast<float*>(a.out)[at] = o[i];
   }
 }
 
-// Heads of 64 or 128 numbers, up to about a wave per SIMD: more waves share a SIMD, and then the preparation in
-// each of them costs what the launches did. Us in turn, separate launches | here, heads of 128, rows x heads x splits: norms, 1 x 16
-// x 2 11.1 | 7.2, 3 x 16 x 17 16.0 | 11.8, 1 x 16 x 33 15.0 | 11.5, 2 x 16 x 33 18.2 | 17.1, 6 x 16 x 17 19.8 | 19.2, 13 x 16 x 9
-// 19.9 | 20.6, 8 x 32 x 8 34.4 | 38.7; rotations, 1 x 16 x 13 12.0 | 9.0, 2 x 32 x 16 14.1 | 11.0, 6 x 16 x 17 16.8 | 17.4, 4 x 32 x 16
-// 17.5 | 20.0.
-constexpr long long AS_MAX_WAVES = 1280;
+// Heads of 64 or 128 numbers, as far as the splits of a call go before its rows and heads alone fill the chip (hy_attn_decode_splits): a
+// decode step with two of these launches in the place of three or four each, us, separate | here, heads of 128, rows x heads x splits: norms, 2 x
+// 16 x 47 317 | 312, 3 x 16 x 33 384 | 378, 8 x 16 x 16 442 | 435, 8 x 32 x 5 1164 | 1146, 32 x 16 x 4 663 | 662; rotations, 8 x 16 x 16 274 | 268, 13 x 32 x 5
+// 708 | 695, 32 x 16 x 4 447 | 435, 128 x 16 x 1 721 | 707.
+constexpr long long AS_MAX_WAVES = 2560;
 constexpr int AS_PAIR_SPLITS = 16;  // more of them: two per workgroup (hy_attn_step)
 
 bool hy_attn_step_takes(const AttnStep& p) {
