@@ -106,7 +106,8 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   constexpr int H = G == 16 ? 2 : 1;         // MFMAs of a K step (G = 16: the two halves of a 128-byte line)
   constexpr int STEP = 32 * SEG * H;         // K of a step
   constexpr bool WIDE = sizeof(SUM) > sizeof(float);
-  constexpr int RUN = WIDE ? 4 / H : U;      // steps (four MFMAs) whose sums share an fp32 accumulator; SUM float: all of them do
+  // steps whose sums share an fp32 accumulator: up to four MFMAs, two where the batches were of two; SUM float: all of them
+  constexpr int RUN = !WIDE ? U : (G == 4 && NT == 2 && XB == 4 ? 2 : 4 / H);
   constexpr int ROWS = G * MT;               // rows of a pass
   using XNum = std::conditional_t<XB == 2, bf16_t, float>;
   __shared__ f32x4 red[WAVES][NT * MT][64];
@@ -1052,7 +1053,13 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   // tiles' one fp32 chain over all of K, 2.7e-7 at K 2048, here 1.3e-7 in one chain per wave: 33 rows of 4096 x 10304 60.5 us,
   // 64.5 in 64 bits)
   if (G == 4) {
+    // Two tiles: batches of four or three steps where they divide a wave's (a step past the end costs its loads), their sums added in 64 bits
+    // every two as in batches of two. Us, weights in no cache, two | three | four steps, one row: 10304 x 2048 10.3 | 13.0 | 9.9, 32000 x 2048 (two
+    // tiles) 23.3 | 31.7 | 22.8, 4096 x 4096 9.1 | 9.3 | 8.6, 4096 x 14336 23.0 | 23.2 | 22.6; four rows of 8 experts of 2048 x 2816 12.0 | 10.9 | 13.7.
+    const int mine = (p.K + 511) / 512;  // steps of a wave
     if (p.a_norm_w) RV_NT(4, 1, double);  // (at most two rows)
+    else if (nt == 2 && mine % 4 == 0) RV_RUN(4, 2, 1, 4, 0, double);
+    else if (nt == 2 && mine % 3 == 0) RV_RUN(4, 2, 1, 3, 0, double);
     else RV_NT(4, 0, double);
   } else if (G == 8) {
     RV_NT(8, 0, double);
