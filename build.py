@@ -76,7 +76,8 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-munsafe-f
              "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__"]
 # A source's own flags. delta_chunk: with a wave per SIMD the compiler puts the products' sums into the matrix unit's own registers, and
 # the 64 of a chunk that are added up pass through a move each (2048 tokens of 16 heads of 128 x 128, delta rule 210 -> 195 us, scalar gates 121 -> 111).
-FILE_FLAGS = {"delta_chunk": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# rows_mid, linear_mid: they are copied out of those registers and back at the loop's edge otherwise.
+FILE_FLAGS = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("delta_chunk", "rows_mid", "linear_mid")}
 
 
 def _scratch_users(remarks: str):

@@ -41,15 +41,6 @@ JLA_DEV int mid_row_tile(int m, int wn) {
   return SS ? (m + wn * MID_SQ<MT, WN>) % MT : m;
 }
 
-// The sums are pinned to the matrix unit's own registers: with one wave per SIMD, and registers to spare, the compiler copied them there
-// and back at the loop's edge. PAD: an operand comes from the vector unit, whose writes a product may read two states later (those from
-// LDS are waited for).
-template <bool PAD>
-JLA_DEV void mid_mfma(f32x4& acc, const u32x4& w, const u32x4& x) {
-  if constexpr (PAD) asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-}
-
 // acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 mid_row_tile(m) + c of the tile at weight columns 4 q .. + 3 of this wave's
 // 16-column tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64, a positive multiple of WK. xrow(r), wrow(r): the address of row r
 // of the tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py
@@ -90,10 +81,7 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-      asm volatile("" : "+a"(acc[t][m]));
-    }
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < (SS ? MID_SQ<MT, WN> : 1); ++m) ss[m] = 0.f;
   int xat[MT];  // where accumulator m's rows start in a slice (wave-uniform)
@@ -113,10 +101,13 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
       for (int i = 0; i < 2; ++i) x[i] = xs[h * H::BM * 8 + mid_cell(2 * q + i, c, 4)];
     }
   };
-  // the products of half a stage, with the reads of the next half (of slot, h) between them
+  // The products of half a stage, with the reads of the next half (of slot, h) between them, in this order. The products are the
+  // compiler's, which waits for their sums wherever it moves or reads them; build.py has their sums in the vector unit's registers, as it
+  // copied them out of the matrix unit's own and back at the loop's edge.
   auto half = [&](u32x4 (&w)[NT], u32x4 (&x)[MT][XR], u32x4 (&wnext)[NT], u32x4 (&xnext)[MT][XR], int slot, int h) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) read_w(wnext[t], slot, h, t);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       u32x4 f = x[m][0];
@@ -126,7 +117,7 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
         f = pack8(v);
       }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) mid_mfma<XB == 4>(acc[t][m], w[t], f);
+      for (int t = 0; t < NT; ++t) acc[t][m] = mfma16x16x32(w[t], f, acc[t][m]);
       if constexpr (SS) {
         if (m < MID_SQ<MT, WN>) {  // (plain FMAs: a dot product beside the products costs them more)
 #pragma unroll
@@ -138,6 +129,7 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
         }
       }
       read_x(xnext[m], slot, h, m);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   u32x4 w0[NT], w1[NT], x0[MT][XR], x1[MT][XR];
@@ -164,11 +156,6 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
     half(w1, x1, w0, x0, slot, 0);  // (behind the last stage: reads that nothing uses)
   }
   wait_vmcnt<0>();
-  asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // the last products, before their sums are read
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) asm volatile("" : "+a"(acc[t][m]));
   if constexpr (WK > 1) {  // the K groups' sums
     f32x4* red = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
