@@ -25,8 +25,8 @@ JLA_DEV void rm_store(const RowLinear& p, int d, int col, f32x4 v) {
 
 // grid: tiles x splits, rounded up to 8; slabs (several splits): [splits][R][weight rows] partial sums instead of the output.
 // gated: the 16-column tiles of a wave are gate and up tiles in turn (NT even).
-template <int MT, int NT, int WN, int WK, int S, int XB>
-__global__ void __launch_bounds__(64 * WN * WK, 2) rows_mid_kernel(RowLinear p, int gated, int tiles_n, int splits, int steps, float* slabs) {
+template <int MT, int NT, int WN, int WK, int S, int XB, bool WIDE>
+__global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, XB>::PER_SIMD)) rows_mid_kernel(RowLinear p, int gated, int tiles_n, int splits, int steps, float* slabs) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
   __shared__ u32x4 lds[H::LDS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) rows_mid_kernel(RowLinear p, 
   };
   f32x4 acc[NT][MT];
   float none[1];
-  mid_tile<MT, NT, WN, WK, S, XB, false, false>(lds, xrow, wrow, t0, t1, acc, none);
+  mid_tile<MT, NT, WN, WK, S, XB, false, false, WIDE>(lds, xrow, wrow, t0, t1, acc, none, p.offs ? 2 : 4);
   if (wave >= WN) return;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -76,12 +76,21 @@ __global__ void __launch_bounds__(256) rows_mid_sum_kernel(RowLinear p, const fl
   if (r >= p.R) return;
   const int col = 4 * (int)(i - r * n4), nw = gated ? 2 * p.N : p.N;
   const float* at = ws + r * nw + col;
-  f32x4 g = *reinterpret_cast<const f32x4*>(at), u = gated ? *reinterpret_cast<const f32x4*>(at + p.N) : f32x4{0.f, 0.f, 0.f, 0.f}, v;
-  for (int s = 1; s < splits; ++s) {
-    const float* more = at + (size_t)s * p.R * nw;
-    g += *reinterpret_cast<const f32x4*>(more);
-    if (gated) u += *reinterpret_cast<const f32x4*>(more + p.N);
-  }
+  auto sum = [&](const float* from) {  // in 64 bits, four loads in flight
+    double t[4] = {};
+    for (int s0 = 0; s0 < splits; s0 += 4) {
+      f32x4 f[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const f32x4*>(from + (size_t)min(s0 + j, splits - 1) * p.R * nw);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) t[x] += s0 + j < splits ? (double)f[j][x] : 0.;
+    }
+    return f32x4{(float)t[0], (float)t[1], (float)t[2], (float)t[3]};
+  };
+  const f32x4 g = sum(at), u = gated ? sum(at + p.N) : g;
+  f32x4 v;
 #pragma unroll
   for (int x = 0; x < 4; ++x) v[x] = lr_act(p, g[x], u[x]);
   rm_store(p, p.dst_idx ? p.dst_idx[r] : (int)r, col, v);
@@ -94,9 +103,22 @@ struct RmForm {
   float fill, stage, more, sum, mb;
   void (*run)(unsigned, hipStream_t, const RowLinear&, int, int, int, int, float*);
 };
+// Up to RM_WIDE_SUM_ROWS rows are summed in 64 bits (WIDE), rows by expert every four products as rows_gemv.hip sums them, dense rows, which
+// have one fp32 chain per wave there, every eight (every four: up to 3 % slower); more rows had one chain over K on the tiles of before,
+// too. Relative errors against 64 bits, one chain | wide: dense, K 2048 2.7e-7 | 8.9e-8, K 14336 3.7e-7 | 9.2e-8; by expert, K 7168 5.3e-7 | 6.5e-8
+// (rows_gemv.hip 1.3e-7 dense, 7.0e-8). Us, one chain -> wide, weights in no cache, 16 | 33 | 64 rows: 2048 x 2048 7.6 | 10.2 | 12.3 -> 7.7 | 10.7 | 12.5,
+// bf16 rows 6.4 | 7.4 | 7.9 -> 6.5 | 7.5 | 8.0; 4096 x 4096 13.1 | 15.5 | 16.5 -> 13.2 | 16.4 | 17.3; 4096 x 14336 29.1 | 29.8 | 32.5 -> 28.9 | 30.1 | 32.8; 64 rows of
+// 8 experts of 4096 x 7168 88 -> 91.
+constexpr int RM_WIDE_SUM_ROWS = 64;
 template <int MT, int NT, int WN, int WK, int S, int XB>
 static void rm_launch(unsigned grid, hipStream_t s, const RowLinear& p, int gated, int tiles_n, int splits, int steps, float* slabs) {
-  rows_mid_kernel<MT, NT, WN, WK, S, XB><<<grid, 64 * WN * WK, 0, s>>>(p, gated, tiles_n, splits, steps, slabs);
+  if constexpr (16 * MT <= RM_WIDE_SUM_ROWS) {
+    if (p.R <= RM_WIDE_SUM_ROWS) {
+      rows_mid_kernel<MT, NT, WN, WK, S, XB, true><<<grid, 64 * WN * WK, 0, s>>>(p, gated, tiles_n, splits, steps, slabs);
+      return;
+    }
+  }
+  rows_mid_kernel<MT, NT, WN, WK, S, XB, false><<<grid, 64 * WN * WK, 0, s>>>(p, gated, tiles_n, splits, steps, slabs);
 }
 #define RM_FORM(MT, NT, WN, WK, S, XB, ...) {MT, NT, WN, WK, XB, __VA_ARGS__, rm_launch<MT, NT, WN, WK, S, XB>}
 static const RmForm RM_FORMS[] = {
@@ -135,7 +157,7 @@ static RmPlan rm_plan(const RowLinear& p) {
   const float stream = (float)E * (float)nw * (float)p.K * 2 / 5.4e6f;  // the weights themselves
   RmPlan best;
   for (const RmForm& f : RM_FORMS) {
-    if (f.xb != xb || (gated && f.nt % 2) || T % f.wk) continue;
+    if (f.xb != xb || (gated && f.nt % 2) || T % f.wk || (p.R <= RM_WIDE_SUM_ROWS && 16 * f.mt > RM_WIDE_SUM_ROWS)) continue;
     const long long tiles = rm_row_tiles(p, 16 * f.mt) * ((nw + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
     int last = 0;
     for (int want = 1; want <= RM_MAX_SPLITS && want <= T; ++want) {

@@ -28,7 +28,7 @@ struct LinearMid {
 
 // SS: the norm's statistic is wanted
 template <int MT, int NT, int WN, int WK, int S, bool SS>
-__global__ void __launch_bounds__(64 * WN * WK, 2) linear_mid_kernel(LinearMid p) {
+__global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, 2>::PER_SIMD)) linear_mid_kernel(LinearMid p) {
   using H = MidShape<MT, NT, WN, WK, S, 2>;
   constexpr int LD = H::BN + 4;  // floats of a row of the staged sums: the 16 rows of a store on different banks
   static_assert(H::BM * LD / 4 <= H::LDS, "the sums reuse the ring");
@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(64 * WN * WK, 2) linear_mid_kernel(LinearMid p
   auto wrow = [&](int r) { return reinterpret_cast<const char*>(p.w + (size_t)min((n0 + r) >> 4, (N >> 4) - 1) * 16 * K); };
   float ss[SS ? MID_SQ<MT, WN> : 1];
   f32x4 acc[NT][MT];
-  mid_tile<MT, NT, WN, WK, S, 2, true, SS>(lds, xrow, wrow, t0, t1, acc, ss);
+  mid_tile<MT, NT, WN, WK, S, 2, true, SS, false>(lds, xrow, wrow, t0, t1, acc, ss);
   if constexpr (SS) {
 #pragma unroll
     for (int m = 0; m < MID_SQ<MT, WN>; ++m) {

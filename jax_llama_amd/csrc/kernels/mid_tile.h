@@ -22,8 +22,10 @@ struct MidShape {
   static constexpr int SLICE = (XP + WP) * 64, SLOT = SLICE * WK;                     // u32x4
   static constexpr int LDS = SLOT * S;
   static_assert(S >= 3 && LDS * 16 <= 160 * 1024, "ring");
-  static_assert(WK * NT * MT * WN / 2 * 64 <= LDS, "the waves' sums reuse the ring");
+  // waves per SIMD that a compute unit's LDS has room for, two at most
+  static constexpr int PER_SIMD = WAVES >= 8 || LDS * 16 * 2 <= 160 * 1024 ? 2 : 1;
 };
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // 16-byte cell of chunk x of row r in its 128-byte line of LDS: the 16 lanes that a fragment read serves at a time (rows 0-3 and 12-15
 // of one quarter, 4-11 of the next) fall on all 64 banks; fp32 rows, whose quarter is two chunks, need another order for that
@@ -44,11 +46,13 @@ JLA_DEV int mid_row_tile(int m, int wn) {
 // acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 mid_row_tile(m) + c of the tile at weight columns 4 q .. + 3 of this wave's
 // 16-column tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64, a positive multiple of WK. xrow(r), wrow(r): the address of row r
 // of the tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py
-// pack_frag16x32). SS (bf16 rows): ss[m] is this lane's share of the squares of row 16 mid_row_tile(m) + c, over quarters q and K groups
+// pack_frag16x32). WIDE: the sums of every `run` steps (a power of two; two products each) are added in
+// 64 bits, the K groups' too. SS (bf16 rows): ss[m] is this lane's share of the squares of row 16 mid_row_tile(m) + c, over quarters q and K groups
 // (the row tiles beyond MT, counted from wn MID_SQ on, are another wave's). The waves deal the row tiles, without a branch, which would
 // keep a stage's reads and products apart.
-template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, bool SS, class XRow, class WRow>
-JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], float (&ss)[SS ? MID_SQ<MT, WN> : 1]) {
+template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, bool SS, bool WIDE, class XRow, class WRow>
+JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], float (&ss)[SS ? MID_SQ<MT, WN> : 1],
+                      int run = 0) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, q = lane >> 4;
   const int wn = wave % WN, wk = wave / WN, ns = (t1 - t0) / WK;
@@ -84,6 +88,18 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
     for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < (SS ? MID_SQ<MT, WN> : 1); ++m) ss[m] = 0.f;
+  f64x4 tot[WIDE ? NT : 1][WIDE ? MT : 1];
+  auto widen = [&](bool first) {
+#pragma unroll
+    for (int t = 0; t < (WIDE ? NT : 0); ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tot[t][m][i] = first ? 0. : tot[t][m][i] + (double)acc[t][m][i];
+        acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  widen(true);
   int xat[MT];  // where accumulator m's rows start in a slice (wave-uniform)
 #pragma unroll
   for (int m = 0; m < MT; ++m) xat[m] = 128 * mid_row_tile<MT, WN, SS>(m, wn);
@@ -154,10 +170,14 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
     slot = slot + 1 == S ? 0 : slot + 1;
     fill = fill + 1 == S ? 0 : fill + 1;
     half(w1, x1, w0, x0, slot, 0);  // (behind the last stage: reads that nothing uses)
+    if (WIDE && !((st + 1) & (run - 1))) widen(false);
   }
   wait_vmcnt<0>();
-  if constexpr (WK > 1) {  // the K groups' sums
-    f32x4* red = reinterpret_cast<f32x4*>(lds);
+  widen(false);
+  auto join = [&](auto& sum) {  // the K groups' sums
+    using Sum = std::remove_reference_t<decltype(sum[0][0])>;
+    static_assert(WK == 1 || WK * NT * MT * WN / 2 * 64 * (int)sizeof(Sum) <= H::LDS * 16, "they reuse the ring");
+    Sum* red = reinterpret_cast<Sum*>(lds);
 #pragma unroll
     for (int half = WK / 2; half > 0; half /= 2) {
       __syncthreads();
@@ -165,16 +185,27 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) red[((((wk - half) * WN + wn) * NT + t) * MT + m) * 64 + lane] = acc[t][m];
+          for (int m = 0; m < MT; ++m) red[((((wk - half) * WN + wn) * NT + t) * MT + m) * 64 + lane] = sum[t][m];
       }
       __syncthreads();
       if (wk < half) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) acc[t][m] += red[(((wk * WN + wn) * NT + t) * MT + m) * 64 + lane];
+          for (int m = 0; m < MT; ++m) sum[t][m] += red[(((wk * WN + wn) * NT + t) * MT + m) * 64 + lane];
       }
     }
+  };
+  if constexpr (WIDE) {
+    join(tot);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][m][i] = (float)tot[t][m][i];
+  } else {
+    join(acc);
   }
 }
 
