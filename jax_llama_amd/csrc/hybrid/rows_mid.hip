@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(256) rows_mid_sum_kernel(RowLinear p, const fl
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   const int n4 = p.N / 4;
   const long long r = i / n4;
-  if (r >= p.R) return;
+  if (r >= p.R || (p.offs && r >= p.offs[p.E])) return;  // (rows of experts without weights: nothing wrote their sums)
   const int col = 4 * (int)(i - r * n4), nw = gated ? 2 * p.N : p.N;
   const float* at = ws + r * nw + col;
   auto sum = [&](const float* from) {  // in 64 bits, four loads in flight

@@ -116,6 +116,23 @@ def test_rows_by_expert(counts, n, k, rows):
         assert _err(out, want) < (2.0 ** -8 if odt == BF16 else 16 * _tol(k))
 
 
+@pytest.mark.parametrize("rows", ["f32", "bf16"])
+@pytest.mark.parametrize("act", [hy.ACT_NONE, hy.ACT_SWIGLU])
+def test_rows_of_experts_without_weights_are_left_alone(rows, act):
+    """Rows behind the last offset (identity experts) keep what the output holds, with a K split as without one."""
+    for n, k in ((64, 4096), (64, 128), (4096, 1024)):
+        g = torch.Generator(device=DEV).manual_seed(k)
+        x = torch.randn(100, k, generator=g, device=DEV).to(BF16)
+        w = (torch.randn(2, 2 * n if hy.act_gated(act) else n, k, generator=g, device=DEV) * k ** -0.5).to(BF16)
+        offs = torch.tensor([0, 30, 77], dtype=torch.int32, device=DEV)
+        dst = torch.randperm(100, generator=g, device=DEV).to(torch.int32)
+        out = torch.full((100, n), 7.0, device=DEV)
+        hy.ext().linear_rows(x if rows == "bf16" else x.float(), None, w, out, dst, offs, None, 100, act, 0.0, 1.0, None, None, 0.0)
+        assert (out[dst[77:].long()] == 7.0).all(), (n, k)
+        for lo, hi, i in ((0, 30, 0), (30, 77, 1)):
+            assert _err(out[dst[lo:hi].long()], _act64(x[lo:hi].double() @ w[i].double().t(), act, 0, 1)) < 16 * _tol(k)
+
+
 def test_a_row_that_is_no_number_stays_in_its_row_and_replays_repeat():
     m, n, k = 70, 132, 2048
     x, w = _operands(m, n, k, 3)
