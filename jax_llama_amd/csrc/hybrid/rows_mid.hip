@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, XB>
   };
   f32x4 acc[NT][MT];
   float none[1];
-  mid_tile<MT, NT, WN, WK, S, XB, false, false, WIDE>(lds, xrow, wrow, t0, t1, acc, none, p.offs ? 2 : 4);
+  mid_tile<MT, NT, WN, WK, S, XB, false, false, std::conditional_t<WIDE, f64x4, void>>(lds, xrow, wrow, t0, t1, acc, none, p.offs ? 2 : 4);
   if (wave >= WN) return;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {

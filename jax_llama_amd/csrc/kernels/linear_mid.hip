@@ -1,4 +1,4 @@
-// 17 to some 300 rows on packed bf16 weights: y [M, N] = epilogue([inv_rms(x) *] x [M, K] @ W^T), the decode step of a mid-sized
+// 17 to 256 rows on packed bf16 weights: y [M, N] = epilogue([inv_rms(x) *] x [M, K] @ W^T), the decode step of a mid-sized
 // batch and short prompts (reference ops: the projections of jax_llama/model.py:210, :294, :338 and the head, :736, with the norm
 // before them, :384, :395, :662). mid_tile.h says what bounds it and why the tile is as it is; here are its forms and the choice among them.
 //
@@ -26,6 +26,15 @@ struct LinearMid {
   QKVArgs qa;
 };
 
+// What was here before, GEMVs that deal K to their waves and tiles that split it over workgroups, has fp32 chains of an eighth to a half of K. One chain
+// over a workgroup's steps would be longer, so every LM_RUN steps (eight products) of it are added in 64 bits, or in 32 where a wave's sums would
+// not fit its registers twice. Relative errors against 64 bits, before | one chain | now, 64 and 128 rows: 6144 x 4096 1.9e-7 | 1.9e-7 | 9.3e-8, 1.3e-7 |
+// 2.7e-7 | 8.9e-8; 28672 x 4096 1.9e-7 | 3.9e-7 | 8.9e-8, 2.7e-7 | 3.9e-7 | 1.2e-7 (32 bits); 4096 x 14336 1.9e-7 | 3.7e-7 | 9.8e-8, 1.9e-7 | 2.6e-7 | 1.2e-7. Us, one
+// chain -> now: 19.9 -> 20.8, 23.1 -> 23.5; 49.4 -> 49.3, 51.3 -> 54.2; 29.5 -> 29.9, 33.6 -> 33.9.
+constexpr int LM_RUN = 4;
+template <int MT, int NT>
+using LmSum = std::conditional_t<MT * NT <= 8, f64x4, f32x4>;
+
 // SS: the norm's statistic is wanted
 template <int MT, int NT, int WN, int WK, int S, bool SS>
 __global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, 2>::PER_SIMD)) linear_mid_kernel(LinearMid p) {
@@ -43,7 +52,7 @@ __global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, 2>:
   auto wrow = [&](int r) { return reinterpret_cast<const char*>(p.w + (size_t)min((n0 + r) >> 4, (N >> 4) - 1) * 16 * K); };
   float ss[SS ? MID_SQ<MT, WN> : 1];
   f32x4 acc[NT][MT];
-  mid_tile<MT, NT, WN, WK, S, 2, true, SS, false>(lds, xrow, wrow, t0, t1, acc, ss);
+  mid_tile<MT, NT, WN, WK, S, 2, true, SS, LmSum<MT, NT>>(lds, xrow, wrow, t0, t1, acc, ss, LM_RUN);
   if constexpr (SS) {
 #pragma unroll
     for (int m = 0; m < MID_SQ<MT, WN>; ++m) {
@@ -142,8 +151,8 @@ bool linear_mid_tile(int tile) { return tile >= LINEAR_MID_TILE && tile < LINEAR
 // measured (11 matrices from 256 x 512 to 128256 x 4096, 17 to 256 rows, the epilogues that follow them). Against what ran before, the
 // tiles of 128 and 256 rows with their splits and the GEMVs (us here | there, weights in no cache, rows 48 to 128; 17 to 32 within 5 % either
 // way, so these stay a measured choice, as do 129 to LINEAR_MID_MAX_M, where narrow outputs gain and wide ones lose):
-//   6144 x 4096, 64 | 128 rows 19.3 | 24.2, 22.8 | 28.9;  4096 x 4096 residual 14.4 | 19.9, 17.9 | 24.2;
-//   28672 x 4096 gated 45.3 | 56.0, 53.8 | 62.6;  4096 x 14336 residual 28.4 | 34.7, 34.1 | 39.5.
+//   6144 x 4096, 64 | 128 rows 20.8 | 24.8, 23.5 | 26.6;  4096 x 4096 14.7 | 20.8, 18.5 | 23.1;
+//   28672 x 4096 49.3 | 62.7, 54.2 | 67.8;  4096 x 14336 29.9 | 34.4, 33.9 | 39.1.
 // A head's N from 100 rows on is better off in tiles of more columns: 128256 x 4096, 100 | 128 rows 228 | 217, 238 | 227 (64: 196 | 205).
 constexpr int LM_WIDE_M = 96, LM_WIDE_N = 65536;
 int linear_mid_plan(int M, int N, int K, int* ksplit) {
@@ -176,7 +185,7 @@ int linear_mid_plan(int M, int N, int K, int* ksplit) {
   return tile;
 }
 
-// The product's launch (of splits > 1, or slabs for another reason: the partial sums' one): K in `ksplit` runs, as linear_mid_splits says
+// The product's launch (of splits > 1, or slabs for another reason: the partial sums' one): K in `ksplit` runs, as linear_mid_plan cuts it
 int linear_mid(const bf16_t* x, const void* W, void* out, int M, int N, int K, int mode, int accumulate, int out_f32, bf16_t* mirror,
                const QKVArgs* qkv, float* slabs, float* ssq, int ksplit, float rms_eps, int tile, hipStream_t s) {
   if (!linear_mid_tile(tile) || (N & 15) || (K & 63) || K < 64 || M <= 0 || ksplit < 1) return -1;

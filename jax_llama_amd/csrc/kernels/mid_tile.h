@@ -46,11 +46,12 @@ JLA_DEV int mid_row_tile(int m, int wn) {
 // acc[t][m]: lane (c = lane & 15, q = lane >> 4) holds row 16 mid_row_tile(m) + c of the tile at weight columns 4 q .. + 3 of this wave's
 // 16-column tile t; after the call in the waves of K group 0 only. Steps [t0, t1) of 64, a positive multiple of WK. xrow(r), wrow(r): the address of row r
 // of the tile (BM, BN of them) at K 0; PACKED: wrow(16 j) is where 16-column tile j's fragments start (ops/reference.py
-// pack_frag16x32). WIDE: the sums of every `run` steps (a power of two; two products each) are added in
-// 64 bits, the K groups' too. SS (bf16 rows): ss[m] is this lane's share of the squares of row 16 mid_row_tile(m) + c, over quarters q and K groups
+// pack_frag16x32). Tot: the type in which the sums of every `run` steps (a power of two;
+// two products each) are added, f64x4 or f32x4, and the K groups' (the squares
+// in 64 bits); void: one fp32 chain over all steps. SS (bf16 rows): ss[m] is this lane's share of the squares of row 16 mid_row_tile(m) + c, over quarters q and K groups
 // (the row tiles beyond MT, counted from wn MID_SQ on, are another wave's). The waves deal the row tiles, without a branch, which would
 // keep a stage's reads and products apart.
-template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, bool SS, bool WIDE, class XRow, class WRow>
+template <int MT, int NT, int WN, int WK, int S, int XB, bool PACKED, bool SS, class Tot, class XRow, class WRow>
 JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&acc)[NT][MT], float (&ss)[SS ? MID_SQ<MT, WN> : 1],
                       int run = 0) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
@@ -88,18 +89,25 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
     for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < (SS ? MID_SQ<MT, WN> : 1); ++m) ss[m] = 0.f;
-  f64x4 tot[WIDE ? NT : 1][WIDE ? MT : 1];
-  auto widen = [&](bool first) {
+  constexpr bool RUNS = !std::is_void_v<Tot>;
+  using Sum = std::conditional_t<RUNS, Tot, f32x4>;
+  Sum tot[RUNS ? NT : 1][RUNS ? MT : 1];
+  double sq[RUNS && SS ? MID_SQ<MT, WN> : 1];
+  auto end_run = [&](bool first) {
 #pragma unroll
-    for (int t = 0; t < (WIDE ? NT : 0); ++t)
+    for (int t = 0; t < (RUNS ? NT : 0); ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) tot[t][m][i] = first ? 0. : tot[t][m][i] + (double)acc[t][m][i];
+        tot[t][m] = first ? Sum{0, 0, 0, 0} : tot[t][m] + __builtin_convertvector(acc[t][m], Sum);
         acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
+#pragma unroll
+    for (int m = 0; m < (RUNS && SS ? MID_SQ<MT, WN> : 0); ++m) {
+      sq[m] = first ? 0. : sq[m] + (double)ss[m];
+      ss[m] = 0.f;
+    }
   };
-  widen(true);
+  end_run(true);
   int xat[MT];  // where accumulator m's rows start in a slice (wave-uniform)
 #pragma unroll
   for (int m = 0; m < MT; ++m) xat[m] = 128 * mid_row_tile<MT, WN, SS>(m, wn);
@@ -170,12 +178,11 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
     slot = slot + 1 == S ? 0 : slot + 1;
     fill = fill + 1 == S ? 0 : fill + 1;
     half(w1, x1, w0, x0, slot, 0);  // (behind the last stage: reads that nothing uses)
-    if (WIDE && !((st + 1) & (run - 1))) widen(false);
+    if (RUNS && !((st + 1) & (run - 1))) end_run(false);
   }
   wait_vmcnt<0>();
-  widen(false);
-  auto join = [&](auto& sum) {  // the K groups' sums
-    using Sum = std::remove_reference_t<decltype(sum[0][0])>;
+  end_run(false);
+  auto join = [&](Sum (&sum)[NT][MT]) {  // the K groups' sums
     static_assert(WK == 1 || WK * NT * MT * WN / 2 * 64 * (int)sizeof(Sum) <= H::LDS * 16, "they reuse the ring");
     Sum* red = reinterpret_cast<Sum*>(lds);
 #pragma unroll
@@ -196,14 +203,14 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
       }
     }
   };
-  if constexpr (WIDE) {
+  if constexpr (RUNS) {
     join(tot);
+#pragma unroll
+    for (int m = 0; m < (SS ? MID_SQ<MT, WN> : 0); ++m) ss[m] = (float)sq[m];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][m][i] = (float)tot[t][m][i];
+      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_convertvector(tot[t][m], f32x4);
   } else {
     join(acc);
   }
