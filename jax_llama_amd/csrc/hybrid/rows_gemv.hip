@@ -106,8 +106,8 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   constexpr int H = G == 16 ? 2 : 1;         // MFMAs of a K step (G = 16: the two halves of a 128-byte line)
   constexpr int STEP = 32 * SEG * H;         // K of a step
   constexpr bool WIDE = sizeof(SUM) > sizeof(float);
-  // steps whose sums share an fp32 accumulator: up to four MFMAs, two where the batches were of two; SUM float: all of them
-  constexpr int RUN = !WIDE ? U : (G == 4 && NT == 2 && XB == 4 ? 2 : 4 / H);
+  // steps whose sums share an fp32 accumulator: up to four MFMAs, two of four rows and several tiles; SUM float: all of them
+  constexpr int RUN = !WIDE ? U : (G == 4 && NT > 1 ? 2 : 4 / H);
   constexpr int ROWS = G * MT;               // rows of a pass
   using XNum = std::conditional_t<XB == 2, bf16_t, float>;
   __shared__ f32x4 red[WAVES][NT * MT][64];
