@@ -114,6 +114,29 @@ def _compile_hip(src: Path, obj: Path, headers, force: bool, extra=()):
     return False
 
 
+# What the compiler does not know about inline asm is checked in the assembly: the hand-counted load rings must not be read before their
+# waits (attn_decode: the v4 ring), nor the sums of matrix products before they are there.
+ASM_CHECKS = {"gemv": ("check_asm_ring", "check_mfma_waits"), "attn_decode": ("check_asm_ring",),
+              "attn_decode_mma": ("check_asm_ring", "check_mfma_waits"), "gemm": ("check_mfma_waits",), "rows_gemm": ("check_mfma_waits",)}
+
+
+def _check_asm(built, odir: Path, jobs: int, extra=()):
+    """The checks above of every (source, object, whether it was compiled just now); an object that fails one does not survive it: it
+    would look up to date to the next build."""
+    def check(src, obj):
+        asm = odir / (src.stem + ".s")
+        _run([HIPCC, *HIP_FLAGS, *FILE_FLAGS.get(src.stem, []), *extra, "--cuda-device-only", "-S", str(src), "-o", str(asm)])
+        try:
+            for tool in ASM_CHECKS[src.stem]:
+                _run([sys.executable, str(ROOT / "tools" / f"{tool}.py"), str(asm)])
+        except SystemExit:
+            obj.unlink(missing_ok=True)
+            raise
+    with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        for f in [ex.submit(check, src, obj) for src, obj, did in built if did and src.stem in ASM_CHECKS]:
+            f.result()
+
+
 def build_C(jobs: int, force: bool, debug_bounds: bool = False) -> Path:
     tdir, tinc, tlib = _torch_paths()
     kdir = CSRC / "kernels"
@@ -125,17 +148,7 @@ def build_C(jobs: int, force: bool, debug_bounds: bool = False) -> Path:
     objs = [odir / (s.stem + ".o") for s in srcs]
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         rebuilt = list(ex.map(lambda so: _compile_hip(so[0], so[1], headers, force, extra), zip(srcs, objs)))
-    # the hand-counted load rings must never be read before their waits: check the assembly
-    for src, did in zip(srcs, rebuilt):
-        if did and src.stem in ("gemv", "attn_decode", "attn_decode_mma"):  # (attn_decode: the v4 ring)
-            asm = odir / (src.stem + ".s")
-            _run([HIPCC, *HIP_FLAGS, *extra, "--cuda-device-only", "-S", str(src), "-o", str(asm)])
-            try:
-                _run([sys.executable, str(ROOT / "tools" / "check_asm_ring.py"), str(asm)])
-            except SystemExit:
-                # the object must not survive a failed check: it would look up to date to the next build
-                (odir / (src.stem + ".o")).unlink(missing_ok=True)
-                raise
+    _check_asm(zip(srcs, objs, rebuilt), odir, jobs, extra)
     bsrc = CSRC / "bindings.cpp"
     bobj = odir / "bindings.o"
     if force or _stale(bobj, [bsrc, *headers]):
@@ -183,9 +196,10 @@ def build_hybrid(jobs: int, force: bool) -> Path:
     bobj = odir / "bindings.o"
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         futs = [ex.submit(_compile_hip, s, o, headers, force) for s, o in zip(srcs, objs)]
-        futs.append(ex.submit(_compile_bindings, hdir / "bindings.cpp", bobj, headers, "_C_hybrid", force))
-        for f in futs:
-            f.result()
+        bind = ex.submit(_compile_bindings, hdir / "bindings.cpp", bobj, headers, "_C_hybrid", force)
+        rebuilt = [f.result() for f in futs]
+        bind.result()
+    _check_asm(zip(srcs, objs, rebuilt), odir, jobs)
     out = PKG / f"_C_hybrid{EXT_SUFFIX}"
     _link(out, [*objs, bobj], force)
     return out

@@ -36,9 +36,15 @@ constexpr int G4_SLOT_U4 = G4_A_U4 + G4_B_U4;    // 64 KiB
 // loop-carried accumulators between the two register files and shuffles them with v_accvgpr moves around every
 // MFMA. Volatile, so the MFMAs keep their program order relative to the DMA issues and fragment reads placed between
 // them. Hazards: the A / B fragments come from ds_reads (counted by hipcc: the asm names them as inputs), each
-// accumulator is read by one MFMA per 64, and g4_acc_fence() pads the MFMA -> v_accvgpr_read hand-off after the loop.
+// accumulator is read by one MFMA per 64, and g4_acc_fence() pads the MFMA -> v_accvgpr_read hand-off after the loop. That holds
+// for as long as the compiler copies no accumulator in front of the fence, which build.py checks in the assembly
+// (tools/check_mfma_waits.py); where it does, at the edges of the loop's phases, their last MFMA is g4_mfma_wait.
 JLA_DEV void g4_mfma(f32x4& acc, const u32x4& a, const u32x4& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// ... with the wait states behind it after which its sum may be read, in the one statement that the compiler cannot get into
+JLA_DEV void g4_mfma_wait(f32x4& acc, const u32x4& a, const u32x4& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 7\n\ts_nop 7" : "+a"(acc) : "v"(a), "v"(b));
 }
 // an accumulator tile for the epilogue, read out of its AGPRs at this point in program order
 JLA_DEV f32x4 g4_take(f32x4& a) {
@@ -126,6 +132,8 @@ JLA_DEV void g4_mainloop(const G4Args& g, u32x4* lds, int m0, int n0, int t0, in
         const int e = 4 * q + u, j = e >> 3, i = e & 7;
         if constexpr (DIAG & 1)
           asm volatile("" ::"v"(wf[j]), "v"(xf[i]));
+        else if (RMS && W3 && rh == 0 && e == 63)  // (the second half of a K-tile, whose end may be a phase's; 16 of some 2200 cycles)
+          g4_mfma_wait(acc[j][i], wf[j], xf[i]);
         else
           g4_mfma(acc[j][i], wf[j], xf[i]);
       }

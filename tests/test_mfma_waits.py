@@ -46,3 +46,26 @@ def test_mid_sized_products(src, tmp_path):
                     path, "-o", str(out)], check=True, capture_output=True)
     text = out.read_text()
     assert text.count("v_mfma") > 100 and not waits.check(text)
+
+
+def test_the_build_checks_every_source_with_products_in_asm():
+    """Also through the headers that it includes."""
+    import re
+    csrc = os.path.join(ROOT, "jax_llama_amd", "csrc")
+
+    def text_of(path, seen):
+        seen.add(path)
+        text = open(path).read()
+        for name in re.findall(r'#include "([^"]+)"', text):
+            at = os.path.normpath(os.path.join(os.path.dirname(path), name))
+            if at not in seen and os.path.exists(at):
+                text += text_of(at, seen)
+        return text
+
+    listed = _load("repo_build", "build.py").ASM_CHECKS
+    found = set()
+    for part in ("kernels", "hybrid"):
+        for name in sorted(os.listdir(os.path.join(csrc, part))):
+            if name.endswith(".hip") and re.search(r'asm volatile\([^;]*v_mfma', text_of(os.path.join(csrc, part, name), set())):
+                found.add(name[:-4])
+    assert found and found <= {src for src, tools in listed.items() if "check_mfma_waits" in tools}
