@@ -101,15 +101,18 @@ SCRATCH_OK: dict = {}
 
 
 def _compile_hip(src: Path, obj: Path, headers, force: bool, extra=()):
-    if force or _stale(obj, [src, *headers]):
+    cmd = [HIPCC, *HIP_FLAGS, *FILE_FLAGS.get(src.stem, []), *extra, "-Rpass-analysis=kernel-resource-usage", "-c", str(src), "-o", str(obj)]
+    made_by = obj.with_suffix(".cmd")  # (other flags: another object)
+    if force or _stale(obj, [src, *headers]) or not made_by.exists() or made_by.read_text() != "\n".join(cmd):
         obj.parent.mkdir(parents=True, exist_ok=True)
-        out = _run([HIPCC, *HIP_FLAGS, *FILE_FLAGS.get(src.stem, []), *extra, "-Rpass-analysis=kernel-resource-usage", "-c", str(src), "-o",
-                    str(obj)])
+        obj.unlink(missing_ok=True)
+        out = _run(cmd)
         bad = [(n, b) for n, b in _scratch_users(out) if not any(ok in n and b <= lim for ok, lim in SCRATCH_OK.items())]
         if bad:
             obj.unlink(missing_ok=True)
             raise SystemExit(f"{src.name}: kernels use scratch memory (runtime-indexed register array or spill): "
                              + ", ".join(f"{n} ({b} B/lane)" for n, b in bad))
+        made_by.write_text("\n".join(cmd))
         return True
     return False
 
