@@ -968,8 +968,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_dbg for the bounds-chec
     const int tile = mm > 0x7fffffff ? 0 : jla::linear_mid_plan((int)mm, (int)n, (int)k, &ks);
     return std::make_pair(ks, tile);
   });
-  m.attr("LINEAR_MID_TILE") = jla::LINEAR_MID_TILE;
-  m.attr("LINEAR_MID_MAX_M") = jla::LINEAR_MID_MAX_M;
+  m.def("linear_mid_tiles", []() {  // its tile configs
+    std::vector<int> tiles;
+    for (int t = jla::LINEAR_MID_TILE; jla::linear_mid_tile(t); ++t) tiles.push_back(t);
+    return tiles;
+  });
   m.def("gemm5_ksplit", [](int64_t k, int64_t ks) { return jla::gemm5_ksplit((int)k, (int)ks); });
   m.def("attn_set_v6", [](int64_t mode) { jla::attn_set_v6((int)mode); });
   m.def("attn_set_v6_wpp", [](int64_t wpp) { jla::attn_set_v6_wpp((int)wpp); });

@@ -304,7 +304,7 @@ KS_CANDIDATES = (1, 2, 3, 4, 6, 8, 12, 16)
 # 32 to 38: the tiles of mid-sized batches (csrc/kernels/linear_mid.hip), the one of them and the split that its model picks. They win on
 #   narrow outputs (M = 200: 8192 x 1024 20.4 -> 13.1 us, 4096 x 4096 residual 23.9 -> 20.8, 1280 x 8192 24.2 -> 19.5) and lose on wide ones
 #   (28672 x 4096 gated 65 -> 79).
-MID_TILES = tuple(range(32, 39))
+MID_TILES = tuple(range(32, 39))  # (csrc: LINEAR_MID_TILE and its forms)
 TILE_CANDIDATES = (1, 2, 3, 7, 11, 12, 14, 16, 17, *MID_TILES)
 if os.environ.get("JLA_TUNE_TILES"):  # A/B tooling: restrict the tile candidates, e.g. JLA_TUNE_TILES=1,2,3,7,11,12
     TILE_CANDIDATES = tuple(int(v) for v in os.environ["JLA_TUNE_TILES"].split(","))
@@ -325,7 +325,8 @@ def choose_gemm_plan(e, m: int, n: int, k: int, device, mode: int = 0, rms: bool
         return plan
     if m <= 128:  # the tiles of mid-sized batches, by their model (linear_mid.hip has both sides' times)
         plan = e.linear_mid_plan(m, n, k)
-        if plan[1]:
+        if plan[1] in TILE_CANDIDATES:
+            _KS_CACHE[key] = plan
             return plan
     heur = e.gemm_ksplit(m, n, k)
     # tuned band: decode-sized M (prefill-sized M has enough 256x256 tiles; tuning it would also need

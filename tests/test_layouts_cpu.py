@@ -82,3 +82,28 @@ def test_packaged_tune_table_is_current():
             assert tile in autotune.TILE_CANDIDATES and ks >= 1, (key, v)
         else:
             assert kind == "gemv" and v in gemv_ok, (key, v)
+
+
+def test_mid_sized_tiles_are_those_of_the_extension_and_can_be_left_out(monkeypatch):
+    """The tuner's list of them is the extension's; a restricted candidate list (JLA_TUNE_TILES) holds for them too; and a plan is asked
+    for once per shape."""
+    from jax_llama_amd.ops import _ext, autotune
+    if _ext.available():
+        assert tuple(_ext.ext().linear_mid_tiles()) == autotune.MID_TILES
+
+    class Ext:
+        asked = 0
+
+        def linear_mid_plan(self, m, n, k):
+            self.asked += 1
+            return (2, 33)
+
+        def gemm_ksplit(self, m, n, k):
+            return 5
+
+    e, dev = Ext(), torch.device("cpu")
+    monkeypatch.setattr(autotune, "_KS_CACHE", {})
+    assert [autotune.choose_gemm_plan(e, 100, 512, 256, dev) for _ in range(3)] == [(2, 33)] * 3 and e.asked == 1
+    monkeypatch.setattr(autotune, "_KS_CACHE", {})
+    monkeypatch.setattr(autotune, "TILE_CANDIDATES", (1, 2, 3, 7))
+    assert autotune.choose_gemm_plan(e, 100, 512, 256, dev) == (5, 0)
