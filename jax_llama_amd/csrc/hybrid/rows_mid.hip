@@ -151,7 +151,7 @@ static long long rm_row_tiles(const RowLinear& p, int bm) {
 
 // The form and split with the least time by the figures above: on average 2.0 % above the best of all that were measured (384 shapes: one
 // matrix, 8 and 32 experts, N 64 to 32000, K 512 to 14336, 9 to 3200 rows)
-static RmPlan rm_plan(const RowLinear& p) {
+static RmPlan rm_best(const RowLinear& p) {
   const int gated = hy_act_gated(p.act), T = p.K >> 6, xb = p.a_bf16 ? 2 : 4, E = p.offs ? (p.E < p.R ? p.E : p.R) : 1;
   const long long nw = gated ? 2LL * p.N : p.N;
   const float stream = (float)E * (float)nw * (float)p.K * 2 / 5.4e6f;  // the weights themselves
@@ -173,6 +173,19 @@ static RmPlan rm_plan(const RowLinear& p) {
     }
   }
   return best;
+}
+
+// ... of the shapes that this thread has had last (the choice takes 1.1 us of host time, and a product asks for it twice)
+static RmPlan rm_plan(const RowLinear& p) {
+  struct Kept {
+    int R, N, K, E, how;
+    RmPlan plan;
+  };
+  thread_local Kept kept[64];
+  const int how = 1 + p.a_bf16 + 2 * hy_act_gated(p.act) + 4 * (p.offs ? 1 : 0) + 8 * (p.even_rows > 0);
+  Kept& k = kept[((unsigned)p.R * 31u + (unsigned)p.N / 4 * 7u + (unsigned)p.K / 64 * 5u + (unsigned)p.E + (unsigned)how) % 64];
+  if (k.R != p.R || k.N != p.N || k.K != p.K || k.E != p.E || k.how != how) k = Kept{p.R, p.N, p.K, p.E, how, rm_best(p)};
+  return k.plan;
 }
 
 // The range, and what is faster outside of it:
