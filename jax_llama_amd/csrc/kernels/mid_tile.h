@@ -56,6 +56,9 @@ JLA_DEV void mid_tile(u32x4* lds, XRow xrow, WRow wrow, int t0, int t1, f32x4 (&
                       int run = 0) {
   using H = MidShape<MT, NT, WN, WK, S, XB>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, q = lane >> 4;
+  // (a tile's place comes from ballots, in vector registers: without this the stage loop ran under a mask, every address formed per lane)
+  t0 = __builtin_amdgcn_readfirstlane(t0);
+  t1 = __builtin_amdgcn_readfirstlane(t1);
   const int wn = wave % WN, wk = wave / WN, ns = (t1 - t0) / WK;
   const char* src[H::OPS];
 #pragma unroll
