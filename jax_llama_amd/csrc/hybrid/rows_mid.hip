@@ -96,9 +96,7 @@ __global__ void __launch_bounds__(256) rows_mid_sum_kernel(RowLinear p, const fl
   rm_store(p, p.dst_idx ? p.dst_idx[r] : (int)r, col, v);
 }
 
-// A form's measured times, us: launch and fill; a stage; a stage's rise with every further workgroup of a compute unit; a split's second
-// launch, and a megabyte through the slabs (write and read)
-struct RmForm {
+struct RmForm {  // (mid_plan)
   int mt, nt, wn, wk, xb;
   float fill, stage, more, sum, mb;
   void (*run)(unsigned, hipStream_t, const RowLinear&, int, int, int, int, float*);
@@ -133,15 +131,7 @@ static const RmForm RM_FORMS[] = {
     RM_FORM(4, 1, 4, 1, 4, 4, 6.66f, 0.436f, 1.02f, 0.0f, 0.484f), RM_FORM(4, 2, 4, 1, 4, 4, 7.55f, 0.601f, 1.09f, 0.0f, 0.382f),
 };
 #undef RM_FORM
-constexpr int RM_MAX_SPLITS = 16;
-
-struct RmPlan {
-  const RmForm* form = nullptr;
-  int splits = 1, steps = 0;
-  float us = 1e30f;
-};
-
-// ... of rows: with experts, whose counts only the device knows, one and a half standard deviations above the mean each
+// Tiles of rows: with experts, whose counts only the device knows, one and a half standard deviations above the mean each
 static long long rm_row_tiles(const RowLinear& p, int bm) {
   if (!p.offs) return (p.R + bm - 1LL) / bm;
   const int E = p.E < p.R ? p.E : p.R;
@@ -151,35 +141,18 @@ static long long rm_row_tiles(const RowLinear& p, int bm) {
 
 // The form and split with the least time by the figures above: on average 2.0 % above the best of all that were measured (384 shapes: one
 // matrix, 8 and 32 experts, N 64 to 32000, K 512 to 14336, 9 to 3200 rows)
-static RmPlan rm_best(const RowLinear& p) {
-  const int gated = hy_act_gated(p.act), T = p.K >> 6, xb = p.a_bf16 ? 2 : 4, E = p.offs ? (p.E < p.R ? p.E : p.R) : 1;
-  const long long nw = gated ? 2LL * p.N : p.N;
-  const float stream = (float)E * (float)nw * (float)p.K * 2 / 5.4e6f;  // the weights themselves
-  RmPlan best;
-  for (const RmForm& f : RM_FORMS) {
-    if (f.xb != xb || (gated && f.nt % 2) || T % f.wk || (p.R <= RM_WIDE_SUM_ROWS && 16 * f.mt > RM_WIDE_SUM_ROWS)) continue;
-    const long long tiles = rm_row_tiles(p, 16 * f.mt) * ((nw + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
-    int last = 0;
-    for (int want = 1; want <= RM_MAX_SPLITS && want <= T; ++want) {
-      const int steps = ((T + want - 1) / want + f.wk - 1) / f.wk * f.wk, splits = (T + steps - 1) / steps;
-      if (splits == last || (want > 1 && (steps < 2 * f.wk || tiles * splits > 700))) continue;
-      last = splits;
-      const float load = (float)(tiles * splits) / 256.f, deep = load > 2.f ? load + .3f : (load > 1.f ? 2.f : 1.f);
-      float us = f.fill + f.stage * (float)(steps / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
-      if (us < 3.5f + stream) us = 3.5f + stream;
-      if (splits > 1) us += f.sum + .15f * (float)splits + f.mb * (float)p.R * (float)nw * (float)splits * 8e-6f;
-      if (f.wk > 1 && load > 2.f) us *= 3.f;  // (16 columns a workgroup: x over and over)
-      if (us < best.us) best = RmPlan{&f, splits, steps, us};
-    }
-  }
-  return best;
+static MidPlan rm_best(const RowLinear& p) {
+  const bool gated = hy_act_gated(p.act);
+  return mid_plan(RM_FORMS, p.R, gated ? 2LL * p.N : p.N, p.K, p.offs ? (p.E < p.R ? p.E : p.R) : 1, [&](const RmForm& f) {
+    return f.xb == (p.a_bf16 ? 2 : 4) && !(gated && f.nt % 2) && !(p.R <= RM_WIDE_SUM_ROWS && 16 * f.mt > RM_WIDE_SUM_ROWS);
+  }, [&](int bm) { return rm_row_tiles(p, bm); });
 }
 
 // ... of the shapes that this thread has had last (the choice takes 1.1 us of host time, and a product asks for it twice)
-static RmPlan rm_plan(const RowLinear& p) {
+static MidPlan rm_plan(const RowLinear& p) {
   struct Kept {
     int R, N, K, E, how;
-    RmPlan plan;
+    MidPlan plan;
   };
   thread_local Kept kept[64];
   const int how = 1 + p.a_bf16 + 2 * hy_act_gated(p.act) + 4 * (p.offs ? 1 : 0) + 8 * (p.even_rows > 0);
@@ -224,22 +197,23 @@ bool hy_rows_mid_takes(const RowLinear& p) {
 }
 
 long long hy_rows_mid_floats(const RowLinear& p) {
-  const RmPlan pl = rm_plan(p);
+  const MidPlan pl = rm_plan(p);
   return pl.splits > 1 ? (long long)pl.splits * p.R * (hy_act_gated(p.act) ? 2 : 1) * p.N : 0;
 }
 
 int hy_rows_mid(const RowLinear& p, float* ws, hipStream_t s) {
   const int gated = hy_act_gated(p.act), E = p.offs ? p.E : 1;
-  const RmPlan pl = rm_plan(p);
-  if (!pl.form) return -13;
-  const int bm = 16 * pl.form->mt, bn = 16 * pl.form->nt * pl.form->wn;
+  const MidPlan pl = rm_plan(p);
+  if (pl.form < 0) return -13;
+  const RmForm& f = RM_FORMS[pl.form];
+  const int bm = 16 * f.mt, bn = 16 * f.nt * f.wn;
   const long long tn = ((gated ? 2LL : 1LL) * p.N + bn - 1) / bn;
   const long long grid = ((p.offs ? p.R / bm + (long long)E : (p.R + bm - 1LL) / bm) * tn * pl.splits + 7) / 8 * 8;
   if (grid > 0x7fffffffLL) return -4;
   if (pl.splits > 1 && (!ws || ((uintptr_t)ws & 15))) return -12;
   RowLinear q = p;
   q.row_expert = nullptr;
-  pl.form->run((unsigned)grid, s, q, gated, (int)tn, pl.splits, pl.steps, pl.splits > 1 ? ws : nullptr);
+  f.run((unsigned)grid, s, q, gated, (int)tn, pl.splits, pl.steps, pl.splits > 1 ? ws : nullptr);
   JLA_CHECK_LAUNCH();
   if (pl.splits > 1) {
     const long long n = (long long)p.R * (p.N / 4);

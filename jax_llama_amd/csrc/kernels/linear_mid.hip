@@ -123,9 +123,7 @@ __global__ void __launch_bounds__(64 * WN * WK, (MidShape<MT, NT, WN, WK, S, 2>:
   }
 }
 
-// A form's measured times, us: launch and fill; a stage; a stage's rise with every further workgroup of a compute unit; a split's second
-// launch, and a megabyte through the slabs (write and read)
-struct LmForm {
+struct LmForm {  // (mid_plan)
   int mt, nt, wn, wk;
   float fill, stage, more, sum, mb;
   void (*run)(unsigned, hipStream_t, const LinearMid&);
@@ -143,7 +141,7 @@ static const LmForm LM_FORMS[] = {
     LM_FORM(8, 2, 4, 1, 4, 7.85f, 0.586f, 1.28f, 0.0f, 0.225f),
 };
 #undef LM_FORM
-constexpr int LM_N_FORMS = sizeof(LM_FORMS) / sizeof(LM_FORMS[0]), LM_MAX_SPLITS = 16;
+constexpr int LM_N_FORMS = sizeof(LM_FORMS) / sizeof(LM_FORMS[0]);
 
 bool linear_mid_tile(int tile) { return tile >= LINEAR_MID_TILE && tile < LINEAR_MID_TILE + LM_N_FORMS; }
 
@@ -158,31 +156,9 @@ constexpr int LM_WIDE_M = 96, LM_WIDE_N = 65536;
 int linear_mid_plan(int M, int N, int K, int* ksplit) {
   *ksplit = 1;
   if (M < LINEAR_MID_MIN_M || M > LINEAR_MID_MAX_M || (N & 15) || (K & 63) || K < 128 || (M > LM_WIDE_M && N > LM_WIDE_N)) return 0;
-  const int T = K >> 6;
-  const float stream = (float)N * (float)K * 2 / 5.4e6f;  // us of the weights themselves
-  int tile = 0;
-  float best = 1e30f;
-  for (int i = 0; i < LM_N_FORMS; ++i) {
-    const LmForm& f = LM_FORMS[i];
-    if (T % f.wk) continue;
-    const long long tiles = (M + 16LL * f.mt - 1) / (16LL * f.mt) * ((N + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
-    int last = 0;
-    for (int want = 1; want <= LM_MAX_SPLITS && want <= T; ++want) {
-      const int steps = ((T + want - 1) / want + f.wk - 1) / f.wk * f.wk, splits = (T + steps - 1) / steps;
-      if (splits == last || (want > 1 && (steps < 2 * f.wk || tiles * splits > 700))) continue;
-      last = splits;
-      const float load = (float)(tiles * splits) / 256.f, deep = load > 2.f ? load + .3f : (load > 1.f ? 2.f : 1.f);
-      float us = f.fill + f.stage * (float)(steps / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
-      if (us < 3.5f + stream) us = 3.5f + stream;
-      if (splits > 1) us += f.sum + .15f * (float)splits + f.mb * (float)M * (float)N * (float)splits * 8e-6f;
-      if (us < best) {
-        best = us;
-        tile = LINEAR_MID_TILE + i;
-        *ksplit = splits;
-      }
-    }
-  }
-  return tile;
+  const MidPlan p = mid_plan(LM_FORMS, M, N, K, 1, [](const LmForm&) { return true; }, [&](int bm) { return (M + bm - 1LL) / bm; });
+  *ksplit = p.splits;
+  return p.form < 0 ? 0 : LINEAR_MID_TILE + p.form;
 }
 
 // The product's launch (of splits > 1, or slabs for another reason: the partial sums' one): K in `ksplit` runs, as linear_mid_plan cuts it

@@ -27,6 +27,40 @@ struct MidShape {
 };
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+// The form and K split with the least time of a product of `rows` rows and `cols` weight rows (of `matrices` matrices). A form's measured
+// times, us: launch and fill; a stage; a stage's rise with every further workgroup of a compute unit (more); a split's second launch (sum), and a
+// megabyte through the slabs, write and read (mb). takes(form): whether it runs these operands; row_tiles(height).
+struct MidPlan {
+  int form = -1, splits = 1, steps = 0;
+  float us = 1e30f;
+};
+constexpr int MID_MAX_SPLITS = 16;
+
+template <class Form, int N, class Takes, class RowTiles>
+inline MidPlan mid_plan(const Form (&forms)[N], long long rows, long long cols, int K, int matrices, Takes takes, RowTiles row_tiles) {
+  const int T = K >> 6;
+  const float stream = (float)matrices * (float)cols * (float)K * 2 / 5.4e6f;  // the weights themselves
+  MidPlan best;
+  for (int i = 0; i < N; ++i) {
+    const Form& f = forms[i];
+    if (T % f.wk || !takes(f)) continue;
+    const long long tiles = row_tiles(16 * f.mt) * ((cols + 16LL * f.nt * f.wn - 1) / (16LL * f.nt * f.wn));
+    int last = 0;
+    for (int want = 1; want <= MID_MAX_SPLITS && want <= T; ++want) {
+      const int steps = ((T + want - 1) / want + f.wk - 1) / f.wk * f.wk, splits = (T + steps - 1) / steps;
+      if (splits == last || (want > 1 && (steps < 2 * f.wk || tiles * splits > 700))) continue;
+      last = splits;
+      const float load = (float)(tiles * splits) / 256.f, deep = load > 2.f ? load + .3f : (load > 1.f ? 2.f : 1.f);
+      float us = f.fill + f.stage * (float)(steps / f.wk) * (1.f + f.more * (deep - 1.f)) + deep - 1.f;
+      if (us < 3.5f + stream) us = 3.5f + stream;
+      if (splits > 1) us += f.sum + .15f * (float)splits + f.mb * (float)rows * (float)cols * (float)splits * 8e-6f;
+      if (f.wn == 1 && load > 2.f) us *= 3.f;  // (16 columns a workgroup: x over and over)
+      if (us < best.us) best = MidPlan{i, splits, steps, us};
+    }
+  }
+  return best;
+}
+
 // 16-byte cell of chunk x of row r in its 128-byte line of LDS: the 16 lanes that a fragment read serves at a time (rows 0-3 and 12-15
 // of one quarter, 4-11 of the next) fall on all 64 banks; fp32 rows, whose quarter is two chunks, need another order for that
 JLA_DEV int mid_cell(int x, int r, int xb) {
