@@ -322,10 +322,11 @@ __global__ void __launch_bounds__(64 * WAVES) attn_step_kernel(AttnStep p) {
   }
 }
 
-// Heads of 64 or 128 numbers, as far as the splits of a call go before its rows and heads alone fill the chip (hy_attn_decode_splits): a
-// decode step with two of these launches in the place of three or four each, us, separate | here, heads of 128, rows x heads x splits: norms, 2 x
-// 16 x 47 317 | 312, 3 x 16 x 33 384 | 378, 8 x 16 x 16 442 | 435, 8 x 32 x 5 1164 | 1146, 32 x 16 x 4 663 | 662; rotations, 8 x 16 x 16 274 | 268, 13 x 32 x 5
-// 708 | 695, 32 x 16 x 4 447 | 435, 128 x 16 x 1 721 | 707.
+// Heads of 64 or 128 numbers, up to 2560 splits in all. hy_attn_decode_splits cuts rows x heads = P of long caches in 2048 / P, rounded up: that
+// is within it for P up to 640 and most beyond (683 to 853, 1024 to 1280, 2048 to 2560), while P of 641 to 682, 854 to 1023 and 1281 to 2047,
+// which round up past it, keep the separate launches that they had (not measured here). A decode step with two of these launches in the place of
+// three or four each, us, separate | here, heads of 128, rows x heads x splits: norms, 2 x 16 x 47 317 | 312, 3 x 16 x 33 384 | 378, 8 x 16 x 16 442 |
+// 435, 8 x 32 x 5 1164 | 1146, 32 x 16 x 4 663 | 662; rotations, 8 x 16 x 16 274 | 268, 13 x 32 x 5 708 | 695, 32 x 16 x 4 447 | 435, 128 x 16 x 1 721 | 707.
 constexpr long long AS_MAX_WAVES = 2560;
 constexpr int AS_PAIR_SPLITS = 16;  // more of them: two per workgroup (hy_attn_step)
 

@@ -7,7 +7,7 @@
 //   one to 64 rows on bf16 weights otherwise, 16-byte rows      rows_gemv.hip, on the matrix cores
 //   one or two rows on fp32 weights (up to 8 with an expert each), K 512 (two rows: 1024) to 8192, 16-byte rows   rows_gemv.hip
 //   up to 8 rows, or 64 sorted by expert, otherwise             the vector GEMV below (fp32 weights, odd or short K)
-//   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, 256-row tiles
+//   a prompt's bf16 rows, K >= 1024                             rows_gemm.hip, tiles of 128 to 256 rows
 //   fp32 weights, 16-byte rows, K >= 512 (256 with many rows)   rows_f32.hip, split products on the bf16 matrix cores
 //   the rest                                                    the tiles below
 // The tiles round an fp32 A to bf16 while it is staged where the weights are bf16 (v_mfma_f32_32x32x16_bf16, fp32

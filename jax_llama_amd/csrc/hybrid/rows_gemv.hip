@@ -12,7 +12,8 @@
 // of four MFMAs, and then the waves', are added in 64 bits: the matrix instruction cuts the small ones of the 8 products that it adds at a
 // time at 24 bits of the largest, and that already is the error of the vector unit's six lane exchanges (against 64 bits, one row
 // of K 2048 | 7168: vector unit 7.5e-8 | 9.5e-8; one chain per wave and the waves one by one 9.7e-8 | 13.9e-8; now 6.4e-8 |
-// 6.9e-8; 64 rows of 8 experts, K 7168: 9.5e-8, 25.4e-8, 7.0e-8).
+// 6.9e-8; 64 rows of 8 experts, K 7168: 9.5e-8, 25.4e-8, 7.0e-8). From nine rows on of one matrix, and from five per expert of several large
+// ones, rows_mid.hip takes what it can (hy_rows_mid_takes); the figures of 33 rows are of before that.
 // Us before -> after, weights in no cache, 1 | 8 | 33 rows: K 2048 x N 5152 11.1 -> 7.7 | 27.4 -> 10.7 | 54 -> 21; 4096 x 10304 42.6 ->
 // 19.1 | 62.6 -> 26.6 | 108 -> 59; 2048 x 32000 49.6 -> 24.3 (5.4 TB/s) | 99 -> 29.4 | 67 -> 63; gated 2048 x 5632 17.2 -> 12.4 |
 // 44.8 -> 16.0 | 82 -> 34; both products of 2 of 8 experts (4096 x 7168) for 1 | 8 tokens 105 -> 68 | 403 -> 230. With one output element
@@ -290,6 +291,9 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
         }
       }
     } else {
+      // The same loop for fp32 rows without a pipeline, written out: through load() and use() the compiler makes slower code of it (us, here |
+      // there: one row of 1024 x 1024 3.5 | 4.0, 10304 x 2048 10.0 | 11.0, gated 2048 x 5632 11.5 | 13.6, 8 rows of 4096 x 14336 34.6 | 45.6; some
+      // sorted rows a tenth faster, 64 of 8 experts of 2048 x 2816 30.3 | 28.3)
       for (int s0 = wave; s0 < steps; s0 += WAVES * U) {
         u32x4 wf[U][H][NT];
         f32x4 xa[U][H][MT], xb[U][H][MT];
@@ -1049,9 +1053,9 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
       RV_NT(16, 0, T);                   \
     }                                    \
   } while (0)
-  // (rows that had the vector unit's form are added in 64 bits, to lose no more than it did; more than eight dense rows had the
-  // tiles' one fp32 chain over all of K, 2.7e-7 at K 2048, here 1.3e-7 in one chain per wave: 33 rows of 4096 x 10304 60.5 us,
-  // 64.5 in 64 bits)
+  // (rows that had the vector unit's form are added in 64 bits, to lose no more than it did; more than eight dense rows, those that
+  // rows_mid.hip leaves, had the tiles' one fp32 chain over all of K, 2.7e-7 at K 2048, here 1.3e-7 in one chain per wave: 33 rows of 4096 x
+  // 10304 60.5 us, 64.5 in 64 bits)
   if (G == 4) {
     // Two tiles: batches of four or three steps where they divide a wave's (a step past the end costs its loads), their sums added in 64 bits
     // every two as in batches of two. Us, weights in no cache, two | three | four steps, one row: 10304 x 2048 10.3 | 13.0 | 9.9, 32000 x 2048 (two
