@@ -1,11 +1,11 @@
 // Some ten to a few hundred rows on row-major bf16 weights: out[dst(r), :] = act(A[src(r), :] @ W[expert(r)]^T), dense or with some
 // rows per expert, the rows bf16 or fp32 (rounded as a fragment is read). kernels/mid_tile.h says what bounds it and why the tile is
 // as it is; here are its forms, the choice among them, and the epilogue.
-// Us, weights in no cache, 16 | 64 | 128 | 255 rows, the forms before (rows_gemv.hip to 64 rows, lr_gemm_kernel's tiles) -> here, from 65 rows on
-// with the rounding of the rows: 2048 x 2048 9.5 | 23.8 | 41 | 41 -> 7.3 | 10.0 | 12.4 | 16.6; 2048 x 5632 20.7 | 55 | 157 | 157 -> 14 | 17 | 20 | 25;
-// 4096 x 4096 16.4 | 42 | 108 | 103 -> 13.5 | 19 | 23 | 28; 4096 x 14336 50 | 132 | 392 | 392 -> 29 | 35 | 46 | 55; gated 5632 x 2048 20 | 41 | 87 | 87 ->
-// 17 | 22 | 26 | 39. A mixture of 8 experts of 2816 x 2048 (7168 x 4096), two per token, both products, 33 | 100 | 256 tokens: 165 | 172 | 133 -> 77 |
-// 80 | 88 (452 | 473 | 425 -> 257 | 289 | 297; its weights 237 at 5.95 TB/s).
+// Us, weights in no cache, 16 | 64 | 100 | 200 fp32 rows, the forms before (rows_gemv.hip to 64 rows, lr_gemm_kernel's tiles) -> here, from 65 rows
+// on with the rounding of the rows: 2048 x 2048 8.7 | 23.5 | 41 | 39 -> 7.7 | 12.3 | 11.7 | 13.1 (bf16 rows 6.4 | 7.9 | 9.5 | 10.3); 2048 x 5632 19.9 | 55 | 154 |
+// 144 -> 13.1 | 16.1 | 19.9 | 24; 4096 x 4096 16.5 | 42 | 107 | 95 -> 13.2 | 17.3 | 21 | 28; 4096 x 14336 50 | 132 | 376 | 354 -> 29 | 33 | 40 | 53. A mixture
+// of 8 experts of 2816 x 2048 (7168 x 4096), two per token, both products, 33 | 100 | 256 tokens: 165 | 172 | 133 -> 77 | 80 | 88 (452 | 473 | 425 ->
+// 257 | 289 | 297; its weights 237 at 5.95 TB/s).
 #include "../kernels/mid_tile.h"
 #include "../kernels/row_tiles.h"
 #include "hy_util.h"
