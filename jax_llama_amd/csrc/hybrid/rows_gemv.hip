@@ -6,8 +6,12 @@
 // instructions per weight (1.5-3.0 TB/s), eight rows re-read eight fp32 activation rows per column (0.6-1.6 TB/s).
 // Here a lane's 16 bytes of a row-major weight row are the A operand of v_mfma_f32_16x16x32_bf16. With up to G = 4 or 8
 // rows the instruction's 16 A rows are G output columns times 16 / G neighbouring K ranges and its 16 B columns the G
-// activation rows times the same ranges: the diagonal blocks of the product hold the sums, a load covers G rows x 1024 / G
+// activation rows times the same ranges: the diagonals of the product's blocks hold the sums, a load covers G rows x 1024 / G
 // contiguous bytes, and a workgroup needs only G columns -- enough workgroups for every compute unit from 1024 columns on.
+// Lanes next to each other take the ranges of one row, so that they read 64 (G = 8: 32) bytes in one piece: from a cache a compute unit
+// takes 128 bytes per ns in pieces of 64, 75 in pieces of 32 and 38 in pieces of 16, where every lane has another row. Us with a row per lane -> now,
+// weights in no cache, 1 | 2 | 8 rows: K 2048 x N 5152 6.8 -> 6.2 | 7.5 -> 6.5 | 9.0 -> 7.7; 4096 x 10304 18.4 -> 16.7 | 20.1 -> 17.1 | 21.0 -> 18.5;
+// 5632 x 2048 7.9 -> 7.2 | 9.1 -> 7.4 | 9.9 -> 8.1; gated and normed 2048 x 5632 11.2 -> 10.3 | 12.4 -> 11.3 | 15.2 -> 13.8.
 // The waves of a workgroup deal the K steps among themselves, U in flight each, and sum their blocks through LDS. The sums
 // of four MFMAs, and then the waves', are added in 64 bits: the matrix instruction cuts the small ones of the 8 products that it adds at a
 // time at 24 bits of the largest, and that already is the error of the vector unit's six lane exchanges (against 64 bits, one row
@@ -75,6 +79,22 @@ JLA_DEV float rv_sum(const float (&f)[N]) {
   return (float)s[0];
 }
 
+// The products of a lane of mfma16x16x32 whose A row SEG i + sg is column i, and whose B column SEG r + sg is row r, on K range sg: lane (c, q) holds
+// A rows 4 q + 0..3 of B column c, of which those of range c % SEG count, the j-th of 4 / SEG (column q 4 / SEG + j)
+template <int SEG>
+JLA_DEV float rv_own(float v0, float v1, float v2, float v3, int c, int j) {
+  if constexpr (SEG == 1) return j == 0 ? v0 : j == 1 ? v1 : j == 2 ? v2 : v3;
+  const float lo = c & 1 ? v1 : v0, hi = c & 1 ? v3 : v2;
+  if constexpr (SEG == 2) return j == 0 ? lo : hi;
+  return c & 2 ? hi : lo;
+}
+// where they lie for column y and row x, range by range, among 4 / SEG planes of 64 lanes
+template <int SEG>
+JLA_DEV int rv_place(int x, int y) {
+  constexpr int EL = 4 / SEG;
+  return 64 * (y % EL) + 16 * (y / EL) + SEG * x;
+}
+
 // the better of two candidates of a maximum: the larger, ties to the lower index, a NaN never
 JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
   if (v > bv || (v == bv && i < bi)) {
@@ -111,7 +131,8 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   constexpr int RUN = !WIDE ? U : (G == 4 && NT > 1 ? 2 : 4 / H);
   constexpr int ROWS = G * MT;               // rows of a pass
   using XNum = std::conditional_t<XB == 2, bf16_t, float>;
-  __shared__ f32x4 red[WAVES][NT * MT][64];
+  constexpr int EL = 4 / SEG;                // products of a lane that count
+  __shared__ __align__(16) float red[WAVES][NT * MT][64 * EL];
   __shared__ float stat[NORM ? WAVES : 1][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
   rv_arguments(p);
@@ -126,13 +147,13 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
     if (e < 0) return;
   }
   const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP;
-  const int k0 = 32 * (c / G) + 8 * q;  // this lane's place in a step
+  const int k0 = 8 * (c % SEG) + 8 * SEG * q;  // this lane's place in a step
   const bf16_t* wbase = reinterpret_cast<const bf16_t*>(p.w) + (size_t)e * p.w_stride;
   const bf16_t* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int T = blockIdx.x * NT + t;
-    const int col = min(G * (gated ? T >> 1 : T) + c % G, N - 1);
+    const int col = min(G * (gated ? T >> 1 : T) + c / SEG, N - 1);
     wp[t] = wbase + (size_t)(gated && (T & 1) ? N + col : col) * K;
   }
   for (int r0 = g0; r0 < g1; r0 += ROWS) {
@@ -141,7 +162,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
     float xs[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const int rr = r0 + min(16 * m + c % G, nr - 1);  // (surplus lanes repeat the last row; their results are dropped)
+      const int rr = r0 + min(16 * m + c / SEG, nr - 1);  // (surplus lanes repeat the last row; their results are dropped)
       xp[m] = reinterpret_cast<const XNum*>(p.a) + (size_t)(p.a_idx ? p.a_idx[rr] : (p.a_div > 1 ? rr / p.a_div : rr)) * p.lda;
       xs[m] = p.a_scale ? p.a_scale[rr] : 1.f;
     }
@@ -165,12 +186,13 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
         }
       }
 #pragma unroll
-      for (int o = G; o < 64; o <<= 1) ss += __shfl_xor(ss, o, 64);
-      if (lane < G) stat[wave][lane] = ss;
+      for (int o = 1; o < 64; o <<= 1)
+        if (o < SEG || o >= 16) ss += __shfl_xor(ss, o, 64);
+      if (q == 0 && c % SEG == 0) stat[wave][c / SEG] = ss;
       __syncthreads();
       ss = 0.f;
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) ss += stat[w][c % G];
+      for (int w = 0; w < WAVES; ++w) ss += stat[w][c / SEG];
       xs[0] = 1.f / sqrtf(ss / (float)K + p.a_norm_eps);
     }
     SUM acc[NT][MT][4];  // (64 bits cost little beside the stream: 8 rows, K 7168 x N 4096: 16.7 -> 17.0 us)
@@ -365,13 +387,16 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
         }
       }
     }
-    // lane: row (B column) c, columns (A rows) 4 q + 0..3 of tile t
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        red[wave][t * MT + m][lane] = WIDE ? f32x4{(float)acc[t][m][0], (float)acc[t][m][1], (float)acc[t][m][2], (float)acc[t][m][3]}
-                                           : part[t][m];
+      for (int m = 0; m < MT; ++m) {
+        float own[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) own[i] = WIDE ? (float)acc[t][m][i] : part[t][m][i];
+#pragma unroll
+        for (int j = 0; j < EL; ++j) red[wave][t * MT + m][64 * j + lane] = rv_own<SEG>(own[0], own[1], own[2], own[3], c, j);
+      }
     __syncthreads();
     // one output element per thread: the epilogue's code, which a short launch has to fetch, stays small
     constexpr int PER = G * G;  // (column, row) pairs of a tile
@@ -383,12 +408,11 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
       const int slot = (gated ? 2 * to : to) * MT + m;
       auto total = [&](int at) {
         float f[SEG * WAVES];
+        const int from = rv_place<SEG>(x, y);
 #pragma unroll
-        for (int sg = 0; sg < SEG; ++sg) {  // the diagonal block of range sg
-          const int l = 16 * (G / 4 * sg + y / 4) + G * sg + x;
+        for (int w = 0; w < WAVES; ++w)
 #pragma unroll
-          for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[w][at][l][y % 4];
-        }
+          for (int sg = 0; sg < SEG; ++sg) f[sg * WAVES + w] = red[w][at][from + sg];
         return rv_sum<SUM>(f);
       };
       const float g = total(slot), v = gated ? total(slot + MT) : 0.f;
@@ -524,9 +548,9 @@ struct RvRow {
 // a run of the workgroups, the rows blended for it as they are staged.
 template <int NT, int U, int V, int PARTS, int BEST = 0>
 __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
-  constexpr int G = 4, WAVES = 4, STEP = 128;
+  constexpr int G = 4, SEG = 4, WAVES = 4, STEP = 128;
   extern __shared__ f32x4 staged[];  // [rows][K]
-  __shared__ f32x4 red[2][WAVES][NT][64];
+  __shared__ __align__(16) float red[2][WAVES][NT][64];
   __shared__ float stat[WAVES][16];
   __shared__ float2 cand[BEST ? NT * 4 * RV_WALK_ROWS : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
@@ -550,7 +574,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   const int r0 = blockIdx.y * rows_per_group, nr = min(rows_per_group, p.R - r0);
   const int e = rv_expert(p, r0);
   if (e < 0) return;  // (the whole workgroup)
-  const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP, k0 = 32 * (c / G) + 8 * q;
+  const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP, k0 = 8 * (c % SEG) + 8 * SEG * q;
   const bf16_t* wbase = reinterpret_cast<const bf16_t*>(p.w) + (size_t)e * p.w_stride;
   // this lane's place in step u (a lane past the end of K reads the row's start; its operand is zero)
   auto at = [&](int u) {
@@ -559,7 +583,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   };
   u32x4 wf[U][NT];
   auto weight_row = [&](int tg, int t) {
-    const int T = tg * NT + t, col = min(G * (gated ? T >> 1 : T) + c % G, N - 1);
+    const int T = tg * NT + t, col = min(G * (gated ? T >> 1 : T) + c / SEG, N - 1);
     return wbase + (size_t)(gated && (T & 1) ? N + col : col) * K;
   };
   RvRow<V, PARTS> row;
@@ -586,7 +610,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   u32x4 xr[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {  // (surplus B columns repeat the last row; their results are dropped)
-    const f32x4* x = staged + ((size_t)min(c % G, nr - 1) * K + at(u)) / 4;
+    const f32x4* x = staged + ((size_t)min(c / SEG, nr - 1) * K + at(u)) / 4;
     xr[u] = STEP * (wave + WAVES * u) + k0 < K ? rv_round8(x[0], x[1]) : u32x4{0, 0, 0, 0};
   }
   for (int buf = 0; tg < tgroups; tg += walk, buf ^= 1) {
@@ -606,7 +630,7 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
       }
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) red[buf][wave][t][lane] = acc[t];
+    for (int t = 0; t < NT; ++t) red[buf][wave][t][lane] = rv_own<SEG>(acc[t][0], acc[t][1], acc[t][2], acc[t][3], c, 0);
     __syncthreads();  // (one per group: the other buffer's readers are past the barrier before)
     const int outs = (gated ? NT / 2 : NT) * nr * G;
     if (tid < outs) {
@@ -615,9 +639,11 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
       auto total = [&](int at) {
         float f[4 * WAVES];
 #pragma unroll
-        for (int sg = 0; sg < 4; ++sg)  // the diagonal block of K range sg
+        for (int w = 0; w < WAVES; ++w) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(&red[buf][w][at][rv_place<SEG>(x, y)]);
 #pragma unroll
-          for (int w = 0; w < WAVES; ++w) f[sg * WAVES + w] = red[buf][w][at][20 * sg + x][y];
+          for (int sg = 0; sg < 4; ++sg) f[sg * WAVES + w] = v[sg];
+        }
         return rv_sum<double>(f);
       };
       const float g = total(slot), v = gated ? total(slot + 1) : 0.f;
