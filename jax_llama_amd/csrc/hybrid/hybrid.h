@@ -93,7 +93,7 @@ struct RowParts {
 };
 bool hy_rows_parts_takes(const RowLinear& p, const RowParts& t);  // p: a, lda, K, R, a_norm_w, a_norm_eps
 int hy_rows_parts(const RowLinear& p, const RowParts& t, hipStream_t s);
-inline bool hy_act_gated(int act) {
+constexpr bool hy_act_gated(int act) {
   return act == HY_ACT_SWIGLU || act == HY_ACT_CLAMP_GLU || act == HY_ACT_GELU_GLU;
 }
 // rows up to which the vector GEMV takes a dense batch or rows with an expert each (one wave per output column, weights

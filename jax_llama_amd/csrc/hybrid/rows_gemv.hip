@@ -103,6 +103,29 @@ JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
   }
 }
 
+// FORM of a kernel: -1, any call; else one of plain rows -- in place and order, of one matrix or the table's experts -- whose results go to fp32 rows
+// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm and with RV_ONE one row per group: the branches that such a call does not take are
+// not in its code. A launch of a few microseconds waits for the code on its path, some 0.13 us per KB. One row, weights in no cache, any call's code ->
+// its own: 2048 x 2048 8.4 -> 5.9 KB, 4.1 -> 3.7 us; 2048 x 5152 5.5 -> 3.1 KB, 6.2 -> 5.8; walking, normed 2048 x 2048 9.8 -> 3.2 KB, 4.9 -> 4.3,
+// 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096 with a residual 10.3 -> 9.5. Two rows keep any call's walk (as a loop over the rows it was
+// smaller and slower: the first weights were waited for at its edge).
+constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32;
+template <int FORM>
+JLA_DEV void rv_form(RowLinear& p) {
+  if constexpr (FORM >= 0) {
+    p.a_idx = p.dst_idx = p.offs = p.row_expert = p.mul_ids = nullptr;
+    p.a_scale = nullptr;
+    p.out_bf16 = p.add_out = 0;
+    p.act = FORM % 8;
+    if (!(FORM & RV_RES)) p.res_y = nullptr;
+    if (!(FORM & RV_NORM)) p.a_norm_w = nullptr;
+  }
+}
+static int rv_form_of(const RowLinear& p, int rows_per_group) {
+  const bool plain = !p.a_idx && !p.dst_idx && !p.offs && !p.row_expert && !p.mul_ids && !p.a_scale && !p.out_bf16 && !p.add_out;
+  return plain ? p.act + (p.res_y ? RV_RES : 0) + (p.a_norm_w ? RV_NORM : 0) + (rows_per_group == 1 || p.R == 1 ? RV_ONE : 0) : -1;
+}
+
 // output column col of linear row r from its accumulators
 JLA_DEV void rv_store(const RowLinear& p, int r, int col, float g, float v) {
   const size_t at = (size_t)(p.dst_idx ? p.dst_idx[r] : r) * p.ldo + col;
@@ -120,8 +143,9 @@ JLA_DEV void rv_store(const RowLinear& p, int r, int col, float g, float v) {
 // alternate); MT: 16-row tiles (G = 16); U: K steps in flight per wave. NORM 1 (MT = 1): rows are RMS-normed with a gain
 // first, in the order (a * scale) * gain of the norm kernel. SUM: the type that the MFMAs' sums are added in. XB: bytes of an activation.
 // PIPE: a batch of loads goes out before the one ahead of it is waited for.
-template <int G, int NT, int MT, int WAVES, int U, int NORM, class SUM, int XB, bool PIPE>
+template <int G, int NT, int MT, int WAVES, int U, int NORM, class SUM, int XB, bool PIPE, int FORM = -1>
 __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int rows_per_group, int gated) {
+  if constexpr (FORM >= 0) gated = hy_act_gated(FORM % 8);
   static_assert(G == 16 || MT == 1, "several row tiles: whole 16-column tiles");
   constexpr int SEG = 16 / G;                // neighbouring K ranges of one MFMA
   constexpr int H = G == 16 ? 2 : 1;         // MFMAs of a K step (G = 16: the two halves of a 128-byte line)
@@ -135,6 +159,7 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   __shared__ __align__(16) float red[WAVES][NT * MT][64 * EL];
   __shared__ float stat[NORM ? WAVES : 1][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, q = lane >> 4;
+  rv_form<FORM>(p);
   rv_arguments(p);
   // rows of this group: a fixed count, one row with its own expert, or (offs) every row of expert blockIdx.y
   int g0 = blockIdx.y * rows_per_group, g1 = min(g0 + rows_per_group, p.R), e = 0;
@@ -546,7 +571,7 @@ struct RvRow {
 // through LDS once per workgroup, where a pending residual add (res_y) and the norm are applied behind the first weights.
 // grid (workgroups, linear rows with their own expert, else 1). PARTS: several matrices (RowParts) that read the same rows, each with
 // a run of the workgroups, the rows blended for it as they are staged.
-template <int NT, int U, int V, int PARTS, int BEST = 0>
+template <int NT, int U, int V, int PARTS, int BEST = 0, int FORM = -1>
 __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
   constexpr int G = 4, SEG = 4, WAVES = 4, STEP = 128;
   extern __shared__ f32x4 staged[];  // [rows][K]
@@ -558,6 +583,11 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   int bi = 0x7fffffff;
   int part = 0, tg = blockIdx.x, walk = gridDim.x;  // this workgroup's first group of tiles, and from one to its next
   if constexpr (PARTS) {
+    rv_form<FORM>(p);
+    if constexpr (FORM >= 0) {
+      gated = 0;
+      p.tab = nullptr;
+    }
     while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
     tg -= parts.first[part];
     walk = parts.first[part + 1] - parts.first[part];
@@ -569,9 +599,11 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
     p.act = parts.cap[part] > 0.f ? HY_ACT_SOFTCAP : HY_ACT_NONE;
     p.act_limit = parts.cap[part];
   } else {
+    rv_form<FORM>(p);
+    if constexpr (FORM >= 0) gated = hy_act_gated(FORM % 8);
     rv_arguments(p);
   }
-  const int r0 = blockIdx.y * rows_per_group, nr = min(rows_per_group, p.R - r0);
+  const int r0 = blockIdx.y * rows_per_group, nr = FORM >= 0 && (FORM & RV_ONE) ? 1 : min(rows_per_group, p.R - r0);
   const int e = rv_expert(p, r0);
   if (e < 0) return;  // (the whole workgroup)
   const int K = p.K, N = p.N, steps = (K + STEP - 1) / STEP, k0 = 8 * (c % SEG) + 8 * SEG * q;
@@ -902,7 +934,10 @@ int hy_rows_parts(const RowLinear& p, const RowParts& parts, hipStream_t s) {
     return 0;
   }
   const unsigned lds = (unsigned)(p.R * p.K * sizeof(float));
-  if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1><<<grid, 256, lds, s>>>(p, p.R, 0, 0, t);
+  // (its rows are in place and order; one row's form without the second's code)
+  if (p.R == 1 && p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1, 0, RV_ONE + RV_NORM><<<grid, 256, lds, s>>>(p, 1, 0, 0, t);
+  else if (p.R == 1) rows_gemv_walk_kernel<2, 8, 4, 1, 0, RV_ONE + RV_NORM><<<grid, 256, lds, s>>>(p, 1, 0, 0, t);
+  else if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 1><<<grid, 256, lds, s>>>(p, p.R, 0, 0, t);
   else rows_gemv_walk_kernel<2, 8, 4, 1><<<grid, 256, lds, s>>>(p, p.R, 0, 0, t);
   JLA_CHECK_LAUNCH();
   return 0;
@@ -1014,11 +1049,34 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
     if (!rv_walk_grid(p, groups, wnt, tg, wgs)) return -4;
     const dim3 grid((unsigned)wgs, groups);
     const unsigned lds = (unsigned)(rows * p.K * sizeof(float));
-#define RV_WALK(NT, U, V) rows_gemv_walk_kernel<NT, U, V, 0><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
+#define RV_WALK_FORM(NT, U, V, F) rows_gemv_walk_kernel<NT, U, V, 0, 0, F><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
+#define RV_WALK_ACT(NT, U, V, A)                                                              \
+  do {                                                                                        \
+    if (form == (A) + RV_ONE + RV_RES) RV_WALK_FORM(NT, U, V, (A) + RV_ONE + RV_RES);         \
+    else if (form == (A) + RV_ONE + RV_NORM) RV_WALK_FORM(NT, U, V, (A) + RV_ONE + RV_NORM);  \
+    else RV_WALK_FORM(NT, U, V, (A) + RV_ONE + RV_RES + RV_NORM);                             \
+  } while (0)
+#define RV_WALK(NT, U, V)                                                                     \
+  do {                                                                                        \
+    const int act = form >= RV_ONE ? form % 8 : -1;                                           \
+    if (act == HY_ACT_NONE) RV_WALK_ACT(NT, U, V, HY_ACT_NONE);                               \
+    else if (NT == 2 && act == HY_ACT_SWIGLU) RV_WALK_ACT(2, U, V, HY_ACT_SWIGLU);            \
+    else if (NT == 2 && act == HY_ACT_CLAMP_GLU) RV_WALK_ACT(2, U, V, HY_ACT_CLAMP_GLU);      \
+    else RV_WALK_FORM(NT, U, V, -1);                                                          \
+  } while (0)
+#define RV_BEST_FORM(U, V, F) rows_gemv_walk_kernel<2, U, V, 0, 1, F><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
+#define RV_BEST(U, V)                                                                                                  \
+  do {                                                                                                                 \
+    if (form == HY_ACT_NONE + RV_ONE + RV_NORM) RV_BEST_FORM(U, V, HY_ACT_NONE + RV_ONE + RV_NORM);                    \
+    else if (form == HY_ACT_NONE + RV_ONE + RV_NORM + RV_RES) RV_BEST_FORM(U, V, HY_ACT_NONE + RV_ONE + RV_NORM + RV_RES); \
+    else if (form == HY_ACT_SOFTCAP + RV_ONE + RV_NORM) RV_BEST_FORM(U, V, HY_ACT_SOFTCAP + RV_ONE + RV_NORM);         \
+    else RV_BEST_FORM(U, V, -1);                                                                                       \
+  } while (0)
+    const int form = rv_form_of(q, rpg);
     if (p.best) {
       if (wnt != 2 || groups != 1 || gated) return -11;
-      if (p.K <= 2048) rows_gemv_walk_kernel<2, 4, 2, 0, 1><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{});
-      else rows_gemv_walk_kernel<2, 8, 4, 0, 1><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{});
+      if (p.K <= 2048) RV_BEST(4, 2);
+      else RV_BEST(8, 4);
     } else if (p.K <= 2048) {
       if (wnt == 1) RV_WALK(1, 4, 2);
       else RV_WALK(2, 4, 2);
@@ -1026,7 +1084,11 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
       if (wnt == 1) RV_WALK(1, 8, 4);
       else RV_WALK(2, 8, 4);
     }
+#undef RV_BEST
+#undef RV_BEST_FORM
 #undef RV_WALK
+#undef RV_WALK_ACT
+#undef RV_WALK_FORM
     JLA_CHECK_LAUNCH();
     return 0;
   }
@@ -1056,8 +1118,10 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
 #define RV_RUN(G, NT, MT, U, NORM, T) rows_gemv_kernel<G, NT, MT, 4, U, NORM, T, 4, false><<<grid, 256, 0, s>>>(q, rpg, gated)
   // (up to two workgroups per compute unit nobody else hides a wave's wait for its batch: one row of 2048 x 5632 7.9 -> 7.2 us, 2048 x 2048 4.6
   // -> 4.3; three per unit 5.3 -> 6.2)
+  const bool plain = rv_form_of(q, rpg) % RV_ONE == HY_ACT_NONE;
   if (G == 4 && nt == 1 && !p.a_norm_w && all <= 512) {
-    rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true><<<grid, 256, 0, s>>>(q, rpg, gated);
+    if (plain) rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, gated);
+    else rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true><<<grid, 256, 0, s>>>(q, rpg, gated);
     JLA_CHECK_LAUNCH();
     return 0;
   }
@@ -1088,6 +1152,8 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
     // tiles) 23.3 | 31.7 | 22.8, 4096 x 4096 9.1 | 9.3 | 8.6, 4096 x 14336 23.0 | 23.2 | 22.6; four rows of 8 experts of 2048 x 2816 12.0 | 10.9 | 13.7.
     const int mine = (p.K + 511) / 512;  // steps of a wave
     if (p.a_norm_w) RV_NT(4, 1, double);  // (at most two rows)
+    else if (nt == 2 && mine % 4 == 0 && plain) rows_gemv_kernel<4, 2, 1, 4, 4, 0, double, 4, false, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, 0);
+    else if (nt == 2 && mine % 3 == 0 && plain) rows_gemv_kernel<4, 2, 1, 4, 3, 0, double, 4, false, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, 0);
     else if (nt == 2 && mine % 4 == 0) RV_RUN(4, 2, 1, 4, 0, double);
     else if (nt == 2 && mine % 3 == 0) RV_RUN(4, 2, 1, 3, 0, double);
     else RV_NT(4, 0, double);
