@@ -3,6 +3,7 @@
 // The dispatch of every such product (hy_linear_rows), and the forms that take what no other does. In this order:
 //   a handful of output columns (a router), any rows            the vector GEMV below
 //   one or two normed rows, K <= 512, N <= 2048                 the vector GEMV below
+//   one or two rows of up to 128 numbers on bf16 weights, 64 columns and more   rows_gemv.hip (rows_short_kernel)
 //   nine to some hundred rows on bf16 weights, K a multiple of 64  rows_mid.hip, tiles of 16 to 128 rows
 //   one to 64 rows on bf16 weights otherwise, 16-byte rows      rows_gemv.hip, on the matrix cores
 //   one or two rows on fp32 weights (up to 8 with an expert each), K 512 (two rows: 1024) to 8192, 16-byte rows   rows_gemv.hip

@@ -104,16 +104,18 @@ JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
 }
 
 // FORM of a kernel: -1, any call; else one of plain rows -- in place and order, of one matrix or the table's experts -- whose results go to fp32 rows
-// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm and with RV_ONE one row per group: the branches that such a call does not take are
+// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm, with RV_MUL the gate table and with RV_ONE one row per group: the branches that such a call does not take are
 // not in its code. A launch of a few microseconds waits for the code on its path, some 0.13 us per KB. One row, weights in no cache, any call's code ->
 // its own: 2048 x 2048 8.4 -> 5.9 KB, 4.1 -> 3.7 us; 2048 x 5152 5.5 -> 3.1 KB, 6.2 -> 5.8; walking, normed 2048 x 2048 9.8 -> 3.2 KB, 4.9 -> 4.3,
 // 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096 with a residual 10.3 -> 9.5. Two rows keep any call's walk (as a loop over the rows it was
 // smaller and slower: the first weights were waited for at its edge).
-constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32;
+constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32, RV_MUL = 64;
+constexpr int RV_GATE = HY_ACT_NONE + RV_RES + RV_ONE + RV_MUL;
 template <int FORM>
 JLA_DEV void rv_form(RowLinear& p) {
   if constexpr (FORM >= 0) {
-    p.a_idx = p.dst_idx = p.offs = p.row_expert = p.mul_ids = nullptr;
+    p.a_idx = p.dst_idx = p.offs = p.row_expert = nullptr;
+    if (!(FORM & RV_MUL)) p.mul_ids = nullptr;
     p.a_scale = nullptr;
     p.out_bf16 = p.add_out = 0;
     p.act = FORM % 8;
@@ -122,8 +124,10 @@ JLA_DEV void rv_form(RowLinear& p) {
   }
 }
 static int rv_form_of(const RowLinear& p, int rows_per_group) {
-  const bool plain = !p.a_idx && !p.dst_idx && !p.offs && !p.row_expert && !p.mul_ids && !p.a_scale && !p.out_bf16 && !p.add_out;
-  return plain ? p.act + (p.res_y ? RV_RES : 0) + (p.a_norm_w ? RV_NORM : 0) + (rows_per_group == 1 || p.R == 1 ? RV_ONE : 0) : -1;
+  const bool plain = !p.a_idx && !p.dst_idx && !p.offs && !p.row_expert && !p.a_scale && !p.out_bf16 && !p.add_out;
+  return plain ? p.act + (p.res_y ? RV_RES : 0) + (p.a_norm_w ? RV_NORM : 0) + (rows_per_group == 1 || p.R == 1 ? RV_ONE : 0) +
+                     (p.mul_ids ? RV_MUL : 0)
+               : -1;
 }
 
 // output column col of linear row r from its accumulators
@@ -447,6 +451,42 @@ __global__ void __launch_bounds__(64 * WAVES) rows_gemv_kernel(RowLinear p, int 
   }
 }
 
+// v plus that of the lane whose number differs in the bits of a DPP control (quad_perm 0xb1: 1, 0x4e: 2; row_half_mirror 0x141 and row_mirror 0x140
+// pair the halves once those hold one sum)
+template <int CTRL>
+JLA_DEV double rw_add(double v) {
+  const u32x2 b = __builtin_bit_cast(u32x2, v);
+  const u32x2 o = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[0], CTRL, 0xf, 0xf, true), (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[1], CTRL, 0xf, 0xf, true)};
+  return v + __builtin_bit_cast(double, o);
+}
+
+// One or two rows of up to 128 numbers: K is one step, so a wave has whole tiles and nothing passes through LDS. What bounds it: the launch and
+// one trip to memory. 0.8 KB of code for the vector GEMV's 9: one | two rows of 2048 x 64 3.1 | 3.7 -> 2.1 | 2.2 us, 4096 x 64 3.4 | 4.1 -> 2.2 |
+// 2.3, 512 x 32 2.4 | 2.8 -> 2.0 (a launch that does nothing takes 1.9).
+constexpr int RV_SHORT_STEP = 128, RV_SHORT_NT = 2;
+__global__ void __launch_bounds__(256) rows_short_kernel(RowLinear p) {
+  rv_form<HY_ACT_NONE>(p);
+  const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4, k0 = 8 * (c % 4) + 32 * q;
+  const int T = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RV_SHORT_NT;
+  const bool in = k0 < p.K;
+  const bf16_t* w = reinterpret_cast<const bf16_t*>(p.w) + (in ? k0 : 0);
+  u32x4 wf[RV_SHORT_NT];
+#pragma unroll
+  for (int t = 0; t < RV_SHORT_NT; ++t) wf[t] = load_nt(reinterpret_cast<const u32x4*>(w + (size_t)min(4 * (T + t) + c / 4, p.N - 1) * p.K));
+  const f32x4* x = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(p.a) + (size_t)min(c / 4, p.R - 1) * p.lda + (in ? k0 : 0));
+  const u32x4 xr = in ? rv_round8(x[0], x[1]) : u32x4{0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < RV_SHORT_NT; ++t) {
+    const f32x4 d = mfma16x16x32(in ? wf[t] : u32x4{0, 0, 0, 0}, xr, f32x4{0.f, 0.f, 0.f, 0.f});
+    // lane: row c / 4, column q of the tile, K range c % 4
+    double v = rv_own<4>(d[0], d[1], d[2], d[3], c, 0);
+    v = rw_add<0xb1>(v);
+    v = rw_add<0x4e>(v);
+    const int col = 4 * (T + t) + q;
+    if (c % 4 == 0 && c / 4 < p.R && col < p.N) reinterpret_cast<float*>(p.out)[(size_t)(c / 4) * p.ldo + col] = (float)v;
+  }
+}
+
 // Linear row r as the product reads it; K <= 1024 V. Every thread of the workgroup (256)
 // holds columns 4 tid + 1024 u. load() only issues loads: the weights of the first steps are issued behind
 // them, and a wave's loads return in order. With res_y: x + rms(ysc * sum of the row's nsum rows of y) * w, in the
@@ -708,15 +748,6 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
   }
 }
 
-// v plus that of the lane whose number differs in the bits of a DPP control (quad_perm 0xb1: 1, 0x4e: 2; row_half_mirror 0x141 and row_mirror 0x140
-// pair the halves once those hold one sum)
-template <int CTRL>
-JLA_DEV double rw_add(double v) {
-  const u32x2 b = __builtin_bit_cast(u32x2, v);
-  const u32x2 o = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[0], CTRL, 0xf, 0xf, true), (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b[1], CTRL, 0xf, 0xf, true)};
-  return v + __builtin_bit_cast(double, o);
-}
-
 // One or two rows on fp32 weights, K <= 1024 V, each number multiplied as it is: a thread's numbers of the rows stay in its registers
 // (columns 4 tid + 1024 u, whole lines per wave), a workgroup walks over groups of NT weight rows (gated: gate and up alternate) with the
 // next group's loads issued as this one's are consumed, and the first group's go out ahead of the norm. What bounds it: the weight
@@ -875,7 +906,15 @@ static bool rv_takes32(const RowLinear& p) {
          aligned(p.a) && aligned(p.w) && (!p.a_norm_w || (!p.a_scale && !each && (p.a_norm_one || aligned(p.a_norm_w))));
 }
 
+// rows_short_kernel's calls: few rows as they are, one matrix, more than a few columns (a router stays on the vector unit)
+static bool rv_short(const RowLinear& p) {
+  auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
+  return p.wbf16 && !p.a_bf16 && p.R >= 1 && p.R <= RV_WALK_ROWS && p.E == 1 && !p.tab && (rv_form_of(p, p.R) & ~RV_ONE) == HY_ACT_NONE && !p.best && p.a_div <= 1 &&
+         p.K % 8 == 0 && p.K >= 8 && p.K <= RV_SHORT_STEP && p.N >= 64 && p.lda % 4 == 0 && aligned(p.a) && aligned(p.w);
+}
+
 bool hy_rows_gemv_takes(const RowLinear& p) {
+  if (rv_short(p)) return true;
   if (!p.wbf16) return rv_takes32(p);
   if (p.a_bf16 || p.out_bf16) return rv_takes16(p);
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
@@ -1031,6 +1070,12 @@ static int rv_rows32(const RowLinear& p, hipStream_t s) {
 }
 
 int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
+  if (rv_short(p)) {
+    constexpr int cols = 4 * 4 * RV_SHORT_NT;
+    rows_short_kernel<<<(p.N + cols - 1) / cols, 256, 0, s>>>(p);
+    JLA_CHECK_LAUNCH();
+    return 0;
+  }
   if (!p.wbf16) return rv_rows32(p, s);
   const int gated = hy_act_gated(p.act);
   RowLinear q = p;
@@ -1058,10 +1103,11 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   } while (0)
 #define RV_WALK(NT, U, V)                                                                     \
   do {                                                                                        \
-    const int act = form >= RV_ONE ? form % 8 : -1;                                           \
+    const int act = form >= RV_ONE && form < RV_MUL ? form % 8 : -1;                          \
     if (act == HY_ACT_NONE) RV_WALK_ACT(NT, U, V, HY_ACT_NONE);                               \
     else if (NT == 2 && act == HY_ACT_SWIGLU) RV_WALK_ACT(2, U, V, HY_ACT_SWIGLU);            \
     else if (NT == 2 && act == HY_ACT_CLAMP_GLU) RV_WALK_ACT(2, U, V, HY_ACT_CLAMP_GLU);      \
+    else if (NT == 1 && form == RV_GATE) RV_WALK_FORM(1, U, V, RV_GATE);                      \
     else RV_WALK_FORM(NT, U, V, -1);                                                          \
   } while (0)
 #define RV_BEST_FORM(U, V, F) rows_gemv_walk_kernel<2, U, V, 0, 1, F><<<grid, 256, lds, s>>>(q, rpg, gated, (int)tg, RowParts{})
@@ -1118,7 +1164,7 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
 #define RV_RUN(G, NT, MT, U, NORM, T) rows_gemv_kernel<G, NT, MT, 4, U, NORM, T, 4, false><<<grid, 256, 0, s>>>(q, rpg, gated)
   // (up to two workgroups per compute unit nobody else hides a wave's wait for its batch: one row of 2048 x 5632 7.9 -> 7.2 us, 2048 x 2048 4.6
   // -> 4.3; three per unit 5.3 -> 6.2)
-  const bool plain = rv_form_of(q, rpg) % RV_ONE == HY_ACT_NONE;
+  const bool plain = (rv_form_of(q, rpg) & ~RV_ONE) == HY_ACT_NONE;
   if (G == 4 && nt == 1 && !p.a_norm_w && all <= 512) {
     if (plain) rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, gated);
     else rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true><<<grid, 256, 0, s>>>(q, rpg, gated);

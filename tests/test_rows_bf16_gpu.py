@@ -42,6 +42,22 @@ def test_products(m, n, k):
     assert _err(hy.linear(x.float(), w), want) < _tol(k)
 
 
+@pytest.mark.parametrize("m", [1, 2])
+@pytest.mark.parametrize("n,k", [(64, 8), (65, 64), (70, 128), (2048, 64), (2050, 120), (300, 32)])
+def test_short_rows(m, n, k):
+    """One or two fp32 rows of up to 128 numbers: every product is exact in fp32, of which a lane adds 8 per fourth of the row in 24 bits (2^-24 each)."""
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    x = torch.randn(m, k + 4, generator=g, device=DEV)[:, :k]  # (rows apart)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF16)
+    want = x.to(BF16).double() @ w.double().t()
+    got = hy.linear(x, w)
+    assert got.shape == (m, n) and _err(got, want) < 32 * 2.0 ** -24
+    # a weight that is none stays in its column, also where the row ends inside the instruction's step
+    w[n - 1, k - 1] = float("inf")
+    bad = hy.linear(x, w)
+    assert torch.equal(bad[:, :-1], got[:, :-1]) and not bool(torch.isfinite(bad[:, -1]).any())
+
+
 @pytest.mark.parametrize("n,k", [(2048, 5632), (10304, 2048), (4096, 4096)])
 def test_three_and_four_rows_are_no_less_exact_than_fp32_ones_were(n, k):
     """fp32 rows, rounded in the launch, were added in 64 bits every two products: 5.5e-8 to 5.6e-8 (every four: 6.4e-8 to 7.0e-8)."""
