@@ -104,12 +104,12 @@ JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
 }
 
 // FORM of a kernel: -1, any call; else one of plain rows -- in place and order, of one matrix or the table's experts -- whose results go to fp32 rows
-// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm, with RV_MUL the gate table and with RV_ONE one row per group: the branches that such a call does not take are
+// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm, with RV_MUL the gate table, with RV_ADD onto the output and with RV_ONE one row per group: the branches that such a call does not take are
 // not in its code. A launch of a few microseconds waits for the code on its path, some 0.13 us per KB. One row, weights in no cache, any call's code ->
 // its own: 2048 x 2048 8.4 -> 5.9 KB, 4.1 -> 3.7 us; 2048 x 5152 5.5 -> 3.1 KB, 6.2 -> 5.8; walking, normed 2048 x 2048 9.8 -> 3.2 KB, 4.9 -> 4.3,
-// 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096 with a residual 10.3 -> 9.5. Two rows keep any call's walk (as a loop over the rows it was
+// 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096 with a residual 10.3 -> 9.5. A trace of eight tokens on fp32 weights 4.76 -> 4.62 ms. Two rows keep any call's walk (as a loop over the rows it was
 // smaller and slower: the first weights were waited for at its edge).
-constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32, RV_MUL = 64;
+constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32, RV_MUL = 64, RV_ADD = 128;
 constexpr int RV_GATE = HY_ACT_NONE + RV_RES + RV_ONE + RV_MUL;
 template <int FORM>
 JLA_DEV void rv_form(RowLinear& p) {
@@ -117,16 +117,17 @@ JLA_DEV void rv_form(RowLinear& p) {
     p.a_idx = p.dst_idx = p.offs = p.row_expert = nullptr;
     if (!(FORM & RV_MUL)) p.mul_ids = nullptr;
     p.a_scale = nullptr;
-    p.out_bf16 = p.add_out = 0;
+    p.out_bf16 = 0;
+    p.add_out = (FORM & RV_ADD) != 0;
     p.act = FORM % 8;
     if (!(FORM & RV_RES)) p.res_y = nullptr;
     if (!(FORM & RV_NORM)) p.a_norm_w = nullptr;
   }
 }
 static int rv_form_of(const RowLinear& p, int rows_per_group) {
-  const bool plain = !p.a_idx && !p.dst_idx && !p.offs && !p.row_expert && !p.a_scale && !p.out_bf16 && !p.add_out;
+  const bool plain = !p.a_idx && !p.dst_idx && !p.offs && !p.row_expert && !p.a_scale && !p.out_bf16;
   return plain ? p.act + (p.res_y ? RV_RES : 0) + (p.a_norm_w ? RV_NORM : 0) + (rows_per_group == 1 || p.R == 1 ? RV_ONE : 0) +
-                     (p.mul_ids ? RV_MUL : 0)
+                     (p.mul_ids ? RV_MUL : 0) + (p.add_out ? RV_ADD : 0)
                : -1;
 }
 
@@ -757,14 +758,17 @@ __global__ void __launch_bounds__(256) rows_gemv_walk_kernel(RowLinear p, int ro
 // threads' parts added by lane exchanges in 32 bits: 0.8e-7 to 1.2e-7, and 1 to 3 % slower). The same kernel on bf16 weights is as fast as the
 // matrix cores' there, not faster (normed 8224 x 2048 9.6 | 8.8, 2048 x 2048 4.2 | 4.4, 2048 x 5632 7.9 | 8.3).
 // grid and PARTS as in rows_gemv_walk_kernel; V > 4: rows as they are.
-template <int NT, int V, int RW, int PARTS>
+template <int NT, int V, int RW, int PARTS, int FORM = -1>
 __global__ void __launch_bounds__(256) rows_walk_f32_kernel(RowLinear p, int rows_per_group, int gated, int tgroups, RowParts parts) {
   static_assert(NT * RW <= 16, "sixteen threads per sum");
   __shared__ float red[2][NT * RW][256];
   __shared__ float stat[4][16];
   const int tid = threadIdx.x;
   int part = 0, tg = blockIdx.x, walk = gridDim.x;
+  rv_form<FORM>(p);
+  if constexpr (FORM >= 0) gated = !PARTS && hy_act_gated(FORM % 8);
   if constexpr (PARTS) {
+    if constexpr (FORM >= 0) p.tab = nullptr;
     while (part + 1 < parts.n && tg >= parts.first[part + 1]) ++part;
     tg -= parts.first[part];
     walk = parts.first[part + 1] - parts.first[part];
@@ -909,7 +913,7 @@ static bool rv_takes32(const RowLinear& p) {
 // rows_short_kernel's calls: few rows as they are, one matrix, more than a few columns (a router stays on the vector unit)
 static bool rv_short(const RowLinear& p) {
   auto aligned = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-  return p.wbf16 && !p.a_bf16 && p.R >= 1 && p.R <= RV_WALK_ROWS && p.E == 1 && !p.tab && (rv_form_of(p, p.R) & ~RV_ONE) == HY_ACT_NONE && !p.best && p.a_div <= 1 &&
+  return p.wbf16 && !p.a_bf16 && p.R >= 1 && p.R <= RV_WALK_ROWS && p.E == 1 && !p.tab && rv_form_of(p, p.R) >= 0 && (rv_form_of(p, p.R) & ~RV_ONE) == HY_ACT_NONE && !p.best && p.a_div <= 1 &&
          p.K % 8 == 0 && p.K >= 8 && p.K <= RV_SHORT_STEP && p.N >= 64 && p.lda % 4 == 0 && aligned(p.a) && aligned(p.w);
 }
 
@@ -962,10 +966,10 @@ int hy_rows_parts(const RowLinear& p, const RowParts& parts, hipStream_t s) {
   const dim3 grid(t.first[t.n], 1);
   if (!p.wbf16) {
     if (p.K <= 2048) {
-      if (p.R == 1) rows_walk_f32_kernel<4, 2, 1, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+      if (p.R == 1) rows_walk_f32_kernel<4, 2, 1, 1, RV_NORM><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
       else rows_walk_f32_kernel<4, 2, 2, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
     } else if (p.R == 1) {
-      rows_walk_f32_kernel<2, 4, 1, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
+      rows_walk_f32_kernel<2, 4, 1, 1, RV_NORM><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
     } else {
       rows_walk_f32_kernel<2, 4, 2, 1><<<grid, 256, 0, s>>>(p, p.R, 0, 0, t);
     }
@@ -1012,7 +1016,12 @@ static int rv_rows16(const RowLinear& p, int rows, int groups, int gated, hipStr
   const long long wgs = (tiles + nt - 1) / nt;
   if (wgs > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)wgs, groups);
-#define RV_RUN16(G, NT, U, PIPE) rows_gemv_kernel<G, NT, 1, 4, U, 0, double, 2, PIPE><<<grid, 256, 0, s>>>(p, p.R, gated)
+  const bool plain = rv_form_of(p, p.R) >= 0 && (rv_form_of(p, p.R) & ~RV_ONE) == HY_ACT_NONE;
+#define RV_RUN16(G, NT, U, PIPE)                                                                                              \
+  do {                                                                                                                        \
+    if (plain) rows_gemv_kernel<G, NT, 1, 4, U, 0, double, 2, PIPE, HY_ACT_NONE><<<grid, 256, 0, s>>>(p, p.R, gated);          \
+    else rows_gemv_kernel<G, NT, 1, 4, U, 0, double, 2, PIPE><<<grid, 256, 0, s>>>(p, p.R, gated);                             \
+  } while (0)
   if (G == 4) {
     if (nt == 2) RV_RUN16(4, 2, 4, true);
     else RV_RUN16(4, 4, 4, false);
@@ -1040,6 +1049,34 @@ static int rv_rows32(const RowLinear& p, hipStream_t s) {
   if (tg > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
 #define RV_RUN32(NT, V, RW) rows_walk_f32_kernel<NT, V, RW, 0><<<grid, 256, 0, s>>>(p, rpg, gated, (int)tg, RowParts{})
+// (one row: the forms of this file's first comment on them, for the activations and additions that a decode step has)
+#define RV_FORM32(NT, V, F)                                                                                        \
+  if (form == (F)) {                                                                                               \
+    rows_walk_f32_kernel<NT, V, 1, 0, F><<<grid, 256, 0, s>>>(p, rpg, gated, (int)tg, RowParts{});                 \
+    break;                                                                                                         \
+  }
+#define RV_ASIS32(NT, V)                 \
+  RV_FORM32(NT, V, HY_ACT_NONE)          \
+  RV_FORM32(NT, V, HY_ACT_NONE + RV_ADD)
+#define RV_ONE32(NT, V)                                          \
+  do {                                                           \
+    RV_ASIS32(NT, V)                                             \
+    RV_FORM32(NT, V, HY_ACT_NONE + RV_RES)                       \
+    RV_FORM32(NT, V, HY_ACT_NONE + RV_NORM)                      \
+    RV_FORM32(NT, V, HY_ACT_SOFTCAP + RV_NORM)                   \
+    RV_FORM32(NT, V, HY_ACT_NONE + RV_RES + RV_NORM)             \
+    if constexpr (NT > 1) {                                      \
+      RV_FORM32(NT, V, HY_ACT_SWIGLU + RV_RES)                   \
+      RV_FORM32(NT, V, HY_ACT_CLAMP_GLU + RV_NORM)               \
+    }                                                            \
+    RV_RUN32(NT, V, 1);                                          \
+  } while (0)
+#define RV_LONE32(NT, V)  \
+  do {                    \
+    RV_ASIS32(NT, V)      \
+    RV_RUN32(NT, V, 1);   \
+  } while (0)
+  const int form = rpg == 1 && rv_form_of(p, 1) >= 0 ? rv_form_of(p, 1) & ~RV_ONE : -1;
 #define RV_SHORT32(V)                   \
   do {                                  \
     if (nt == 2) {                      \
@@ -1053,15 +1090,24 @@ static int rv_rows32(const RowLinear& p, hipStream_t s) {
   } while (0)
 #define RV_LONG32(V)                    \
   do {                                  \
-    if (nt == 1) RV_RUN32(1, V, 1);     \
-    else if (rpg == 1) RV_RUN32(2, V, 1); \
+    if (rpg == 1) RV_RUN32(2, V, 1);    \
     else RV_RUN32(2, V, 2);             \
   } while (0)
   if (p.K <= 1024) RV_SHORT32(1);
+  else if (p.K <= 2048 && rpg == 1 && nt == 2) RV_ONE32(2, 2);
+  else if (p.K <= 2048 && rpg == 1) RV_ONE32(4, 2);
   else if (p.K <= 2048) RV_SHORT32(2);
-  else if (p.K <= 4096) RV_LONG32(4);
+  else if (p.K <= 4096 && nt == 1) RV_ONE32(1, 4);
+  else if (p.K <= 4096 && rpg == 1) RV_ONE32(2, 4);
+  else if (p.K <= 4096) RV_RUN32(2, 4, 2);
+  else if (p.K <= 6144 && nt == 1) RV_LONE32(1, 6);
   else if (p.K <= 6144) RV_LONG32(6);
+  else if (nt == 1) RV_LONE32(1, 8);
   else RV_LONG32(8);
+#undef RV_LONE32
+#undef RV_ONE32
+#undef RV_ASIS32
+#undef RV_FORM32
 #undef RV_LONG32
 #undef RV_SHORT32
 #undef RV_RUN32
@@ -1164,13 +1210,15 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
 #define RV_RUN(G, NT, MT, U, NORM, T) rows_gemv_kernel<G, NT, MT, 4, U, NORM, T, 4, false><<<grid, 256, 0, s>>>(q, rpg, gated)
   // (up to two workgroups per compute unit nobody else hides a wave's wait for its batch: one row of 2048 x 5632 7.9 -> 7.2 us, 2048 x 2048 4.6
   // -> 4.3; three per unit 5.3 -> 6.2)
-  const bool plain = (rv_form_of(q, rpg) & ~RV_ONE) == HY_ACT_NONE;
+  const int form = rv_form_of(q, rpg) < 0 ? -1 : rv_form_of(q, rpg) & ~RV_ONE;
   if (G == 4 && nt == 1 && !p.a_norm_w && all <= 512) {
-    if (plain) rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, gated);
+    if (form == HY_ACT_NONE) rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, gated);
+    else if (form == HY_ACT_NONE + RV_ADD) rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true, HY_ACT_NONE + RV_ADD><<<grid, 256, 0, s>>>(q, rpg, gated);
     else rows_gemv_kernel<4, 1, 1, 4, 4, 0, double, 4, true><<<grid, 256, 0, s>>>(q, rpg, gated);
     JLA_CHECK_LAUNCH();
     return 0;
   }
+#define RV_PLAIN(U, F) rows_gemv_kernel<4, 2, 1, 4, U, 0, double, 4, false, F><<<grid, 256, 0, s>>>(q, rpg, 0)
 #define RV_NT(G, NORM, T)                     \
   do {                                        \
     if (nt == 1) RV_RUN(G, 1, 1, 4, NORM, T);  \
@@ -1198,8 +1246,10 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
     // tiles) 23.3 | 31.7 | 22.8, 4096 x 4096 9.1 | 9.3 | 8.6, 4096 x 14336 23.0 | 23.2 | 22.6; four rows of 8 experts of 2048 x 2816 12.0 | 10.9 | 13.7.
     const int mine = (p.K + 511) / 512;  // steps of a wave
     if (p.a_norm_w) RV_NT(4, 1, double);  // (at most two rows)
-    else if (nt == 2 && mine % 4 == 0 && plain) rows_gemv_kernel<4, 2, 1, 4, 4, 0, double, 4, false, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, 0);
-    else if (nt == 2 && mine % 3 == 0 && plain) rows_gemv_kernel<4, 2, 1, 4, 3, 0, double, 4, false, HY_ACT_NONE><<<grid, 256, 0, s>>>(q, rpg, 0);
+    else if (nt == 2 && mine % 4 == 0 && form == HY_ACT_NONE) RV_PLAIN(4, HY_ACT_NONE);
+    else if (nt == 2 && mine % 4 == 0 && form == HY_ACT_NONE + RV_ADD) RV_PLAIN(4, HY_ACT_NONE + RV_ADD);
+    else if (nt == 2 && mine % 3 == 0 && form == HY_ACT_NONE) RV_PLAIN(3, HY_ACT_NONE);
+    else if (nt == 2 && mine % 3 == 0 && form == HY_ACT_NONE + RV_ADD) RV_PLAIN(3, HY_ACT_NONE + RV_ADD);
     else if (nt == 2 && mine % 4 == 0) RV_RUN(4, 2, 1, 4, 0, double);
     else if (nt == 2 && mine % 3 == 0) RV_RUN(4, 2, 1, 3, 0, double);
     else RV_NT(4, 0, double);
@@ -1212,6 +1262,7 @@ int hy_rows_gemv(const RowLinear& p, hipStream_t s) {
   }
 #undef RV_16
 #undef RV_NT
+#undef RV_PLAIN
 #undef RV_RUN
   JLA_CHECK_LAUNCH();
   return 0;
