@@ -3,28 +3,29 @@
 // generation.py:28-41 with do_sample = temperature != 0, top_k = 50).
 //
 // Two kernels, no host sync, hipGraph-capturable:
-//   topk_chunk:  grid (ceil(V/4096), B). A 256-thread workgroup holds a 4096-logit chunk in
-//                registers (16 keys per thread, order-preserving uint32 of the fp32 logit) and finds
-//                the chunk's K-th largest key by 4-pass LDS radix select (8 bits per pass, one wave
-//                scans the 256-bin histogram with lane moves). It emits exactly K candidates:
-//                everything above the threshold plus the lowest-index ties.
-//   topk_merge:  one workgroup per row merges the C = chunks*K candidates the same way, sorts the K
-//                survivors in one wave (64-lane bitonic network on (key, -index)), and either writes
+//   topk_chunk:  grid (ceil(V/4096), B). A 256-thread workgroup holds a 4096-logit chunk in registers (16 keys per thread,
+//                order-preserving uint32 of the fp32 logit, whole lines per load). A bound that at least K keys reach comes from the
+//                threads' maxima (LDS radix select, 8 bits per pass, one wave scans the 256-bin histogram with lane moves, two passes);
+//                the survivors, about K, rank themselves by counting the better ones. It emits exactly K candidates, sorted.
+//   topk_merge:  one workgroup per row ranks the C = chunks*K candidates the same way, and either writes
 //                them (vocab-parallel TP: each rank's top-K is all-gathered, 400 B per rank per row,
 //                then merged again -- exact, since the global top-K is inside the union) or samples:
 //                temperature, top-p over the sorted survivors (HF keep rule: a token survives if the
 //                probability mass strictly before it is < top_p; the first always survives), then
 //                Gumbel-max with counter-based Philox4x32-10 keyed by (seed, step, row, rank) -- every
 //                TP rank draws the same token from the same candidates without communicating.
+// More survivors than threads (flat, tied or clustered keys): the exact select on all keys of the chunk.
 // Ties: lower vocabulary index first (lax.top_k order).
-// What bounds it: dependent steps within a wave (scans of up to eight radix passes, 21 exchanges of the sort). With lane moves in the place of
-// shuffles through LDS the two kernels take 20 us of seven rows x 128256 columns, 23 before.
+// What bounds it: dependent steps within a wave and code on its path (some 0.13 us per KB in a launch of a few us). Seven rows x 128256 columns, the
+// two kernels: 64 keys per thread in 8 chunks, read 256 bytes apart, exact select and sort of the survivors in six radix passes and 21 exchanges
+// 10.9 + 8.9 us; here 6.2 + 9.4. Warm, both, before -> now: 1 row 17.7 -> 14.7, 7 18.0 -> 15.1, 64 20.9 -> 20.7, 300 42.0 -> 44.5, 1400 186 -> 184;
+// 200 x 32000 22.8 -> 19.5. (32 keys per thread: 7 rows 16.0, 1400 302; the rare case's keys in registers: 1400 203.)
 #include "common.h"
 #include "launchers.h"
 
 namespace jla {
 
-constexpr int TK_THREADS = 256, TK_E = 64, TK_CHUNK = TK_THREADS * TK_E;
+constexpr int TK_THREADS = 256, TK_E = 16, TK_CHUNK = TK_THREADS * TK_E, TK_MAX_E = 64;
 
 JLA_DEV uint32_t fkey(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -36,28 +37,26 @@ struct TkShared {
   uint32_t hist[256];
   uint32_t wsum[TK_THREADS / 64];
   uint32_t sel[2];
-  uint32_t sk[64];  // merge: compacted survivors
-  int32_t si[64];
-  uint32_t ck[TK_THREADS];  // chunk: prefiltered candidates (key, element index), in element order
-  int32_t cj[TK_THREADS];
+  uint64_t c[TK_THREADS];   // survivors: key, then the index from its end (the better of two is the larger)
   uint32_t total;
 };
 
-// Block-wide radix select over TK_E keys per thread: T = the K-th largest key; need_eq = how many
+// Block-wide radix select over E keys per thread, key(j) the j-th: T = the K-th largest key; need_eq = how many
 // keys equal to T are part of the top K (all keys > T are). Requires K <= number of keys.
 // last_shift 16: two passes only, T = the K-th largest key with its low 16 bits cleared (a lower bound with at least K
 // keys >= T; need_eq is then meaningless).
-template <int E>
-JLA_DEV void radix_select(const uint32_t (&key)[E], int K, TkShared& sh, uint32_t& T, int& need_eq,
-                          int last_shift = 0) {
+template <class Key>
+JLA_DEV void radix_select(int E, Key key, int K, TkShared& sh, uint32_t& T, int& need_eq, int last_shift = 0) {
   uint32_t prefix = 0, mask = 0;
   int kr = K;
   for (int shift = 24; shift >= last_shift; shift -= 8) {
     for (int i = threadIdx.x; i < 256; i += TK_THREADS) sh.hist[i] = 0;
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < E; ++j)
-      if ((key[j] & mask) == prefix) atomicAdd(&sh.hist[(key[j] >> shift) & 255u], 1u);
+#pragma unroll 1
+    for (int j = 0; j < E; ++j) {
+      const uint32_t k = key(j);
+      if ((k & mask) == prefix) atomicAdd(&sh.hist[(k >> shift) & 255u], 1u);
+    }
     __syncthreads();
     if (threadIdx.x < 64) {
       const int l = threadIdx.x;
@@ -102,89 +101,83 @@ JLA_DEV uint32_t block_excl_scan(uint32_t v, TkShared& sh) {
   return base + incl - v;
 }
 
-// Emit exactly K (key, index) pairs: keys > T in thread-major order, then the first need_eq keys == T.
-template <int E, typename F>
-JLA_DEV void emit_topk(const uint32_t (&key)[E], uint32_t T, int need_eq, int K, TkShared& sh, F&& put) {
-  uint32_t ngt = 0, neq = 0;
+JLA_DEV uint64_t tk_word(uint32_t key, int idx) { return (uint64_t)key << 32 | (uint32_t)(0x7fffffff - idx); }
+
+// The top K of the block's keys, sorted, where few enough reach the bound: calls put(slot, word) once per slot 0..K-1. word(j): key j's and its index
+// (0 .. 0x7fffffff). The bound: the top 16 bits (sign, exponent, 7 mantissa bits) of the K-th largest of the 256 per-thread maxima; at least K keys
+// reach it, and about that many of logits. False: more than threads.
+template <int E, class Word, class F>
+JLA_DEV bool select_few(const uint32_t (&key)[E], int K, TkShared& sh, Word word, F put, bool over = false) {
+  uint32_t most = 0, T0, ns = 0;
+  int none;
 #pragma unroll
+  for (int j = 0; j < E; ++j) most = max(most, key[j]);
+  radix_select(1, [&](int) { return most; }, K, sh, T0, none, 16);
+#pragma unroll
+  for (int j = 0; j < E; ++j) ns += key[j] >= T0;
+  uint32_t at = block_excl_scan(ns, sh);
+  if (threadIdx.x == TK_THREADS - 1) sh.total = at + ns;
+  __syncthreads();
+  const int S = sh.total;
+  if (S > TK_THREADS) return false;
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (key[j] >= T0) sh.c[at++] = word(j);
+  if ((int)threadIdx.x >= S && threadIdx.x < ((S + 3) & ~3)) sh.c[threadIdx.x] = 0;  // (better than none)
+  __syncthreads();
+  int rank = K;
+  uint64_t own = 0;
+  if ((int)threadIdx.x < S) {
+    own = sh.c[threadIdx.x];
+    rank = 0;
+    for (int i = 0; i < S; i += 4) {
+      uint64_t o[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o[u] = sh.c[i + u];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) rank += o[u] > own || (o[u] == own && i + u < (int)threadIdx.x);
+    }
+  }
+  if (over) __syncthreads();  // (put writes where others read)
+  if (rank < K) put(rank, own);
+  return true;
+}
+
+// ... of any keys, E neighbouring ones per thread, key(j) this thread's j-th: put(slot, key, j), slots above the threshold in element order, then
+// the lowest elements at it. (The keys are read again for every pass: the rare case takes no registers from the other.)
+template <class Key, class F>
+JLA_DEV void select_all(int E, Key key, int K, TkShared& sh, F put) {
+  uint32_t T, ngt = 0, neq = 0;
+  int need_eq;
+  radix_select(E, key, K, sh, T, need_eq);
+#pragma unroll 1
   for (int j = 0; j < E; ++j) {
-    ngt += key[j] > T;
-    neq += key[j] == T;
+    const uint32_t k = key(j);
+    ngt += k > T;
+    neq += k == T;
   }
   const uint32_t ex = block_excl_scan((ngt << 16) | neq, sh);
   int gpos = ex >> 16, epos = ex & 0xffff;
-  const int count_gt = K - need_eq;
-#pragma unroll
+#pragma unroll 1
   for (int j = 0; j < E; ++j) {
-    if (key[j] > T) {
-      put(gpos++, j);
-    } else if (key[j] == T) {
-      if (epos < need_eq) put(count_gt + epos, j);
-      ++epos;
-    }
+    const uint32_t k = key(j);
+    if (k > T) put(gpos++, k, j);
+    else if (k == T && epos++ < need_eq) put(K - need_eq + epos - 1, k, j);
   }
 }
 
-// Exact top K of the block's TK_CHUNK keys (thread t holds elements base .. base + TK_E - 1; key 0 = padding past
-// n_valid), calling put(slot, key, element) once per slot 0..K-1 (ties at the threshold keep the lowest elements).
-// Prefilter: T0 = the K-th largest of the 256 per-thread maxima (bound_shift 16: its top 16 bits). At least K keys are >= T0, so the top
-// K are all >= T0; on logits only ~K keys survive, and the exact select runs on the survivors, one per thread (256
-// LDS-histogram adds per radix pass instead of TK_CHUNK that pile onto the few hot exponent bins). More survivors
-// than threads (flat, tied or clustered keys): the full TK_E-keys-per-thread select.
-template <int E, typename F>
-JLA_DEV void select_topk(const uint32_t (&key)[E], int base, int n_valid, int K, TkShared& sh, F&& put,
-                         int bound_shift = 0) {
-  uint32_t tmax = 0;
-#pragma unroll
-  for (int j = 0; j < E; ++j) tmax = max(tmax, key[j]);
-  uint32_t T0;
-  int ne0;
-  {
-    const uint32_t k1[1] = {tmax};
-    radix_select(k1, K, sh, T0, ne0, bound_shift);  // a bound is enough
-  }
-  uint32_t ns = 0;
-#pragma unroll
-  for (int j = 0; j < E; ++j) ns += key[j] >= T0;
-  const uint32_t pos = block_excl_scan(ns, sh);
-  if (threadIdx.x == TK_THREADS - 1) sh.total = pos + ns;
-  __syncthreads();
-  const uint32_t S = sh.total;
-  uint32_t T;
-  int need_eq;
-  if (S <= (uint32_t)TK_THREADS) {
-    uint32_t r = pos;
-#pragma unroll
-    for (int j = 0; j < E; ++j)
-      if (key[j] >= T0) {  // compacted in element order (thread-major, j ascending): ties keep index order
-        sh.ck[r] = key[j];
-        sh.cj[r] = base + j;
-        ++r;
-      }
-    __syncthreads();
-    const bool have = threadIdx.x < S;
-    const uint32_t k1[1] = {have ? sh.ck[threadIdx.x] : 0u};
-    const int e1 = have ? sh.cj[threadIdx.x] : n_valid;
-    radix_select(k1, K, sh, T, need_eq);
-    emit_topk(k1, T, need_eq, K, sh, [&](int slot, int) { put(slot, k1[0], e1); });
-    return;
-  }
-  radix_select(key, K, sh, T, need_eq);
-  emit_topk(key, T, need_eq, K, sh, [&](int slot, int j) { put(slot, key[j], base + j); });
-}
-
-__global__ void __launch_bounds__(TK_THREADS)
+__global__ void __launch_bounds__(TK_THREADS, 8)
     topk_chunk_kernel(const float* __restrict__ logits, int V, int K, int idx_offset, float* __restrict__ cv,
                       int32_t* __restrict__ ci) {
   __shared__ TkShared sh;
-  const int b = blockIdx.y, c = blockIdx.x, nch = gridDim.x;
-  const int base = c * TK_CHUNK + threadIdx.x * TK_E;
+  const int b = blockIdx.y, c = blockIdx.x, nch = gridDim.x, base = c * TK_CHUNK;
   const float* x = logits + (size_t)b * V;
   uint32_t key[TK_E];
-  if ((V & 3) == 0 && base + TK_E <= V) {
+  auto element = [&](int j) { return base + 4 * TK_THREADS * (j / 4) + 4 * (int)threadIdx.x + j % 4; };
+  if ((V & 3) == 0 && base + TK_CHUNK <= V) {
 #pragma unroll
     for (int q = 0; q < TK_E / 4; ++q) {
-      const float4 v = reinterpret_cast<const float4*>(x + base)[q];
+      const float4 v = *reinterpret_cast<const float4*>(x + element(4 * q));
       key[4 * q] = fkey(v.x);
       key[4 * q + 1] = fkey(v.y);
       key[4 * q + 2] = fkey(v.z);
@@ -192,16 +185,20 @@ __global__ void __launch_bounds__(TK_THREADS)
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < TK_E; ++j) key[j] = base + j < V ? fkey(x[base + j]) : 0u;  // 0 < key(-inf)
+    for (int j = 0; j < TK_E; ++j) key[j] = element(j) < V ? fkey(x[element(j)]) : 0u;  // 0 < key(-inf)
   }
   float* ov = cv + ((size_t)b * nch + c) * K;
   int32_t* oi = ci + ((size_t)b * nch + c) * K;
-  // logits: the top 16 bits (sign, exponent, 7 mantissa bits) of the bound admit ~K survivors; two radix passes saved
-  select_topk(key, base, V, K, sh, [&](int slot, uint32_t k, int e) {
-    const bool valid = e < V;
-    ov[slot] = valid ? kfloat(k) : -INFINITY;
-    oi[slot] = valid ? idx_offset + e : 0x7fffffff;
-  }, 16);
+  auto put = [&](int slot, uint32_t k, int e) {
+    ov[slot] = e < V ? kfloat(k) : -INFINITY;
+    oi[slot] = e < V ? idx_offset + e : 0x7fffffff;
+  };
+  if (select_few(key, K, sh, [&](int j) { return tk_word(key[j], element(j)); },
+                 [&](int slot, uint64_t w) { put(slot, (uint32_t)(w >> 32), 0x7fffffff - (int)(uint32_t)w); }))
+    return;
+  const int first = base + TK_E * (int)threadIdx.x;  // (in element order now)
+  __syncthreads();
+  select_all(TK_E, [&](int j) { return first + j < V ? fkey(x[first + j]) : 0u; }, K, sh, [&](int slot, uint32_t k, int j) { put(slot, k, first + j); });
 }
 
 JLA_DEV uint4 philox4x32_10(uint4 ctr, uint2 k) {
@@ -228,31 +225,42 @@ __global__ void __launch_bounds__(TK_THREADS)
                       const int32_t* __restrict__ step) {
   __shared__ TkShared sh;
   const int b = blockIdx.x;
-  const int base = threadIdx.x * E;
+  const float* bv = cv + (size_t)b * C;
+  const int32_t* bi = ci + (size_t)b * C;
   uint32_t key[E];
+  int32_t at[E];
 #pragma unroll
-  for (int j = 0; j < E; ++j) key[j] = base + j < C ? fkey(cv[(size_t)b * C + base + j]) : 0u;
-  select_topk(key, base, C, K, sh, [&](int slot, uint32_t k, int e) {
-    sh.sk[slot] = k;
-    sh.si[slot] = e < C ? ci[(size_t)b * C + e] : 0x7fffffff;
-  });
+  for (int j = 0; j < E; ++j) {  // (a chunk's candidates are sorted: dealt out, so that the threads' maxima are the row's best)
+    const int e = threadIdx.x + TK_THREADS * j;
+    key[j] = e < C ? fkey(bv[e]) : 0u;
+    at[j] = e < C ? bi[e] : 0x7fffffff;
+  }
+  const bool few = select_few(key, K, sh, [&](int j) { return tk_word(key[j], at[j]); }, [&](int slot, uint64_t w) { sh.c[slot] = w; }, true);
+  if (!few) {
+    const int base = threadIdx.x * E;
+    __syncthreads();
+    select_all(E, [&](int j) { return base + j < C ? fkey(bv[base + j]) : 0u; }, K, sh,
+               [&](int slot, uint32_t k, int j) { sh.c[slot] = tk_word(k, base + j < C ? bi[base + j] : 0x7fffffff); });
+  }
   __syncthreads();
   if (threadIdx.x >= 64) return;
   const int lane = threadIdx.x;
-  // composite sort key: value descending, then index ascending
-  uint64_t v = lane < K ? ((uint64_t)sh.sk[lane] << 32) | (uint32_t)(0x7fffffff - sh.si[lane]) : 0ull;
+  // value descending, then index ascending
+  uint64_t v = lane < K ? sh.c[lane] : 0ull;
+  if (!few) {
 #pragma unroll
-  for (int k = 2; k <= 64; k <<= 1) {
-    lane_halves([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      if (j >= k) return;
-      const uint32_t lo = lane_xor<j>((uint32_t)v), hi = lane_xor<j>((uint32_t)(v >> 32));
-      const uint64_t o = ((uint64_t)hi << 32) | lo;
-      const bool desc = (lane & k) == 0;  // final k = 64: whole wave descending
-      const bool lower = (lane & j) == 0;
-      const bool take_max = desc == lower;
-      v = take_max ? (o > v ? o : v) : (o < v ? o : v);
-    });
+    for (int k = 2; k <= 64; k <<= 1) {
+      lane_halves([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        if (j >= k) return;
+        const uint32_t lo = lane_xor<j>((uint32_t)v), hi = lane_xor<j>((uint32_t)(v >> 32));
+        const uint64_t o = ((uint64_t)hi << 32) | lo;
+        const bool desc = (lane & k) == 0;  // final k = 64: whole wave descending
+        const bool lower = (lane & j) == 0;
+        const bool take_max = desc == lower;
+        v = take_max ? (o > v ? o : v) : (o < v ? o : v);
+      });
+    }
   }
   const float val = lane < K ? kfloat((uint32_t)(v >> 32)) : -INFINITY;
   const int32_t idx = lane < K ? 0x7fffffff - (int32_t)(uint32_t)v : 0x7fffffff;
@@ -309,7 +317,7 @@ int topk_chunk(const float* logits, int B, int V, int K, int idx_offset, float* 
 int topk_merge(const float* cv, const int32_t* ci, int B, int C, int K, int mode, float* out_v, int32_t* out_i,
                int32_t* nxt, float temperature, float top_p, uint64_t seed, const int32_t* step, hipStream_t s) {
   if (B <= 0) return 0;
-  if (K < 1 || K > 64 || K > C || C > TK_CHUNK) return -1;
+  if (K < 1 || K > 64 || K > C || C > TK_THREADS * TK_MAX_E) return -1;
   if (mode == 1 && (!nxt || !step || !(temperature > 0.f))) return -2;
 #define JLA_TKM(E)                                                                                          \
   topk_merge_kernel<E><<<B, TK_THREADS, 0, s>>>(cv, ci, C, K, mode, out_v, out_i, nxt, 1.0f / temperature, top_p, \
@@ -321,7 +329,7 @@ int topk_merge(const float* cv, const int32_t* ci, int B, int C, int K, int mode
   else if (C <= 16 * TK_THREADS)
     JLA_TKM(16);
   else
-    JLA_TKM(TK_E);
+    JLA_TKM(TK_MAX_E);
 #undef JLA_TKM
   JLA_CHECK_LAUNCH();
   return 0;

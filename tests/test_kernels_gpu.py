@@ -586,6 +586,16 @@ def test_topk_candidates_exact(b, v, k):
     assert torch.equal(gv.cpu(), rv)
 
 
+@pytest.mark.parametrize("v", [64, 255, 1023, 4095, 4096, 4097, 4100, 8191, 12352])
+def test_topk_candidates_at_chunk_edges(v):
+    """Rows that end inside, at or just behind a chunk of 4096, unaligned ones too; equal numbers across the edge; as many as a whole wave."""
+    logits = torch.randn(2, v, generator=torch.Generator().manual_seed(v)) * 4
+    logits[1, max(0, min(v, 4096) - 3):4100] = logits[1].max() + 1
+    gv, gi = ops.topk_candidates(logits.to(DEV), 64)
+    rv, ri = ref.topk_sorted(logits, 64)
+    assert torch.equal(gi.cpu(), ri) and torch.equal(gv.cpu(), rv)
+
+
 @pytest.mark.parametrize("case", ["block", "flat", "ties"])
 def test_topk_candidates_prefilter_fallbacks(case):
     """Chunks whose survivors of the per-thread-maximum prefilter exceed one per thread (a run of 300 large
