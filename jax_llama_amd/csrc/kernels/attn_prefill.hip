@@ -191,10 +191,12 @@ __global__ void __launch_bounds__(256)
 //                  registers used in place with the permuted k order of the accumulator layout): 4 d tiles x
 //                  4 key steps = 16 MFMAs. O^T again has the query on the lane, so the rescale by
 //                  exp2(m_old - m_new) is lane-local too.
-// K/V tiles are register-staged (loads for tile t+1 issued before tile t's MFMAs, written to LDS after
-// the barrier that ends tile t). Causal: the workgroup stops at its last query's slot; a wave whose
-// queries all precede a tile skips its MFMAs; only tiles that cross the diagonal, kv_start or T are
-// masked element-wise. Each workgroup runs a heavy and a light query block (causal balance).
+// K/V tiles come by LDS-DMA into two slots each (64 KiB per workgroup): K(i+1) and V(i) are there during tile i while
+// K(i+2) and V(i+1) go into the slots that tile i-1 was done with, so a tile ends with ONE wait and barrier. The DMA is
+// inline asm: with the builtin, hipcc waits for the DMA of the next tiles before the first V read of a tile.
+// Causal: the workgroup stops at its last query's slot; a wave whose queries all precede a tile skips its MFMAs; only
+// tiles that cross the diagonal, kv_start or T are masked element-wise. Each workgroup runs a heavy and a light query
+// block (causal balance).
 constexpr int FA_KT = 64;  // keys per tile
 
 // byte offset of 16-byte chunk ch (0..15) of row `row` in a [rows][128 bf16] image whose XOR swizzle
@@ -216,33 +218,28 @@ JLA_DEV u32x2 ld_tr(const char* lds, int off) {
 // One query block of 32 per wave (a 64-query "QB = 2" form halved the LDS bytes per MFMA but needed ~340 registers,
 // one workgroup per CU, and ran 1.4-2x slower: profiles/r2_attn_prefill_qb2_ab.jsonl -- removed).
 //
-// PIPE: the scores of tile i+1 are issued before the softmax of tile i, so one wave's MFMA pipe works
-// through S(i+1) while its VALU runs exp / sum / pack of tile i (independent instructions in one basic block).
-// K and V each get a 2-slot LDS ring (64 KiB per workgroup): K(i+1) and V(i) are resident during tile i while
-// the registers stage K(i+2) and V(i+1) into the slots freed by tile i-1, so each tile ends with ONE barrier.
+// What bounds it: the matrix pipe (1024 cycles a tile and wave) and the VALU (about 900: 32 exp at a quarter of the
+// rate, fma, sum, pack, max) of a wave take turns unless the code puts independent work of both next to each other: two
+// waves per SIMD in step with each other don't. So all of a tile is in the fixed order of `tile`: an MFMA, then one
+// element's exp of the NEXT key step, then an LDS read, ten times a key step (sched_group_barrier); the scores of tile
+// i+1 are spread over key steps 0..2 of tile i, its max stands beside the PV MFMAs of key step 3, and only the P of its
+// first key step has no MFMA beside it. The max exchange of the two lane halves is a permlane32 swap, the halves of the
+// sum meet once at the end, two tiles are unrolled (constant LDS slots, no scores moved), and the masks take a lane's
+// two limits instead of 32 key indexes held in registers.
+// Measured (32 heads, 8 kv heads of 128, causal): S = 8192 604 -> 496 us (1.1 PFLOP/s), 16 x 2048 735 -> 623 us,
+// S = 2048 62.5 -> 50.7, S = 600 with 32 kv heads 26.3 -> 20.0, 2048 x 128 1411 -> 1325 us.
 // Lazy rescale (every launch): the running max (and with it the O / l rescale) moves only when a lane's tile max
 // exceeds it by more than 8 (log2 units): exp2 of the rest stays <= 256, exact in fp32 and bf16-representable for P;
 // the 64 O multiplies per tile run only in a wave-uniform branch when some lane needs them (mostly the first tiles).
-// (The eager-rescale launches, impls 4 / 5 / 6 / 10, were slower everywhere and removed in round 4:
-// profiles/r3_attn_prefill_pipe_ab.jsonl, profiles/r4_variant_pruning.md.)
-// PIPE 2: the same loop with the K / V DMA as inline asm (glds16_asm: with the builtin, hipcc put a vmcnt(0) before
-// the first V read of every tile, i.e. waited for the DMA of the NEXT tiles it had just issued), and branch-free, with
-// the next tile's 16 scores MFMAs spread over the 4 key steps (4 per step, fenced by sched_barrier) beside the exps and
-// PV MFMAs instead of sunk into one serial read -> wait -> MFMA chain at the end of the tile.
-template <int NW, int PIPE>
+template <int NW>
 __global__ void __launch_bounds__(NW * 64, 2)
     attn_prefill_v2_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
                            const int32_t* __restrict__ slot_ptr, const int32_t* __restrict__ kv_start,
                            const uint8_t* __restrict__ key_mask, int mask_len, bf16_t* __restrict__ out, int S, int H,
                            int Hkv, int T, float scale_log2, int npb, int hgroups, int n_qb, int split) {
-  constexpr int QB = 1;  // query blocks of 32 per wave
-  constexpr int NT = NW * 64;
   constexpr int TILE_BYTES = FA_KT * AP_DH * 2;            // 16 KiB
-  constexpr int CH_PER_T = FA_KT * 16 / NT;                 // 16-byte chunks per thread per tile (K or V)
-  constexpr int QW = 32 * QB;                               // queries per wave
-  __shared__ __attribute__((aligned(16))) char lds[(PIPE ? 4 : 2) * TILE_BYTES];
-  char* Ks = lds;
-  char* Vs = lds + TILE_BYTES;
+  constexpr int QW = 32;                                    // queries per wave
+  __shared__ __attribute__((aligned(16))) char lds[4 * TILE_BYTES];
 
   // split = 1 (small grids): the heavy and the light block of a pair are two workgroups of a 1-D grid, all heavy
   // ones first -- ids g and g + items are the same pair, so when the second round of dispatch lands on the CUs in
@@ -262,7 +259,7 @@ __global__ void __launch_bounds__(NW * 64, 2)
   }
   const int kvh = by / hgroups, hg = by - kvh * hgroups;
   const int b = bz;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5, col = lane & 31;
   const int rep = H / Hkv, hpw = NW / npb;
   const int r = w / npb, pb = w - r * npb;
@@ -280,26 +277,17 @@ __global__ void __launch_bounds__(NW * 64, 2)
   const int lo = kv_start[b];
   const uint8_t* mrow = key_mask ? key_mask + (size_t)b * mask_len : nullptr;
 
-  // Q^T fragments (B operand) of query block qq: lane holds Q[p0 + 32 qq + col][16 ks + 8 hi .. +7]
-  u32x4 qf[QB][8];
+  // Q^T fragments (B operand): lane holds Q[p0 + col][16 ks + 8 hi .. +7]
+  u32x4 qf[8];
+  const bf16_t* qrow = q + (((size_t)b * S + min(p0 + col, S - 1)) * H + h) * AP_DH + 8 * hi;
 #pragma unroll
-  for (int qq = 0; qq < QB; ++qq) {
-    const int pos = p0 + 32 * qq + col;
-    const bf16_t* qrow = q + (((size_t)b * S + min(pos, S - 1)) * H + h) * AP_DH + 8 * hi;
+  for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
+  f32x16 o[4];
+  float m_run = -INFINITY, l_run = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[qq][ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
-  }
-  f32x16 o[QB][4];
-  float m_run[QB], l_run[QB];
+  for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-  for (int qq = 0; qq < QB; ++qq) {
-    m_run[qq] = -INFINITY;
-    l_run[qq] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[qq][dt][i] = 0.f;
-  }
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
 
   const int wg_last_pos = min(S, (qb + 1) * QW * npb) - 1;
   const int last_key = min(slot0 + wg_last_pos, T - 1);
@@ -308,296 +296,203 @@ __global__ void __launch_bounds__(NW * 64, 2)
   const bf16_t* kb = kc + ((size_t)b * Hkv + kvh) * T * AP_DH;
   const bf16_t* vb = vc + ((size_t)b * Hkv + kvh) * T * AP_DH;
 
-  // staging: thread handles chunks c = tid + NT * i (row = c >> 4, ch = c & 15) of each tile
-  u32x4 sk[CH_PER_T], sv[CH_PER_T];
-  auto load_tile = [&](int t0) {
-#pragma unroll
-    for (int i = 0; i < CH_PER_T; ++i) {
-      const int c = tid + NT * i, row = c >> 4, ch = c & 15;
-      const size_t src = (size_t)min(t0 + row, T - 1) * AP_DH + 8 * ch;
-      sk[i] = *reinterpret_cast<const u32x4*>(kb + src);
-      sv[i] = *reinterpret_cast<const u32x4*>(vb + src);
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int i = 0; i < CH_PER_T; ++i) {
-      const int c = tid + NT * i, row = c >> 4, ch = c & 15;
-      *reinterpret_cast<u32x4*>(Ks + fa_off(row, ch)) = sk[i];
-      *reinterpret_cast<u32x4*>(Vs + fa_off(row, ch)) = sv[i];
-    }
-  };
   // per-lane LDS read offsets: K row reads (key block kb, dk step ks -> chunk 2 ks + hi)
   // V transposed reads: 16-lane group G = lane >> 4 covers d columns 16 (G & 1) .. +15 of a 32-wide d tile,
   // lane 4q + p of the group addresses row q of the 4-key block, columns 4p .. 4p + 3.
   const int gq = (lane & 15) >> 2, gp = lane & 3, G = lane >> 4;
-  if constexpr (PIPE) {
-    // LDS-DMA staging (no VGPRs held across the tile): wave w fills 1-KiB blocks w, w + NW, ... of a tile
-    // image; lane L of block bi writes row 4 bi + L / 16, slot L % 16, so it fetches the source chunk that
-    // fa_off's swizzle puts in that slot
-    auto Kr = [&](int i) { return lds + i * TILE_BYTES; };
-    auto Vr = [&](int i) { return lds + (2 + i) * TILE_BYTES; };
-    auto dma = [&](const bf16_t* src, int t0, char* dst) {
+  // LDS-DMA staging (no VGPRs held across the tile): wave w fills 1-KiB blocks w, w + NW, ... of a tile
+  // image; lane L of block bi writes row 4 bi + L / 16, slot L % 16, so it fetches the source chunk that
+  // fa_off's swizzle puts in that slot
+  auto Kr = [&](int i) { return lds + i * TILE_BYTES; };
+  auto Vr = [&](int i) { return lds + (2 + i) * TILE_BYTES; };
+  auto dma = [&](const bf16_t* src, int t0, char* dst) {
 #pragma unroll
-      for (int i = 0; i < 16 / NW; ++i) {
-        const int bi = w + NW * i, row = 4 * bi + (lane >> 4);
-        const int ch = (lane & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3));
-        if constexpr (PIPE == 2)
-          glds16_asm(src + (size_t)min(t0 + row, T - 1) * AP_DH + 8 * ch, dst + 1024 * bi);
-        else
-          glds16(src + (size_t)min(t0 + row, T - 1) * AP_DH + 8 * ch, dst + 1024 * bi);
-      }
-    };
-    auto scores = [&](const char* Kt, f32x16 (&s)[2]) {
-#pragma unroll
-      for (int kbk = 0; kbk < 2; ++kbk) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[kbk][i] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-          s[kbk] = mfma32(*reinterpret_cast<const u32x4*>(Kt + fa_off(32 * kbk + col, 2 * ks + hi)), qf[0][ks], s[kbk]);
-      }
-    };
-    const int n_t = t_begin <= last_key ? (last_key - t_begin) / FA_KT + 1 : 0;
-    const int qfirst = slot0 + p0, qslot = qfirst + col;
-    f32x16 st[2];
-    if (n_t > 0) {
-      dma(kb, t_begin, Kr(0));
-      dma(vb, t_begin, Vr(0));
+    for (int i = 0; i < 16 / NW; ++i) {
+      const int bi = w + NW * i, row = 4 * bi + (lane >> 4);
+      const int ch = (lane & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3));
+      // (ch is the same for every i: 4 NW i rows leave the swizzle as it is)
+      glds16_asm(src + (size_t)t0 * AP_DH, 256 * min(row, T - 1 - t0) + 16 * ch, dst + 1024 * bi);
     }
-    if (n_t > 1) dma(kb, t_begin + FA_KT, Kr(1));
-    wait_vmcnt<0>();
-    __syncthreads();
-    if (n_t > 0 && t_begin <= wave_last_slot) scores(Kr(0), st);
-    // the first iteration's DMA of K(2) lands in K(0)'s slot: every wave must be done reading it
-    if (n_t > 2) __syncthreads();
-    for (int it = 0; it < n_t; ++it) {
-      const int t0 = t_begin + it * FA_KT, cur = it & 1;
-      const bool has1 = it + 1 < n_t, has2 = it + 2 < n_t;
-      // K(i+2) into K(i)'s slot and V(i+1) into V(i-1)'s: both last read before the previous barrier
-      if (has2) dma(kb, t0 + 2 * FA_KT, Kr(cur));
-      if (has1) dma(vb, t0 + FA_KT, Vr(cur ^ 1));
-      if (t0 <= wave_last_slot) {  // wave-uniform; every later tile is inactive too
-        // masking (wave-uniform branch: only tiles crossing kv_start, the diagonal, T, or a key mask)
-        const bool full = !mrow && t0 >= lo && t0 + FA_KT - 1 <= qfirst && t0 + FA_KT - 1 < T;
-        if (!full) {
+  };
+  auto scores = [&](const char* Kt, f32x16 (&s)[2]) {
 #pragma unroll
-          for (int kbk = 0; kbk < 2; ++kbk)
+    for (int kbk = 0; kbk < 2; ++kbk) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int j = t0 + 32 * kbk + (i & 3) + 8 * (i >> 2) + 4 * hi;
-              bool ok = j >= lo && j <= qslot && j < T;
-              if (mrow) ok = ok && j < mask_len && mrow[j] != 0;
-              st[kbk][i] = ok ? st[kbk][i] : -INFINITY;
-            }
-        }
-        float tmax = -INFINITY;
+      for (int i = 0; i < 16; ++i) s[kbk][i] = 0.f;
 #pragma unroll
-        for (int kbk = 0; kbk < 2; ++kbk)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, st[kbk][i]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * scale_log2;  // scale > 0: max of the scaled scores
-        if (__ballot(tmax > m_run[0] + 8.f)) {
-          const float m_new = fmaxf(m_run[0], tmax);
-          const float alpha = __builtin_amdgcn_exp2f(m_run[0] - (m_new == -INFINITY ? 0.f : m_new));
-          l_run[0] *= alpha;
-          m_run[0] = m_new;
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[0][dt][i] *= alpha;
-        }
-        const float m_use = m_run[0] == -INFINITY ? 0.f : m_run[0];
-        // one straight-line block: S(i+1) on the matrix pipe beside exp / sum / pack of tile i (VALU), then
-        // O += V(i) P(i); NEXT is a compile-time copy so no branch splits the MFMAs from the VALU work
-        auto body = [&](auto NEXT) {
-          f32x16 sn[2];
-          if constexpr (decltype(NEXT)::value) {
-            if constexpr (PIPE == 2) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) sn[0][i] = sn[1][i] = 0.f;
-            } else {
-              scores(Kr(cur ^ 1), sn);
-            }
-          }
-          // key step s: 8 exps -> one P fragment -> its 4 PV MFMAs (one fragment live, exp beside the MFMAs)
-          float rs = 0.f;
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            if constexpr (PIPE == 2) {
-              // PIPE 2: a quarter of the next tile's scores (dk steps 2s, 2s + 1, both key blocks: 4 MFMAs on two
-              // alternating accumulators) in each key step, fenced so the scheduler keeps them beside this step's
-              // exps and PV MFMAs instead of sinking all 16 into a serial read -> wait -> MFMA chain at the end
-              __builtin_amdgcn_sched_barrier(0);
-              if constexpr (decltype(NEXT)::value) {
-                const char* Kt = Kr(cur ^ 1);
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-                  for (int kbk = 0; kbk < 2; ++kbk)
-                    sn[kbk] = mfma32(*reinterpret_cast<const u32x4*>(Kt + fa_off(32 * kbk + col, 4 * s + 2 * kk + hi)),
-                                     qf[0][2 * s + kk], sn[kbk]);
-              }
-            }
-            float e[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              e[j] = __builtin_amdgcn_exp2f(fmaf(st[s >> 1][8 * (s & 1) + j], scale_log2, -m_use));
-              rs += e[j];
-            }
-            const u32x4 pf = pack8(e);
-            const int r0 = 16 * s + 4 * (G >> 1) + gq;
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-              const int c0 = 4 * dt + 2 * (G & 1) + (gp >> 1);
-              const u32x2 lo4 = ld_tr(Vr(cur), fa_off(r0, c0) + 8 * (gp & 1));
-              const u32x2 hi4 = ld_tr(Vr(cur), fa_off(r0 + 8, c0) + 8 * (gp & 1));
-              const u32x4 vf = {lo4[0], lo4[1], hi4[0], hi4[1]};
-              o[0][dt] = mfma32(vf, pf, o[0][dt]);
-            }
-          }
-          rs += __shfl_xor(rs, 32, 64);
-          l_run[0] += rs;
-          if constexpr (decltype(NEXT)::value) {
-            st[0] = sn[0];
-            st[1] = sn[1];
-          }
-        };
-        // (the branch lets LLVM hoist the shared exp block above the scores MFMAs; a branch-free variant that always
-        // runs the NEXT copy interleaves them but measured neutral: profiles/r3_attn_prefill_branchfree_ab.jsonl)
-        // PIPE 2: branch-free (the next tile's scores always run; past the wave's last tile they read a settled stale
-        // slot and are never used), so the exps stay in the fenced key steps beside the MFMAs
-        if (PIPE == 2 || (has1 && t0 + FA_KT <= wave_last_slot))
-          body(std::true_type{});
-        else
-          body(std::false_type{});
-      }
-      wait_vmcnt<0>();
-      __syncthreads();
+      for (int ks = 0; ks < 8; ++ks)
+        s[kbk] = mfma32(*reinterpret_cast<const u32x4*>(Kt + fa_off(32 * kbk + col, 2 * ks + hi)), qf[ks], s[kbk]);
     }
-  } else {
-  if (t_begin <= last_key) {
-    load_tile(t_begin);
-    store_tile();
+  };
+  const int n_t = t_begin <= last_key ? (last_key - t_begin) / FA_KT + 1 : 0;
+  const int qfirst = slot0 + p0, qslot = qfirst + col;
+  f32x16 st[2];
+  if (n_t > 0) {
+    dma(kb, t_begin, Kr(0));
+    dma(vb, t_begin, Vr(0));
   }
+  if (n_t > 1) dma(kb, t_begin + FA_KT, Kr(1));
+  wait_vmcnt<0>();
   __syncthreads();
-  for (int t0 = t_begin; t0 <= last_key; t0 += FA_KT) {
-    const bool has_next = t0 + FA_KT <= last_key;
-    if (has_next) load_tile(t0 + FA_KT);
-    if (t0 <= wave_last_slot) {
-      // ---- S^T = K Q^T (each K fragment feeds the QB query blocks)
-      f32x16 st[QB][2];
+  if (n_t > 0 && t_begin <= wave_last_slot) scores(Kr(0), st);
+  // the first iteration's DMA of K(2) lands in K(0)'s slot: every wave must be done reading it
+  if (n_t > 2) __syncthreads();
+  // a lane's LDS offsets, of which the rest of fa_off is constants: K row read (dk step ks: ^ 32 ks; key block: + 8192),
+  // V transposed read (d tile dt: ^ 64 dt; keys + 8: ^ 32, + 2048; key step s: + 4096 s)
+  const int k_off = fa_off(col, hi), v_off = fa_off(4 * (G >> 1) + gq, 2 * (G & 1) + (gp >> 1)) + 8 * (gp & 1);
+  f32x16 st2[2];
+  float m_use = 0.f, rs = 0.f;
+  u32x4 pf = {0, 0, 0, 0};
+  // P of key step s: 8 of a lane's 32 scores
+  auto probs = [&](const f32x16 (&s2)[2], int s) {
+    float e[8];
 #pragma unroll
-      for (int kbk = 0; kbk < 2; ++kbk) {
+    for (int j = 0; j < 8; ++j) {
+      e[j] = __builtin_amdgcn_exp2f(fmaf(s2[s >> 1][8 * (s & 1) + j], scale_log2, -m_use));
+      rs += e[j];
+    }
+    return pack8(e);
+  };
+  auto largest = [&](const f32x16 (&s2)[2]) {
+    float m = -INFINITY;
 #pragma unroll
-        for (int qq = 0; qq < QB; ++qq)
+    for (int kbk = 0; kbk < 2; ++kbk)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) st[qq][kbk][i] = 0.f;
+      for (int i = 0; i < 16; ++i) m = fmaxf(m, s2[kbk][i]);
+    return m;
+  };
+  // what a tile needs before its PV: masks (wave-uniform branch: only tiles crossing kv_start, the diagonal, T, or a
+  // key mask), the running max, P of its first key step; raw: the lane's largest score before masks
+  auto enter = [&](int t0, f32x16 (&s2)[2], float raw) {
+    const bool full = !mrow && t0 >= lo && t0 + FA_KT - 1 <= qfirst && t0 + FA_KT - 1 < T;
+    if (!full) {
+      int first = t0 + 4 * hi;  // (opaque: or the keys of a lane's 32 scores are kept in registers over the loop)
+      asm volatile("" : "+v"(first));
+      const int from = lo - first, upto = min(min(qslot, T - 1), mrow ? mask_len - 1 : T) - first;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-          const u32x4 kf = *reinterpret_cast<const u32x4*>(Ks + fa_off(32 * kbk + col, 2 * ks + hi));
+      for (int kbk = 0; kbk < 2; ++kbk)
 #pragma unroll
-          for (int qq = 0; qq < QB; ++qq) st[qq][kbk] = mfma32(kf, qf[qq][ks], st[qq][kbk]);
+        for (int i = 0; i < 16; ++i) {
+          const int j = 32 * kbk + (i & 3) + 8 * (i >> 2);
+          s2[kbk][i] = j >= from && j <= upto ? s2[kbk][i] : -INFINITY;
         }
-      }
-      // ---- online softmax per query block (log2 domain); element (kbk, i) is key
-      // t0 + 32 kbk + (i & 3) + 8 (i >> 2) + 4 hi
-      u32x4 pf[QB][4];  // B fragments of P^T for the 4 key steps
-#pragma unroll
-      for (int qq = 0; qq < QB; ++qq) {
-        const int qfirst = slot0 + p0 + 32 * qq, qslot = qfirst + col;
-        const bool full = !mrow && t0 >= lo && t0 + FA_KT - 1 <= qfirst && t0 + FA_KT - 1 < T;
-        float tmax = -INFINITY;
+      if (mrow && mask_len > 0) {
 #pragma unroll
         for (int kbk = 0; kbk < 2; ++kbk)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            float v = st[qq][kbk][i] * scale_log2;
-            if (!full) {
-              const int j = t0 + 32 * kbk + (i & 3) + 8 * (i >> 2) + 4 * hi;
-              bool ok = j >= lo && j <= qslot && j < T;
-              if (mrow) ok = ok && j < mask_len && mrow[j] != 0;
-              v = ok ? v : -INFINITY;
-            }
-            st[qq][kbk][i] = v;
-            tmax = fmaxf(tmax, v);
+            const int j = 32 * kbk + (i & 3) + 8 * (i >> 2);
+            s2[kbk][i] = mrow[min(first + j, mask_len - 1)] ? s2[kbk][i] : -INFINITY;
           }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-        if (__ballot(tmax > m_run[qq] + 8.f)) {
-          const float m_new = fmaxf(m_run[qq], tmax);
-          const float alpha = __builtin_amdgcn_exp2f(m_run[qq] - (m_new == -INFINITY ? 0.f : m_new));
-          l_run[qq] *= alpha;
-          m_run[qq] = m_new;
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[qq][dt][i] *= alpha;
-        }
-        const float m_use = m_run[qq] == -INFINITY ? 0.f : m_run[qq];
-        float rs = 0.f;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          float e[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            e[j] = __builtin_amdgcn_exp2f(st[qq][s >> 1][8 * (s & 1) + j] - m_use);
-            rs += e[j];
-          }
-          pf[qq][s] = pack8(e);
-        }
-        rs += __shfl_xor(rs, 32, 64);
-        l_run[qq] += rs;
       }
-      // ---- O^T += V^T P^T; A element j of lane half hi = V[key 16 s + 8 (j >> 2) + 4 hi + (j & 3)][d]
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const int c0 = 4 * dt + 2 * (G & 1) + (gp >> 1);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int r0 = 16 * s + 4 * (G >> 1) + gq;
-          const u32x2 lo4 = ld_tr(Vs, fa_off(r0, c0) + 8 * (gp & 1));
-          const u32x2 hi4 = ld_tr(Vs, fa_off(r0 + 8, c0) + 8 * (gp & 1));
-          const u32x4 vf = {lo4[0], lo4[1], hi4[0], hi4[1]};
-#pragma unroll
-          for (int qq = 0; qq < QB; ++qq) o[qq][dt] = mfma32(vf, pf[qq][s], o[qq][dt]);
-        }
-      }
+      raw = largest(s2);
     }
-    __syncthreads();  // every wave is done with this tile's LDS images
-    if (has_next) {
-      store_tile();
-      __syncthreads();
-    }
-  }
-  }  // !PIPE
-
-  // ---- epilogue: lane (query pos, half hi) holds d = 32 dt + 8 g + 4 hi + (0..3) in o[dt][4 g .. 4 g + 3]
-#pragma unroll
-  for (int qq = 0; qq < QB; ++qq) {
-    const int pos = p0 + 32 * qq + col;
-    if (pos < S) {
-      const float inv = l_run[qq] > 0.f ? 1.f / l_run[qq] : 0.f;
-      bf16_t* dst = out + ((size_t)b * S + pos) * H * AP_DH + (size_t)h * AP_DH + 4 * hi;
+    const float tmax = lane_max32(raw) * scale_log2;  // scale > 0: max of the scaled scores
+    if (__ballot(tmax > m_run + 8.f)) {
+      const float m_new = fmaxf(m_run, tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+      l_run *= alpha;
+      m_run = m_new;
+      m_use = m_new == -INFINITY ? 0.f : m_new;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          u32x2 pk;
-          pk[0] = pack2bf(o[qq][dt][4 * g] * inv, o[qq][dt][4 * g + 1] * inv);
-          pk[1] = pack2bf(o[qq][dt][4 * g + 2] * inv, o[qq][dt][4 * g + 3] * inv);
-          *reinterpret_cast<u32x2*>(dst + 32 * dt + 8 * g) = pk;
-        }
+        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
+    rs = 0.f;
+    pf = probs(s2, 0);
+  };
+  // tile it of parity cur (a constant: an LDS address is a lane's own and an immediate, and no scores move): key
+  // step s has the PV MFMAs of P(s), a share of the next tile's scores and, on the VALU beside them, P(s + 1)
+  auto tile = [&](int it, auto parity, f32x16 (&s2)[2], f32x16 (&sn)[2]) {
+    constexpr int cur = decltype(parity)::value;
+    const int t0 = t_begin + it * FA_KT;
+    const bool has1 = it + 1 < n_t, has2 = it + 2 < n_t;
+    // K(i+2) into K(i)'s slot and V(i+1) into V(i-1)'s: both last read before the previous barrier
+    if (has2) dma(kb, t0 + 2 * FA_KT, Kr(cur));
+    if (has1) dma(vb, t0 + FA_KT, Vr(cur ^ 1));
+    if (t0 <= wave_last_slot) {  // wave-uniform; every later tile is inactive too
+      auto score = [&](int f) {
+        sn[f & 1] = mfma32(*reinterpret_cast<const u32x4*>(Kr(cur ^ 1) + (k_off ^ (32 * (f >> 1))) + 8192 * (f & 1)),
+                           qf[f >> 1], sn[f & 1]);
+      };
+      auto pv = [&](int s, int dt) {
+        const u32x2 lo4 = ld_tr(Vr(cur), (v_off ^ (64 * dt)) + 4096 * s);
+        const u32x2 hi4 = ld_tr(Vr(cur), (v_off ^ (64 * dt) ^ 32) + 2048 + 4096 * s);
+        const u32x4 vf = {lo4[0], lo4[1], hi4[0], hi4[1]};
+        o[dt] = mfma32(vf, pf, o[dt]);
+      };
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sn[0][i] = sn[1][i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int f = 6 * s; f < (s < 2 ? 6 * s + 6 : 16); ++f) score(f);
+        const u32x4 next = probs(s2, s + 1);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) pv(s, dt);
+        pf = next;
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int i = 0; i < (s < 2 ? 10 : 8); ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      l_run += rs;  // (this half's keys; the halves meet at the end)
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) pv(3, dt);
+      const float raw = largest(sn);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+
+      __builtin_amdgcn_sched_barrier(0);
+      if (has1 && t0 + FA_KT <= wave_last_slot) enter(t0 + FA_KT, sn, raw);
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+  };
+  if (n_t > 0 && t_begin <= wave_last_slot) enter(t_begin, st, largest(st));
+  for (int it = 0; it < n_t; it += 2) {
+    tile(it, std::integral_constant<int, 0>{}, st, st2);
+    if (it + 1 < n_t) tile(it + 1, std::integral_constant<int, 1>{}, st2, st);
+  }
+  l_run = lane_sum32(l_run);
+
+  // ---- epilogue: lane (query pos, half hi) holds d = 32 dt + 8 g + 4 hi + (0..3) in o[dt][4 g .. 4 g + 3]
+  const int pos = p0 + col;
+  if (pos < S) {
+    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+    bf16_t* dst = out + ((size_t)b * S + pos) * H * AP_DH + (size_t)h * AP_DH + 4 * hi;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        u32x2 pk;
+        pk[0] = pack2bf(o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv);
+        pk[1] = pack2bf(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv);
+        *reinterpret_cast<u32x2*>(dst + 32 * dt + 8 * g) = pk;
+      }
   }
   }  // pass
 }
 
 // v2 launch with NW waves per workgroup: NW / rep position blocks (rep < NW) or NW of the rep q heads (rep >= NW) share
-// each K/V tile the workgroup stages; `paired_only`: always the (heavy, light) pair per workgroup
-template <int NW, int PIPE>
+// each K/V tile the workgroup stages
+template <int NW>
 static void launch_prefill_v2(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, const int32_t* slot,
                               const int32_t* kv_start, const uint8_t* key_mask, int mask_len, bf16_t* out, int B, int S,
-                              int H, int Hkv, int T, int rep, bool paired_only, hipStream_t s) {
+                              int H, int Hkv, int T, int rep, hipStream_t s) {
   const int npb = rep >= NW ? 1 : NW / rep;    // position blocks per workgroup
   const int hpw = NW / npb;                    // q heads per workgroup
   const int hgroups = rep / hpw;
@@ -605,21 +500,20 @@ static void launch_prefill_v2(const bf16_t* q, const bf16_t* kc, const bf16_t* v
   const int n_qb = (S + 32 * npb - 1) / (32 * npb);
   const int pairs = (n_qb + 1) / 2 * Hkv * hgroups * B;
   // fewer pairs than two workgroups per CU (B = 1 prefill): each half of a pair is its own workgroup, so a CU
-  // holds two resident workgroups instead of one
-  const bool split = !paired_only && pairs < 2 * 256;
+  // holds two resident workgroups instead of one (of 4 waves: of 8, a CU holds one)
+  const bool split = NW == 4 && pairs < 2 * 256;
   if (split) {
-    attn_prefill_v2_kernel<NW, PIPE><<<dim3(2 * pairs, 1, 1), NW * 64, 0, s>>>(
+    attn_prefill_v2_kernel<NW><<<dim3(2 * pairs, 1, 1), NW * 64, 0, s>>>(
         q, kc, vc, slot, kv_start, key_mask, mask_len, out, S, H, Hkv, T, sl2, npb, hgroups, n_qb, 1);
   } else {
     dim3 grid2((n_qb + 1) / 2, Hkv * hgroups, B);  // a (heavy, light) pair of query blocks per workgroup
-    attn_prefill_v2_kernel<NW, PIPE><<<grid2, NW * 64, 0, s>>>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, S,
+    attn_prefill_v2_kernel<NW><<<grid2, NW * 64, 0, s>>>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, S,
                                                                 H, Hkv, T, sl2, npb, hgroups, n_qb, 0);
   }
 }
 
-// impl (attn_prefill_set_impl, A/B): 2 = default dispatch; 7 = pipelined 4 waves, 8 = unpipelined 4 waves, 9 =
-// pipelined 8 waves (paired), 13 = the same with asm LDS-DMA and the next tile's scores spread over the key steps
-// (PIPE 2); 1 = the v1 kernel (also the fallback for a non-power-of-two GQA ratio)
+// impl (attn_prefill_set_impl, A/B): 2 = default dispatch; 7 (and 8) = 4 waves per workgroup, 13 (and 9) = 8 waves; 1 =
+// the v1 kernel (also the fallback for a non-power-of-two GQA ratio)
 static int g_attn_prefill_impl = 2;
 void attn_prefill_set_impl(int impl) { g_attn_prefill_impl = impl; }
 
@@ -631,36 +525,25 @@ int attn_prefill(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, const int3
   const int rep = H / Hkv;
   const bool pow2rep = rep == 1 || rep == 2 || rep == 4 || rep == 8;
   int impl = g_attn_prefill_impl;
-  // default (impl 2): the software-pipelined loop from S = 512 (a query block needs a few tiles to pipeline), with 8
-  // waves per workgroup when that paired grid fills the CUs without exceeding ~4 workgroups per CU (256..1023
-  // workgroups: twice the queries per staged K/V tile), else 4 waves; up to S = 256 the unpipelined 4-wave loop. Interleaved A/B
-  // (profiles/r3_attn_prefill_pipe_ab.jsonl, TFLOP/s, previous default -> now): 8B B = 1 S = 2048 454 -> 509,
-  // B = 16 S = 2048 672 -> 746, S = 8192 854 -> 903, B = 2048 S = 128 186 -> 198, 70B S = 2048 698 -> 733.
-  // The 8-wave launch is PIPE 2 (impl 13) since round 4: bit-identical to impl 9, +1-5 % on the 8-wave shapes
-  // (profiles/r4_attn_prefill_asm_dma_ab.jsonl).
+  // default (impl 2): 8 waves per workgroup (twice the queries per staged K / V tile, one workgroup resident per CU)
+  // where the prompt is long and the paired grid's rounds over the 256 CUs are nearly full (a last round of >= 90 %; with
+  // one round, >= 75 %), else 4 waves. Measured, 4 -> 8 waves, us: S = 4096 143 -> 133 (one full round), 2 x 4096 279 -> 265
+  // (two), S = 3000 103 -> 89 (192 workgroups), 124 -> 107 (240); but S = 4096 226 -> 250 (320), 4 x 1500 101 -> 111 (384),
+  // S = 1500 39 -> 53 (96); at S <= 1024 4 waves are ahead nearly everywhere (16 x 512 76 -> 79, 64 x 128 60 -> 83): a query
+  // block is then twice as many rows for the same few tiles.
   if (impl == 2 && pow2rep) {
-    if (S <= 256) {
-      impl = 8;
-    } else {
-      const int npb8 = rep >= 8 ? 1 : 8 / rep;
-      const int n_qb8 = (S + 32 * npb8 - 1) / (32 * npb8);
-      const int wg8 = (n_qb8 + 1) / 2 * Hkv * (rep / (8 / npb8)) * B;
-      // 8 waves only for mid-sized grids: from 4 paired 8-wave workgroups per CU up, the 4-wave grid (twice the
-      // workgroups, 2 resident per CU) measured faster or tied on 4 of 4 boxes (8B B = 16 S = 2048 747-784 vs 731-762
-      // TFLOP/s, 7B MHA B = 16 661-687 vs 597-675; profiles/r4_attn_prefill_dispatch_ab.jsonl)
-      impl = wg8 >= 256 && wg8 < 1024 ? 13 : 7;
-    }
+    const int npb8 = rep >= 8 ? 1 : 8 / rep;
+    const int n_qb8 = (S + 32 * npb8 - 1) / (32 * npb8);
+    const long long wg8 = (long long)((n_qb8 + 1) / 2) * Hkv * (rep / (8 / npb8)) * B;
+    const long long rounds = (wg8 + 255) / 256;
+    impl = S > 1024 && (10 * wg8 >= 9 * 256 * rounds || (rounds == 1 && wg8 >= 192)) ? 13 : 7;
   }
-  const int nw_impl = impl == 9 || impl == 13 ? 8 : 4;
-  if ((impl == 7 || impl == 8 || impl == 9 || impl == 13) && (rep % nw_impl == 0 || nw_impl % rep == 0)) {
-    if (impl == 7)
-      launch_prefill_v2<4, 1>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, false, s);
-    else if (impl == 8)
-      launch_prefill_v2<4, 0>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, false, s);
-    else if (impl == 9)
-      launch_prefill_v2<8, 1>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, true, s);
+  const int nw = impl == 7 || impl == 8 ? 4 : impl == 9 || impl == 13 ? 8 : 0;
+  if (nw && (rep % nw == 0 || nw % rep == 0)) {
+    if (nw == 4)
+      launch_prefill_v2<4>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, s);
     else
-      launch_prefill_v2<8, 2>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, true, s);
+      launch_prefill_v2<8>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, s);
     JLA_CHECK_LAUNCH();
     return 0;
   }

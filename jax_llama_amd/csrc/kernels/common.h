@@ -129,6 +129,13 @@ JLA_DEV void glds16_asm(const void* gsrc, void* lds_wave_base) {
       (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_wave_base);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gsrc), "s"(m0) : "memory", "m0");
 }
+// the same from a wave's base and a lane's offset in bytes (one register a lane instead of two)
+JLA_DEV void glds16_asm(const void* wave_base, int off, void* lds_wave_base) {
+  const unsigned m0 = __builtin_amdgcn_readfirstlane(
+      (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_wave_base);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(wave_base), "s"(m0)
+               : "memory", "m0");
+}
 #pragma clang diagnostic pop
 // s_waitcnt vmcnt(N) only (expcnt/lgkmcnt left at their maxima)
 template <int N>

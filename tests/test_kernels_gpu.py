@@ -294,6 +294,40 @@ def test_attention_prefill_long(impl, rep, s, slot0, masked):
         assert got.reshape(b, s, h * dh)[1, : s // 3].float().abs().max().item() == 0.0
 
 
+@pytest.mark.parametrize("impl", [7, 13])
+@pytest.mark.parametrize("s,slot0,masked", [(1, 0, False), (32, 31, True), (64, 0, False), (65, 0, True), (128, 64, True),
+                                            (129, 127, False), (257, 3, True), (1025, 0, False)])
+def test_attention_prefill_tile_edges(impl, s, slot0, masked):
+    """The pipelined loop at one tile, at odd and even tile counts and at their edges, with a padded row and a key mask
+    that ends before the last keys (so a query's own key can be masked, and some tiles wholly)."""
+    e = ops.ext()
+    b, hkv, rep, dh = 2, 2, 2, 128
+    t = slot0 + s
+    g = torch.Generator(device=DEV).manual_seed(31 * s + slot0)
+    kc = (torch.randn(b, hkv, t, dh, device=DEV, generator=g) * 2).to(BF16)  # scores far enough apart to move the max
+    vc = torch.randn(b, hkv, t, dh, device=DEV, generator=g).to(BF16)
+    q = (torch.randn(b, s, hkv * rep, dh, device=DEV, generator=g) * 2).to(BF16)
+    kv_start = torch.tensor([0, min(70, t // 2)], dtype=torch.int32, device=DEV)
+    mask = None
+    if masked:
+        mask = (torch.rand(b, max(t - 5, 1), device=DEV, generator=g) > 0.3).to(torch.uint8)
+        mask[:, 64:128] = 0
+    slot = torch.tensor([slot0], dtype=torch.int32, device=DEV)
+    try:
+        e.attn_prefill_set_impl(impl)
+        got = ops.attention(q, kc, vc, slot, kv_start, mask)
+        torch.cuda.synchronize()
+    finally:
+        e.attn_prefill_set_impl(2)
+    full = torch.zeros(b, t, dtype=torch.uint8, device=DEV)
+    if masked:
+        full[:, :mask.shape[1]] = mask
+    want = _attn_ref_gpu(q, kc, vc, slot0, kv_start, full if masked else None)
+    # P and the result are rounded to bf16 (2^-9 each of a weighted mean of values), the rest is fp32
+    bound = 2 * 2.0 ** -9 * vc.float().abs().max().item() + 1e-3
+    assert (got.float() - want).abs().max().item() < bound
+
+
 def test_attention_prefill_8k():
     """S = 8192 causal prefill (Llama-3 max_seq_len), rep 4, one batch row."""
     b, hkv, rep, s, dh = 1, 2, 4, 8192, 128
