@@ -3,7 +3,7 @@
 //
 // What bounds it: the matrix cores, and the rows that whole tiles pad. lr_gemm_kernel (64- or 128-row tiles, one LDS stage, VGPR staging)
 // pulls 11 TB/s from L2 and stops at 300-450 TFLOP/s. Here one wave per SIMD owns a 16 MI x 16 NJ output block (NJ x MI accumulators
-// of v_mfma_f32_16x16x32_bf16 in AGPRs), K advances 64 per LDS slot, two slots filled by LDS-DMA, and every fragment read and
+// of v_mfma_f32_16x16x32_bf16 in AGPRs), K advances 64 per LDS slot, slots filled by LDS-DMA, and every fragment read and
 // DMA issue sits between MFMAs -- the schedule of the packed GEMM (kernels/gemm4w.h), with both operands row-major: the
 // activation rows are gathered by per-lane addresses and the weight rows are read as they lie in the checkpoint, so an
 // expert's weights need no second, packed copy. MI = NJ = 8 (256 x 256 tiles) reads 256 B of LDS per MFMA and is for launches of many
@@ -12,16 +12,24 @@
 // rows 125 | 188 | 271 | 571 -> 95 | 137 | 211 | 444 (416 | 712 | 1025 | 2265 -> 360 | 533 | 939 | 2056); one gated matrix of 5632 x 2048, 600 | 1500 |
 // 3000 rows 65 | 117 | 194 -> 36 | 77 | 136.
 //
+// Of 256 x 256 tiles a compute unit runs one, and waits are its own: at two slots for both operands a wave stood in them for 18 % of its time
+// (the DMAs of K-tile t + 2 could not begin before the second half of t, and spread over it, the last had half a K-tile to land). With a third
+// slot for the gathered rows (160 KiB in all) half of the DMAs go out half a K-tile earlier: 8 experts of 7168 x 4096, both products,
+// 24000 | 6000 rows 3927 | 1143 -> 3659 | 1111 us. The smaller tiles' DMAs go out within the first half of a half K-tile instead (2600 rows of
+// 2816 x 2048 156 -> 151 us).
+//
 // LDS images of both operands: [rows][8 cells of 16 B] (64 k); cell c of row r holds k-chunk c ^ ((r & 15) >> 1), so the 16
 // lanes of a fragment read fall on all 64 banks. A gated activation interleaves 16 gate rows and 16 up rows of W, which
 // puts a column's gate and up accumulators into neighbouring tiles of one wave.
-// The epilogue passes 64 rows at a time through the wave's own 32 KiB of LDS: the activation is then one small loop and
-// rows leave as full lines (fp32: 512 B per row and wave).
+// The epilogue passes 64 rows at a time through the wave's own 32 KiB of LDS: the activation is then one small loop (of its own for SwiGLU and
+// for none: 2 % of a product) and rows leave as full lines (fp32: 512 B per row and wave).
 #include "../kernels/gemm4w.h"
 #include "../kernels/row_tiles.h"
 #include "hy_util.h"
 #include "hybrid.h"
 #include "row_act.h"
+
+#include <type_traits>
 
 namespace jla {
 
@@ -34,11 +42,13 @@ constexpr int RG_PER_CU = (32 * MI + 32 * NJ) * RG_BK * 2 * 2 <= 80 * 1024 ? 2 :
 template <int NJ, int MI>
 __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(RowLinear p, int gated, int tiles_n) {
   static_assert((NJ == 4 || NJ == 8) && MI >= 4 && MI <= 8, "16-column and 16-row tiles per wave");
-  constexpr int BM = 32 * MI, SLOT = (BM + 32 * NJ) * RG_BK * 2 / 16;  // u32x4 of a slot: A, then W
+  constexpr bool A3 = RG_PER_CU<NJ, MI> == 1;  // three slots of A, two of W
+  constexpr int BM = 32 * MI, SA = BM * RG_BK * 2 / 16, SW = 32 * NJ * RG_BK * 2 / 16;  // u32x4 of a slot
+  constexpr int W0 = (A3 ? 3 : 2) * SA, CELLS = W0 + 2 * SW;
   constexpr int T = NJ * MI;      // MFMAs of half a K-tile, in 16 groups
   constexpr int EG = MI == 8 ? 4 : (MI % 2 ? 1 : 2);  // row tiles that pass through LDS at a time at the end
-  static_assert(2 * SLOT >= 4 * EG * 16 * 4 * NJ, "the epilogue's staging");
-  __shared__ u32x4 lds[2 * SLOT];
+  static_assert(CELLS >= 4 * EG * 16 * 4 * NJ && CELLS * 16 <= 160 * 1024, "the epilogue's staging");
+  __shared__ u32x4 lds[CELLS];
   const int lane = threadIdx.x & 63;
   const int wu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wu >> 1, wc = wu & 1;
@@ -67,16 +77,16 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
     const int wrow = gated && (jt & 1) ? N + col : col;
     ow[j] = ((unsigned)wrow * (unsigned)K + 8u * (unsigned)chunk) * 2u;
   }
+  auto a_slot = [&](int t) { return (A3 ? t % 3 : t & 1) * SA; };
   auto dma = [&](int t, int j) {  // the j-th of this wave's MI + NJ DMAs of K-tile t
-    u32x4* slot = lds + (t & 1) * SLOT;
-    if (j < MI) glds16(pa[j < MI ? j : 0] + (size_t)t * 128, slot + (wu + 4 * j) * 64);
-    else glds16(wbase + (size_t)t * 128 + ow[j < MI ? 0 : j - MI], slot + BM * 8 + (wu + 4 * (j - MI)) * 64);
+    if (j < MI) glds16(pa[j < MI ? j : 0] + (size_t)t * 128, lds + a_slot(t) + (wu + 4 * j) * 64);
+    else glds16(wbase + (size_t)t * 128 + ow[j < MI ? 0 : j - MI], lds + W0 + (t & 1) * SW + (wu + 4 * (j - MI)) * 64);
   };
-  const int xrd = (wr * 16 * MI + (lane & 15)) * 8, wrd = BM * 8 + (wc * 16 * NJ + (lane & 15)) * 8;
+  const int xrd = (wr * 16 * MI + (lane & 15)) * 8, wrd = W0 + (wc * 16 * NJ + (lane & 15)) * 8;
   const int c0 = (0 + (lane >> 4)) ^ ((lane >> 1) & 7), c1 = (4 + (lane >> 4)) ^ ((lane >> 1) & 7);
-  auto rd = [&](u32x4& dst, int slot, int h, int q) {  // q < NJ: W n-tile q; then the MI m-tiles of A
-    const u32x4* s = lds + slot * SLOT + (h ? c1 : c0);
-    dst = q < NJ ? s[wrd + q * 128] : s[xrd + (q - NJ) * 128];
+  auto rd = [&](u32x4& dst, int t, int h, int q) {  // of K-tile t: q < NJ: W n-tile q; then the MI m-tiles of A
+    const u32x4* s = lds + (h ? c1 : c0);
+    dst = q < NJ ? s[wrd + (t & 1) * SW + q * 128] : s[xrd + a_slot(t) + (q - NJ) * 128];
   };
 
   f32x4 acc[NJ][MI];
@@ -86,21 +96,26 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
     for (int i = 0; i < MI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 w0[NJ], x0[MI], w1[NJ], x1[MI];
 
-  // MI NJ MFMAs on (wf, xf) with the MI + NJ fragment reads of the next half tile and the DMAs of tile td between them
-  auto substep = [&](u32x4 (&wf)[NJ], u32x4 (&xf)[MI], u32x4 (&wn)[NJ], u32x4 (&xn)[MI], bool do_rd, int rslot, int rh,
-                     bool do_dma, int td) {
+  // MI NJ MFMAs on (wf, xf) with the MI + NJ fragment reads of the next half tile (K-tile tr) and the DMAs [d0, d1) of K-tile td
+  // between them
+  auto substep = [&](u32x4 (&wf)[NJ], u32x4 (&xf)[MI], u32x4 (&wn)[NJ], u32x4 (&xn)[MI], bool do_rd, int tr, int rh, bool do_dma,
+                     int td, int d0, int d1) {
+    constexpr int DQ = A3 ? 16 : 8;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
 #pragma unroll
       for (int m = q * T / 16; m < (q + 1) * T / 16; ++m) g4_mfma(acc[m / MI][m % MI], wf[m / MI], xf[m % MI]);
-      if (q < MI + NJ) {
-        if (do_rd) rd(q < NJ ? wn[q < NJ ? q : 0] : xn[q < NJ ? 0 : (q - NJ) % MI], rslot, rh, q);
-        if (do_dma) dma(td, q);
+      if (do_dma && q < DQ) {
+#pragma unroll
+        for (int j = d0 + q * (d1 - d0) / DQ; j < d0 + (q + 1) * (d1 - d0) / DQ; ++j) dma(td, j);
       }
+      if (q < MI + NJ && do_rd) rd(q < NJ ? wn[q < NJ ? q : 0] : xn[q < NJ ? 0 : (q - NJ) % MI], tr, rh, q);
     }
   };
-  auto mid_barrier = [&]() {  // this wave's DMAs of the next tile have landed; then every wave's have
-    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  // this wave's DMAs of the next tile have landed (the rows of the tile behind it, the last MI issued, may be under way); then every wave's have
+  auto mid_barrier = [&](bool rows_under_way) {
+    if (rows_under_way) __builtin_amdgcn_s_waitcnt(0x0070 | (MI & 15) | ((MI >> 4) << 14));  // vmcnt(MI) lgkmcnt(0)
+    else __builtin_amdgcn_s_waitcnt(0x0070);                                                   // vmcnt(0) lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
@@ -119,20 +134,22 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
 #pragma unroll
   for (int q = 0; q < MI + NJ; ++q) rd(q < NJ ? w0[q < NJ ? q : 0] : x0[q < NJ ? 0 : (q - NJ) % MI], 0, 0, q);
 
+  // (A3: the rows of K-tile t + 2 go into the slot of t - 1 already during the first half of t, the weights into t's own during the second)
+  constexpr int DS = A3 ? MI : 0;
   int t = 0;
   for (; t + 2 < KT; ++t) {
-    substep(w0, x0, w1, x1, true, t & 1, 1, false, 0);
-    mid_barrier();
-    substep(w1, x1, w0, x0, true, (t + 1) & 1, 0, true, t + 2);
+    substep(w0, x0, w1, x1, true, t, 1, A3, t + 2, 0, DS);
+    mid_barrier(A3);
+    substep(w1, x1, w0, x0, true, t + 1, 0, true, t + 2, DS, MI + NJ);
   }
   if (t + 1 < KT) {
-    substep(w0, x0, w1, x1, true, t & 1, 1, false, 0);
-    mid_barrier();
-    substep(w1, x1, w0, x0, true, (t + 1) & 1, 0, false, 0);
+    substep(w0, x0, w1, x1, true, t, 1, false, 0, 0, 0);
+    mid_barrier(false);
+    substep(w1, x1, w0, x0, true, t + 1, 0, false, 0, 0, 0);
     ++t;
   }
-  substep(w0, x0, w1, x1, true, t & 1, 1, false, 0);
-  substep(w1, x1, w0, x0, false, 0, 0, false, 0);
+  substep(w0, x0, w1, x1, true, t, 1, false, 0, 0, 0);
+  substep(w1, x1, w0, x0, false, 0, 0, false, 0, 0, 0);
   g4_acc_fence();
   __syncthreads();  // every wave is past its last fragment read: the slots become the epilogue's staging
 
@@ -154,30 +171,37 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
     const int rbase = r0 + wr * 16 * MI + 16 * EG * part;
     int drow = rbase + (lane & (16 * EG - 1));  // lane l: where the part's row l goes (-1: past the expert's rows)
     drow = drow < rend ? (p.dst_idx ? p.dst_idx[drow] : drow) : -1;
+    auto rows_out = [&](auto known) {
+      constexpr int ACT = decltype(known)::value;  // -1: whatever p.act says
 #pragma unroll 4
-    for (int s = 0; s < 16 * EG; s += rpi) {
-      const int rr = s + rr0;
-      const int d = __shfl(drow, rr, 64);
-      const f32x4 g = wl[rr * CH + (gch ^ (rr & 15))];
-      f32x4 v = g;
-      if (gated) {
-        const f32x4 u = wl[rr * CH + ((gch + 4) ^ (rr & 15))];
+      for (int s = 0; s < 16 * EG; s += rpi) {
+        const int rr = s + rr0;
+        const int d = __shfl(drow, rr, 64);
+        f32x4 v = wl[rr * CH + (gch ^ (rr & 15))];
+        if constexpr (ACT == HY_ACT_SWIGLU) {
+          const f32x4 u = wl[rr * CH + ((gch + 4) ^ (rr & 15))];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = lr_act(p, g[x], u[x]);
-      } else if (p.act != HY_ACT_NONE) {
+          for (int x = 0; x < 4; ++x) v[x] = hy_silu(v[x]) * u[x];
+        } else if constexpr (ACT != HY_ACT_NONE) {
+          const f32x4 u = gated ? wl[rr * CH + ((gch + 4) ^ (rr & 15))] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = lr_act(p, g[x], 0.f);
-      }
-      if (d >= 0 && col < N) {
-        if (p.out_bf16) {
-          *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + (size_t)d * p.ldo + col) =
-              u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
-        } else {
-          f32x4* o = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + (size_t)d * p.ldo + col);
-          *o = p.add_out ? *o + v : v;
+          for (int x = 0; x < 4; ++x) v[x] = lr_act(p, v[x], u[x]);
+        }
+        if (d >= 0 && col < N) {
+          if (p.out_bf16) {
+            *reinterpret_cast<u32x2*>(reinterpret_cast<bf16_t*>(p.out) + (size_t)d * p.ldo + col) =
+                u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
+          } else {
+            f32x4* o = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + (size_t)d * p.ldo + col);
+            *o = p.add_out ? *o + v : v;
+          }
         }
       }
-    }
+    };
+    // (the switch over activations stays out of the loop)
+    if (p.act == HY_ACT_SWIGLU) rows_out(std::integral_constant<int, HY_ACT_SWIGLU>{});
+    else if (p.act == HY_ACT_NONE) rows_out(std::integral_constant<int, HY_ACT_NONE>{});
+    else rows_out(std::integral_constant<int, -1>{});
   }
 }
 

@@ -53,3 +53,21 @@ def test_rows_by_expert(counts, n, k):
 def test_where_the_tiles_for_fewer_rows_end(per):
     _check([per - 3, per + 3, per, per], 8200, 1024, per)
     _check([per - 3, per + 3, per, per], 512, 1024, per)
+
+
+@pytest.mark.parametrize("k", [1024, 1088, 1152])  # every phase of the rows' three slots
+def test_largest_tiles(k):
+    """256 x 256 tiles (rounds enough for them), their last row tile nearly empty, and the activations outside the two fast loops."""
+    rows, n = 2050, 30000
+    g = torch.Generator(device=DEV).manual_seed(k)
+    x = torch.randn(rows, k, generator=g, device=DEV).to(BF16)
+    w = (torch.randn(2 * n, k, generator=g, device=DEV) * k ** -0.5).to(BF16)
+    y = x.double() @ w.double().t()
+    gate, up = y.chunk(2, -1)
+    gc, uc = gate.clamp(max=1.5), up.clamp(-1.5, 1.5)
+    for act, ww, want in ((hy.ACT_SWIGLU, w, torch.nn.functional.silu(gate) * up), (hy.ACT_NONE, w, y),
+                          (hy.ACT_CLAMP_GLU, w, gc * torch.sigmoid(1.7 * gc) * (uc + 1)), (hy.ACT_RELU2, w, y.clamp(min=0) ** 2)):
+        out = torch.full((rows, want.shape[1]), float("nan"), device=DEV)
+        hy.ext().linear_rows(x, None, ww, out, None, None, None, rows, act, 1.5, 1.7, None, None, 0.0)
+        # the product's error as above; each of these activations grows a relative error at most about twice
+        assert _err(out, want) < (1 if act == hy.ACT_NONE else 2) * 9e-9 * k ** 0.5 + 2.0 ** -22, act
