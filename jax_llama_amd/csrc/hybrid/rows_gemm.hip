@@ -242,13 +242,15 @@ struct RgForm {
   float fill, step, more, last;
 };
 static const RgForm RG_FORMS[] = {{4, 4, 1.0f, 0.644f, 0.833f, 1.0f}, {4, 5, 9.75f, 0.608f, 0.965f, 0.99f}, {4, 6, 5.17f, 0.819f, 0.795f, 0.945f},
-                                  {8, 8, 17.5f, 1.407f, 1.3f, 1.0f}};
+                                  {8, 8, 16.3f, 1.31f, 1.3f, 1.0f}};
 
 // The form with the least time by the figures above: on average 1.8 % above the best of those measured (54 products: 8 experts of 2816 x
 // 2048 and 7168 x 4096 with 1000 to 12000 rows, one matrix of 5632 x 2048 with 300 to 4000, gated and down), where 256-row tiles, 128 or 256
 // wide, took 1.22 times as long. With experts, whose counts only the device knows, the row tiles are a mean over four
 // counts around the average. Eight rounds of 256 x 256 tiles and more: these (8 experts of gated 7168 x 4096, 6000 | 12000 rows 667 | 1295, 192
-// x 128 688 | 1336: fewer bytes cost less power).
+// x 128 688 | 1336: fewer bytes cost less power). These figures are of two slots for both operands; the 256 x 256 form's are scaled by what
+// the third gave it (0.93), by which it is now chosen for more: 8 experts of 7168 x 4096, both products, 9000 | 6000 rows 1582 | 1083 -> 1481 |
+// 988 us, of 2816 x 2048, 12000 rows 495 -> 467; scaled by 0.82 instead, 8000 rows of 2816 x 2048 and the like lose 3 to 5 %.
 constexpr long long RG_MANY = 8 * 256;
 
 static const RgForm& rg_form(const RowLinear& p) {
