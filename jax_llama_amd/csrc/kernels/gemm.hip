@@ -1027,13 +1027,14 @@ __global__ void __launch_bounds__(256, 1)
 // Persistent gemm4 (tile config 13): one workgroup per CU walks the launch order round by round (tile wg, wg + CUs,
 // ...), so a CU's next tile starts without a workgroup teardown and relaunch, and the CUs drift apart over the rounds:
 // their epilogues (the residual's fp32 read-modify-write above all) stop arriving at HBM as one chip-wide burst.
-template <int MODE, int RMSM>
+// X3: three x slots, so that half of a K-tile's DMAs go out half a K-tile earlier (g4_mainloop).
+template <int MODE, int RMSM, bool X3 = false>
 __global__ void __launch_bounds__(256, 1)
     gemm4p_kernel(const bf16_t* __restrict__ x, const u32x4* __restrict__ W, void* __restrict__ out, int M, int N,
                   int K, int accumulate, int out_f32, bf16_t* __restrict__ mirror, int tiles_m, int tiles_n,
                   float rms_eps, QKVArgs qa, const float* __restrict__ rms_inv, int group_m) {
   constexpr bool RMS = RMSM == 1;
-  __shared__ u32x4 lds[2 * G4_SLOT_U4 + 64];
+  __shared__ u32x4 lds[X3 ? 3 * G4_A_U4 + 2 * G4_B_U4 : 2 * G4_SLOT_U4 + 64];
   const int lane0 = threadIdx.x & 63;
   const int wu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nwg = gridDim.x, orig = blockIdx.x;
@@ -1056,7 +1057,7 @@ __global__ void __launch_bounds__(256, 1)
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float ss[4] = {0.f, 0.f, 0.f, 0.f};
-    g4_mainloop<RMS>(g, lds, m0, n0, 0, K >> 6, wu, lane, acc, ss);
+    g4_mainloop<RMS, decltype(acc), 0, false, X3>(g, lds, m0, n0, 0, K >> 6, wu, lane, acc, ss);
     g4_epilogue<MODE, RMSM>(acc, ss, lds, wu, lane, m0, n0, 0, ep, qa);
     __syncthreads();  // the epilogue's staging / row scales are done with LDS before the next tile's DMA
   }
@@ -1283,6 +1284,11 @@ static int g4_group_m(int tiles_m, int tiles_n, int K) {
   return gm < tiles_m ? gm : tiles_m;
 }
 static int g_g5_diag = 0;  // tools only (gemm5ws.h diag bits 1-16; gemm4 store ablations 64 / 128: wrong results)
+// The persistent residual form takes three x slots where the loop outweighs its ends, long K or more than two rounds of tiles. Two
+// -> three, us: N 4096 K 14336, M 8192 | 12800 721 -> 680 | 1134 -> 1092; K 4096, M 12800 (800 tiles) 386 -> 375, M 8192 (two
+// rounds) 216 -> 219. (The non-persistent form gains at K 14336 only, 686 -> 652, and loses up to 1 % elsewhere: it keeps two.)
+constexpr int G4_X3_K = 8192;
+
 template <int MODE, int NJ = 8>
 static void launch_g4(const bf16_t* x, const u32x4* w, void* out, int M, int N, int K, int accumulate, int out_f32,
                       bf16_t* mirror, int ksplit, float rms_eps, float* ssq, hipStream_t s, const QKVArgs& qa,
@@ -1302,6 +1308,9 @@ static void launch_g4(const bf16_t* x, const u32x4* w, void* out, int M, int N, 
       } else if (rms) {
         gemm4p_kernel<MODE, 1><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps, qa,
                                                   nullptr, gm);
+      } else if (MODE == MODE_RESIDUAL && (K >= G4_X3_K || grid > 2 * num_cus())) {
+        gemm4p_kernel<MODE, 0, true><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps,
+                                                        qa, nullptr, gm);
       } else {
         gemm4p_kernel<MODE, 0><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps, qa,
                                                   nullptr, gm);

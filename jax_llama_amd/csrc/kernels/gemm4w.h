@@ -71,7 +71,9 @@ struct G4Args {
 // kept alive), 2 no LDS-DMA past the prologue (every K-tile re-reads the first two tiles' slots). (Moving the
 // sub-step's fragment reads or DMAs into its first 8 slots, two per slot, measured within noise or slower:
 // profiles/r5_gemm4_schedule_ab.jsonl.)
-template <bool RMS = false, typename Acc, int DIAG = 0, bool W3 = false>
+// X3: x three slots deep (160 KiB), its DMAs of tile t + 2 beside the first half of tile t, W's beside the second, one every second slot:
+// with two slots all 16 go out beside the second half, and the last have half a K-tile to land.
+template <bool RMS = false, typename Acc, int DIAG = 0, bool W3 = false, bool X3 = false>
 JLA_DEV void g4_mainloop(const G4Args& g, u32x4* lds, int m0, int n0, int t0, int KT, int wu, int lane, Acc& acc,
                          float* ss = nullptr) {
   const int wr = wu >> 1, wc = wu & 1;
@@ -95,14 +97,16 @@ JLA_DEV void g4_mainloop(const G4Args& g, u32x4* lds, int m0, int n0, int t0, in
     offB[j] = ((unsigned)nt * (unsigned)KS + (unsigned)(f & 1)) * 1024u + 16u * (unsigned)lane;
   }
   // slot images: two x + two W halves of 64 KiB slots, or (W3) x slots [0, 2) then three W slots
-  auto xslot = [&](int sl) -> u32x4* { return lds + sl * (W3 ? G4_A_U4 : G4_SLOT_U4); };
+  // or (X3) three x slots then two W slots
+  static_assert(!X3 || (!W3 && !RMS), "160 KiB");
+  auto xslot = [&](int sl) -> u32x4* { return lds + sl * (W3 || X3 ? G4_A_U4 : G4_SLOT_U4); };
   auto wslot = [&](int sl) -> u32x4* {
-    return W3 ? lds + 2 * G4_A_U4 + sl * G4_B_U4 : lds + sl * G4_SLOT_U4 + G4_A_U4;
+    return W3 || X3 ? lds + (X3 ? 3 : 2) * G4_A_U4 + sl * G4_B_U4 : lds + sl * G4_SLOT_U4 + G4_A_U4;
   };
-  // the j-th of this wave's 16 DMAs of K-tile t (0..7 x into x slot t & 1, 8..15 W into W slot wsl)
+  // the j-th of this wave's 16 DMAs of K-tile t (0..7 x into its x slot, 8..15 W into W slot wsl)
   auto dma = [&](int t, int j, int wsl) {
     if (j < 8) {
-      glds16(baseA + (size_t)t * 128 + offA[j], xslot(t & 1) + (wu + 4 * j) * 64);
+      glds16(baseA + (size_t)t * 128 + offA[j], xslot(X3 ? t % 3 : t & 1) + (wu + 4 * j) * 64);
     } else {
       glds16(baseB + (size_t)t * 2048 + offB[j - 8], wslot(wsl) + (wu + 4 * (j - 8)) * 64);
     }
@@ -138,7 +142,11 @@ JLA_DEV void g4_mainloop(const G4Args& g, u32x4* lds, int m0, int n0, int t0, in
           g4_mfma(acc[j][i], wf[j], xf[i]);
       }
       if (do_rd) rd(q < 8 ? wn[q] : xn[q - 8], rslot, rw, rh, q);
-      if (!(DIAG & 2) && (q < 8 ? do_dma : do_wdma)) dma(q < 8 ? td : tw, q, tws);
+      if constexpr (X3) {  // a half's 8 DMAs, one every second slot
+        if (!(DIAG & 2) && (do_dma || do_wdma) && !(q & 1)) dma(do_dma ? td : tw, (do_dma ? 0 : 8) + (q >> 1), tws);
+      } else {
+        if (!(DIAG & 2) && (q < 8 ? do_dma : do_wdma)) dma(q < 8 ? td : tw, q, tws);
+      }
       if constexpr (RMS) {
         if (q < 4) {  // m-tile 4wc + q: the runtime wc selects between two named fragments (no indexed array)
           const u32x4 f = wc ? xf[4 + q] : xf[q];
@@ -249,6 +257,33 @@ JLA_DEV void g4_mainloop(const G4Args& g, u32x4* lds, int m0, int n0, int t0, in
   }
 
   int t = 0;
+  if constexpr (X3) {
+    int xt = 0;  // t % 3
+    for (; t + 2 < KT; ++t) {
+      const int xn = xt == 2 ? 0 : xt + 1;
+      // x of tile t + 2 into the slot of t - 1 already beside the first half of t, W into t's own beside the second
+      substep(w0, x0, w1, x1, true, xt, t & 1, 1, true, t + 2, false, 0, 0);
+      __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0): all but x of tile t + 2
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      substep(w1, x1, w0, x0, true, xn, (t + 1) & 1, 0, false, 0, true, t + 2, t & 1);
+      xt = xn;
+    }
+    if (t + 1 < KT) {  // second to last: nothing left to DMA
+      const int xn = xt == 2 ? 0 : xt + 1;
+      substep(w0, x0, w1, x1, true, xt, t & 1, 1, false, 0, false, 0, 0);
+      mid_barrier();
+      substep(w1, x1, w0, x0, true, xn, (t + 1) & 1, 0, false, 0, false, 0, 0);
+      xt = xn;
+      ++t;
+    }
+    if (t < KT) {  // last K-tile
+      substep(w0, x0, w1, x1, true, xt, t & 1, 1, false, 0, false, 0, 0);
+      substep(w1, x1, w0, x0, false, 0, 0, 0, false, 0, false, 0, 0);
+    }
+    g4_acc_fence();
+    return;
+  }
   for (; t + 2 < KT; ++t) {  // steady state: reads of tile t+1 and DMA of tile t+2 in every K-tile
     substep(w0, x0, w1, x1, true, t & 1, t & 1, 1, false, 0, false, 0, 0);
     mid_barrier();

@@ -176,6 +176,24 @@ def test_gemm4_model_prefill_matches_gemm2():
     _close(got, base, 2e-2, 2e-2)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 512, 8192), (300, 512, 8256), (257, 512, 8320), (4352, 8192, 64), (4352, 8192, 128),
+                                   (4300, 8192, 192), (4352, 8192, 256)])
+def test_gemm4_persistent_residual_three_slots(m, n, k):
+    """The persistent residual form with three x slots (long K, or more than two rounds of tiles; every phase of the slots and
+    one to four K-tiles) runs the same chain of products as tile 7: bit-identical."""
+    e = ops.ext()
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    x = torch.randn(m, k, device=DEV, generator=g).to(BF16)
+    w = PackedLinear.from_dense((torch.randn(n, k) * 0.05).to(BF16), DEV)
+    h0 = torch.randn(m, n, device=DEV, generator=g)
+    outs = []
+    for tile in (13, G4):
+        h, mir = h0.clone(), torch.empty(m, n, dtype=BF16, device=DEV)
+        e.gemm(x, w.weight, n, k, h, ops.MODE_RESIDUAL, True, mir, 1, None, -1.0, tile)
+        outs.append((h, mir))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("tile", [13, 14])
 @pytest.mark.parametrize("m,n,k", [(2048, 4096, 1024), (700, 2560, 512), (4352, 1536, 256), (256, 1280, 192),
                                    (256, 2048, 128), (300, 1024, 64)])
