@@ -608,7 +608,7 @@ void topk_merge(Tensor cv, Tensor ci, int64_t k, int64_t mode, c10::optional<Ten
             ci.scalar_type() == torch::kInt32,
         "topk_merge: candidates [B, C] fp32/int32");
   const int64_t b = cv.size(0), c = cv.size(1);
-  check(k >= 1 && k <= 64 && k <= c && c <= 4096, "topk_merge: 1 <= k <= 64, k <= C <= 4096");
+  check(k >= 1 && k <= 64 && k <= c && c <= jla::TOPK_MAX_CANDIDATES, "topk_merge: 1 <= k <= 64, k <= C <= 16384");
   float* ov = nullptr;
   int32_t* oi = nullptr;
   int32_t* nx = nullptr;

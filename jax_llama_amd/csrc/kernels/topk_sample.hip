@@ -25,7 +25,7 @@
 
 namespace jla {
 
-constexpr int TK_THREADS = 256, TK_E = 16, TK_CHUNK = TK_THREADS * TK_E, TK_MAX_E = 64;
+constexpr int TK_THREADS = 256, TK_E = 16, TK_CHUNK = TK_THREADS * TK_E, TK_MAX_E = TOPK_MAX_CANDIDATES / TK_THREADS;
 
 JLA_DEV uint32_t fkey(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -317,7 +317,7 @@ int topk_chunk(const float* logits, int B, int V, int K, int idx_offset, float* 
 int topk_merge(const float* cv, const int32_t* ci, int B, int C, int K, int mode, float* out_v, int32_t* out_i,
                int32_t* nxt, float temperature, float top_p, uint64_t seed, const int32_t* step, hipStream_t s) {
   if (B <= 0) return 0;
-  if (K < 1 || K > 64 || K > C || C > TK_THREADS * TK_MAX_E) return -1;
+  if (K < 1 || K > 64 || K > C || C > TOPK_MAX_CANDIDATES) return -1;
   if (mode == 1 && (!nxt || !step || !(temperature > 0.f))) return -2;
 #define JLA_TKM(E)                                                                                          \
   topk_merge_kernel<E><<<B, TK_THREADS, 0, s>>>(cv, ci, C, K, mode, out_v, out_i, nxt, 1.0f / temperature, top_p, \

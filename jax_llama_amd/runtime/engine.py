@@ -94,7 +94,8 @@ def _sample(model, logits_local: torch.Tensor, gc: GenerationConfig, gen: Option
     v_local = logits_local.shape[1]
     k = min(gc.top_k or 0, v_local * comm.size)
     if step is not None and 1 <= k <= ops.SAMPLER_MAX_K and gc.temperature and gc.temperature > 0:
-        if logits_local.device.type == "cpu" or (ops.ext().topk_chunks(v_local) + 3) // 4 * min(k, v_local) <= 4096:
+        # (vocabularies of up to 4096 / k times 16384 columns a rank, for which the merge's limit has room; larger ones sort)
+        if logits_local.device.type == "cpu" or -(-v_local // 16384) * min(k, v_local) <= 4096:
             return ops.topk_sample(logits_local.float().contiguous(), k, gc.temperature, gc.top_p,
                                    gc.seed, step, comm if comm.size > 1 else None)
     x = logits_local.float()

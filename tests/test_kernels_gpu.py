@@ -649,6 +649,43 @@ def test_topk_candidates_prefilter_fallbacks(case):
     assert torch.equal(gv.cpu(), rv)
 
 
+@pytest.mark.parametrize("case", ["random", "flat", "ties"])
+@pytest.mark.parametrize("v,k", [(150000, 64), (300001, 64), (600000, 64), (1048576, 64), (2000000, 33)])
+def test_topk_candidates_of_many_chunks(v, k, case):
+    """Merges of more than 2048 and 4096 candidates and as many as there may be, with the exact select for rows that are flat or tied."""
+    b = 2
+    logits = torch.randn(b, v, generator=torch.Generator().manual_seed(k)) * 4
+    if case == "flat":
+        logits[:] = -1.0
+    elif case == "ties":
+        logits[:, ::997] = 30.0  # more than a merge's threads, in every chunk
+        logits[1, v - 1] = 31.0
+    gv, gi = ops.topk_candidates(logits.to(DEV), k)
+    rv, ri = ref.topk_sorted(logits, k)
+    assert torch.equal(gi.cpu(), ri) and torch.equal(gv.cpu(), rv)
+    st = torch.tensor([3], dtype=torch.int32, device=DEV)
+    got = ops.topk_sample(logits.to(DEV), k, 0.8, 0.9, 21, st)
+    assert torch.equal(got.cpu(), ref.topk_sample(logits, k, 0.8, 0.9, 21, 3))
+
+
+@pytest.mark.parametrize("v,k", [(128256, 50), (262145, 64), (1048576, 64), (1048577, 64)])
+def test_sampler_takes_what_generation_sends_it(v, k):
+    """The engine's rule for sampling on the device and the merge's limit agree: the first three do, the last goes another way."""
+    import types
+
+    from jax_llama_amd.runtime import engine as eng
+    from jax_llama_amd.runtime.engine import GenerationConfig
+    logits = torch.randn(2, v, generator=torch.Generator().manual_seed(v)) * 3
+    model = types.SimpleNamespace(comm=types.SimpleNamespace(size=1, rank=0))
+    gc = GenerationConfig(max_length=8, do_sample=True, temperature=0.7, top_k=k, top_p=0.9, seed=5)
+    st = torch.tensor([4], dtype=torch.int32, device=DEV)
+    got = eng._sample(model, logits.to(DEV), gc, torch.Generator(device=DEV).manual_seed(1), st).cpu()
+    if v <= 1048576:
+        assert torch.equal(got, ref.topk_sample(logits, k, 0.7, 0.9, 5, 4))
+    else:
+        assert all(int(t) in row.topk(k).indices for t, row in zip(got, logits))
+
+
 @pytest.mark.parametrize("b,v,k,temp,top_p", [(16, 128256, 50, 1.0, 1.0), (8, 32000, 50, 0.7, 0.9),
                                               (4, 1000, 64, 1.3, 0.5), (2, 50, 1, 1.0, 1.0)])
 def test_topk_sample_matches_reference(b, v, k, temp, top_p):
