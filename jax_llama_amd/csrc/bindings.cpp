@@ -584,7 +584,7 @@ void gemm_argmax(Tensor x, Tensor w, int64_t n, int64_t k, Tensor ws, double rms
      "gemm_argmax");
 }
 
-// stage 1 of the sampler: per-4096-chunk top-K candidates (global indices = local + idx_offset)
+// stage 1 of the sampler: per-8192-chunk top-K candidates (global indices = local + idx_offset)
 void topk_chunk(Tensor logits, int64_t k, int64_t idx_offset, Tensor cv, Tensor ci) {
   for (auto* t : {&logits, &cv, &ci}) check_gpu(*t, "topk_chunk arg");
   check(logits.scalar_type() == torch::kFloat32 && logits.dim() == 2, "logits must be fp32 [B, V]");
@@ -608,7 +608,7 @@ void topk_merge(Tensor cv, Tensor ci, int64_t k, int64_t mode, c10::optional<Ten
             ci.scalar_type() == torch::kInt32,
         "topk_merge: candidates [B, C] fp32/int32");
   const int64_t b = cv.size(0), c = cv.size(1);
-  check(k >= 1 && k <= 64 && k <= c && c <= jla::TOPK_MAX_CANDIDATES, "topk_merge: 1 <= k <= 64, k <= C <= 16384");
+  check(k >= 1 && k <= 64 && k <= c && c <= jla::TOPK_MAX_CANDIDATES, "topk_merge: 1 <= k <= 64, k <= C <= 8192");
   float* ov = nullptr;
   int32_t* oi = nullptr;
   int32_t* nx = nullptr;

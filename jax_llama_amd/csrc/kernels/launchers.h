@@ -152,7 +152,7 @@ int attn_prefill(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, const int3
 long long argmax_workspace(int B, int V);
 int argmax(const float* logits, int B, int V, int32_t* idx, float* val, float* ws, hipStream_t s);
 // top-k / top-p sampler (topk_sample.hip): cv/ci [B, topk_chunks(V) * K] candidates, of which a merge takes TOPK_MAX_CANDIDATES
-constexpr int TOPK_MAX_CANDIDATES = 16384;
+constexpr int TOPK_MAX_CANDIDATES = 8192;
 int topk_chunks(int V);
 int topk_chunk(const float* logits, int B, int V, int K, int idx_offset, float* cv, int32_t* ci, hipStream_t s);
 int topk_merge(const float* cv, const int32_t* ci, int B, int C, int K, int mode, float* out_v, int32_t* out_i,

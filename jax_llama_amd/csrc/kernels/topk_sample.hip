@@ -3,10 +3,9 @@
 // generation.py:28-41 with do_sample = temperature != 0, top_k = 50).
 //
 // Two kernels, no host sync, hipGraph-capturable:
-//   topk_chunk:  grid (ceil(V/4096), B). A 256-thread workgroup holds a 4096-logit chunk in registers (16 keys per thread,
-//                order-preserving uint32 of the fp32 logit, whole lines per load). A bound that at least K keys reach comes from the
-//                threads' maxima (LDS radix select, 8 bits per pass, one wave scans the 256-bin histogram with lane moves, two passes);
-//                the survivors, about K, rank themselves by counting the better ones. It emits exactly K candidates, sorted.
+//   topk_chunk:  grid (ceil(V/8192), B). A 256-thread workgroup holds a chunk of 8192 logits in registers, 32 per thread, in whole lines
+//                per load. A bound that at least K of them reach comes from the threads' maxima, wave by wave (16 ballots); the survivors, about
+//                1.5 K, rank themselves by counting the better ones, a fourth of the list per wave. It emits exactly K candidates, sorted.
 //   topk_merge:  one workgroup per row ranks the C = chunks*K candidates the same way, and either writes
 //                them (vocab-parallel TP: each rank's top-K is all-gathered, 400 B per rank per row,
 //                then merged again -- exact, since the global top-K is inside the union) or samples:
@@ -14,18 +13,20 @@
 //                probability mass strictly before it is < top_p; the first always survives), then
 //                Gumbel-max with counter-based Philox4x32-10 keyed by (seed, step, row, rank) -- every
 //                TP rank draws the same token from the same candidates without communicating.
-// More survivors than threads (flat, tied or clustered keys): the exact select on all keys of the chunk.
+// More survivors than threads (flat, tied or clustered keys, mostly -inf), and always a last chunk of fewer than K + 3 columns: the exact select
+// (four radix passes over keys as order-preserving uint32) on all keys of the chunk, read again for every pass.
 // Ties: lower vocabulary index first (lax.top_k order).
-// What bounds it: dependent steps within a wave and code on its path (some 0.13 us per KB in a launch of a few us). Seven rows x 128256 columns, the
-// two kernels: 64 keys per thread in 8 chunks, read 256 bytes apart, exact select and sort of the survivors in six radix passes and 21 exchanges
-// 10.9 + 8.9 us; here 6.2 + 9.4. Warm, both, before -> now: 1 row 17.7 -> 14.7, 7 18.0 -> 15.1, 64 20.9 -> 20.7, 300 42.0 -> 44.5, 1400 186 -> 184;
-// 200 x 32000 22.8 -> 19.5. (32 keys per thread: 7 rows 16.0, 1400 302; the rare case's keys in registers: 1400 203.)
+// What bounds it: of few rows the dependent steps and the code on their path (some 0.13 us per KB in a launch of a few us), of many the vector unit's
+// issue and the logits' bytes. Warm, both launches, top 50, us: chunks of 16384 with two radix selects and a sort | of 4096, bound by a radix select
+// | here: 128256 columns, 1 row 17.4 | 13.7 | 11.7, 7 17.7 | 14.9 | 12.1, 64 20.5 | 20.1 | 16.8, 300 42.0 | 43.0 | 34.1, 1400 188 | 182 | 141; 32000,
+// 1 row 19.6 | 12.4 | 9.9, 1400 57.4 | 66.0 | 36.5; top 64 of 300 x 128256 42.0 | 62.4 | 35.7. Chunks of 4096 here: 1 x 16032 9.1 for 10.5, 300 x
+// 128256 39.1, 1400 x 32000 43.9.
 #include "common.h"
 #include "launchers.h"
 
 namespace jla {
 
-constexpr int TK_THREADS = 256, TK_E = 16, TK_CHUNK = TK_THREADS * TK_E, TK_MAX_E = TOPK_MAX_CANDIDATES / TK_THREADS;
+constexpr int TK_THREADS = 256, TK_E = 32, TK_CHUNK = TK_THREADS * TK_E, TK_MAX_E = TOPK_MAX_CANDIDATES / TK_THREADS;
 
 JLA_DEV uint32_t fkey(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -35,21 +36,19 @@ JLA_DEV float kfloat(uint32_t k) { return __uint_as_float((k & 0x80000000u) ? (k
 
 struct TkShared {
   uint32_t hist[256];
-  uint32_t wsum[TK_THREADS / 64];
+  uint32_t wsum[TK_THREADS / 64], bound[TK_THREADS / 64];
   uint32_t sel[2];
   uint64_t c[TK_THREADS];   // survivors: key, then the index from its end (the better of two is the larger)
-  uint32_t total;
+  uint64_t best[64];        // merge: the best K
 };
 
 // Block-wide radix select over E keys per thread, key(j) the j-th: T = the K-th largest key; need_eq = how many
 // keys equal to T are part of the top K (all keys > T are). Requires K <= number of keys.
-// last_shift 16: two passes only, T = the K-th largest key with its low 16 bits cleared (a lower bound with at least K
-// keys >= T; need_eq is then meaningless).
 template <class Key>
-JLA_DEV void radix_select(int E, Key key, int K, TkShared& sh, uint32_t& T, int& need_eq, int last_shift = 0) {
+JLA_DEV void radix_select(int E, Key key, int K, TkShared& sh, uint32_t& T, int& need_eq) {
   uint32_t prefix = 0, mask = 0;
   int kr = K;
-  for (int shift = 24; shift >= last_shift; shift -= 8) {
+  for (int shift = 24; shift >= 0; shift -= 8) {
     for (int i = threadIdx.x; i < 256; i += TK_THREADS) sh.hist[i] = 0;
     __syncthreads();
 #pragma unroll 1
@@ -103,43 +102,80 @@ JLA_DEV uint32_t block_excl_scan(uint32_t v, TkShared& sh) {
 
 JLA_DEV uint64_t tk_word(uint32_t key, int idx) { return (uint64_t)key << 32 | (uint32_t)(0x7fffffff - idx); }
 
-// The top K of the block's keys, sorted, where few enough reach the bound: calls put(slot, word) once per slot 0..K-1. word(j): key j's and its index
-// (0 .. 0x7fffffff). The bound: the top 16 bits (sign, exponent, 7 mantissa bits) of the K-th largest of the 256 per-thread maxima; at least K keys
-// reach it, and about that many of logits. False: more than threads.
-template <int E, class Word, class F>
-JLA_DEV bool select_few(const uint32_t (&key)[E], int K, TkShared& sh, Word word, F put, bool over = false) {
-  uint32_t most = 0, T0, ns = 0;
-  int none;
+// the largest number of 16 bits (of a key: sign, exponent, 7 mantissa bits), zeros behind it, that at least k lanes of the wave reach
+JLA_DEV uint32_t wave_bound(uint32_t key, int k) {
+  uint32_t t = 0;
 #pragma unroll
-  for (int j = 0; j < E; ++j) most = max(most, key[j]);
-  radix_select(1, [&](int) { return most; }, K, sh, T0, none, 16);
-#pragma unroll
-  for (int j = 0; j < E; ++j) ns += key[j] >= T0;
-  uint32_t at = block_excl_scan(ns, sh);
-  if (threadIdx.x == TK_THREADS - 1) sh.total = at + ns;
+  for (int bit = 31; bit >= 16; --bit) {
+    const uint32_t c = t | 1u << bit;
+    if (__popcll(__ballot(key >= c)) >= k) t = c;
+  }
+  return t;
+}
+
+// Survivors sh.c[0 .. S), S <= threads, in any order, sh.hist cleared: calls put(rank, word) for the best K. Every wave counts for all of them the
+// better ones in its fourth. TIED: words may be equal (then the first is the better one).
+template <bool TIED, class F>
+JLA_DEV void rank_few(int S, int K, TkShared& sh, F put) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, part = (S + 15) / 16 * 4;
+  if ((int)threadIdx.x >= S && (int)threadIdx.x < 4 * part) sh.c[threadIdx.x] = 0;  // (better than none)
   __syncthreads();
-  const int S = sh.total;
-  if (S > TK_THREADS) return false;
-#pragma unroll
-  for (int j = 0; j < E; ++j)
-    if (key[j] >= T0) sh.c[at++] = word(j);
-  if ((int)threadIdx.x >= S && threadIdx.x < ((S + 3) & ~3)) sh.c[threadIdx.x] = 0;  // (better than none)
-  __syncthreads();
-  int rank = K;
-  uint64_t own = 0;
-  if ((int)threadIdx.x < S) {
-    own = sh.c[threadIdx.x];
-    rank = 0;
-    for (int i = 0; i < S; i += 4) {
+  for (int g = 0; g < S; g += 64) {
+    const uint64_t own = sh.c[g + lane];
+    uint32_t better = 0;
+    for (int i = wave * part; i < (wave + 1) * part; i += 4) {
       uint64_t o[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) o[u] = sh.c[i + u];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) rank += o[u] > own || (o[u] == own && i + u < (int)threadIdx.x);
+      for (int u = 0; u < 4; ++u) better += o[u] > own || (TIED && o[u] == own && i + u < g + lane);
     }
+    if (g + lane < S) atomicAdd(&sh.hist[g + lane], better);
   }
-  if (over) __syncthreads();  // (put writes where others read)
-  if (rank < K) put(rank, own);
+  __syncthreads();
+  if ((int)threadIdx.x < S) {
+    const int rank = sh.hist[threadIdx.x];
+    if (rank < K) put(rank, sh.c[threadIdx.x]);
+  }
+}
+
+// A bound that at least K keys of the block reach, and of logits about 1.5 K: a fourth of K of every wave's threads hold a key that reaches their
+// wave's, `most` a thread's largest. Clears sh.hist.
+JLA_DEV uint32_t block_bound(uint32_t most, int K, TkShared& sh) {
+  constexpr int WAVES = TK_THREADS / 64;
+  const uint32_t own = wave_bound(most, (K + WAVES - 1) / WAVES);
+  if ((threadIdx.x & 63) == 0) sh.bound[threadIdx.x >> 6] = own;
+  sh.hist[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t t = sh.bound[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) t = min(t, sh.bound[w]);
+  return __builtin_amdgcn_readfirstlane(t);
+}
+
+// The top K of the block's keys, sorted, where few enough reach the bound: calls put(slot, word) once per slot 0..K-1. reaches(j): whether this
+// thread's j-th of E does; word(j): the key and its index (0 .. 0x7fffffff). False: more than threads.
+template <int E, bool TIED, class Reaches, class Word, class F>
+JLA_DEV bool select_few(Reaches reaches, int K, TkShared& sh, Word word, F put) {
+  const int wave = threadIdx.x >> 6;
+  uint32_t ns = 0;
+#pragma unroll
+  for (int j = 0; j < E; ++j) ns += reaches(j);
+  const uint32_t incl = wave_scan(ns);
+  if ((threadIdx.x & 63) == 63) sh.wsum[wave] = incl;
+  __syncthreads();
+  uint32_t at = incl - ns;
+  int S = 0;
+#pragma unroll
+  for (int w = 0; w < TK_THREADS / 64; ++w) {
+    if (w < wave) at += sh.wsum[w];
+    S += sh.wsum[w];
+  }
+  if (S > TK_THREADS) return false;
+#pragma unroll
+  for (int j = 0; j < E; ++j)
+    if (reaches(j)) sh.c[at++] = word(j);
+  rank_few<TIED>(S, K, sh, put);
   return true;
 }
 
@@ -172,20 +208,27 @@ __global__ void __launch_bounds__(TK_THREADS, 8)
   __shared__ TkShared sh;
   const int b = blockIdx.y, c = blockIdx.x, nch = gridDim.x, base = c * TK_CHUNK;
   const float* x = logits + (size_t)b * V;
-  uint32_t key[TK_E];
-  auto element = [&](int j) { return base + 4 * TK_THREADS * (j / 4) + 4 * (int)threadIdx.x + j % 4; };
-  if ((V & 3) == 0 && base + TK_CHUNK <= V) {
+  // four numbers per access; else one, and of the last few columns neighbours are dealt to the waves in turn (the bound needs K / 4 in each)
+  const bool last = V - base < 4 * TK_THREADS, vec = (V & 3) == 0 && !last;
+  const int place = last ? 4 * ((int)threadIdx.x & 63) + ((int)threadIdx.x >> 6) : (int)threadIdx.x;
+  auto element = [&](int j) { return base + (vec ? 4 * TK_THREADS * (j / 4) + 4 * (int)threadIdx.x + j % 4 : TK_THREADS * j + place); };
+  float v[TK_E];
+  if (vec && base + TK_CHUNK <= V) {
 #pragma unroll
     for (int q = 0; q < TK_E / 4; ++q) {
-      const float4 v = *reinterpret_cast<const float4*>(x + element(4 * q));
-      key[4 * q] = fkey(v.x);
-      key[4 * q + 1] = fkey(v.y);
-      key[4 * q + 2] = fkey(v.z);
-      key[4 * q + 3] = fkey(v.w);
+      const float4 f = *reinterpret_cast<const float4*>(x + element(4 * q));
+      v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
+    }
+  } else if (vec) {
+#pragma unroll
+    for (int q = 0; q < TK_E / 4; ++q) {
+      const bool in = element(4 * q) < V;
+      const float4 f = in ? *reinterpret_cast<const float4*>(x + element(4 * q)) : float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      v[4 * q] = f.x, v[4 * q + 1] = f.y, v[4 * q + 2] = f.z, v[4 * q + 3] = f.w;
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < TK_E; ++j) key[j] = element(j) < V ? fkey(x[element(j)]) : 0u;  // 0 < key(-inf)
+    for (int j = 0; j < TK_E; ++j) v[j] = element(j) < V ? x[element(j)] : -INFINITY;
   }
   float* ov = cv + ((size_t)b * nch + c) * K;
   int32_t* oi = ci + ((size_t)b * nch + c) * K;
@@ -193,8 +236,13 @@ __global__ void __launch_bounds__(TK_THREADS, 8)
     ov[slot] = e < V ? kfloat(k) : -INFINITY;
     oi[slot] = e < V ? idx_offset + e : 0x7fffffff;
   };
-  if (select_few(key, K, sh, [&](int j) { return tk_word(key[j], element(j)); },
-                 [&](int slot, uint64_t w) { put(slot, (uint32_t)(w >> 32), 0x7fffffff - (int)(uint32_t)w); }))
+  float most = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < TK_E; ++j) most = fmaxf(most, v[j]);
+  const float bound = kfloat(block_bound(fkey(most), K, sh));
+  // (not below the bound: a NaN, which comes first, is kept; where the bound is that of -inf everything is)
+  if (select_few<TK_E, false>([&](int j) { return !(v[j] < bound); }, K, sh, [&](int j) { return element(j) < V ? tk_word(fkey(v[j]), element(j)) : 0; },
+                              [&](int slot, uint64_t w) { put(slot, (uint32_t)(w >> 32), 0x7fffffff - (int)(uint32_t)w); }))
     return;
   const int first = base + TK_E * (int)threadIdx.x;  // (in element order now)
   __syncthreads();
@@ -214,9 +262,7 @@ JLA_DEV uint4 philox4x32_10(uint4 ctr, uint2 k) {
 }
 
 // mode 0: write the sorted top-K (out_v/out_i [B, K]); mode 1: sample one token per row into nxt[B].
-// E candidates per thread: the smallest that covers C, so the candidates spread over most threads and the
-// per-thread-maximum prefilter of select_topk compacts them (with TK_E per thread, 16 chunks x 50 candidates sat
-// in 25 threads and every merge fell back to the full select)
+// E candidates per thread: the smallest that covers C, so that the candidates spread over most threads and the bound from their maxima is close.
 template <int E>
 __global__ void __launch_bounds__(TK_THREADS)
     topk_merge_kernel(const float* __restrict__ cv, const int32_t* __restrict__ ci, int C, int K, int mode,
@@ -227,26 +273,42 @@ __global__ void __launch_bounds__(TK_THREADS)
   const int b = blockIdx.x;
   const float* bv = cv + (size_t)b * C;
   const int32_t* bi = ci + (size_t)b * C;
-  uint32_t key[E];
-  int32_t at[E];
+  auto put = [&](int slot, uint64_t w) { sh.best[slot] = w; };
+  bool few = true;
+  if constexpr (E == 1) {  // every candidate is ranked
+    if ((int)threadIdx.x < C) sh.c[threadIdx.x] = tk_word(fkey(bv[threadIdx.x]), bi[threadIdx.x]);
+    sh.hist[threadIdx.x] = 0;
+    rank_few<true>(C, K, sh, put);
+  } else {
+    // (the candidates of a chunk are sorted: dealt to the waves in turn and, turned by 37 threads from one 256 to the next, to threads of
+    // their own, whatever K divides, so that the bound is close: K 64 without the turn: 16 threads in 64 held the best of every chunk, and
+    // from 20 chunks on more candidates than threads reached it)
+    auto from = [&](int j) { return (4 * ((int)threadIdx.x & 63) + ((int)threadIdx.x >> 6) + 37 * j) % TK_THREADS + TK_THREADS * j; };
+    constexpr int AT = E <= 16 ? E : 1;  // indices held; of more candidates they are read where needed (registers)
+    uint32_t key[E], most = 0;
+    int32_t at[AT];
 #pragma unroll
-  for (int j = 0; j < E; ++j) {  // (a chunk's candidates are sorted: dealt out, so that the threads' maxima are the row's best)
-    const int e = threadIdx.x + TK_THREADS * j;
-    key[j] = e < C ? fkey(bv[e]) : 0u;
-    at[j] = e < C ? bi[e] : 0x7fffffff;
+    for (int j = 0; j < E; ++j) {
+      const int e = from(j);
+      key[j] = e < C ? fkey(bv[e]) : 0u;
+      if constexpr (AT == E) at[j] = e < C ? bi[e] : 0x7fffffff;
+      most = max(most, key[j]);
+    }
+    const uint32_t bound = block_bound(most, K, sh);
+    few = select_few<E, true>([&](int j) { return key[j] >= bound; }, K, sh,
+                              [&](int j) { return tk_word(key[j], AT == E ? at[j % AT] : (from(j) < C ? bi[from(j)] : 0x7fffffff)); }, put);
   }
-  const bool few = select_few(key, K, sh, [&](int j) { return tk_word(key[j], at[j]); }, [&](int slot, uint64_t w) { sh.c[slot] = w; }, true);
   if (!few) {
     const int base = threadIdx.x * E;
     __syncthreads();
     select_all(E, [&](int j) { return base + j < C ? fkey(bv[base + j]) : 0u; }, K, sh,
-               [&](int slot, uint32_t k, int j) { sh.c[slot] = tk_word(k, base + j < C ? bi[base + j] : 0x7fffffff); });
+               [&](int slot, uint32_t k, int j) { sh.best[slot] = tk_word(k, base + j < C ? bi[base + j] : 0x7fffffff); });
   }
   __syncthreads();
   if (threadIdx.x >= 64) return;
   const int lane = threadIdx.x;
   // value descending, then index ascending
-  uint64_t v = lane < K ? sh.c[lane] : 0ull;
+  uint64_t v = lane < K ? sh.best[lane] : 0ull;
   if (!few) {
 #pragma unroll
     for (int k = 2; k <= 64; k <<= 1) {
@@ -322,7 +384,9 @@ int topk_merge(const float* cv, const int32_t* ci, int B, int C, int K, int mode
 #define JLA_TKM(E)                                                                                          \
   topk_merge_kernel<E><<<B, TK_THREADS, 0, s>>>(cv, ci, C, K, mode, out_v, out_i, nxt, 1.0f / temperature, top_p, \
                                                 (uint32_t)seed, (uint32_t)(seed >> 32), step)
-  if (C <= 4 * TK_THREADS)
+  if (C <= TK_THREADS / 2)
+    JLA_TKM(1);
+  else if (C <= 4 * TK_THREADS)
     JLA_TKM(4);
   else if (C <= 8 * TK_THREADS)
     JLA_TKM(8);

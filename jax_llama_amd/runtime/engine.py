@@ -87,7 +87,7 @@ def _sample(model, logits_local: torch.Tensor, gc: GenerationConfig, gen: Option
             step: Optional[torch.Tensor] = None):
     """temperature -> top-k -> top-p -> categorical (Gumbel-max), exact under vocab sharding.
 
-    top_k in [1, 64] (HF default 50): the on-device sampler (ops.topk_sample: radix-select top-k
+    top_k in [1, 64] (HF default 50): the on-device sampler (ops.topk_sample: exact top-k
     kernels + Philox Gumbel-max keyed by (seed, step)), graph-capturable and identical on CPU.
     Otherwise (top_k = 0 / > 64): torch sort path."""
     comm = model.comm

@@ -630,6 +630,36 @@ def test_topk_candidates_at_chunk_edges(v):
     assert torch.equal(gi.cpu(), ri) and torch.equal(gv.cpu(), rv)
 
 
+@pytest.mark.parametrize("v,k", [(8191, 64), (8192, 64), (8193, 50), (8192 + 52, 50), (8192 + 53, 50), (8195, 3), (9215, 64), (9216, 64), (9217, 64),
+                                 (16388, 50), (20003, 17)])
+def test_topk_candidates_at_the_ends_of_chunks_of_8192(v, k):
+    """Last chunks of a few columns (fewer than K + 3: the exact select), of up to 1024, and more, aligned and not; the best in the last columns; NaNs first."""
+    logits = torch.randn(3, v, generator=torch.Generator().manual_seed(v + k)) * 4
+    logits[1, -(v % 8192 or 5):] += 20
+    logits[2, v // 2:v // 2 + 2] = float("nan")
+    gv, gi = ops.topk_candidates(logits.to(DEV), k)
+    rv, ri = ref.topk_sorted(logits[:2], k)
+    assert torch.equal(gi[:2].cpu(), ri) and torch.equal(gv[:2].cpu(), rv)
+    rest = logits[2].clone()
+    rest[v // 2:v // 2 + 2] = float("-inf")
+    assert gi[2, :2].tolist() == [v // 2, v // 2 + 1] and torch.equal(gi[2, 2:].cpu(), ref.topk_sorted(rest[None], k)[1][0, :k - 2])
+
+
+@pytest.mark.parametrize("chunks,k", [(1, 64), (2, 64), (3, 50), (4, 64), (16, 64), (17, 64), (32, 64), (33, 64), (64, 64), (65, 64), (128, 64), (1, 1), (40, 32)])
+def test_merge_of_sorted_lists(chunks, k):
+    """Lists of which each has its best first, as chunks and ranks emit them, in every form of the merge; equal numbers, and padding behind them."""
+    g = torch.Generator().manual_seed(chunks * k)
+    v = (torch.randn(2, chunks, k, generator=g) * 3).sort(-1, descending=True).values
+    v[1] = v[1].round() + 0.0  # (no -0.0: the kernel has it behind 0.0)
+    i = (torch.arange(chunks)[:, None] * 1000 + torch.arange(k)).expand(2, chunks, k).to(torch.int32).contiguous()
+    if k > 8:
+        v[:, -1, k // 2:], i[:, -1, k // 2:] = float("-inf"), 0x7fffffff
+    out_v, out_i = torch.empty(2, k, device=DEV), torch.empty(2, k, dtype=torch.int32, device=DEV)
+    ops.ext().topk_merge(v.view(2, -1).to(DEV), i.view(2, -1).to(DEV), k, 0, out_v=out_v, out_i=out_i)
+    rv, at = ref.topk_sorted(v.view(2, -1), k)
+    assert torch.equal(out_v.cpu(), rv) and torch.equal(out_i.cpu(), i.view(2, -1).gather(1, at.long()))
+
+
 @pytest.mark.parametrize("case", ["block", "flat", "ties"])
 def test_topk_candidates_prefilter_fallbacks(case):
     """Chunks whose survivors of the per-thread-maximum prefilter exceed one per thread (a run of 300 large
