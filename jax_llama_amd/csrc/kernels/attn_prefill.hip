@@ -292,7 +292,8 @@ __global__ void __launch_bounds__(NW * 64, 2)
   const int wg_last_pos = min(S, (qb + 1) * QW * npb) - 1;
   const int last_key = min(slot0 + wg_last_pos, T - 1);
   const int t_begin = (lo / FA_KT) * FA_KT;
-  const int wave_last_slot = slot0 + min(p0 + QW - 1, S - 1);
+  // (a wave behind the last query only helps to stage: 1000 rows of 33 queries, 32 kv heads, 404 -> 364 us)
+  const int wave_last_slot = p0 < S ? slot0 + min(p0 + QW - 1, S - 1) : -1;
   const bf16_t* kb = kc + ((size_t)b * Hkv + kvh) * T * AP_DH;
   const bf16_t* vb = vc + ((size_t)b * Hkv + kvh) * T * AP_DH;
 

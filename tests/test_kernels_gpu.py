@@ -328,6 +328,30 @@ def test_attention_prefill_tile_edges(impl, s, slot0, masked):
     assert (got.float() - want).abs().max().item() < bound
 
 
+@pytest.mark.parametrize("impl", [7, 13])
+@pytest.mark.parametrize("rep,s,slot0", [(1, 2, 0), (1, 32, 0), (1, 33, 64), (1, 97, 3), (1, 257, 0), (1, 289, 30), (2, 17, 127), (2, 130, 0), (8, 33, 0),
+                                         (8, 129, 65)])
+def test_attention_prefill_waves_without_queries(impl, rep, s, slot0):
+    """Workgroups whose last waves have no query: they stage and compute nothing, the others' rows are what they are."""
+    e = ops.ext()
+    b, hkv, dh, t = 2, 2, 128, slot0 + s
+    g = torch.Generator(device=DEV).manual_seed(7 * s + rep)
+    kc = (torch.randn(b, hkv, t, dh, device=DEV, generator=g) * 2).to(BF16)
+    vc = torch.randn(b, hkv, t, dh, device=DEV, generator=g).to(BF16)
+    q = (torch.randn(b, s, hkv * rep, dh, device=DEV, generator=g) * 2).to(BF16)
+    kv_start = torch.tensor([0, t // 3], dtype=torch.int32, device=DEV)
+    slot = torch.tensor([slot0], dtype=torch.int32, device=DEV)
+    try:
+        e.attn_prefill_set_impl(impl)
+        got = ops.attention(q, kc, vc, slot, kv_start)
+        torch.cuda.synchronize()
+    finally:
+        e.attn_prefill_set_impl(2)
+    want = _attn_ref_gpu(q, kc, vc, slot0, kv_start)
+    # P and the result are rounded to bf16 (2^-9 each of a weighted mean of values), the rest is fp32
+    assert (got.float() - want).abs().max().item() < 2 * 2.0 ** -9 * vc.float().abs().max().item() + 1e-3
+
+
 def test_attention_prefill_8k():
     """S = 8192 causal prefill (Llama-3 max_seq_len), rep 4, one batch row."""
     b, hkv, rep, s, dh = 1, 2, 4, 8192, 128
