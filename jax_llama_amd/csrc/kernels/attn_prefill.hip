@@ -226,7 +226,7 @@ JLA_DEV u32x2 ld_tr(const char* lds, int off) {
 // first key step has no MFMA beside it. The max exchange of the two lane halves is a permlane32 swap, the halves of the
 // sum meet once at the end, two tiles are unrolled (constant LDS slots, no scores moved), and the masks take a lane's
 // two limits instead of 32 key indexes held in registers.
-// Measured (32 heads, 8 kv heads of 128, causal): S = 8192 604 -> 496 us (1.1 PFLOP/s), 16 x 2048 735 -> 623 us,
+// Measured (32 heads, 8 kv heads of 128, causal): S = 8192 604 -> 496 us (1.1 PFLOP/s), 16 x 2048 735 -> 649 us,
 // S = 2048 62.5 -> 50.7, S = 600 with 32 kv heads 26.3 -> 20.0, 2048 x 128 1411 -> 1325 us.
 // Lazy rescale (every launch): the running max (and with it the O / l rescale) moves only when a lane's tile max
 // exceeds it by more than 8 (log2 units): exp2 of the rest stays <= 256, exact in fp32 and bf16-representable for P;
@@ -513,8 +513,8 @@ static void launch_prefill_v2(const bf16_t* q, const bf16_t* kc, const bf16_t* v
   }
 }
 
-// impl (attn_prefill_set_impl, A/B): 2 = default dispatch; 7 (and 8) = 4 waves per workgroup, 13 (and 9) = 8 waves; 1 =
-// the v1 kernel (also the fallback for a non-power-of-two GQA ratio)
+// impl (attn_prefill_set_impl, A/B): 2 = default dispatch; 7 = 4 waves per workgroup, 13 = 8 waves; 1 = the v1 kernel (also the
+// fallback for a non-power-of-two GQA ratio)
 static int g_attn_prefill_impl = 2;
 void attn_prefill_set_impl(int impl) { g_attn_prefill_impl = impl; }
 
@@ -527,19 +527,22 @@ int attn_prefill(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, const int3
   const bool pow2rep = rep == 1 || rep == 2 || rep == 4 || rep == 8;
   int impl = g_attn_prefill_impl;
   // default (impl 2): 8 waves per workgroup (twice the queries per staged K / V tile, one workgroup resident per CU)
-  // where the prompt is long and the paired grid's rounds over the 256 CUs are nearly full (a last round of >= 90 %; with
-  // one round, >= 75 %), else 4 waves. Measured, 4 -> 8 waves, us: S = 4096 143 -> 133 (one full round), 2 x 4096 279 -> 265
-  // (two), S = 3000 103 -> 89 (192 workgroups), 124 -> 107 (240); but S = 4096 226 -> 250 (320), 4 x 1500 101 -> 111 (384),
-  // S = 1500 39 -> 53 (96); at S <= 1024 4 waves are ahead nearly everywhere (16 x 512 76 -> 79, 64 x 128 60 -> 83): a query
+  // where the prompt is long, the paired grid's rounds over the 256 CUs are nearly full (a last round of >= 90 %; with
+  // one round, >= 75 %) and so are the workgroups' query rows (>= 73 % of what the rounds have room for: an odd number of query blocks leaves
+  // half a pair, the last block may be nearly empty), else 4 waves. Measured, 4 -> 8 waves, us: S = 4096 143 -> 133 (one full round), 2 x 4096
+  // 279 -> 265 (two), S = 3000 103 -> 89 (192 workgroups), 124 -> 107 (240); but S = 4096 226 -> 250 (320), 4 x 1500 101 -> 111 (384),
+  // S = 1500 39 -> 53 (96); of 32 kv heads 2 x 1025 39 -> 54 (192, rows 50 %), 2 x 1300 57 -> 60 (192, 63 %), 16 x 1100 293 -> 326 (1536, 72 %),
+  // of 40 4 x 1200 118 -> 110 (480, 73 %), of 32 2 x 1531 67 -> 63 (192, 75 %); at S <= 1024 4 waves are ahead nearly everywhere (16 x 512 76 -> 79, 64 x 128 60 -> 83): a query
   // block is then twice as many rows for the same few tiles.
   if (impl == 2 && pow2rep) {
     const int npb8 = rep >= 8 ? 1 : 8 / rep;
     const int n_qb8 = (S + 32 * npb8 - 1) / (32 * npb8);
     const long long wg8 = (long long)((n_qb8 + 1) / 2) * Hkv * (rep / (8 / npb8)) * B;
     const long long rounds = (wg8 + 255) / 256;
-    impl = S > 1024 && (10 * wg8 >= 9 * 256 * rounds || (rounds == 1 && wg8 >= 192)) ? 13 : 7;
+    const long long rows = (long long)S * Hkv * (rep / (8 / npb8)) * B;  // a workgroup takes 64 npb8
+    impl = S > 1024 && (10 * wg8 >= 9 * 256 * rounds || (rounds == 1 && wg8 >= 192)) && 100 * rows >= 73LL * 256 * rounds * 64 * npb8 ? 13 : 7;
   }
-  const int nw = impl == 7 || impl == 8 ? 4 : impl == 9 || impl == 13 ? 8 : 0;
+  const int nw = impl == 7 ? 4 : impl == 13 ? 8 : 0;
   if (nw && (rep % nw == 0 || nw % rep == 0)) {
     if (nw == 4)
       launch_prefill_v2<4>(q, kc, vc, slot, kv_start, key_mask, mask_len, out, B, S, H, Hkv, T, rep, s);
