@@ -236,21 +236,22 @@ bool hy_rows_gemm_pays(const RowLinear& p) {
 }
 
 // A form's measured times, us: launch and fill; a 64-deep step of one workgroup; its rise with every further one of a compute unit, whose
-// last round counts as `last` workgroups more
+// last round counts as `last` workgroups more; what such a one takes besides (of one workgroup per unit nobody hides its first copies and its stores)
 struct RgForm {
   int nj, mi;
-  float fill, step, more, last;
+  float fill, step, more, last, ends;
 };
-static const RgForm RG_FORMS[] = {{4, 4, 1.0f, 0.644f, 0.833f, 1.0f}, {4, 5, 9.75f, 0.608f, 0.965f, 0.99f}, {4, 6, 5.17f, 0.819f, 0.795f, 0.945f},
-                                  {8, 8, 16.3f, 1.31f, 1.3f, 1.0f}};
+static const RgForm RG_FORMS[] = {{4, 4, 1.0f, 0.644f, 0.833f, 1.0f, 0.f}, {4, 5, 9.75f, 0.608f, 0.965f, 0.99f, 0.f},
+                                  {4, 6, 5.17f, 0.819f, 0.795f, 0.945f, 0.f}, {8, 8, 22.f, 1.3f, 1.2f, 1.0f, 8.f}};
 
-// The form with the least time by the figures above: on average 1.8 % above the best of those measured (54 products: 8 experts of 2816 x
-// 2048 and 7168 x 4096 with 1000 to 12000 rows, one matrix of 5632 x 2048 with 300 to 4000, gated and down), where 256-row tiles, 128 or 256
-// wide, took 1.22 times as long. With experts, whose counts only the device knows, the row tiles are a mean over four
-// counts around the average. Eight rounds of 256 x 256 tiles and more: these (8 experts of gated 7168 x 4096, 6000 | 12000 rows 667 | 1295, 192
-// x 128 688 | 1336: fewer bytes cost less power). These figures are of two slots for both operands; the 256 x 256 form's are scaled by what
-// the third gave it (0.93), by which it is now chosen for more: 8 experts of 7168 x 4096, both products, 9000 | 6000 rows 1582 | 1083 -> 1481 |
-// 988 us, of 2816 x 2048, 12000 rows 495 -> 467; scaled by 0.82 instead, 8000 rows of 2816 x 2048 and the like lose 3 to 5 %.
+// The form with the least time by the figures above: on average 4.0 % above the best of those measured (375 products, gated and down: 2 to 32
+// experts and one matrix, 300 to 24000 rows, K 1024 to 14336, rows dealt unevenly as the rule cannot know). With experts, whose counts only
+// the device knows, the row tiles are a mean over four counts around the average. Eight rounds of 256 x 256 tiles and more: these (8 experts of
+// gated 7168 x 4096, 6000 | 12000 rows 667 | 1295, 192 x 128 688 | 1336: fewer bytes cost less power).
+// The third slot of the 256 x 256 form takes its time off every step, not off a round's ends: of a short K the 192-row tiles stay ahead. Us, 192 rows |
+// 256: 8 experts of 4096 x 7168, 9000 rows 590 | 507, gated 7168 x 4096, 6000 rows 740 | 667, 4 of 5120 x 3584, 24000 rows 865 | 760; but 4
+// of 1024 x 2048, 24000 rows 98 | 115, 16 of 2048 x 1408, 12000 rows 87 | 93, gated 2048 x 1024, 24000 rows 211 | 236, 8 of 2816 x 2048, 4000
+// rows 111 | 115, clamped 119 | 132. (Figures without `ends`: 4.4 % above the best, and those of two slots 4.6 %.)
 constexpr long long RG_MANY = 8 * 256;
 
 static const RgForm& rg_form(const RowLinear& p) {
@@ -266,7 +267,7 @@ static const RgForm& rg_form(const RowLinear& p) {
     const float tiles = mt * .25f * (float)E * (float)((wrows + 32 * f.nj - 1) / (32 * f.nj)), load = tiles / 256.f;
     if (f.mi == 8 && tiles >= (float)RG_MANY) return f;
     const float deep = f.mi == 8 ? ceilf(load - .02f) : (load <= 1.f ? 1.f : (load <= 2.f ? 2.f : load + f.last));
-    float us = f.fill + f.step * (float)(p.K / RG_BK) * (1.f + f.more * (deep - 1.f));
+    float us = f.fill + f.ends * (deep - 1.f) + f.step * (float)(p.K / RG_BK) * (1.f + f.more * (deep - 1.f));
     if (us < stream) us = stream;
     if (us < least) {
       least = us;
