@@ -8,6 +8,10 @@ namespace jla {
 JLA_DEV void lr_out(float* p, float v) { *p = v; }
 JLA_DEV void lr_out(bf16_t* p, float v) { *p = f2bf(v); }
 
+JLA_DEV float lr_clamp_glu(const RowLinear& p, float g, float u) {
+  const float gc = fminf(g, p.act_limit), uc = fminf(fmaxf(u, -p.act_limit), p.act_limit);
+  return gc * hy_sigmoid(p.act_alpha * gc) * (uc + 1.f);
+}
 // the epilogue of one output element: g the (gate) accumulator, u the up accumulator of the gated forms
 JLA_DEV float lr_act(const RowLinear& p, float g, float u) {
   switch (p.act) {
@@ -17,10 +21,8 @@ JLA_DEV float lr_act(const RowLinear& p, float g, float u) {
     }
     case HY_ACT_SWIGLU:
       return hy_silu(g) * u;
-    case HY_ACT_CLAMP_GLU: {
-      const float gc = fminf(g, p.act_limit), uc = fminf(fmaxf(u, -p.act_limit), p.act_limit);
-      return gc * hy_sigmoid(p.act_alpha * gc) * (uc + 1.f);
-    }
+    case HY_ACT_CLAMP_GLU:
+      return lr_clamp_glu(p, g, u);
     case HY_ACT_SOFTCAP:
       return p.act_limit * tanhf(g / p.act_limit);
     case HY_ACT_GELU_GLU:

@@ -21,8 +21,8 @@
 // LDS images of both operands: [rows][8 cells of 16 B] (64 k); cell c of row r holds k-chunk c ^ ((r & 15) >> 1), so the 16
 // lanes of a fragment read fall on all 64 banks. A gated activation interleaves 16 gate rows and 16 up rows of W, which
 // puts a column's gate and up accumulators into neighbouring tiles of one wave.
-// The epilogue passes 64 rows at a time through the wave's own 32 KiB of LDS: the activation is then one small loop (of its own for SwiGLU and
-// for none: 2 % of a product) and rows leave as full lines (fp32: 512 B per row and wave).
+// The epilogue passes 64 rows at a time through the wave's own 32 KiB of LDS: the activation is then one small loop (of its own for SwiGLU, the
+// clamped gate and for none: 2 to 4 % of a product; in the loop for all activations the clamped gate had lost 2 %) and rows leave as full lines (fp32: 512 B per row and wave).
 #include "../kernels/gemm4w.h"
 #include "../kernels/row_tiles.h"
 #include "hy_util.h"
@@ -182,6 +182,10 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
           const f32x4 u = wl[rr * CH + ((gch + 4) ^ (rr & 15))];
 #pragma unroll
           for (int x = 0; x < 4; ++x) v[x] = hy_silu(v[x]) * u[x];
+        } else if constexpr (ACT == HY_ACT_CLAMP_GLU) {
+          const f32x4 u = wl[rr * CH + ((gch + 4) ^ (rr & 15))];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = lr_clamp_glu(p, v[x], u[x]);
         } else if constexpr (ACT != HY_ACT_NONE) {
           const f32x4 u = gated ? wl[rr * CH + ((gch + 4) ^ (rr & 15))] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -200,6 +204,7 @@ __global__ void __launch_bounds__(256, (RG_PER_CU<NJ, MI>)) rows_gemm_kernel(Row
     };
     // (the switch over activations stays out of the loop)
     if (p.act == HY_ACT_SWIGLU) rows_out(std::integral_constant<int, HY_ACT_SWIGLU>{});
+    else if (p.act == HY_ACT_CLAMP_GLU) rows_out(std::integral_constant<int, HY_ACT_CLAMP_GLU>{});
     else if (p.act == HY_ACT_NONE) rows_out(std::integral_constant<int, HY_ACT_NONE>{});
     else rows_out(std::integral_constant<int, -1>{});
   }
