@@ -1284,10 +1284,19 @@ static int g4_group_m(int tiles_m, int tiles_n, int K) {
   return gm < tiles_m ? gm : tiles_m;
 }
 static int g_g5_diag = 0;  // tools only (gemm5ws.h diag bits 1-16; gemm4 store ablations 64 / 128: wrong results)
-// The persistent residual form takes three x slots where the loop outweighs its ends, long K or more than two rounds of tiles. Two
-// -> three, us: N 4096 K 14336, M 8192 | 12800 721 -> 680 | 1134 -> 1092; K 4096, M 12800 (800 tiles) 386 -> 375, M 8192 (two
-// rounds) 216 -> 219. (The non-persistent form gains at K 14336 only, 686 -> 652, and loses up to 1 % elsewhere: it keeps two.)
-constexpr int G4_X3_K = 8192;
+// Where the persistent residual form takes three x slots: the loop has to outweigh its ends (a long K, the longer the fewer rounds there are),
+// and of wide outputs, whose W does not stay in the L2s, the steps too. Two -> three, us, tiles in brackets: N 4096, K 14336 734 -> 693 (512),
+// 1357 -> 1281 (800); K 4096 462 -> 435 (800); K 2048 287 -> 272 (800), 306 -> 290 (1024); K 1024 203 -> 196 (800); K 28672 634 -> 540 (128); but
+// N 8192, K 1024 237 -> 252 (1024), 287 -> 303 (1280), K 2048 326 -> 342 (1024); K 8192 429 -> 437 (512), N 4096 158 to 167 -> 169 (128), N
+// 5120, K 14336 290 to 294 -> 300 (160). Even or less than 2 %: N 8192, K 4096 (1024 and more), N 5120, K 1024 to 4096 (800). (The
+// non-persistent form gains at K 14336 only, 686 -> 652, and loses up to 1 % elsewhere: it keeps two.)
+static bool g4_x3(int tiles, int tn, int K) {
+  const int cus = num_cus();
+  const bool wide = tn > 20;  // more than 5120 columns
+  if (tiles < cus) return K >= 16384;
+  if (tiles <= 2 * cus) return K >= (wide ? 10240 : 8192);
+  return !wide || K >= 4096;
+}
 
 template <int MODE, int NJ = 8>
 static void launch_g4(const bf16_t* x, const u32x4* w, void* out, int M, int N, int K, int accumulate, int out_f32,
@@ -1308,10 +1317,14 @@ static void launch_g4(const bf16_t* x, const u32x4* w, void* out, int M, int N, 
       } else if (rms) {
         gemm4p_kernel<MODE, 1><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps, qa,
                                                   nullptr, gm);
-      } else if (MODE == MODE_RESIDUAL && (K >= G4_X3_K || grid > 2 * num_cus())) {
-        gemm4p_kernel<MODE, 0, true><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps,
-                                                        qa, nullptr, gm);
       } else {
+        if constexpr (MODE == MODE_RESIDUAL) {
+          if (g4_x3(grid, tn, K)) {
+            gemm4p_kernel<MODE, 0, true><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn,
+                                                            rms_eps, qa, nullptr, gm);
+            return;
+          }
+        }
         gemm4p_kernel<MODE, 0><<<pg, 256, 0, s>>>(x, w, out, M, N, K, accumulate, out_f32, mirror, tm, tn, rms_eps, qa,
                                                   nullptr, gm);
       }

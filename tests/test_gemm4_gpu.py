@@ -177,10 +177,13 @@ def test_gemm4_model_prefill_matches_gemm2():
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 512, 8192), (300, 512, 8256), (257, 512, 8320), (4352, 8192, 64), (4352, 8192, 128),
-                                   (4300, 8192, 192), (4352, 8192, 256)])
+                                   (4300, 8192, 192), (4352, 8192, 256), (6912, 5120, 64), (6800, 5120, 128), (6912, 5104, 192),
+                                   (6912, 5120, 256), (300, 512, 16384), (300, 512, 16448), (257, 512, 16512), (4096, 4096, 8192),
+                                   (4096, 4096, 8128), (4352, 8192, 4096)])
 def test_gemm4_persistent_residual_three_slots(m, n, k):
-    """The persistent residual form with three x slots (long K, or more than two rounds of tiles; every phase of the slots and
-    one to four K-tiles) runs the same chain of products as tile 7: bit-identical."""
+    """The persistent residual form with three x slots (more than two rounds of tiles of up to 5120 columns, one round and K
+    8192, fewer and K 16384, and what is just short of that; every phase of the slots and one to four K-tiles) runs the same
+    chain of products as tile 7: bit-identical."""
     e = ops.ext()
     g = torch.Generator(device=DEV).manual_seed(m + k)
     x = torch.randn(m, k, device=DEV, generator=g).to(BF16)
