@@ -103,12 +103,17 @@ JLA_DEV void rv_better(float& bv, int& bi, float v, int i) {
   }
 }
 
-// FORM of a kernel: -1, any call; else one of plain rows -- in place and order, of one matrix or the table's experts -- whose results go to fp32 rows
-// in order through RowAct FORM % 8, with RV_RES a pending residual add, with RV_NORM a norm, with RV_MUL the gate table, with RV_ADD onto the output and with RV_ONE one row per group: the branches that such a call does not take are
-// not in its code. A launch of a few microseconds waits for the code on its path, some 0.13 us per KB. One row, weights in no cache, any call's code ->
-// its own: 2048 x 2048 8.4 -> 5.9 KB, 4.1 -> 3.7 us; 2048 x 5152 5.5 -> 3.1 KB, 6.2 -> 5.8; walking, normed 2048 x 2048 9.8 -> 3.2 KB, 4.9 -> 4.3,
-// 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096 with a residual 10.3 -> 9.5. A trace of eight tokens on fp32 weights 4.76 -> 4.62 ms. Two rows keep any call's walk (as a loop over the rows it was
-// smaller and slower: the first weights were waited for at its edge).
+// FORM of a kernel: -1, any call; else one of plain rows -- in place and order, of one matrix or the table's experts -- whose results go to
+// fp32 rows in order through RowAct FORM % 8; RV_RES: with a pending residual add, RV_NORM: a norm, RV_MUL: the gate table, RV_ADD: onto the
+// output, RV_ONE: one row per group. The branches that such a call does not take are not in its code: a launch of a few microseconds waits for
+// the code on its path, some 0.13 us per KB. One row, weights in no cache, any call's code -> its own: 2048 x 2048 8.4 -> 5.9 KB, 4.1 -> 3.7 us;
+// 2048 x 5152 5.5 -> 3.1 KB, 6.2 -> 5.8; walking, normed 2048 x 2048 9.8 -> 3.2 KB, 4.9 -> 4.3, 2048 x 32000 10.6 -> 3.6 KB, 22.8 -> 21.7; 4096 x 4096
+// with a residual 10.3 -> 9.5. Over 11 to 13 shapes of K 512 to 4096 and N 1024 to 32000, in parts of the time in any call's code, one row: normed
+// 0.92 (no activation, SwiGLU, clamped gate), a pending add 0.94, both 0.97 (up to 3072 columns 0.94, of 5152 and 10304 1.05 to 1.08, of more 0.97); on
+// fp32 weights normed 0.97 (soft cap, clamped gate and none), a pending add 0.97 (none, SwiGLU), both 0.98, as it is or onto the output 0.99.
+// Only these have one, with the greedy choice behind a norm and the gate table behind a pending add: a token's calls in the families that this was
+// measured for. Squared ReLU, GELU gates, the soft cap without its choice on bf16 weights, results in bf16 and two walking rows keep any call's
+// (those as a loop over the rows were smaller and slower: the first weights were waited for at its edge).
 constexpr int RV_RES = 8, RV_NORM = 16, RV_ONE = 32, RV_MUL = 64, RV_ADD = 128;
 constexpr int RV_GATE = HY_ACT_NONE + RV_RES + RV_ONE + RV_MUL;
 template <int FORM>
@@ -1049,7 +1054,7 @@ static int rv_rows32(const RowLinear& p, hipStream_t s) {
   if (tg > 0x7fffffffLL) return -4;
   const dim3 grid((unsigned)((tg + rounds - 1) / rounds), groups);
 #define RV_RUN32(NT, V, RW) rows_walk_f32_kernel<NT, V, RW, 0><<<grid, 256, 0, s>>>(p, rpg, gated, (int)tg, RowParts{})
-// (one row: the forms of this file's first comment on them, for the activations and additions that a decode step has)
+// (one row: FORM's comment says which forms have code of their own)
 #define RV_FORM32(NT, V, F)                                                                                        \
   if (form == (F)) {                                                                                               \
     rows_walk_f32_kernel<NT, V, 1, 0, F><<<grid, 256, 0, s>>>(p, rpg, gated, (int)tg, RowParts{});                 \

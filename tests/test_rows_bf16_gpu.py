@@ -45,13 +45,14 @@ def test_products(m, n, k):
 @pytest.mark.parametrize("m", [1, 2])
 @pytest.mark.parametrize("n,k", [(64, 8), (65, 64), (70, 128), (2048, 64), (2050, 120), (300, 32)])
 def test_short_rows(m, n, k):
-    """One or two fp32 rows of up to 128 numbers: every product is exact in fp32, of which a lane adds 8 per fourth of the row in 24 bits (2^-24 each)."""
+    """One or two fp32 rows of up to 128 numbers: exact products, eight at a time added in 24 bits, these sums in 64: 3.3e-8 (K 64) and 4.1e-8
+    (K 128) of the result measured, with the result's own rounding; twice that."""
     g = torch.Generator(device=DEV).manual_seed(n + k)
     x = torch.randn(m, k + 4, generator=g, device=DEV)[:, :k]  # (rows apart)
     w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF16)
     want = x.to(BF16).double() @ w.double().t()
     got = hy.linear(x, w)
-    assert got.shape == (m, n) and _err(got, want) < 32 * 2.0 ** -24
+    assert got.shape == (m, n) and _err(got, want) < 8e-8
     # a weight that is none stays in its column, also where the row ends inside the instruction's step
     w[n - 1, k - 1] = float("inf")
     bad = hy.linear(x, w)
