@@ -18,9 +18,9 @@
 // Ties: lower vocabulary index first (lax.top_k order).
 // What bounds it: of few rows the dependent steps and the code on their path (some 0.13 us per KB in a launch of a few us), of many the vector unit's
 // issue and the logits' bytes. Warm, both launches, top 50, us: chunks of 16384 with two radix selects and a sort | of 4096, bound by a radix select
-// | here: 128256 columns, 1 row 17.4 | 13.7 | 11.7, 7 17.7 | 14.9 | 12.1, 64 20.5 | 20.1 | 16.8, 300 42.0 | 43.0 | 34.1, 1400 188 | 182 | 141; 32000,
-// 1 row 19.6 | 12.4 | 9.9, 1400 57.4 | 66.0 | 36.5; top 64 of 300 x 128256 42.0 | 62.4 | 35.7. Chunks of 4096 here: 1 x 16032 9.1 for 10.5, 300 x
-// 128256 39.1, 1400 x 32000 43.9.
+// | here: 128256 columns, 1 row 17.5 | 13.8 | 11.8, 7 17.8 | 15.0 | 12.5, 64 20.9 | 19.7 | 17.2, 300 42.1 | 42.8 | 36.2, 1400 188 | 181 | 145; 32000,
+// 1 row 19.4 | 12.3 | 10.0, 1000 45.1 | 50.5 | 30.9, 2048 73.6 | 92.3 | 52.0; top 64 of 300 x 128256 41.9 | 62.1 | 37.1. Chunks of 4096 in the present
+// form: 1 x 16032 9.1 for 10.4, 300 x 128256 39.1, 1400 x 32000 43.9 for 38.7.
 #include "common.h"
 #include "launchers.h"
 
